@@ -11,6 +11,7 @@
 // K rows are permuted inside a tile so that the accumulators of two 16-key sub-tiles are the 32-key B operand of the second
 // product.
 #include "latent_attn.h"
+#include "prompt_tiles.h"
 
 namespace tlf {
 
@@ -25,7 +26,8 @@ struct LatentPrefillArgs {
   const float *gate;                // [rows, H] or NULL
   unsigned short *out;              // [rows, ldo]
   int64_t lde, ldo;
-  int32_t first_seq, window, xtiles, total, per_xcd;
+  PromptTiles tiles;
+  int32_t first_seq, window;
   float scale_log2;
 };
 
@@ -39,12 +41,10 @@ template <int DC, int VC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_prefill_kernel(const LatentPrefillArgs p) {
   constexpr int CT = 2, DP = DC * 32, VP = VC * 32;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kPK][DP + 8], Vs[kPK][VP + 16];
-  // consecutive row tiles of one head share keys: they go to the same XCD (workgroup w runs on XCD w % 8)
-  const int id = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
-  if (id >= p.total) return;
+  int sq, h, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, sq, h, xt)) return;
   const LatentShape &s = p.s;
-  const int xt = id % p.xtiles, rest = id / p.xtiles;
-  const int h = rest % s.H, sq = rest / s.H, seq = p.first_seq + sq;
+  const int seq = p.first_seq + sq;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
   const int row0 = xt * kPQ;
   if (row0 >= lq) return;
@@ -262,12 +262,8 @@ extern "C" int tlf_latent_prefill(const void *q, const void *expanded, int64_t e
   a.latents = static_cast<const unsigned short *>(latents); a.cu_q = cu_seqlens_q; a.starts = seq_starts; a.kv_off = kv_offsets;
   a.out = static_cast<unsigned short *>(out); a.lde = expanded_stride; a.ldo = out_stride; a.first_seq = first_seq;
   a.gate = gate; a.window = window; a.scale_log2 = scale * 1.4426950408889634f;
-  a.xtiles = (max_tokens + kPQ - 1) / kPQ;
-  const int64_t total = static_cast<int64_t>(a.xtiles) * heads * num_seqs;
-  if (total > (1 << 30)) return TLF_E_SHAPE;
-  a.total = static_cast<int32_t>(total);
-  a.per_xcd = (a.total + 7) / 8;
-  const dim3 grid(a.per_xcd * 8);
+  const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + kPQ - 1) / kPQ, heads, num_seqs));
+  if (!grid.x) return TLF_E_SHAPE;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int dc = fit_units(a.s.Dq / 32), vc = (vdim + 31) / 32;
 #define TLF_LP(DC, VC) TLF_LAUNCH((latent_prefill_kernel<DC, VC>), grid, dim3(256), 0, st, a)

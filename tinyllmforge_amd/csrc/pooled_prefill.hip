@@ -10,6 +10,7 @@
 // The weights are not normalised: no running maximum, no rescaling, no second pass.  K rows are permuted inside a
 // tile so that the accumulators of two 16-key sub-tiles are the 32-key B operand of the second product.
 #include "pooled_attn.h"
+#include "prompt_tiles.h"
 
 namespace tlf {
 
@@ -24,8 +25,8 @@ struct PooledPrefillArgs {
   unsigned short *out;
   int64_t ldo;
   int32_t H, group, hpp, passes;   // query heads, per KV head, per pass
-  int32_t bq, xtiles, total;       // query rows per workgroup, row tiles, workgroups
-  int32_t first_seq, per_xcd;
+  int32_t bq, first_seq;           // query rows per workgroup
+  PromptTiles tiles;
   float scale_log2;
 };
 
@@ -40,14 +41,10 @@ template <int DC, int CT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void pooled_prefill_kernel(const PooledPrefillArgs p) {
   constexpr int DP = DC * 32, NCH = DC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kTK][DP + 8], Vs[kTK][DP + 16];
-  // consecutive row tiles of one KV head share keys: they go to the same XCD (workgroup w runs on XCD w % 8)
-  const int id = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
-  if (id >= p.total) return;
+  int sq, plane, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
   const PooledCache &c = p.c;
-  const int xt = id % p.xtiles, rest = id / p.xtiles;
-  const int planes = c.G * p.passes;
-  const int plane = rest % planes, seq = p.first_seq + rest / planes;
-  const int kvh = plane / p.passes, pass = plane % p.passes;
+  const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
   const int row0 = xt * p.bq;
   if (row0 >= lq) return;
@@ -244,16 +241,12 @@ extern "C" int tlf_pooled_attn_prefill(const void *q, const void *score_bias, co
   const int dc = c.Dp / 32, ct = dc <= 4 ? 2 : 1, units = 64 * ct;
   PooledPrefillArgs a{c, static_cast<const unsigned short *>(q), static_cast<const unsigned short *>(score_bias), gate,
                       cu_seqlens_q, seq_starts, static_cast<unsigned short *>(out), out_stride, num_q_heads,
-                      num_q_heads / num_kv_heads, 0, 0, 0, 0, 0, first_seq, 0, scale * kLog2e};
+                      num_q_heads / num_kv_heads, 0, 0, 0, first_seq, {}, scale * kLog2e};
   a.hpp = a.group < units ? a.group : units;
   a.passes = (a.group + a.hpp - 1) / a.hpp;
   a.bq = units / a.hpp;
-  a.xtiles = (max_tokens + a.bq - 1) / a.bq;
-  const int64_t total = static_cast<int64_t>(a.xtiles) * num_kv_heads * a.passes * num_seqs;
-  if (total > (1 << 30)) return TLF_E_SHAPE;
-  a.total = static_cast<int32_t>(total);
-  a.per_xcd = (a.total + 7) / 8;
-  const dim3 grid(a.per_xcd * 8);
+  const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, num_kv_heads * a.passes, num_seqs));
+  if (!grid.x) return TLF_E_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dc) {
     case 1: TLF_LAUNCH((pooled_prefill_kernel<1, 2>), grid, dim3(256), 0, s, a); break;

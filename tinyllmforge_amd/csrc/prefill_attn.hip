@@ -37,6 +37,7 @@
 #include <stdlib.h>
 
 #include "common.h"
+#include "prompt_tiles.h"
 
 namespace tlf {
 
@@ -105,7 +106,7 @@ struct PrefillParams {
   int32_t block_size;
   int64_t num_cache_blocks;
   float scale_log2;
-  int32_t pair_group;  // (sequence, KV head) pairs an XCD walks together, row tiles outermost
+  PromptTiles tiles;
 };
 
 // LDS transpose read: within each group of 16 lanes, lane i receives
@@ -167,26 +168,11 @@ void prefill_attn_kernel(const PrefillParams p) {
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kBKV][kPRowK];  // bf16, rows in k_tile_row order
   __shared__ __attribute__((aligned(16))) unsigned short Vs[kBKV][kPRowV];  // fp16 (bf16 for a tile fp16 cannot hold)
   __shared__ __attribute__((aligned(16))) unsigned int vvote[8];            // per wave: what its V slice holds
-  // Workgroup -> (sequence, KV head, row tile).  Workgroups go to the 8 XCDs round robin by their linear id, and
-  // each XCD has its own L2: when the (sequence, KV head) pairs divide evenly, pair j runs entirely on XCD j % 8,
-  // so the K/V rows its row tiles share are fetched into one L2 instead of eight.  An XCD takes its pairs
-  // pair_group at a time and walks their row tiles together, the last row tiles (the longest key ranges) first,
-  // so that the launch ends on short workgroups.
-  int seq = blockIdx.z, h = blockIdx.y, xt = blockIdx.x;
-  const int pairs = gridDim.y * gridDim.z;
-  if (pairs % 8 == 0) {
-    const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int slot = lin >> 3;
-    const int gx = static_cast<int>(gridDim.x), G = p.pair_group;   // G divides pairs / 8 (host)
-    const int grp = slot / (G * gx), within = slot % (G * gx);
-    const int pair = (lin & 7) + 8 * (grp * G + within % G);
-    xt = within / G;
-    h = pair % static_cast<int>(gridDim.y);
-    seq = pair / static_cast<int>(gridDim.y);
-  }
+  int seq, h, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, seq, h, xt)) return;
   const int group = p.num_q_heads / p.num_kv_heads;
   const int bq = (16 * NWV * CT) / group;  // query rows per workgroup
-  const int row0 = (gridDim.x - 1 - xt) * bq;
+  const int row0 = xt * bq;
   const int q_begin = p.cu_q[seq];
   const int lq = p.cu_q[seq + 1] - q_begin;
   if (row0 >= lq) return;
@@ -559,23 +545,9 @@ extern "C" int tlf_varlen_prefill_attn(const void *q, int64_t q_stride, const vo
   }();
   const int nwv = forced ? forced : 8;
   const int ct = nwv == 8 ? 3 : 2;
-  // An XCD walks its (sequence, KV head) pairs four at a time with the row tiles outermost, longest first: with
-  // one pair after the other the last pair's long row tiles start when most slots are already idle (16 x 1024
-  // tokens 304 -> 287 us, 28 x 560 190 -> 182, 4 x 4096 779 -> 757); four pairs' K/V rows (2 MB at 1024 tokens)
-  // still share the XCD's L2.  TLF_PREFILL_PAIR_GROUP overrides for tuning (a power of two).
-  static const int forced_group = [] {
-    const char *e = getenv("TLF_PREFILL_PAIR_GROUP");
-    const int v = e ? atoi(e) : 0;
-    return v >= 1 && v <= 64 && (v & (v - 1)) == 0 ? v : 0;
-  }();
-  {
-    const int per_xcd = (num_kv_heads * num_seqs) / 8;  // only used when the pairs divide evenly over the XCDs
-    int grp = forced_group ? forced_group : 4;
-    while (grp > 1 && (per_xcd < 1 || per_xcd % grp)) grp >>= 1;
-    p.pair_group = grp;
-  }
   const int bq = (16 * nwv * ct) / group;
-  const dim3 grid((max_seqlen_q + bq - 1) / bq, num_kv_heads, num_seqs);
+  const dim3 grid(prompt_tiles_make(p.tiles, (max_seqlen_q + bq - 1) / bq, num_kv_heads, num_seqs));
+  if (!grid.x) return TLF_E_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (paged && kv_dtype == TLF_KV_FP8_E4M3) {
     // the K scale is a per-head constant of the scores: fold it in on the device side per head

@@ -1,0 +1,47 @@
+// Which (sequence, plane, row tile) of a batch of prompt portions a workgroup takes.  A plane is what shares keys: a KV head, or a
+// pass over some of its query heads.
+//
+// Workgroup w runs on XCD w % 8, and each XCD has its own L2.  Portions have unequal lengths and a row tile's work grows with its
+// place, so every XCD gets the same planes of every sequence: plane p of any sequence goes to XCD p % 8.  Planes that do not come
+// out even over eight XCDs are cut into `parts`, a plane's row tiles dealt to its parts in turn.  (Handing each XCD a run of
+// consecutive (sequence, plane) pairs gives it whole sequences, and the launch waits for the XCD with the longest one.)
+//
+// An XCD takes its planes four at a time and walks their row tiles together, the last ones (the longest key ranges) first, so that
+// it ends on short workgroups while the planes at work still fit its L2 (4 x 1 MB at 2048 keys of 2 x 128 bf16).  The order of the
+// four turns by one from row tile to row tile: an XCD deals its workgroups to its four shader engines in turn as well, and without
+// the turn each engine gets all row tiles of one sequence, and the launch waits for the engine with the longest.
+//
+// Eight prompts of 1061 to 2048 tokens, 32 heads on 8 KV heads (sink_prefill.hip): 521 us with either of the two mistakes, as long
+// as eight prompts of 2048; 355 us so.
+#pragma once
+#include "common.h"
+
+namespace tlf {
+
+struct PromptTiles {
+  int32_t xtiles, planes, parts, per_part, per_xcd;   // row tiles; planes of a sequence; parts of a plane, their tiles; parts per XCD
+};
+
+// Workgroups to launch, 0: too many.
+inline int prompt_tiles_make(PromptTiles &t, int64_t xtiles, int64_t planes, int64_t seqs) {
+  int parts = 8;
+  while (parts > 1 && planes * (parts / 2) % 8 == 0) parts /= 2;
+  const int64_t most = 1 << 27, per_part = (xtiles + parts - 1) / parts, per_xcd = planes * parts / 8 * seqs;
+  if (per_part > most || per_xcd > most || per_part * per_xcd > most) return 0;
+  t = PromptTiles{static_cast<int32_t>(xtiles), static_cast<int32_t>(planes), parts, static_cast<int32_t>(per_part), static_cast<int32_t>(per_xcd)};
+  return static_cast<int>(per_part * per_xcd * 8);
+}
+
+// False: nothing to do.
+__host__ __device__ inline bool prompt_tile(const PromptTiles &t, int block, int &seq, int &plane, int &xt) {
+  constexpr int kTogether = 4;
+  const int i = block >> 3, first = i / (kTogether * t.per_part) * kTogether;
+  const int together = t.per_xcd - first < kTogether ? t.per_xcd - first : kTogether, within = i - first * t.per_part;
+  const int step = within / together, part = (first + (within + step) % together) * 8 + (block & 7), of_seq = t.planes * t.parts;
+  seq = part / of_seq;
+  plane = part % of_seq / t.parts;
+  xt = t.xtiles - 1 - (step * t.parts + part % t.parts);
+  return xt >= 0;
+}
+
+}  // namespace tlf

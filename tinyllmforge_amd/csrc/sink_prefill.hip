@@ -9,6 +9,7 @@
 //   O^T[dim, unit] += V^T . P^T   V^T by LDS transpose reads; P as a bf16 hi + lo pair (16 significant bits)
 // K rows are permuted inside a tile so that the accumulators of two 16-key sub-tiles are the 32-key B operand of the second
 // product.  Only tiles that the diagonal cuts are masked.  The sink and the gate are applied at the end.
+#include "prompt_tiles.h"
 #include "sink_attn.h"
 
 namespace tlf {
@@ -25,7 +26,8 @@ struct SinkPrefillArgs {
   unsigned short *out;
   int64_t ldo, ldg;
   int32_t H, group, hpp, passes;    // query heads, per KV head, per pass
-  int32_t bq, xtiles, total, first_seq, per_xcd, table_cols;
+  PromptTiles tiles;
+  int32_t bq, first_seq, table_cols;
 };
 
 __device__ __forceinline__ int sink_tile_row(int t) { return (t & 32) | ((t & 4) << 2) | ((t & 24) >> 1) | (t & 3); }
@@ -38,15 +40,10 @@ template <int DC, int VC, int CT, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void sink_prefill_kernel(const SinkPrefillArgs p) {
   constexpr int DP = DC * 32, VP = VC * 32, KCH = DC * 4, VCH = VC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kSK][DP + 8], Vs[kSK][VP + 16];
-  // consecutive row tiles of one KV head share keys: they go to the same XCD (workgroup w runs on XCD w % 8); the last row
-  // tiles, which see the most keys, come first
-  const int id = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
-  if (id >= p.total) return;
+  int sq, plane, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
   const SinkCache &c = p.c;
-  const int xt = p.xtiles - 1 - id % p.xtiles, rest = id / p.xtiles;
-  const int planes = c.G * p.passes;
-  const int plane = rest % planes, seq = p.first_seq + rest / planes;
-  const int kvh = plane / p.passes, pass = plane % p.passes;
+  const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
   const int row0 = xt * p.bq;
   if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
@@ -299,13 +296,9 @@ extern "C" int tlf_sink_attn_prefill(const void *q, const void *k_cache, const v
   a.H = heads; a.group = heads / kv_heads; a.hpp = a.group < units ? a.group : units;
   a.passes = (a.group + a.hpp - 1) / a.hpp;
   a.bq = units / a.hpp;
-  a.xtiles = (max_tokens + a.bq - 1) / a.bq;
   a.first_seq = first_seq; a.table_cols = static_cast<int32_t>(bt_stride);
-  const int64_t total = static_cast<int64_t>(a.xtiles) * kv_heads * a.passes * num_seqs;
-  if (total > (1 << 30)) return TLF_E_SHAPE;
-  a.total = static_cast<int32_t>(total);
-  a.per_xcd = (a.total + 7) / 8;
-  const dim3 grid(a.per_xcd * 8);
+  const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, kv_heads * a.passes, num_seqs));
+  if (!grid.x) return TLF_E_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define TLF_SP(DC, VC)                                                                                                        \
   do {                                                                                                                        \

@@ -14,6 +14,7 @@
 // from the cache into LDS directly, behind the weights and the mix; rows are unpadded and pairs of their 16-byte pieces swizzled
 // against bank conflicts (the lane that fills a position picks the matching piece).
 #include "gemm_shared.h"
+#include "prompt_tiles.h"
 #include "talk_attn.h"
 
 namespace tlf {
@@ -31,7 +32,8 @@ struct TalkPrefillArgs {
   int64_t ldo;
   int32_t H, group;
   int32_t hpp, passes, bq;          // stats: query heads per pass, passes, rows per workgroup
-  int32_t xtiles, total, first_seq, per_xcd, table_cols;
+  PromptTiles tiles;
+  int32_t first_seq, table_cols;
 };
 
 template <typename T>
@@ -46,11 +48,10 @@ template <int DC, int CT>
 __global__ __launch_bounds__(256) void talk_stats_kernel(const TalkPrefillArgs p) {
   constexpr int DP = DC * 32, KCH = DC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[2][kTS][DP + 8];
-  const int id = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);   // row tiles of one KV head share keys: the same XCD
-  if (id >= p.total) return;
+  int sq, plane, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
   const SinkCache &c = p.c;
-  const int xt = p.xtiles - 1 - id % p.xtiles, rest = id / p.xtiles, planes = c.G * p.passes;    // the longest first
-  const int plane = rest % planes, seq = p.first_seq + rest / planes, kvh = plane / p.passes, pass = plane % p.passes;
+  const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
   const int row0 = xt * p.bq;
   if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
@@ -188,10 +189,10 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
   constexpr int kAtOnce = HT == 1 ? 4 : 1;                           // rows of the mix, as registers allow
   extern __shared__ __attribute__((aligned(1024))) unsigned short lds[];
   unsigned short *Vs = lds, *Wh = lds + p.c.G * kTK * VP, *Wl = Wh + TQ * ROW, *Ts = Wl + TQ * ROW;    // Vs [G][32][VP], Ts [16 HT][TS]
-  const int id = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);   // neighbours in rows share keys: the same XCD
-  if (id >= p.total) return;
+  int sq, plane, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
   const SinkCache &c = p.c;
-  const int xt = p.xtiles - 1 - id % p.xtiles, seq = p.first_seq + id / p.xtiles;       // the longest first
+  const int seq = p.first_seq + sq;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
   const int row0 = xt * TQ;
   if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
@@ -461,12 +462,9 @@ int launch_talk_stats(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStrea
   a.hpp = a.group < kUnits ? a.group : kUnits;
   a.passes = (a.group + a.hpp - 1) / a.hpp;
   a.bq = kUnits / a.hpp;
-  a.xtiles = (max_tokens + a.bq - 1) / a.bq;
-  const int64_t total = static_cast<int64_t>(a.xtiles) * a.c.G * a.passes * num_seqs;
-  if (total > (1 << 28)) return TLF_E_SHAPE;
-  a.total = static_cast<int32_t>(total);
-  a.per_xcd = (a.total + 7) / 8;
-  TLF_LAUNCH((talk_stats_kernel<DC, CT>), dim3(a.per_xcd * 8), dim3(256), 0, s, a);
+  const int grid = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, a.c.G * a.passes, num_seqs);
+  if (!grid) return TLF_E_SHAPE;
+  TLF_LAUNCH((talk_stats_kernel<DC, CT>), dim3(grid), dim3(256), 0, s, a);
   return launch_status();
 }
 
@@ -475,12 +473,9 @@ int launch_talk_prefill(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStr
   static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&talk_prefill_kernel<WV, RT, DC, VC, GS>),
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, kTalkLds);
   if (allowed != hipSuccess) return static_cast<int>(allowed);
-  a.xtiles = (max_tokens + RT * 16 - 1) / (RT * 16);
-  const int64_t total = static_cast<int64_t>(a.xtiles) * num_seqs;
-  if (total > (1 << 28)) return TLF_E_SHAPE;
-  a.total = static_cast<int32_t>(total);
-  a.per_xcd = (a.total + 7) / 8;
-  TLF_LAUNCH((talk_prefill_kernel<WV, RT, DC, VC, GS>), dim3(a.per_xcd * 8), dim3(WV * RT * 64), talk_prefill_lds(WV, RT, a.c.G, a.c.Vp), s, a);
+  const int grid = prompt_tiles_make(a.tiles, (max_tokens + RT * 16 - 1) / (RT * 16), 1, num_seqs);
+  if (!grid) return TLF_E_SHAPE;
+  TLF_LAUNCH((talk_prefill_kernel<WV, RT, DC, VC, GS>), dim3(grid), dim3(WV * RT * 64), talk_prefill_lds(WV, RT, a.c.G, a.c.Vp), s, a);
   return launch_status();
 }
 template <int WV, int RT>
