@@ -52,3 +52,33 @@ def test_every_row_of_uneven_batches(lens, heads, kv_heads):
                                None, out)
     want = torch.cat([plain(scaled[a:b].float() * 0.6931471805599453, k[a:b], v[a:b]) for a, b in zip(cu.tolist(), cu.tolist()[1:])])
     close(out)
+
+
+@pytest.mark.parametrize("dim,vdim", [(32, 32), (56, 100), (96, 64), (128, 128), (136, 128), (128, 136)])
+@pytest.mark.parametrize("cap", [None, 20.0, 50.0])
+def test_weights_follow_a_growing_maximum(dim, vdim, cap):
+    """Scores that climb by more than 2^8 at random keys, in even and odd halves of a tile, behind a prefix in the cache."""
+    torch.manual_seed(dim + vdim)
+    dev, BF, heads, start, new, log2e = "cuda", torch.bfloat16, 4, 70, 203, 1.4426950408889634
+    total = start + new
+    kv = ops.SinkKV(-(-total // 64), 64, 1, dim, vdim, BF, dev)
+    k, v = torch.randn(total, dim) * 0.2, torch.randn(total, vdim)
+    k[:, 0] = torch.cumsum((torch.rand(total) < 0.05).float() * torch.rand(total) * 30, 0)
+    k, v = k.to(BF), v.to(BF)
+    for j in range(0, total, 64):
+        rows = min(64, total - j)
+        kv.k[j // 64, 0, :rows, :dim], kv.v[j // 64, 0, :rows, :vdim] = k[j:j + rows].to(dev), v[j:j + rows].to(dev)
+    q = torch.randn(new, heads, dim) * 0.3
+    q[:, :, 0] = torch.tensor([1.0, -1.0, 0.0, 0.3])
+    q = q.to(BF)
+    padded = torch.zeros(new, heads, kv.k.shape[3], dtype=BF, device=dev)
+    padded[..., :dim] = q.to(dev)
+    out = torch.full((new, heads * vdim), torch.nan, device=dev, dtype=BF)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=dev)
+    ops.sink_attention_prefill(padded, kv, i32(*range(kv.k.shape[0])).view(1, -1), i32(0, new), i32(start), 0, 1, new, None, None, cap, out)
+    s = torch.einsum("ihd,jd->hij", q.double(), k.double())             # scores in log 2 units, or 2 log2(e) / cap times them
+    s = s / log2e if cap is None else cap * torch.tanh(s / log2e / 2)
+    s = s.masked_fill(torch.arange(total) > torch.arange(start, total)[:, None], -torch.inf)
+    want = torch.einsum("hij,jd->ihd", torch.softmax(s, -1), v.double())
+    # bf16 result (2^-9) of weights with 16 significant bits and fp32 scores of up to 2^8
+    torch.testing.assert_close(out.view(new, heads, vdim).double().cpu(), want, rtol=2 ** -8, atol=2 ** -10)

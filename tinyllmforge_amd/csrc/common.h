@@ -75,6 +75,20 @@ __device__ __forceinline__ unsigned int pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(unsigned int, r);
 }
 
+// Two fp32 values as bf16 pairs, hi + lo: 16 significant bits.  For weights of attention: hi must be finite, since the other value's
+// hi enters each difference times zero.  v_dot2 takes the difference a - hi straight from the packed halves (exact: checked against
+// the subtraction over all exponents), four instructions where shifting and masking the halves takes six, and seven as the compiler
+// writes it.  The constant (-1, 0) has to come from a register: as the inline constant -1.0 the hardware reads (0, -1).
+__device__ __forceinline__ void weight_pairs(float a, float b, unsigned int &hi, unsigned int &lo) {
+  typedef __bf16 pair __attribute__((ext_vector_type(2)));
+  unsigned int low;
+  asm("s_mov_b32 %0, 0xbf80" : "=s"(low));
+  hi = pack_bf16x2(a, b);
+  const pair h = __builtin_bit_cast(pair, hi);
+  lo = pack_bf16x2(__builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, low), a, false),
+                   __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, 0xbf800000u), b, false));
+}
+
 __device__ __forceinline__ void unpack8(const uint4 &p, float (&f)[8]) {
   f[0] = __uint_as_float(p.x << 16);
   f[1] = __uint_as_float(p.x & 0xffff0000u);

@@ -93,6 +93,10 @@ inline int partials_check(const void *partials, const float *scale, int32_t spli
 }
 
 __device__ __forceinline__ float sigmoid_f32(float z) { return 1.0f / (1.0f + expf(-z)); }
+// The same from the hardware's exponential and reciprocal, 4 instructions instead of 25; relative error below 2^-21 + |z| 2^-24.
+__device__ __forceinline__ float sigmoid_fast(float z) {
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
+}
 __device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + expf(-z)); }
 
 // xIELU: a z^2 + z / 2 above zero, b (e^z - 1 - z) + z / 2 below; a = softplus(p), b = 1/2 + softplus(q).

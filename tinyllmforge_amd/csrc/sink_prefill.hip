@@ -1,14 +1,13 @@
 // Attention of sink_attn.h for prompt portions, bf16, on the matrix cores, from the paged cache.
 //
 // A workgroup owns one portion, one KV head and a tile of query rows; the (row, head) pairs of the KV head's query heads are
-// flattened into 64 CT units, 16 CT per wave.  It walks the keys up to its last row 64 at a time (a tile of 64 keys is one
-// contiguous piece of a page; global -> registers one tile ahead -> LDS):
-//   S^T[key, unit] = K . Q^T      v_mfma_f32_16x16x32_bf16
-//   P = 2^(score - m)             fp32; m follows a unit's maximum only when that has grown by more than 8 (a factor of 256,
-//                                 which the fp32 sums and the bf16 pair hold), so the accumulators are rarely rescaled
-//   O^T[dim, unit] += V^T . P^T   V^T by LDS transpose reads; P as a bf16 hi + lo pair (16 significant bits)
-// K rows are permuted inside a tile so that the accumulators of two 16-key sub-tiles are the 32-key B operand of the second
-// product.  Only tiles that the diagonal cuts are masked.  The sink and the gate are applied at the end.
+// flattened into 64 CT units, 16 CT per wave.  The loop is prompt_core.h's; a tile of 64 keys is one contiguous piece of a page.
+//   P = 2^(score - m)   fp32; m follows a unit's maximum only when that has grown by more than 8 (a factor of 256, which the fp32
+//                       sums and the bf16 pair hold), so the accumulators are rarely rescaled.  Without a cap the scores begin at -m,
+//                       and whether any has grown is asked lane by lane; maxima of units are only formed when one has
+// Only tiles that the diagonal cuts are masked.  The sink and the gate are applied at the end, the gate's sigmoid from the hardware's
+// exponential and reciprocal (25 instructions per value otherwise, as much as ten tiles).
+#include "prompt_core.h"
 #include "prompt_tiles.h"
 #include "sink_attn.h"
 
@@ -35,9 +34,201 @@ __device__ __forceinline__ shortx4 sinkp_read_tr16(const unsigned short *p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((shortx4 __attribute__((address_space(3))) *)(p));
 }
 
+// The sink, the gate and the result of a wave's units.
+template <int VC, int CT>
+__device__ __forceinline__ void sink_finish(const SinkPrefillArgs &p, const floatx4 (&acc)[CT][2 * VC], const float (&m)[CT], const float (&l)[CT],
+                                            const bool (&uok)[CT], const int (&urow)[CT], const int (&uhead)[CT], int g) {
+  const SinkCache &c = p.c;
+  const bool vec = (c.Dv & 3) == 0 && (p.ldo & 3) == 0 && (p.ldg & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 &&
+                   (reinterpret_cast<uintptr_t>(p.gate) & 7) == 0;
+#pragma unroll
+  for (int k = 0; k < CT; ++k) {
+    const float den = sum_lanes_16_32_48(l[k]);
+    if (!uok[k]) continue;
+    const float sk = p.sink ? bf16_bits_to_float(p.sink[uhead[k]]) * kSinkLog2e : -INFINITY;
+    const float top = fmaxf(m[k], sk), f = __builtin_amdgcn_exp2f(m[k] - top);
+    const float inv = f / (den * f + __builtin_amdgcn_exp2f(sk - top));
+    unsigned short *o = p.out + static_cast<int64_t>(urow[k]) * p.ldo + static_cast<int64_t>(uhead[k]) * c.Dv;
+    const unsigned short *gp = p.gate + static_cast<int64_t>(urow[k]) * p.ldg + static_cast<int64_t>(uhead[k]) * c.Dv;
+#pragma unroll
+    for (int d = 0; d < 2 * VC; ++d) {
+      const int col = d * 16 + g * 4;
+      float gt[4] = {1.f, 1.f, 1.f, 1.f};
+      if (p.gate) {
+        if (vec && col < c.Dv) {
+          const uint2 b = *reinterpret_cast<const uint2 *>(gp + col);
+          gt[0] = __uint_as_float(b.x << 16); gt[1] = __uint_as_float(b.x & 0xffff0000u);
+          gt[2] = __uint_as_float(b.y << 16); gt[3] = __uint_as_float(b.y & 0xffff0000u);
+        } else if (!vec) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (col + r < c.Dv) gt[r] = bf16_bits_to_float(gp[col + r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) gt[r] = sigmoid_fast(gt[r]);
+      }
+      const uint2 v = make_uint2(pack_bf16x2(acc[k][d][0] * inv * gt[0], acc[k][d][1] * inv * gt[1]),
+                                 pack_bf16x2(acc[k][d][2] * inv * gt[2], acc[k][d][3] * inv * gt[3]));
+      if (vec) {
+        if (col < c.Dv) *reinterpret_cast<uint2 *>(o + col) = v;
+      } else {
+        const unsigned int e[2] = {v.x, v.y};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col + r < c.Dv) o[col + r] = static_cast<unsigned short>(e[r / 2] >> (16 * (r & 1)));
+      }
+    }
+  }
+}
+
 // MODE 0: no cap, 1: a cap, 2: a cap small enough to take the largest score it allows as everyone's maximum
+template <int DC, int VC, int MODE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void sink_prefill_kernel(const SinkPrefillArgs p) {
+  constexpr int CT = 2;
+  using Core = PromptCore<DC, VC, CT>;
+  __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
+  int sq, plane, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
+  const SinkCache &c = p.c;
+  const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
+  const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
+  const int row0 = xt * p.bq;
+  if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
+  const int32_t *bt = c.bt + seq * c.bt_stride;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int nh = min(p.hpp, p.group - pass * p.hpp);         // heads of this pass
+  const int last_row = min(row0 + p.bq, lq) - 1;
+  const int i_last = start + last_row;
+  Core core;
+  core.start(TLF_DL_LDSADDR(Ks), TLF_DL_LDSADDR(Vs), tid);
+  const int wave_first = start + row0 + core.wave * CT * 16 / p.hpp;
+
+  int upos[CT], urow[CT], uhead[CT];
+  bool uok[CT];
+#pragma unroll
+  for (int k = 0; k < CT; ++k) {
+    const int u = core.wave * CT * 16 + k * 16 + n;
+    const int r = row0 + u / p.hpp, hh = u % p.hpp;
+    uok[k] = u < p.bq * p.hpp && r <= last_row && hh < nh;
+    uhead[k] = kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0);
+    const int row = min(r, last_row);
+    upos[k] = start + row;
+    urow[k] = q0 + row;
+    const unsigned short *qp = p.q + (static_cast<int64_t>(urow[k]) * p.H + uhead[k]) * Core::DP + g * 8;
+#pragma unroll
+    for (int kc = 0; kc < DC; ++kc) {
+      Pack16 t;
+      t.u = *reinterpret_cast<const uint4 *>(qp + kc * 32);
+      core.qf[k][kc] = t.v;
+    }
+  }
+
+  const int tiles = i_last / kSK + 1;
+  unsigned int koff[DC], voff[VC];                           // this lane's pieces in a tile, which is one piece of a page
+#pragma unroll
+  for (int i = 0; i < DC; ++i) {
+    int row, piece;
+    core.k_piece(i, lane, row, piece);
+    koff[i] = (row * Core::KCH + piece) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < VC; ++i) {
+    int row, piece;
+    core.v_piece(i, lane, row, piece);
+    voff[i] = (row * (c.Vp / 8) + (piece < c.Vp / 8 ? piece : 0)) * 16;
+  }
+  // K of a tile is asked for first, its V a tile later from the row carried over; the page is looked up another tile ahead
+  auto page_of = [&](int t) __attribute__((always_inline)) { return bt[sink_page_of(c, min(t * kSK, i_last))]; };
+  int64_t row_k = 0;
+  int page_next = page_of(0);
+  auto copy_k = [&](int t) __attribute__((always_inline)) {  // rows past the last query are masked
+    row_k = sink_row(c, page_next, sink_page_of(c, t * kSK), kvh, t * kSK);
+    page_next = page_of(t + 1);
+    const unsigned char *kp = static_cast<const unsigned char *>(c.k) + row_k * (Core::DP * 2);
+#pragma unroll
+    for (int i = 0; i < DC; ++i) TLF_DL_COPY(koff[i], kp, core.k_place(t, i));
+  };
+  auto copy_v = [&](int t) __attribute__((always_inline)) {  // before the next copy_k: of the tile that was asked for last
+    const unsigned char *vp = static_cast<const unsigned char *>(c.v) + row_k * (c.Vp * 2);
+#pragma unroll
+    for (int i = 0; i < VC; ++i) TLF_DL_COPY(voff[i], vp, core.v_place(t, i));
+  };
+
+  float m[CT], l[CT];
+  float x[CT];                                               // this lane's largest score of the half that comes next,
+  float over[CT];                                            // and what it must not exceed
+#pragma unroll
+  for (int k = 0; k < CT; ++k) {
+    m[k] = MODE == 2 ? p.cap_log2 : -INFINITY;
+    l[k] = 0.f;
+    over[k] = -INFINITY;                                     // no key yet
+  }
+  core.template walk<false>(
+      tiles, 0, min(tiles, (wave_first + 1) / kSK), copy_k, copy_v,            // the diagonal cuts the tiles behind
+      [&](float (&f)[CT]) __attribute__((always_inline)) {   // without a cap: the score less the maximum so far
+#pragma unroll
+        for (int k = 0; k < CT; ++k) f[k] = MODE == 0 && m[k] != -INFINITY ? -m[k] : 0.f;
+      },
+      [&](int h, typename Core::Scores &s, auto mask) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            float v = s[j >> 2][k][j & 3];
+            if (MODE == 2) v = -2.f * p.cap_log2 * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(v));
+            if (MODE == 1) v = sink_score_log2<true>(v, p.cap_log2);
+            if (mask.value) v = h * 32 + g * 8 + j <= upos[k] ? v : -INFINITY;
+            s[j >> 2][k][j & 3] = v;
+          }
+          if (MODE != 2) {
+            x[k] = s[0][k][0];
+#pragma unroll
+            for (int j = 1; j < 8; ++j) x[k] = fmaxf(x[k], s[j >> 2][k][j & 3]);
+          }
+        }
+      },
+      [&](int h, typename Core::Scores &s, typename Core::Weights &w) __attribute__((always_inline)) {
+        if constexpr (MODE != 2) {
+          bool grown = false;
+#pragma unroll
+          for (int k = 0; k < CT; ++k) grown = grown || x[k] > over[k];
+          if (!__any(grown)) return;
+          if (h > 0) core.add_values(h - 1, w);
+#pragma unroll
+          for (int k = 0; k < CT; ++k) {                     // sums, accumulators and scores to the new maximum
+            const float most = max_lanes_16_32_48(x[k]), base = MODE == 0 && m[k] != -INFINITY ? m[k] : 0.f;
+            const bool up = most > over[k];
+            const float top = up ? base + most : m[k], back = up ? __builtin_amdgcn_exp2f(m[k] - top) : 1.f;
+            l[k] *= back;
+#pragma unroll
+            for (int d = 0; d < 2 * VC; ++d) core.acc[k][d] *= back;
+            if (MODE == 0 && up) {
+              s[0][k] -= floatx4{most, most, most, most};
+              s[1][k] -= floatx4{most, most, most, most};
+            }
+            m[k] = top;
+            over[k] = top == -INFINITY ? top : MODE == 0 ? 8.f : top + 8.f;
+          }
+        }
+      },
+      [&](int h, const typename Core::Scores &s, typename Core::Weights &w, auto mask) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {
+          const float ms = MODE == 1 && m[k] != -INFINITY ? m[k] : 0.f;
+          float e[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) e[j] = __builtin_amdgcn_exp2f(MODE == 1 ? s[j >> 2][k][j & 3] - ms : s[j >> 2][k][j & 3]);
+          l[k] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+          Core::split(k, e, w);
+        }
+      });
+  sink_finish<VC, CT>(p, core.acc, m, l, uok, urow, uhead, g);
+}
+
+// Heads beyond 128: the stages of a tile one after the other, a tile staged through registers, one in LDS at a time (two of these
+// dimensions would leave one workgroup per CU).
 template <int DC, int VC, int CT, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void sink_prefill_kernel(const SinkPrefillArgs p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void sink_prefill_wide_kernel(const SinkPrefillArgs p) {
   constexpr int DP = DC * 32, VP = VC * 32, KCH = DC * 4, VCH = VC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kSK][DP + 8], Vs[kSK][VP + 16];
   int sq, plane, xt;
@@ -199,10 +390,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           l[k] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
           unsigned int hi[4], lo[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            hi[j] = pack_bf16x2(e[2 * j], e[2 * j + 1]);
-            lo[j] = pack_bf16x2(e[2 * j] - __uint_as_float(hi[j] << 16), e[2 * j + 1] - __uint_as_float(hi[j] & 0xffff0000u));
-          }
+          for (int j = 0; j < 4; ++j) weight_pairs(e[2 * j], e[2 * j + 1], hi[j], lo[j]);
           ph[k] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
           pl[k] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
         }
@@ -227,46 +415,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
 
-  const bool vec = (c.Dv & 3) == 0 && (p.ldo & 3) == 0 && (p.ldg & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0 &&
-                   (reinterpret_cast<uintptr_t>(p.gate) & 7) == 0;
-#pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    const float den = sum_lanes_16_32_48(l[k]);
-    if (!uok[k]) continue;
-    const float sk = p.sink ? bf16_bits_to_float(p.sink[uhead[k]]) * kSinkLog2e : -INFINITY;
-    const float top = fmaxf(m[k], sk), f = __builtin_amdgcn_exp2f(m[k] - top);
-    const float inv = f / (den * f + __builtin_amdgcn_exp2f(sk - top));
-    unsigned short *o = p.out + static_cast<int64_t>(urow[k]) * p.ldo + static_cast<int64_t>(uhead[k]) * c.Dv;
-    const unsigned short *gp = p.gate + static_cast<int64_t>(urow[k]) * p.ldg + static_cast<int64_t>(uhead[k]) * c.Dv;
-#pragma unroll
-    for (int d = 0; d < 2 * VC; ++d) {
-      const int col = d * 16 + g * 4;
-      float gt[4] = {1.f, 1.f, 1.f, 1.f};
-      if (p.gate) {
-        if (vec && col < c.Dv) {
-          const uint2 b = *reinterpret_cast<const uint2 *>(gp + col);
-          gt[0] = __uint_as_float(b.x << 16); gt[1] = __uint_as_float(b.x & 0xffff0000u);
-          gt[2] = __uint_as_float(b.y << 16); gt[3] = __uint_as_float(b.y & 0xffff0000u);
-        } else if (!vec) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (col + r < c.Dv) gt[r] = bf16_bits_to_float(gp[col + r]);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) gt[r] = sigmoid_f32(gt[r]);
-      }
-      const uint2 v = make_uint2(pack_bf16x2(acc[k][d][0] * inv * gt[0], acc[k][d][1] * inv * gt[1]),
-                                 pack_bf16x2(acc[k][d][2] * inv * gt[2], acc[k][d][3] * inv * gt[3]));
-      if (vec) {
-        if (col < c.Dv) *reinterpret_cast<uint2 *>(o + col) = v;
-      } else {
-        const unsigned int e[2] = {v.x, v.y};
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col + r < c.Dv) o[col + r] = static_cast<unsigned short>(e[r / 2] >> (16 * (r & 1)));
-      }
-    }
-  }
+  sink_finish<VC, CT>(p, acc, m, l, uok, urow, uhead, g);
 }
 
 }  // namespace tlf
@@ -300,25 +449,32 @@ extern "C" int tlf_sink_attn_prefill(const void *q, const void *k_cache, const v
   const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, kv_heads * a.passes, num_seqs));
   if (!grid.x) return TLF_E_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define TLF_SP(DC, VC)                                                                                                        \
-  do {                                                                                                                        \
-    constexpr int kCT = (DC) <= 4 && (VC) <= 4 ? 2 : 1;                                                                       \
-    if (cap <= 0.f) TLF_LAUNCH((sink_prefill_kernel<DC, VC, kCT, 0>), grid, dim3(256), 0, s, a);                              \
-    else if (cap <= 32.f) TLF_LAUNCH((sink_prefill_kernel<DC, VC, kCT, 2>), grid, dim3(256), 0, s, a);                        \
-    else TLF_LAUNCH((sink_prefill_kernel<DC, VC, kCT, 1>), grid, dim3(256), 0, s, a);                                         \
+#define TLF_SP(...)                                                                     \
+  do {                                                                                  \
+    if (cap <= 0.f) TLF_LAUNCH((__VA_ARGS__, 0>), grid, dim3(256), 0, s, a);            \
+    else if (cap <= 32.f) TLF_LAUNCH((__VA_ARGS__, 2>), grid, dim3(256), 0, s, a);      \
+    else TLF_LAUNCH((__VA_ARGS__, 1>), grid, dim3(256), 0, s, a);                       \
   } while (0)
-#define TLF_SP_V(DC)                \
-  do {                              \
-    if (vc <= 1) TLF_SP(DC, 1);     \
-    else if (vc <= 2) TLF_SP(DC, 2); \
-    else if (vc <= 4) TLF_SP(DC, 4); \
-    else TLF_SP(DC, 8);             \
+#define TLF_SP_V(DC)                                                                    \
+  case DC:                                                                              \
+    if (vc <= 1) TLF_SP(sink_prefill_kernel<DC, 1);                                     \
+    else if (vc <= 2) TLF_SP(sink_prefill_kernel<DC, 2);                                \
+    else if (vc <= 4) TLF_SP(sink_prefill_kernel<DC, 4);                                \
+    else TLF_SP(sink_prefill_wide_kernel<DC, 8, 1);                                     \
+    break;
+#define TLF_SP_W(DC)                                                                    \
+  do {                                                                                  \
+    if (vc <= 1) TLF_SP(sink_prefill_wide_kernel<DC, 1, 1);                             \
+    else if (vc <= 2) TLF_SP(sink_prefill_wide_kernel<DC, 2, 1);                        \
+    else if (vc <= 4) TLF_SP(sink_prefill_wide_kernel<DC, 4, 1);                        \
+    else TLF_SP(sink_prefill_wide_kernel<DC, 8, 1);                                     \
   } while (0)
-  if (dc <= 1) TLF_SP_V(1);
-  else if (dc <= 2) TLF_SP_V(2);
-  else if (dc <= 4) TLF_SP_V(4);
-  else if (dc <= 6) TLF_SP_V(6);
-  else TLF_SP_V(8);
+  switch (dc) {
+    TLF_SP_V(1) TLF_SP_V(2) TLF_SP_V(3) TLF_SP_V(4)
+    case 5: case 6: TLF_SP_W(6); break;
+    default: TLF_SP_W(8); break;
+  }
+#undef TLF_SP_W
 #undef TLF_SP_V
 #undef TLF_SP
   return launch_status();
