@@ -3,13 +3,13 @@
 //
 // A workgroup owns one sequence, one KV head and a tile of query rows; the (row, head) pairs of the KV head's query
 // heads are flattened into 64 CT units, 16 CT per wave.  It walks the pooled rows its last query sees and then the
-// tokens from its first query's window on, 64 keys at a time (global -> registers one tile ahead -> LDS):
-//   S^T[key, unit] = K . Q^T       v_mfma_f32_16x16x32_bf16
-//   P = sigmoid(S * scale + bias)  fp32, masked on the tiles that a window's or the diagonal's edge cuts
-//   O^T[dim, unit] += V^T . P^T    the V^T operand by LDS transpose reads; P as a bf16 hi + lo pair (16 significant bits)
-// The weights are not normalised: no running maximum, no rescaling, no second pass.  K rows are permuted inside a
-// tile so that the accumulators of two 16-key sub-tiles are the 32-key B operand of the second product.
+// tokens from its first query's window on; the loop is prompt_core.h's:
+//   P = sigmoid(S * scale + bias)  fp32, masked on the pooled tiles and on those that a window's or the diagonal's edge cuts
+// The weights are not normalised: no maximum, no rescaling, no second pass.  Bound by the vector ALU: two quarter-rate operations
+// per score.  Eight prompts of 1061 to 2048 tokens, 32 heads of 128 on 8 KV heads, window 1024: layer 372 us with the stages of a tile
+// one after the other (and the staging registers, which the compiler had put in LDS), 299 so.
 #include "pooled_attn.h"
+#include "prompt_core.h"
 #include "prompt_tiles.h"
 
 namespace tlf {
@@ -38,7 +38,153 @@ __device__ __forceinline__ shortx4 pooled_read_tr16(const unsigned short *p) {
 }
 
 template <int DC, int CT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void pooled_prefill_kernel(const PooledPrefillArgs p) {
+__device__ __forceinline__ void pooled_finish(const PooledPrefillArgs &p, const floatx4 (&acc)[CT][2 * DC], const bool (&uok)[CT], const int (&uoff)[CT], int g) {
+  const PooledCache &c = p.c;
+  const bool vec = (c.D & 3) == 0 && (p.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
+#pragma unroll
+  for (int k = 0; k < CT; ++k) {
+    if (!uok[k]) continue;
+    const float gt = p.gate[uoff[k]];
+    const int row = uoff[k] / p.H, head = uoff[k] - row * p.H;
+    unsigned short *o = p.out + static_cast<int64_t>(row) * p.ldo + static_cast<int64_t>(head) * c.D;
+#pragma unroll
+    for (int d = 0; d < 2 * DC; ++d) {
+      const int col = d * 16 + g * 4;
+      const uint2 v = make_uint2(pack_bf16x2(acc[k][d][0] * gt, acc[k][d][1] * gt), pack_bf16x2(acc[k][d][2] * gt, acc[k][d][3] * gt));
+      if (vec) {
+        if (col < c.D) *reinterpret_cast<uint2 *>(o + col) = v;
+      } else {
+        const unsigned int e[2] = {v.x, v.y};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col + r < c.D) o[col + r] = static_cast<unsigned short>(e[r / 2] >> (16 * (r & 1)));
+      }
+    }
+  }
+}
+
+template <int DC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void pooled_prefill_kernel(const PooledPrefillArgs p) {
+  constexpr int CT = 2;
+  using Core = PromptCore<DC, DC, CT>;
+  __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
+  int sq, plane, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
+  const PooledCache &c = p.c;
+  const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
+  const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
+  const int row0 = xt * p.bq;
+  if (row0 >= lq) return;
+  const int32_t *bt = c.bt + seq * c.bt_stride;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int nh = min(p.hpp, p.group - pass * p.hpp);         // heads of this pass
+  const int last_row = min(row0 + p.bq, lq) - 1;
+  const int i_first = start + row0, i_last = start + last_row;
+
+  Core core;
+  core.start(TLF_DL_LDSADDR(Ks), TLF_DL_LDSADDR(Vs), tid);
+
+  int upos[CT], unb[CT], uoff[CT];
+  bool uok[CT];
+  float pb[CT];
+  #pragma unroll
+  for (int k = 0; k < CT; ++k) {
+    const int u = core.wave * CT * 16 + k * 16 + n;
+    const int r = row0 + u / p.hpp, hh = u % p.hpp;
+    uok[k] = u < p.bq * p.hpp && r <= last_row && hh < nh;
+    const int head = kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0);
+    const int row = uok[k] ? r : row0;
+    upos[k] = start + row;
+    unb[k] = pooled_visible(upos[k], c.size, c.pool);
+    uoff[k] = (q0 + row) * p.H + head;
+    pb[k] = -kLog2e * bf16_bits_to_float(p.bias[head]);
+    const unsigned short *qp = p.q + static_cast<int64_t>(uoff[k]) * Core::DP + g * 8;
+#pragma unroll
+    for (int kc = 0; kc < DC; ++kc) {
+      Pack16 t;
+      t.u = *reinterpret_cast<const uint4 *>(qp + kc * 32);
+      core.qf[k][kc] = t.v;
+    }
+  }
+  const float nscale = -p.scale_log2;
+
+  const int nb = pooled_visible(i_last, c.size, c.pool), nb_first = pooled_visible(i_first, c.size, c.pool);
+  const int ptiles = (nb + kTK - 1) / kTK;
+  const int w0 = max(0, i_first - c.size + 1) / kTK * kTK;
+  const int tiles = ptiles + (i_last - w0) / kTK + 1;
+  const int64_t rs = static_cast<int64_t>(c.G) * Core::DP;
+  const unsigned short *kc_ = static_cast<const unsigned short *>(c.k) + kvh * Core::DP;
+  const unsigned short *vc_ = static_cast<const unsigned short *>(c.v) + kvh * Core::DP;
+  const unsigned short *pk_ = static_cast<const unsigned short *>(c.pk) + kvh * Core::DP;
+  const unsigned short *pv_ = static_cast<const unsigned short *>(c.pv) + kvh * Core::DP;
+
+  unsigned int koff[DC], voff[DC];                           // this lane's pieces in a tile of tokens
+#pragma unroll
+  for (int i = 0; i < DC; ++i) {
+    int row, piece;
+    core.k_piece(i, lane, row, piece);
+    koff[i] = static_cast<unsigned int>(row * static_cast<int>(rs) * 2 + piece * 16);
+    core.v_piece(i, lane, row, piece);
+    voff[i] = static_cast<unsigned int>(row * static_cast<int>(rs) * 2 + piece * 16);
+  }
+  auto copy_k = [&](int t, auto part) __attribute__((always_inline)) {
+    if (part.lead && t < ptiles) {                           // rows of one page's blocks, then the next page's
+#pragma unroll
+      for (int i = 0; i < DC; ++i) {
+        int row, piece;
+        core.k_piece(i, lane, row, piece);
+        prompt_copy_at(pk_ + block_row(c, bt, min(t * kTK + row, nb - 1)) * rs + piece * 8, core.k_place(t, i));
+      }
+      return;
+    }
+    // 64 tokens from a multiple of 64 on lie in one page; rows past the last query are masked
+    const unsigned short *base = kc_ + token_row(c, bt, w0 + (t - ptiles) * kTK) * rs;
+#pragma unroll
+    for (int i = 0; i < DC; ++i) prompt_copy(koff[i], base, core.k_place(t, i));
+  };
+  auto copy_v = [&](int t, auto part) __attribute__((always_inline)) {
+    if (part.lead && t < ptiles) {
+#pragma unroll
+      for (int i = 0; i < DC; ++i) {
+        int row, piece;
+        core.v_piece(i, lane, row, piece);
+        prompt_copy_at(pv_ + block_row(c, bt, min(t * kTK + row, nb - 1)) * rs + piece * 8, core.v_place(t, i));
+      }
+      return;
+    }
+    const unsigned short *base = vc_ + token_row(c, bt, w0 + (t - ptiles) * kTK) * rs;
+#pragma unroll
+    for (int i = 0; i < DC; ++i) prompt_copy(voff[i], base, core.v_place(t, i));
+  };
+  // tiles between the window's edge and the diagonal hide nothing from anyone
+  const int edge = i_last - c.size >= w0 ? (i_last - c.size - w0) / kTK + 1 : 0;
+  core.template walk<true>(
+      tiles, ptiles + edge, min(tiles, ptiles + max(0, (i_first + 1 - w0) / kTK)),
+      copy_k, copy_v,
+      [](float (&f)[CT]) __attribute__((always_inline)) { f[0] = f[1] = 0.f; }, [](int, typename Core::Scores &, auto) __attribute__((always_inline)) {},
+      [](int, typename Core::Scores &, typename Core::Weights &) __attribute__((always_inline)) {},
+      [&](int h, const typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {
+          float e[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) e[j] = sigmoid_neg_log2(fmaf(s[j >> 2][k][j & 3], nscale, pb[k]));
+          if (part.mask) {
+            const bool pooled = part.lead && h / 2 < ptiles;  // workgroup uniform
+            const int key = h * 32 + (pooled ? 0 : w0 - ptiles * kTK) + g * 8;
+            const int lo = pooled ? 0 : upos[k] - c.size + 1, hi = pooled ? unb[k] : upos[k] + 1;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) e[j] = key + j >= lo && key + j < hi ? e[j] : 0.f;
+          }
+          Core::split(k, e, w);
+        }
+      });
+  pooled_finish<DC, CT>(p, core.acc, uok, uoff, g);
+}
+
+// Heads beyond 128: the stages of a tile one after the other, staged through registers, one tile in LDS at a time.
+template <int DC, int CT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void pooled_prefill_wide_kernel(const PooledPrefillArgs p) {
   constexpr int DP = DC * 32, NCH = DC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kTK][DP + 8], Vs[kTK][DP + 16];
   int sq, plane, xt;
@@ -90,6 +236,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const unsigned short *pv_ = static_cast<const unsigned short *>(c.pv) + kvh * DP;
 
   uint4 kreg[DC], vreg[DC];
+#pragma unroll
+  for (int i = 0; i < DC; ++i) kreg[i] = vreg[i] = make_uint4(0, 0, 0, 0);   // keeps the arrays in registers: without it the compiler puts them in LDS
   auto load_tile = [&](int t) __attribute__((always_inline)) {
     if (t < ptiles) {
 #pragma unroll
@@ -167,10 +315,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         unsigned int h[4], l[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          h[j] = pack_bf16x2(w[2 * j], w[2 * j + 1]);
-          l[j] = pack_bf16x2(w[2 * j] - __uint_as_float(h[j] << 16), w[2 * j + 1] - __uint_as_float(h[j] & 0xffff0000u));
-        }
+        for (int j = 0; j < 4; ++j) weight_pairs(w[2 * j], w[2 * j + 1], h[j], l[j]);
         ph[k] = make_uint4(h[0], h[1], h[2], h[3]);
         pl[k] = make_uint4(l[0], l[1], l[2], l[3]);
       }
@@ -195,27 +340,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
 
-  const bool vec = (c.D & 3) == 0 && (p.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
-#pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    if (!uok[k]) continue;
-    const float gt = p.gate[uoff[k]];
-    const int row = uoff[k] / p.H, head = uoff[k] - row * p.H;
-    unsigned short *o = p.out + static_cast<int64_t>(row) * p.ldo + static_cast<int64_t>(head) * c.D;
-#pragma unroll
-    for (int d = 0; d < 2 * DC; ++d) {
-      const int col = d * 16 + g * 4;
-      const uint2 v = make_uint2(pack_bf16x2(acc[k][d][0] * gt, acc[k][d][1] * gt), pack_bf16x2(acc[k][d][2] * gt, acc[k][d][3] * gt));
-      if (vec) {
-        if (col < c.D) *reinterpret_cast<uint2 *>(o + col) = v;
-      } else {
-        const unsigned int e[2] = {v.x, v.y};
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col + r < c.D) o[col + r] = static_cast<unsigned short>(e[r / 2] >> (16 * (r & 1)));
-      }
-    }
-  }
+  pooled_finish<DC, CT>(p, acc, uok, uoff, g);
 }
 
 }  // namespace tlf
@@ -249,14 +374,14 @@ extern "C" int tlf_pooled_attn_prefill(const void *q, const void *score_bias, co
   if (!grid.x) return TLF_E_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dc) {
-    case 1: TLF_LAUNCH((pooled_prefill_kernel<1, 2>), grid, dim3(256), 0, s, a); break;
-    case 2: TLF_LAUNCH((pooled_prefill_kernel<2, 2>), grid, dim3(256), 0, s, a); break;
-    case 3: TLF_LAUNCH((pooled_prefill_kernel<3, 2>), grid, dim3(256), 0, s, a); break;
-    case 4: TLF_LAUNCH((pooled_prefill_kernel<4, 2>), grid, dim3(256), 0, s, a); break;
-    case 5: TLF_LAUNCH((pooled_prefill_kernel<5, 1>), grid, dim3(256), 0, s, a); break;
-    case 6: TLF_LAUNCH((pooled_prefill_kernel<6, 1>), grid, dim3(256), 0, s, a); break;
-    case 7: TLF_LAUNCH((pooled_prefill_kernel<7, 1>), grid, dim3(256), 0, s, a); break;
-    default: TLF_LAUNCH((pooled_prefill_kernel<8, 1>), grid, dim3(256), 0, s, a); break;
+    case 1: TLF_LAUNCH((pooled_prefill_kernel<1>), grid, dim3(256), 0, s, a); break;
+    case 2: TLF_LAUNCH((pooled_prefill_kernel<2>), grid, dim3(256), 0, s, a); break;
+    case 3: TLF_LAUNCH((pooled_prefill_kernel<3>), grid, dim3(256), 0, s, a); break;
+    case 4: TLF_LAUNCH((pooled_prefill_kernel<4>), grid, dim3(256), 0, s, a); break;
+    case 5: TLF_LAUNCH((pooled_prefill_wide_kernel<5, 1>), grid, dim3(256), 0, s, a); break;
+    case 6: TLF_LAUNCH((pooled_prefill_wide_kernel<6, 1>), grid, dim3(256), 0, s, a); break;
+    case 7: TLF_LAUNCH((pooled_prefill_wide_kernel<7, 1>), grid, dim3(256), 0, s, a); break;
+    default: TLF_LAUNCH((pooled_prefill_wide_kernel<8, 1>), grid, dim3(256), 0, s, a); break;
   }
   return launch_status();
 }

@@ -17,8 +17,6 @@
 // Measured and not taken: eight waves per workgroup (8 % slower), LDS reads of a whole step ahead of its products (4 %
 // slower), wave priorities around the products (no difference).
 #pragma once
-#include <type_traits>
-
 #include "gemm_shared.h"
 
 namespace tlf {
@@ -33,14 +31,23 @@ __device__ __forceinline__ T prompt_lds(unsigned int at) {
 __device__ __forceinline__ uint2 prompt_lds_tr16(unsigned int at) {
   return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<shortx4 __attribute__((address_space(3))) *>(at)));
 }
-// The same copy as TLF_DL_COPY from a 64-bit address per lane.
-#define TLF_DL_COPY_AT(ADDR, LDS) \
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(ADDR), "s"(LDS) : "memory")
+// 16 bytes per lane into LDS at a wave's address: from a uniform base and an offset per lane, or from an address per lane.
+__device__ __forceinline__ void prompt_copy(unsigned int offset, const void *base, unsigned int lds) { TLF_DL_COPY(offset, base, lds); }
+__device__ __forceinline__ void prompt_copy_at(const void *from, unsigned int lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds) : "memory");
+}
 
 // DC, VC: key and value dimensions in units of 32.  LDS holds two tiles of K and two of V, rows unpadded; the 16-byte pieces of a K row
 // are swapped with its neighbours in groups of 4 or 8 and pairs of pieces of a V row permuted by the row, against bank conflicts.
+template <bool LEAD, bool MASK>
+struct PromptPart {
+  static constexpr bool lead = LEAD, mask = MASK;
+};
+
 template <int DC, int VC, int CT>
 struct PromptCore {
+  template <bool LEAD, bool MASK>
+  using Part = PromptPart<LEAD, MASK>;
   static constexpr int DP = DC * 32, VP = VC * 32, KCH = DC * 4, VCH = VC * 4, KX = KCH % 8 == 0 ? 7 : 3;
   static constexpr int KB = kPromptKeys * DP * 2, VB = kPromptKeys * VP * 2;        // bytes of a tile
   typedef floatx4 Scores[2][CT];      // of a half: [16 keys][16 units]; lane (n, g): keys g * 8 + 4 s + r of unit n
@@ -93,7 +100,8 @@ struct PromptCore {
     const unsigned int at = vat + (h >> 1 & 1) * VB + (h & 1) * (32 * VP * 2);
 #pragma unroll
     for (int d = 0; d < 2 * VC; ++d) {
-      const uint2 v0 = prompt_lds_tr16(at ^ (d * 32)), v1 = prompt_lds_tr16((at ^ (d * 32)) + 8 * VP);
+      const unsigned int to = VC == 3 ? (at ^ ((d & 1) * 32)) + d / 2 * 64 : at ^ (d * 32);   // rows of 192 bytes swap neighbours only
+      const uint2 v0 = prompt_lds_tr16(to), v1 = prompt_lds_tr16(to + 8 * VP);
       vf[d] = __builtin_bit_cast(bf16x8, make_uint4(v0.x, v0.y, v1.x, v1.y));
     }
   }
@@ -126,17 +134,19 @@ struct PromptCore {
   }
 
   // The walk over `tiles` tiles.  The kernel's parts:
-  //   copy_k(t), copy_v(t)        the tile's copies; called for t = 0, 1, .. in turn
+  //   copy_k(t, part), copy_v     the tile's copies; called for t = 0, 1, .. in turn
   //   from(f)                     where a unit's scores begin (read once per half)
-  //   finish(h, s, mask)          what is done to the scores of half h as soon as they are there
+  //   finish(h, s, part)          what is done to the scores of half h as soon as they are there
   //   before(h, s, w)             ahead of the weights of half h; `w`: weights of half h - 1 whose values are not added yet (add_values)
-  //   weights(h, s, w, mask)
-  // `mask` is not set where all keys of the half's tile are seen by all units: tiles clear_from <= t < clear_to of them (wave uniform),
-  // clear_from 0 without LEAD.
+  //   weights(h, s, w, part)
+  // part.mask is not set where all keys of the half's tile are seen by all units: tiles clear_from <= t < clear_to of them (wave
+  // uniform), clear_from 0 without LEAD.  part.lead is set where t may be below clear_from.
   template <bool LEAD, class CopyK, class CopyV, class From, class Finish, class Before, class Weigh>
   __device__ __forceinline__ void walk(int tiles, int clear_from, int clear_to, CopyK copy_k, CopyV copy_v, From from, Finish finish, Before before, Weigh weights) {
-    constexpr std::integral_constant<bool, true> masked{};
-    constexpr std::integral_constant<bool, false> plain{};
+    constexpr Part<true, true> lead{};
+    constexpr Part<false, false> plain{};
+    constexpr Part<false, true> tail{};
+    constexpr Part<LEAD, true> first{};
     Scores se, so;                    // of even and odd halves
     Weights we{}, wo{};
     auto make_scores = [&](Scores &s) __attribute__((always_inline)) {
@@ -144,47 +154,47 @@ struct PromptCore {
       from(f);
       scores(f, s);
     };
-    copy_k(0);
+    copy_k(0, first);
     TLF_DL_BARRIER(0);
-    copy_v(0);
-    if (tiles > 1) copy_k(1);
+    copy_v(0, first);
+    if (tiles > 1) copy_k(1, first);
     read_k(0);
     make_scores(se);
-    finish(0, se, masked);
+    finish(0, se, first);
     before(0, se, wo);
     read_k(1);
     make_scores(so);
-    weights(0, se, we, masked);
-    finish(1, so, masked);
+    weights(0, se, we, first);
+    finish(1, so, first);
     // scores of 2 t + 2 and 2 t + 3, weights of 2 t + 1 and 2 t + 2, values of 2 t and 2 t + 1
-    auto two_steps = [&](int t, auto mask) __attribute__((always_inline)) {
+    auto two_steps = [&](int t, auto part) __attribute__((always_inline)) {
       TLF_DL_BARRIER(0);              // K of tile t + 1 and V of tile t are there; the buffers of K t and V t - 1 are free
-      copy_v(t + 1);
-      if (t + 2 < tiles) copy_k(t + 2);
+      copy_v(t + 1, part);
+      if (t + 2 < tiles) copy_k(t + 2, part);
       before(2 * t + 1, so, we);
       read_k(2 * t + 2);
       read_v(2 * t);
       make_scores(se);
-      weights(2 * t + 1, so, wo, mask);
+      weights(2 * t + 1, so, wo, part);
       values(we);
-      finish(2 * t + 2, se, mask);
+      finish(2 * t + 2, se, part);
       before(2 * t + 2, se, wo);
       read_k(2 * t + 3);
       read_v(2 * t + 1);
       make_scores(so);
-      weights(2 * t + 2, se, we, mask);
+      weights(2 * t + 2, se, we, part);
       values(wo);
-      finish(2 * t + 3, so, mask);
+      finish(2 * t + 3, so, part);
     };
     // loops of their own: as a choice inside one loop the two forms do not fit the registers
     int t = 0;
     if constexpr (LEAD)
-      for (; t + 1 < tiles && t < clear_from; ++t) two_steps(t, masked);
+      for (; t + 1 < tiles && t < clear_from; ++t) two_steps(t, lead);
     for (; t + 1 < clear_to; ++t) two_steps(t, plain);
-    for (; t + 1 < tiles; ++t) two_steps(t, masked);
+    for (; t + 1 < tiles; ++t) two_steps(t, tail);
     TLF_DL_BARRIER(0);
     before(2 * tiles - 1, so, we);
-    weights(2 * tiles - 1, so, wo, masked);
+    weights(2 * tiles - 1, so, wo, first);
     read_v(2 * tiles - 2);
     values(we);
     read_v(2 * tiles - 1);

@@ -141,17 +141,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   auto page_of = [&](int t) __attribute__((always_inline)) { return bt[sink_page_of(c, min(t * kSK, i_last))]; };
   int64_t row_k = 0;
   int page_next = page_of(0);
-  auto copy_k = [&](int t) __attribute__((always_inline)) {  // rows past the last query are masked
+  auto copy_k = [&](int t, auto) __attribute__((always_inline)) {  // rows past the last query are masked
     row_k = sink_row(c, page_next, sink_page_of(c, t * kSK), kvh, t * kSK);
     page_next = page_of(t + 1);
     const unsigned char *kp = static_cast<const unsigned char *>(c.k) + row_k * (Core::DP * 2);
 #pragma unroll
-    for (int i = 0; i < DC; ++i) TLF_DL_COPY(koff[i], kp, core.k_place(t, i));
+    for (int i = 0; i < DC; ++i) prompt_copy(koff[i], kp, core.k_place(t, i));
   };
-  auto copy_v = [&](int t) __attribute__((always_inline)) {  // before the next copy_k: of the tile that was asked for last
+  auto copy_v = [&](int t, auto) __attribute__((always_inline)) {  // before the next copy_k: of the tile that was asked for last
     const unsigned char *vp = static_cast<const unsigned char *>(c.v) + row_k * (c.Vp * 2);
 #pragma unroll
-    for (int i = 0; i < VC; ++i) TLF_DL_COPY(voff[i], vp, core.v_place(t, i));
+    for (int i = 0; i < VC; ++i) prompt_copy(voff[i], vp, core.v_place(t, i));
   };
 
   float m[CT], l[CT];
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
 #pragma unroll
         for (int k = 0; k < CT; ++k) f[k] = MODE == 0 && m[k] != -INFINITY ? -m[k] : 0.f;
       },
-      [&](int h, typename Core::Scores &s, auto mask) __attribute__((always_inline)) {
+      [&](int h, typename Core::Scores &s, auto part) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < CT; ++k) {
 #pragma unroll
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
             float v = s[j >> 2][k][j & 3];
             if (MODE == 2) v = -2.f * p.cap_log2 * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(v));
             if (MODE == 1) v = sink_score_log2<true>(v, p.cap_log2);
-            if (mask.value) v = h * 32 + g * 8 + j <= upos[k] ? v : -INFINITY;
+            if (part.mask) v = h * 32 + g * 8 + j <= upos[k] ? v : -INFINITY;
             s[j >> 2][k][j & 3] = v;
           }
           if (MODE != 2) {
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
           }
         }
       },
-      [&](int h, const typename Core::Scores &s, typename Core::Weights &w, auto mask) __attribute__((always_inline)) {
+      [&](int h, const typename Core::Scores &s, typename Core::Weights &w, auto) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < CT; ++k) {
           const float ms = MODE == 1 && m[k] != -INFINITY ? m[k] : 0.f;
