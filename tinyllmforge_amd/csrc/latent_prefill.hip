@@ -2,20 +2,20 @@
 // latent_attn.h): row r of `expanded` holds the keys' own parts of all heads and then the values, the rotated key part
 // shared by the heads is read from the gathered cache rows.
 //
-// A workgroup owns one portion, one head and 128 query rows, 32 per wave, and walks the keys its window covers 64 at a time
-// (global -> registers one tile ahead -> LDS):
-//   S^T[key, row] = K . Q^T       v_mfma_f32_16x16x32_bf16
+// A workgroup owns one portion, one head and 64 CT query rows, 16 CT per wave, and walks the keys its window covers; the loop is
+// prompt_core.h's:
 //   P = 2^(S * scale - m)         fp32; m follows a row's maximum only when that has grown by more than 8 (a factor of 256,
-//                                 which the fp32 sums and the bf16 pair hold), so the accumulators are rarely rescaled
-//   O^T[dim, row] += V^T . P^T    V^T by LDS transpose reads; P as a bf16 hi + lo pair (16 significant bits)
-// K rows are permuted inside a tile so that the accumulators of two 16-key sub-tiles are the 32-key B operand of the second
-// product.
+//                                 which the fp32 sums and the bf16 pair hold), so the accumulators are rarely rescaled.  Whether any
+//                                 has grown is asked lane by lane; maxima of rows are only formed when one has
+// 16 heads of 96 and 64 dimensions, eight prompts of 1061 to 2048 tokens: layer 189 us with the stages of a tile one after the other and
+// a window of 1024, 173 so; three prompts up to 3000, causal, 208 and 185.
 #include "latent_attn.h"
+#include "prompt_core.h"
 #include "prompt_tiles.h"
 
 namespace tlf {
 
-constexpr int kPK = 64, kPQ = 128;   // keys per tile, query rows per workgroup
+constexpr int kPK = kPromptKeys;      // keys per tile
 
 struct LatentPrefillArgs {
   LatentShape s;
@@ -28,18 +28,193 @@ struct LatentPrefillArgs {
   int64_t lde, ldo;
   PromptTiles tiles;
   int32_t first_seq, window;
-  float scale_log2;
+  float scale_log2;                 // positive; the sign (or zero) of the scale goes into q
+  unsigned int q_keep, q_flip;
 };
+
+template <int VC, int CT>
+__device__ __forceinline__ void latent_finish(const LatentPrefillArgs &p, const floatx4 (&acc)[CT][2 * VC], const float (&l)[CT], const bool (&uok)[CT],
+                                              const int (&upos)[CT], int q0, int start, int h, int g) {
+  const LatentShape &s = p.s;
+  const bool vec = (s.vdim & 3) == 0 && (p.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
+#pragma unroll
+  for (int k = 0; k < CT; ++k) {
+    const float den = sum_lanes_16_32_48(l[k]);
+    if (!uok[k]) continue;
+    float inv = 1.0f / den;                                  // a row sees itself: den > 0
+    if (p.gate) inv *= p.gate[static_cast<int64_t>(q0 + upos[k] - start) * s.H + h];
+    unsigned short *o = p.out + static_cast<int64_t>(q0 + upos[k] - start) * p.ldo + static_cast<int64_t>(h) * s.vdim;
+#pragma unroll
+    for (int d = 0; d < 2 * VC; ++d) {
+      const int col = d * 16 + g * 4;
+      const uint2 v = make_uint2(pack_bf16x2(acc[k][d][0] * inv, acc[k][d][1] * inv), pack_bf16x2(acc[k][d][2] * inv, acc[k][d][3] * inv));
+      if (vec) {
+        if (col < s.vdim) *reinterpret_cast<uint2 *>(o + col) = v;
+      } else {
+        const unsigned int e[2] = {v.x, v.y};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col + r < s.vdim) o[col + r] = static_cast<unsigned short>(e[r / 2] >> (16 * (r & 1)));
+      }
+    }
+  }
+}
+
+// DC, VC: query / key and value dimensions in units of 32 (rounded up to what is instantiated)
+template <int DC, int VC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void latent_prefill_kernel(const LatentPrefillArgs p) {
+  constexpr int CT = 2;
+  using Core = PromptCore<DC, VC, CT>;
+  __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
+  int sq, h, xt;
+  if (!prompt_tile(p.tiles, blockIdx.x, sq, h, xt)) return;
+  const LatentShape &s = p.s;
+  const int seq = p.first_seq + sq;
+  const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
+  const int row0 = xt * 64 * CT;
+  if (row0 >= lq) return;
+  const int kv0 = p.kv_off[sq], kv_n = p.kv_off[sq + 1] - kv0;
+  const int kbase = max(0, start - p.window + 1);            // position of the portion's first dense row
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int last_row = min(row0 + 64 * CT, lq) - 1;
+  const int i_first = start + row0, i_last = start + last_row;
+  Core core;
+  core.start(TLF_DL_LDSADDR(Ks), TLF_DL_LDSADDR(Vs), tid);
+  const int wave_first = i_first + core.wave * 16 * CT, wave_last = min(wave_first + 16 * CT - 1, i_last);
+
+  int upos[CT];
+  bool uok[CT];
+#pragma unroll
+  for (int k = 0; k < CT; ++k) {
+    const int r = row0 + core.wave * 16 * CT + k * 16 + n;
+    uok[k] = r <= last_row;
+    const int row = uok[k] ? r : last_row;
+    upos[k] = start + row;
+    const unsigned short *qp = p.q + (static_cast<int64_t>(q0 + row) * s.H + h) * s.Dq + g * 8;
+#pragma unroll
+    for (int kc = 0; kc < DC; ++kc) {
+      Pack16 t;
+      t.u = kc * 32 < s.Dq ? *reinterpret_cast<const uint4 *>(qp + kc * 32) : make_uint4(0, 0, 0, 0);
+      t.u = make_uint4((t.u.x & p.q_keep) ^ p.q_flip, (t.u.y & p.q_keep) ^ p.q_flip, (t.u.z & p.q_keep) ^ p.q_flip, (t.u.w & p.q_keep) ^ p.q_flip);
+      core.qf[k][kc] = t.v;
+    }
+  }
+
+  // This lane's pieces of a tile's rows: their places in the row 0 of the portion's dense rows, their rows in the tile.  A piece of K
+  // is of the own part or of the rotated one; the pads of a row meet zeros of the queries and repeat its first piece.
+  const unsigned char *kat[DC];
+  int krow[DC], vrow[VC];
+  unsigned int kstep[DC], vat[VC];
+  const unsigned short *own = p.expanded + static_cast<int64_t>(kv0) * p.lde, *turned = p.latents + static_cast<int64_t>(kv0) * s.Lp + s.Ra - s.Da;
+  const unsigned int ostep = static_cast<unsigned int>(p.lde * 2), tstep = static_cast<unsigned int>(s.Lp * 2);
+#pragma unroll
+  for (int i = 0; i < DC; ++i) {
+    int piece;
+    core.k_piece(i, lane, krow[i], piece);
+    const int d = piece * 8 < s.Da + s.Ta ? piece * 8 : 0;
+    kat[i] = reinterpret_cast<const unsigned char *>(d < s.Da ? own + h * s.Da + d : turned + d);
+    kstep[i] = d < s.Da ? ostep : tstep;
+  }
+#pragma unroll
+  for (int i = 0; i < VC; ++i) {
+    int piece;
+    core.v_piece(i, lane, vrow[i], piece);
+    vat[i] = piece * 8 < s.Va ? piece * 16 : 0;
+  }
+  const int w0 = max(0, i_first - p.window + 1);             // >= kbase
+  const int tiles = (i_last - w0) / kPK + 1;
+  auto copy_k = [&](int t, auto) __attribute__((always_inline)) {
+    const int r0 = w0 - kbase + t * kPK;
+#pragma unroll
+    for (int i = 0; i < DC; ++i)
+      prompt_copy_at(kat[i] + static_cast<uint64_t>(kstep[i]) * static_cast<unsigned int>(min(r0 + krow[i], kv_n - 1)), core.k_place(t, i));
+  };
+  auto copy_v = [&](int t, auto) __attribute__((always_inline)) {
+    const int r0 = w0 - kbase + t * kPK;                     // its own row is below kv_n
+    const unsigned short *base = own + static_cast<int64_t>(r0) * p.lde + s.H * s.Da + h * s.Va;
+#pragma unroll
+    for (int i = 0; i < VC; ++i)
+      prompt_copy(ostep * static_cast<unsigned int>(min(vrow[i], kv_n - 1 - r0)) + vat[i], base, core.v_place(t, i));
+  };
+
+  float m[CT], l[CT];
+  float x[CT];                                               // this lane's largest score of the half that comes next,
+  float over[CT];                                            // and what it must not exceed
+#pragma unroll
+  for (int k = 0; k < CT; ++k) {
+    m[k] = over[k] = -INFINITY;                              // no key yet
+    l[k] = 0.f;
+  }
+  // tiles between the window's edge and the diagonal hide nothing from any of the wave's rows
+  const int edge = wave_last - p.window >= w0 ? (wave_last - p.window - w0) / kPK + 1 : 0;
+  core.template walk<true, true>(
+      tiles, edge, min(tiles, max(0, (wave_first + 1 - w0) / kPK)), copy_k, copy_v,
+      [](float (&f)[CT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < CT; ++k) f[k] = 0.f;
+      },
+      [&](int hf, typename Core::Scores &sc, auto part) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {
+          if (part.mask) {
+            const int key = w0 + hf * 32 + g * 8;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const bool seen = key + j <= upos[k] && (!part.lead || key + j > upos[k] - p.window);
+              sc[j >> 2][k][j & 3] = seen ? sc[j >> 2][k][j & 3] : -INFINITY;
+            }
+          }
+          float y = sc[0][k][0];
+#pragma unroll
+          for (int j = 1; j < 8; ++j) y = fmaxf(y, sc[j >> 2][k][j & 3]);
+          y *= p.scale_log2;
+          x[k] = part.start && hf == 1 ? fmaxf(x[k], y) : y;     // the first maximum is that of the whole first tile
+        }
+      },
+      [&](int hf, typename Core::Scores &, typename Core::Weights &w) __attribute__((always_inline)) {
+        bool grown = false;
+#pragma unroll
+        for (int k = 0; k < CT; ++k) grown = grown || x[k] > over[k];
+        if (!__any(grown)) return;
+        if (hf > 0) core.add_values(hf - 1, w);
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {                       // sums and accumulators to the new maximum
+          const float most = max_lanes_16_32_48(x[k]);
+          const bool up = most > over[k];
+          const float back = up ? __builtin_amdgcn_exp2f(m[k] - most) : 1.f;
+          m[k] = up ? most : m[k];
+          over[k] = m[k] + 8.f;
+          l[k] *= back;
+#pragma unroll
+          for (int d = 0; d < 2 * VC; ++d) core.acc[k][d] *= back;
+        }
+      },
+      [&](int hf, const typename Core::Scores &sc, typename Core::Weights &w, auto) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {
+          const float ms = m[k] == -INFINITY ? 0.f : m[k];
+          float e[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) e[j] = __builtin_amdgcn_exp2f(sc[j >> 2][k][j & 3] * p.scale_log2 - ms);
+          l[k] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+          Core::split(k, e, w);
+        }
+      });
+
+  latent_finish<VC, CT>(p, core.acc, l, uok, upos, q0, start, h, g);
+}
 
 __device__ __forceinline__ int prefill_tile_row(int t) { return (t & 32) | ((t & 4) << 2) | ((t & 24) >> 1) | (t & 3); }
 __device__ __forceinline__ shortx4 prefill_read_tr16(const unsigned short *p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((shortx4 __attribute__((address_space(3))) *)(p));
 }
 
-// DC, VC: query / key and value dimensions in units of 32 (rounded up to what is instantiated)
+// Queries beyond 128: the stages of a tile one after the other, a tile staged through registers, one in LDS at a time.  The shared loop
+// does not fit the registers with two units per lane, and with one the reads of K and V out of LDS bound it (192 and 128 dimensions,
+// 32 heads, eight prompts of 1061 to 2048 tokens: layer 585 us, 687 with the shared loop and spills, 615 with one unit per lane).
 template <int DC, int VC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_prefill_kernel(const LatentPrefillArgs p) {
-  constexpr int CT = 2, DP = DC * 32, VP = VC * 32;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_prefill_wide_kernel(const LatentPrefillArgs p) {
+  constexpr int CT = 2, kPQ = 64 * CT, DP = DC * 32, VP = VC * 32;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kPK][DP + 8], Vs[kPK][VP + 16];
   int sq, h, xt;
   if (!prompt_tile(p.tiles, blockIdx.x, sq, h, xt)) return;
@@ -69,6 +244,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int kc = 0; kc < DC; ++kc) {
       Pack16 t;
       t.u = kc * 32 < s.Dq ? *reinterpret_cast<const uint4 *>(qp + kc * 32) : make_uint4(0, 0, 0, 0);
+      t.u = make_uint4((t.u.x & p.q_keep) ^ p.q_flip, (t.u.y & p.q_keep) ^ p.q_flip, (t.u.z & p.q_keep) ^ p.q_flip, (t.u.w & p.q_keep) ^ p.q_flip);
       qf[k][kc] = t.v;
     }
   }
@@ -184,10 +360,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           l[k] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
           unsigned int hi[4], lo[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            hi[j] = pack_bf16x2(e[2 * j], e[2 * j + 1]);
-            lo[j] = pack_bf16x2(e[2 * j] - __uint_as_float(hi[j] << 16), e[2 * j + 1] - __uint_as_float(hi[j] & 0xffff0000u));
-          }
+          for (int j = 0; j < 4; ++j) weight_pairs(e[2 * j], e[2 * j + 1], hi[j], lo[j]);
           ph[k] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
           pl[k] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
         }
@@ -212,28 +385,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
 
-  const bool vec = (s.vdim & 3) == 0 && (p.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
-#pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    const float den = sum_lanes_16_32_48(l[k]);
-    if (!uok[k]) continue;
-    float inv = 1.0f / den;                                  // a row sees itself: den > 0
-    if (p.gate) inv *= p.gate[static_cast<int64_t>(q0 + upos[k] - start) * s.H + h];
-    unsigned short *o = p.out + static_cast<int64_t>(q0 + upos[k] - start) * p.ldo + static_cast<int64_t>(h) * s.vdim;
-#pragma unroll
-    for (int d = 0; d < 2 * VC; ++d) {
-      const int col = d * 16 + g * 4;
-      const uint2 v = make_uint2(pack_bf16x2(acc[k][d][0] * inv, acc[k][d][1] * inv), pack_bf16x2(acc[k][d][2] * inv, acc[k][d][3] * inv));
-      if (vec) {
-        if (col < s.vdim) *reinterpret_cast<uint2 *>(o + col) = v;
-      } else {
-        const unsigned int e[2] = {v.x, v.y};
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col + r < s.vdim) o[col + r] = static_cast<unsigned short>(e[r / 2] >> (16 * (r & 1)));
-      }
-    }
-  }
+  latent_finish<VC, CT>(p, acc, l, uok, upos, q0, start, h, g);
 }
 
 inline int fit_units(int units) { return units <= 4 ? units : units <= 6 ? 6 : 8; }   // of 32, as instantiated
@@ -261,23 +413,27 @@ extern "C" int tlf_latent_prefill(const void *q, const void *expanded, int64_t e
   a.q = static_cast<const unsigned short *>(q); a.expanded = static_cast<const unsigned short *>(expanded);
   a.latents = static_cast<const unsigned short *>(latents); a.cu_q = cu_seqlens_q; a.starts = seq_starts; a.kv_off = kv_offsets;
   a.out = static_cast<unsigned short *>(out); a.lde = expanded_stride; a.ldo = out_stride; a.first_seq = first_seq;
-  a.gate = gate; a.window = window; a.scale_log2 = scale * 1.4426950408889634f;
-  const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + kPQ - 1) / kPQ, heads, num_seqs));
+  a.gate = gate; a.window = window; a.scale_log2 = scale == 0.f ? 1.f : fabsf(scale) * 1.4426950408889634f;
+  a.q_keep = scale == 0.f ? 0u : ~0u; a.q_flip = scale < 0.f ? 0x80008000u : 0u;
+  const int dc = fit_units(a.s.Dq / 32), vc = (vdim + 31) / 32;
+  constexpr int rows = 128;
+  const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + rows - 1) / rows, heads, num_seqs));
   if (!grid.x) return TLF_E_SHAPE;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int dc = fit_units(a.s.Dq / 32), vc = (vdim + 31) / 32;
 #define TLF_LP(DC, VC) TLF_LAUNCH((latent_prefill_kernel<DC, VC>), grid, dim3(256), 0, st, a)
-#define TLF_LP_V(DC)              \
-  case DC:                        \
-    if (vc == 1) TLF_LP(DC, 1);   \
-    else if (vc == 2) TLF_LP(DC, 2); \
-    else TLF_LP(DC, 4);           \
+#define TLF_LW(DC, VC) TLF_LAUNCH((latent_prefill_wide_kernel<DC, VC>), grid, dim3(256), 0, st, a)
+#define TLF_LP_V(KERNEL, DC)          \
+  case DC:                            \
+    if (vc == 1) KERNEL(DC, 1);       \
+    else if (vc == 2) KERNEL(DC, 2);  \
+    else KERNEL(DC, 4);               \
     break;
   switch (dc) {
-    TLF_LP_V(1) TLF_LP_V(2) TLF_LP_V(3) TLF_LP_V(4) TLF_LP_V(6) TLF_LP_V(8)
+    TLF_LP_V(TLF_LP, 1) TLF_LP_V(TLF_LP, 2) TLF_LP_V(TLF_LP, 3) TLF_LP_V(TLF_LP, 4) TLF_LP_V(TLF_LW, 6) TLF_LP_V(TLF_LW, 8)
     default: return TLF_E_UNSUPPORTED;
   }
 #undef TLF_LP_V
+#undef TLF_LW
 #undef TLF_LP
   return launch_status();
 }

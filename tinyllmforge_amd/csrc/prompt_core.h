@@ -39,15 +39,15 @@ __device__ __forceinline__ void prompt_copy_at(const void *from, unsigned int ld
 
 // DC, VC: key and value dimensions in units of 32.  LDS holds two tiles of K and two of V, rows unpadded; the 16-byte pieces of a K row
 // are swapped with its neighbours in groups of 4 or 8 and pairs of pieces of a V row permuted by the row, against bank conflicts.
-template <bool LEAD, bool MASK>
+template <bool LEAD, bool MASK, bool START = false>
 struct PromptPart {
-  static constexpr bool lead = LEAD, mask = MASK;
+  static constexpr bool lead = LEAD, mask = MASK, start = START;
 };
 
 template <int DC, int VC, int CT>
 struct PromptCore {
-  template <bool LEAD, bool MASK>
-  using Part = PromptPart<LEAD, MASK>;
+  template <bool LEAD, bool MASK, bool START = false>
+  using Part = PromptPart<LEAD, MASK, START>;
   static constexpr int DP = DC * 32, VP = VC * 32, KCH = DC * 4, VCH = VC * 4, KX = KCH % 8 == 0 ? 7 : 3;
   static constexpr int KB = kPromptKeys * DP * 2, VB = kPromptKeys * VP * 2;        // bytes of a tile
   typedef floatx4 Scores[2][CT];      // of a half: [16 keys][16 units]; lane (n, g): keys g * 8 + 4 s + r of unit n
@@ -92,8 +92,9 @@ struct PromptCore {
     const unsigned int at = kat + (h >> 1 & 1) * KB + (h & 1) * (32 * DP * 2);
 #pragma unroll
     for (int kc = 0; kc < DC; ++kc) {
-      kf[0][kc] = prompt_lds<bf16x8>(KX == 7 ? at ^ (kc * 64) : at + kc * 64);
-      kf[1][kc] = prompt_lds<bf16x8>(KX == 7 ? (at + 16 * DP * 2) ^ (kc * 64) : at + 16 * DP * 2 + kc * 64);
+      const unsigned int to = KX == 7 ? (at ^ ((kc & 1) * 64)) + kc / 2 * 128 : at + kc * 64;
+      kf[0][kc] = prompt_lds<bf16x8>(to);
+      kf[1][kc] = prompt_lds<bf16x8>(to + 16 * DP * 2);
     }
   }
   __device__ __forceinline__ void read_v(int h) {
@@ -140,13 +141,14 @@ struct PromptCore {
   //   before(h, s, w)             ahead of the weights of half h; `w`: weights of half h - 1 whose values are not added yet (add_values)
   //   weights(h, s, w, part)
   // part.mask is not set where all keys of the half's tile are seen by all units: tiles clear_from <= t < clear_to of them (wave
-  // uniform), clear_from 0 without LEAD.  part.lead is set where t may be below clear_from.
-  template <bool LEAD, class CopyK, class CopyV, class From, class Finish, class Before, class Weigh>
+  // uniform), clear_from 0 without LEAD.  part.lead is set where t may be below clear_from, part.start in the first tile.
+  // BOTH: `before` is first called when the scores of both halves of the first tile are there.
+  template <bool LEAD, bool BOTH, class CopyK, class CopyV, class From, class Finish, class Before, class Weigh>
   __device__ __forceinline__ void walk(int tiles, int clear_from, int clear_to, CopyK copy_k, CopyV copy_v, From from, Finish finish, Before before, Weigh weights) {
     constexpr Part<true, true> lead{};
     constexpr Part<false, false> plain{};
     constexpr Part<false, true> tail{};
-    constexpr Part<LEAD, true> first{};
+    constexpr Part<LEAD, true, true> first{};
     Scores se, so;                    // of even and odd halves
     Weights we{}, wo{};
     auto make_scores = [&](Scores &s) __attribute__((always_inline)) {
@@ -161,11 +163,15 @@ struct PromptCore {
     read_k(0);
     make_scores(se);
     finish(0, se, first);
-    before(0, se, wo);
+    if constexpr (!BOTH) before(0, se, wo);
     read_k(1);
     make_scores(so);
+    if constexpr (BOTH) {
+      finish(1, so, first);
+      before(0, se, wo);
+    }
     weights(0, se, we, first);
-    finish(1, so, first);
+    if constexpr (!BOTH) finish(1, so, first);
     // scores of 2 t + 2 and 2 t + 3, weights of 2 t + 1 and 2 t + 2, values of 2 t and 2 t + 1
     auto two_steps = [&](int t, auto part) __attribute__((always_inline)) {
       TLF_DL_BARRIER(0);              // K of tile t + 1 and V of tile t are there; the buffers of K t and V t - 1 are free

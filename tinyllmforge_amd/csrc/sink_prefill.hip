@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
     l[k] = 0.f;
     over[k] = -INFINITY;                                     // no key yet
   }
-  core.template walk<false>(
+  core.template walk<false, false>(
       tiles, 0, min(tiles, (wave_first + 1) / kSK), copy_k, copy_v,            // the diagonal cuts the tiles behind
       [&](float (&f)[CT]) __attribute__((always_inline)) {   // without a cap: the score less the maximum so far
 #pragma unroll
