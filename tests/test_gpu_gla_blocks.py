@@ -1,0 +1,80 @@
+"""Gated linear attention over blocks of 32 tokens: lengths around the edges of chunks and blocks, every width of key and value,
+several sequences and segments, channels that fade at once beside ones that last."""
+import pytest
+import torch
+
+from oracle import gitopel as O
+
+pytestmark = pytest.mark.gpu
+
+
+def portions(lens):
+    crow, clen, cu, at = [], [], [0], 0
+    for n in lens:
+        crow += list(range(at, at + n, 16))
+        clen += [min(16, n - c) for c in range(0, n, 16)]
+        cu.append(len(crow))
+        at += n
+    return [torch.tensor(x, dtype=torch.int32, device="cuda") for x in (crow, clen, cu)]
+
+
+def run(H, dk, dv, rank, lens, start, tau, seed, lost=None, scale=1.0):
+    from tinyllmforge_amd import ops as P
+    g, dt, eps = torch.Generator().manual_seed(seed), torch.bfloat16, 1e-5
+    proj = [torch.randn(n, 2 * H * (dk + dv) + rank, generator=g).to(dt) for n in lens]
+    for p in proj:
+        p[:, H * dk:2 * H * dk] *= scale
+        p[:, :H * dk] /= scale
+    a2, a2b, nw = torch.randn(H * dk, rank, generator=g).to(dt), 2 + torch.randn(H * dk, generator=g).to(dt), torch.randn(dv, generator=g).to(dt)
+    a2[::7] *= 4                                             # some channels fade much faster than others
+    if lost is not None:
+        proj[lost][:] = float("nan")
+    first = [torch.randn(H, dk, dv, generator=g) for _ in lens]
+    state = torch.stack([torch.full((H, dk, dv), 5.0)] + first).cuda()
+    out = torch.full((sum(lens), H * dv), 7.0, dtype=dt, device="cuda")
+    t = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    P.gla_portions(torch.cat(proj).cuda(), a2.cuda(), a2b.cuda(), nw.cuda(), state, t([i + 1 for i in range(len(lens))]), t(start), *portions(lens), 0, len(lens),
+                   tau, eps, out)
+    assert (state[0] == 5.0).all()
+    at, errs = 0, []
+    for i, n in enumerate(lens):
+        if i != lost:
+            p = proj[i].double()
+            q, k, v, gt, r = p.split([H * dk, H * dk, H * dv, H * dv, rank], dim=1)
+            la = -torch.nn.functional.softplus(-(r @ a2.double().T + a2b.double())).view(-1, H, dk) / tau
+            o, s = O.gla_recurrence(q.view(-1, H, dk) * dk ** -0.5, k.view(-1, H, dk), v.view(-1, H, dv), la, first[i].double() if start[i] else None)
+            want = (O.unit_rms(o, eps) * nw.double()).reshape(-1, H * dv) * O.silu(gt)
+            err = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()
+            errs.append((n, err(out[at:at + n], want), err(state[i + 1], s)))
+        at += n
+    return errs
+
+
+# The output is rounded to bfloat16, by at most 2^-8 of each value.  Products are exact to 2^-24 and sums of 32 tokens' logarithms
+# towards the block's end (below 16 where a power still counts, to 2^-20 in the exponent) are in single precision.
+OUT, STATE = 2 ** -8, 2 ** -20
+
+
+@pytest.mark.parametrize("dk,dv", [(32, 32), (32, 256), (64, 96), (128, 64), (128, 256)])
+@pytest.mark.parametrize("tau", [16.0, 0.25])
+def test_lengths_around_chunks_and_blocks(dk, dv, tau):
+    lens = [1, 15, 16, 17, 31, 32, 33, 47, 49, 63, 64, 65]
+    for n, out, state in run(2, dk, dv, 16, lens, [5 * (i % 2) for i in range(len(lens))], tau, dk + dv):
+        assert out < OUT and state < STATE, (n, out, state)
+
+
+@pytest.mark.parametrize("dk,rank,lens", [(128, 8, [2100]), (64, 64, [1500, 700, 33]), (32, 24, [513, 2000])])
+def test_segments_of_whole_blocks(dk, rank, lens):
+    for n, out, state in run(1, dk, 64, rank, lens, [0] + [3] * (len(lens) - 1), 8.0, dk):
+        assert out < OUT and state < STATE, (n, out, state)
+
+
+def test_keys_that_leave_no_room_for_growing_powers():
+    for n, out, state in run(1, 64, 64, 16, [70], [0], 8.0, 3, scale=1e25):
+        assert out < OUT and state < STATE, (n, out, state)
+
+
+@pytest.mark.parametrize("lost", [0, 1, 2])
+def test_rows_of_another_sequence_are_not_touched(lost):
+    for n, out, state in run(2, 128, 64, 16, [17, 40, 50], [0, 5, 5], 16.0, lost, lost=lost):
+        assert out < OUT and state < STATE, (n, out, state)

@@ -8,7 +8,8 @@
 //
 //   gla_decode_kernel  one token: one workgroup per (row, head) streams the state through once (HBM bound: 8 dk dv
 //                      bytes per head), norm and output gate included
-//   portions of prompts, three kernels over chunks of 16 tokens (a chunk never crosses a sequence):
+//   portions of prompts in bf16 with the usual sizes: gla_blocks.hip.  Others, and fp32: three kernels over chunks of 16 tokens (a chunk
+//   never crosses a sequence):
 //   gla_chunk_kernel   per (chunk, head), parallel: decays b_t = sum of log2 alpha within the chunk,
 //                      Qd = q 2^b_t, Kd = k 2^(b_end - b_t), A[t, s] = sum_d q k 2^(b_t - b_s) for s <= t.  The
 //                      exponents of A are formed pair by pair: every factor is <= 1, whatever the decay
@@ -21,49 +22,9 @@
 //                      from zero (half the work), gla_segments_kernel chains them, and the scan starts every segment
 //                      from its state
 //   gla_out_kernel     norm and output gate
-#include "elem.h"
+#include "gla.h"
 
 namespace tlf {
-
-constexpr int kGlaMaxDk = 256, kGlaMaxDv = 512, kGlaMaxR = 256;
-
-struct GlaArgs {
-  const void *proj;        // [n, ld]
-  Partials part;           // decode: or its partial sums
-  int64_t ld;
-  const void *a2;          // [H * dk, R]
-  const void *a2_bias;     // [H * dk]
-  const void *norm_w;      // [dv]
-  float *state;            // [slots, H, dk, dv]
-  const int32_t *state_slots;
-  int32_t num_slots;
-  const int64_t *positions;   // decode: [rows]
-  void *out;               // [n, ldo]
-  int64_t ldo;
-  int32_t rows, H, dk, dv, R;
-  float inv_tau, q_scale, eps;
-  // portions
-  const int32_t *chunk_tok, *chunk_len;   // [chunks]: first row of the chunk in the step, tokens in it
-  const int32_t *cu_chunks;               // [seqs + 1]
-  const int32_t *starts;                  // [seqs]: tokens before this step, 0: the state starts at zero
-  int32_t chunks, seqs;
-  // workspace.  One record per (chunk, head): Qd, Kd, A, decays, 64 floats of padding (records a power of two apart
-  // would fall into few sets of the L2); o: [chunks, H, 16, dv]
-  float *rec, *o;
-  int32_t vec;                            // bf16 projection rows may be read 8 bytes at a time, key dim a full row
-  int32_t segs;                           // segments per sequence
-  float *seg_state, *seg_dec;             // [seqs, segs, H, dk, dv], [seqs, segs, H, DKP]
-};
-
-// log2 of sigmoid(z)^(1/tau) = -(max(-z, 0) log2 e + log2(1 + e)) / tau with e = 2^(-|z| log2 e).  log2(1 + e) keeps its
-// relative accuracy for small e: the rounding of u = 1 + e is undone by the factor e / (u - 1).
-__device__ __forceinline__ float log2_alpha(float z, float inv_tau) {
-  const float kL2e = 1.4426950408889634f;
-  const float e = __builtin_amdgcn_exp2f(-fabsf(z) * kL2e);
-  const float u = 1.0f + e, d = u - 1.0f;
-  const float l = d == 0.f ? e * kL2e : __builtin_amdgcn_logf(u) * e * __builtin_amdgcn_rcpf(d);
-  return -fmaf(fmaxf(-z, 0.f), kL2e, l) * inv_tau;
-}
 
 template <int VEC>
 struct Vf {
@@ -502,6 +463,10 @@ __global__ __launch_bounds__(256) void gla_segments_kernel(const GlaArgs a, int 
   }
 }
 
+void launch_gla_segments(const GlaArgs &a, int first_seq, int dkp, hipStream_t stream) {
+  TLF_LAUNCH(gla_segments_kernel, dim3((a.dk * a.dv + 255) / 256, a.H, a.seqs), dim3(256), 0, stream, a, first_seq, dkp);
+}
+
 // One wave per (row of a chunk, head).
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void gla_out_kernel(const GlaArgs a) {
@@ -595,8 +560,7 @@ int launch_gla_portions(GlaArgs &a, int first_seq, hipStream_t stream) {
       TLF_LAUNCH((gla_scan_kernel<T, NT, 0>), sgrid, dim3(256), 0, stream, a, first_seq);              \
     } else {                                                                                              \
       TLF_LAUNCH((gla_scan_kernel<T, NT, 1>), sgrid, dim3(256), 0, stream, a, first_seq);              \
-      TLF_LAUNCH(gla_segments_kernel, dim3((a.dk * a.dv + 255) / 256, a.H, a.seqs), dim3(256), 0, stream, \
-                 a, first_seq, (NT) * 16);                                                                \
+      launch_gla_segments(a, first_seq, (NT) * 16, stream);                                               \
       TLF_LAUNCH((gla_scan_kernel<T, NT, 2>), sgrid, dim3(256), 0, stream, a, first_seq);              \
     }                                                                                                     \
   } while (0)
@@ -664,8 +628,10 @@ extern "C" size_t tlf_gla_portions_workspace_bytes(int32_t rows, int32_t chunks,
   const size_t ch = static_cast<size_t>(chunks) * heads, dkp = gla_tiles(key_dim) * 16;
   const size_t segs = gla_segments(chunks, num_seqs, heads, value_dim);
   const size_t sg = segs > 1 ? segs * num_seqs * heads : 0;
-  return 4 * (ch * (gla_rec_size(static_cast<int>(dkp)) + static_cast<size_t>(kGC) * ((value_dim + 3) / 4 * 4)) +
-              sg * (dkp + static_cast<size_t>(key_dim) * value_dim));
+  const size_t chunked = 4 * (ch * (gla_rec_size(static_cast<int>(dkp)) + static_cast<size_t>(kGC) * ((value_dim + 3) / 4 * 4)) +
+                              sg * (dkp + static_cast<size_t>(key_dim) * value_dim));
+  const size_t blocks = gla_blocks_sizes(key_dim, value_dim) ? gla_blocks_workspace_bytes(chunks, num_seqs, heads, key_dim, value_dim) : 0;
+  return chunked > blocks ? chunked : blocks;        // dtype and alignments decide between them
 }
 
 extern "C" int tlf_gla_portions(const void *proj, int64_t proj_stride, const void *a2, const void *a2_bias,
@@ -689,6 +655,7 @@ extern "C" int tlf_gla_portions(const void *proj, int64_t proj_stride, const voi
   if (!workspace || !aligned16(workspace) ||
       workspace_bytes < tlf_gla_portions_workspace_bytes(rows, chunks, num_seqs, heads, key_dim, value_dim))
     return TLF_E_WORKSPACE;
+  if (gla_blocks_take(a, dtype)) return launch_gla_blocks(a, first_seq, workspace, static_cast<hipStream_t>(stream));
   const size_t ch = static_cast<size_t>(chunks) * heads, dkp = gla_tiles(key_dim) * 16;
   a.rec = static_cast<float *>(workspace);
   a.o = a.rec + ch * gla_rec_size(static_cast<int>(dkp));

@@ -1,0 +1,568 @@
+// Gated linear attention of prompt portions (gla.hip) on the bf16 matrix cores, in blocks of 32 tokens and at 32-bit precision.
+//
+// A product of fp32 values is the sum of products of their bf16 pieces: three pieces of 8 significant bits are an fp32 value, v is
+// one piece by itself.  Kd^T V and A V take three products, Qd S takes six (those of at least 2^-16 of the whole), and a bf16 product
+// runs at sixteen times the rate of an fp32 one.
+//
+//   gla_block_kernel       per (block of a sequence, head), parallel: b_t = sum of log2 alpha within the block,
+//                          Qd = q 2^b_t, Kd = k 2^(b_end - b_t), A[t, s] = sum_d q k 2^(b_t - b_s) for s <= t, each as three pieces in
+//                          the order the matrix cores read.  A = (q 2^b_t) (k 2^-b_s)^T as products of pieces, too, unless some channel
+//                          decays by more than 2^64 within the block.  Then every exponent is kept <= 0: the 8 x 8 blocks on A's
+//                          diagonal are formed pair by pair, those left of it through the value at the boundary in front of them
+//   gla_block_scan_kernel  per (sequence or segment, head) a workgroup with 32 columns of v per wave, sequential over the blocks:
+//                          O^T = S^T Qd^T + V^T A^T, out = norm and output gate of O;  S = diag(2^b_end) S + Kd^T V.  S stays in fp32
+//                          accumulators; their layout is the next block's operand when the summation index is labelled as Qd is laid
+//                          out.  A block's record and rows of v come into LDS one block ahead, and the rows' sums of squares
+//                          go from wave to wave across the barrier in front of the next block
+// Where (sequences, heads) alone leave CUs idle a sequence is cut into segments as in gla.hip.
+//
+// Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256: chunk 122 + scan 470 (both passes) + norm and gate 92 us
+// over 16-token chunks with fp32 products; here blocks 148 + first pass 57 + segments 18 + scan 265 us.  The blocks write 55 KB a record,
+// 4 TB/s with what they read; the scan is held by its barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's
+// error against 64 bits falls from 1e-7 .. 3e-6 (with the decay) to 1e-7 or less, the output's is its rounding to bf16 on both.
+#include "gemm_shared.h"
+#include "gla.h"
+
+namespace tlf {
+
+constexpr int kGB = 32, kGlaBlockMaxR = 64;   // tokens per block, rank of the decay projection
+
+template <int DK>
+struct GlaBlock {   // a record, in bytes: pieces of Qd, of Kd, of A, decays
+  static constexpr int kPiece = DK * kGB * 2, kAPiece = kGB * kGB * 2;
+  static constexpr int kK = 3 * kPiece, kA = 6 * kPiece, kDec = kA + 3 * kAPiece, kSize = kDec + 1024;
+};
+size_t gla_block_record(int dk) { return dk * kGB * 2 * 6 + kGB * kGB * 2 * 3 + 1024; }
+// Records of sequence s begin at (first chunk + s + 1) / 2: two chunks of 16 tokens are a block, and a sequence may end on one.
+__device__ __forceinline__ int gla_first_block(int first_chunk, int seq) { return (first_chunk + seq + 1) / 2; }
+
+// 16 bytes per lane into LDS from a base that is the same in all lanes, which the compiler does not always see.
+__device__ __forceinline__ void gla_copy(unsigned int offset, const void *base, unsigned int lds) {
+  const uint64_t p = reinterpret_cast<uintptr_t>(base);
+  const uint64_t u = static_cast<uint64_t>(static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(p >> 32)))) << 32 |
+                     static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(p)));
+  TLF_DL_COPY(offset, u, __builtin_amdgcn_readfirstlane(static_cast<int>(lds)));
+}
+
+// Eight fp32 values as three bf16 pieces each.
+__device__ __forceinline__ void gla_pieces(const float (&v)[8], uint4 (&p)[3]) {
+  typedef __bf16 pair __attribute__((ext_vector_type(2)));
+  unsigned int low, w[3][4];
+  asm("s_mov_b32 %0, 0xbf80" : "=s"(low));       // (-1, 0), see weight_pairs
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a = v[2 * j], b = v[2 * j + 1];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      w[i][j] = pack_bf16x2(a, b);
+      const pair h = __builtin_bit_cast(pair, w[i][j]);
+      a = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, low), a, false);
+      b = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, 0xbf800000u), b, false);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
+}
+
+template <int DK>
+__global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
+  typedef unsigned short T;
+  using Rec = GlaBlock<DK>;
+  constexpr int TH = DK * 4, LD = DK + 4, LPT = DK / 8;      // lanes per token, eight channels each
+  constexpr int NW = DK / 16;
+  static_assert(NW * kGB * kGB <= 2 * kGB * LD, "the waves' parts of A take the place of keys and decays");
+  __shared__ __attribute__((aligned(16))) float kb2[2][kGB][LD], kh[48][LD], am[kGB][kGB + 4], rs[kGB][kGlaBlockMaxR + 4];
+  float (&ks)[kGB][LD] = kb2[0], (&bs)[kGB][LD] = kb2[1];
+  __shared__ float tots[4][DK];
+  __shared__ int where[2], harsh;
+  const int chunk = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  if (tid == 0) where[1] = -1, harsh = 0;
+  __syncthreads();
+  for (int i = tid; i < a.seqs; i += TH)
+    if (a.cu_chunks[i] <= chunk && chunk < a.cu_chunks[i + 1]) {
+      where[0] = a.cu_chunks[i];
+      where[1] = i;
+    }
+  __syncthreads();
+  const int cbeg = where[0], seq = where[1];
+  if (seq < 0 || (chunk - cbeg) & 1) return;                 // the second chunk of a block
+  const int64_t tok0 = a.chunk_tok[chunk];
+  const int len = a.chunk_len[chunk] + (chunk + 1 < a.cu_chunks[seq + 1] ? a.chunk_len[chunk + 1] : 0);
+  const int64_t hk = static_cast<int64_t>(a.H) * DK, hv = static_cast<int64_t>(a.H) * a.dv;
+  const T *pr = static_cast<const T *>(a.proj) + tok0 * a.ld;
+  unsigned char *rec = reinterpret_cast<unsigned char *>(a.rec) + (static_cast<int64_t>(gla_first_block(cbeg, seq) + (chunk - cbeg) / 2) * a.H + h) * Rec::kSize;
+  for (int i = tid; i < kGB * a.R; i += TH) {
+    const int t = i / a.R, r = i - t * a.R;
+    rs[t][r] = t < len ? Elem<T>::ld(pr + t * a.ld + 2 * hk + 2 * hv + r) : 0.f;
+  }
+  for (int i = tid; i < kGB * (kGB + 4); i += TH) (&am[0][0])[i] = 0.f;
+  // token t, channels l * 4 .. and DK / 2 + l * 4 .. of it
+  const int t = tid / LPT, l = tid % LPT;
+  auto load_bf16 = [&](const T *p, float (&x)[8], int apart) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; i += 4) {
+      const uint2 u = *reinterpret_cast<const uint2 *>(p + i / 4 * apart);
+      x[i] = __uint_as_float(u.x << 16); x[i + 1] = __uint_as_float(u.x & 0xffff0000u);
+      x[i + 2] = __uint_as_float(u.y << 16); x[i + 3] = __uint_as_float(u.y & 0xffff0000u);
+    }
+  };
+  bool large;
+  {
+    float k[8];
+    load_bf16(pr + min(t, len - 1) * a.ld + hk + h * DK + l * 4, k, DK / 2);
+#pragma unroll
+    for (int i = 0; i < 8; i += 4)
+      *reinterpret_cast<float4 *>(&ks[t][i / 4 * (DK / 2) + l * 4]) = t < len ? make_float4(k[i], k[i + 1], k[i + 2], k[i + 3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    float most = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) most = fmaxf(most, fabsf(k[i]));
+    large = !(most < 1e9f);                                  // 2^64 times a key stays finite
+  }
+  // this thread's item of a 16-channel operand: token lane & 31, channels 16 (tid / 64) + 4 hi .. and + 8 + 4 hi ..
+  const int lane = tid & 63, hi = lane >> 5, kb = tid >> 6, qt = lane & 31, qc = kb * 16 + hi * 4;
+  float q[8], v[8], left[8];                                 // left: decay from a token to the block's end, in Kd's order
+  load_bf16(pr + min(qt, len - 1) * a.ld + h * DK + qc, q, 8);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q[j] = qt < len ? q[j] * a.q_scale : 0.f;
+  __syncthreads();
+  {
+    // decays: a thread has one channel and eight tokens, summed up here; the sums of the eights around them through LDS.  Sums towards the
+    // end are made on their own: as differences they would lose what the tokens before have decayed by
+    const int d = (tid >> 7) * 32 + qt, t0 = (tid >> 6 & 1) * 16 + hi * 8;
+    const T *w = static_cast<const T *>(a.a2) + (static_cast<int64_t>(h) * DK + d) * a.R;
+    const float bias = Elem<T>::ld(static_cast<const T *>(a.a2_bias) + h * DK + d);
+    float z[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) z[j] = bias;
+    int r = 0;
+    for (; r + 4 <= a.R; r += 4) {
+      float wr[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) wr[e] = Elem<T>::ld(w + r + e);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float4 x = *reinterpret_cast<const float4 *>(&rs[t0 + j][r]);
+        z[j] = fmaf(wr[0], x.x, z[j]);
+        z[j] = fmaf(wr[1], x.y, z[j]);
+        z[j] = fmaf(wr[2], x.z, z[j]);
+        z[j] = fmaf(wr[3], x.w, z[j]);
+      }
+    }
+    for (; r < a.R; ++r) {
+      const float wr = Elem<T>::ld(w + r);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) z[j] = fmaf(wr, rs[t0 + j][r], z[j]);
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      left[j] = t0 + j < len ? log2_alpha(z[j], a.inv_tau) : 0.f;
+      z[j] = sum += left[j];
+    }
+    tots[t0 / 8][d] = sum;
+    __syncthreads();
+    float before = 0.f, after = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      before += i < t0 / 8 ? tots[i][d] : 0.f;
+      after += 3 - i > t0 / 8 ? tots[3 - i][d] : 0.f;
+    }
+#pragma unroll
+    for (int j = 7; j >= 0; --j) {
+      const float own = left[j];
+      left[j] = after;
+      after += own;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bs[t0 + j][d] = before + z[j];
+    if (large || !(before + sum >= -64.f)) harsh = 1;
+  }
+  __syncthreads();
+  const bool apart = harsh != 0;
+  if (apart)                                                 // keys towards the boundaries at 8, 16 and 24 tokens, for A
+    for (int i = tid; i < 48 * DK; i += TH) {
+      const int row = i / DK, d = i % DK, sub = row < 8 ? 1 : row < 24 ? 2 : 3, s = row - (sub == 1 ? 0 : sub == 2 ? 8 : 24);
+      kh[row][d] = ks[s][d] * __builtin_amdgcn_exp2f(bs[sub * 8 - 1][d] - bs[s][d]);
+    }
+  uint4 p3[3], k3[3];
+  float bq[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) bq[j] = bs[qt][qc + (j >> 2) * 8 + (j & 3)];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = q[j] * __builtin_amdgcn_exp2f(bq[j]);
+  gla_pieces(v, p3);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4 *>(rec + i * Rec::kPiece + tid * 16) = p3[i];
+  floatx16 part;                                             // A^T over the wave's 16 channels: lane (hi, t), rows s
+#pragma unroll
+  for (int r = 0; r < 16; ++r) part[r] = 0.f;
+  if (!apart) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = ks[qt][qc + (j >> 2) * 8 + (j & 3)] * __builtin_amdgcn_exp2f(-bq[j]);
+    gla_pieces(v, k3);
+    bf16x8 x[3], y[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      x[i] = __builtin_bit_cast(bf16x8, k3[i]);
+      y[i] = __builtin_bit_cast(bf16x8, p3[i]);
+    }
+    part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[2], y[0], part, 0, 0, 0);
+    part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[0], y[2], part, 0, 0, 0);
+    part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[1], y[1], part, 0, 0, 0);
+    part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[1], y[0], part, 0, 0, 0);
+    part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[0], y[1], part, 0, 0, 0);
+    part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[0], y[0], part, 0, 0, 0);
+  }
+  {
+    const int d = (tid >> 7) * 32 + qt, s0 = (tid >> 6 & 1) * 16 + hi * 8;    // Kd's: channel d, eight tokens
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = ks[s0 + j][d] * __builtin_amdgcn_exp2f(left[j]);
+    gla_pieces(v, k3);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4 *>(rec + Rec::kK + i * Rec::kPiece + tid * 16) = k3[i];
+  }
+  if (tid < DK) reinterpret_cast<float *>(rec + Rec::kDec)[tid] = __builtin_amdgcn_exp2f(bs[kGB - 1][tid]);
+  __syncthreads();
+  if (!apart) {                                              // the waves' parts added up
+    float (*parts)[kGB][kGB] = reinterpret_cast<float (*)[kGB][kGB]>(&kb2[0][0][0]);     // [wave][s][t]
+#pragma unroll
+    for (int r = 0; r < 16; ++r) parts[kb][(r >> 2) * 8 + hi * 4 + (r & 3)][qt] = part[r];
+    __syncthreads();
+    for (int i = tid; i < kGB * kGB; i += TH) {
+      const int s = i / kGB, tt = i % kGB;
+      float x = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) x += parts[w][s][tt];
+      am[tt][s] = s <= tt ? x : 0.f;
+    }
+  } else {
+    auto load_row = [&](const float *row, float (&x)[8]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 8; i += 4) {
+        const float4 y = *reinterpret_cast<const float4 *>(row + i / 4 * (DK / 2) + l * 4);
+        x[i] = y.x; x[i + 1] = y.y; x[i + 2] = y.z; x[i + 3] = y.w;
+      }
+    };
+    float bt[8], q[8];
+    load_row(bs[t], bt);
+    load_bf16(pr + min(t, len - 1) * a.ld + h * DK + l * 4, q, DK / 2);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = t < len ? q[i] * a.q_scale : 0.f;
+    const int my = t >> 3;
+    if (my) {
+      float ref[8], qh[8];
+      load_row(bs[my * 8 - 1], ref);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) qh[i] = q[i] * __builtin_amdgcn_exp2f(bt[i] - ref[i]);
+      const int base = my == 1 ? 0 : my == 2 ? 8 : 24;
+      for (int s = 0; s < my * 8; ++s) {
+        float kv[8], acc = 0.f;
+        load_row(kh[base + s], kv);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc = fmaf(qh[i], kv[i], acc);
+        acc = group_sum<LPT>(acc);
+        if (l == 0) am[t][s] = acc;
+      }
+    }
+    for (int s = my * 8; s < my * 8 + 8; ++s) {
+      float kv[8], bv[8], acc = 0.f;
+      load_row(ks[s], kv);
+      load_row(bs[s], bv);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc = fmaf(q[i] * kv[i], __builtin_amdgcn_exp2f(fminf(bt[i] - bv[i], 0.f)), acc);
+      acc = group_sum<LPT>(acc);
+      if (l == 0 && s <= t) am[t][s] = acc;
+    }
+  }
+  __syncthreads();
+  if (tid < 128) {                                           // A's items: token lane & 31, eight tokens s
+    const int s0 = (tid >> 6) * 16 + hi * 8;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = am[qt][s0 + j];
+    gla_pieces(v, p3);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4 *>(rec + Rec::kA + i * Rec::kAPiece + tid * 16) = p3[i];
+  }
+}
+
+// MODE 0: the whole sequence from the state slot and back.  MODE 1: a segment's own contribution from zero.  MODE 2: a segment from
+// the state gla_segments_kernel left for it.
+template <int DK, int MODE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gla_block_scan_kernel(const GlaArgs a, int first_seq) {
+  typedef unsigned short T;
+  using Rec = GlaBlock<DK>;
+  constexpr int NI = DK / 32, VB = kGB * 32 * 2;             // tiles of S, bytes of a wave's rows of v
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hi = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = a.dv / 32;
+  const int h = blockIdx.x, seq = MODE == 0 ? blockIdx.z : blockIdx.z / a.segs, seg = MODE == 0 ? 0 : blockIdx.z % a.segs;
+  const bool last_seg = MODE == 0 || seg == a.segs - 1;
+  if (MODE == 1 && last_seg) return;                         // nobody starts behind the last segment
+  const unsigned int recs = TLF_DL_LDSADDR(lds), vs = recs + 2 * Rec::kSize + wave * 2 * VB;
+  float *rowsum = reinterpret_cast<float *>(lds + 2 * Rec::kSize + waves * 2 * VB);        // [2][waves][32]
+  const int slot = a.state_slots[first_seq + seq];
+  const bool slot_ok = slot >= 0 && slot < a.num_slots;
+  float *st = a.state + (static_cast<int64_t>(slot_ok ? slot : 0) * a.H + h) * DK * a.dv;
+  const int64_t sg = (static_cast<int64_t>(seq) * a.segs + seg) * a.H + h;
+  float *gst = MODE == 0 ? st : a.seg_state + sg * DK * a.dv;
+  const bool from_zero = MODE == 1 || (MODE == 0 && (!slot_ok || a.starts[first_seq + seq] == 0));
+  const int col = wave * 32 + n;
+  // lane (hi, n), register r of tile i: row 32 i + 8 (r / 4) + 4 hi + r % 4 of column n
+  floatx16 S[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int d = i * 32 + (r >> 2) * 8 + hi * 4 + (r & 3);
+      S[i][r] = from_zero ? 0.f : gst[static_cast<int64_t>(d) * a.dv + col];
+    }
+  const int64_t hk = static_cast<int64_t>(a.H) * DK;
+  const int cbeg = a.cu_chunks[seq], cend = a.cu_chunks[seq + 1], blocks = (cend - cbeg + 1) / 2;
+  const int64_t row0 = cbeg < cend ? a.chunk_tok[cbeg] : 0;
+  const int tokens = cbeg < cend ? (cend - 1 - cbeg) * 16 + a.chunk_len[cend - 1] : 0;
+  int b0 = 0, b1 = blocks;
+  if (MODE != 0) {
+    const int per = (blocks + a.segs - 1) / a.segs;
+    b0 = min(seg * per, blocks);
+    b1 = min(b0 + per, blocks);
+  }
+  const T *vbase = static_cast<const T *>(a.proj) + 2 * hk + static_cast<int64_t>(h) * a.dv + wave * 32;
+  const T *gbase = vbase + static_cast<int64_t>(a.H) * a.dv + hi * 4;
+  const unsigned char *rbase = reinterpret_cast<const unsigned char *>(a.rec) + (static_cast<int64_t>(gla_first_block(cbeg, seq)) * a.H + h) * Rec::kSize;
+  auto copy = [&](int b, int buf) __attribute__((always_inline)) {
+    const unsigned char *rec = rbase + static_cast<int64_t>(b) * a.H * Rec::kSize;
+    for (int i = (MODE == 1 ? Rec::kK / 1024 : 0) + wave; i < (MODE == 1 ? Rec::kA : Rec::kSize) / 1024; i += waves)
+      gla_copy(lane * 16, rec + i * 1024, recs + buf * Rec::kSize + i * 1024);
+    if (MODE == 1 && wave == waves - 1) gla_copy(lane * 16, rec + Rec::kDec, recs + buf * Rec::kSize + Rec::kDec);
+    const T *vp = vbase + (row0 + static_cast<int64_t>(b) * kGB) * a.ld;
+    const int last = min(kGB, tokens - b * kGB) - 1;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int row = min(j * 16 + (lane >> 2), last);
+      gla_copy(static_cast<unsigned int>(row * static_cast<int>(a.ld) * 2 + (lane & 3) * 16), vp, vs + buf * VB + j * 1024);
+    }
+  };
+  uint2 nw[MODE == 1 ? 1 : 4];
+  if constexpr (MODE != 1) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) nw[c] = *reinterpret_cast<const uint2 *>(static_cast<const T *>(a.norm_w) + wave * 32 + c * 8 + hi * 4);
+  }
+  floatx16 o;                                                // of the block before: lane (hi, n): token n, columns 8 (r / 4) + 4 hi + r % 4
+  uint2 gate[4];
+  auto put = [&](int b, int buf) __attribute__((always_inline)) {
+    float ss = 0.f;
+    for (int w = 0; w < waves; ++w) ss += rowsum[(buf * waves + w) * 32 + n];
+    const float inv = 1.0f / sqrtf(ss / static_cast<float>(a.dv) + a.eps);
+    if (n >= tokens - b * kGB) return;
+    T *out = static_cast<T *>(a.out) + (row0 + static_cast<int64_t>(b) * kGB + n) * a.ldo + static_cast<int64_t>(h) * a.dv + wave * 32 + hi * 4;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float g[4] = {__uint_as_float(gate[c].x << 16), __uint_as_float(gate[c].x & 0xffff0000u), __uint_as_float(gate[c].y << 16),
+                          __uint_as_float(gate[c].y & 0xffff0000u)};
+      const float w[4] = {__uint_as_float(nw[c].x << 16), __uint_as_float(nw[c].x & 0xffff0000u), __uint_as_float(nw[c].y << 16), __uint_as_float(nw[c].y & 0xffff0000u)};
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[e] = o[c * 4 + e] * inv * w[e] * g[e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g[e]));
+      *reinterpret_cast<uint2 *>(out + c * 8) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+    }
+  };
+  float sd[DK >= 64 ? DK / 64 : 1];                          // MODE 1: decay of the whole segment
+#pragma unroll
+  for (float &x : sd) x = 1.f;
+
+  if (b0 < b1) copy(b0, 0);
+  for (int b = b0; b < b1; ++b) {
+    const int buf = (b - b0) & 1;
+    TLF_DL_BARRIER(0);
+    if (b + 1 < b1) copy(b + 1, buf ^ 1);
+    if constexpr (MODE != 1) {
+      if (b > b0) put(b - 1, buf ^ 1);
+    }
+    const int len = min(kGB, tokens - b * kGB);
+    const unsigned int rec = recs + buf * Rec::kSize, vt = vs + buf * VB;
+    if (len < kGB) {                                         // rows behind the sequence: zeros, whatever lies there
+      for (int i = len * 4 + lane; i < kGB * 4; i += 64)
+        *reinterpret_cast<u32x4 __attribute__((address_space(3))) *>(vt + i * 16) = u32x4{0, 0, 0, 0};
+      wave_lds_fence();
+    }
+    auto tile = [&](unsigned int at) __attribute__((always_inline)) {
+      return *reinterpret_cast<const bf16x8 __attribute__((address_space(3))) *>(at + lane * 16);
+    };
+    bf16x8 vf[2];                                            // lane (hi, n): column n, tokens 16 tb + 8 hi ..
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+      const unsigned int at = vt + (tb * 16 + hi * 8 + (lane >> 2 & 3)) * 64 + (lane >> 4 & 1) * 32 + (lane & 3) * 8;
+      const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<shortx4 __attribute__((address_space(3))) *>(at)));
+      const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<shortx4 __attribute__((address_space(3))) *>(at + 256)));
+      vf[tb] = __builtin_bit_cast(bf16x8, make_uint4(x.x, x.y, y.x, y.y));
+    }
+    if constexpr (MODE != 1) {
+      const T *gp = gbase + (row0 + static_cast<int64_t>(b) * kGB + min(n, len - 1)) * a.ld;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) gate[c] = *reinterpret_cast<const uint2 *>(gp + c * 8);
+      floatx16 o0, o1;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o0[r] = o1[r] = 0.f;
+      // a step of 16 channels: its products, behind them the pieces of the next and the reads of the one after that
+      bf16x8 s3[2][3], q3[2][3];
+      auto pieces = [&](int kb) __attribute__((always_inline)) {
+        float x[8];
+        uint4 p[3];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = S[kb / 2][kb % 2 * 8 + j];
+        gla_pieces(x, p);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) s3[kb & 1][i] = __builtin_bit_cast(bf16x8, p[i]);
+      };
+      auto read = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) q3[kb & 1][i] = tile(rec + i * Rec::kPiece + kb * 1024);
+      };
+      read(0);
+      read(1);
+      pieces(0);
+      bf16x8 af[2][3];
+#pragma unroll
+      for (int kb = 0; kb < DK / 16; ++kb) {
+        __builtin_amdgcn_sched_barrier(0);
+        const auto &x = s3[kb & 1], &q = q3[kb & 1];
+        o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[0], q[0], o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[0], q[1], o1, 0, 0, 0);
+        o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[1], q[0], o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[1], q[1], o1, 0, 0, 0);
+        o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[0], q[2], o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[2], q[0], o1, 0, 0, 0);
+        if (kb + 1 < DK / 16) pieces(kb + 1);
+        if (kb + 2 < DK / 16) read(kb + 2);
+        if (kb + 2 == DK / 16) {
+#pragma unroll
+          for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) af[tb][i] = tile(rec + Rec::kA + i * Rec::kAPiece + tb * 1024);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          if (i & 1) o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[tb], af[tb][i], o1, 0, 0, 0);
+          else o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[tb], af[tb][i], o0, 0, 0, 0);
+        }
+      float ss = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        o[r] = o0[r] + o1[r];
+        ss = fmaf(o[r], o[r], ss);
+      }
+      const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
+      ss = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+      if (hi == 0) rowsum[(buf * waves + wave) * 32 + n] = ss;
+    }
+    const unsigned int dec = rec + Rec::kDec;
+    if constexpr (MODE == 1) {
+#pragma unroll
+      for (int j = 0; j < static_cast<int>(sizeof(sd) / 4); ++j) sd[j] *= *reinterpret_cast<const float __attribute__((address_space(3))) *>(dec + (j * 64 + lane % DK) * 4);
+    }
+    // six groups of products, the operands of the next group read behind those of this one
+    bf16x8 kf[2][NI];
+    auto read_k = [&](int at) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) kf[at & 1][i] = tile(rec + Rec::kK + at / 2 * Rec::kPiece + (i * 2 + (at & 1)) * 1024);
+    };
+    read_k(0);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const floatx4 f = *reinterpret_cast<const floatx4 __attribute__((address_space(3))) *>(dec + (i * 32 + c * 8 + hi * 4) * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[i][c * 4 + e] *= f[e];
+      }
+#pragma unroll
+    for (int at = 0; at < 6; ++at) {                         // piece at / 2, tokens 16 (at & 1) ..
+      __builtin_amdgcn_sched_barrier(0);
+      if (at + 1 < 6) read_k(at + 1);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) S[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[at & 1][i], vf[at & 1], S[i], 0, 0, 0);
+    }
+  }
+  if constexpr (MODE == 1) {
+    if (wave == 0) {
+#pragma unroll
+      for (int j = 0; j < static_cast<int>(sizeof(sd) / 4); ++j)
+        if (lane < DK) a.seg_dec[sg * DK + j * 64 + lane] = sd[j];
+    }
+  } else {
+    if (b0 < b1) {
+      TLF_DL_BARRIER(0);
+      put(b1 - 1, (b1 - 1 - b0) & 1);
+    }
+    if (!last_seg || !slot_ok) return;
+  }
+  float *dst = MODE == 1 ? gst : st;
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dst[static_cast<int64_t>(i * 32 + (r >> 2) * 8 + hi * 4 + (r & 3)) * a.dv + col] = S[i][r];
+}
+
+bool gla_blocks_sizes(int32_t dk, int32_t dv) { return (dk == 32 || dk == 64 || dk == 128) && dv % 32 == 0 && dv >= 32 && dv <= 256; }
+
+bool gla_blocks_take(const GlaArgs &a, int32_t dtype) {
+  return dtype == TLF_DT_BF16 && gla_blocks_sizes(a.dk, a.dv) && a.R <= kGlaBlockMaxR && a.ld % 8 == 0 && a.ld < (1 << 24) && a.ldo % 4 == 0 && aligned16(a.proj) &&
+         (reinterpret_cast<uintptr_t>(a.out) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.norm_w) & 7) == 0;
+}
+
+// Segments per sequence: a workgroup for every CU (two where LDS holds two), segments of at least 8 blocks.
+int gla_block_segments(int chunks, int seqs, int heads, int dk) {
+  const int64_t wgs = static_cast<int64_t>(seqs) * heads, full = dk == 128 ? 256 : 512, want = wgs >= full ? 1 : (full + wgs - 1) / wgs, most = chunks / seqs / 16;
+  const int64_t s = want < most ? want : most;
+  return static_cast<int>(s < 1 || seqs * s > 65535 ? 1 : s > 32 ? 32 : s);
+}
+
+size_t gla_blocks_workspace_bytes(int32_t chunks, int32_t seqs, int32_t heads, int32_t dk, int32_t dv) {
+  const size_t slots = (static_cast<size_t>(chunks) + seqs + 1) / 2 + 1, segs = gla_block_segments(chunks, seqs, heads, dk);
+  return slots * heads * gla_block_record(dk) + (segs > 1 ? 4 * segs * seqs * heads * (dk + static_cast<size_t>(dk) * dv) : 0);
+}
+
+template <int DK>
+int launch_gla_blocks_of(GlaArgs &a, int first_seq, hipStream_t stream) {
+  const int waves = a.dv / 32;
+  const size_t lds = 2 * GlaBlock<DK>::kSize + waves * (2 * kGB * 32 * 2 + 2 * 32 * 4);
+  constexpr int kMost = 2 * GlaBlock<DK>::kSize + 8 * (2 * kGB * 32 * 2 + 2 * 32 * 4);
+  static const hipError_t allowed = [] {
+    hipError_t e = hipSuccess;
+    for (const void *k : {reinterpret_cast<const void *>(&gla_block_scan_kernel<DK, 0>), reinterpret_cast<const void *>(&gla_block_scan_kernel<DK, 1>),
+                          reinterpret_cast<const void *>(&gla_block_scan_kernel<DK, 2>)})
+      if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kMost);
+    return e;
+  }();
+  if (allowed != hipSuccess) return static_cast<int>(allowed);
+  TLF_LAUNCH((gla_block_kernel<DK>), dim3(a.chunks, a.H), dim3(DK * 4), 0, stream, a);
+  const dim3 grid(a.H, 1, a.seqs * a.segs);
+  if (a.segs == 1) {
+    TLF_LAUNCH((gla_block_scan_kernel<DK, 0>), grid, dim3(waves * 64), lds, stream, a, first_seq);
+  } else {
+    TLF_LAUNCH((gla_block_scan_kernel<DK, 1>), grid, dim3(waves * 64), lds, stream, a, first_seq);
+    launch_gla_segments(a, first_seq, DK, stream);
+    TLF_LAUNCH((gla_block_scan_kernel<DK, 2>), grid, dim3(waves * 64), lds, stream, a, first_seq);
+  }
+  return launch_status();
+}
+
+int launch_gla_blocks(GlaArgs &a, int first_seq, void *workspace, hipStream_t stream) {
+  a.segs = gla_block_segments(a.chunks, a.seqs, a.H, a.dk);
+  const size_t slots = (static_cast<size_t>(a.chunks) + a.seqs + 1) / 2 + 1;
+  a.rec = static_cast<float *>(workspace);
+  a.seg_dec = a.rec + slots * a.H * gla_block_record(a.dk) / 4;
+  a.seg_state = a.seg_dec + static_cast<size_t>(a.seqs) * a.segs * a.H * a.dk;
+  switch (a.dk) {
+    case 32: return launch_gla_blocks_of<32>(a, first_seq, stream);
+    case 64: return launch_gla_blocks_of<64>(a, first_seq, stream);
+    default: return launch_gla_blocks_of<128>(a, first_seq, stream);
+  }
+}
+
+}  // namespace tlf
