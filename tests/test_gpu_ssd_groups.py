@@ -1,0 +1,44 @@
+"""State-space portions with the heads of a group in one workgroup: lengths around the edges of chunks, workgroups that are not full, every
+state size, heads whose decay leaves the common scale, segments."""
+import pytest
+import torch
+
+from tests.test_gpu_tibenex import rel, run_ssd, ssd_case
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+# x, B and C are rounded to bfloat16 before the sums and y * silu(z) after them: four relative errors of at most 2^-9 on average over
+# a product, three of them of one term's factors.
+TOL = 4 * 2 ** -9 * 0.77
+
+
+def copies(sizes, seqs):
+    """How often so many short sequences make 256 workgroups of 8 x 32 columns."""
+    H, Pv, N, G, taps = sizes
+    return -(-256 // (seqs * G * -(-(H // G * Pv // 32) // 8)))
+
+
+@pytest.mark.parametrize("sizes", [(24, 64, 128, 8, 4), (32, 32, 64, 8, 3), (64, 96, 32, 16, 4), (32, 64, 128, 4, 4), (40, 64, 64, 4, 2)])
+@pytest.mark.parametrize("decay,step", [(0.0, -1.5), (-4.0, -3.0), (3.0, 3.0), (2.0, 0.0)])
+def test_lengths_around_chunks(sizes, decay, step):
+    """Whole prompts, and a second portion that starts from the first one's state; the last two decays leave 2^63 within a chunk for
+    every head, and for some."""
+    lens = [2, 63, 64, 65, 127, 129]
+    proj, w, want = ssd_case(sizes, lens, BF, sum(sizes), decay, step)
+    times = copies(sizes, len(lens))
+    for steps in ([lens], [[0, 50, 60, 2, 64, 65], [2, 13, 4, 63, 63, 64]]):
+        got = run_ssd(sizes, proj * times, w, [x * times for x in steps], BF, list(range(1, 6 * times + 1)))
+        for s in list(range(6)) + list(range(6 * times - 6, 6 * times)):
+            assert rel(got[s], want[s % 6]) < TOL, (steps[0][s % 6], s, rel(got[s], want[s % 6]))
+
+
+@pytest.mark.parametrize("sizes,lens", [((64, 32, 128, 8, 4), [1500, 300]), ((32, 64, 32, 8, 4), [4111]), ((64, 64, 64, 8, 4), [600, 2, 1000])])
+def test_segments(sizes, lens):
+    """Sequences cut into segments, of which short ones leave some empty; late rows still see the first through a slow decay."""
+    proj, w, want = ssd_case(sizes, lens, BF, 5, decay=-5.0, step=-3.0)
+    for first in (0, 70):
+        steps = ([[min(first, n - 2) for n in lens]] if first else []) + [[n - (min(first, n - 2) if first else 0) for n in lens]]
+        got = run_ssd(sizes, proj, w, steps, BF, list(range(1, len(lens) + 1)))
+        for s in range(len(lens)):
+            assert rel(got[s], want[s]) < TOL, (first, s)
+            assert rel(got[s][-50:], want[s][-50:]) < 8e-3, (first, s)

@@ -313,4 +313,12 @@ __device__ __forceinline__ void gemm_epilogue_activated(const GemmParams &p, flo
                : "memory")
 #define TLF_DL_LDSADDR(P) static_cast<unsigned int>(reinterpret_cast<uintptr_t>(TLF_LPTR(P)))
 
+// 16 bytes per lane into LDS from a base that is the same in all lanes, which the compiler does not always see.
+__device__ __forceinline__ void dl_copy(unsigned int offset, const void *base, unsigned int lds) {
+  const uint64_t p = reinterpret_cast<uintptr_t>(base);
+  const uint64_t u = static_cast<uint64_t>(static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(p >> 32)))) << 32 |
+                     static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(p)));
+  TLF_DL_COPY(offset, u, __builtin_amdgcn_readfirstlane(static_cast<int>(lds)));
+}
+
 }  // namespace tlf

@@ -36,14 +36,6 @@ size_t gla_block_record(int dk) { return dk * kGB * 2 * 6 + kGB * kGB * 2 * 3 + 
 // Records of sequence s begin at (first chunk + s + 1) / 2: two chunks of 16 tokens are a block, and a sequence may end on one.
 __device__ __forceinline__ int gla_first_block(int first_chunk, int seq) { return (first_chunk + seq + 1) / 2; }
 
-// 16 bytes per lane into LDS from a base that is the same in all lanes, which the compiler does not always see.
-__device__ __forceinline__ void gla_copy(unsigned int offset, const void *base, unsigned int lds) {
-  const uint64_t p = reinterpret_cast<uintptr_t>(base);
-  const uint64_t u = static_cast<uint64_t>(static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(p >> 32)))) << 32 |
-                     static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(p)));
-  TLF_DL_COPY(offset, u, __builtin_amdgcn_readfirstlane(static_cast<int>(lds)));
-}
-
 // Eight fp32 values as three bf16 pieces each.
 __device__ __forceinline__ void gla_pieces(const float (&v)[8], uint4 (&p)[3]) {
   typedef __bf16 pair __attribute__((ext_vector_type(2)));
@@ -332,14 +324,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto copy = [&](int b, int buf) __attribute__((always_inline)) {
     const unsigned char *rec = rbase + static_cast<int64_t>(b) * a.H * Rec::kSize;
     for (int i = (MODE == 1 ? Rec::kK / 1024 : 0) + wave; i < (MODE == 1 ? Rec::kA : Rec::kSize) / 1024; i += waves)
-      gla_copy(lane * 16, rec + i * 1024, recs + buf * Rec::kSize + i * 1024);
-    if (MODE == 1 && wave == waves - 1) gla_copy(lane * 16, rec + Rec::kDec, recs + buf * Rec::kSize + Rec::kDec);
+      dl_copy(lane * 16, rec + i * 1024, recs + buf * Rec::kSize + i * 1024);
+    if (MODE == 1 && wave == waves - 1) dl_copy(lane * 16, rec + Rec::kDec, recs + buf * Rec::kSize + Rec::kDec);
     const T *vp = vbase + (row0 + static_cast<int64_t>(b) * kGB) * a.ld;
     const int last = min(kGB, tokens - b * kGB) - 1;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int row = min(j * 16 + (lane >> 2), last);
-      gla_copy(static_cast<unsigned int>(row * static_cast<int>(a.ld) * 2 + (lane & 3) * 16), vp, vs + buf * VB + j * 1024);
+      dl_copy(static_cast<unsigned int>(row * static_cast<int>(a.ld) * 2 + (lane & 3) * 16), vp, vs + buf * VB + j * 1024);
     }
   };
   uint2 nw[MODE == 1 ? 1 : 4];

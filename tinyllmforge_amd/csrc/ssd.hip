@@ -22,51 +22,13 @@
 //                      their accumulators are the next product's operand.  Where (sequences, heads, columns) alone leave CUs idle
 //                      a sequence is cut into segments: a first pass gathers each segment's own contribution from zero,
 //                      ssd_segments_kernel chains them, and the second pass starts every segment from its state.
+//   ssd_group_kernel   (ssd_groups.hip) the same formulas where several heads share B and C and sequences are long or many
 //   ssd_scan_kernel    any size and dtype, token by token
 #include <algorithm>
 
-#include "elem.h"
+#include "ssd.h"
 
 namespace tlf {
-
-constexpr int kSsdMaxN = 512, kSsdMaxP = 512, kSC = 64;   // kSC: tokens per chunk
-
-struct SsdArgs {
-  const void *proj;        // [n, ld]
-  Partials part;           // decode: or its partial sums
-  int64_t ld;
-  const void *conv, *conv_bias;              // [taps, channels], [channels]
-  const void *dt_bias, *A_log, *D;           // [H]
-  void *ring;              // [slots, taps, channels]
-  float *state;            // [slots, H, N, P]
-  const int32_t *state_slots;                // per sequence
-  int32_t num_slots;
-  const int64_t *positions;                  // per row
-  const int32_t *row_seq, *cu_q, *starts;
-  void *xbc;               // [rows, channels] activated
-  float *dt, *decay;       // [rows, H]: step size, log2 of the decay
-  void *out;               // [n, ldo]
-  int64_t ldo;
-  int32_t rows, H, P, N, G, taps, inner, channels;
-  int32_t first_seq, seqs, first_row, segs, slices;
-  float *seg_state, *seg_decay;              // [seqs, segs, H, N, P], [seqs, segs, H]
-};
-
-template <typename T>
-__device__ __forceinline__ float ssd_step(const SsdArgs &a, float raw, int h) {
-  return softplus_f32(raw + Elem<T>::ld(static_cast<const T *>(a.dt_bias) + h));
-}
-template <typename T>
-__device__ __forceinline__ float ssd_log2_decay(const SsdArgs &a, float dt, int h) {
-  return -expf(Elem<T>::ld(static_cast<const T *>(a.A_log) + h)) * dt * 1.4426950408889634f;
-}
-
-// 32-bit rows: the library's exponential; bf16 rows: the hardware's, far more exact than the rounding that follows.
-template <typename T>
-__device__ __forceinline__ float ssd_silu(float z) {
-  if constexpr (sizeof(T) == 4) return silu_f32(z);
-  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
-}
 
 // The state's N rows are dealt to teams of lanes_v threads, VEC columns each; osum[team][P] gets the teams' parts of S^T C.
 template <int VEC>
@@ -294,20 +256,6 @@ __device__ __forceinline__ void ssd_pair(const float (&w)[8], uint4 &hi, uint4 &
   }
   hi = make_uint4(h[0], h[1], h[2], h[3]);
   lo = make_uint4(l[0], l[1], l[2], l[3]);
-}
-
-// Inclusive sum over the wave's 64 lanes, on the vector ALU.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float ssd_dpp_add(float v) {
-  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
-}
-__device__ __forceinline__ float ssd_wave_scan(float v) {
-  v = ssd_dpp_add<0x111, 0xf>(v);      // row_shr 1, 2, 4, 8: within rows of 16 lanes
-  v = ssd_dpp_add<0x112, 0xf>(v);
-  v = ssd_dpp_add<0x114, 0xf>(v);
-  v = ssd_dpp_add<0x118, 0xf>(v);
-  v = ssd_dpp_add<0x142, 0xa>(v);      // row_bcast 15 into rows 1 and 3
-  return ssd_dpp_add<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3
 }
 
 // NN: N in units of 32, PT: columns of P in units of 16.  MODE 0: the whole portion from the state slot and back, 1: a
@@ -664,6 +612,7 @@ int ssd_segments(int64_t wgs, int max_tokens) {
 struct SsdPlan {
   bool chunked;
   int pt, slices, segs;
+  int group_segs;                                    // 0: ssd_chunk_kernel takes these sizes
   size_t xbc, steps, seg_state, seg_decay;           // bytes; `steps` twice
 };
 SsdPlan ssd_plan(int rows, int seqs, int max_tokens, int H, int P, int N, int G, int dtype) {
@@ -677,7 +626,9 @@ SsdPlan ssd_plan(int rows, int seqs, int max_tokens, int H, int P, int N, int G,
   if (static_cast<int64_t>(seqs) * p.segs > 65535) p.segs = 1;
   p.xbc = up(item * rows * (static_cast<size_t>(H) * P + 2 * static_cast<size_t>(G) * N));
   p.steps = up(4 * static_cast<size_t>(rows) * H);
-  const size_t sg = p.segs > 1 ? static_cast<size_t>(seqs) * p.segs * H : 0;
+  p.group_segs = ssd_groups_segments(H, P, N, G, seqs, max_tokens, dtype);
+  const int most = std::max(p.segs, p.group_segs);
+  const size_t sg = most > 1 ? static_cast<size_t>(seqs) * most * H : 0;
   p.seg_decay = up(4 * sg);
   p.seg_state = up(4 * sg * N * P);
   return p;
@@ -821,6 +772,10 @@ extern "C" int tlf_ssd_portions(const void *proj, int64_t proj_stride, const voi
   // pieces of 8: channels, groups and heads begin at multiples of 8
   const bool vec = vdim % 8 == 0 && state_dim % 8 == 0 && a.channels % 8 == 0 && a.ld % 4 == 0 && out_stride % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(proj) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
+  if (vec && p.group_segs && a.ld % 8 == 0 && a.ld < (1 << 24) && out_stride % 8 == 0 && aligned16(proj) && aligned16(out)) {
+    a.segs = p.group_segs;
+    return launch_ssd_groups(a, s);
+  }
 #define TLF_SK(NN, PT)                                      \
   do {                                                      \
     if (vec) launch_ssd_chunks<NN, PT, true>(a, s);         \
