@@ -320,6 +320,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
   }
+  if (MODE == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no copy is under way when the LDS is given back
   if (!active) return;
   if constexpr (MODE == 1) {
     const int64_t sg = (static_cast<int64_t>(sq) * a.segs + seg) * a.H + h;
