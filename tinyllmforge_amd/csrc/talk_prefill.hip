@@ -13,6 +13,11 @@
 // Nothing is rescaled.  The rows of two 16-key tiles are picked so that their accumulators are eight consecutive keys.  V travels
 // from the cache into LDS directly, behind the weights and the mix; rows are unpadded and pairs of their 16-byte pieces swizzled
 // against bank conflicts (the lane that fills a position picks the matching piece).
+//
+// A wave of the second kernel has 128 accumulators and 64 registers of q, and the scheduler is held back where it would gather operands:
+// with q partly in memory a tile of 32 rows took 14800 cycles, 9800 of them before the mix, waiting for it behind the loads of K; so 11000,
+// 3600 of them products.  Eight prompts of 1061 to 2048 tokens, 128 dimensions, both kernels: 16 heads on 8 KV heads 500 -> 356 us, on 4
+// 455 -> 336, 32 heads 734 -> 609.
 #include "gemm_shared.h"
 #include "prompt_tiles.h"
 #include "talk_attn.h"
@@ -271,7 +276,8 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
   unsigned int tat = TLF_DL_LDSADDR(Ts) + (n * TS + g * 8) * 2;
   unsigned int wat = w0 + ((rt + n) * ROW + g * 8 * HP + h0) * 2;    // where this lane puts weights
   unsigned int mat = w0 + ((rt + n) * ROW + h0 * kTM + g * 8) * 2;   // where it finds mixed ones
-  unsigned int rat = w0 + (wave * ROW + krow * HP + g * 8) * 2;      // a row's weights as the mix's operand
+  unsigned int rat = w0 + (wave * ROW + krow * HP + g % (HP < 32 ? HP / 8 : 4) * 8) * 2;     // a row's weights as the mix's operand; heads that
+                                                                     // there is no room for read others, times zeros
   unsigned int pat = w0 + (wave * ROW + n * kTM + g * 8) * 2;        // and its result
 
   bf16x8 kb[DC];
@@ -327,8 +333,8 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
 #pragma unroll
             for (int e = 0; e < HK; e += 2) {
               const float a = __builtin_amdgcn_exp2f(w[e1 + e][r] - m[e0 + e1 + e]), b = __builtin_amdgcn_exp2f(w[e1 + e + 1][r] - m[e0 + e1 + e + 1]);
-              hi[e / 2] = pack_bf16x2(a, b);
-              lo[e / 2] = pack_bf16x2(a - __uint_as_float(hi[e / 2] << 16), b - __uint_as_float(hi[e / 2] & 0xffff0000u));
+              weight_pairs(a, b, hi[e / 2], lo[e / 2]);
+              __builtin_amdgcn_sched_barrier(0);                     // one pair at a time, for the registers' sake
             }
             if constexpr (HK == 4) {
               talk_st<u32x2>(to, u32x2{hi[0], hi[1]});
@@ -360,7 +366,7 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
           hi[s] = lo[s] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
-          if (k * 32 + g * 8 < HP) {                                 // heads there are room for
+          if (HP < 32 || k * 32 + g * 8 < HP) {                      // heads there are room for
             hi[s] = talk_ld<bf16x8>(rat + row_at + (s * 4 * HP + k * 32) * 2);
             lo[s] = talk_ld<bf16x8>(rat + row_at + (s * 4 * HP + k * 32) * 2 + LO);
           }
@@ -401,6 +407,9 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
       }
 #pragma unroll
       for (int d = 0; d < 2 * VC; ++d) {
+        // V's reads stay beside their products: gathered ahead they push parts of q out of the registers, and each half of a tile then waits
+        // for q to come back from memory behind the loads of K
+        __builtin_amdgcn_sched_barrier(0);
         bf16x8 vb[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e)
