@@ -17,7 +17,7 @@
 // Where (sequences, heads) alone leave CUs idle a sequence is cut into segments as in gla.hip.
 //
 // Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256: chunk 122 + scan 470 (both passes) + norm and gate 92 us
-// over 16-token chunks with fp32 products; here blocks 148 + first pass 57 + segments 18 + scan 265 us.  The blocks write 55 KB a record,
+// over 16-token chunks with fp32 products; here blocks 148 + first pass 57 + segments 18 + scan 255 us.  The blocks write 55 KB a record,
 // 4 TB/s with what they read; the scan is held by its barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's
 // error against 64 bits falls from 1e-7 .. 3e-6 (with the decay) to 1e-7 or less, the output's is its rounding to bf16 on both.
 #include "gemm_shared.h"
@@ -366,6 +366,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (b0 < b1) copy(b0, 0);
   for (int b = b0; b < b1; ++b) {
     const int buf = (b - b0) & 1;
+    // addresses are made from the lane anew in each block: kept, they would not fit beside the state
+    int here = tid & 63;
+    asm volatile("" : "+v"(here));
+    const int lane = here, n = here & 31, hi = here >> 5;
     TLF_DL_BARRIER(0);
     if (b + 1 < b1) copy(b + 1, buf ^ 1);
     if constexpr (MODE != 1) {
