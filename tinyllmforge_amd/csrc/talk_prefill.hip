@@ -16,8 +16,8 @@
 //
 // A wave of the second kernel has 128 accumulators and 64 registers of q, and the scheduler is held back where it would gather operands:
 // with q partly in memory a tile of 32 rows took 14800 cycles, 9800 of them before the mix, waiting for it behind the loads of K; so 11000,
-// 3600 of them products.  Eight prompts of 1061 to 2048 tokens, 128 dimensions, both kernels: 16 heads on 8 KV heads 500 -> 356 us, on 4
-// 455 -> 336, 32 heads 734 -> 609.
+// 3600 of them products.  Eight prompts of 1061 to 2048 tokens, 128 dimensions, both kernels: 16 heads on 8 KV heads 500 -> 357 us, on 4
+// 455 -> 331, 32 heads 734 -> 612.
 #include "gemm_shared.h"
 #include "prompt_tiles.h"
 #include "talk_attn.h"
@@ -49,8 +49,10 @@ __device__ __forceinline__ T talk_uniform(const T *p) {              // through 
 constexpr int kTS = 64;             // keys per tile of the first kernel
 __device__ __forceinline__ int talk_tile_row(int t) { return (t & 32) | ((t & 4) << 2) | ((t & 24) >> 1) | (t & 3); }
 
+// Bound by its exponentials and the vector ALU.  128 registers: with more, the compiler keeps the scores in accumulator registers and moves
+// each out and in (both kernels on 16 heads, eight prompts of up to 2048 tokens: 371 -> 344 us).
 template <int DC, int CT>
-__global__ __launch_bounds__(256) void talk_stats_kernel(const TalkPrefillArgs p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void talk_stats_kernel(const TalkPrefillArgs p) {
   constexpr int DP = DC * 32, KCH = DC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[2][kTS][DP + 8];
   int sq, plane, xt;
