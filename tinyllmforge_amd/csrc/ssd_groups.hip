@@ -41,7 +41,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
   const int sq = MODE == 0 ? blockIdx.z : blockIdx.z / a.segs, seg = MODE == 0 ? 0 : blockIdx.z % a.segs;
   const bool last_seg = MODE == 0 || seg == a.segs - 1;
-  if (MODE == 1 && last_seg) return;                         // nobody starts behind the last segment
   // workgroup w runs on XCD w % 8: those of one group on one where the groups are a multiple of 8
   const int grp = blockIdx.x % a.G, share = a.H / a.G, cols = a.P / 32, units = share * cols, unit = blockIdx.x / a.G * waves + wave;
   const bool active = unit < units;
@@ -68,11 +67,24 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (int i = 0; i < NN; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) S[i][r] = 0.f;
-  if (MODE != 1 && active && slot_ok && a.starts[seq] != 0) {
+  // The last segment writes the state back while others may yet have to start: the second pass reads it from the last segment's place,
+  // which holds no contribution and where the first pass has put it.
+  const bool held = slot_ok && a.starts[seq] != 0;
+  float *const at_start = MODE == 0 ? st : a.seg_state + ((static_cast<int64_t>(sq) * a.segs + a.segs - 1) * a.H + h) * plane + p0 + n;
+  if (MODE == 1 && last_seg) {
+    if (active && held) {
+#pragma unroll
+      for (int i = 0; i < NN; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) at_start[state_at(i, r)] = st[state_at(i, r)];
+    }
+    return;
+  }
+  if (MODE != 1 && active && held) {
 #pragma unroll
     for (int i = 0; i < NN; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) S[i][r] = st[state_at(i, r)];
+      for (int r = 0; r < 16; ++r) S[i][r] = at_start[state_at(i, r)];
   }
   if (MODE == 2 && active) {
     for (int e = 0; e < seg; ++e) {
