@@ -42,3 +42,31 @@ def test_segments(sizes, lens):
         for s in range(len(lens)):
             assert rel(got[s], want[s]) < TOL, (first, s)
             assert rel(got[s][-50:], want[s][-50:]) < 8e-3, (first, s)
+
+
+@pytest.mark.parametrize("state_dim", [32, 64, 128])
+def test_the_state_is_summed_in_single_precision(state_dim):
+    """Sums of three tokens, whose factors no rounding to bfloat16 touches: x, B and C pass the convolution and SiLU as they are, and
+    softplus leaves the step sizes."""
+    from tinyllmforge_amd import ops as P
+    H, Pv, G, seqs, n = 24, 64, 8, 64, 3
+    inner, chan = H * Pv, H * Pv + 2 * G * state_dim
+    g = torch.Generator().manual_seed(state_dim)
+    between = lambda lo, hi, *s: (lo + (hi - lo) * torch.rand(*s, generator=g)).to(BF)
+    proj = torch.cat([torch.zeros(seqs * n, inner), between(32, 64, seqs * n, chan), between(20, 30, seqs * n, H)], dim=1).to(BF)
+    conv, a_log = torch.zeros(4, chan, dtype=BF), between(-6, -4, H)
+    conv[-1] = 1
+    w = P.SsdWeights(conv.cuda(), torch.zeros(chan, dtype=BF).cuda(), torch.zeros(H, dtype=BF).cuda(), a_log.cuda(), torch.ones(H, dtype=BF).cuda())
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    state, ring = torch.full((seqs, H, state_dim, Pv), 5.0, device="cuda"), torch.zeros(seqs, 4, chan, dtype=BF, device="cuda")
+    out = torch.empty(seqs * n, inner, dtype=BF, device="cuda")
+    P.ssd_portions(proj.cuda(), w, ring, state, i32(range(seqs)), torch.arange(n).repeat(seqs).cuda(), i32([s for s in range(seqs) for _ in range(n)]),
+                   i32(range(0, seqs * n + 1, n)), i32([0] * seqs), 0, seqs, 0, n, G, out)
+    x, B, _, dt = proj[:, inner:].double().view(seqs, n, -1).split([inner, G * state_dim, G * state_dim, H], dim=2)
+    x, B = x.view(seqs, n, H, Pv), B.reshape(seqs, n, G, state_dim).repeat_interleave(H // G, 2)
+    want = torch.zeros(seqs, H, state_dim, Pv, dtype=torch.float64)
+    for t in range(n):
+        want = want * torch.exp(-torch.exp(a_log.double()) * dt[:, t])[..., None, None] + (dt[:, t, :, None] * B[:, t])[..., None] * x[:, t, :, None]
+    # a factor's roundings (an exponential, two products) and those of three sums, at most 2^-23 each and half of that on average; with
+    # pairs of bfloat16, 2^-17 at most for each token, the sums were 2^-20 off and more
+    assert rel(state, want) < 2 ** -21

@@ -89,6 +89,26 @@ __device__ __forceinline__ void weight_pairs(float a, float b, unsigned int &hi,
                    __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, 0xbf800000u), b, false));
 }
 
+// Eight fp32 values as three bf16 pieces each: all 24 significant bits.
+__device__ __forceinline__ void bf16_pieces(const float (&v)[8], uint4 (&p)[3]) {
+  typedef __bf16 pair __attribute__((ext_vector_type(2)));
+  unsigned int low, w[3][4];
+  asm("s_mov_b32 %0, 0xbf80" : "=s"(low));       // (-1, 0), see weight_pairs
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a = v[2 * j], b = v[2 * j + 1];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      w[i][j] = pack_bf16x2(a, b);
+      const pair h = __builtin_bit_cast(pair, w[i][j]);
+      a = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, low), a, false);
+      b = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, 0xbf800000u), b, false);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
+}
+
 __device__ __forceinline__ void unpack8(const uint4 &p, float (&f)[8]) {
   f[0] = __uint_as_float(p.x << 16);
   f[1] = __uint_as_float(p.x & 0xffff0000u);

@@ -36,26 +36,6 @@ size_t gla_block_record(int dk) { return dk * kGB * 2 * 6 + kGB * kGB * 2 * 3 + 
 // Records of sequence s begin at (first chunk + s + 1) / 2: two chunks of 16 tokens are a block, and a sequence may end on one.
 __device__ __forceinline__ int gla_first_block(int first_chunk, int seq) { return (first_chunk + seq + 1) / 2; }
 
-// Eight fp32 values as three bf16 pieces each.
-__device__ __forceinline__ void gla_pieces(const float (&v)[8], uint4 (&p)[3]) {
-  typedef __bf16 pair __attribute__((ext_vector_type(2)));
-  unsigned int low, w[3][4];
-  asm("s_mov_b32 %0, 0xbf80" : "=s"(low));       // (-1, 0), see weight_pairs
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float a = v[2 * j], b = v[2 * j + 1];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      w[i][j] = pack_bf16x2(a, b);
-      const pair h = __builtin_bit_cast(pair, w[i][j]);
-      a = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, low), a, false);
-      b = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, 0xbf800000u), b, false);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 3; ++i) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
-}
-
 template <int DK>
 __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   typedef unsigned short T;
@@ -182,7 +162,7 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   for (int j = 0; j < 8; ++j) bq[j] = bs[qt][qc + (j >> 2) * 8 + (j & 3)];
 #pragma unroll
   for (int j = 0; j < 8; ++j) v[j] = q[j] * __builtin_amdgcn_exp2f(bq[j]);
-  gla_pieces(v, p3);
+  bf16_pieces(v, p3);
 #pragma unroll
   for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4 *>(rec + i * Rec::kPiece + tid * 16) = p3[i];
   floatx16 part;                                             // A^T over the wave's 16 channels: lane (hi, t), rows s
@@ -191,7 +171,7 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   if (!apart) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = ks[qt][qc + (j >> 2) * 8 + (j & 3)] * __builtin_amdgcn_exp2f(-bq[j]);
-    gla_pieces(v, k3);
+    bf16_pieces(v, k3);
     bf16x8 x[3], y[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -209,7 +189,7 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
     const int d = (tid >> 7) * 32 + qt, s0 = (tid >> 6 & 1) * 16 + hi * 8;    // Kd's: channel d, eight tokens
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = ks[s0 + j][d] * __builtin_amdgcn_exp2f(left[j]);
-    gla_pieces(v, k3);
+    bf16_pieces(v, k3);
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4 *>(rec + Rec::kK + i * Rec::kPiece + tid * 16) = k3[i];
   }
@@ -271,7 +251,7 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
     const int s0 = (tid >> 6) * 16 + hi * 8;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = am[qt][s0 + j];
-    gla_pieces(v, p3);
+    bf16_pieces(v, p3);
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4 *>(rec + Rec::kA + i * Rec::kAPiece + tid * 16) = p3[i];
   }
@@ -407,7 +387,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         uint4 p[3];
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = S[kb / 2][kb % 2 * 8 + j];
-        gla_pieces(x, p);
+        bf16_pieces(x, p);
 #pragma unroll
         for (int i = 0; i < 3; ++i) s3[kb & 1][i] = __builtin_bit_cast(bf16x8, p[i]);
       };

@@ -6,15 +6,18 @@
 //                        Y^T = S^T C^T + X^T (w_s G)^T, y = 2^(c_t) Y with w_s = dt_s 2^(-c_s)
 //                        S = 2^(c_end) S + B^T (dt_s 2^(c_end - c_s) X)
 //                      S stays in fp32 accumulators, and their layout is the next product's operand: rows of S are labelled so that C
-//                      is read in whole granules.  S, w G and the scaled X enter as bf16 hi + lo pairs, x, B and C are exact.  A chunk's
-//                      rows come into LDS one chunk ahead, granules of 16 bytes swizzled by the row.  Where some w_s leaves 2^63
-//                      (or a head decays by more than 2^100 within a chunk), the head takes 2^(c_t - c_s) dt_s pair by pair instead.
+//                      is read in whole granules.  S and w G enter as bf16 hi + lo pairs, x, B and C are exact.  The scaled X enters as
+//                      three pieces: what it lacks stays in the state.  A chunk's rows come into LDS one chunk ahead, granules of
+//                      16 bytes swizzled by the row.  Where some w_s leaves 2^63 (or a head decays by more than 2^100 within a
+//                      chunk), the head takes 2^(c_t - c_s) dt_s pair by pair instead.
 //
 // A segment's contribution comes from a first pass over B and X (MODE 1); a segment adds up what lies before it as it starts.
 //
 // 128 heads of 64 in 8 groups, state 128, 4 sequences of up to 3000 tokens: 430 us with ssd_chunk_kernel, which forms G for every head and
-// passes S through LDS as pairs; here 209 + 68.  A chunk of 4 heads takes 18700 cycles, 5000 of them products and 9200 vector instructions on
-// each SIMD, the rest latency of two waves per SIMD (S alone takes 64 registers).  16 columns per wave and four waves per SIMD were slower
+// passes S through LDS as pairs; here 218 + 83.  With the scaled X as pairs 209 + 68, but then 1 to 4 % more outputs than with
+// ssd_chunk_kernel missed their nearest bf16 value (1.3 in a thousand do; the state's error is 1.1e-6 to 2.4e-6, and 2e-7 to 8e-7 with pieces).  So a chunk of
+// 4 heads took 18700 cycles, 5000 of them products and 9200 vector instructions on each SIMD, the rest latency of two waves per SIMD (S alone
+// takes 64 registers).  16 columns per wave and four waves per SIMD were slower
 // (285 + 71: twice the reads of B and C, twice the weights), and so were copies issued in a row (+2300 cycles a chunk: a wave waits where
 // several are queued) and step sizes masked as they are loaded (+2200: that waits for them).
 #include <algorithm>
@@ -316,8 +319,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       unpack8(__builtin_bit_cast(uint4, xf[ks]), x8);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x8[j] *= f8[j];
-      bf16x8 xh, xl;
-      pairs(x8, xh, xl);
+      uint4 x3[3];
+      bf16_pieces(x8, x3);
 #pragma unroll
       for (int i = 0; i < NN; ++i) {
         uint2 b[2];                                          // row m of the operand is state row m with bits 2 and 3 exchanged
@@ -327,8 +330,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           b[q] = turned(bs + at_row(row, i * 4 + (lane >> 4 & 1) * 2 + (chunk >> 1)) + (chunk & 1) * 8);
         }
         const bf16x8 bt = __builtin_bit_cast(bf16x8, make_uint4(b[0].x, b[0].y, b[1].x, b[1].y));
-        S[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt, xh, S[i], 0, 0, 0);
-        S[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt, xl, S[i], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 3; ++e) S[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt, __builtin_bit_cast(bf16x8, x3[e]), S[i], 0, 0, 0);
       }
     }
   }
