@@ -82,3 +82,52 @@ def test_weights_follow_a_growing_maximum(dim, vdim, cap):
     want = torch.einsum("hij,jd->ihd", torch.softmax(s, -1), v.double())
     # bf16 result (2^-9) of weights with 16 significant bits and fp32 scores of up to 2^8
     torch.testing.assert_close(out.view(new, heads, vdim).double().cpu(), want, rtol=2 ** -8, atol=2 ** -10)
+
+
+# A value that is infinite or no number belongs to the rows that see its key: weights of zero times it are no numbers.  Keys are taken in
+# tiles of 64 and rows by waves of 32 (one head per KV head), and a wave computes no tile that none of its rows sees.
+@pytest.mark.parametrize("dim,vdim", [(32, 32), (96, 64), (128, 128), (136, 128)])
+@pytest.mark.parametrize("cap", [None, 20.0, 50.0])
+def test_sinks_a_value_without_a_number_stays_in_its_tile(dim, vdim, cap):
+    torch.manual_seed(dim)
+    dev, BF, n = "cuda", torch.bfloat16, 200
+    kv = ops.SinkKV(4, 64, 2, dim, vdim, BF, dev)
+    kv.k.normal_()
+    kv.v.normal_()
+    q = torch.randn(n, 2, kv.k.shape[3], device=dev).mul(0.1).to(BF)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=dev)
+    def run():
+        out = torch.full((n, 2 * vdim), 7.0, device=dev, dtype=BF)
+        return ops.sink_attention_prefill(q, kv, i32(2, 0, 3, 1).view(1, -1), i32(0, n), i32(0), 0, 1, n, None, None, cap, out)
+    want = run().clone()
+    assert want.isfinite().all()
+    for key, value in ((100, torch.nan), (127, torch.inf), (64, -torch.inf)):    # rows 0 .. 63: two waves of the same workgroup
+        kept = kv.v[0, :, key - 64].clone()
+        kv.v[0, :, key - 64] = value
+        got = run()
+        assert torch.equal(got[:64], want[:64]) and not got[key:].isfinite().any(), key
+        kv.v[0, :, key - 64] = kept
+
+
+@pytest.mark.parametrize("dim,rot,vdim", [(24, 8, 32), (64, 32, 64), (64, 64, 128), (128, 64, 128)])
+def test_latent_a_value_without_a_number_stays_in_its_tile(dim, rot, vdim):
+    torch.manual_seed(dim)
+    dev, BF, n, heads = "cuda", torch.bfloat16, 300, 2
+    s = ops.LatentShape(heads, dim, rot, 64, vdim)
+    q, latents = torch.randn(n, heads, s.dq, device=dev).to(BF), torch.randn(n, s.lp, device=dev).to(BF)
+    expanded = torch.randn(n, heads * (dim + vdim), device=dev).to(BF)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=dev)
+    def run(window):
+        out = torch.full((n, heads * vdim), 7.0, device=dev, dtype=BF)
+        return ops.latent_prefill(q, expanded, latents, i32(0, n), i32(0), i32(0, n), 0, 1, n, window, 0.1, s, out)
+    # rows 0 .. 63 do not see the tile of key 100.  With a window of 100 the tiles of rows 128 .. 255 begin at key 29, and the first one is
+    # not seen by rows 224 .. 255; the second one, of key 100, is
+    for window, key, kept in ((1 << 20, 100, [(0, 64)]), (100, 40, [(224, 300)]), (100, 100, [(0, 64), (256, 300)])):
+        want, held = run(window).clone(), expanded[key].clone()
+        assert want.isfinite().all()
+        expanded[key, heads * dim:] = torch.nan
+        got = run(window)
+        expanded[key] = held
+        for a, b in kept:
+            assert torch.equal(got[a:b], want[a:b]), (window, key, a)
+        assert got[key:min(key + window, n)].isnan().all(), (window, key)

@@ -146,9 +146,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     l[k] = 0.f;
   }
   // tiles between the window's edge and the diagonal hide nothing from any of the wave's rows
+  const int to = max(0, wave_last - w0) / kPK + 1;
   const int edge = wave_last - p.window >= w0 ? (wave_last - p.window - w0) / kPK + 1 : 0;
-  core.template walk<true, true>(
-      tiles, edge, min(tiles, max(0, (wave_first + 1 - w0) / kPK)), copy_k, copy_v,
+  core.template walk<true, true, true>(
+      tiles, min(max(0, wave_first - p.window + 1 - w0) / kPK, to - 1), to, edge, min(tiles, max(0, (wave_first + 1 - w0) / kPK)), copy_k, copy_v,
       [](float (&f)[CT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < CT; ++k) f[k] = 0.f;

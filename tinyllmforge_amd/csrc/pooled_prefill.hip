@@ -158,8 +158,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   };
   // tiles between the window's edge and the diagonal hide nothing from anyone
   const int edge = i_last - c.size >= w0 ? (i_last - c.size - w0) / kTK + 1 : 0;
-  core.template walk<true, false>(
-      tiles, ptiles + edge, min(tiles, ptiles + max(0, (i_first + 1 - w0) / kTK)),
+  core.template walk<true, false, false>(
+      tiles, 0, tiles, ptiles + edge, min(tiles, ptiles + max(0, (i_first + 1 - w0) / kTK)),
       copy_k, copy_v,
       [](float (&f)[CT]) __attribute__((always_inline)) { f[0] = f[1] = 0.f; }, [](int, typename Core::Scores &, auto) __attribute__((always_inline)) {},
       [](int, typename Core::Scores &, typename Core::Weights &) __attribute__((always_inline)) {},

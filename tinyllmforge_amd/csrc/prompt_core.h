@@ -134,17 +134,19 @@ struct PromptCore {
     w.lo[c] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
   }
 
-  // The walk over `tiles` tiles.  The kernel's parts:
+  // The workgroup's walk over `tiles` tiles, of which the wave computes first_tile <= t < end: those that some of its units see.  A value
+  // behind or before them, infinite or no number as it may be, does not reach its rows.  The kernel's parts:
   //   copy_k(t, part), copy_v     the tile's copies; called for t = 0, 1, .. in turn
   //   from(f)                     where a unit's scores begin (read once per half)
   //   finish(h, s, part)          what is done to the scores of half h as soon as they are there
   //   before(h, s, w)             ahead of the weights of half h; `w`: weights of half h - 1 whose values are not added yet (add_values)
   //   weights(h, s, w, part)
   // part.mask is not set where all keys of the half's tile are seen by all units: tiles clear_from <= t < clear_to of them (wave
-  // uniform), clear_from 0 without LEAD.  part.lead is set where t may be below clear_from, part.start in the first tile.
-  // BOTH: `before` is first called when the scores of both halves of the first tile are there.
-  template <bool LEAD, bool BOTH, class CopyK, class CopyV, class From, class Finish, class Before, class Weigh>
-  __device__ __forceinline__ void walk(int tiles, int clear_from, int clear_to, CopyK copy_k, CopyV copy_v, From from, Finish finish, Before before, Weigh weights) {
+  // uniform), clear_from 0 without LEAD.  part.lead is set where t may be below clear_from, part.start in the wave's first tile.
+  // BOTH: `before` is first called when the scores of both halves of that tile are there.
+  // SOME: it may be some only; otherwise first_tile is 0 and `end` is `tiles`.
+  template <bool LEAD, bool SOME, bool BOTH, class CopyK, class CopyV, class From, class Finish, class Before, class Weigh>
+  __device__ __forceinline__ void walk(int tiles, int first_tile, int end, int clear_from, int clear_to, CopyK copy_k, CopyV copy_v, From from, Finish finish, Before before, Weigh weights) {
     constexpr Part<true, true> lead{};
     constexpr Part<false, false> plain{};
     constexpr Part<false, true> tail{};
@@ -156,25 +158,34 @@ struct PromptCore {
       from(f);
       scores(f, s);
     };
+    // K of tile t and V of tile t - 1 are there; the buffers of K t - 1 and V t - 2 are free
+    auto arrive = [&](int t, auto part) __attribute__((always_inline)) {
+      TLF_DL_BARRIER(0);
+      if (t < tiles) copy_v(t, part);
+      if (t + 1 < tiles) copy_k(t + 1, part);
+    };
     copy_k(0, first);
+    int t = SOME ? first_tile : 0;
+    if constexpr (LEAD && SOME)
+      for (int i = 0; i < t; ++i) arrive(i, first);
     TLF_DL_BARRIER(0);
-    copy_v(0, first);
-    if (tiles > 1) copy_k(1, first);
-    read_k(0);
+    copy_v(t, first);
+    if (t + 1 < tiles) copy_k(t + 1, first);
+    read_k(2 * t);
     make_scores(se);
-    finish(0, se, first);
-    if constexpr (!BOTH) before(0, se, wo);
-    read_k(1);
+    finish(2 * t, se, first);
+    if constexpr (!BOTH) before(2 * t, se, wo);
+    read_k(2 * t + 1);
     make_scores(so);
     if constexpr (BOTH) {
-      finish(1, so, first);
-      before(0, se, wo);
+      finish(2 * t + 1, so, first);
+      before(2 * t, se, wo);
     }
-    weights(0, se, we, first);
-    if constexpr (!BOTH) finish(1, so, first);
+    weights(2 * t, se, we, first);
+    if constexpr (!BOTH) finish(2 * t + 1, so, first);
     // scores of 2 t + 2 and 2 t + 3, weights of 2 t + 1 and 2 t + 2, values of 2 t and 2 t + 1
     auto two_steps = [&](int t, auto part) __attribute__((always_inline)) {
-      TLF_DL_BARRIER(0);              // K of tile t + 1 and V of tile t are there; the buffers of K t and V t - 1 are free
+      TLF_DL_BARRIER(0);
       copy_v(t + 1, part);
       if (t + 2 < tiles) copy_k(t + 2, part);
       before(2 * t + 1, so, we);
@@ -193,18 +204,24 @@ struct PromptCore {
       finish(2 * t + 3, so, part);
     };
     // loops of their own: as a choice inside one loop the two forms do not fit the registers
-    int t = 0;
     if constexpr (LEAD)
-      for (; t + 1 < tiles && t < clear_from; ++t) two_steps(t, lead);
+      for (; t + 1 < end && t < clear_from; ++t) two_steps(t, lead);
     for (; t + 1 < clear_to; ++t) two_steps(t, plain);
-    for (; t + 1 < tiles; ++t) two_steps(t, tail);
-    TLF_DL_BARRIER(0);
-    before(2 * tiles - 1, so, we);
-    weights(2 * tiles - 1, so, wo, first);
-    read_v(2 * tiles - 2);
+    for (; t + 1 < end; ++t) two_steps(t, tail);
+    if constexpr (SOME) {
+      arrive(t + 1, first);
+    } else {
+      TLF_DL_BARRIER(0);
+      t = tiles - 1;
+    }
+    before(2 * t + 1, so, we);
+    weights(2 * t + 1, so, wo, first);
+    read_v(2 * t);
     values(we);
-    read_v(2 * tiles - 1);
+    read_v(2 * t + 1);
     values(wo);
+    if constexpr (SOME)
+      for (t += 2; t <= tiles; ++t) arrive(t, first);        // for the other waves
   }
   // For `before`: the values of half h with weights `w`, which are used up.
   __device__ __forceinline__ void add_values(int h, Weights &w) {

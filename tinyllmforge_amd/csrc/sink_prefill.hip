@@ -102,6 +102,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   Core core;
   core.start(TLF_DL_LDSADDR(Ks), TLF_DL_LDSADDR(Vs), tid);
   const int wave_first = start + row0 + core.wave * CT * 16 / p.hpp;
+  const int wave_last = min(start + row0 + ((core.wave + 1) * CT * 16 - 1) / p.hpp, i_last);
 
   int upos[CT], urow[CT], uhead[CT];
   bool uok[CT];
@@ -163,8 +164,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
     l[k] = 0.f;
     over[k] = -INFINITY;                                     // no key yet
   }
-  core.template walk<false, false>(
-      tiles, 0, min(tiles, (wave_first + 1) / kSK), copy_k, copy_v,            // the diagonal cuts the tiles behind
+  core.template walk<false, true, false>(
+      tiles, 0, wave_last / kSK + 1, 0, min(tiles, (wave_first + 1) / kSK), copy_k, copy_v,            // the diagonal cuts the tiles behind
       [&](float (&f)[CT]) __attribute__((always_inline)) {   // without a cap: the score less the maximum so far
 #pragma unroll
         for (int k = 0; k < CT; ++k) f[k] = MODE == 0 && m[k] != -INFINITY ? -m[k] : 0.f;
