@@ -78,3 +78,24 @@ def test_keys_that_leave_no_room_for_growing_powers():
 def test_rows_of_another_sequence_are_not_touched(lost):
     for n, out, state in run(2, 128, 64, 16, [17, 40, 50], [0, 5, 5], 16.0, lost, lost=lost):
         assert out < OUT and state < STATE, (n, out, state)
+
+
+@pytest.mark.parametrize("dk,dv", [(32, 32), (64, 128), (128, 256)])
+@pytest.mark.parametrize("token", [16, 20, 31, 50])
+def test_a_value_without_a_number_reaches_no_earlier_chunk(dk, dv, token):
+    """Sixteen tokens are a chunk; an earlier token meets values behind it as zeros times them."""
+    from tinyllmforge_amd import ops as P
+    H, rank, n = 2, 16, 70
+    g, dt = torch.Generator().manual_seed(token), torch.bfloat16
+    proj = torch.randn(n, 2 * H * (dk + dv) + rank, generator=g).to(dt).cuda()
+    a2, a2b, nw = (torch.randn(s, generator=g).to(dt).cuda() for s in ((H * dk, rank), (H * dk,), (dv,)))
+    t = lambda *x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    def run():
+        out = torch.full((n, H * dv), 7.0, dtype=dt, device="cuda")
+        P.gla_portions(proj, a2, a2b, nw, torch.zeros(1, H, dk, dv, device="cuda"), t(0), t(0), *portions([n]), 0, 1, 8.0, 1e-5, out)
+        return out
+    want = run()
+    for value in (torch.nan, torch.inf):
+        proj[token, 2 * H * dk:2 * H * dk + H * dv] = value
+        got, first = run(), token // 16 * 16
+        assert torch.equal(got[:first], want[:first]) and not got[token:].isfinite().any()

@@ -13,7 +13,8 @@
 //                          O^T = S^T Qd^T + V^T A^T, out = norm and output gate of O;  S = diag(2^b_end) S + Kd^T V.  S stays in fp32
 //                          accumulators; their layout is the next block's operand when the summation index is labelled as Qd is laid
 //                          out.  A block's record and rows of v come into LDS one block ahead, and the rows' sums of squares
-//                          go from wave to wave across the barrier in front of the next block
+//                          go from wave to wave across the barrier in front of the next block.
+//                          A value that is no number reaches no row before its half of a block
 // Where (sequences, heads) alone leave CUs idle a sequence is cut into segments as in gla.hip.
 //
 // Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256: chunk 122 + scan 470 (both passes) + norm and gate 92 us
@@ -395,10 +396,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int i = 0; i < 3; ++i) q3[kb & 1][i] = tile(rec + i * Rec::kPiece + kb * 1024);
       };
+      // The block's second half of tokens first: for the tokens before it these are zeros times values that may be no number, which
+      // they drop.
+      bf16x8 af[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) af[i] = tile(rec + Rec::kA + i * Rec::kAPiece + 1024);
       read(0);
       read(1);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1], af[i], o1, 0, 0, 0);
       pieces(0);
-      bf16x8 af[2][3];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o1[r] = n < 16 ? 0.f : o1[r];
 #pragma unroll
       for (int kb = 0; kb < DK / 16; ++kb) {
         __builtin_amdgcn_sched_barrier(0);
@@ -413,19 +422,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (kb + 2 < DK / 16) read(kb + 2);
         if (kb + 2 == DK / 16) {
 #pragma unroll
-          for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-            for (int i = 0; i < 3; ++i) af[tb][i] = tile(rec + Rec::kA + i * Rec::kAPiece + tb * 1024);
+          for (int i = 0; i < 3; ++i) af[i] = tile(rec + Rec::kA + i * Rec::kAPiece);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          if (i & 1) o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[tb], af[tb][i], o1, 0, 0, 0);
-          else o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[tb], af[tb][i], o0, 0, 0, 0);
-        }
+      for (int i = 0; i < 3; ++i) o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0], af[i], o0, 0, 0, 0);
       float ss = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
