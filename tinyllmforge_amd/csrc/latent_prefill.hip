@@ -6,7 +6,8 @@
 // prompt_core.h's:
 //   P = 2^(S * scale - m)         fp32; m follows a row's maximum only when that has grown by more than 8 (a factor of 256,
 //                                 which the fp32 sums and the bf16 pair hold), so the accumulators are rarely rescaled.  Whether any
-//                                 has grown is asked lane by lane; maxima of rows are only formed when one has
+//                                 has grown is asked lane by lane; maxima of rows are only formed when one has, and all rows of the wave
+//                                 follow theirs then: a largest weight of 1 is not rounded
 // 16 heads of 96 and 64 dimensions, eight prompts of 1061 to 2048 tokens: layer 189 us with the stages of a tile one after the other and
 // a window of 1024, 173 so; three prompts up to 3000, causal, 208 and 185.
 #include "latent_attn.h"
@@ -180,10 +181,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
         if (hf > 0) core.add_values(hf - 1, w);
 #pragma unroll
         for (int k = 0; k < CT; ++k) {                       // sums and accumulators to the new maximum
-          const float most = max_lanes_16_32_48(x[k]);
-          const bool up = most > over[k];
-          const float back = up ? __builtin_amdgcn_exp2f(m[k] - most) : 1.f;
-          m[k] = up ? most : m[k];
+          const float most = fmaxf(m[k], max_lanes_16_32_48(x[k]));
+          const float back = most == m[k] ? 1.f : __builtin_amdgcn_exp2f(m[k] - most);
+          m[k] = most;
           over[k] = m[k] + 8.f;
           l[k] *= back;
 #pragma unroll
