@@ -157,3 +157,14 @@ def test_latent_maxima_follow_where_one_of_the_wave_grows():
     # the roundings of exponents and sums.  A result 2^-22 off misses its nearest value where it lies that close to the middle between two
     # of them, which are 2^-8 to 2^-7 of it apart: 2^-14 of the results at most.  Largest weights of 16 bits made 2^-12 of them miss
     assert (out.view(n, heads, vdim).cpu() != want.to(BF)).double().mean().item() < 2 ** -14
+
+
+def test_more_workgroups_than_a_dimension_of_a_launch_holds():
+    """The longest portion is the caller's bound: 2000 short ones under a bound of 300000 tokens are 12.5 million workgroups."""
+    torch.manual_seed(0)
+    lens = torch.tensor([1 + i % 3 for i in range(2000)])
+    n, dev, BF = int(lens.sum()), "cuda", torch.bfloat16
+    q, k, v = (torch.randn(n, 8, 128, device=dev).to(BF) for _ in range(3))
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)]).to(torch.int32).to(dev)
+    want = ops.varlen_prefill_attention(q, k, v, cu, cu, 3, 128 ** -0.5)
+    assert torch.equal(ops.varlen_prefill_attention(q, k, v, cu, cu, 300000, 128 ** -0.5), want)

@@ -18,6 +18,26 @@ extern "C" int place(long xtiles, long planes, long seqs, int most, int *out) {
     if (!tlf::prompt_tile(t, b, out[3 * b], out[3 * b + 1], out[3 * b + 2])) out[3 * b] = -1;
   return blocks;
 }
+struct Grid {
+  long x, y;
+  Grid(long x, long y = 1) : x(x), y(y) {}
+};
+// The grid, and how many of its workgroups behind the last one have a tile, or of those before have none but should
+extern "C" void limits(long xtiles, long planes, long seqs, long *out) {
+  tlf::PromptTiles t;
+  const int blocks = tlf::prompt_tiles_make(t, xtiles, planes, seqs);
+  const Grid g = tlf::prompt_grid<Grid>(blocks);
+  long tiles = 0, beyond = 0;
+  for (long y = 0; y < g.y; ++y)
+    for (long x = 0; x < g.x && blocks; ++x) {
+      const int b = tlf::prompt_block(x, y);
+      int s, p, i;
+      if (!tlf::prompt_tile(t, b, s, p, i)) continue;
+      ++tiles;
+      beyond += b >= blocks || s < 0 || s >= seqs || p < 0 || p >= planes || i < 0 || i >= xtiles;
+    }
+  out[0] = blocks; out[1] = g.x; out[2] = g.y; out[3] = beyond + (blocks ? tiles - xtiles * planes * seqs : 0);
+}
 """
 
 
@@ -25,8 +45,9 @@ extern "C" int place(long xtiles, long planes, long seqs, int most, int *out) {
 def place(tmp_path_factory):
     at = tmp_path_factory.mktemp("tiles")
     (at / "place.cpp").write_text(SOURCE)
-    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-O1", "-I", CSRC, str(at / "place.cpp"), "-o", str(at / "place.so")], check=True)
-    call = ctypes.CDLL(str(at / "place.so")).place
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-O2", "-I", CSRC, str(at / "place.cpp"), "-o", str(at / "place.so")], check=True)
+    lib = ctypes.CDLL(str(at / "place.so"))
+    call = lib.place
     call.argtypes = [ctypes.c_long] * 3 + [ctypes.c_int, ctypes.c_void_p]
 
     def table(xtiles, planes, seqs):
@@ -35,6 +56,12 @@ def place(tmp_path_factory):
         blocks = call(xtiles, planes, seqs, most, out.ctypes.data)
         assert 0 < blocks <= most
         return out[:blocks]
+
+    def limits(xtiles, planes, seqs):
+        out = (ctypes.c_long * 4)()
+        lib.limits(ctypes.c_long(xtiles), ctypes.c_long(planes), ctypes.c_long(seqs), out)
+        return list(out)
+    table.limits = limits
     return table
 
 
@@ -51,3 +78,13 @@ def test_every_tile_once_and_every_xcd_its_share(place, planes):
             load = np.bincount(xcd[used], weights=tile + 1, minlength=8)       # a tile's keys grow with its place
             if len(where) >= 8 * 32:                                        # enough for the kinds of tiles to come out even
                 assert load.max() <= 1.1 * load.mean(), (xtiles, seqs, load)
+
+
+def test_a_grid_of_many_workgroups(place):
+    """2^23 workgroups of 512 threads and more, which one dimension of a launch does not hold."""
+    places = place.limits
+    for xtiles, planes, seqs in ((683, 8, 2000), (1366, 3, 3000), (1, 1, 1 << 22), (100000, 8, 100)):
+        blocks, x, y, beyond = places(xtiles, planes, seqs)
+        assert blocks >= xtiles * planes * seqs and x * 512 < 1 << 32 and y <= 65535 and x * y >= blocks and x % 8 == 0
+        assert beyond == 0
+    assert places(1 << 20, 8, 1 << 12)[0] == 0

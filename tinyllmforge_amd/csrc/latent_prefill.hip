@@ -68,7 +68,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
   using Core = PromptCore<DC, VC, CT>;
   __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
   int sq, h, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, sq, h, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, h, xt)) return;
   const LatentShape &s = p.s;
   const int seq = p.first_seq + sq;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int CT = 2, kPQ = 64 * CT, DP = DC * 32, VP = VC * 32;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kPK][DP + 8], Vs[kPK][VP + 16];
   int sq, h, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, sq, h, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, h, xt)) return;
   const LatentShape &s = p.s;
   const int seq = p.first_seq + sq;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -418,8 +418,9 @@ extern "C" int tlf_latent_prefill(const void *q, const void *expanded, int64_t e
   a.q_keep = scale == 0.f ? 0u : ~0u; a.q_flip = scale < 0.f ? 0x80008000u : 0u;
   const int dc = fit_units(a.s.Dq / 32), vc = (vdim + 31) / 32;
   constexpr int rows = 128;
-  const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + rows - 1) / rows, heads, num_seqs));
-  if (!grid.x) return TLF_E_SHAPE;
+  const int blocks = prompt_tiles_make(a.tiles, (max_tokens + rows - 1) / rows, heads, num_seqs);
+  const dim3 grid = prompt_grid<dim3>(blocks);
+  if (!blocks) return TLF_E_SHAPE;
   hipStream_t st = static_cast<hipStream_t>(stream);
 #define TLF_LP(DC, VC) TLF_LAUNCH((latent_prefill_kernel<DC, VC>), grid, dim3(256), 0, st, a)
 #define TLF_LW(DC, VC) TLF_LAUNCH((latent_prefill_wide_kernel<DC, VC>), grid, dim3(256), 0, st, a)

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   using Core = PromptCore<DC, DC, CT>;
   __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
   int sq, plane, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
   const PooledCache &c = p.c;
   const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int DP = DC * 32, NCH = DC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kTK][DP + 8], Vs[kTK][DP + 16];
   int sq, plane, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
   const PooledCache &c = p.c;
   const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -370,8 +370,9 @@ extern "C" int tlf_pooled_attn_prefill(const void *q, const void *score_bias, co
   a.hpp = a.group < units ? a.group : units;
   a.passes = (a.group + a.hpp - 1) / a.hpp;
   a.bq = units / a.hpp;
-  const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, num_kv_heads * a.passes, num_seqs));
-  if (!grid.x) return TLF_E_SHAPE;
+  const int blocks = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, num_kv_heads * a.passes, num_seqs);
+  const dim3 grid = prompt_grid<dim3>(blocks);
+  if (!blocks) return TLF_E_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dc) {
     case 1: TLF_LAUNCH((pooled_prefill_kernel<1>), grid, dim3(256), 0, s, a); break;

@@ -169,7 +169,7 @@ void prefill_attn_kernel(const PrefillParams p) {
   __shared__ __attribute__((aligned(16))) unsigned short Vs[kBKV][kPRowV];  // fp16 (bf16 for a tile fp16 cannot hold)
   __shared__ __attribute__((aligned(16))) unsigned int vvote[8];            // per wave: what its V slice holds
   int seq, h, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, seq, h, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), seq, h, xt)) return;
   const int group = p.num_q_heads / p.num_kv_heads;
   const int bq = (16 * NWV * CT) / group;  // query rows per workgroup
   const int row0 = xt * bq;
@@ -546,8 +546,9 @@ extern "C" int tlf_varlen_prefill_attn(const void *q, int64_t q_stride, const vo
   const int nwv = forced ? forced : 8;
   const int ct = nwv == 8 ? 3 : 2;
   const int bq = (16 * nwv * ct) / group;
-  const dim3 grid(prompt_tiles_make(p.tiles, (max_seqlen_q + bq - 1) / bq, num_kv_heads, num_seqs));
-  if (!grid.x) return TLF_E_SHAPE;
+  const int blocks = prompt_tiles_make(p.tiles, (max_seqlen_q + bq - 1) / bq, num_kv_heads, num_seqs);
+  const dim3 grid = prompt_grid<dim3>(blocks);
+  if (!blocks) return TLF_E_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (paged && kv_dtype == TLF_KV_FP8_E4M3) {
     // the K scale is a per-head constant of the scores: fold it in on the device side per head

@@ -42,10 +42,20 @@ inline int prompt_tiles_make(PromptTiles &t, int64_t xtiles, int64_t planes, int
   return static_cast<int>(per_part * per_xcd * 8);
 }
 
+// The grid, in rows of 2^20: a dimension of a launch holds less than 2^32 threads, 2^23 workgroups of 512.
+constexpr int kPromptRow = 1 << 20;
+template <class Dim3>
+Dim3 prompt_grid(int blocks) {
+  return blocks <= kPromptRow ? Dim3(blocks) : Dim3(kPromptRow, (blocks + kPromptRow - 1) / kPromptRow);
+}
+__host__ __device__ inline int prompt_block(unsigned int x, unsigned int y) { return static_cast<int>(y * kPromptRow + x); }
+
 // False: nothing to do.
 __host__ __device__ inline bool prompt_tile(const PromptTiles &t, int block, int &seq, int &plane, int &xt) {
   constexpr int kTogether = 4;
-  const int i = block >> 3, first = i / (kTogether * t.per_part) * kTogether;
+  const int i = block >> 3;
+  if (i >= t.per_part * t.per_xcd) return false;
+  const int first = i / (kTogether * t.per_part) * kTogether;
   const int together = t.per_xcd - first < kTogether ? t.per_xcd - first : kTogether, within = i - first * t.per_part;
   const int step = within / together, part = (first + (within + step) % together) * 8 + (block & 7), of_seq = t.planes * t.parts;
   seq = part / of_seq;

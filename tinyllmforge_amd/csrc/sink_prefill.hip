@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   using Core = PromptCore<DC, VC, CT>;
   __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
   int sq, plane, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
   const SinkCache &c = p.c;
   const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int DP = DC * 32, VP = VC * 32, KCH = DC * 4, VCH = VC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[kSK][DP + 8], Vs[kSK][VP + 16];
   int sq, plane, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
   const SinkCache &c = p.c;
   const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -447,8 +447,9 @@ extern "C" int tlf_sink_attn_prefill(const void *q, const void *k_cache, const v
   a.passes = (a.group + a.hpp - 1) / a.hpp;
   a.bq = units / a.hpp;
   a.first_seq = first_seq; a.table_cols = static_cast<int32_t>(bt_stride);
-  const dim3 grid(prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, kv_heads * a.passes, num_seqs));
-  if (!grid.x) return TLF_E_SHAPE;
+  const int blocks = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, kv_heads * a.passes, num_seqs);
+  const dim3 grid = prompt_grid<dim3>(blocks);
+  if (!blocks) return TLF_E_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define TLF_SP(...)                                                                     \
   do {                                                                                  \

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
   constexpr int DP = DC * 32, KCH = DC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[2][kTS][DP + 8];
   int sq, plane, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
   const SinkCache &c = p.c;
   const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
   extern __shared__ __attribute__((aligned(1024))) unsigned short lds[];
   unsigned short *Vs = lds, *Wh = lds + p.c.G * kTK * VP, *Wl = Wh + TQ * ROW, *Ts = Wl + TQ * ROW;    // Vs [G][32][VP], Ts [16 HT][TS]
   int sq, plane, xt;
-  if (!prompt_tile(p.tiles, blockIdx.x, sq, plane, xt)) return;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
   const SinkCache &c = p.c;
   const int seq = p.first_seq + sq;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -473,9 +473,9 @@ int launch_talk_stats(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStrea
   a.hpp = a.group < kUnits ? a.group : kUnits;
   a.passes = (a.group + a.hpp - 1) / a.hpp;
   a.bq = kUnits / a.hpp;
-  const int grid = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, a.c.G * a.passes, num_seqs);
-  if (!grid) return TLF_E_SHAPE;
-  TLF_LAUNCH((talk_stats_kernel<DC, CT>), dim3(grid), dim3(256), 0, s, a);
+  const int blocks = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, a.c.G * a.passes, num_seqs);
+  if (!blocks) return TLF_E_SHAPE;
+  TLF_LAUNCH((talk_stats_kernel<DC, CT>), prompt_grid<dim3>(blocks), dim3(256), 0, s, a);
   return launch_status();
 }
 
@@ -484,9 +484,9 @@ int launch_talk_prefill(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStr
   static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&talk_prefill_kernel<WV, RT, DC, VC, GS>),
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, kTalkLds);
   if (allowed != hipSuccess) return static_cast<int>(allowed);
-  const int grid = prompt_tiles_make(a.tiles, (max_tokens + RT * 16 - 1) / (RT * 16), 1, num_seqs);
-  if (!grid) return TLF_E_SHAPE;
-  TLF_LAUNCH((talk_prefill_kernel<WV, RT, DC, VC, GS>), dim3(grid), dim3(WV * RT * 64), talk_prefill_lds(WV, RT, a.c.G, a.c.Vp), s, a);
+  const int blocks = prompt_tiles_make(a.tiles, (max_tokens + RT * 16 - 1) / (RT * 16), 1, num_seqs);
+  if (!blocks) return TLF_E_SHAPE;
+  TLF_LAUNCH((talk_prefill_kernel<WV, RT, DC, VC, GS>), prompt_grid<dim3>(blocks), dim3(WV * RT * 64), talk_prefill_lds(WV, RT, a.c.G, a.c.Vp), s, a);
   return launch_status();
 }
 template <int WV, int RT>
