@@ -99,3 +99,11 @@ def test_a_value_without_a_number_reaches_no_earlier_chunk(dk, dv, token):
         proj[token, 2 * H * dk:2 * H * dk + H * dv] = value
         got, first = run(), token // 16 * 16
         assert torch.equal(got[:first], want[:first]) and not got[token:].isfinite().any()
+
+
+@pytest.mark.parametrize("dk,dv", [(48, 40), (100, 32), (256, 64)])
+@pytest.mark.parametrize("tau", [16.0, 0.25])
+def test_other_sizes_in_chunks_of_16_tokens(dk, dv, tau):
+    lens = [1, 15, 16, 17, 31, 33, 200]
+    for n, out, state in run(2, dk, dv, 16, lens, [5 * (i % 2) for i in range(len(lens))], tau, dk + dv):
+        assert out < OUT and state < STATE, (n, out, state)

@@ -223,18 +223,33 @@ __global__ __launch_bounds__(256) void gla_chunk_kernel(const GlaArgs a) {
     }
   }
   __syncthreads();
+  const int64_t ch = static_cast<int64_t>(chunk) * a.H + h;
+  // operand order of the scan: Qd [tile][t][16 channels], Kd [tile][channel][16 tokens]
+  float *qd = a.rec + ch * GlaRec<DKP>::kSize, *kd = qd + GlaRec<DKP>::kKd;
   if (tid < DKP) {
-    float b = 0.f;
+    float la[kGC], b = 0.f;
 #pragma unroll
-    for (int s = 0; s < kGC; ++s) bs[s][tid] = b += bs[s][tid];
+    for (int s = 0; s < kGC; ++s) {
+      la[s] = bs[s][tid];
+      bs[s][tid] = b += la[s];
+    }
+    // sums towards the end on their own: as differences they would lose what the tokens before have decayed by
+    float after = 0.f;
+#pragma unroll
+    for (int s = kGC - 4; s >= 0; s -= 4) {
+      float k[4];
+#pragma unroll
+      for (int e = 3; e >= 0; --e) {
+        k[e] = ks[s + e][tid] * __builtin_amdgcn_exp2f(after);
+        after += la[s + e];
+      }
+      *reinterpret_cast<float4 *>(kd + tid * kGC + s) = make_float4(k[0], k[1], k[2], k[3]);
+    }
   }
   __syncthreads();
-  const int64_t ch = static_cast<int64_t>(chunk) * a.H + h;
   float bt[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i) bt[i] = bs[t][dmap(i)];
-  // operand order of the scan: Qd [tile][t][16 channels], Kd [tile][channel][16 tokens]
-  float *qd = a.rec + ch * GlaRec<DKP>::kSize, *kd = qd + GlaRec<DKP>::kKd;
   if constexpr (NT % 4 == 0) {
 #pragma unroll
     for (int i = 0; i < NT; i += 4) {
@@ -249,10 +264,6 @@ __global__ __launch_bounds__(256) void gla_chunk_kernel(const GlaArgs a) {
       const int d = dmap(i);
       qd[(d / 16) * 256 + t * 16 + d % 16] = q[i] * __builtin_amdgcn_exp2f(bt[i]);
     }
-  }
-  for (int i = tid; i < DKP * kGC; i += 256) {
-    const int d = i / kGC, s = i % kGC;
-    kd[i] = ks[s][d] * __builtin_amdgcn_exp2f(bs[kGC - 1][d] - bs[s][d]);
   }
   if (tid < DKP) qd[GlaRec<DKP>::kDec + tid] = __builtin_amdgcn_exp2f(bs[kGC - 1][tid]);
   // A[t, s].  For t >= 8 > s the factors 2^(b_t - b_7) and 2^(b_7 - b_s) are both <= 1 and the product needs no exponential
