@@ -299,6 +299,19 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     assert lib.tlf_f32_gemm(a, 8, a, a, 2, 4, 16, None) == -2 and lib.tlf_f32_argmax(a, 4, a, 1, 8, None) == -2
 
 
+def test_narrow_values_take_chunks_of_16_tokens():
+    """Their workspace is the chunks' alone: a record of 16 tokens, padded by 64 numbers, and 16 rows of the result for every chunk and
+    head.  Blocks of 32 tokens need more for every wider size."""
+    from tinyllmforge_amd import _lib
+    nbytes, (chunks, heads) = _lib.load().tlf_gla_portions_workspace_bytes, (512, 64)
+    chunked = lambda dk, dv: 4 * chunks * heads * (2 * 16 * dk + 256 + dk + 64 + 16 * dv)
+    for dk, narrow, wide in ((128, (32, 64), (96, 128)), (64, (32,), (64,)), (32, (32,), (64,))):
+        for dv in narrow:
+            assert nbytes(chunks * 16, chunks, 8, heads, dk, dv) == chunked(dk, dv), (dk, dv)
+        for dv in wide:
+            assert nbytes(chunks * 16, chunks, 8, heads, dk, dv) > chunked(dk, dv), (dk, dv)
+
+
 def test_interleaved_table_is_exact_to_fp32():
     from tinyllmforge_amd.layers.rotary_embedding import rotation_table
     t = rotation_table(6, 5000, 10000.0)

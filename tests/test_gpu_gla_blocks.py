@@ -1,5 +1,5 @@
-"""Gated linear attention over blocks of 32 tokens: lengths around the edges of chunks and blocks, every width of key and value,
-several sequences and segments, channels that fade at once beside ones that last."""
+"""Gated linear attention over blocks of 32 tokens, and over chunks of 16 where values are narrow: lengths around the edges of chunks and
+blocks, every width of key and value, several sequences and segments, channels that fade at once beside ones that last."""
 import pytest
 import torch
 
@@ -55,7 +55,7 @@ def run(H, dk, dv, rank, lens, start, tau, seed, lost=None, scale=1.0):
 OUT, STATE = 2 ** -8, 2 ** -20
 
 
-@pytest.mark.parametrize("dk,dv", [(32, 32), (32, 256), (64, 96), (128, 64), (128, 256)])
+@pytest.mark.parametrize("dk,dv", [(32, 32), (32, 64), (32, 256), (64, 96), (128, 64), (128, 96), (128, 256)])
 @pytest.mark.parametrize("tau", [16.0, 0.25])
 def test_lengths_around_chunks_and_blocks(dk, dv, tau):
     lens = [1, 15, 16, 17, 31, 32, 33, 47, 49, 63, 64, 65]
@@ -63,9 +63,9 @@ def test_lengths_around_chunks_and_blocks(dk, dv, tau):
         assert out < OUT and state < STATE, (n, out, state)
 
 
-@pytest.mark.parametrize("dk,rank,lens", [(128, 8, [2100]), (64, 64, [1500, 700, 33]), (32, 24, [513, 2000])])
-def test_segments_of_whole_blocks(dk, rank, lens):
-    for n, out, state in run(1, dk, 64, rank, lens, [0] + [3] * (len(lens) - 1), 8.0, dk):
+@pytest.mark.parametrize("dk,dv,rank,lens", [(128, 64, 8, [2100]), (128, 96, 8, [2100]), (64, 64, 64, [1500, 700, 33]), (32, 64, 24, [513, 2000])])
+def test_segments_of_whole_blocks(dk, dv, rank, lens):
+    for n, out, state in run(1, dk, dv, rank, lens, [0] + [3] * (len(lens) - 1), 8.0, dk):
         assert out < OUT and state < STATE, (n, out, state)
 
 
@@ -74,13 +74,14 @@ def test_keys_that_leave_no_room_for_growing_powers():
         assert out < OUT and state < STATE, (n, out, state)
 
 
+@pytest.mark.parametrize("dv", [64, 128])
 @pytest.mark.parametrize("lost", [0, 1, 2])
-def test_rows_of_another_sequence_are_not_touched(lost):
-    for n, out, state in run(2, 128, 64, 16, [17, 40, 50], [0, 5, 5], 16.0, lost, lost=lost):
+def test_rows_of_another_sequence_are_not_touched(lost, dv):
+    for n, out, state in run(2, 128, dv, 16, [17, 40, 50], [0, 5, 5], 16.0, lost, lost=lost):
         assert out < OUT and state < STATE, (n, out, state)
 
 
-@pytest.mark.parametrize("dk,dv", [(32, 32), (64, 128), (128, 256)])
+@pytest.mark.parametrize("dk,dv", [(32, 64), (64, 128), (128, 32), (128, 256)])
 @pytest.mark.parametrize("token", [16, 20, 31, 50])
 def test_a_value_without_a_number_reaches_no_earlier_chunk(dk, dv, token):
     """Sixteen tokens are a chunk; an earlier token meets values behind it as zeros times them."""

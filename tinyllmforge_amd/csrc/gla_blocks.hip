@@ -486,7 +486,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int r = 0; r < 16; ++r) dst[static_cast<int64_t>(i * 32 + (r >> 2) * 8 + hi * 4 + (r & 3)) * a.dv + col] = S[i][r];
 }
 
-bool gla_blocks_sizes(int32_t dk, int32_t dv) { return (dk == 32 || dk == 64 || dk == 128) && dv % 32 == 0 && dv >= 32 && dv <= 256; }
+// A workgroup of the scan has a wave per 32 value columns and holds two records, 117 KB with 128 keys: with fewer than three waves there, or
+// two otherwise, a CU has too few to hide their latencies, and the 16-token chunks are faster.  8 heads, 16-token chunks / blocks, us, at
+// 64 x 128, 8 x 300 and 8 x 2048 tokens: 128 x 32 90 / 118, 68 / 81, 231 / 288, 128 x 64 99 / 118, 69 / 71, 268 / 278, 128 x 96 128 / 118,
+// 68 / 68, 345 / 283; 64 x 32 66 / 69, 49 / 54, 137 / 142, 64 x 64 71 / 73, 50 / 49, 152 / 151; 32 x 32 55 / 52, 36 / 42, 111 / 105 (1 x 1500
+// 50 / 53).
+bool gla_blocks_sizes(int32_t dk, int32_t dv) {
+  return (dk == 32 || dk == 64 || dk == 128) && dv % 32 == 0 && dv >= (dk == 128 ? 96 : 64) && dv <= 256;
+}
 
 bool gla_blocks_take(const GlaArgs &a, int32_t dtype) {
   return dtype == TLF_DT_BF16 && gla_blocks_sizes(a.dk, a.dv) && a.R <= kGlaBlockMaxR && a.ld % 8 == 0 && a.ld < (1 << 24) && a.ldo % 4 == 0 && aligned16(a.proj) &&
