@@ -384,3 +384,15 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     lat = lambda halves=1, q=None, cache=a, cq=a, cqn=a, stride=64, gate=a, ld=80, dt=0, sizes=(3, 11, 6, 21, 9): lib.tlf_latent_prep(
         a, ld, None, 1, None, 17, a, a, a, 10, halves, a, 99, q, cache, 0, 17, cqn, cq, stride, 44, gate, 2, *sizes, 1e-6, dt, None)
     assert lat(cache=None) == NULL and lat(cq=None) == NULL and lat(stride=16) == SHAPE and lat(ld=40) == SHAPE and lat(dt=9) == TYPE
+
+
+@pytest.mark.parametrize("sizes,seqs,tokens,segments", [((32, 64, 128, 1), 1, 2000, 8), ((32, 64, 128, 1), 1, 4000, 16), ((32, 64, 128, 1), 6, 520, 1),
+                                                        ((16, 64, 128, 1), 1, 4000, 15), ((32, 64, 64, 1), 1, 1500, 12), ((128, 64, 128, 8), 4, 3000, 4)])
+def test_few_state_space_groups_keep_a_head_per_workgroup(sizes, seqs, tokens, segments):
+    """Their segments are of at least four chunks, so there are fewer of them than the heads of a group together would need; what a segment
+    leaves behind is in the workspace."""
+    from tinyllmforge_amd import _lib
+    (H, P, N, G), rows, up = sizes, seqs * tokens, lambda v: -(-v // 256) * 256
+    parts = seqs * segments * H if segments > 1 else 0
+    want = up(2 * rows * (H * P + 2 * G * N)) + 2 * up(4 * rows * H) + up(4 * parts) + up(4 * parts * N * P)
+    assert _lib.load().tlf_ssd_portions_workspace_bytes(rows, seqs, tokens, *sizes, 0) == want

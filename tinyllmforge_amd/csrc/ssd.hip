@@ -609,6 +609,17 @@ int ssd_segments(int64_t wgs, int max_tokens) {
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({want, most, 64})));
 }
 
+// Whether ssd_chunk_kernel does as well as ssd_group_kernel although heads share B and C: where its workgroups are all on the chip at
+// once and go through few chunks each, or through ten of a sequence without segments, while the other one needs segments.  Their number is
+// what costs it: each adds up all that lie before it, N rows of state apiece.  Layer, us, chunks / groups: 32 heads of 64, state 128, one
+// group, 1 x 1200 tokens 64 / 67, 1 x 2000 66 / 71, 1 x 3000 110 / 93 (more workgroups than CUs), 6 x 520 74 / 79, 4 x 600 79 / 68 (segments);
+// 16 heads 1 x 4000 75 / 95; state 64 1 x 1500 64 / 59, 2 groups of 8 heads 1 x 6000 77 / 114.
+bool ssd_chunks_suffice(int64_t wgs, int segs, int group_segs, int N, int max_tokens) {
+  const int chunks = (max_tokens + kSC - 1) / kSC, each = (chunks + segs - 1) / segs;
+  if (group_segs <= 1 || wgs * segs > 268) return false;
+  return (segs == 1 && chunks <= 10) || each * 128 < group_segs * N * 13 / 20;
+}
+
 struct SsdPlan {
   bool chunked;
   int pt, slices, segs;
@@ -627,6 +638,7 @@ SsdPlan ssd_plan(int rows, int seqs, int max_tokens, int H, int P, int N, int G,
   p.xbc = up(item * rows * (static_cast<size_t>(H) * P + 2 * static_cast<size_t>(G) * N));
   p.steps = up(4 * static_cast<size_t>(rows) * H);
   p.group_segs = ssd_groups_segments(H, P, N, G, seqs, max_tokens, dtype);
+  if (ssd_chunks_suffice(static_cast<int64_t>(H) * p.slices * seqs, p.segs, p.group_segs, N, max_tokens)) p.group_segs = 0;
   const int most = std::max(p.segs, p.group_segs);
   const size_t sg = most > 1 ? static_cast<size_t>(seqs) * most * H : 0;
   p.seg_decay = up(4 * sg);

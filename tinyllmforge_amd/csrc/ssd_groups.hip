@@ -353,7 +353,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // A workgroup has the work of up to eight waves, so there are fewer of them than of ssd_chunk_kernel's, and short sequences have to be many:
 // with 8 chunks it is faster with segments (1 x 700 tokens, 32 or 128 heads: 56 -> 47 us, 69 -> 57; 1 x 3000: 100 -> 74, 225 -> 167), with 4
 // once the chip is full (8 x 200, 128 heads: 116 -> 64), not below that (2 x 300: 42 -> 52).  Segments: two workgroups per CU, one after the
-// other, even out the sequences where they keep 6 chunks; else one per CU, of at least 2 (1 x 1500: 8 segments 77 us, 6 83, 12 98).
+// other, even out the sequences where they keep 6 chunks; else one per CU, of at least 2 (1 x 1500: 8 segments 77 us, 6 83, 12 98).  Where many
+// segments would have to make up for few groups, ssd.hip: ssd_chunks_suffice keeps a head per workgroup.
 int ssd_groups_segments(int H, int P, int N, int G, int seqs, int max_tokens, int dtype) {
   const int64_t channels = static_cast<int64_t>(H) * P + 2ll * G * N, units = static_cast<int64_t>(H / G) * (P / 32);
   if (dtype != TLF_DT_BF16 || (N != 32 && N != 64 && N != 128) || P % 32 || units < 4 || channels % 8 || channels >= (1 << 24)) return 0;
