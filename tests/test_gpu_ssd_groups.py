@@ -44,6 +44,29 @@ def test_segments(sizes, lens):
             assert rel(got[s][-50:], want[s][-50:]) < 8e-3, (first, s)
 
 
+@pytest.mark.parametrize("sizes", [(24, 64, 128, 8, 4), (32, 32, 64, 8, 3), (64, 96, 32, 16, 4)])
+def test_portions_behind_single_tokens(sizes):
+    """A step's single tokens come first: portions begin at rows and sequences of their own, in the inputs and behind the convolution.
+    The last step's tokens see the states that the portions left (a row alone: errors that do not average out)."""
+    steps = [[50, 1, 2, 64, 1, 65], [13, 1, 63, 1, 70, 1], [1, 1, 1, 1, 1, 1]]
+    lens = [sum(x) for x in zip(*steps)]
+    proj, w, want = ssd_case(sizes, lens, BF, sum(sizes), 0.0, -1.5)
+    times = copies(sizes, 3)
+    got = run_ssd(sizes, proj * times, w, [x * times for x in steps], BF, list(range(1, 6 * times + 1)))
+    for s in list(range(6)) + list(range(6 * times - 6, 6 * times)):
+        assert rel(got[s], want[s % 6]) < TOL and rel(got[s][-1], want[s % 6][-1]) < 2 * TOL, (s, rel(got[s], want[s % 6]))
+
+
+@pytest.mark.parametrize("sizes", [(64, 32, 128, 8, 4), (64, 64, 64, 8, 4)])
+def test_segments_behind_single_tokens(sizes):
+    steps = [[700, 1, 100, 1], [800, 1, 200, 1], [1, 1, 1, 1]]
+    lens = [sum(x) for x in zip(*steps)]
+    proj, w, want = ssd_case(sizes, lens, BF, 7, decay=-5.0, step=-3.0)
+    got = run_ssd(sizes, proj, w, steps, BF, [3, 0, 2, 1])
+    for s in range(4):
+        assert rel(got[s], want[s]) < TOL and rel(got[s][-1], want[s][-1]) < 2 * TOL, s
+
+
 @pytest.mark.parametrize("state_dim", [32, 64, 128])
 def test_the_state_is_summed_in_single_precision(state_dim):
     """Sums of three tokens, whose factors no rounding to bfloat16 touches: x, B and C pass the convolution and SiLU as they are, and
