@@ -170,15 +170,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
 #pragma unroll
           for (int j = 1; j < 8; ++j) y = fmaxf(y, sc[j >> 2][k][j & 3]);
           y *= p.scale_log2;
-          x[k] = part.start && hf == 1 ? fmaxf(x[k], y) : y;     // the first maximum is that of the whole first tile
+          x[k] = part.start && (hf & 1) ? fmaxf(x[k], y) : y;     // the first maximum is that of the whole first tile
         }
       },
-      [&](int hf, typename Core::Scores &, typename Core::Weights &w) __attribute__((always_inline)) {
+      [&](int hf, typename Core::Scores &, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
         bool grown = false;
 #pragma unroll
         for (int k = 0; k < CT; ++k) grown = grown || x[k] > over[k];
         if (!__any(grown)) return;
-        if (hf > 0) core.add_values(hf - 1, w);
+        if (!part.start) core.add_values(hf - 1, w);
 #pragma unroll
         for (int k = 0; k < CT; ++k) {                       // sums and accumulators to the new maximum
           const float most = fmaxf(m[k], max_lanes_16_32_48(x[k]));

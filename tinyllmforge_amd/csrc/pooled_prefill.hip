@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
       tiles, 0, tiles, ptiles + edge, min(tiles, ptiles + max(0, (i_first + 1 - w0) / kTK)),
       copy_k, copy_v,
       [](float (&f)[CT]) __attribute__((always_inline)) { f[0] = f[1] = 0.f; }, [](int, typename Core::Scores &, auto) __attribute__((always_inline)) {},
-      [](int, typename Core::Scores &, typename Core::Weights &) __attribute__((always_inline)) {},
+      [](int, typename Core::Scores &, typename Core::Weights &, auto) __attribute__((always_inline)) {},
       [&](int h, const typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < CT; ++k) {

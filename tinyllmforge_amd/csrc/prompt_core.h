@@ -139,7 +139,8 @@ struct PromptCore {
   //   copy_k(t, part), copy_v     the tile's copies; called for t = 0, 1, .. in turn
   //   from(f)                     where a unit's scores begin (read once per half)
   //   finish(h, s, part)          what is done to the scores of half h as soon as they are there
-  //   before(h, s, w)             ahead of the weights of half h; `w`: weights of half h - 1 whose values are not added yet (add_values)
+  //   before(h, s, w, part)       ahead of the weights of half h; `w`: weights of half h - 1 whose values are not added yet (add_values),
+  //                               none with part.start, which is set in the wave's first half
   //   weights(h, s, w, part)
   // part.mask is not set where all keys of the half's tile are seen by all units: tiles clear_from <= t < clear_to of them (wave
   // uniform), clear_from 0 without LEAD.  part.lead is set where t may be below clear_from, part.start in the wave's first tile.
@@ -174,12 +175,12 @@ struct PromptCore {
     read_k(2 * t);
     make_scores(se);
     finish(2 * t, se, first);
-    if constexpr (!BOTH) before(2 * t, se, wo);
+    if constexpr (!BOTH) before(2 * t, se, wo, first);
     read_k(2 * t + 1);
     make_scores(so);
     if constexpr (BOTH) {
       finish(2 * t + 1, so, first);
-      before(2 * t, se, wo);
+      before(2 * t, se, wo, first);
     }
     weights(2 * t, se, we, first);
     if constexpr (!BOTH) finish(2 * t + 1, so, first);
@@ -188,14 +189,14 @@ struct PromptCore {
       TLF_DL_BARRIER(0);
       copy_v(t + 1, part);
       if (t + 2 < tiles) copy_k(t + 2, part);
-      before(2 * t + 1, so, we);
+      before(2 * t + 1, so, we, part);
       read_k(2 * t + 2);
       read_v(2 * t);
       make_scores(se);
       weights(2 * t + 1, so, wo, part);
       values(we);
       finish(2 * t + 2, se, part);
-      before(2 * t + 2, se, wo);
+      before(2 * t + 2, se, wo, part);
       read_k(2 * t + 3);
       read_v(2 * t + 1);
       make_scores(so);
@@ -214,7 +215,7 @@ struct PromptCore {
       TLF_DL_BARRIER(0);
       t = tiles - 1;
     }
-    before(2 * t + 1, so, we);
+    before(2 * t + 1, so, we, tail);
     weights(2 * t + 1, so, wo, first);
     read_v(2 * t);
     values(we);

@@ -188,13 +188,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
           }
         }
       },
-      [&](int h, typename Core::Scores &s, typename Core::Weights &w) __attribute__((always_inline)) {
+      [&](int h, typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
         if constexpr (MODE != 2) {
           bool grown = false;
 #pragma unroll
           for (int k = 0; k < CT; ++k) grown = grown || x[k] > over[k];
           if (!__any(grown)) return;
-          if (h > 0) core.add_values(h - 1, w);
+          if (!part.start) core.add_values(h - 1, w);
 #pragma unroll
           for (int k = 0; k < CT; ++k) {                     // sums, accumulators and scores to the new maximum
             const float most = max_lanes_16_32_48(x[k]), base = MODE == 0 && m[k] != -INFINITY ? m[k] : 0.f;
