@@ -13,7 +13,7 @@ def plain(q, k, v):
     """``q [T, H, D]``, ``k, v [T, G, D]``: causal softmax attention in fp32, on the host."""
     q, k, v = q.float().cpu(), k.float().cpu(), v.float().cpu()
     T, H = q.shape[:2]
-    out = torch.empty(q.shape)
+    out = torch.empty(T, H, v.shape[2])
     for h in range(H):
         s = q[:, h] @ k[:, h * k.shape[1] // H].T
         w = torch.softmax(s.masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), -torch.inf), dim=-1)
@@ -82,6 +82,28 @@ def test_weights_follow_a_growing_maximum(dim, vdim, cap):
     want = torch.einsum("hij,jd->ihd", torch.softmax(s, -1), v.double())
     # bf16 result (2^-9) of weights with 16 significant bits and fp32 scores of up to 2^8
     torch.testing.assert_close(out.view(new, heads, vdim).double().cpu(), want, rtol=2 ** -8, atol=2 ** -10)
+
+
+@pytest.mark.parametrize("lens", [(1,), (128,), (128, 5, 77), (100,) * 9, (129, 128, 3)], ids=str)
+@pytest.mark.parametrize("dim,rot,vdim", [(64, 32, 64), (128, 64, 128)])
+@pytest.mark.parametrize("heads", [3, 16])
+def test_latent_portions_of_one_row_tile(lens, dim, rot, vdim, heads):
+    """Up to 128 tokens the heads of a portion are dealt like row tiles."""
+    torch.manual_seed(sum(lens))
+    dev, BF, n = "cuda", torch.bfloat16, sum(lens)
+    s = ops.LatentShape(heads, dim, rot, 64, vdim)
+    q, turned = torch.randn(n, heads, dim + rot).to(BF), torch.randn(n, rot).to(BF)
+    k, v = torch.randn(n, heads, dim).to(BF), torch.randn(n, heads, vdim).to(BF)
+    latents = torch.zeros(n, s.lp, dtype=BF)
+    latents[:, 64:64 + rot] = turned
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0)], dtype=torch.int32, device=dev)
+    out = torch.full((n, heads * vdim), torch.nan, device=dev, dtype=BF)
+    scale = (dim + rot) ** -0.5
+    ops.latent_prefill(q.to(dev), torch.cat([k.flatten(1), v.flatten(1)], 1).to(dev), latents.to(dev), cu, torch.zeros_like(cu), cu, 0, len(lens), max(lens),
+                       1 << 20, scale, s, out)
+    keys = torch.cat([k, turned[:, None].expand(-1, heads, -1)], 2)
+    want = torch.cat([plain(q[a:b].float() * scale, keys[a:b], v[a:b]) for a, b in zip(cu.tolist(), cu.tolist()[1:])])
+    torch.testing.assert_close(out.float().cpu().view(want.shape), want, rtol=2 ** -8, atol=2 ** -8)
 
 
 # A value that is infinite or no number belongs to the rows that see its key: weights of zero times it are no numbers.  Keys are taken in

@@ -11,9 +11,9 @@ SOURCE = """
 #define __host__
 #define __device__
 #include "prompt_tiles.h"
-extern "C" int place(long xtiles, long planes, long seqs, int most, int *out) {
+extern "C" int place(long xtiles, long planes, long seqs, int together, int most, int *out) {
   tlf::PromptTiles t;
-  const int blocks = tlf::prompt_tiles_make(t, xtiles, planes, seqs);
+  const int blocks = tlf::prompt_tiles_make(t, xtiles, planes, seqs, together);
   for (int b = 0; b < blocks && b < most; ++b)
     if (!tlf::prompt_tile(t, b, out[3 * b], out[3 * b + 1], out[3 * b + 2])) out[3 * b] = -1;
   return blocks;
@@ -48,12 +48,12 @@ def place(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-O2", "-I", CSRC, str(at / "place.cpp"), "-o", str(at / "place.so")], check=True)
     lib = ctypes.CDLL(str(at / "place.so"))
     call = lib.place
-    call.argtypes = [ctypes.c_long] * 3 + [ctypes.c_int, ctypes.c_void_p]
+    call.argtypes = [ctypes.c_long] * 3 + [ctypes.c_int] * 2 + [ctypes.c_void_p]
 
-    def table(xtiles, planes, seqs):
+    def table(xtiles, planes, seqs, together=4):
         most = 8 * (xtiles + 7) * planes * seqs
         out = np.full((most, 3), -1, dtype=np.int32)
-        blocks = call(xtiles, planes, seqs, most, out.ctypes.data)
+        blocks = call(xtiles, planes, seqs, together, most, out.ctypes.data)
         assert 0 < blocks <= most
         return out[:blocks]
 
@@ -69,7 +69,7 @@ def place(tmp_path_factory):
 def test_every_tile_once_and_every_xcd_its_share(place, planes):
     for xtiles in (1, 2, 3, 4, 7, 8, 9, 10, 16, 17, 33, 64):
         for seqs in (1, 2, 3, 8, 15, 16, 64, 100):
-            t = place(xtiles, planes, seqs)
+            t = place(xtiles, planes, seqs, 1 if seqs == 15 else 4)
             xcd, used = np.arange(len(t)) % 8, t[:, 0] >= 0
             seq, plane, tile = t[used].T
             assert seq.max() < seqs and plane.min() >= 0 and plane.max() < planes and tile.min() >= 0 and tile.max() < xtiles

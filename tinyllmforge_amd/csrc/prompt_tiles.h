@@ -16,7 +16,8 @@
 // An XCD takes its planes four at a time and walks their row tiles together, the last ones (the longest key ranges) first, so that
 // it ends on short workgroups while the planes at work still fit its L2 (4 x 1 MB at 2048 keys of 2 x 128 bf16).  The order of the
 // four turns by one from row tile to row tile: an XCD deals its workgroups to its four shader engines in turn as well, and without
-// the turn each engine gets all row tiles of one sequence, and the launch waits for the engine with the longest.
+// the turn each engine gets all row tiles of one sequence, and the launch waits for the engine with the longest.  (`together`: others
+// than four, where tiles of a plane share more than keys.)
 //
 // Eight prompts of 1061 to 2048 tokens, 32 heads on 8 KV heads (sink_prefill.hip): 521 us with either of the two mistakes, as long
 // as eight prompts of 2048; 355 us so.
@@ -27,18 +28,18 @@ namespace tlf {
 
 struct PromptTiles {
   int32_t xtiles, planes, parts, per_part;   // row tiles; planes of a sequence; parts of a plane, their tiles
-  int32_t all_parts, per_xcd;                // of all sequences; for an XCD, at most
+  int32_t all_parts, per_xcd, together;                // of all sequences; for an XCD, at most
 };
 
 // Workgroups to launch, 0: too many.
-inline int prompt_tiles_make(PromptTiles &t, int64_t xtiles, int64_t planes, int64_t seqs) {
+inline int prompt_tiles_make(PromptTiles &t, int64_t xtiles, int64_t planes, int64_t seqs, int together = 4) {
   int parts = 1;
   auto enough = [&](int64_t all) { return all >= 80 || (all >= 48 && all % 8 == 0); };
   while (parts < 8 && planes * parts % 8 && !enough(planes * parts * seqs)) parts *= 2;
   const int64_t most = 1 << 27, per_part = (xtiles + parts - 1) / parts, all_parts = planes * parts * seqs, per_xcd = (all_parts + 7) / 8;
   if (per_part > most || per_xcd > most || per_part * per_xcd > most) return 0;
   t = PromptTiles{static_cast<int32_t>(xtiles), static_cast<int32_t>(planes), parts, static_cast<int32_t>(per_part), static_cast<int32_t>(all_parts),
-                  static_cast<int32_t>(per_xcd)};
+                  static_cast<int32_t>(per_xcd), together};
   return static_cast<int>(per_part * per_xcd * 8);
 }
 
@@ -52,11 +53,10 @@ __host__ __device__ inline int prompt_block(unsigned int x, unsigned int y) { re
 
 // False: nothing to do.
 __host__ __device__ inline bool prompt_tile(const PromptTiles &t, int block, int &seq, int &plane, int &xt) {
-  constexpr int kTogether = 4;
   const int i = block >> 3;
   if (i >= t.per_part * t.per_xcd) return false;
-  const int first = i / (kTogether * t.per_part) * kTogether;
-  const int together = t.per_xcd - first < kTogether ? t.per_xcd - first : kTogether, within = i - first * t.per_part;
+  const int first = i / (t.together * t.per_part) * t.together;
+  const int together = t.per_xcd - first < t.together ? t.per_xcd - first : t.together, within = i - first * t.per_part;
   const int step = within / together, part = (first + (within + step) % together) * 8 + (block & 7), of_seq = t.planes * t.parts;
   seq = part / of_seq;
   plane = part % of_seq / t.parts;
