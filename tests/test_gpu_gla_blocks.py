@@ -86,7 +86,7 @@ def test_rows_of_another_sequence_are_not_touched(lost, dv):
 def test_a_value_without_a_number_reaches_no_earlier_chunk(dk, dv, token):
     """Sixteen tokens are a chunk; an earlier token meets values behind it as zeros times them."""
     from tinyllmforge_amd import ops as P
-    H, rank, n = 2, 16, 70
+    H, rank, n = 2, 16, 60
     g, dt = torch.Generator().manual_seed(token), torch.bfloat16
     proj = torch.randn(n, 2 * H * (dk + dv) + rank, generator=g).to(dt).cuda()
     a2, a2b, nw = (torch.randn(s, generator=g).to(dt).cuda() for s in ((H * dk, rank), (H * dk,), (dv,)))
@@ -108,3 +108,16 @@ def test_other_sizes_in_chunks_of_16_tokens(dk, dv, tau):
     lens = [1, 15, 16, 17, 31, 33, 200]
     for n, out, state in run(2, dk, dv, 16, lens, [5 * (i % 2) for i in range(len(lens))], tau, dk + dv):
         assert out < OUT and state < STATE, (n, out, state)
+
+
+@pytest.mark.parametrize("H,dk,dv,lens,kernels", [
+    (16, 128, 256, [64], 2), (16, 128, 256, [65], 3), (16, 128, 256, [400], 3), (16, 128, 256, [200] * 5, 2), (16, 128, 256, [600], 4),
+    (8, 64, 128, [200], 2), (8, 64, 128, [224, 209], 3), (8, 64, 128, [240] * 12, 2), (16, 128, 128, [500] * 8, 3)])
+def test_short_portions_keep_the_chunks(H, dk, dv, lens, kernels):
+    """Two kernels over blocks of 32 tokens, two more where there are segments; three over chunks of 16."""
+    from tinyllmforge_amd import _lib
+    count = _lib.load().tlf_kernel_launches
+    before = count()
+    for n, out, state in run(H, dk, dv, 16, lens, [5] * len(lens), 8.0, dk):
+        assert out < OUT and state < STATE, (n, out, state)
+    assert count() - before == kernels

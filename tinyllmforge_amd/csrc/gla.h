@@ -45,7 +45,7 @@ __device__ __forceinline__ float log2_alpha(float z, float inv_tau) {
 }
 
 // Prompt portions in blocks of 32 tokens (gla_blocks.hip): what it takes, its workspace, the launches.
-bool gla_blocks_take(const GlaArgs &a, int32_t dtype);
+bool gla_blocks_take(const GlaArgs &a, int32_t dtype, int chunk_segs);     // chunk_segs: segments the chunks would have
 bool gla_blocks_sizes(int32_t key_dim, int32_t value_dim);
 size_t gla_blocks_workspace_bytes(int32_t chunks, int32_t num_seqs, int32_t heads, int32_t key_dim, int32_t value_dim);
 int launch_gla_blocks(GlaArgs &a, int first_seq, void *workspace, hipStream_t stream);

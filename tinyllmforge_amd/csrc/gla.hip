@@ -666,7 +666,7 @@ extern "C" int tlf_gla_portions(const void *proj, int64_t proj_stride, const voi
   if (!workspace || !aligned16(workspace) ||
       workspace_bytes < tlf_gla_portions_workspace_bytes(rows, chunks, num_seqs, heads, key_dim, value_dim))
     return TLF_E_WORKSPACE;
-  if (gla_blocks_take(a, dtype)) return launch_gla_blocks(a, first_seq, workspace, static_cast<hipStream_t>(stream));
+  if (gla_blocks_take(a, dtype, gla_segments(chunks, num_seqs, heads, value_dim))) return launch_gla_blocks(a, first_seq, workspace, static_cast<hipStream_t>(stream));
   const size_t ch = static_cast<size_t>(chunks) * heads, dkp = gla_tiles(key_dim) * 16;
   a.rec = static_cast<float *>(workspace);
   a.o = a.rec + ch * gla_rec_size(static_cast<int>(dkp));

@@ -495,16 +495,31 @@ bool gla_blocks_sizes(int32_t dk, int32_t dv) {
   return (dk == 32 || dk == 64 || dk == 128) && dv % 32 == 0 && dv >= (dk == 128 ? 96 : 64) && dv <= 256;
 }
 
-bool gla_blocks_take(const GlaArgs &a, int32_t dtype) {
-  return dtype == TLF_DT_BF16 && gla_blocks_sizes(a.dk, a.dv) && a.R <= kGlaBlockMaxR && a.ld % 8 == 0 && a.ld < (1 << 24) && a.ldo % 4 == 0 && aligned16(a.proj) &&
-         (reinterpret_cast<uintptr_t>(a.out) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.norm_w) & 7) == 0;
-}
-
 // Segments per sequence: a workgroup for every CU (two where LDS holds two), segments of at least 8 blocks.
 int gla_block_segments(int chunks, int seqs, int heads, int dk) {
   const int64_t wgs = static_cast<int64_t>(seqs) * heads, full = dk == 128 ? 256 : 512, want = wgs >= full ? 1 : (full + wgs - 1) / wgs, most = chunks / seqs / 16;
   const int64_t s = want < most ? want : most;
   return static_cast<int>(s < 1 || seqs * s > 65535 ? 1 : s > 32 ? 32 : s);
+}
+
+// Whether the scan over 16-token chunks does as well: where its waves, one per 16 value columns, are all on the chip at once, in one segment,
+// and go through few chunks.  A block takes a workgroup of dv / 32 waves as long as it takes them for two and a half chunks (eight waves
+// wait at one barrier), so with wide values five chunks are enough to be faster, with narrower ones fourteen, and only where CUs are
+// idle; and a second segment is not worth its first pass there.  Layer, us, chunks / blocks: 16 heads of 128 x 256, 1 x 70 tokens 32 / 31,
+// 1 x 130 36 / 42, 1 x 400 65 / 90, 1 x 550 (two segments) 117 / 100, 4 x 130 46 / 51, 5 x 200 (1280 waves) 81 / 67, 4 x 500 95 / 127,
+// 4 x 1000 183 / 168; 8 of 64 x 128 1 x 130 31 / 27, 1 x 400 43 / 46, 12 x 400 (96 workgroups) 65 / 60; 16 of 128 x 128 8 x 500 118 / 143.
+bool gla_chunks_suffice(const GlaArgs &a, int chunk_segs) {
+  const int64_t wgs = static_cast<int64_t>(a.seqs) * a.H, waves = (a.dv + 15) / 16 * wgs;
+  const int each = (a.chunks + a.seqs - 1) / a.seqs;
+  if (waves > 1024 || chunk_segs > 1 || each > 40) return false;
+  if (a.dv > 128) return each >= 5;
+  return gla_block_segments(a.chunks, a.seqs, a.H, a.dk) > 1 || (wgs <= 64 && each >= 14);
+}
+
+bool gla_blocks_take(const GlaArgs &a, int32_t dtype, int chunk_segs) {
+  return dtype == TLF_DT_BF16 && gla_blocks_sizes(a.dk, a.dv) && a.R <= kGlaBlockMaxR && a.ld % 8 == 0 && a.ld < (1 << 24) && a.ldo % 4 == 0 && aligned16(a.proj) &&
+         (reinterpret_cast<uintptr_t>(a.out) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.norm_w) & 7) == 0 &&
+         !gla_chunks_suffice(a, chunk_segs);
 }
 
 size_t gla_blocks_workspace_bytes(int32_t chunks, int32_t seqs, int32_t heads, int32_t dk, int32_t dv) {

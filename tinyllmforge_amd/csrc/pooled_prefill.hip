@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   }
   const float nscale = -p.scale_log2;
 
-  const int nb = pooled_visible(i_last, c.size, c.pool), nb_first = pooled_visible(i_first, c.size, c.pool);
+  const int nb = pooled_visible(i_last, c.size, c.pool);
   const int ptiles = (nb + kTK - 1) / kTK;
   const int w0 = max(0, i_first - c.size + 1) / kTK * kTK;
   const int tiles = ptiles + (i_last - w0) / kTK + 1;
