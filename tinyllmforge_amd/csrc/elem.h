@@ -93,7 +93,8 @@ inline int partials_check(const void *partials, const float *scale, int32_t spli
 }
 
 __device__ __forceinline__ float sigmoid_f32(float z) { return 1.0f / (1.0f + expf(-z)); }
-// The same from the hardware's exponential and reciprocal, 4 instructions instead of 25; relative error below 2^-21 + |z| 2^-24.
+// The same from the hardware's exponential and reciprocal, 4 instructions instead of 25; relative error below 2^-21 + |z| 2^-24 from
+// z = -87 on (below that, where it is under 2^-125, the result may be zero).
 __device__ __forceinline__ float sigmoid_fast(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
 }

@@ -17,10 +17,11 @@
 //                          A value that is no number reaches no row before its half of a block
 // Where (sequences, heads) alone leave CUs idle a sequence is cut into segments as in gla.hip.
 //
-// Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256: chunk 122 + scan 470 (both passes) + norm and gate 92 us
-// over 16-token chunks with fp32 products; here blocks 148 + first pass 57 + segments 18 + scan 255 us.  The blocks write 55 KB a record,
-// 4 TB/s with what they read; the scan is held by its barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's
-// error against 64 bits falls from 1e-7 .. 3e-6 (with the decay) to 1e-7 or less, the output's is its rounding to bf16 on both.
+// Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256, medians under the profiler: chunk 122 + scan 470 (both
+// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 149 + first pass 62 + segments 19 + scan
+// 278 us (whole layer without it 614 and 449 us).  The blocks write 55 KB a record, 4 TB/s with what they read; the scan is held by its
+// barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's error against 64 bits is 5e-8 to 1.1e-7 on both, the
+// output's is its rounding to bf16.
 #include "gemm_shared.h"
 #include "gla.h"
 

@@ -9,7 +9,7 @@
 //                                 has grown is asked lane by lane; maxima of rows are only formed when one has, and all rows of the wave
 //                                 follow theirs then: a largest weight of 1 is not rounded
 // 16 heads of 96 and 64 dimensions, eight prompts of 1061 to 2048 tokens: layer 189 us with the stages of a tile one after the other and
-// a window of 1024, 173 so; three prompts up to 3000, causal, 208 and 185.
+// a window of 1024, 171 so; three prompts up to 3000, causal, 208 and 188.
 #include "latent_attn.h"
 #include "prompt_core.h"
 #include "prompt_tiles.h"

@@ -13,13 +13,13 @@
 //
 // A segment's contribution comes from a first pass over B and X (MODE 1); a segment adds up what lies before it as it starts.
 //
-// 128 heads of 64 in 8 groups, state 128, 4 sequences of up to 3000 tokens: 430 us with ssd_chunk_kernel, which forms G for every head and
-// passes S through LDS as pairs; here 218 + 83.  With the scaled X as pairs 209 + 68, but then 1 to 4 % more outputs than with
-// ssd_chunk_kernel missed their nearest bf16 value (1.3 in a thousand do; the state's error is 1.1e-6 to 2.4e-6, and 2e-7 to 8e-7 with pieces).  So a chunk of
-// 4 heads took 18700 cycles, 5000 of them products and 9200 vector instructions on each SIMD, the rest latency of two waves per SIMD (S alone
-// takes 64 registers).  16 columns per wave and four waves per SIMD were slower
-// (285 + 71: twice the reads of B and C, twice the weights), and so were copies issued in a row (+2300 cycles a chunk: a wave waits where
-// several are queued) and step sizes masked as they are loaded (+2200: that waits for them).
+// 128 heads of 64 in 8 groups, state 128, 4 sequences of up to 3000 tokens, medians under the profiler: 437 us with ssd_chunk_kernel, which
+// forms G for every head and passes S through LDS as pairs; here 254 + 95.  With the scaled X as pairs 249 + 81, but then 1 to 4 % more outputs
+// than with ssd_chunk_kernel missed their nearest bf16 value (1.3 in a thousand do; the state's error is 1.1e-6 to 2.6e-6 on both, and 2e-7
+// to 8e-7 with pieces).  With pairs a chunk of 4 heads took 18700 cycles, 5000 of them products and 9200 vector instructions on each SIMD, the
+// rest latency of two waves per SIMD (S alone takes 64 registers).  16 columns per wave and four waves per SIMD were slower (285 + 71, the
+// least of twelve, where this took 209 + 68: twice the reads of B and C, twice the weights), and so were copies issued in a row (+2300 cycles
+// a chunk: a wave waits where several are queued) and step sizes masked as they are loaded (+2200: that waits for them).
 #include <algorithm>
 
 #include "gemm_shared.h"
