@@ -177,6 +177,41 @@ def test_talking_heads_over_paged_rows(dtype, sizes):
         assert rel(out[lens[0]:, :H * V], want[lens[0]:]) < tol
 
 
+# (tokens before the portion, its tokens): one long portion, a few rows behind a long context, a tile's edges, nothing to cut, unequal ones
+CUTS = [[(0, 1500)], [(2048, 40)], [(0, 31), (0, 32), (0, 33), (96, 64), (95, 65)], [(0, 20), (64, 1)], [(0, 700), (128, 513), (0, 64), (1000, 2)]]
+
+
+@pytest.mark.parametrize("portions", CUTS, ids=str)
+@pytest.mark.parametrize("sizes", [(4, 2, 64, 64), (8, 8, 96, 40), (16, 8, 128, 128), (12, 12, 96, 80), (32, 8, 128, 128)], ids=str)
+def test_talking_heads_with_keys_cut(sizes, portions):
+    """Parts of a row tile's keys added up against whole tiles: sums of the same products in another order."""
+    from tinyllmforge_amd import _lib, ops as P
+    (H, G, D, V), g, bs = sizes, torch.Generator(device="cuda").manual_seed(3), 64
+    need = [-(-(a + n) // bs) for a, n in portions]
+    kv = P.SinkKV(sum(need) + 2, bs, G, D, V, torch.bfloat16, "cuda")
+    kv.k[..., :D].normal_(generator=g)
+    kv.v[..., :V].normal_(generator=g)
+    perm, bt = torch.randperm(sum(need) + 2, generator=g, device="cuda").to(torch.int32), torch.full((len(need) + 1, max(need)), -1, dtype=torch.int32, device="cuda")
+    for s, k in enumerate(need):
+        bt[s + 1, :k] = perm[sum(need[:s]):sum(need[:s]) + k]
+    lens, rows = [1] + [n for _, n in portions], 1 + sum(n for _, n in portions)         # a sequence in front that is not asked for
+    cu, starts = i32(*([0] + torch.tensor(lens).cumsum(0).tolist())), i32(0, *[a for a, _ in portions])
+    q = torch.zeros(rows, H, kv.k.shape[3], dtype=torch.bfloat16, device="cuda")
+    q[..., :D].normal_(0, 1.5 * D ** -0.5, generator=g)
+    talk = (torch.eye(H, device="cuda") + 0.3 * torch.randn(H, H, device="cuda", generator=g)).to(torch.bfloat16)
+    got, whole, stats = (torch.full((rows, H * V), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(3))
+    lib, ptr, most = _lib.load(), lambda t: t.data_ptr(), max(lens)
+    stats = torch.empty(rows, H, device="cuda")
+    assert lib.tlf_talk_attn_prefill_workspace_bytes(len(need), most, bt.stride(0) * bs, H, G, D, V) or bt.stride(0) * bs <= 96
+    P.talk_attention_prefill(q, kv, bt, cu, starts, 1, len(need), most, talk, got)
+    assert lib.tlf_talk_attn_prefill(ptr(q), ptr(kv.k), ptr(kv.v), ptr(bt), bt.stride(0), ptr(cu), ptr(starts), 1, len(need), most, ptr(talk), ptr(stats),
+                                     ptr(whole), whole.stride(0), H, G, D, V, bs, kv.k.shape[0], torch.cuda.current_stream().cuda_stream) == 0
+    assert (got[0] == 7).all()
+    # fp32 sums of up to 2^11 terms in another order, off by 2^-24 of the terms' sizes, which are a few units at most; then a rounding to bf16
+    # that may fall to either side, an ulp apart: 2^-7 of the value at the lower end of a binade
+    torch.testing.assert_close(got.float(), whole.float(), rtol=2 ** -7, atol=2 ** -14)
+
+
 def test_supported_sizes_run_in_tiles():
     from tinyllmforge_amd import ops as P
     for H, G, D, V in ((32, 8, 128, 128), (16, 8, 128, 128), (8, 4, 64, 64), (1, 1, 1, 1), (12, 12, 96, 80), (32, 4, 64, 128)):

@@ -368,6 +368,10 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     assert size(0, *shape, 200, 0) == 0 and size(2, *shape, 200, 0) >= 2 * 6 * 200 * 4 and att(ws=a, nb=size(2, *shape, 200, 0) - 1) == WORK
     pre = lambda sizes=shape, ldo=78, out=a, n=1, stats=a: lib.tlf_talk_attn_prefill(a, a, a, a, 4, a, a, 0, n, 8, a, stats, out, ldo, *sizes, 64, 10, None)
     assert pre(ldo=70) == SHAPE and pre(out=None) == NULL and pre(stats=None) == NULL and pre(n=0) == 0 and pre(sizes=(3, 1, 140, 13)) == TYPE
+    room = lambda n=1, most=8, keys=256, sizes=shape: lib.tlf_talk_attn_prefill_workspace_bytes(n, most, keys, *sizes)
+    assert room() > 0 and room(keys=96) == 0 and room(n=0) == 0 and room(n=600) == 0 and room(sizes=(33, 1, 20, 13)) == 0
+    cut = lambda ws=None, nb=0, ldo=78, out=a, n=1: lib.tlf_talk_attn_prefill_cut(a, a, a, a, 4, a, a, 0, n, 8, a, a, out, ldo, *shape, 64, 10, ws, nb, None)
+    assert cut() == WORK and cut(ws=a, nb=room() - 1) == WORK and cut(ldo=70) == SHAPE and cut(out=None) == NULL and cut(n=0) == 0
     ok = lib.tlf_talk_attn_prefill_supported
     assert ok(32, 8, 128, 128) == 1 and ok(33, 1, 64, 64) == 0 and ok(4, 2, 129, 64) == 0 and ok(4, 2, 64, 129) == 0 and ok(1, 1, 1, 1) == 1
 

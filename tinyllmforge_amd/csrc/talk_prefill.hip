@@ -18,14 +18,29 @@
 // with q partly in memory a tile of 32 rows took 14800 cycles, 9800 of them before the mix, waiting for it behind the loads of K; so 11000,
 // 3600 of them products.  Eight prompts of 1061 to 2048 tokens, 128 dimensions, both kernels: 16 heads on 8 KV heads 500 -> 357 us, on 4
 // 455 -> 331, 32 heads 734 -> 612.
+//
+// A workgroup fills a compute unit, and a launch of whole tiles ends with its longest one, 64 steps of 4.8 us at 2048 keys where an even share is
+// 39.  So the keys of long tiles are cut (talk_split.h): a workgroup of the first kernel plans it beside the others' work, the second one's take
+// tiles and parts from its list, and talk_join_kernel adds up what the parts of a tile have left in fp32: 312 -> 246 + 15 us.
+#include <algorithm>
+
 #include "gemm_shared.h"
 #include "prompt_tiles.h"
 #include "talk_attn.h"
+#include "talk_split.h"
 
 namespace tlf {
 
 constexpr int kTK = 32;             // keys per tile
 constexpr int kTM = kTK + 8;        // keys of a head's mixed weights, padded
+
+// How row tiles are cut; plan NULL: they stay whole, a workgroup each.
+struct TalkSplit {
+  int32_t *plan;                    // steps of a part, items, tiles that are cut, items taken beyond each workgroup's first
+  int4 *items, *cuts;               // (sequence, row tile, first key tile, slot); (sequence, row tile, its first extra part's slot, extra parts)
+  floatx4 *parts;                   // slots of `size`: `most` extra parts, then what stays with a tile
+  int32_t seqs, xtiles, tq, most, size;
+};
 
 struct TalkPrefillArgs {
   SinkCache c;
@@ -38,8 +53,106 @@ struct TalkPrefillArgs {
   int32_t H, group;
   int32_t hpp, passes, bq;          // stats: query heads per pass, passes, rows per workgroup
   PromptTiles tiles;
+  TalkSplit split;
   int32_t first_seq, table_cols;
 };
+
+// Where a sequence's portion lies; rows that the block table does not reach are left out.
+__device__ __forceinline__ void talk_portion(const TalkPrefillArgs &p, int sq, int &start, int &tokens) {
+  const int seq = p.first_seq + sq;
+  start = p.starts[seq];
+  tokens = p.cu_q[seq + 1] - p.cu_q[seq];
+  if (start + static_cast<int64_t>(tokens) > static_cast<int64_t>(p.table_cols) * p.c.bs) tokens = 0;
+}
+
+// Key tiles from `first` on; slot: where partial sums go, < 0: the result itself.
+struct TalkItem {
+  int sq, xt, first, slot;
+};
+
+// One workgroup of 256: how the row tiles of the second kernel are cut, and the order of the work.  A thread has a row tile.
+__device__ __forceinline__ void talk_plan(const TalkPrefillArgs &p, int32_t *shared) {
+  const TalkSplit &sp = p.split;
+  constexpr int kMine = (kTalkTiles + 255) / 256;
+  const int tid = threadIdx.x;
+  int sq[kMine], xt[kMine], steps[kMine], all = 0;
+#pragma unroll
+  for (int m = 0; m < kMine; ++m) steps[m] = 0;
+  for (int first = 0; first < sp.seqs; first += 256) {
+    int start = 0, tokens = 0;
+    if (first + tid < sp.seqs) talk_portion(p, first + tid, start, tokens);
+    __syncthreads();
+    shared[tid] = start;
+    shared[256 + tid] = min(talk_tiles(tokens, sp.tq), sp.xtiles);
+    shared[512 + tid] = tokens;
+    __syncthreads();
+    for (int s = 0; s < min(256, sp.seqs - first); ++s) {
+      const int n = min(shared[256 + s], kTalkTiles - all);
+#pragma unroll
+      for (int m = 0; m < kMine; ++m) {
+        const int x = tid + m * 256 - all;
+        if (x < 0 || x >= n) continue;
+        sq[m] = first + s;
+        xt[m] = x;
+        steps[m] = talk_steps(shared[s], shared[512 + s], sp.tq, x);
+      }
+      all += n;
+    }
+  }
+  __syncthreads();
+  auto sum_of = [&](auto value) {                                    // over all tiles
+    int v = 0;
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) v += steps[m] ? value(steps[m]) : 0;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) v += __shfl_xor(v, d);
+    __syncthreads();
+    if ((tid & 63) == 0) shared[tid >> 6] = v;
+    __syncthreads();
+    return (shared[0] + shared[1]) + (shared[2] + shared[3]);
+  };
+  const int64_t work = sum_of([](int n) { return n >> 12; }) * 4096ll + sum_of([](int n) { return n & 4095; });
+  auto extras_of = [&](int per) { return sum_of([&](int n) { return min(talk_extras(n, per), kTalkExtras); }); };
+  const int per = talk_per(work, all, extras_of), items = all + extras_of(per);
+  int32_t *const count = shared + 4, *const taken = shared + 4 + 128;      // by length; slots, cut tiles
+  __syncthreads();
+  if (tid < 128 + 2) count[tid] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < kMine; ++m)
+    if (steps[m]) {
+      const int extras = talk_extras(steps[m], per);
+      if (extras) atomicAdd(count, extras);
+      atomicAdd(count + talk_class(steps[m] - extras * per, per), 1);
+    }
+  __syncthreads();
+  int before = 0;                                                    // a class's place
+  if (tid < 128)
+    for (int i = 0; i < tid; ++i) before += count[i];
+  __syncthreads();
+  if (tid < 128) count[tid] = before;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < kMine; ++m)
+    if (steps[m]) {
+      const int extras = talk_extras(steps[m], per);
+      int slot = -1;
+      if (extras) {
+        const int first = atomicAdd(taken, extras), cut = atomicAdd(taken + 1, 1);
+        for (int i = 0; i < extras; ++i) sp.items[atomicAdd(count, 1)] = make_int4(sq[m], xt[m], i * per, first + i);
+        sp.cuts[cut] = make_int4(sq[m], xt[m], first, extras);
+        slot = sp.most + cut;
+      }
+      sp.items[atomicAdd(count + talk_class(steps[m] - extras * per, per), 1)] = make_int4(sq[m], xt[m], extras * per, slot);
+    }
+  __syncthreads();
+  if (tid == 0) {
+    sp.plan[0] = per;
+    sp.plan[1] = items;
+    sp.plan[2] = taken[1];
+    sp.plan[3] = 0;
+  }
+}
 
 template <typename T>
 __device__ __forceinline__ T talk_uniform(const T *p) {              // through the scalar path
@@ -55,8 +168,13 @@ template <int DC, int CT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void talk_stats_kernel(const TalkPrefillArgs p) {
   constexpr int DP = DC * 32, KCH = DC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[2][kTS][DP + 8];
-  int sq, plane, xt;
-  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
+  int sq, plane, xt, block = prompt_block(blockIdx.x, blockIdx.y);
+  if (p.split.plan) {                                                // eight workgroups in front: the XCDs keep their tiles
+    if (block == 0) talk_plan(p, reinterpret_cast<int32_t *>(Ks));
+    block -= 8;
+    if (block < 0) return;
+  }
+  if (!prompt_tile(p.tiles, block, sq, plane, xt)) return;
   const SinkCache &c = p.c;
   const int seq = p.first_seq + sq, kvh = plane / p.passes, pass = plane % p.passes;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
@@ -164,6 +282,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
   }
 }
 
+// Four values of a head's output.
+__device__ __forceinline__ bool talk_out_in_fours(const TalkPrefillArgs &p) {
+  return (p.c.Dv & 3) == 0 && (p.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
+}
+__device__ __forceinline__ void talk_put(unsigned short *o, int col, int dims, bool vec, const floatx4 &x) {
+  const uint2 v = make_uint2(pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]));
+  if (vec) {
+    if (col < dims) *reinterpret_cast<uint2 *>(o + col) = v;
+  } else {
+    const unsigned int y[2] = {v.x, v.y};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (col + r < dims) o[col + r] = static_cast<unsigned short>(y[r / 2] >> (16 * (r & 1)));
+  }
+}
+
 // A row's place in LDS for heads of WV waves: W [key][head], later M [head][key]; hi and lo apart; rows begin in different banks.
 __host__ __device__ constexpr int talk_heads_held(int wv) { return wv == 1 ? 8 : wv * 4; }
 __host__ __device__ constexpr int talk_row_size(int wv) {
@@ -188,30 +322,29 @@ __device__ __forceinline__ void talk_st(unsigned int at, const T &v) {
 // WV: quads of heads, RT: tiles of 16 rows; DC: key dimensions in units of 32, VC: of values, rounded up to 2 or 4; GS: heads of a
 // quad that share a KV head (1, 2 or 4).  A wave has RW row tiles of HW heads of KV KV heads, HK each: item e = (KV head, row tile, head).
 template <int WV, int RT, int DC, int VC, int GS>
-__global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPrefillArgs p) {
+__device__ __forceinline__ void talk_prefill_tile(const TalkPrefillArgs &p, const TalkItem item, const int wave, unsigned short *lds) {
   constexpr int HP = talk_heads_held(WV), HT = (HP + 15) / 16, KH = (HP + 31) / 32, ROW = talk_row_size(WV), TQ = RT * 16, NW = WV * RT;
   constexpr int VP = VC * 32, PIECES = VP / 8, RW = RT < 4 / GS ? RT : 4 / GS, HW = 4 / RW, KV = HW > GS ? HW / GS : 1, HK = HW / KV;
   constexpr int PER = 4 / KV;                                        // items of a KV head
   constexpr int TS = KH * 32 + 8;                                    // heads of a talk row in LDS
   constexpr int kAtOnce = HT == 1 ? 4 : 1;                           // rows of the mix, as registers allow
-  extern __shared__ __attribute__((aligned(1024))) unsigned short lds[];
   unsigned short *Vs = lds, *Wh = lds + p.c.G * kTK * VP, *Wl = Wh + TQ * ROW, *Ts = Wl + TQ * ROW;    // Vs [G][32][VP], Ts [16 HT][TS]
-  int sq, plane, xt;
-  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
   const SinkCache &c = p.c;
-  const int seq = p.first_seq + sq;
-  const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
-  const int row0 = xt * TQ;
+  const int seq = p.first_seq + item.sq;
+  const int q0 = talk_uniform(p.cu_q + seq), lq = talk_uniform(p.cu_q + seq + 1) - q0, start = talk_uniform(p.starts + seq);
+  const int row0 = item.xt * TQ;
   if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
   const int32_t *bt = c.bt + seq * c.bt_stride;
   const int G = c.G;
-  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), h0 = wave % (WV * 4 / HW) * HW, rt = wave / (WV * 4 / HW) * RW * 16;
+  int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  asm volatile("" : "+v"(lane));                                     // what follows from it is made anew for each item, not kept in registers
+  const int tid = wave * 64 + lane, n = lane & 15, g = lane >> 4;
+  const int h0 = wave % (WV * 4 / HW) * HW, rt = wave / (WV * 4 / HW) * RW * 16;
   const int last_row = min(row0 + TQ, lq) - 1, i_last = start + last_row;
   const int wave_first = start + min(row0 + rt, last_row);           // keys behind it are masked for some row of the wave
   auto head_of = [](int e) { return e / PER * HK + e % HK; };        // of the wave's heads; and the row tile
   auto tile_of = [](int e) { return e % PER / HK; };
-  const int tiles = i_last / kTK + 1;
+  const int first = item.first, tiles = item.slot >= 0 && item.slot < p.split.most ? first + talk_uniform(p.split.plan) : i_last / kTK + 1;
   // where a tile lies: its page (an unmapped one reads page 0) and its first row there, stepped tile by tile
   struct Place {
     int index, page, row;
@@ -283,10 +416,12 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
   unsigned int pat = w0 + (wave * ROW + n * kTM + g * 8) * 2;        // and its result
 
   bf16x8 kb[DC];
-  Place at{0, page_at(0), 0};
+  Place at{sink_page_of(c, first * kTK), 0, 0};
+  at.page = page_at(at.index);
+  at.row = first * kTK - at.index * c.bs;
   load_k(kb, at, kvh[0], 0);
   lds_barrier();
-  for (int t = 0; t < tiles; ++t) {
+  for (int t = first; t < tiles; ++t) {
     const int j0 = t * kTK;
     const Place next = after(at, t + 1 < tiles);
     auto copy_v = [&]() __attribute__((always_inline)) {
@@ -432,7 +567,15 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
     at = next;
   }
 
-  const bool vec = (c.Dv & 3) == 0 && (p.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
+  if (item.slot >= 0) {                                              // as it lies in the registers: whole lines
+    floatx4 *const part = p.split.parts + static_cast<int64_t>(item.slot) * p.split.size + (wave * (8 * VC)) * 64 + lane;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int d = 0; d < 2 * VC; ++d) part[(e * 2 * VC + d) * 64] = acc[e][d];
+    return;
+  }
+  const bool vec = talk_out_in_fours(p);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int row = row0 + rt + tile_of(e) * 16 + n, h = h0 + head_of(e);
@@ -440,18 +583,70 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
     unsigned short *o = p.out + static_cast<int64_t>(q0 + row) * p.ldo + static_cast<int64_t>(h) * c.Dv;
 #pragma unroll
     for (int d = 0; d < 2 * VC; ++d) {
-      const int col = d * 16 + g * 4;
-      const uint2 v = make_uint2(pack_bf16x2(acc[e][d][0], acc[e][d][1]), pack_bf16x2(acc[e][d][2], acc[e][d][3]));
-      if (vec) {
-        if (col < c.Dv) *reinterpret_cast<uint2 *>(o + col) = v;
-      } else {
-        const unsigned int x[2] = {v.x, v.y};
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col + r < c.Dv) o[col + r] = static_cast<unsigned short>(x[r / 2] >> (16 * (r & 1)));
-      }
+      talk_put(o, d * 16 + g * 4, c.Dv, vec, acc[e][d]);
     }
   }
+}
+
+// Without a plan a workgroup has the tile of its place.  With one, a workgroup per compute unit takes items until there are none: the hardware
+// deals workgroups to XCDs and shader engines by their number, whatever runs there.
+template <int WV, int RT, int DC, int VC, int GS>
+__global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPrefillArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned short lds[];
+  int *const at = reinterpret_cast<int *>(lds);                      // the item, where the tile's arrays begin
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (bool more = false;; more = true) {
+    // the arguments are read anew for each item: kept across the loop, what follows from them would not fit into the scalar registers
+    auto args = (const TalkPrefillArgs __attribute__((address_space(4))) *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    const TalkPrefillArgs &p = *(const TalkPrefillArgs *)args;
+    if (wave == 0 && __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)) == 0) {
+      int4 item = make_int4(0, 0, 0, -1);
+      int plane;
+      if (p.split.plan) {
+        const int i = more ? gridDim.x + atomicAdd(p.split.plan + 3, 1) : blockIdx.x;
+        at[4] = i < p.split.plan[1];
+        if (i < p.split.plan[1]) item = p.split.items[i];
+      } else {
+        at[4] = !more && prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), item.x, plane, item.y);
+      }
+      *reinterpret_cast<int4 *>(at) = item;
+    }
+    lds_barrier();
+    auto same = [&](int i) { return __builtin_amdgcn_readfirstlane(at[i]); };
+    if (!same(4)) return;
+    const TalkItem item{same(0), same(1), same(2), same(3)};
+    lds_barrier();
+    talk_prefill_tile<WV, RT, DC, VC, GS>(p, item, wave, lds);
+    if (!a.split.plan) return;
+  }
+}
+
+// Row tiles that were cut: their parts, added up in the order of the keys.  blockIdx.x: the tile, blockIdx.y: a wave of the second kernel.
+template <int WV, int RT, int VC, int GS>
+__global__ __launch_bounds__(256) void talk_join_kernel(const TalkPrefillArgs p) {
+  constexpr int RW = RT < 4 / GS ? RT : 4 / GS, HW = 4 / RW, KV = HW > GS ? HW / GS : 1, HK = HW / KV, PER = 4 / KV;
+  const TalkSplit &sp = p.split;
+  if (static_cast<int>(blockIdx.x) >= sp.plan[2]) return;
+  const int4 cut = sp.cuts[blockIdx.x];
+  const int seq = p.first_seq + cut.x, row0 = cut.y * (RT * 16), wave = blockIdx.y, lane = threadIdx.x & 63, e = threadIdx.x >> 6;
+  const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, n = lane & 15, g = lane >> 4;
+  const int row = row0 + wave / (WV * 4 / HW) * RW * 16 + e % PER / HK * 16 + n, h = wave % (WV * 4 / HW) * HW + e / PER * HK + e % HK;
+  const int64_t at = (wave * 4 + e) * 2 * VC * 64 + lane, size = sp.size;
+  const floatx4 *const extra = sp.parts + cut.z * size + at, *const rest = sp.parts + (sp.most + blockIdx.x) * size + at;
+  floatx4 sum[2 * VC];
+#pragma unroll
+  for (int d = 0; d < 2 * VC; ++d) sum[d] = extra[d * 64];
+  for (int part = 1; part < cut.w; ++part)
+#pragma unroll
+    for (int d = 0; d < 2 * VC; ++d) sum[d] += extra[part * size + d * 64];
+#pragma unroll
+  for (int d = 0; d < 2 * VC; ++d) sum[d] += rest[d * 64];
+  if (row >= lq || h >= p.H) return;
+  const bool vec = talk_out_in_fours(p);
+  unsigned short *const o = p.out + static_cast<int64_t>(q0 + row) * p.ldo + static_cast<int64_t>(h) * p.c.Dv;
+#pragma unroll
+  for (int d = 0; d < 2 * VC; ++d) talk_put(o, d * 16 + g * 4, p.c.Dv, vec, sum[d]);
 }
 
 // Quads of heads as instantiated, 0: too many.
@@ -467,6 +662,22 @@ int talk_row_tiles(int quads, int G, int Vp) {
   return talk_prefill_lds(quads, most, G, Vp) <= kTalkLds ? most : quads == 4 && talk_prefill_lds(quads, 1, G, Vp) <= kTalkLds ? 1 : 0;
 }
 
+// What a workspace holds; bytes = 0: row tiles stay whole.
+struct TalkRoom {
+  int most, size;
+  int64_t cuts, parts, bytes;            // where they begin
+};
+TalkRoom talk_room(int64_t seqs, int64_t max_tokens, int64_t max_keys, int quads, int tq, int Vp) {
+  TalkRoom r{0, quads * 4 * tq * talk_units(Vp) * 8, 0, 0, 0};
+  if (!talk_cuts(seqs, max_tokens, max_keys, tq)) return r;
+  const int64_t tiles = (max_tokens + tq - 1) / tq * seqs;
+  r.most = static_cast<int>(std::min<int64_t>(kTalkExtras, tiles * std::min<int64_t>(kTalkExtras, (max_keys + kTK - 1) / kTK / kTalkLeast)));
+  r.cuts = 16 + (kTalkTiles + kTalkExtras) * 16;
+  r.parts = (r.cuts + kTalkTiles * 16 + 255) / 256 * 256;
+  r.bytes = r.parts + (r.most + tiles) * r.size * 16;
+  return r;
+}
+
 template <int DC>
 int launch_talk_stats(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStream_t s) {
   constexpr int CT = 2, kUnits = 64 * CT;
@@ -475,7 +686,7 @@ int launch_talk_stats(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStrea
   a.bq = kUnits / a.hpp;
   const int blocks = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, a.c.G * a.passes, num_seqs);
   if (!blocks) return TLF_E_SHAPE;
-  TLF_LAUNCH((talk_stats_kernel<DC, CT>), prompt_grid<dim3>(blocks), dim3(256), 0, s, a);
+  TLF_LAUNCH((talk_stats_kernel<DC, CT>), prompt_grid<dim3>(blocks + (a.split.plan ? 8 : 0)), dim3(256), 0, s, a);
   return launch_status();
 }
 
@@ -486,7 +697,9 @@ int launch_talk_prefill(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStr
   if (allowed != hipSuccess) return static_cast<int>(allowed);
   const int blocks = prompt_tiles_make(a.tiles, (max_tokens + RT * 16 - 1) / (RT * 16), 1, num_seqs);
   if (!blocks) return TLF_E_SHAPE;
-  TLF_LAUNCH((talk_prefill_kernel<WV, RT, DC, VC, GS>), prompt_grid<dim3>(blocks), dim3(WV * RT * 64), talk_prefill_lds(WV, RT, a.c.G, a.c.Vp), s, a);
+  TLF_LAUNCH((talk_prefill_kernel<WV, RT, DC, VC, GS>), a.split.plan ? dim3(kTalkUnits) : prompt_grid<dim3>(blocks),
+             dim3(WV * RT * 64), talk_prefill_lds(WV, RT, a.c.G, a.c.Vp), s, a);
+  if (a.split.plan) TLF_LAUNCH((talk_join_kernel<WV, RT, VC, GS>), dim3((max_tokens + RT * 16 - 1) / (RT * 16) * num_seqs, WV * RT), dim3(256), 0, s, a);
   return launch_status();
 }
 template <int WV, int RT>
@@ -516,12 +729,12 @@ extern "C" int tlf_talk_attn_prefill_supported(int32_t heads, int32_t kv_heads, 
          tlf::talk_row_tiles(tlf::talk_quads(heads), kv_heads, (vdim + 31) / 32 * 32) > 0;
 }
 
-extern "C" int tlf_talk_attn_prefill(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables,
-                                     int64_t bt_stride, const int32_t *cu_seqlens_q, const int32_t *seq_starts, int32_t first_seq,
-                                     int32_t num_seqs, int32_t max_tokens, const void *talk, float *stats, void *out, int64_t out_stride,
-                                     int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, int32_t block_size,
-                                     int64_t num_pages, void *stream) {
-  using namespace tlf;
+namespace tlf {
+int talk_attn_prefill(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables, int64_t bt_stride,
+                      const int32_t *cu_seqlens_q, const int32_t *seq_starts, int32_t first_seq, int32_t num_seqs, int32_t max_tokens,
+                      const void *talk, float *stats, void *out, int64_t out_stride, int32_t heads, int32_t kv_heads, int32_t dim,
+                      int32_t vdim, int32_t block_size, int64_t num_pages, bool cut, void *workspace, size_t workspace_bytes,
+                      void *stream) {
   if (num_seqs < 0 || max_tokens < 0 || first_seq < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads) return TLF_E_SHAPE;
   if (out_stride < static_cast<int64_t>(heads) * vdim || bt_stride <= 0) return TLF_E_SHAPE;
   if (num_seqs == 0 || max_tokens == 0) return TLF_OK;
@@ -534,7 +747,18 @@ extern "C" int tlf_talk_attn_prefill(const void *q, const void *k_cache, const v
   a.starts = seq_starts; a.out = static_cast<unsigned short *>(out); a.ldo = out_stride; a.H = heads; a.group = heads / kv_heads;
   a.first_seq = first_seq; a.table_cols = static_cast<int32_t>(bt_stride);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int quads = talk_quads(heads);
+  const int quads = talk_quads(heads), row_tiles = talk_row_tiles(quads, kv_heads, a.c.Vp);
+  if (cut) {
+    const TalkRoom room = talk_room(num_seqs, max_tokens, bt_stride * block_size, quads, row_tiles * 16, a.c.Vp);
+    if (room.bytes) {
+      if (!workspace || workspace_bytes < static_cast<size_t>(room.bytes)) return TLF_E_WORKSPACE;
+      if (!aligned16(workspace)) return TLF_E_ALIGN;
+      char *const ws = static_cast<char *>(workspace);
+      a.split = TalkSplit{reinterpret_cast<int32_t *>(ws), reinterpret_cast<int4 *>(ws + 16), reinterpret_cast<int4 *>(ws + room.cuts),
+                          reinterpret_cast<floatx4 *>(ws + room.parts), num_seqs, (max_tokens + row_tiles * 16 - 1) / (row_tiles * 16),
+                          row_tiles * 16, room.most, room.size};
+    }
+  }
   int rc;
   switch (a.c.Dp / 32) {
     case 1: rc = launch_talk_stats<1>(a, num_seqs, max_tokens, s); break;
@@ -545,9 +769,36 @@ extern "C" int tlf_talk_attn_prefill(const void *q, const void *k_cache, const v
   if (rc != TLF_OK) return rc;
 #define TLF_TP(WV, RT) \
   case (WV) * 8 + (RT): return launch_talk_prefill_dims<WV, RT>(a, num_seqs, max_tokens, s);
-  switch (quads * 8 + talk_row_tiles(quads, kv_heads, a.c.Vp)) {
+  switch (quads * 8 + row_tiles) {
     TLF_TP(1, 4) TLF_TP(2, 4) TLF_TP(4, 1) TLF_TP(4, 2) TLF_TP(8, 1)
     default: return TLF_E_UNSUPPORTED;
   }
 #undef TLF_TP
+}
+}  // namespace tlf
+
+extern "C" int tlf_talk_attn_prefill(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables,
+                                     int64_t bt_stride, const int32_t *cu_seqlens_q, const int32_t *seq_starts, int32_t first_seq,
+                                     int32_t num_seqs, int32_t max_tokens, const void *talk, float *stats, void *out, int64_t out_stride,
+                                     int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, int32_t block_size,
+                                     int64_t num_pages, void *stream) {
+  return tlf::talk_attn_prefill(q, k_cache, v_cache, block_tables, bt_stride, cu_seqlens_q, seq_starts, first_seq, num_seqs, max_tokens, talk, stats,
+                                out, out_stride, heads, kv_heads, dim, vdim, block_size, num_pages, false, nullptr, 0, stream);
+}
+
+extern "C" size_t tlf_talk_attn_prefill_workspace_bytes(int32_t num_seqs, int32_t max_tokens, int64_t max_keys, int32_t heads,
+                                                        int32_t kv_heads, int32_t dim, int32_t vdim) {
+  using namespace tlf;
+  if (num_seqs <= 0 || max_tokens <= 0 || max_keys <= 0 || !tlf_talk_attn_prefill_supported(heads, kv_heads, dim, vdim)) return 0;
+  const int Vp = (vdim + 31) / 32 * 32;
+  return static_cast<size_t>(talk_room(num_seqs, max_tokens, max_keys, talk_quads(heads), talk_row_tiles(talk_quads(heads), kv_heads, Vp) * 16, Vp).bytes);
+}
+
+extern "C" int tlf_talk_attn_prefill_cut(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables,
+                                         int64_t bt_stride, const int32_t *cu_seqlens_q, const int32_t *seq_starts, int32_t first_seq,
+                                         int32_t num_seqs, int32_t max_tokens, const void *talk, float *stats, void *out, int64_t out_stride,
+                                         int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, int32_t block_size, int64_t num_pages,
+                                         void *workspace, size_t workspace_bytes, void *stream) {
+  return tlf::talk_attn_prefill(q, k_cache, v_cache, block_tables, bt_stride, cu_seqlens_q, seq_starts, first_seq, num_seqs, max_tokens, talk, stats,
+                                out, out_stride, heads, kv_heads, dim, vdim, block_size, num_pages, true, workspace, workspace_bytes, stream);
 }
