@@ -212,6 +212,50 @@ def test_talking_heads_with_keys_cut(sizes, portions):
     torch.testing.assert_close(got.float(), whole.float(), rtol=2 ** -7, atol=2 ** -14)
 
 
+@pytest.mark.parametrize("portions,tiles", [([9] * 7, False), ([16] * 4, True), ([60, 2, 3], True), ([2] * 33, True)], ids=str)
+def test_short_portions_in_tiles(portions, tiles, monkeypatch):
+    """From 64 rows on, short portions run in row tiles; both ways give the rows' attention."""
+    from types import SimpleNamespace
+    from tinyllmforge_amd import ops as P
+    from tinyllmforge_amd.engine.inputs import portion_inputs
+    from tinyllmforge_amd.layers.rotary_embedding import rotation_table
+    from tinyllmforge_amd.layers.talking_attention import TalkingHeadsAttention
+    from tinyllmforge_amd.utils.context import reset_context, set_portions_context
+    H, G, D, BF, g = 8, 4, 64, torch.bfloat16, torch.Generator(device="cuda").manual_seed(1)
+    lens, starts = [1, 1] + portions + [130], [5, 64] + [70 * (i % 2) for i in range(len(portions))] + [64]
+    need, at, seqs = [-(-(a + n) // 64) for a, n in zip(starts, lens)], 0, []
+    for i, (a, n) in enumerate(zip(starts, lens)):
+        seqs.append(SimpleNamespace(num_scheduled=n, num_computed=a, token_ids=range(a + n), block_table=list(range(at, at + need[i])), state_slot=i))
+        at += need[i]
+    d = {k: torch.from_numpy(v).cuda() if hasattr(v, "dtype") else v for k, v in portion_inputs(seqs, 64, 128).items()}
+    positions = d.pop("positions")
+    d.pop("input_ids")
+    with torch.device("cuda"):
+        layer = TalkingHeadsAttention(H, G, D, D, D ** -0.5, 1e-6, BF, D).to(BF)
+    layer.cos_sin = rotation_table(D, 512, 1e6).cuda()
+    layer.talk.data = (torch.eye(H, device="cuda") + 0.3 * torch.randn(H, H, device="cuda", generator=g)).to(BF)
+    layer.bind_pages(at, 64, "cuda")
+    proj, k, v = (torch.randn(*s, device="cuda", generator=g).to(BF) for s in ((sum(lens), (H + 2 * G) * D), layer.kv.k.shape, layer.kv.v.shape))
+    firsts, prefill = [], P.talk_attention_prefill
+
+    def call(by_rows):
+        layer.kv.k.copy_(k)
+        layer.kv.v.copy_(v)
+        set_portions_context(**d, max_len=512)
+        with torch.inference_mode(), monkeypatch.context() as m:
+            m.setattr(P, "talk_attention_prefill", lambda *a: (firsts.append(a[5]), prefill(*a))[1])
+            if by_rows:
+                m.setattr(P, "talk_prefill_supported", lambda *a: False)
+            out = layer(proj, positions)
+        reset_context()
+        return out.float()
+
+    got, want = call(False), call(True)
+    assert firsts == [2 if tiles else 2 + len(portions)]
+    # by rows the weights enter as bf16 pairs of 16 bits too, in another order: a bf16 ulp of the result, and 2^-14 of terms of a few units
+    torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -10)
+
+
 def test_supported_sizes_run_in_tiles():
     from tinyllmforge_amd import ops as P
     for H, G, D, V in ((32, 8, 128, 128), (16, 8, 128, 128), (8, 4, 64, 64), (1, 1, 1, 1), (12, 12, 96, 80), (32, 4, 64, 128)):

@@ -37,12 +37,16 @@ class TalkingHeadsAttention(nn.Module):
                           self.temp.data, self.cos_sin, self.rot_dims, self.eps, self.scale)
         out = torch.empty(n, self.num_heads * self.value_dim, dtype=self.dtype, device=q.device)
         tiles = self.dtype == torch.bfloat16 and ops.talk_prefill_supported(self.num_heads, self.num_kv_heads, self.dim, self.value_dim)
-        rows = ctx.num_short_rows if tiles else n
+        # Short portions go row by row only where they are few rows: a row tile starts with more latency, and its keys are read once for
+        # all its rows.  16 heads, portions behind 1024 keys, the layer by rows and in tiles: 8 of up to 8 tokens 57 and 67 us, one of 64 63 and
+        # 62, 8 of up to 16 93 and 67, 60 of up to 32 818 and 135.
+        short = ctx.num_short if ctx.num_short_rows - ctx.num_single < 64 else 0
+        rows = (ctx.num_short_rows if short else ctx.num_single) if tiles else n
         if rows:
             ops.talk_attention_rows(q[:rows], kv, ctx.block_tables, positions[:rows], ctx.slot_mapping[:rows], self.talk.data, ctx.max_len,
                                     out[:rows], ctx.row_seq[:rows] if ctx.num_single < rows else None)
         if rows < n:
-            first = ctx.num_single + ctx.num_short
+            first = ctx.num_single + short
             ops.talk_attention_prefill(q, kv, ctx.block_tables, ctx.cu_seqlens_q, ctx.seq_starts, first,
                                        ctx.cu_seqlens_q.numel() - 1 - first, ctx.max_portion, self.talk.data, out)
         return out
