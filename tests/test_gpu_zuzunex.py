@@ -326,6 +326,49 @@ def test_rows_of_many_unequal_sequences(dtype):
             assert rel(out[i, :H * V], want) < (6e-3 if dtype == "bf16" else 4e-6), (B, i, n)
 
 
+@pytest.mark.parametrize("taps", [0, 2, 3, 4])
+@pytest.mark.parametrize("sizes,rot", [((32, 8, 128, 128), 128), ((6, 2, 56, 104), 48), ((3, 3, 64, 8), 0), ((16, 4, 96, 128), 32)], ids=str)
+def test_preparation_of_many_rows(sizes, rot, taps):
+    """More rows than the kernel for few takes, in runs that begin and end anywhere in a sequence, against the same rows sequence by
+    sequence, which that kernel works on: the same operations in the same order, bit for bit."""
+    from tinyllmforge_amd import ops as P
+    (H, G, D, V), g, BF, dev = sizes, torch.Generator(device="cuda").manual_seed(taps), torch.bfloat16, "cuda"
+    lens = [1, 1, 1] + [700, 2, 3, 23, 24, 25, 1, 47, 600, 5]        # singles too, some behind others
+    starts = [0, 9, 64, 0, 1, 2, 70, 0, 3, 0, 200, 64, 1]
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=dev)
+    rows, channels = sum(lens), (H + G) * D + G * V
+    need = [-(-(a + n) // 64) for a, n in zip(starts, lens)]
+    randn = lambda *s: torch.randn(*s, generator=g, device=dev).to(BF)
+    proj, bias, conv, ring0 = randn(rows, channels + H * V), randn(channels), randn(max(taps, 1), channels), randn(len(lens) + 2, max(taps, 1), channels)
+    qn, kn, table, temps = 1 + 0.1 * randn(D), 1 + 0.1 * randn(D), torch.randn(1024, max(rot, 1), generator=g, device=dev), torch.rand(1024, generator=g, device=dev)
+    states = i32(*[(i * 4) % (len(lens) + 2) for i in range(len(lens))])
+    states[9] = -1                                                   # no state: nothing before it, nothing kept
+    pages = torch.randperm(sum(need), generator=g, device=dev)
+    pos, slots, at = [], [], 0
+    for a, n, k in zip(starts, lens, need):
+        p = torch.arange(a, a + n, device=dev)
+        pos.append(p)
+        slots.append(pages[at:at + k][p // 64] * 64 + p % 64)
+        at += k
+    slots[4] = torch.full_like(slots[4], -1)                         # not stored
+    pos, slots = torch.cat(pos), torch.cat(slots).to(torch.int32)
+    first = [sum(lens[:i]) for i in range(len(lens) + 1)]
+
+    def prepared(parts):
+        kv, ring, q = P.SinkKV(sum(need), 64, G, D, V, BF, dev), ring0.clone(), []
+        for lo, hi in parts:
+            at = slice(first[lo], first[hi])
+            seq = torch.repeat_interleave(torch.arange(hi - lo), torch.tensor(lens[lo:hi])).to(torch.int32).to(dev)
+            cu = i32(*[f - first[lo] for f in first[lo:hi + 1]])
+            held = dict(conv=conv, ring=ring, state_slots=states[lo:hi].contiguous()) if taps else {}
+            q.append(P.sink_prep(proj[at], kv, H, pos[at].contiguous(), slots[at].contiguous(), 1e-5, 0.3, 20.0, bias, row_seq=seq, cu_seqlens_q=cu, q_norm=qn, k_norm=kn,
+                                 cos_sin=table if rot else None, rot_dims=rot, q_mult=temps, **held)[0])
+        return torch.cat(q), kv.k, kv.v, ring
+
+    for got, want in zip(prepared([(0, len(lens))]), prepared([(i, i + 1) for i in range(len(lens))])):
+        assert torch.equal(got, want)
+
+
 # ---------------------------------------------------------------------------------------------- experts
 @pytest.mark.parametrize("corr_dtype", DTYPES)
 @pytest.mark.parametrize("n,E,ident,top,splits", [(1, 5, 2, 2, 1), (64, 70, 7, 6, 3), (500, 16, 1, 1, 2), (1500, 33, 3, 4, 1), (9, 500, 12, 20, 1),

@@ -348,6 +348,168 @@ __global__ __launch_bounds__(256) void sink_prep_kernel(const SinkPrepArgs a) {
   }
 }
 
+// The same for rows of prompts: bf16 projections, head dimensions up to 128 in whole granules, rotations whose halves are granules, no gate.
+// A workgroup has 16 heads of `run` consecutive rows, 16 lanes a head, so the weights are loaded and unpacked once, and a row is read once more
+// only by the next run's first rows.  What is the same for all heads of a row (where it goes, what lies before it, its cosines and sines) is
+// in LDS.  Rows are on their way four at a time while four are worked on.  A rotation by 64 meets its partner eight lanes on.
+//
+// Bound by the vector ALU, some 170 instructions for eight values, and HBM: 12237 rows of 32 + 2 x 8 heads of 128, four taps, 127 us with
+// four rows a workgroup and weights unpacked for each, 84 so; 300 MB take 59.  Three waves per SIMD: with four, registers go to memory (136).
+constexpr int kRun = 24;                  // rows of a workgroup at most
+struct PrepRow {
+  int64_t at;               // cache row of KV head 0, negative: not stored
+  int32_t pos, back, end;   // position; rows of its sequence in the step before it, up to taps - 1; the run's first row behind the sequence
+  int32_t state, single, pad;         // state slot, negative: none
+};
+
+template <int TAPS, bool HALF64>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void sink_prep_rows_kernel(const SinkPrepArgs a, const int run) {
+  typedef unsigned short T;
+  constexpr int kBack = TAPS > 0 ? TAPS - 1 : 1, kAhead = 4;
+  __shared__ __attribute__((aligned(16))) PrepRow rows[kRun];
+  __shared__ __attribute__((aligned(16))) float turn[kRun][3 * 64];  // cosines, sines negated, sines
+  const SinkCache &c = a.c;
+  const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * run;
+  const int count = static_cast<int>(min(static_cast<int64_t>(run), a.n - tok0)), half = a.rot_dims / 2, tid = threadIdx.x;
+  if (tid < count) {
+    const int64_t tok = tok0 + tid, pos = a.positions[tok], slot = a.slots[tok];
+    const int64_t page = slot / c.bs;
+    PrepRow r{slot >= 0 && slot < c.pages * c.bs ? page * c.G * c.bs + (slot - page * c.bs) : -1,
+              pos >= 0 && pos < (1 << 30) ? static_cast<int32_t>(pos) : -1, 0, count, -1, 0, 0};
+    if constexpr (TAPS > 0) {
+      const int seq = a.row_seq ? a.row_seq[tok] : static_cast<int>(tok), st = a.state_slots[seq];
+      const int first = a.row_seq ? a.cu_q[seq] : static_cast<int>(tok);
+      r.back = static_cast<int>(min(tok - first, static_cast<int64_t>(kBack)));
+      r.end = a.row_seq ? static_cast<int>(min(a.cu_q[seq + 1] - tok0, static_cast<int64_t>(count))) : tid + 1;
+      r.single = !a.row_seq || a.cu_q[seq + 1] - first == 1;
+      r.state = st >= 0 && st < a.num_state_slots && r.pos >= 0 ? st : -1;
+    }
+    rows[tid] = r;
+  }
+  for (int i = tid; i < count * half; i += 256) {
+    const int k = i / half, d = i - k * half;
+    const int64_t pos = a.positions[tok0 + k];
+    const float *cs = a.cos_sin + (pos >= 0 && pos < a.max_pos ? pos : 0) * a.rot_dims + d;
+    const float sn = cs[half];
+    turn[k][d] = cs[0];
+    turn[k][64 + d] = -sn;
+    turn[k][128 + d] = sn;
+  }
+  __syncthreads();
+  const int head = blockIdx.y * 16 + tid / 16, j = tid % 16, G = c.G;
+  if (head >= a.heads) return;                                       // whole 16-lane groups leave together
+  const int kind = head < a.H ? 0 : head < a.H + G ? 1 : 2, dims = kind < 2 ? c.D : c.Dv;
+  const int chan = (kind < 2 ? head * c.D : (a.H + G) * c.D + (head - a.H - G) * c.Dv) + min(j * 8, dims - 8);
+  const bool live = j * 8 < dims;                                    // lanes behind the head's dimensions hold zeros
+  const T *const proj = static_cast<const T *>(a.proj) + chan;
+
+  float bias[8], wn[8], wc[TAPS > 0 ? TAPS : 1][8], hist[kBack][8];
+  auto weights = [&](const void *p, int64_t at, float other, float (&w)[8]) __attribute__((always_inline)) {
+    if (p) Elem<T>::ld8(static_cast<const T *>(p) + at, w);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = live ? p ? w[e] : other : 0.f;
+  };
+  weights(a.bias, chan, 0.f, bias);
+  weights(kind == 0 ? a.q_norm : kind == 1 ? a.k_norm : nullptr, min(j * 8, dims - 8), 1.f, wn);
+  if constexpr (TAPS > 0) {
+#pragma unroll
+    for (int t = 0; t < TAPS; ++t) weights(a.conv, static_cast<int64_t>(t) * a.channels + chan, 0.f, wc[t]);
+  }
+  auto row_at = [&](int k) __attribute__((always_inline)) { return *reinterpret_cast<const uint4 *>(proj + (tok0 + min(k, count - 1)) * a.ld); };
+  auto earlier = [&](int k, const PrepRow &r) __attribute__((always_inline)) {     // the rows before row k of the run, with their bias
+#pragma unroll
+    for (int b = 0; b < kBack; ++b) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) hist[b][e] = 0.f;
+      if (r.state < 0 || r.pos <= b) continue;
+      const T *from = b < r.back ? proj + (tok0 + k - 1 - b) * a.ld
+                                 : static_cast<const T *>(a.ring) + (static_cast<int64_t>(r.state) * TAPS + (r.pos - 1 - b) % (TAPS > 0 ? TAPS : 1)) * a.channels + chan;
+      Elem<T>::ld8(from, hist[b]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) hist[b][e] = live ? hist[b][e] + bias[e] : 0.f;
+    }
+  };
+  const int partner = half / 8;
+  for (int k0 = 0; k0 < count;) {                                    // a sequence's rows
+    const int end = __builtin_amdgcn_readfirstlane(rows[k0].end);
+    uint4 raw[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) raw[i] = row_at(k0 + i);
+    if constexpr (TAPS > 0) earlier(k0, rows[k0]);
+    for (; k0 < end; k0 += kAhead)
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int k = k0 + i;
+      const PrepRow r = rows[min(k, kRun - 1)];                      // behind `end`: worked on, not stored
+      const uint4 in = live ? raw[i] : make_uint4(0, 0, 0, 0);
+      raw[i] = row_at(k + kAhead);
+      float x[8];
+      unpack8(in, x);
+      if constexpr (TAPS > 0) {
+        if (r.single && r.state >= 0 && live && k < end)
+          *reinterpret_cast<uint4 *>(static_cast<T *>(a.ring) + (static_cast<int64_t>(r.state) * TAPS + r.pos % TAPS) * a.channels + chan) = in;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float now = x[e] + bias[e];
+          float y = 0.f;
+#pragma unroll
+          for (int b = kBack - 1; b >= 0; --b) y = fmaf(wc[TAPS - 2 - b][e], hist[b][e], y);
+          x[e] = fmaf(wc[TAPS - 1][e], now, y);
+#pragma unroll
+          for (int b = kBack - 1; b > 0; --b) hist[b][e] = hist[b - 1][e];
+          hist[0][e] = now;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] += bias[e];
+      }
+      if (kind < 2) {
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
+        ss = group_sum<16>(ss);
+        const float inv = 1.0f / sqrtf(ss / static_cast<float>(c.D) + a.eps);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = x[e] * inv * wn[e];
+        const bool pos_ok = r.pos >= 0 && r.pos < a.max_pos;
+        if (kind == 0) {
+          const float m = a.q_mult ? a.q_mult[pos_ok ? r.pos : 0] * a.q_scale : a.q_scale;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] *= m;
+        }
+        if (half > 0 && pos_ok) {
+          float other[8], cv[8], sv[8];
+          if constexpr (HALF64) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) other[e] = dpp_move<0x128>(x[e]);        // row_ror 8
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) other[e] = __shfl(x[e], (tid & 48) | (j < partner ? j + partner : j < 2 * partner ? j - partner : j), 64);
+          }
+          if (j < 2 * partner) {
+            const bool low = j < partner;
+            const float *cp = turn[min(k, kRun - 1)] + (low ? j : j - partner) * 8;
+            Elem<float>::ld8(cp, cv);
+            Elem<float>::ld8(cp + (low ? 64 : 128), sv);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = __fmul_rn(x[e], cv[e]) + __fmul_rn(other[e], sv[e]);
+          }
+        }
+      }
+      const uint4 packed = pack8(x);
+      if (k >= end) continue;
+      if (kind == 0) {
+        if (j * 8 < c.Dp) *reinterpret_cast<uint4 *>(static_cast<T *>(a.q_out) + ((tok0 + k) * a.H + head) * c.Dp + j * 8) = packed;
+      } else if (r.at >= 0) {
+        const int padded = kind == 1 ? c.Dp : c.Vp;
+        T *to = static_cast<T *>(const_cast<void *>(kind == 1 ? c.k : c.v)) + (r.at + static_cast<int64_t>(head - a.H - (kind - 1) * G) * c.bs) * padded;
+        if (j * 8 < padded) *reinterpret_cast<uint4 *>(to + j * 8) = packed;
+      }
+    }
+    k0 = end;
+  }
+}
+
 template <typename T>
 int launch_sink_prep(const SinkPrepArgs &a, bool vec, bool part, hipStream_t s) {
   const int most = a.c.Dp > a.c.Vp ? a.c.Dp : a.c.Vp;
@@ -360,6 +522,24 @@ int launch_sink_prep(const SinkPrepArgs &a, bool vec, bool part, hipStream_t s) 
     else TLF_PREP(4, 1, TAPS, false, false);              \
   } while (0)
   if constexpr (sizeof(T) == 2) {
+    // Rows of prompts in runs: long ones where they still are six workgroups for each compute unit (the rows above: runs of 32 90 us, 24 84,
+    // 16 92, 8 106), shorter ones with fewer rows (1700 rows of 16 + 2 x 8 heads: 16 23 us, 8 19, the kernel in front of this one 21).
+    if (vec && !part && most <= 128 && a.n > 1024 && a.rot_dims % 16 == 0 && !a.gate_out && (!a.conv || (a.taps >= 2 && a.taps <= 4))) {
+      const int64_t rows = static_cast<int64_t>(a.n) * hy;
+      const int run = rows >= 24 * 1024 ? 24 : rows >= 16 * 768 ? 16 : 8;
+      const dim3 grid((a.n + run - 1) / run, hy);
+#define TLF_RUNS(TAPS)                                                                                               \
+  if (a.rot_dims == 128) TLF_LAUNCH((sink_prep_rows_kernel<TAPS, true>), grid, dim3(256), 0, s, a, run);              \
+  else TLF_LAUNCH((sink_prep_rows_kernel<TAPS, false>), grid, dim3(256), 0, s, a, run)
+      switch (a.conv ? a.taps : 0) {
+        case 0: TLF_RUNS(0); break;
+        case 2: TLF_RUNS(2); break;
+        case 3: TLF_RUNS(3); break;
+        default: TLF_RUNS(4); break;
+      }
+#undef TLF_RUNS
+      return launch_status();
+    }
     if (vec && most <= 256) {
 #define TLF_PREP_C(MAXC, TAPS)                                     \
   do {                                                             \
