@@ -358,6 +358,22 @@ def test_mixture_of_experts(dtype, n, width, E, top, ff, limit):
         assert clear.float().mean() > 0.5 and rel(got[clear], want[clear]) < (6e-3 if dtype == "bf16" else 2e-6), kind
 
 
+@pytest.mark.parametrize("n,width", [(131, 1984), (131, 2048), (257, 2048), (390, 1984)])
+def test_grouped_tiles_on_both_sides_of_a_short_reduction(n, width):
+    """128-row tiles: pairs of workgroups up to 31 K-tiles, one large tile beyond; both against fp32 products of the same rows."""
+    from tinyllmforge_amd import ops as P
+    g, E, ff = torch.Generator().manual_seed(n), 3, 136
+    x, w = torch.randn(n, width, generator=g).bfloat16().cuda(), (torch.randn(E, 2 * ff, width, generator=g) * width ** -0.5).bfloat16().cuda()
+    logits = torch.zeros(1, n, 16, device="cuda")
+    logits[0, torch.arange(n), torch.randint(0, E, (n,), generator=g)] = 5.0
+    rows = P.moe_group(logits, E, 1, 128)
+    got = P.moe_gemm(x, w, rows, gather=True, swiglu=True).float().cpu()[rows.row_of.cpu()[:, 0].long()]
+    y = torch.stack([x.float().cpu()[i] @ w[e].float().cpu().T for i, e in enumerate(rows.ids.cpu()[:, 0].tolist())]).view(n, -1, 2, 8)
+    want = (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).reshape(n, -1)
+    # gate and up are sums of a few units in fp32, 2^-20 off at most; one rounding to bf16
+    torch.testing.assert_close(got, want, rtol=2 ** -8, atol=2 ** -12)
+
+
 def test_consumers_add_up_split_projections():
     """A projection left as partial sums gives the bits of the finished one, in every kernel that may read it."""
     from tinyllmforge_amd import ops as P

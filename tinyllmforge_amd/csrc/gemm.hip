@@ -1594,12 +1594,19 @@ int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *sca
 //   2 rows (64 tokens, 32 experts of 768 at width 1024)     128 x 32: 19.2 / 11.8    64 x 32, K split by 4 wave sets: 26.0 / 14.8
 //   8 rows (64 tokens, 64 of 1536 at 4096)                  64 x 32, K split: 266 / 154    128 x 32: 290 / 140 (chosen for K < 4096)
 //   64 rows (512 tokens, 4096)                              256 x 128: 307 / 168     128 x 64: 347 / 186    128 x 128: 345 / 177
+// 128 rows run on eight waves, 256 x 128 with four waves (one per SIMD) behind it, as it was before; and with an activation behind a short K in
+// 128 x 128, two workgroups per CU: one's products run beside the other's first copies and activation, which are half of 16 K-tiles' time.
+//   113 rows (1021 tokens, 32 of 768 at 1024)               128 x 128 35.0, 256 x 128 41.4, four waves 48.0 / 256 x 128 19.6, 128 x 128 19.5, four waves 20.5
+//   390 rows (3500 tokens, 1024)                            61.5, 78.9, 87.4 / 36.8, 40.1, 39.1
+//   47 rows (400 tokens, 64 of 1536 at 4096)                256 x 128 347, 128 x 128 393, four waves 367 / 168, 174, 175
+//   350 rows (3000 tokens, 4096)                            699, 766, 718 / 383, 419, 384
 //   2048 rows (16,384 tokens, 4096)                         256 x 256: 3066 / 1704   256 x 128: 3187 / 1879 128 x 128: 3865 / 2298
 int launch_grouped(GemmParams p, int bm, hipStream_t stream) {
   if (p.N % 16 || p.K % kBK || p.m_tiles <= 0) return TLF_E_SHAPE;
   const int ktiles = p.K / kBK;
   const bool deep = bm == 32 && ktiles >= 64 && ktiles % 4 == 0;
-  const int bn = deep ? 64 : bm <= 64 ? 128 : 256;
+  const bool pairs = bm == 128 && p.act && ktiles < 32;
+  const int bn = deep ? 64 : bm <= 64 || pairs ? 128 : 256;
   p.splits = 1;
   p.k_per_split = p.K;
   p.n_tiles = (p.N + bn - 1) / bn;
@@ -1619,7 +1626,8 @@ int launch_grouped(GemmParams p, int bm, hipStream_t stream) {
   if (deep) TLF_GROUPED(64, 32, 2, 1, 3, 4, 4);
   else if (bm == 32) TLF_GROUPED(128, 32, 4, 1, 4, 4, 1);
   else if (bm == 64) TLF_GROUPED(128, 64, 4, 1, 2, 3, 1);
-  else if (bm == 128) TLF_GROUPED(256, 128, 2, 2, 3, 1, 1);
+  else if (pairs) TLF_GROUPED(128, 128, 4, 2, 2, 2, 1);
+  else if (bm == 128) TLF_GROUPED(256, 128, 4, 2, 3, 2, 1);
   else if (bm == 256) TLF_GROUPED(256, 256, 4, 2, 2, 2, 1);
   else return TLF_E_SHAPE;
 #undef TLF_GROUPED
