@@ -292,3 +292,23 @@ def test_embedding_bit_exact(ops):
     ids = torch.randint(0, 1000, (77,), generator=g(1))
     got = ops.embedding(ids.to(DEV), w.to(DEV))
     assert torch.equal(got.cpu().view(torch.int16), O.embedding(ids, w).view(torch.int16))
+
+
+def test_launches_follow_the_current_stream():
+    """The handle that wrappers launch on is torch's current stream, of each thread by itself."""
+    import threading
+    from tinyllmforge_amd import ops as P
+    own, other, seen = torch.cuda.Stream(), torch.cuda.Stream(), []
+
+    def elsewhere():
+        with torch.cuda.stream(other):
+            seen.append(P._stream())
+
+    default = torch.cuda.current_stream().cuda_stream
+    assert P._stream() == default
+    with torch.cuda.stream(own):
+        t = threading.Thread(target=elsewhere)
+        t.start()
+        t.join()
+        assert P._stream() == own.cuda_stream == torch.cuda.current_stream().cuda_stream
+    assert P._stream() == default and seen == [other.cuda_stream]
