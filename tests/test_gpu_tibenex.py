@@ -177,6 +177,30 @@ def test_talking_heads_over_paged_rows(dtype, sizes):
         assert rel(out[lens[0]:, :H * V], want[lens[0]:]) < tol
 
 
+@pytest.mark.parametrize("heads,rot,temp", [((4, 4, 128, 128), 128, True), ((8, 4, 128, 256), 64, False), ((32, 8, 128, 128), 128, True), ((16, 8, 128, 64), 0, True),
+                                            ((32, 16, 64, 64), 8, False)], ids=str)
+def test_preparation_of_many_rows(heads, rot, temp):
+    """From 2048 rows on, granules of whole waves: another kernel, against the one for few rows.  Squares are added up in another order."""
+    from tinyllmforge_amd import ops as P
+    (H, G, D, V), n, bs, BF, g = heads, 2051, 64, torch.bfloat16, torch.Generator(device="cuda").manual_seed(rot)
+    randn = lambda *s: torch.randn(*s, device="cuda", generator=g).to(BF)
+    proj, qn, kn, table = randn(n, (H + G) * D + G * V + 16), 1 + 0.1 * randn(H * D), 1 + 0.1 * randn(G * D), torch.randn(600, max(rot, 1), device="cuda", generator=g)
+    pos, slots = torch.randint(0, 600, (n,), device="cuda", generator=g), torch.randperm(40 * bs, device="cuda", generator=g)[:n].to(torch.int32)
+    slots[[0, 8, 2050]] = -1
+    pos[5] = 600                                                 # behind the table: not turned
+
+    def prepared(parts):
+        kv = P.SinkKV(40, bs, G, D, V, BF, "cuda")
+        q = [P.talk_prep(proj[a:b], kv, H, pos[a:b].contiguous(), slots[a:b].contiguous(), qn, kn, 1 + 0.1 * qn[:H] if temp else None, table if rot else None, rot,
+                         1e-5, 0.3) for a, b in parts]
+        return torch.cat(q), kv.k, kv.v
+
+    for got, want in zip(prepared([(0, n)]), prepared([(0, 1000), (1000, n)])):
+        # sums of up to 4096 squares in fp32: 2^-18 of the norm at most, then a bf16 rounding that may fall to the other side, 2^-7 of the
+        # value; a rotation takes the difference of two such values before it is rounded
+        torch.testing.assert_close(got.float(), want.float(), rtol=2 ** -7, atol=2 ** -14)
+
+
 # (tokens before the portion, its tokens): one long portion, a few rows behind a long context, a tile's edges, nothing to cut, unequal ones
 CUTS = [[(0, 1500)], [(2048, 40)], [(0, 31), (0, 32), (0, 33), (96, 64), (95, 65)], [(0, 20), (64, 1)], [(0, 700), (128, 513), (0, 64), (1000, 2)]]
 

@@ -101,8 +101,139 @@ __global__ __launch_bounds__(256) void talk_prep_kernel(const TalkPrepArgs a) {
   }
 }
 
+// The same for rows of prompts: bf16 projections, head dimensions that are padded nowhere, q of 64, 128, 256 or 512 granules of 8 values, k and v
+// of one of these.  A workgroup has eight rows of one part; WPR waves have a row, CH granules a lane, and NB rows each are on their way
+// at once: the kernel above waits for a row, for its sum and then for norm weights, cosines and sines.
+//
+// HBM bound: 12237 rows of 16 + 2 x 8 heads of 128, 200 MB, 65 us a row and part a workgroup, 53 so (a large copy 39); 32 heads 111 and 70.
+constexpr int kPrepRows = 8;
+
+template <int WPR, int CH>
+__device__ __forceinline__ void talk_prep_rows(const TalkPrepArgs &a, int kind, float (&part)[kPrepRows][4]) {
+  typedef unsigned short T;
+  constexpr int AT = 4 / WPR, NB = kPrepRows / AT < 4 / CH ? kPrepRows / AT : 4 / CH;   // rows at a time; of a thread
+  const SinkCache &c = a.c;
+  const int heads = kind == 0 ? a.H : c.G, dims = kind < 2 ? c.D : c.Dv, nch = dims / 8;
+  const int col0 = kind == 0 ? 0 : kind == 1 ? a.H * c.D : (a.H + c.G) * c.D;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, own = wave / WPR, half = a.rot_dims / 2;
+  uint4 x[NB][CH];
+  int piece[CH];
+#pragma unroll
+  for (int q = 0; q < CH; ++q) piece[q] = (q * WPR + wave % WPR) * 64 + lane;
+  for (int first = 0; first < kPrepRows; first += NB * AT) {
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kPrepRows + first + own;
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const T *from = static_cast<const T *>(a.proj) + min(row0 + k * AT, static_cast<int64_t>(a.n) - 1) * a.ld + col0;
+#pragma unroll
+    for (int q = 0; q < CH; ++q) x[k][q] = *reinterpret_cast<const uint4 *>(from + piece[q] * 8);
+  }
+  int64_t pos[NB];
+  int32_t slot[NB];
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const int64_t row = min(row0 + k * AT, static_cast<int64_t>(a.n) - 1);
+    pos[k] = a.positions[row];
+    slot[k] = a.slots[row];
+  }
+  float inv[NB];
+  uint4 w[CH];
+  if (kind < 2) {
+    const T *wp = static_cast<const T *>(kind == 0 ? a.q_norm : a.k_norm);
+#pragma unroll
+    for (int q = 0; q < CH; ++q) w[q] = *reinterpret_cast<const uint4 *>(wp + piece[q] * 8);
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      float ss = 0.f;
+#pragma unroll
+      for (int q = 0; q < CH; ++q) {
+        float f[8];
+        unpack8(x[k][q], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
+      }
+      inv[k] = wave_sum(ss);
+    }
+    if constexpr (WPR > 1) {
+      if (lane == 0)
+#pragma unroll
+        for (int k = 0; k < NB; ++k) part[first + own + k * AT][wave % WPR] = inv[k];
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        const float *s = part[first + own + k * AT];
+        inv[k] = WPR == 2 ? s[0] + s[1] : (s[0] + s[1]) + (s[2] + s[3]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NB; ++k) inv[k] = 1.0f / sqrtf(inv[k] / static_cast<float>(heads * dims) + a.eps);
+  }
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const int64_t row = row0 + k * AT;
+    const bool store = row < a.n && (kind == 0 || (slot[k] >= 0 && slot[k] < c.pages * c.bs));
+    const int page = c.bs_shift >= 0 ? slot[k] >> c.bs_shift : slot[k] / c.bs;
+    const bool turns = pos[k] >= 0 && pos[k] < a.max_pos && half;
+    const float *cs = a.cos_sin + (turns ? pos[k] : 0) * a.rot_dims;
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      const int head = piece[q] / nch, d = (piece[q] - head * nch) * 8;
+      uint4 out = x[k][q];
+      if (kind < 2) {
+        float f[8], wn[8];
+        unpack8(x[k][q], f);
+        unpack8(w[q], wn);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = f[e] * inv[k] * wn[e];
+        if (turns && d < a.rot_dims) {                               // rotations end between granules
+          const float4 co = *reinterpret_cast<const float4 *>(cs + d / 2), si = *reinterpret_cast<const float4 *>(cs + half + d / 2);
+          const float cv[4] = {co.x, co.y, co.z, co.w}, sv[4] = {si.x, si.y, si.z, si.w};
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            const float u = f[e], v = f[e + 1];
+            f[e] = __fmul_rn(u, cv[e / 2]) - __fmul_rn(v, sv[e / 2]);
+            f[e + 1] = __fmul_rn(v, cv[e / 2]) + __fmul_rn(u, sv[e / 2]);
+          }
+        }
+        if (kind == 0) {
+          const float m = a.q_scale * (a.temp ? Elem<T>::ld(static_cast<const T *>(a.temp) + head) : 1.f);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] *= m;
+        }
+        out = pack8(f);
+      }
+      if (!store) continue;
+      T *to = kind == 0 ? static_cast<T *>(a.q_out) + (row * a.H + head) * dims + d
+                        : static_cast<T *>(const_cast<void *>(kind == 1 ? c.k : c.v)) + ((static_cast<int64_t>(page) * c.G + head) * c.bs + (slot[k] - page * c.bs)) * dims + d;
+      *reinterpret_cast<uint4 *>(to) = out;
+    }
+  }
+  }
+}
+
+__global__ __launch_bounds__(256) void talk_prep_rows_kernel(const TalkPrepArgs a) {
+  __shared__ float part[kPrepRows][4];
+  const int kind = blockIdx.y, granules = (kind == 0 ? a.H * a.c.D : a.c.G * (kind == 1 ? a.c.D : a.c.Dv)) / 8;
+  if (granules == 512) talk_prep_rows<4, 2>(a, kind, part);
+  else if (granules == 256) talk_prep_rows<4, 1>(a, kind, part);
+  else if (granules == 128) talk_prep_rows<2, 1>(a, kind, part);
+  else talk_prep_rows<1, 1>(a, kind, part);
+}
+// Sizes it takes, from 2048 rows on (4000 rows of 16 heads 26 and 20 us, 2100 of 32 heads 22 and 22); with fewer, a row a workgroup fills the chip.
+inline bool talk_prep_takes_rows(const TalkPrepArgs &a) {
+  auto whole = [](int64_t granules) { return granules == 64 || granules == 128 || granules == 256 || granules == 512; };
+  const SinkCache &c = a.c;
+  return a.vec && a.n >= 2048 && c.D == c.Dp && c.Dv == c.Vp && a.rot_dims % 8 == 0 && (!a.rot_dims || aligned16(a.cos_sin)) &&
+         whole(static_cast<int64_t>(a.H) * c.D / 8) && whole(static_cast<int64_t>(c.G) * c.D / 8) && whole(static_cast<int64_t>(c.G) * c.Dv / 8);
+}
+
 template <typename T, bool PART>
 int launch_talk_prep(const TalkPrepArgs &a, int pieces, hipStream_t s) {
+  if constexpr (sizeof(T) == 2 && !PART)
+    if (talk_prep_takes_rows(a)) {
+      TLF_LAUNCH(talk_prep_rows_kernel, dim3((a.n + kPrepRows - 1) / kPrepRows, 3), dim3(256), 0, s, a);
+      return launch_status();
+    }
   const dim3 grid(a.n, 3);
   if (pieces <= 256) TLF_LAUNCH((talk_prep_kernel<T, 1, PART>), grid, dim3(256), 0, s, a);
   else if (pieces <= 512) TLF_LAUNCH((talk_prep_kernel<T, 2, PART>), grid, dim3(256), 0, s, a);
