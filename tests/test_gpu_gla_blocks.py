@@ -121,3 +121,12 @@ def test_short_portions_keep_the_chunks(H, dk, dv, lens, kernels):
     for n, out, state in run(H, dk, dv, 16, lens, [5] * len(lens), 8.0, dk):
         assert out < OUT and state < STATE, (n, out, state)
     assert count() - before == kernels
+
+
+@pytest.mark.parametrize("lens,start", [([1500, 33, 1700, 2, 1024, 32], [0, 5, 7, 0, 64, 0]), ([2047], [3]), ([512, 512, 512, 512], [0, 1, 0, 1]),
+                                        ([17, 3000, 31, 40], [1, 1, 0, 9]), ([640, 1, 640], [1, 1, 1])], ids=str)
+@pytest.mark.parametrize("H,dk,dv", [(2, 128, 256), (3, 64, 96)])
+def test_stretches_over_sequences(H, dk, dv, lens, start):
+    """Stretches that begin and end anywhere: within a sequence, at its ends, several sequences in one, one sequence in many."""
+    for n, out, state in run(H, dk, dv, 16, lens, start, 16.0, sum(lens)):
+        assert out < OUT and state < STATE, (n, out, state)

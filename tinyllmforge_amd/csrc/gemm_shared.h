@@ -302,6 +302,15 @@ __device__ __forceinline__ void gemm_epilogue_activated(const GemmParams &p, flo
 // (they count as LDS writes), which is exactly the wait the pipeline must not do.
 #define TLF_DL_BARRIER(N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory")
 
+// The same with nothing under way, for loops that also load into registers: the wait is the compiler's own kind, so it knows that what was loaded
+// before is there.  Behind TLF_DL_BARRIER(0) it would wait again where such a value is first used, and by its count of loads under way: for all
+// but a few of the copies that were issued in between, which it does not see.
+#define TLF_DL_BARRIER_KNOWN()                   \
+  do {                                           \
+    __builtin_amdgcn_s_waitcnt(0x0f70); /* vmcnt(0) */ \
+    TLF_DL_BARRIER(0);                           \
+  } while (0)
+
 // The copies are issued from inline asm so that the compiler does not see them: it cannot tell
 // which LDS object a copy writes, and would otherwise wait for every outstanding copy (and for
 // every outstanding LDS read) before each ds_read.  Ordering is explicit instead: TLF_DL_BARRIER.

@@ -31,7 +31,8 @@ struct GlaArgs {
   float *rec, *o;
   int32_t vec;                            // bf16 projection rows may be read 8 bytes at a time, key dim a full row
   int32_t segs;                           // segments per sequence
-  float *seg_state, *seg_dec;             // [seqs, segs, H, dk, dv], [seqs, segs, H, DKP]
+  float *seg_state, *seg_dec;             // [seqs, segs, H, dk, dv], [seqs, segs, H, DKP]; of stretches (gla_blocks.hip): [2, units, H, ..], [units, H, ..]
+  int32_t units;                          // stretches of all sequences' blocks, 0: whole sequences
 };
 
 // log2 of sigmoid(z)^(1/tau) = -(max(-z, 0) log2 e + log2(1 + e)) / tau with e = 2^(-|z| log2 e).  log2(1 + e) keeps its
@@ -49,7 +50,5 @@ bool gla_blocks_take(const GlaArgs &a, int32_t dtype, int chunk_segs);     // ch
 bool gla_blocks_sizes(int32_t key_dim, int32_t value_dim);
 size_t gla_blocks_workspace_bytes(int32_t chunks, int32_t num_seqs, int32_t heads, int32_t key_dim, int32_t value_dim);
 int launch_gla_blocks(GlaArgs &a, int first_seq, void *workspace, hipStream_t stream);
-// Contributions of the segments -> the state each of them starts from, in place.
-void launch_gla_segments(const GlaArgs &a, int first_seq, int dkp, hipStream_t stream);
 
 }  // namespace tlf

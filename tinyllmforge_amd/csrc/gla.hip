@@ -474,10 +474,6 @@ __global__ __launch_bounds__(256) void gla_segments_kernel(const GlaArgs a, int 
   }
 }
 
-void launch_gla_segments(const GlaArgs &a, int first_seq, int dkp, hipStream_t stream) {
-  TLF_LAUNCH(gla_segments_kernel, dim3((a.dk * a.dv + 255) / 256, a.H, a.seqs), dim3(256), 0, stream, a, first_seq, dkp);
-}
-
 // One wave per (row of a chunk, head).
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void gla_out_kernel(const GlaArgs a) {
@@ -571,7 +567,7 @@ int launch_gla_portions(GlaArgs &a, int first_seq, hipStream_t stream) {
       TLF_LAUNCH((gla_scan_kernel<T, NT, 0>), sgrid, dim3(256), 0, stream, a, first_seq);              \
     } else {                                                                                              \
       TLF_LAUNCH((gla_scan_kernel<T, NT, 1>), sgrid, dim3(256), 0, stream, a, first_seq);              \
-      launch_gla_segments(a, first_seq, (NT) * 16, stream);                                               \
+      TLF_LAUNCH(gla_segments_kernel, dim3((a.dk * a.dv + 255) / 256, a.H, a.seqs), dim3(256), 0, stream, a, first_seq, (NT) * 16); \
       TLF_LAUNCH((gla_scan_kernel<T, NT, 2>), sgrid, dim3(256), 0, stream, a, first_seq);              \
     }                                                                                                     \
   } while (0)

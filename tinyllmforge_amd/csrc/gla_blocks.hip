@@ -15,13 +15,19 @@
 //                          out.  A block's record and rows of v come into LDS one block ahead, and the rows' sums of squares
 //                          go from wave to wave across the barrier in front of the next block.
 //                          A value that is no number reaches no row before its half of a block
-// Where (sequences, heads) alone leave CUs idle a sequence is cut into segments as in gla.hip.
+// Where (sequences, heads) alone leave CUs idle, the blocks of all sequences in a row are cut into `units` equal stretches, one workgroup per
+// stretch and head: a stretch has the end of a sequence, whole ones, the beginning of another.  What a stretch adds to the sequence that it does
+// not end comes from a first pass over that sequence's blocks in it (MODE 1), gla_stretches_kernel chains these, and the second pass starts from
+// them.  Segments of a sequence's own length waited for the longest: 8 sequences of 1061 to 2048 tokens, 16 heads of 128 x 256, with
+// segments 59 + 18 + 255 us, so 58 + 15 + 209; 12 of 450 to 900 48 + 24 + 216, and in one pass over whole ones 204.
 //
 // Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256, medians under the profiler: chunk 122 + scan 470 (both
 // passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 149 + first pass 62 + segments 19 + scan
 // 278 us (whole layer without it 614 and 449 us).  The blocks write 55 KB a record, 4 TB/s with what they read; the scan is held by its
 // barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's error against 64 bits is 5e-8 to 1.1e-7 on both, the
 // output's is its rounding to bf16.
+#include <algorithm>
+
 #include "gemm_shared.h"
 #include "gla.h"
 
@@ -259,8 +265,30 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   }
 }
 
-// MODE 0: the whole sequence from the state slot and back.  MODE 1: a segment's own contribution from zero.  MODE 2: a segment from
-// the state gla_segments_kernel left for it.
+// A value that is the same in all lanes and that nothing in the launch writes, through the scalar path: behind stores of an earlier sequence the
+// compiler would load it for every lane.
+template <typename T>
+__device__ __forceinline__ T gla_uniform(const T *p) {
+  return *(const T __attribute__((address_space(4))) *)(reinterpret_cast<uintptr_t>(p));
+}
+
+// Lane s: sequence s has the blocks first .. end - 1 of all of them, lanes behind the last sequence none.  Up to 64 sequences.
+__device__ __forceinline__ void gla_block_ranges(const GlaArgs &a, int lane, int &first, int &end, int &all) {
+  const int n = lane < a.seqs ? (a.cu_chunks[lane + 1] - a.cu_chunks[lane] + 1) / 2 : 0;
+  end = n;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int x = __shfl_up(end, d, 64);
+    end += lane >= d ? x : 0;
+  }
+  first = end - n;
+  all = __builtin_amdgcn_readlane(end, 63);
+}
+__device__ __forceinline__ int gla_stretch_begin(int unit, int units, int all) { return static_cast<int>(static_cast<int64_t>(unit) * all / units); }
+__device__ __forceinline__ int gla_stretch_of(int block, int units, int all) { return static_cast<int>(((block + 1ll) * units - 1) / all); }
+
+// MODE 0: the whole sequence from the state slot and back.  MODE 1: from zero, what a stretch adds to the sequence that goes on behind it.
+// MODE 2: a stretch; that sequence starts from seg_state[unit], one that began before the stretch and ends in it from seg_state[units + unit].
 template <int DK, int MODE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gla_block_scan_kernel(const GlaArgs a, int first_seq) {
   typedef unsigned short T;
@@ -269,37 +297,62 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = a.dv / 32;
-  const int h = blockIdx.x, seq = MODE == 0 ? blockIdx.z : blockIdx.z / a.segs, seg = MODE == 0 ? 0 : blockIdx.z % a.segs;
-  const bool last_seg = MODE == 0 || seg == a.segs - 1;
-  if (MODE == 1 && last_seg) return;                         // nobody starts behind the last segment
+  const int h = blockIdx.x;
   const unsigned int recs = TLF_DL_LDSADDR(lds), vs = recs + 2 * Rec::kSize + wave * 2 * VB;
   float *rowsum = reinterpret_cast<float *>(lds + 2 * Rec::kSize + waves * 2 * VB);        // [2][waves][32]
-  const int slot = a.state_slots[first_seq + seq];
+  int *const ranges = reinterpret_cast<int *>(rowsum + 2 * waves * 32);                    // MODE 1 and 2: [2][64]
+  unsigned long long left = 1;                               // sequences of the stretch
+  int lo = 0, hi_block = 0;
+  if constexpr (MODE != 0) {
+    int first, end, all;
+    gla_block_ranges(a, lane, first, end, all);
+    if (all == 0) return;
+    lo = gla_stretch_begin(blockIdx.z, a.units, all);
+    hi_block = gla_stretch_begin(blockIdx.z + 1, a.units, all);
+    left = __ballot(first < hi_block && end > lo);
+    if (left == 0) return;
+    if constexpr (MODE == 1) {
+      const int last = 63 - __builtin_clzll(left);
+      if (__builtin_amdgcn_readlane(end, last) <= hi_block) return;    // the stretch ends with it
+      left = 1ull << last;
+    }
+    if (wave == 0) {
+      ranges[lane] = first;
+      ranges[64 + lane] = end;
+    }
+    lds_barrier();
+  }
+  do {
+  const int seq = MODE == 0 ? blockIdx.z : __builtin_ctzll(left);
+  const int first_block = MODE == 0 ? 0 : __builtin_amdgcn_readfirstlane(ranges[seq]), end_block = MODE == 0 ? 0 : __builtin_amdgcn_readfirstlane(ranges[64 + seq]);
+  const bool ends = MODE == 0 || end_block <= hi_block, begins = MODE == 0 || first_block >= lo;
+  const int slot = gla_uniform(a.state_slots + first_seq + seq);
   const bool slot_ok = slot >= 0 && slot < a.num_slots;
   float *st = a.state + (static_cast<int64_t>(slot_ok ? slot : 0) * a.H + h) * DK * a.dv;
-  const int64_t sg = (static_cast<int64_t>(seq) * a.segs + seg) * a.H + h;
-  float *gst = MODE == 0 ? st : a.seg_state + sg * DK * a.dv;
-  const bool from_zero = MODE == 1 || (MODE == 0 && (!slot_ok || a.starts[first_seq + seq] == 0));
-  const int col = wave * 32 + n;
-  // lane (hi, n), register r of tile i: row 32 i + 8 (r / 4) + 4 hi + r % 4 of column n
+  const int64_t sg = static_cast<int64_t>(MODE != 0 && ends ? a.units + blockIdx.z : blockIdx.z) * a.H + h;
+  float *gst = ends && begins ? st : a.seg_state + sg * DK * a.dv;
+  const bool from_zero = MODE == 1 || (ends && begins && (!slot_ok || a.starts[first_seq + seq] == 0));
+  // lane (hi, n), register r of tile i: row 32 i + 8 (r / 4) + 4 hi + r % 4 of column n.  A row's address is the same in all lanes and the lane's part
+  // one register: 64 addresses would go to memory, and each that comes back waits for all values before it.
+  const unsigned int mine = static_cast<unsigned int>(hi * 4 * a.dv + wave * 32 + n) * 4;
+  auto row_of = [&](int i, int r) __attribute__((always_inline)) { return static_cast<int64_t>(i * 32 + (r >> 2) * 8 + (r & 3)) * a.dv * 4; };
   floatx16 S[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = i * 32 + (r >> 2) * 8 + hi * 4 + (r & 3);
-      S[i][r] = from_zero ? 0.f : gst[static_cast<int64_t>(d) * a.dv + col];
-    }
-  const int64_t hk = static_cast<int64_t>(a.H) * DK;
-  const int cbeg = a.cu_chunks[seq], cend = a.cu_chunks[seq + 1], blocks = (cend - cbeg + 1) / 2;
-  const int64_t row0 = cbeg < cend ? a.chunk_tok[cbeg] : 0;
-  const int tokens = cbeg < cend ? (cend - 1 - cbeg) * 16 + a.chunk_len[cend - 1] : 0;
-  int b0 = 0, b1 = blocks;
-  if (MODE != 0) {
-    const int per = (blocks + a.segs - 1) / a.segs;
-    b0 = min(seg * per, blocks);
-    b1 = min(b0 + per, blocks);
+    for (int r = 0; r < 16; ++r) S[i][r] = 0.f;
+  if (!from_zero) {
+    const char *from = reinterpret_cast<const char *>(gst);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) S[i][r] = *reinterpret_cast<const float *>(from + row_of(i, r) + mine);
   }
+  const int64_t hk = static_cast<int64_t>(a.H) * DK;
+  const int cbeg = gla_uniform(a.cu_chunks + seq), cend = gla_uniform(a.cu_chunks + seq + 1), blocks = (cend - cbeg + 1) / 2;
+  const int64_t row0 = cbeg < cend ? gla_uniform(a.chunk_tok + cbeg) : 0;
+  const int tokens = cbeg < cend ? (cend - 1 - cbeg) * 16 + gla_uniform(a.chunk_len + cend - 1) : 0;
+  const int b0 = MODE == 0 ? 0 : max(lo - first_block, 0), b1 = MODE == 0 ? blocks : min(hi_block - first_block, blocks);
   const T *vbase = static_cast<const T *>(a.proj) + 2 * hk + static_cast<int64_t>(h) * a.dv + wave * 32;
   const T *gbase = vbase + static_cast<int64_t>(a.H) * a.dv + hi * 4;
   const unsigned char *rbase = reinterpret_cast<const unsigned char *>(a.rec) + (static_cast<int64_t>(gla_first_block(cbeg, seq)) * a.H + h) * Rec::kSize;
@@ -352,7 +405,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     int here = tid & 63;
     asm volatile("" : "+v"(here));
     const int lane = here, n = here & 31, hi = here >> 5;
-    TLF_DL_BARRIER(0);
+    TLF_DL_BARRIER_KNOWN();                                  // the gate of the block before, too
     if (b + 1 < b1) copy(b + 1, buf ^ 1);
     if constexpr (MODE != 1) {
       if (b > b0) put(b - 1, buf ^ 1);
@@ -475,16 +528,45 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   } else {
     if (b0 < b1) {
-      TLF_DL_BARRIER(0);
+      TLF_DL_BARRIER_KNOWN();
       put(b1 - 1, (b1 - 1 - b0) & 1);
     }
-    if (!last_seg || !slot_ok) return;
   }
-  float *dst = MODE == 1 ? gst : st;
+  if (MODE == 1 || (ends && slot_ok)) {
+    char *to = reinterpret_cast<char *>(MODE == 1 ? gst : st);
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) dst[static_cast<int64_t>(i * 32 + (r >> 2) * 8 + hi * 4 + (r & 3)) * a.dv + col] = S[i][r];
+      for (int r = 0; r < 16; ++r) *reinterpret_cast<float *>(to + row_of(i, r) + mine) = S[i][r];
+  }
+  left &= left - 1;
+  } while (MODE == 2 && left);
+}
+
+// What the stretches add to a sequence -> the states they start from: seg_state[unit] in place, seg_state[units + unit] where it ends.
+__global__ __launch_bounds__(256) void gla_stretches_kernel(const GlaArgs a, int first_seq) {
+  const int64_t plane = static_cast<int64_t>(a.dk) * a.dv, e = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+  const int h = blockIdx.y, seq = blockIdx.z;
+  int first, end, all;
+  gla_block_ranges(a, threadIdx.x & 63, first, end, all);
+  first = __builtin_amdgcn_readlane(first, seq);
+  end = __builtin_amdgcn_readlane(end, seq);
+  if (first == end) return;
+  const int from = gla_stretch_of(first, a.units, all), to = gla_stretch_of(end - 1, a.units, all);
+  if (from == to || e >= plane) return;                      // in one stretch
+  const int slot = a.state_slots[first_seq + seq];
+  const bool from_zero = slot < 0 || slot >= a.num_slots || a.starts[first_seq + seq] == 0;
+  auto at = [&](float *states, int64_t i) __attribute__((always_inline)) { return reinterpret_cast<float4 *>(states + (i * a.H + h) * plane + e); };
+  float4 run = from_zero ? make_float4(0.f, 0.f, 0.f, 0.f) : *at(a.state, slot);
+  const int d = static_cast<int>(e / a.dv);
+  for (int u = from; u < to; ++u) {
+    float4 *const p = at(a.seg_state, u);
+    const float4 own = *p;
+    const float dec = a.seg_dec[(static_cast<int64_t>(u) * a.H + h) * a.dk + d];
+    *p = run;
+    run = make_float4(fmaf(dec, run.x, own.x), fmaf(dec, run.y, own.y), fmaf(dec, run.z, own.z), fmaf(dec, run.w, own.w));
+  }
+  *at(a.seg_state, a.units + to) = run;
 }
 
 // A workgroup of the scan has a wave per 32 value columns and holds two records, 117 KB with 128 keys: with fewer than three waves there, or
@@ -496,11 +578,19 @@ bool gla_blocks_sizes(int32_t dk, int32_t dv) {
   return (dk == 32 || dk == 64 || dk == 128) && dv % 32 == 0 && dv >= (dk == 128 ? 96 : 64) && dv <= 256;
 }
 
-// Segments per sequence: a workgroup for every CU (two where LDS holds two), segments of at least 8 blocks.
+// Segments that a sequence would have: a workgroup for every CU (two where LDS holds two), segments of at least 8 blocks.
 int gla_block_segments(int chunks, int seqs, int heads, int dk) {
   const int64_t wgs = static_cast<int64_t>(seqs) * heads, full = dk == 128 ? 256 : 512, want = wgs >= full ? 1 : (full + wgs - 1) / wgs, most = chunks / seqs / 16;
   const int64_t s = want < most ? want : most;
   return static_cast<int>(s < 1 || seqs * s > 65535 ? 1 : s > 32 ? 32 : s);
+}
+
+// Stretches, 0: whole sequences.  A workgroup for every CU, with a stretch of at least 8 blocks; not where there are hardly more stretches than
+// sequences, which would be cut for little.
+int gla_block_units(int chunks, int seqs, int heads, int dk) {
+  if (seqs > 64 || chunks > (1 << 20) || gla_block_segments(chunks, seqs, heads, dk) == 1) return 0;
+  const int units = std::min((dk == 128 ? 256 : 512) / heads, chunks / 16);
+  return units * 2 >= seqs * 3 && units > 1 ? units : 0;
 }
 
 // Whether the scan over 16-token chunks does as well: where its waves, one per 16 value columns, are all on the chip at once, in one segment,
@@ -524,15 +614,15 @@ bool gla_blocks_take(const GlaArgs &a, int32_t dtype, int chunk_segs) {
 }
 
 size_t gla_blocks_workspace_bytes(int32_t chunks, int32_t seqs, int32_t heads, int32_t dk, int32_t dv) {
-  const size_t slots = (static_cast<size_t>(chunks) + seqs + 1) / 2 + 1, segs = gla_block_segments(chunks, seqs, heads, dk);
-  return slots * heads * gla_block_record(dk) + (segs > 1 ? 4 * segs * seqs * heads * (dk + static_cast<size_t>(dk) * dv) : 0);
+  const size_t slots = (static_cast<size_t>(chunks) + seqs + 1) / 2 + 1, units = gla_block_units(chunks, seqs, heads, dk);
+  return slots * heads * gla_block_record(dk) + 4 * units * heads * (dk + 2 * static_cast<size_t>(dk) * dv);
 }
 
 template <int DK>
 int launch_gla_blocks_of(GlaArgs &a, int first_seq, hipStream_t stream) {
   const int waves = a.dv / 32;
-  const size_t lds = 2 * GlaBlock<DK>::kSize + waves * (2 * kGB * 32 * 2 + 2 * 32 * 4);
-  constexpr int kMost = 2 * GlaBlock<DK>::kSize + 8 * (2 * kGB * 32 * 2 + 2 * 32 * 4);
+  const size_t lds = 2 * GlaBlock<DK>::kSize + waves * (2 * kGB * 32 * 2 + 2 * 32 * 4) + (a.units ? 2 * 64 * 4 : 0);
+  constexpr int kMost = 2 * GlaBlock<DK>::kSize + 8 * (2 * kGB * 32 * 2 + 2 * 32 * 4) + 2 * 64 * 4;
   static const hipError_t allowed = [] {
     hipError_t e = hipSuccess;
     for (const void *k : {reinterpret_cast<const void *>(&gla_block_scan_kernel<DK, 0>), reinterpret_cast<const void *>(&gla_block_scan_kernel<DK, 1>),
@@ -542,23 +632,23 @@ int launch_gla_blocks_of(GlaArgs &a, int first_seq, hipStream_t stream) {
   }();
   if (allowed != hipSuccess) return static_cast<int>(allowed);
   TLF_LAUNCH((gla_block_kernel<DK>), dim3(a.chunks, a.H), dim3(DK * 4), 0, stream, a);
-  const dim3 grid(a.H, 1, a.seqs * a.segs);
-  if (a.segs == 1) {
-    TLF_LAUNCH((gla_block_scan_kernel<DK, 0>), grid, dim3(waves * 64), lds, stream, a, first_seq);
+  if (!a.units) {
+    TLF_LAUNCH((gla_block_scan_kernel<DK, 0>), dim3(a.H, 1, a.seqs), dim3(waves * 64), lds, stream, a, first_seq);
   } else {
+    const dim3 grid(a.H, 1, a.units);
     TLF_LAUNCH((gla_block_scan_kernel<DK, 1>), grid, dim3(waves * 64), lds, stream, a, first_seq);
-    launch_gla_segments(a, first_seq, DK, stream);
+    TLF_LAUNCH(gla_stretches_kernel, dim3((DK * a.dv + 1023) / 1024, a.H, a.seqs), dim3(256), 0, stream, a, first_seq);
     TLF_LAUNCH((gla_block_scan_kernel<DK, 2>), grid, dim3(waves * 64), lds, stream, a, first_seq);
   }
   return launch_status();
 }
 
 int launch_gla_blocks(GlaArgs &a, int first_seq, void *workspace, hipStream_t stream) {
-  a.segs = gla_block_segments(a.chunks, a.seqs, a.H, a.dk);
+  a.units = aligned16(a.state) ? gla_block_units(a.chunks, a.seqs, a.H, a.dk) : 0;
   const size_t slots = (static_cast<size_t>(a.chunks) + a.seqs + 1) / 2 + 1;
   a.rec = static_cast<float *>(workspace);
   a.seg_dec = a.rec + slots * a.H * gla_block_record(a.dk) / 4;
-  a.seg_state = a.seg_dec + static_cast<size_t>(a.seqs) * a.segs * a.H * a.dk;
+  a.seg_state = a.seg_dec + static_cast<size_t>(a.units) * a.H * a.dk;
   switch (a.dk) {
     case 32: return launch_gla_blocks_of<32>(a, first_seq, stream);
     case 64: return launch_gla_blocks_of<64>(a, first_seq, stream);
