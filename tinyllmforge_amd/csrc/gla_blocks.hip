@@ -265,27 +265,8 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   }
 }
 
-// A value that is the same in all lanes and that nothing in the launch writes, through the scalar path: behind stores of an earlier sequence the
-// compiler would load it for every lane.
-template <typename T>
-__device__ __forceinline__ T gla_uniform(const T *p) {
-  return *(const T __attribute__((address_space(4))) *)(reinterpret_cast<uintptr_t>(p));
-}
-
-// Lane s: sequence s has the blocks first .. end - 1 of all of them, lanes behind the last sequence none.  Up to 64 sequences.
-__device__ __forceinline__ void gla_block_ranges(const GlaArgs &a, int lane, int &first, int &end, int &all) {
-  const int n = lane < a.seqs ? (a.cu_chunks[lane + 1] - a.cu_chunks[lane] + 1) / 2 : 0;
-  end = n;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int x = __shfl_up(end, d, 64);
-    end += lane >= d ? x : 0;
-  }
-  first = end - n;
-  all = __builtin_amdgcn_readlane(end, 63);
-}
-__device__ __forceinline__ int gla_stretch_begin(int unit, int units, int all) { return static_cast<int>(static_cast<int64_t>(unit) * all / units); }
-__device__ __forceinline__ int gla_stretch_of(int block, int units, int all) { return static_cast<int>(((block + 1ll) * units - 1) / all); }
+// Lane s: blocks of sequence s.
+__device__ __forceinline__ int gla_own_blocks(const GlaArgs &a, int lane) { return lane < a.seqs ? (a.cu_chunks[lane + 1] - a.cu_chunks[lane] + 1) / 2 : 0; }
 
 // MODE 0: the whole sequence from the state slot and back.  MODE 1: from zero, what a stretch adds to the sequence that goes on behind it.
 // MODE 2: a stretch; that sequence starts from seg_state[unit], one that began before the stretch and ends in it from seg_state[units + unit].
@@ -305,10 +286,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   int lo = 0, hi_block = 0;
   if constexpr (MODE != 0) {
     int first, end, all;
-    gla_block_ranges(a, lane, first, end, all);
+    stretch_ranges(gla_own_blocks(a, lane), first, end, all);
     if (all == 0) return;
-    lo = gla_stretch_begin(blockIdx.z, a.units, all);
-    hi_block = gla_stretch_begin(blockIdx.z + 1, a.units, all);
+    lo = stretch_begin(blockIdx.z, a.units, all);
+    hi_block = stretch_begin(blockIdx.z + 1, a.units, all);
     left = __ballot(first < hi_block && end > lo);
     if (left == 0) return;
     if constexpr (MODE == 1) {
@@ -326,7 +307,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int seq = MODE == 0 ? blockIdx.z : __builtin_ctzll(left);
   const int first_block = MODE == 0 ? 0 : __builtin_amdgcn_readfirstlane(ranges[seq]), end_block = MODE == 0 ? 0 : __builtin_amdgcn_readfirstlane(ranges[64 + seq]);
   const bool ends = MODE == 0 || end_block <= hi_block, begins = MODE == 0 || first_block >= lo;
-  const int slot = gla_uniform(a.state_slots + first_seq + seq);
+  const int slot = load_uniform(a.state_slots + first_seq + seq);
   const bool slot_ok = slot >= 0 && slot < a.num_slots;
   float *st = a.state + (static_cast<int64_t>(slot_ok ? slot : 0) * a.H + h) * DK * a.dv;
   const int64_t sg = static_cast<int64_t>(MODE != 0 && ends ? a.units + blockIdx.z : blockIdx.z) * a.H + h;
@@ -349,9 +330,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int r = 0; r < 16; ++r) S[i][r] = *reinterpret_cast<const float *>(from + row_of(i, r) + mine);
   }
   const int64_t hk = static_cast<int64_t>(a.H) * DK;
-  const int cbeg = gla_uniform(a.cu_chunks + seq), cend = gla_uniform(a.cu_chunks + seq + 1), blocks = (cend - cbeg + 1) / 2;
-  const int64_t row0 = cbeg < cend ? gla_uniform(a.chunk_tok + cbeg) : 0;
-  const int tokens = cbeg < cend ? (cend - 1 - cbeg) * 16 + gla_uniform(a.chunk_len + cend - 1) : 0;
+  const int cbeg = load_uniform(a.cu_chunks + seq), cend = load_uniform(a.cu_chunks + seq + 1), blocks = (cend - cbeg + 1) / 2;
+  const int64_t row0 = cbeg < cend ? load_uniform(a.chunk_tok + cbeg) : 0;
+  const int tokens = cbeg < cend ? (cend - 1 - cbeg) * 16 + load_uniform(a.chunk_len + cend - 1) : 0;
   const int b0 = MODE == 0 ? 0 : max(lo - first_block, 0), b1 = MODE == 0 ? blocks : min(hi_block - first_block, blocks);
   const T *vbase = static_cast<const T *>(a.proj) + 2 * hk + static_cast<int64_t>(h) * a.dv + wave * 32;
   const T *gbase = vbase + static_cast<int64_t>(a.H) * a.dv + hi * 4;
@@ -548,11 +529,11 @@ __global__ __launch_bounds__(256) void gla_stretches_kernel(const GlaArgs a, int
   const int64_t plane = static_cast<int64_t>(a.dk) * a.dv, e = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
   const int h = blockIdx.y, seq = blockIdx.z;
   int first, end, all;
-  gla_block_ranges(a, threadIdx.x & 63, first, end, all);
+  stretch_ranges(gla_own_blocks(a, threadIdx.x & 63), first, end, all);
   first = __builtin_amdgcn_readlane(first, seq);
   end = __builtin_amdgcn_readlane(end, seq);
   if (first == end) return;
-  const int from = gla_stretch_of(first, a.units, all), to = gla_stretch_of(end - 1, a.units, all);
+  const int from = stretch_of(first, a.units, all), to = stretch_of(end - 1, a.units, all);
   if (from == to || e >= plane) return;                      // in one stretch
   const int slot = a.state_slots[first_seq + seq];
   const bool from_zero = slot < 0 || slot >= a.num_slots || a.starts[first_seq + seq] == 0;
