@@ -380,7 +380,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
       const int seq = a.row_seq ? a.row_seq[tok] : static_cast<int>(tok), st = a.state_slots[seq];
       const int first = a.row_seq ? a.cu_q[seq] : static_cast<int>(tok);
       r.back = static_cast<int>(min(tok - first, static_cast<int64_t>(kBack)));
-      r.end = a.row_seq ? static_cast<int>(min(a.cu_q[seq + 1] - tok0, static_cast<int64_t>(count))) : tid + 1;
+      // never at or before the row itself, whatever the offsets say: the loop below goes on from here
+      r.end = a.row_seq ? max(static_cast<int>(min(a.cu_q[seq + 1] - tok0, static_cast<int64_t>(count))), tid + 1) : tid + 1;
       r.single = !a.row_seq || a.cu_q[seq + 1] - first == 1;
       r.state = st >= 0 && st < a.num_state_slots && r.pos >= 0 ? st : -1;
     }
