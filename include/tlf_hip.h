@@ -569,7 +569,9 @@ int tlf_pooled_attn_prefill(const void *q, const void *score_bias, const float *
  * tlf_gla_portions: sequences first_seq .. + num_seqs - 1 of the step (state_slots and seq_starts are indexed by the
  *   step's sequences, a start of 0 begins with a zero state).  Their tokens are cut into chunks of 16 that do not cross a
  *   sequence (a sequence's last chunk may be shorter) and follow each other: chunk c holds the chunk_lens[c] rows from chunk_rows[c] on, counted from the row `proj` and
- *   `out` point to; sequence first_seq + s owns the chunks cu_chunks[s] .. cu_chunks[s + 1] - 1.  `rows` rows in all. */
+ *   `out` point to; sequence first_seq + s owns the chunks cu_chunks[s] .. cu_chunks[s + 1] - 1.  `rows` rows in all.
+ * tlf_gla_portions_upto: the same where the caller knows that no sequence brings more than max_tokens tokens (0: it does not): it decides
+ *   whether long sequences are cut.  The same workspace. */
 int tlf_gla_decode(const void *proj, int64_t proj_stride, const float *partials, int32_t splits,
                    const float *scale, const void *a2, const void *a2_bias,
                    const void *norm_weight, float *state, const int32_t *state_slots, int32_t num_slots,
@@ -585,6 +587,13 @@ int tlf_gla_portions(const void *proj, int64_t proj_stride, const void *a2, cons
                      int64_t out_stride, int32_t rows, int32_t heads, int32_t key_dim, int32_t value_dim,
                      int32_t rank, float tau, float q_scale, float eps, int32_t dtype, void *workspace,
                      size_t workspace_bytes, void *stream);
+int tlf_gla_portions_upto(const void *proj, int64_t proj_stride, const void *a2, const void *a2_bias,
+                          const void *norm_weight, float *state, const int32_t *state_slots, int32_t num_slots,
+                          const int32_t *seq_starts, const int32_t *chunk_rows, const int32_t *chunk_lens,
+                          const int32_t *cu_chunks, int32_t chunks, int32_t first_seq, int32_t num_seqs, int32_t max_tokens,
+                          void *out, int64_t out_stride, int32_t rows, int32_t heads, int32_t key_dim, int32_t value_dim,
+                          int32_t rank, float tau, float q_scale, float eps, int32_t dtype, void *workspace,
+                          size_t workspace_bytes, void *stream);
 
 /* Residual add with a multiplier and the next RMSNorm, for layers whose sublayers share one norm:
  *   x += mult * (y + sum_k extra[extra_rows[row * top + k]], k < top);   h = x / rms(x) * (w_next + w_offset)

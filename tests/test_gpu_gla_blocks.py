@@ -18,7 +18,7 @@ def portions(lens):
     return [torch.tensor(x, dtype=torch.int32, device="cuda") for x in (crow, clen, cu)]
 
 
-def run(H, dk, dv, rank, lens, start, tau, seed, lost=None, scale=1.0):
+def run(H, dk, dv, rank, lens, start, tau, seed, lost=None, scale=1.0, known=True):
     from tinyllmforge_amd import ops as P
     g, dt, eps = torch.Generator().manual_seed(seed), torch.bfloat16, 1e-5
     proj = [torch.randn(n, 2 * H * (dk + dv) + rank, generator=g).to(dt) for n in lens]
@@ -34,7 +34,7 @@ def run(H, dk, dv, rank, lens, start, tau, seed, lost=None, scale=1.0):
     out = torch.full((sum(lens), H * dv), 7.0, dtype=dt, device="cuda")
     t = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
     P.gla_portions(torch.cat(proj).cuda(), a2.cuda(), a2b.cuda(), nw.cuda(), state, t([i + 1 for i in range(len(lens))]), t(start), *portions(lens), 0, len(lens),
-                   tau, eps, out)
+                   tau, eps, out, max(lens) if known else 0)
     assert (state[0] == 5.0).all()
     at, errs = 0, []
     for i, n in enumerate(lens):
@@ -130,3 +130,17 @@ def test_stretches_over_sequences(H, dk, dv, lens, start):
     """Stretches that begin and end anywhere: within a sequence, at its ends, several sequences in one, one sequence in many."""
     for n, out, state in run(H, dk, dv, 16, lens, start, 16.0, sum(lens)):
         assert out < OUT and state < STATE, (n, out, state)
+
+
+# 64 heads of 32 x 64: 512 workgroups fill the chip, 8 stretches of 64 heads; 7 heads: 73 stretches, in two groups of up to 64 sequences
+@pytest.mark.parametrize("H,lens,known,kernels", [(64, [2500] + [130] * 5, True, 4), (64, [130] * 5 + [2500], True, 4), (64, [520] * 6, True, 2), (64, [520] * 6, False, 4),
+                                                  (7, [470] * 32 + [4000] + [470] * 32, True, 7), (7, [512] * 65, True, 2)],
+                         ids=["long first", "long last", "alike", "not known", "more than 64", "more than 64 alike"])
+def test_one_long_sequence_among_short_ones(H, lens, known, kernels):
+    """Hardly more stretches than sequences: they are cut where one is much longer than an even share."""
+    from tinyllmforge_amd import _lib
+    count = _lib.load().tlf_kernel_launches
+    before = count()
+    for n, out, state in run(H, 32, 64, 16, lens, [i % 3 for i in range(len(lens))], 16.0, H, known=known):
+        assert out < OUT and state < STATE, (n, out, state)
+    assert count() - before == kernels

@@ -88,6 +88,8 @@ SIGNATURES = {
     "tlf_gla_portions_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32, _I32, _I32]),
     "tlf_gla_portions": (c_int32, [_P, _I64, _P, _P, _P, _P, _P, _I32, _P, _P, _P, _P, _I32, _I32, _I32, _P, _I64, _I32,
                                    _I32, _I32, _I32, _I32, _F, _F, _F, _I32, _P, _SZ, _P]),
+    "tlf_gla_portions_upto": (c_int32, [_P, _I64, _P, _P, _P, _P, _P, _I32, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _P, _I64, _I32,
+                                        _I32, _I32, _I32, _I32, _F, _F, _F, _I32, _P, _SZ, _P]),
     "tlf_residual_rmsnorm": (c_int32, [_P, _I64, _P, _I32, _P, _P, _I64, _P, _I32, _F, _P, _P, _F, _P, _I32, _I32,
                                        _F, _I32, _P]),
     "tlf_latent_prep": (c_int32, [_P, _I64, _P, _I32, _P, _I32, _P, _P, _P, _I32, _I32, _P, _I64, _P, _P, _I32, _I32, _P, _P, _I32,

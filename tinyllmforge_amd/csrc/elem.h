@@ -149,7 +149,7 @@ __device__ __forceinline__ int wave_sums_up_to(int v) {
 }
 
 // The pieces (chunks or blocks) of up to 64 sequences in a row, cut into `units` equal stretches: lane s has sequence s of `own` pieces,
-// first .. end - 1 of all.  Products stay below 2^31: the callers have up to 2^20 pieces and 512 stretches.
+// first .. end - 1 of all.  Products stay within 2^31: the callers have up to 2^22 pieces and 512 stretches.
 __device__ __forceinline__ void stretch_ranges(int own, int &first, int &end, int &all) {
   end = wave_sums_up_to(own);
   first = end - own;

@@ -33,6 +33,7 @@ struct GlaArgs {
   int32_t segs;                           // segments per sequence
   float *seg_state, *seg_dec;             // [seqs, segs, H, dk, dv], [seqs, segs, H, DKP]; of stretches (gla_blocks.hip): [2, units, H, ..], [units, H, ..]
   int32_t units;                          // stretches of all sequences' blocks, 0: whole sequences
+  int32_t seq0;                           // sequences of the call before the first of these
 };
 
 // log2 of sigmoid(z)^(1/tau) = -(max(-z, 0) log2 e + log2(1 + e)) / tau with e = 2^(-|z| log2 e).  log2(1 + e) keeps its
@@ -49,6 +50,6 @@ __device__ __forceinline__ float log2_alpha(float z, float inv_tau) {
 bool gla_blocks_take(const GlaArgs &a, int32_t dtype, int chunk_segs);     // chunk_segs: segments the chunks would have
 bool gla_blocks_sizes(int32_t key_dim, int32_t value_dim);
 size_t gla_blocks_workspace_bytes(int32_t chunks, int32_t num_seqs, int32_t heads, int32_t key_dim, int32_t value_dim);
-int launch_gla_blocks(GlaArgs &a, int first_seq, void *workspace, hipStream_t stream);
+int launch_gla_blocks(GlaArgs &a, int first_seq, int longest, void *workspace, hipStream_t stream);
 
 }  // namespace tlf

@@ -641,13 +641,13 @@ extern "C" size_t tlf_gla_portions_workspace_bytes(int32_t rows, int32_t chunks,
   return chunked > blocks ? chunked : blocks;        // dtype and alignments decide between them
 }
 
-extern "C" int tlf_gla_portions(const void *proj, int64_t proj_stride, const void *a2, const void *a2_bias,
-                                const void *norm_weight, float *state, const int32_t *state_slots, int32_t num_slots,
-                                const int32_t *seq_starts, const int32_t *chunk_rows, const int32_t *chunk_lens,
-                                const int32_t *cu_chunks, int32_t chunks, int32_t first_seq, int32_t num_seqs,
-                                void *out, int64_t out_stride, int32_t rows, int32_t heads, int32_t key_dim,
-                                int32_t value_dim, int32_t rank, float tau, float q_scale, float eps, int32_t dtype,
-                                void *workspace, size_t workspace_bytes, void *stream) {
+extern "C" int tlf_gla_portions_upto(const void *proj, int64_t proj_stride, const void *a2, const void *a2_bias,
+                                     const void *norm_weight, float *state, const int32_t *state_slots, int32_t num_slots,
+                                     const int32_t *seq_starts, const int32_t *chunk_rows, const int32_t *chunk_lens,
+                                     const int32_t *cu_chunks, int32_t chunks, int32_t first_seq, int32_t num_seqs, int32_t max_tokens,
+                                     void *out, int64_t out_stride, int32_t rows, int32_t heads, int32_t key_dim,
+                                     int32_t value_dim, int32_t rank, float tau, float q_scale, float eps, int32_t dtype,
+                                     void *workspace, size_t workspace_bytes, void *stream) {
   using namespace tlf;
   GlaArgs a{};
   a.proj = proj; a.ld = proj_stride; a.a2 = a2; a.a2_bias = a2_bias; a.norm_w = norm_weight; a.state = state;
@@ -662,7 +662,7 @@ extern "C" int tlf_gla_portions(const void *proj, int64_t proj_stride, const voi
   if (!workspace || !aligned16(workspace) ||
       workspace_bytes < tlf_gla_portions_workspace_bytes(rows, chunks, num_seqs, heads, key_dim, value_dim))
     return TLF_E_WORKSPACE;
-  if (gla_blocks_take(a, dtype, gla_segments(chunks, num_seqs, heads, value_dim))) return launch_gla_blocks(a, first_seq, workspace, static_cast<hipStream_t>(stream));
+  if (gla_blocks_take(a, dtype, gla_segments(chunks, num_seqs, heads, value_dim))) return launch_gla_blocks(a, first_seq, max_tokens, workspace, static_cast<hipStream_t>(stream));
   const size_t ch = static_cast<size_t>(chunks) * heads, dkp = gla_tiles(key_dim) * 16;
   a.rec = static_cast<float *>(workspace);
   a.o = a.rec + ch * gla_rec_size(static_cast<int>(dkp));
@@ -673,4 +673,16 @@ extern "C" int tlf_gla_portions(const void *proj, int64_t proj_stride, const voi
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == TLF_DT_BF16 ? launch_gla_portions<unsigned short>(a, first_seq, s)
                               : launch_gla_portions<float>(a, first_seq, s);
+}
+
+extern "C" int tlf_gla_portions(const void *proj, int64_t proj_stride, const void *a2, const void *a2_bias,
+                                const void *norm_weight, float *state, const int32_t *state_slots, int32_t num_slots,
+                                const int32_t *seq_starts, const int32_t *chunk_rows, const int32_t *chunk_lens,
+                                const int32_t *cu_chunks, int32_t chunks, int32_t first_seq, int32_t num_seqs,
+                                void *out, int64_t out_stride, int32_t rows, int32_t heads, int32_t key_dim,
+                                int32_t value_dim, int32_t rank, float tau, float q_scale, float eps, int32_t dtype,
+                                void *workspace, size_t workspace_bytes, void *stream) {
+  return tlf_gla_portions_upto(proj, proj_stride, a2, a2_bias, norm_weight, state, state_slots, num_slots, seq_starts, chunk_rows, chunk_lens, cu_chunks, chunks,
+                               first_seq, num_seqs, 0, out, out_stride, rows, heads, key_dim, value_dim, rank, tau, q_scale, eps, dtype, workspace,
+                               workspace_bytes, stream);
 }

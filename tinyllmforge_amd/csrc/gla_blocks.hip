@@ -336,7 +336,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int b0 = MODE == 0 ? 0 : max(lo - first_block, 0), b1 = MODE == 0 ? blocks : min(hi_block - first_block, blocks);
   const T *vbase = static_cast<const T *>(a.proj) + 2 * hk + static_cast<int64_t>(h) * a.dv + wave * 32;
   const T *gbase = vbase + static_cast<int64_t>(a.H) * a.dv + hi * 4;
-  const unsigned char *rbase = reinterpret_cast<const unsigned char *>(a.rec) + (static_cast<int64_t>(gla_first_block(cbeg, seq)) * a.H + h) * Rec::kSize;
+  const unsigned char *rbase = reinterpret_cast<const unsigned char *>(a.rec) + (static_cast<int64_t>(gla_first_block(cbeg, a.seq0 + seq)) * a.H + h) * Rec::kSize;
   auto copy = [&](int b, int buf) __attribute__((always_inline)) {
     const unsigned char *rec = rbase + static_cast<int64_t>(b) * a.H * Rec::kSize;
     for (int i = (MODE == 1 ? Rec::kK / 1024 : 0) + wave; i < (MODE == 1 ? Rec::kA : Rec::kSize) / 1024; i += waves)
@@ -566,12 +566,26 @@ int gla_block_segments(int chunks, int seqs, int heads, int dk) {
   return static_cast<int>(s < 1 || seqs * s > 65535 ? 1 : s > 32 ? 32 : s);
 }
 
-// Stretches, 0: whole sequences.  A workgroup for every CU, with a stretch of at least 8 blocks; not where there are hardly more stretches than
-// sequences, which would be cut for little.
+// A launch cuts up to 64 sequences; more go in groups, one after the other.
+constexpr int kGroup = 64;
+inline int gla_groups(int seqs) { return (seqs + kGroup - 1) / kGroup; }
+
+// Stretches of each group, 0: sequences are never cut.  A workgroup for every CU, with a stretch of at least 8 blocks.
 int gla_block_units(int chunks, int seqs, int heads, int dk) {
-  if (seqs > 64 || chunks > (1 << 20) || gla_block_segments(chunks, seqs, heads, dk) == 1) return 0;
-  const int units = std::min((dk == 128 ? 256 : 512) / heads, chunks / 16);
-  return units * 2 >= seqs * 3 && units > 1 ? units : 0;
+  if (chunks > (1 << 22) || gla_block_segments(chunks, seqs, heads, dk) == 1) return 0;
+  const int units = std::min((dk == 128 ? 256 : 512) / heads, chunks / 16 / gla_groups(seqs));
+  return units > 1 ? units : 0;
+}
+
+// Whether that is faster than whole sequences, the longest of `longest` tokens (0: not known).  With half as many stretches again as sequences
+// it always is.  Otherwise a launch of whole ones takes as long as its longest, and the two passes over stretches 1.3 x an even share and some
+// eight blocks' time more.  16 heads of 128 x 256, the layer, us, cut / whole: 12 sequences of 700 tokens 343 / 307, of 450 to 900 289 / 294, of 300
+// to 1500 382 / 444; one of 1500 with 11 of 450 242 / 377, one of 8192 with 11 of 100 330 / 1630; 2 heads, one of 8192 with 99 of 450 300 / 1590.
+bool gla_blocks_cut(int units, int chunks, int seqs, int longest) {
+  const int64_t groups = gla_groups(seqs), most = (static_cast<int64_t>(longest) + kGB - 1) / kGB, all = (static_cast<int64_t>(chunks) + 1) / 2;
+  if (units == 0) return false;
+  if (longest <= 0 || (groups == 1 && units * 2 >= seqs * 3)) return true;
+  return most * 10 * units >= all * 13 + groups * units * 80;
 }
 
 // Whether the scan over 16-token chunks does as well: where its waves, one per 16 value columns, are all on the chip at once, in one segment,
@@ -615,17 +629,24 @@ int launch_gla_blocks_of(GlaArgs &a, int first_seq, hipStream_t stream) {
   TLF_LAUNCH((gla_block_kernel<DK>), dim3(a.chunks, a.H), dim3(DK * 4), 0, stream, a);
   if (!a.units) {
     TLF_LAUNCH((gla_block_scan_kernel<DK, 0>), dim3(a.H, 1, a.seqs), dim3(waves * 64), lds, stream, a, first_seq);
-  } else {
-    const dim3 grid(a.H, 1, a.units);
-    TLF_LAUNCH((gla_block_scan_kernel<DK, 1>), grid, dim3(waves * 64), lds, stream, a, first_seq);
-    TLF_LAUNCH(gla_stretches_kernel, dim3((DK * a.dv + 1023) / 1024, a.H, a.seqs), dim3(256), 0, stream, a, first_seq);
-    TLF_LAUNCH((gla_block_scan_kernel<DK, 2>), grid, dim3(waves * 64), lds, stream, a, first_seq);
+    return launch_status();
+  }
+  const dim3 grid(a.H, 1, a.units);
+  const int seqs = a.seqs, each = (seqs + gla_groups(seqs) - 1) / gla_groups(seqs);
+  const int32_t *cu_chunks = a.cu_chunks;
+  for (a.seq0 = 0; a.seq0 < seqs; a.seq0 += each) {
+    a.seqs = std::min(each, seqs - a.seq0);
+    a.cu_chunks = cu_chunks + a.seq0;
+    TLF_LAUNCH((gla_block_scan_kernel<DK, 1>), grid, dim3(waves * 64), lds, stream, a, first_seq + a.seq0);
+    TLF_LAUNCH(gla_stretches_kernel, dim3((DK * a.dv + 1023) / 1024, a.H, a.seqs), dim3(256), 0, stream, a, first_seq + a.seq0);
+    TLF_LAUNCH((gla_block_scan_kernel<DK, 2>), grid, dim3(waves * 64), lds, stream, a, first_seq + a.seq0);
   }
   return launch_status();
 }
 
-int launch_gla_blocks(GlaArgs &a, int first_seq, void *workspace, hipStream_t stream) {
+int launch_gla_blocks(GlaArgs &a, int first_seq, int longest, void *workspace, hipStream_t stream) {
   a.units = aligned16(a.state) ? gla_block_units(a.chunks, a.seqs, a.H, a.dk) : 0;
+  if (!gla_blocks_cut(a.units, a.chunks, a.seqs, longest)) a.units = 0;
   const size_t slots = (static_cast<size_t>(a.chunks) + a.seqs + 1) / 2 + 1;
   a.rec = static_cast<float *>(workspace);
   a.seg_dec = a.rec + slots * a.H * gla_block_record(a.dk) / 4;

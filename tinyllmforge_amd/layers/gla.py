@@ -38,5 +38,5 @@ class GatedLinearAttention(nn.Module):
         if single < n:
             ops.gla_portions(proj[single:], *weights, self.state, ctx.state_slots, ctx.seq_starts, ctx.chunk_rows,
                              ctx.chunk_lens, ctx.cu_chunks, single, ctx.cu_chunks.numel() - 1, self.tau, self.eps,
-                             out[single:])
+                             out[single:], ctx.max_portion)
         return out

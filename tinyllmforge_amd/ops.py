@@ -719,8 +719,8 @@ def gla_decode(proj, a2, a2_bias, norm_weight, state, state_slots, positions, ta
 
 
 def gla_portions(proj, a2, a2_bias, norm_weight, state, state_slots, seq_starts, chunk_rows, chunk_lens, cu_chunks,
-                 first_seq, num_seqs, tau, eps, out):
-    """Portions of sequences ``first_seq ..``; ``proj`` / ``out`` begin at the first portion's row."""
+                 first_seq, num_seqs, tau, eps, out, max_tokens=0):
+    """Portions of sequences ``first_seq ..``, of up to ``max_tokens`` tokens (0: not known); ``proj`` / ``out`` begin at the first portion's row."""
     lib = _lib.load()
     _need(proj, a2.dtype, "proj"); _need(state, torch.float32, "state"); _need(state_slots, torch.int32, "state_slots")
     slots, heads, dk, dv = state.shape
@@ -729,12 +729,12 @@ def gla_portions(proj, a2, a2_bias, norm_weight, state, state_slots, seq_starts,
     assert a2.is_contiguous() and a2.shape[0] == heads * dk and cu_chunks.numel() == num_seqs + 1
     assert state_slots.numel() >= first_seq + num_seqs and chunk_lens.numel() == chunks
     ws = _workspace(lib.tlf_gla_portions_workspace_bytes(rows, chunks, num_seqs, heads, dk, dv), proj.device, "gla")
-    check(lib.tlf_gla_portions(
+    check(lib.tlf_gla_portions_upto(
         proj.data_ptr(), proj.stride(0), a2.data_ptr(), a2_bias.data_ptr(), norm_weight.data_ptr(), state.data_ptr(),
         state_slots.data_ptr(), slots, seq_starts.data_ptr(), chunk_rows.data_ptr(), chunk_lens.data_ptr(),
-        cu_chunks.data_ptr(), chunks, first_seq, num_seqs, out.data_ptr(), out.stride(0), rows, heads, dk, dv,
+        cu_chunks.data_ptr(), chunks, first_seq, num_seqs, max_tokens, out.data_ptr(), out.stride(0), rows, heads, dk, dv,
         a2.shape[1], float(tau), dk ** -0.5, float(eps), _dt(proj), ws.data_ptr(), ws.numel(), _stream()),
-        "tlf_gla_portions")
+        "tlf_gla_portions_upto")
     return out
 
 
