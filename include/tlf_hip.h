@@ -799,7 +799,10 @@ int tlf_rows_rmsnorm(const void *x, int64_t x_stride, const void *w, void *out, 
  * tlf_talk_attn_prefill: portions of sequences first_seq .., rows as in the step; bf16, heads <= 32, dim, vdim <= 128 and a limit
  *   on kv_heads * vdim (tlf_talk_attn_prefill_supported).  stats: scratch, [rows of the step, heads].
  * tlf_talk_attn_prefill_cut: the same; with few portions the keys of long row tiles are cut into parts that run at once.  The workspace is
- *   sized for max_keys = bt_stride * block_size; 0 bytes: nothing will be cut, it may be NULL. */
+ *   sized for max_keys = bt_stride * block_size; 0 bytes: nothing will be cut, it may be NULL.
+ * tlf_talk_attn_prefill_cuts: whether that is the faster one for portions of `rows` rows in all.  tlf_talk_attn_prefill_tile_rows: rows of a
+ *   row tile, 0 for sizes that are not supported.  Every portion takes workgroups for the row tiles of the longest: portions of very
+ *   different lengths are better left to calls of their own. */
 int tlf_talk_prep(const void *proj, int64_t proj_stride, const float *partials, int32_t splits, const float *scale, const void
                   *q_norm, const void *k_norm, const void *temp, const int64_t *positions, const float *cos_sin, int32_t
                   max_pos, int32_t rot_dims, const int32_t *slot_mapping, void *q_out, void *k_cache, void *v_cache,
@@ -818,6 +821,9 @@ int tlf_talk_attn_prefill(const void *q, const void *k_cache, const void *v_cach
                           num_seqs, int32_t max_tokens, const void *talk, float *stats, void *out, int64_t out_stride, int32_t heads,
                           int32_t kv_heads, int32_t dim, int32_t vdim, int32_t block_size, int64_t num_pages, void
                           *stream);
+int tlf_talk_attn_prefill_tile_rows(int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim);
+int tlf_talk_attn_prefill_cuts(int32_t num_seqs, int32_t max_tokens, int32_t rows, int64_t max_keys, int32_t heads, int32_t kv_heads,
+                               int32_t dim, int32_t vdim);
 size_t tlf_talk_attn_prefill_workspace_bytes(int32_t num_seqs, int32_t max_tokens, int64_t max_keys, int32_t heads,
                                              int32_t kv_heads, int32_t dim, int32_t vdim);
 int tlf_talk_attn_prefill_cut(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables, int64_t

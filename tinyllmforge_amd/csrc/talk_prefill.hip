@@ -164,12 +164,12 @@ __device__ __forceinline__ int talk_tile_row(int t) { return (t & 32) | ((t & 4)
 
 // Bound by its exponentials and the vector ALU.  128 registers: with more, the compiler keeps the scores in accumulator registers and moves
 // each out and in (both kernels on 16 heads, eight prompts of up to 2048 tokens: 371 -> 344 us).
-template <int DC, int CT>
+template <int DC, int CT, bool PLAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void talk_stats_kernel(const TalkPrefillArgs p) {
   constexpr int DP = DC * 32, KCH = DC * 4;
   __shared__ __attribute__((aligned(16))) unsigned short Ks[2][kTS][DP + 8];
   int sq, plane, xt, block = prompt_block(blockIdx.x, blockIdx.y);
-  if (p.split.plan) {                                                // eight workgroups in front: the XCDs keep their tiles
+  if constexpr (PLAN) {                                              // eight workgroups in front: the XCDs keep their tiles
     if (block == 0) talk_plan(p, reinterpret_cast<int32_t *>(Ks));
     block -= 8;
     if (block < 0) return;
@@ -322,7 +322,7 @@ __device__ __forceinline__ void talk_st(unsigned int at, const T &v) {
 // WV: quads of heads, RT: tiles of 16 rows; DC: key dimensions in units of 32, VC: of values, rounded up to 2 or 4; GS: heads of a
 // quad that share a KV head (1, 2 or 4).  A wave has RW row tiles of HW heads of KV KV heads, HK each: item e = (KV head, row tile, head).
 template <int WV, int RT, int DC, int VC, int GS>
-__device__ __forceinline__ void talk_prefill_tile(const TalkPrefillArgs &p, const TalkItem item, const int wave, unsigned short *lds) {
+__device__ __forceinline__ void talk_prefill_tile(const TalkPrefillArgs &p, const TalkItem item, const int wave, const int lane, unsigned short *lds) {
   constexpr int HP = talk_heads_held(WV), HT = (HP + 15) / 16, KH = (HP + 31) / 32, ROW = talk_row_size(WV), TQ = RT * 16, NW = WV * RT;
   constexpr int VP = VC * 32, PIECES = VP / 8, RW = RT < 4 / GS ? RT : 4 / GS, HW = 4 / RW, KV = HW > GS ? HW / GS : 1, HK = HW / KV;
   constexpr int PER = 4 / KV;                                        // items of a KV head
@@ -336,8 +336,6 @@ __device__ __forceinline__ void talk_prefill_tile(const TalkPrefillArgs &p, cons
   if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
   const int32_t *bt = c.bt + seq * c.bt_stride;
   const int G = c.G;
-  int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
-  asm volatile("" : "+v"(lane));                                     // what follows from it is made anew for each item, not kept in registers
   const int tid = wave * 64 + lane, n = lane & 15, g = lane >> 4;
   const int h0 = wave % (WV * 4 / HW) * HW, rt = wave / (WV * 4 / HW) * RW * 16;
   const int last_row = min(row0 + TQ, lq) - 1, i_last = start + last_row;
@@ -588,10 +586,20 @@ __device__ __forceinline__ void talk_prefill_tile(const TalkPrefillArgs &p, cons
   }
 }
 
-// Without a plan a workgroup has the tile of its place.  With one, a workgroup per compute unit takes items until there are none: the hardware
-// deals workgroups to XCDs and shader engines by their number, whatever runs there.
+// Whole tiles: a workgroup has the tile of its place.  Its own kernel: the loop below costs registers, and with 32 heads 14 % of the time (eight
+// prompts of 1061 to 2048 tokens 643 us, 734 in that loop; nine of 2048 with 16 heads 599, 621).
 template <int WV, int RT, int DC, int VC, int GS>
-__global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPrefillArgs a) {
+__global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPrefillArgs p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned short lds[];
+  int sq, plane, xt;
+  if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
+  talk_prefill_tile<WV, RT, DC, VC, GS>(p, TalkItem{sq, xt, 0, -1}, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, lds);
+}
+
+// With a plan, a workgroup per compute unit takes items until there are none: the hardware deals workgroups to XCDs and shader engines by their
+// number, whatever runs there.
+template <int WV, int RT, int DC, int VC, int GS>
+__global__ __launch_bounds__(WV * RT * 64) void talk_cut_kernel(const TalkPrefillArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned short lds[];
   int *const at = reinterpret_cast<int *>(lds);                      // the item, where the tile's arrays begin
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -602,14 +610,9 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
     const TalkPrefillArgs &p = *(const TalkPrefillArgs *)args;
     if (wave == 0 && __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)) == 0) {
       int4 item = make_int4(0, 0, 0, -1);
-      int plane;
-      if (p.split.plan) {
-        const int i = more ? gridDim.x + atomicAdd(p.split.plan + 3, 1) : blockIdx.x;
-        at[4] = i < p.split.plan[1];
-        if (i < p.split.plan[1]) item = p.split.items[i];
-      } else {
-        at[4] = !more && prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), item.x, plane, item.y);
-      }
+      const int i = more ? gridDim.x + atomicAdd(p.split.plan + 3, 1) : blockIdx.x;
+      at[4] = i < p.split.plan[1];
+      if (i < p.split.plan[1]) item = p.split.items[i];
       *reinterpret_cast<int4 *>(at) = item;
     }
     lds_barrier();
@@ -617,8 +620,9 @@ __global__ __launch_bounds__(WV * RT * 64) void talk_prefill_kernel(const TalkPr
     if (!same(4)) return;
     const TalkItem item{same(0), same(1), same(2), same(3)};
     lds_barrier();
-    talk_prefill_tile<WV, RT, DC, VC, GS>(p, item, wave, lds);
-    if (!a.split.plan) return;
+    int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+    asm volatile("" : "+v"(lane));                                   // what follows from it is made anew for each item, not kept in registers
+    talk_prefill_tile<WV, RT, DC, VC, GS>(p, item, wave, lane, lds);
   }
 }
 
@@ -686,20 +690,29 @@ int launch_talk_stats(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStrea
   a.bq = kUnits / a.hpp;
   const int blocks = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, a.c.G * a.passes, num_seqs);
   if (!blocks) return TLF_E_SHAPE;
-  TLF_LAUNCH((talk_stats_kernel<DC, CT>), prompt_grid<dim3>(blocks + (a.split.plan ? 8 : 0)), dim3(256), 0, s, a);
+  if (a.split.plan) TLF_LAUNCH((talk_stats_kernel<DC, CT, true>), prompt_grid<dim3>(blocks + 8), dim3(256), 0, s, a);
+  else TLF_LAUNCH((talk_stats_kernel<DC, CT, false>), prompt_grid<dim3>(blocks), dim3(256), 0, s, a);
   return launch_status();
 }
 
 template <int WV, int RT, int DC, int VC, int GS>
 int launch_talk_prefill(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStream_t s) {
-  static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&talk_prefill_kernel<WV, RT, DC, VC, GS>),
-                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kTalkLds);
+  static const hipError_t allowed = [] {
+    hipError_t e = hipSuccess;
+    for (const void *k : {reinterpret_cast<const void *>(&talk_prefill_kernel<WV, RT, DC, VC, GS>), reinterpret_cast<const void *>(&talk_cut_kernel<WV, RT, DC, VC, GS>)})
+      if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kTalkLds);
+    return e;
+  }();
   if (allowed != hipSuccess) return static_cast<int>(allowed);
   const int blocks = prompt_tiles_make(a.tiles, (max_tokens + RT * 16 - 1) / (RT * 16), 1, num_seqs);
   if (!blocks) return TLF_E_SHAPE;
-  TLF_LAUNCH((talk_prefill_kernel<WV, RT, DC, VC, GS>), a.split.plan ? dim3(kTalkUnits) : prompt_grid<dim3>(blocks),
-             dim3(WV * RT * 64), talk_prefill_lds(WV, RT, a.c.G, a.c.Vp), s, a);
-  if (a.split.plan) TLF_LAUNCH((talk_join_kernel<WV, RT, VC, GS>), dim3((max_tokens + RT * 16 - 1) / (RT * 16) * num_seqs, WV * RT), dim3(256), 0, s, a);
+  const size_t lds = talk_prefill_lds(WV, RT, a.c.G, a.c.Vp);
+  if (!a.split.plan) {
+    TLF_LAUNCH((talk_prefill_kernel<WV, RT, DC, VC, GS>), prompt_grid<dim3>(blocks), dim3(WV * RT * 64), lds, s, a);
+    return launch_status();
+  }
+  TLF_LAUNCH((talk_cut_kernel<WV, RT, DC, VC, GS>), dim3(kTalkUnits), dim3(WV * RT * 64), lds, s, a);
+  TLF_LAUNCH((talk_join_kernel<WV, RT, VC, GS>), dim3((max_tokens + RT * 16 - 1) / (RT * 16) * num_seqs, WV * RT), dim3(256), 0, s, a);
   return launch_status();
 }
 template <int WV, int RT>
@@ -792,6 +805,17 @@ extern "C" size_t tlf_talk_attn_prefill_workspace_bytes(int32_t num_seqs, int32_
   if (num_seqs <= 0 || max_tokens <= 0 || max_keys <= 0 || !tlf_talk_attn_prefill_supported(heads, kv_heads, dim, vdim)) return 0;
   const int Vp = (vdim + 31) / 32 * 32;
   return static_cast<size_t>(talk_room(num_seqs, max_tokens, max_keys, talk_quads(heads), talk_row_tiles(talk_quads(heads), kv_heads, Vp) * 16, Vp).bytes);
+}
+
+extern "C" int tlf_talk_attn_prefill_tile_rows(int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim) {
+  using namespace tlf;
+  return tlf_talk_attn_prefill_supported(heads, kv_heads, dim, vdim) ? talk_row_tiles(talk_quads(heads), kv_heads, (vdim + 31) / 32 * 32) * 16 : 0;
+}
+
+extern "C" int tlf_talk_attn_prefill_cuts(int32_t num_seqs, int32_t max_tokens, int32_t rows, int64_t max_keys, int32_t heads, int32_t kv_heads,
+                                          int32_t dim, int32_t vdim) {
+  const int tq = tlf_talk_attn_prefill_tile_rows(heads, kv_heads, dim, vdim);
+  return num_seqs > 0 && max_tokens > 0 && tq && tlf::talk_cuts_pay(num_seqs, max_tokens, rows, max_keys, tq);
 }
 
 extern "C" int tlf_talk_attn_prefill_cut(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables,

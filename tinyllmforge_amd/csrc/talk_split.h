@@ -22,6 +22,20 @@ __host__ __device__ inline bool talk_cuts(int64_t portions, int64_t tokens, int6
   return keys > kTalkLeast * 32 && (tiles <= 192 || (tiles <= kTalkTiles && tokens >= 512));
 }
 
+// Whether that pays, with `rows` rows in all portions: not
+// - where no tile is longer than what the parts take, 1.2 even shares and six steps (16 heads, the layer, cut / whole, us: 24 portions of 250 tokens
+//   93 / 89, 48 of 128 79 / 72, the same behind 1024 keys 272 / 251, but 12 of 400 99 / 106);
+// - with row tiles of 16 rows (more than 16 heads) where nearly all places of the plan are taken and portions are long: a step of the kernel that
+//   goes through the list takes 14 % longer there (one of 8000 1530 / 1421, four of 2048 483 / 449, three of 2600 565 / 535, but six of 1300
+//   349 / 392, four of 1024 to 2048 347 / 375).
+inline bool talk_cuts_pay(int64_t portions, int64_t tokens, int64_t rows, int64_t keys, int tq) {
+  if (!talk_cuts(portions, tokens, keys, tq)) return false;
+  const int64_t bound = (tokens + tq - 1) / tq * portions, tiles = rows / tq + (portions + 1) / 2 < bound ? rows / tq + (portions + 1) / 2 : bound;
+  const int64_t longest = (keys + 31) / 32, before = keys > tokens ? (keys - tokens) / 32 : 0;
+  if (tiles <= kTalkUnits && longest * 10 * 2 * kTalkUnits <= tiles * (longest + before) * 12 + 60 * 2 * kTalkUnits) return false;
+  return tq > 16 || tiles <= 448 || tokens < 2048;
+}
+
 __host__ __device__ inline int talk_tiles(int tokens, int tq) { return tokens <= 0 ? 0 : (tokens - 1) / tq + 1; }
 __host__ __device__ inline int talk_steps(int start, int tokens, int tq, int x) {
   const int end = tokens - x * tq < tq ? tokens : (x + 1) * tq;

@@ -1236,8 +1236,13 @@ def talk_prefill_supported(heads, kv_heads, dim, vdim) -> bool:
     return bool(_lib.load().tlf_talk_attn_prefill_supported(heads, kv_heads, dim, vdim))
 
 
-def talk_attention_prefill(q, kv: SinkKV, block_tables, cu_seqlens_q, seq_starts, first_seq, num_seqs, max_tokens, talk, out):
-    """Portions of sequences ``first_seq ..`` on the matrix cores (bf16); rows indexed as in the step."""
+def talk_prefill_cuts(kv: SinkKV, block_tables, num_seqs, max_tokens, rows, heads) -> bool:
+    """Whether the keys of long row tiles are cut into parts, for portions of up to ``max_tokens`` rows and ``rows`` in all."""
+    return bool(_lib.load().tlf_talk_attn_prefill_cuts(num_seqs, max_tokens, rows, block_tables.stride(0) * kv.k.shape[2], heads, kv.k.shape[1], kv.dim, kv.vdim))
+
+
+def talk_attention_prefill(q, kv: SinkKV, block_tables, cu_seqlens_q, seq_starts, first_seq, num_seqs, max_tokens, talk, out, rows=None):
+    """Portions of sequences ``first_seq ..`` on the matrix cores (bf16), of ``rows`` rows in all where that is known; rows indexed as in the step."""
     _need(q, BF16, "q"); _need(talk, BF16, "talk"); _need(block_tables, torch.int32, "block_tables")
     n, heads, dp = q.shape
     pages, G, bs, _ = kv.k.shape
@@ -1246,12 +1251,14 @@ def talk_attention_prefill(q, kv: SinkKV, block_tables, cu_seqlens_q, seq_starts
     assert block_tables.stride(1) == 1 and block_tables.shape[0] >= first_seq + num_seqs
     lib, cols = _lib.load(), block_tables.stride(0)
     stats = torch.empty(n, heads, dtype=torch.float32, device=q.device)
+    args = (q.data_ptr(), kv.k.data_ptr(), kv.v.data_ptr(), block_tables.data_ptr(), cols, cu_seqlens_q.data_ptr(), seq_starts.data_ptr(), first_seq, num_seqs,
+            max_tokens, talk.data_ptr(), stats.data_ptr(), out.data_ptr(), out.stride(0), heads, G, kv.dim, kv.vdim, bs, pages)
+    if not talk_prefill_cuts(kv, block_tables, num_seqs, max_tokens, min(n, num_seqs * max_tokens) if rows is None else rows, heads):
+        check(lib.tlf_talk_attn_prefill(*args, _stream()), "tlf_talk_attn_prefill")
+        return out
     nbytes = lib.tlf_talk_attn_prefill_workspace_bytes(num_seqs, max_tokens, cols * bs, heads, G, kv.dim, kv.vdim)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)          # the partial sums of parts: given back after the call
-    check(lib.tlf_talk_attn_prefill_cut(
-        q.data_ptr(), kv.k.data_ptr(), kv.v.data_ptr(), block_tables.data_ptr(), cols, cu_seqlens_q.data_ptr(),
-        seq_starts.data_ptr(), first_seq, num_seqs, max_tokens, talk.data_ptr(), stats.data_ptr(), out.data_ptr(), out.stride(0), heads, G, kv.dim, kv.vdim,
-        bs, pages, ws.data_ptr(), nbytes, _stream()), "tlf_talk_attn_prefill_cut")
+    check(lib.tlf_talk_attn_prefill_cut(*args, ws.data_ptr(), nbytes, _stream()), "tlf_talk_attn_prefill_cut")
     return out
 
 
