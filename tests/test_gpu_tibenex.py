@@ -236,6 +236,45 @@ def test_talking_heads_with_keys_cut(sizes, portions):
     torch.testing.assert_close(got.float(), whole.float(), rtol=2 ** -7, atol=2 ** -14)
 
 
+def items_of(portions, tq):
+    """Row tiles and extra parts in the list of tlf_talk_attn_prefill_cut (csrc/talk_split.h)."""
+    steps = [(a + min((x + 1) * tq, n) - 1) // 32 + 1 for a, n in portions for x in range(-(-n // tq))]
+    share = max(-(-sum(steps) // 256), 3)
+    count = lambda per: len(steps) + sum((s - 1) // per for s in steps)
+    return next((count(per) for per in range(share, share + 5) if count(per) <= 256), count(share))
+
+
+# a workgroup takes a second item only where there are more than 256: one long portion, unequal ones of 257 to 512 row tiles
+@pytest.mark.parametrize("sizes,portions", [((16, 8, 64, 64), [(0, 5000)]), ((16, 8, 128, 128), [(0, n) for n in (2048, 1100, 1900, 700, 1500, 1300, 1061, 1777)]),
+                                            ((32, 8, 64, 64), [(0, 5000)]), ((32, 8, 128, 128), [(0, n) for n in (1500, 700, 1999, 650)]), ((24, 8, 96, 64), [(300, 2500), (0, 1800)]),
+                                            ((8, 4, 64, 64), [(0, 9000), (5, 4000)]), ((4, 1, 128, 128), [(64, 8500), (0, 3000)])], ids=str)
+def test_lists_of_more_items_than_workgroups(sizes, portions):
+    """Parts of row tiles that workgroups take one after the other, against whole tiles."""
+    from tinyllmforge_amd import _lib
+    (H, G, D, V), g, bs, lib = sizes, torch.Generator(device="cuda").manual_seed(7), 64, _lib.load()
+    tq = lib.tlf_talk_attn_prefill_tile_rows(H, G, D, V)
+    assert tq == (16 if H > 16 else 32 if H > 8 else 64) and 256 < items_of(portions, tq) <= 768
+    need = [-(-(a + n) // bs) for a, n in portions]
+    kv_shape = (sum(need), G, bs)
+    k, v = (torch.randn(*kv_shape, d, device="cuda", generator=g).bfloat16() for d in (D, V))
+    perm, bt = torch.randperm(sum(need), generator=g, device="cuda").to(torch.int32), torch.full((len(need), max(need)), -1, dtype=torch.int32, device="cuda")
+    for s, n in enumerate(need):
+        bt[s, :n] = perm[sum(need[:s]):sum(need[:s + 1])]
+    lens, ptr, stream = [n for _, n in portions], lambda t: t.data_ptr(), torch.cuda.current_stream().cuda_stream
+    rows, cu, starts = sum(lens), i32(*([0] + torch.tensor(lens).cumsum(0).tolist())), i32(*[a for a, _ in portions])
+    q = (1.5 * D ** -0.5 * torch.randn(rows, H, D, device="cuda", generator=g)).bfloat16()
+    talk = (torch.eye(H, device="cuda") + 0.3 * torch.randn(H, H, device="cuda", generator=g)).bfloat16()
+    got, whole = (torch.full((rows, H * V), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    stats, nbytes = torch.empty(rows, H, device="cuda"), lib.tlf_talk_attn_prefill_workspace_bytes(len(need), max(lens), max(need) * bs, H, G, D, V)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    common = lambda out: (ptr(q), ptr(k), ptr(v), ptr(bt), bt.stride(0), ptr(cu), ptr(starts), 0, len(need), max(lens), ptr(talk), ptr(stats), ptr(out), out.stride(0), H, G, D, V,
+                          bs, sum(need))
+    assert nbytes and lib.tlf_talk_attn_prefill_cut(*common(got), ptr(ws), nbytes, stream) == 0 and lib.tlf_talk_attn_prefill(*common(whole), stream) == 0
+    # up to 268 steps of two products, each rounding a partial sum below two in fp32: 2^9 * 2^-24 on either side; then a rounding to bf16 that may
+    # fall to either side, an ulp apart
+    torch.testing.assert_close(got.float(), whole.float(), rtol=2 ** -7, atol=2 ** -14)
+
+
 @pytest.mark.parametrize("portions,tiles", [([9] * 7, False), ([16] * 4, True), ([60, 2, 3], True), ([2] * 33, True)], ids=str)
 def test_short_portions_in_tiles(portions, tiles, monkeypatch):
     """From 64 rows on, short portions run in row tiles; both ways give the rows' attention."""
