@@ -275,9 +275,9 @@ def test_lists_of_more_items_than_workgroups(sizes, portions):
     torch.testing.assert_close(got.float(), whole.float(), rtol=2 ** -7, atol=2 ** -14)
 
 
-@pytest.mark.parametrize("portions,tiles", [([9] * 7, False), ([16] * 4, True), ([60, 2, 3], True), ([2] * 33, True)], ids=str)
-def test_short_portions_in_tiles(portions, tiles, monkeypatch):
-    """From 64 rows on, short portions run in row tiles; both ways give the rows' attention."""
+def layer_in_tiles_and_by_rows(lens, starts, monkeypatch):
+    """What a layer of 8 heads gives for portions of ``lens`` tokens behind ``starts``, as it chooses and row by row, and the calls in row tiles:
+    the first portion of each, their number."""
     from types import SimpleNamespace
     from tinyllmforge_amd import ops as P
     from tinyllmforge_amd.engine.inputs import portion_inputs
@@ -285,7 +285,6 @@ def test_short_portions_in_tiles(portions, tiles, monkeypatch):
     from tinyllmforge_amd.layers.talking_attention import TalkingHeadsAttention
     from tinyllmforge_amd.utils.context import reset_context, set_portions_context
     H, G, D, BF, g = 8, 4, 64, torch.bfloat16, torch.Generator(device="cuda").manual_seed(1)
-    lens, starts = [1, 1] + portions + [130], [5, 64] + [70 * (i % 2) for i in range(len(portions))] + [64]
     need, at, seqs = [-(-(a + n) // 64) for a, n in zip(starts, lens)], 0, []
     for i, (a, n) in enumerate(zip(starts, lens)):
         seqs.append(SimpleNamespace(num_scheduled=n, num_computed=a, token_ids=range(a + n), block_table=list(range(at, at + need[i])), state_slot=i))
@@ -293,30 +292,48 @@ def test_short_portions_in_tiles(portions, tiles, monkeypatch):
     d = {k: torch.from_numpy(v).cuda() if hasattr(v, "dtype") else v for k, v in portion_inputs(seqs, 64, 128).items()}
     positions = d.pop("positions")
     d.pop("input_ids")
+    most = max(a + n for a, n in zip(starts, lens))
     with torch.device("cuda"):
         layer = TalkingHeadsAttention(H, G, D, D, D ** -0.5, 1e-6, BF, D).to(BF)
-    layer.cos_sin = rotation_table(D, 512, 1e6).cuda()
+    layer.cos_sin = rotation_table(D, max(512, most), 1e6).cuda()
     layer.talk.data = (torch.eye(H, device="cuda") + 0.3 * torch.randn(H, H, device="cuda", generator=g)).to(BF)
     layer.bind_pages(at, 64, "cuda")
     proj, k, v = (torch.randn(*s, device="cuda", generator=g).to(BF) for s in ((sum(lens), (H + 2 * G) * D), layer.kv.k.shape, layer.kv.v.shape))
-    firsts, prefill = [], P.talk_attention_prefill
+    calls, prefill = [], P.talk_attention_prefill
 
     def call(by_rows):
         layer.kv.k.copy_(k)
         layer.kv.v.copy_(v)
-        set_portions_context(**d, max_len=512)
+        set_portions_context(**d, max_len=max(512, most))
         with torch.inference_mode(), monkeypatch.context() as m:
-            m.setattr(P, "talk_attention_prefill", lambda *a: (firsts.append(a[5]), prefill(*a))[1])
+            m.setattr(P, "talk_attention_prefill", lambda *a: (calls.append((a[5], a[6])), prefill(*a))[1])
             if by_rows:
                 m.setattr(P, "talk_prefill_supported", lambda *a: False)
             out = layer(proj, positions)
         reset_context()
         return out.float()
 
-    got, want = call(False), call(True)
-    assert firsts == [2 if tiles else 2 + len(portions)]
+    return call(False), call(True), calls
+
+
+@pytest.mark.parametrize("portions,tiles", [([9] * 7, False), ([16] * 4, True), ([60, 2, 3], True), ([2] * 33, True)], ids=str)
+def test_short_portions_in_tiles(portions, tiles, monkeypatch):
+    """From 64 rows on, short portions run in row tiles; both ways give the rows' attention."""
+    lens, starts = [1, 1] + portions + [130], [5, 64] + [70 * (i % 2) for i in range(len(portions))] + [64]
+    got, want, calls = layer_in_tiles_and_by_rows(lens, starts, monkeypatch)
+    assert [first for first, _ in calls] == [2 if tiles else 2 + len(portions)]
     # by rows the weights enter as bf16 pairs of 16 bits too, in another order: a bf16 ulp of the result, and 2^-14 of terms of a few units
     torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -10)
+
+
+@pytest.mark.parametrize("short,long,held,calls", [([20] * 13, [2500], 70, [(1, 13), (14, 1)]), ([20] * 13, [300, 131], 70, [(1, 15)]), ([40] * 30, [500], 1000, [(1, 30), (31, 1)]), ([40] * 20, [700], 1000, [(1, 21)]),
+                                                   ([20] * 7, [2500], 70, [(1, 8)]), ([2] * 3, [2500, 600], 70, [(4, 2)])], ids=str)
+def test_long_portions_among_short_ones(short, long, held, calls, monkeypatch):
+    """Short portions share a call with the long ones only where these do not give them many row tiles that are empty."""
+    lens, starts = [1] + short + long, [64] + [held] * len(short) + [0] * len(long)
+    got, want, made = layer_in_tiles_and_by_rows(lens, starts, monkeypatch)
+    assert made == calls
+    torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -10)      # as above
 
 
 def test_supported_sizes_run_in_tiles():

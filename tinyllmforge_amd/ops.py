@@ -1236,6 +1236,11 @@ def talk_prefill_supported(heads, kv_heads, dim, vdim) -> bool:
     return bool(_lib.load().tlf_talk_attn_prefill_supported(heads, kv_heads, dim, vdim))
 
 
+def talk_tile_rows(heads, kv_heads, dim, vdim) -> int:
+    """Rows of a row tile of ``talk_attention_prefill``."""
+    return _lib.load().tlf_talk_attn_prefill_tile_rows(heads, kv_heads, dim, vdim)
+
+
 def talk_prefill_cuts(kv: SinkKV, block_tables, num_seqs, max_tokens, rows, heads) -> bool:
     """Whether the keys of long row tiles are cut into parts, for portions of up to ``max_tokens`` rows and ``rows`` in all."""
     return bool(_lib.load().tlf_talk_attn_prefill_cuts(num_seqs, max_tokens, rows, block_tables.stride(0) * kv.k.shape[2], heads, kv.k.shape[1], kv.dim, kv.vdim))
