@@ -327,7 +327,8 @@ def test_short_portions_in_tiles(portions, tiles, monkeypatch):
 
 
 @pytest.mark.parametrize("short,long,held,calls", [([20] * 13, [2500], 70, [(1, 13), (14, 1)]), ([20] * 13, [300, 131], 70, [(1, 15)]), ([40] * 30, [500], 1000, [(1, 30), (31, 1)]), ([40] * 20, [700], 1000, [(1, 21)]),
-                                                   ([20] * 7, [2500], 70, [(1, 8)]), ([2] * 3, [2500, 600], 70, [(4, 2)])], ids=str)
+                                                   ([20] * 7, [2500], 70, [(1, 8)]), ([2] * 3, [2500, 600], 70, [(4, 2)]),
+                                                   ([2] * 33, [200], 1000, [(34, 1)]), ([2] * 33, [], 400, []), ([3] * 33, [], 400, [(1, 33)])], ids=str)
 def test_long_portions_among_short_ones(short, long, held, calls, monkeypatch):
     """Short portions share a call with the long ones only where these do not give them many row tiles that are empty."""
     lens, starts = [1] + short + long, [64] + [held] * len(short) + [0] * len(long)

@@ -400,3 +400,11 @@ def test_few_state_space_groups_keep_a_head_per_workgroup(sizes, seqs, tokens, s
     parts = seqs * segments * H if segments > 1 else 0
     want = up(2 * rows * (H * P + 2 * G * N)) + 2 * up(4 * rows * H) + up(4 * parts) + up(4 * parts * N * P)
     assert _lib.load().tlf_ssd_portions_workspace_bytes(rows, seqs, tokens, *sizes, 0) == want
+
+
+def test_short_portions_of_few_rows_go_row_by_row():
+    from tinyllmforge_amd.layers.talking_attention import short_in_tiles
+    for portions, rows, keys in ((1, 64, 4160), (8, 64, 2112), (12, 72, 2112), (100, 200, 1088), (60, 900, 1088), (33, 66, 192), (4, 64, 192)):
+        assert short_in_tiles(portions, rows, keys)
+    for portions, rows, keys in ((0, 0, 64), (7, 63, 192), (33, 66, 512), (33, 66, 4160), (16, 64, 1088), (22, 66, 2112)):
+        assert not short_in_tiles(portions, rows, keys)

@@ -9,6 +9,15 @@ from .. import ops
 from ..utils.context import get_context
 
 
+def short_in_tiles(portions: int, rows: int, keys: int) -> bool:
+    """Whether short portions, ``rows`` rows in all and contexts of up to ``keys``, go in row tiles: where they are few rows, row by row is faster.
+    A row tile starts with more latency, and its keys are read once for all its rows: a row costs what it reads, a tile about as much as one row and
+    all of them together as much as 40.  16 heads, the layer by rows and in tiles, us: portions behind 1024 keys, 8 of up to 8 tokens 57 and 67, 33 of 2
+    74 and 94, 16 of 4 63 and 75, one of 64 63 and 62, 8 of up to 16 93 and 67, 60 of up to 32 818 and 135; behind 2048, 33 of 2 121 and 149, 12 of 6
+    111 and 101, 100 of 2 326 and 310; behind 64, where either waits for the host, 33 of 2 41 and 37."""
+    return rows >= 64 and (keys <= 256 or rows >= 55 + 1.1 * portions)
+
+
 class TalkingHeadsAttention(nn.Module):
     def __init__(self, num_heads: int, num_kv_heads: int, dim: int, value_dim: int, scale: float, eps: float, dtype: torch.dtype,
                  rot_dims: int = 0, rope=None):
@@ -37,10 +46,7 @@ class TalkingHeadsAttention(nn.Module):
                           self.temp.data, self.cos_sin, self.rot_dims, self.eps, self.scale)
         out = torch.empty(n, self.num_heads * self.value_dim, dtype=self.dtype, device=q.device)
         tiles = self.dtype == torch.bfloat16 and ops.talk_prefill_supported(self.num_heads, self.num_kv_heads, self.dim, self.value_dim)
-        # Short portions go row by row only where they are few rows: a row tile starts with more latency, and its keys are read once for
-        # all its rows.  16 heads, portions behind 1024 keys, the layer by rows and in tiles: 8 of up to 8 tokens 57 and 67 us, one of 64 63 and
-        # 62, 8 of up to 16 93 and 67, 60 of up to 32 818 and 135.
-        short = ctx.num_short if ctx.num_short_rows - ctx.num_single < 64 else 0
+        short = 0 if short_in_tiles(ctx.num_short, ctx.num_short_rows - ctx.num_single, ctx.block_tables.stride(0) * kv.k.shape[2]) else ctx.num_short
         rows = (ctx.num_short_rows if short else ctx.num_single) if tiles else n
         if rows:
             ops.talk_attention_rows(q[:rows], kv, ctx.block_tables, positions[:rows], ctx.slot_mapping[:rows], self.talk.data, ctx.max_len,
