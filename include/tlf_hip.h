@@ -735,6 +735,8 @@ int tlf_residual_layernorm(const void *y, int64_t y_stride, const float *partial
  *   (without bias) of a sequence's last positions, p in row p mod taps: rows of one-token sequences (row_seq NULL, or
  *   cu_seqlens_q of row_seq[row]) are written here, those of portions by tlf_conv_tail afterwards.  gate_out [n, heads * vdim]
  *   (NULL: not copied) gets the gate's columns; with splits > 1 it must be there and row_seq NULL.
+ * tlf_sink_prep_step: the same where the caller knows that the first `singles` rows are one-token sequences and how many sequences there are in all
+ *   (num_seqs, 0: it does not): many rows of prompts are then worked on in runs.
  * tlf_conv_tail: last taps - 1 projected rows of sequences first_seq .. (proj: the step's rows) into the ring.
  * tlf_sink_attn_rows: row r of q [rows, heads, Dp] attends to positions 0 .. positions[r] of sequence row_seq[r] (NULL: r);
  *   slot_mapping[r] < 0: a padding row (zeros).  max_len bounds the positions.  bf16 up to 256 dimensions on the matrix cores.
@@ -747,6 +749,14 @@ int tlf_sink_prep(const void *proj, int64_t proj_stride, const float *partials, 
                   *gate_out, int32_t n, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, int32_t
                   block_size, int64_t num_pages, float eps, float score_scale, float cap, int32_t dtype, void
                   *stream);
+int tlf_sink_prep_step(const void *proj, int64_t proj_stride, const float *partials, int32_t splits, const float *scale,
+                       const void *bias, const void *conv, int32_t taps, void *ring, const int32_t *state_slots, int64_t
+                       num_state_slots, const int32_t *row_seq, const int32_t *cu_seqlens_q, int32_t singles, int32_t num_seqs,
+                       const void *q_norm, const void *k_norm, const int64_t *positions, const float *cos_sin, const float *q_mult,
+                       int32_t max_pos, int32_t rot_dims, const int32_t *slot_mapping, void *q_out, void *k_cache, void *v_cache, void
+                       *gate_out, int32_t n, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, int32_t
+                       block_size, int64_t num_pages, float eps, float score_scale, float cap, int32_t dtype, void
+                       *stream);
 int tlf_conv_tail(const void *proj, int64_t proj_stride, void *ring, const int32_t *state_slots, int64_t
                   num_state_slots, const int32_t *cu_seqlens_q, const int32_t *seq_starts, int32_t first_seq, int32_t
                   num_seqs, int32_t taps, int32_t channels, int32_t dtype, void *stream);

@@ -369,6 +369,45 @@ def test_preparation_of_many_rows(sizes, rot, taps):
         assert torch.equal(got, want)
 
 
+# single tokens and portions; workgroups of a row; rows of a run; launches: single tokens that are many go in one of their own
+@pytest.mark.parametrize("singles,portions,sizes,run,launches", [
+    (0, [1500, 23, 24, 25, 47, 5, 2], (32, 8, 128, 128), 8, 1), (3, [3000, 1, 2, 3, 700, 487], (32, 8, 128, 128), 16, 1), (0, [5000, 2, 3, 23, 24, 25, 2500, 47, 601], (32, 8, 128, 128), 24, 1),
+    (50, [3000, 7, 8, 9, 500, 1], (32, 8, 128, 128), 8, 2), (7, [4000, 17, 15, 16, 300], (32, 8, 96, 72), 16, 2), (41, [4000, 23, 25, 24, 8000, 331], (16, 4, 64, 64), 24, 2)], ids=str)
+@pytest.mark.parametrize("taps", [2, 4])
+def test_preparation_in_runs_of_every_length(singles, portions, sizes, run, launches, taps):
+    """Runs that begin and end anywhere, single tokens apart or in front, the last run not whole: bit for bit what the kernel for few rows gives."""
+    from tinyllmforge_amd import _lib, ops as P
+    (H, G, D, V), g, BF, dev = sizes, torch.Generator(device="cuda").manual_seed(run + taps), torch.bfloat16, "cuda"
+    lens = [1] * singles + portions
+    starts = [(7 * i) % 90 if n < 1000 else 0 for i, n in enumerate(lens)]
+    rows, channels = sum(lens), (H + G) * D + G * V
+    hy = -(-(H + 2 * G) // 16)
+    behind = rows if launches == 1 else rows - singles
+    assert run == (24 if behind * hy >= 24 * 1024 else 16 if behind * hy >= 16 * 768 else 8) and behind % run
+    need, i32 = [-(-(a + n) // 64) for a, n in zip(starts, lens)], lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    randn = lambda *s: torch.randn(*s, generator=g, device=dev).to(BF)
+    proj, bias, conv, ring0 = randn(rows, channels + H * V), randn(channels), randn(taps, channels), randn(len(lens) + 1, taps, channels)
+    qn, kn, table = 1 + 0.1 * randn(D), 1 + 0.1 * randn(D), torch.randn(9000, D, generator=g, device=dev)
+    seq = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens))
+    cu = torch.tensor([0] + lens).cumsum(0)
+    pos = torch.arange(rows) - cu[seq] + torch.tensor(starts)[seq]
+    slots = (torch.tensor([0] + need).cumsum(0)[seq] * 64 + pos).to(torch.int32).to(dev)
+    states = i32([(i + 1) % (len(lens) + 1) for i in range(len(lens))])
+
+    def prepared(singles):
+        kv, ring, count = P.SinkKV(sum(need), 64, G, D, V, BF, dev), ring0.clone(), _lib.load().tlf_kernel_launches
+        before = count()
+        q = P.sink_prep(proj, kv, H, pos.to(dev), slots, 1e-5, 0.3, None, bias, row_seq=seq.to(torch.int32).to(dev), cu_seqlens_q=i32(cu.tolist()), q_norm=qn, k_norm=kn,
+                        cos_sin=table, rot_dims=D, conv=conv, ring=ring, state_slots=states, singles=singles)[0]
+        return (q, kv.k, kv.v, ring), count() - before
+
+    got, made = prepared(singles)
+    want, one = prepared(rows)                                       # all rows said to be sequences of their own: no runs
+    assert (made, one) == (launches, 1)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 # ---------------------------------------------------------------------------------------------- experts
 @pytest.mark.parametrize("corr_dtype", DTYPES)
 @pytest.mark.parametrize("n,E,ident,top,splits", [(1, 5, 2, 2, 1), (64, 70, 7, 6, 3), (500, 16, 1, 1, 2), (1500, 33, 3, 4, 1), (9, 500, 12, 20, 1),

@@ -123,6 +123,9 @@ SIGNATURES = {
     "tlf_sink_prep": (c_int32, [_P, _I64, _P, _I32, _P, _P, _P, _I32, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _I32,
                                 _I32, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _F, _F, _F, _I32,
                                 _P]),
+    "tlf_sink_prep_step": (c_int32, [_P, _I64, _P, _I32, _P, _P, _P, _I32, _P, _P, _I64, _P, _P, _I32, _I32, _P, _P, _P, _P, _P, _I32,
+                                     _I32, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _F, _F, _F, _I32,
+                                     _P]),
     "tlf_conv_tail": (c_int32, [_P, _I64, _P, _P, _I64, _P, _P, _I32, _I32, _I32, _I32, _I32, _P]),
     "tlf_sink_attn_rows_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32, _I32, _I32, _I32]),
     "tlf_sink_attn_rows": (c_int32, [_P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _I64, _P, _I64, _I32, _I32, _I32, _I32,

@@ -10,6 +10,7 @@
 // first tokens and their last rows go there in a second launch.  Positions below 0 are zeros, so a ring is never cleared.
 // HBM bound: a row is read once (from the caches again for the convolution of its neighbours) and written once.
 #include "sink_attn.h"
+#include "sink_runs.h"
 
 namespace tlf {
 
@@ -32,6 +33,7 @@ struct SinkPrepArgs {
   void *q_out, *gate_out;      // [n, H, Dp]; [n, H * Dv] or NULL
   SinkCache c;
   int32_t n, H, taps, channels, heads;
+  int32_t row0;                // sink_prep_rows_kernel: its first row
   float eps, q_scale;
 };
 
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
   __shared__ __attribute__((aligned(16))) PrepRow rows[kRun];
   __shared__ __attribute__((aligned(16))) float turn[kRun][3 * 64];  // cosines, sines negated, sines
   const SinkCache &c = a.c;
-  const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * run;
+  const int64_t tok0 = a.row0 + static_cast<int64_t>(blockIdx.x) * run;
   const int count = static_cast<int>(min(static_cast<int64_t>(run), a.n - tok0)), half = a.rot_dims / 2, tid = threadIdx.x;
   if (tid < count) {
     const int64_t tok = tok0 + tid, pos = a.positions[tok], slot = a.slots[tok];
@@ -512,7 +514,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
 }
 
 template <typename T>
-int launch_sink_prep(const SinkPrepArgs &a, bool vec, bool part, hipStream_t s) {
+int launch_sink_prep(const SinkPrepArgs &a, bool vec, bool part, int singles, int seqs, hipStream_t s) {
   const int most = a.c.Dp > a.c.Vp ? a.c.Dp : a.c.Vp;
   const unsigned hy = (a.heads + 15) / 16;
 #define TLF_PREP(MAXC, TOK, TAPS, PART, VEC)                                                                       \
@@ -523,15 +525,22 @@ int launch_sink_prep(const SinkPrepArgs &a, bool vec, bool part, hipStream_t s) 
     else TLF_PREP(4, 1, TAPS, false, false);              \
   } while (0)
   if constexpr (sizeof(T) == 2) {
-    // Rows of prompts in runs: long ones where they still are six workgroups for each compute unit (the rows above: runs of 32 90 us, 24 84,
-    // 16 92, 8 106), shorter ones with fewer rows (1700 rows of 16 + 2 x 8 heads: 16 23 us, 8 19, the kernel in front of this one 21).
-    if (vec && !part && most <= 128 && a.n > 1024 && a.rot_dims % 16 == 0 && !a.gate_out && (!a.conv || (a.taps >= 2 && a.taps <= 4))) {
-      const int64_t rows = static_cast<int64_t>(a.n) * hy;
-      const int run = rows >= 24 * 1024 ? 24 : rows >= 16 * 768 ? 16 : 8;
-      const dim3 grid((a.n + run - 1) / run, hy);
+    const int64_t from = vec && !part && most <= 128 && a.rot_dims % 16 == 0 && !a.gate_out && (!a.conv || (a.taps >= 2 && a.taps <= 4))
+                             ? sink_runs_from(a.n, singles, seqs, hy, a.conv != nullptr) : a.n;
+    if (from < a.n) {
+      SinkPrepArgs p = a;
+      p.row0 = static_cast<int32_t>(from);
+      if (p.row0) {
+        SinkPrepArgs first = a;
+        first.n = p.row0;
+        if (int rc = launch_sink_prep<T>(first, vec, part, 0, 0, s)) return rc;
+      }
+      const int64_t behind = a.n - from;
+      const int run = sink_run_rows(behind, hy);
+      const dim3 grid((behind + run - 1) / run, hy);
 #define TLF_RUNS(TAPS)                                                                                               \
-  if (a.rot_dims == 128) TLF_LAUNCH((sink_prep_rows_kernel<TAPS, true>), grid, dim3(256), 0, s, a, run);              \
-  else TLF_LAUNCH((sink_prep_rows_kernel<TAPS, false>), grid, dim3(256), 0, s, a, run)
+  if (a.rot_dims == 128) TLF_LAUNCH((sink_prep_rows_kernel<TAPS, true>), grid, dim3(256), 0, s, p, run);              \
+  else TLF_LAUNCH((sink_prep_rows_kernel<TAPS, false>), grid, dim3(256), 0, s, p, run)
       switch (a.conv ? a.taps : 0) {
         case 0: TLF_RUNS(0); break;
         case 2: TLF_RUNS(2); break;
@@ -589,18 +598,19 @@ __global__ __launch_bounds__(256) void conv_tail_kernel(const T *proj, int64_t l
 
 }  // namespace tlf
 
-extern "C" int tlf_sink_prep(const void *proj, int64_t proj_stride, const float *partials, int32_t splits, const float *scale,
-                             const void *bias, const void *conv, int32_t taps, void *ring, const int32_t *state_slots,
-                             int64_t num_state_slots, const int32_t *row_seq, const int32_t *cu_seqlens_q, const void *q_norm,
-                             const void *k_norm, const int64_t *positions, const float *cos_sin, const float *q_mult,
-                             int32_t max_pos, int32_t rot_dims, const int32_t *slot_mapping, void *q_out, void *k_cache,
-                             void *v_cache, void *gate_out, int32_t n, int32_t heads, int32_t kv_heads, int32_t dim,
-                             int32_t vdim, int32_t block_size, int64_t num_pages, float eps, float score_scale, float cap, int32_t dtype, void *stream) {
+extern "C" int tlf_sink_prep_step(const void *proj, int64_t proj_stride, const float *partials, int32_t splits, const float *scale,
+                                  const void *bias, const void *conv, int32_t taps, void *ring, const int32_t *state_slots,
+                                  int64_t num_state_slots, const int32_t *row_seq, const int32_t *cu_seqlens_q, int32_t singles, int32_t num_seqs,
+                                  const void *q_norm, const void *k_norm, const int64_t *positions, const float *cos_sin, const float *q_mult,
+                                  int32_t max_pos, int32_t rot_dims, const int32_t *slot_mapping, void *q_out, void *k_cache,
+                                  void *v_cache, void *gate_out, int32_t n, int32_t heads, int32_t kv_heads, int32_t dim,
+                                  int32_t vdim, int32_t block_size, int64_t num_pages, float eps, float score_scale, float cap, int32_t dtype, void *stream) {
   using namespace tlf;
   SinkPrepArgs a{};
   if (n < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || rot_dims < 0 || rot_dims % 2 || rot_dims > dim) return TLF_E_SHAPE;
   if (dtype != TLF_DT_BF16 && dtype != TLF_DT_F32) return TLF_E_UNSUPPORTED;
   if (cap < 0.f || (conv && (taps < 1 || taps > 64))) return TLF_E_SHAPE;
+  if (singles < 0 || singles > n || num_seqs < 0) return TLF_E_SHAPE;
   if (n == 0) return TLF_OK;
   if (int rc = partials_check(partials, scale, splits, dtype)) return rc;
   if (int rc = sink_cache_make(a.c, k_cache, v_cache, nullptr, 0, block_size, kv_heads, dim, vdim, num_pages)) return rc;
@@ -623,7 +633,19 @@ extern "C" int tlf_sink_prep(const void *proj, int64_t proj_stride, const float 
                    aligned16(conv) && aligned16(ring) && aligned16(q_norm) && aligned16(k_norm) && aligned16(gate_out) &&
                    (rot_dims % 16 || aligned16(cos_sin));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == TLF_DT_BF16 ? launch_sink_prep<unsigned short>(a, vec, splits > 1, s) : launch_sink_prep<float>(a, vec, false, s);
+  return dtype == TLF_DT_BF16 ? launch_sink_prep<unsigned short>(a, vec, splits > 1, singles, num_seqs, s) : launch_sink_prep<float>(a, vec, false, 0, 0, s);
+}
+
+extern "C" int tlf_sink_prep(const void *proj, int64_t proj_stride, const float *partials, int32_t splits, const float *scale,
+                             const void *bias, const void *conv, int32_t taps, void *ring, const int32_t *state_slots,
+                             int64_t num_state_slots, const int32_t *row_seq, const int32_t *cu_seqlens_q, const void *q_norm,
+                             const void *k_norm, const int64_t *positions, const float *cos_sin, const float *q_mult,
+                             int32_t max_pos, int32_t rot_dims, const int32_t *slot_mapping, void *q_out, void *k_cache,
+                             void *v_cache, void *gate_out, int32_t n, int32_t heads, int32_t kv_heads, int32_t dim,
+                             int32_t vdim, int32_t block_size, int64_t num_pages, float eps, float score_scale, float cap, int32_t dtype, void *stream) {
+  return tlf_sink_prep_step(proj, proj_stride, partials, splits, scale, bias, conv, taps, ring, state_slots, num_state_slots, row_seq, cu_seqlens_q, 0, 0, q_norm,
+                            k_norm, positions, cos_sin, q_mult, max_pos, rot_dims, slot_mapping, q_out, k_cache, v_cache, gate_out, n, heads, kv_heads, dim, vdim,
+                            block_size, num_pages, eps, score_scale, cap, dtype, stream);
 }
 
 extern "C" int tlf_conv_tail(const void *proj, int64_t proj_stride, void *ring, const int32_t *state_slots, int64_t num_state_slots,

@@ -86,7 +86,7 @@ class SinkAttention(nn.Module):
         q, gate = ops.sink_prep(proj, kv, self.num_heads, positions, ctx.slot_mapping, self.eps, self.scale, self.cap,
                                 data(self.bias), data(self.conv),
                                 ring, ctx.state_slots, ctx.row_seq if single < n else None, ctx.cu_seqlens_q, weight(self.q_norm),
-                                weight(self.k_norm), self.cos_sin, self.rot_dims, self.temperatures)
+                                weight(self.k_norm), self.cos_sin, self.rot_dims, self.temperatures, min(single, n))
         if ring is not None and single < n:
             ops.conv_tail(proj, ring, ctx.state_slots, ctx.cu_seqlens_q, ctx.seq_starts, single, ctx.cu_seqlens_q.numel() - 1 - single)
         out = torch.empty(n, self.num_heads * self.value_dim, dtype=self.dtype, device=q.device)

@@ -1022,9 +1022,9 @@ class SinkKV:
 
 
 def sink_prep(proj, kv: SinkKV, heads, positions, slot_mapping, eps, scale=1.0, cap=None, bias=None, conv=None, ring=None, state_slots=None,
-              row_seq=None, cu_seqlens_q=None, q_norm=None, k_norm=None, cos_sin=None, rot_dims=0, q_mult=None):
+              row_seq=None, cu_seqlens_q=None, q_norm=None, k_norm=None, cos_sin=None, rot_dims=0, q_mult=None, singles=0):
     """Projection rows ``[q | k | v | gate]`` -> ``(q [N, H, Dp], gate rows [N, >= H * vdim])``; keys and values go to the
-    caches, the score's constants into q.  See ``tlf_sink_prep``; ``proj`` may be ``Deferred`` when every row is a sequence of its own."""
+    caches, the score's constants into q.  See ``tlf_sink_prep_step``; the first ``singles`` rows are sequences of their own, ``proj`` may be ``Deferred`` when every row is."""
     lib = _lib.load()
     dt = kv.k.dtype
     assert proj.dtype == dt
@@ -1056,12 +1056,13 @@ def sink_prep(proj, kv: SinkKV, heads, positions, slot_mapping, eps, scale=1.0, 
         gate = out = torch.empty(n, heads * kv.vdim, dtype=dt, device=kv.k.device)
     else:
         gate = proj[:, channels:]
-    check(lib.tlf_sink_prep(*_source(proj), _opt(bias), _opt(conv), taps, _opt(ring), _opt(state_slots),
-                            ring.shape[0] if ring is not None else 0, _opt(row_seq), _opt(cu_seqlens_q), _opt(q_norm),
+    check(lib.tlf_sink_prep_step(*_source(proj), _opt(bias), _opt(conv), taps, _opt(ring), _opt(state_slots),
+                            ring.shape[0] if ring is not None else 0, _opt(row_seq), _opt(cu_seqlens_q), singles,
+                            cu_seqlens_q.numel() - 1 if row_seq is not None else n, _opt(q_norm),
                             _opt(k_norm), positions.data_ptr(), _opt(cos_sin), _opt(q_mult),
                             tables[0].shape[0] if tables else 1 << 30, rot_dims, slot_mapping.data_ptr(), q.data_ptr(),
                             kv.k.data_ptr(), kv.v.data_ptr(), _opt(out), n, heads, G, kv.dim, kv.vdim, bs, pages, float(eps),
-                            float(scale), float(cap or 0), _dt(kv.k), _stream()), "tlf_sink_prep")
+                            float(scale), float(cap or 0), _dt(kv.k), _stream()), "tlf_sink_prep_step")
     return q, gate
 
 
