@@ -733,7 +733,9 @@ int tlf_residual_layernorm(const void *y, int64_t y_stride, const float *partial
  *   log2(e), with a cap also times 2 / cap (what the kernels below expect in q) -> q_out [n, heads, Dp]
  *   and the cache rows slot_mapping[token] (negative: not stored).  ring [state slots, taps, channels] holds the projected rows
  *   (without bias) of a sequence's last positions, p in row p mod taps: rows of one-token sequences (row_seq NULL, or
- *   cu_seqlens_q of row_seq[row]) are written here, those of portions by tlf_conv_tail afterwards.  gate_out [n, heads * vdim]
+ *   cu_seqlens_q of row_seq[row]) are written here, those of portions by tlf_conv_tail afterwards.  Without a state slot (outside
+ *   [0, num_state_slots)) nothing is kept, and a row sees zeros before it, or its neighbours within four rows of the step: only rows whose results
+ *   nobody reads go without one.  gate_out [n, heads * vdim]
  *   (NULL: not copied) gets the gate's columns; with splits > 1 it must be there and row_seq NULL.
  * tlf_sink_prep_step: the same where the caller knows that the first `singles` rows are one-token sequences and how many sequences there are in all
  *   (num_seqs, 0: it does not): many rows of prompts are then worked on in runs.

@@ -373,9 +373,10 @@ def test_preparation_of_many_rows(sizes, rot, taps):
 @pytest.mark.parametrize("singles,portions,sizes,run,launches", [
     (0, [1500, 23, 24, 25, 47, 5, 2], (32, 8, 128, 128), 8, 1), (3, [3000, 1, 2, 3, 700, 487], (32, 8, 128, 128), 16, 1), (0, [5000, 2, 3, 23, 24, 25, 2500, 47, 601], (32, 8, 128, 128), 24, 1),
     (50, [3000, 7, 8, 9, 500, 1], (32, 8, 128, 128), 8, 2), (7, [4000, 17, 15, 16, 300], (32, 8, 96, 72), 16, 2), (41, [4000, 23, 25, 24, 8000, 331], (16, 4, 64, 64), 24, 2)], ids=str)
-@pytest.mark.parametrize("taps", [2, 4])
-def test_preparation_in_runs_of_every_length(singles, portions, sizes, run, launches, taps):
-    """Runs that begin and end anywhere, single tokens apart or in front, the last run not whole: bit for bit what the kernel for few rows gives."""
+@pytest.mark.parametrize("taps,stateless", [(2, False), (4, False), (4, True)])
+def test_preparation_in_runs_of_every_length(singles, portions, sizes, run, launches, taps, stateless):
+    """Runs that begin and end anywhere, single tokens apart or in front, the last run not whole, every other sequence without a state: bit for bit
+    what the kernel for few rows gives."""
     from tinyllmforge_amd import _lib, ops as P
     (H, G, D, V), g, BF, dev = sizes, torch.Generator(device="cuda").manual_seed(run + taps), torch.bfloat16, "cuda"
     lens = [1] * singles + portions
@@ -392,7 +393,7 @@ def test_preparation_in_runs_of_every_length(singles, portions, sizes, run, laun
     cu = torch.tensor([0] + lens).cumsum(0)
     pos = torch.arange(rows) - cu[seq] + torch.tensor(starts)[seq]
     slots = (torch.tensor([0] + need).cumsum(0)[seq] * 64 + pos).to(torch.int32).to(dev)
-    states = i32([(i + 1) % (len(lens) + 1) for i in range(len(lens))])
+    states = i32([-1 if stateless and i % 2 == 0 else (i + 1) % (len(lens) + 1) for i in range(len(lens))])
 
     def prepared(singles):
         kv, ring, count = P.SinkKV(sum(need), 64, G, D, V, BF, dev), ring0.clone(), _lib.load().tlf_kernel_launches

@@ -386,6 +386,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
       r.end = a.row_seq ? max(static_cast<int>(min(a.cu_q[seq + 1] - tok0, static_cast<int64_t>(count))), tid + 1) : tid + 1;
       r.single = !a.row_seq || a.cu_q[seq + 1] - first == 1;
       r.state = st >= 0 && st < a.num_state_slots && r.pos >= 0 ? st : -1;
+      if (r.state < 0 && a.row_seq) {  // no state, nothing before it: zeros in front of every fourth row, as the kernel above has them with many rows
+        r.back = min(r.back, static_cast<int>(tok & 3));
+        r.end = min(r.end, static_cast<int>((tok | 3) + 1 - tok0));
+      }
     }
     rows[tid] = r;
   }
@@ -424,7 +428,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
     for (int b = 0; b < kBack; ++b) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) hist[b][e] = 0.f;
-      if (r.state < 0 || r.pos <= b) continue;
+      if (r.state < 0 ? b >= r.back : r.pos <= b) continue;
       const T *from = b < r.back ? proj + (tok0 + k - 1 - b) * a.ld
                                  : static_cast<const T *>(a.ring) + (static_cast<int64_t>(r.state) * TAPS + (r.pos - 1 - b) % (TAPS > 0 ? TAPS : 1)) * a.channels + chan;
       Elem<T>::ld8(from, hist[b]);
