@@ -124,12 +124,28 @@ def test_short_portions_keep_the_chunks(H, dk, dv, lens, kernels):
 
 
 @pytest.mark.parametrize("lens,start", [([1500, 33, 1700, 2, 1024, 32], [0, 5, 7, 0, 64, 0]), ([2047], [3]), ([512, 512, 512, 512], [0, 1, 0, 1]),
-                                        ([17, 3000, 31, 40], [1, 1, 0, 9]), ([640, 1, 640], [1, 1, 1])], ids=str)
+                                        ([17, 3000, 31, 40], [1, 1, 0, 9]), ([700, 1, 900], [1, 1, 1])], ids=str)
 @pytest.mark.parametrize("H,dk,dv", [(2, 128, 256), (3, 64, 96)])
 def test_stretches_over_sequences(H, dk, dv, lens, start):
     """Stretches that begin and end anywhere: within a sequence, at its ends, several sequences in one, one sequence in many."""
+    from tinyllmforge_amd import _lib
+    count = _lib.load().tlf_kernel_launches
+    before = count()
     for n, out, state in run(H, dk, dv, 16, lens, start, 16.0, sum(lens)):
         assert out < OUT and state < STATE, (n, out, state)
+    assert count() - before == 4                             # blocks, what stretches add, the states they start from, the scan
+
+
+@pytest.mark.parametrize("seqs", [16, 17, 32, 33, 63, 64, 65])
+def test_stretches_over_many_sequences(seqs):
+    """A lane for each sequence, up to all 64 of them; one more makes two groups."""
+    from tinyllmforge_amd import _lib
+    count = _lib.load().tlf_kernel_launches
+    before, lens = count(), [600 + 37 * (5 * i % 7) - 90 * (i % 3) for i in range(seqs)]
+    lens[40 % seqs] += 4000 * (seqs > 64)                    # groups are cut for a long one only
+    for n, out, state in run(1, 32, 64, 16, lens, [i % 2 for i in range(seqs)], 16.0, seqs):
+        assert out < OUT and state < STATE, (n, out, state)
+    assert count() - before == (4 if seqs <= 64 else 7)
 
 
 # 64 heads of 32 x 64: 512 workgroups fill the chip, 8 stretches of 64 heads; 7 heads: 73 stretches, in two groups of up to 64 sequences
