@@ -134,30 +134,6 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
-// Inclusive sum over the wave's lanes, on the vector ALU.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int dpp_add_int(int v) {
-  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
-}
-__device__ __forceinline__ int wave_sums_up_to(int v) {
-  v = dpp_add_int<0x111, 0xf>(v);      // row_shr 1, 2, 4, 8: within rows of 16 lanes
-  v = dpp_add_int<0x112, 0xf>(v);
-  v = dpp_add_int<0x114, 0xf>(v);
-  v = dpp_add_int<0x118, 0xf>(v);
-  v = dpp_add_int<0x142, 0xa>(v);      // row_bcast 15 into rows 1 and 3
-  return dpp_add_int<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3
-}
-
-// The pieces (chunks or blocks) of up to 64 sequences in a row, cut into `units` equal stretches: lane s has sequence s of `own` pieces,
-// first .. end - 1 of all.  Products stay within 2^31: the callers have up to 2^22 pieces and 512 stretches.
-__device__ __forceinline__ void stretch_ranges(int own, int &first, int &end, int &all) {
-  end = wave_sums_up_to(own);
-  first = end - own;
-  all = __builtin_amdgcn_readlane(end, 63);
-}
-__device__ __forceinline__ int stretch_begin(int unit, int units, int all) { return static_cast<unsigned int>(unit) * all / static_cast<unsigned int>(units); }
-__device__ __forceinline__ int stretch_of(int piece, int units, int all) { return (static_cast<unsigned int>(piece + 1) * units - 1) / static_cast<unsigned int>(all); }
-
 // A value that is the same in all lanes and that nothing in the launch writes, through the scalar path: behind stores the compiler would load it
 // for every lane.
 template <typename T>

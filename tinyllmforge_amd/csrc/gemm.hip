@@ -1600,6 +1600,10 @@ int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *sca
 //   390 rows (3500 tokens, 1024)                            61.5, 78.9, 87.4 / 36.8, 40.1, 39.1
 //   47 rows (400 tokens, 64 of 1536 at 4096)                256 x 128 347, 128 x 128 393, four waves 367 / 168, 174, 175
 //   350 rows (3000 tokens, 4096)                            699, 766, 718 / 383, 419, 384
+// Between the two widths, gate_up in 128 x 128 / 256 x 128 / four waves: the first ends where experts are many and wide.
+//   250 rows, 32 of 768 (2000 tokens)                       K 1536 59, 72, 77; 2048 75, 91, 95; 3072 121, 136, 141; 4096 164, 172, 181
+//   62 rows, 64 of 1536 (500 tokens)                        K 1536 127, 130, 138; 2048 195, 175, 185; 3072 231, 229, 240; 4096 363, 307, 319
+//   250 rows, 64 of 1536 (2000 tokens)                      K 1536 235, 235, 245; 2048 299, 295, 310; 3072 431, 421, 435; 4096 565, 546, 571
 //   2048 rows (16,384 tokens, 4096)                         256 x 256: 3066 / 1704   256 x 128: 3187 / 1879 128 x 128: 3865 / 2298
 int launch_grouped(GemmParams p, int bm, hipStream_t stream) {
   if (p.N % 16 || p.K % kBK || p.m_tiles <= 0) return TLF_E_SHAPE;

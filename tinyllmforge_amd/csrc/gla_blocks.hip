@@ -9,7 +9,7 @@
 //                          the order the matrix cores read.  A = (q 2^b_t) (k 2^-b_s)^T as products of pieces, too, unless some channel
 //                          decays by more than 2^64 within the block.  Then every exponent is kept <= 0: the 8 x 8 blocks on A's
 //                          diagonal are formed pair by pair, those left of it through the value at the boundary in front of them
-//   gla_block_scan_kernel  per (sequence or segment, head) a workgroup with 32 columns of v per wave, sequential over the blocks:
+//   gla_block_scan_kernel  per (sequence or stretch, head) a workgroup with 32 columns of v per wave, sequential over the blocks:
 //                          O^T = S^T Qd^T + V^T A^T, out = norm and output gate of O;  S = diag(2^b_end) S + Kd^T V.  S stays in fp32
 //                          accumulators; their layout is the next block's operand when the summation index is labelled as Qd is laid
 //                          out.  A block's record and rows of v come into LDS one block ahead, and the rows' sums of squares
@@ -22,8 +22,8 @@
 // segments 59 + 18 + 255 us, so 58 + 15 + 209; 12 of 450 to 900 48 + 24 + 216, and in one pass over whole ones 204.
 //
 // Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256, medians under the profiler: chunk 122 + scan 470 (both
-// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 149 + first pass 62 + segments 19 + scan
-// 278 us (whole layer without it 614 and 449 us).  The blocks write 55 KB a record, 4 TB/s with what they read; the scan is held by its
+// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 149 + first pass 61 + chaining 15 + scan
+// 210 us (whole layer 614 and 390 us).  The blocks write 55 KB a record, 4 TB/s with what they read; the scan is held by its
 // barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's error against 64 bits is 5e-8 to 1.1e-7 on both, the
 // output's is its rounding to bf16.
 #include <algorithm>
@@ -264,6 +264,30 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
     for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4 *>(rec + Rec::kA + i * Rec::kAPiece + tid * 16) = p3[i];
   }
 }
+
+// Inclusive sum over the wave's lanes, on the vector ALU.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add_int(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ int wave_sums_up_to(int v) {
+  v = dpp_add_int<0x111, 0xf>(v);      // row_shr 1, 2, 4, 8: within rows of 16 lanes
+  v = dpp_add_int<0x112, 0xf>(v);
+  v = dpp_add_int<0x114, 0xf>(v);
+  v = dpp_add_int<0x118, 0xf>(v);
+  v = dpp_add_int<0x142, 0xa>(v);      // row_bcast 15 into rows 1 and 3
+  return dpp_add_int<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3
+}
+
+// The blocks of up to 64 sequences in a row, cut into `units` equal stretches: lane s has sequence s of `own` blocks,
+// first .. end - 1 of all.  Products stay within 2^31: there are up to 2^22 blocks and 512 stretches.
+__device__ __forceinline__ void stretch_ranges(int own, int &first, int &end, int &all) {
+  end = wave_sums_up_to(own);
+  first = end - own;
+  all = __builtin_amdgcn_readlane(end, 63);
+}
+__device__ __forceinline__ int stretch_begin(int unit, int units, int all) { return static_cast<unsigned int>(unit) * all / static_cast<unsigned int>(units); }
+__device__ __forceinline__ int stretch_of(int block, int units, int all) { return (static_cast<unsigned int>(block + 1) * units - 1) / static_cast<unsigned int>(all); }
 
 // Lane s: blocks of sequence s.
 __device__ __forceinline__ int gla_own_blocks(const GlaArgs &a, int lane) { return lane < a.seqs ? (a.cu_chunks[lane + 1] - a.cu_chunks[lane] + 1) / 2 : 0; }

@@ -154,11 +154,6 @@ __device__ __forceinline__ void talk_plan(const TalkPrefillArgs &p, int32_t *sha
   }
 }
 
-template <typename T>
-__device__ __forceinline__ T talk_uniform(const T *p) {              // through the scalar path
-  return *(const T __attribute__((address_space(4))) *)(reinterpret_cast<uintptr_t>(p));
-}
-
 constexpr int kTS = 64;             // keys per tile of the first kernel
 __device__ __forceinline__ int talk_tile_row(int t) { return (t & 32) | ((t & 4) << 2) | ((t & 24) >> 1) | (t & 3); }
 
@@ -331,7 +326,7 @@ __device__ __forceinline__ void talk_prefill_tile(const TalkPrefillArgs &p, cons
   unsigned short *Vs = lds, *Wh = lds + p.c.G * kTK * VP, *Wl = Wh + TQ * ROW, *Ts = Wl + TQ * ROW;    // Vs [G][32][VP], Ts [16 HT][TS]
   const SinkCache &c = p.c;
   const int seq = p.first_seq + item.sq;
-  const int q0 = talk_uniform(p.cu_q + seq), lq = talk_uniform(p.cu_q + seq + 1) - q0, start = talk_uniform(p.starts + seq);
+  const int q0 = load_uniform(p.cu_q + seq), lq = load_uniform(p.cu_q + seq + 1) - q0, start = load_uniform(p.starts + seq);
   const int row0 = item.xt * TQ;
   if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
   const int32_t *bt = c.bt + seq * c.bt_stride;
@@ -342,13 +337,13 @@ __device__ __forceinline__ void talk_prefill_tile(const TalkPrefillArgs &p, cons
   const int wave_first = start + min(row0 + rt, last_row);           // keys behind it are masked for some row of the wave
   auto head_of = [](int e) { return e / PER * HK + e % HK; };        // of the wave's heads; and the row tile
   auto tile_of = [](int e) { return e % PER / HK; };
-  const int first = item.first, tiles = item.slot >= 0 && item.slot < p.split.most ? first + talk_uniform(p.split.plan) : i_last / kTK + 1;
+  const int first = item.first, tiles = item.slot >= 0 && item.slot < p.split.most ? first + load_uniform(p.split.plan) : i_last / kTK + 1;
   // where a tile lies: its page (an unmapped one reads page 0) and its first row there, stepped tile by tile
   struct Place {
     int index, page, row;
   };
   auto page_at = [&](int index) __attribute__((always_inline)) {
-    const int page = talk_uniform(bt + index);
+    const int page = load_uniform(bt + index);
     return page >= 0 && page < c.pages ? page : 0;
   };
   auto after = [&](const Place &at, bool more) __attribute__((always_inline)) {       // the next tile's, if there is one
