@@ -296,6 +296,7 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     gla = lambda dk=16, dv=16, r=4, ld=132, tau=2.0: lib.tlf_gla_decode(a, ld, None, 1, None, a, a, a, a, a, 4, a, a, 64, 2, 2, dk, dv, r, tau, 1.0, 1e-6, 0, None)
     assert gla(dk=300, ld=4000) == -2 and gla(ld=131) == -2 and gla(tau=0.0) == -2 and gla(dv=1000, ld=8000) == -2
     assert lib.tlf_gla_portions(a, 132, a, a, a, a, a, 4, a, a, a, a, 1, 0, 1, a, 64, 8, 2, 16, 16, 4, 2.0, 1.0, 1e-6, 0, None, 0, None) == -4
+    assert lib.tlf_gla_portions_upto(a, 132, a, a, a, a, a, 4, a, a, a, a, 1, 0, 1, 9, a, 64, 8, 2, 16, 16, 4, 2.0, 1.0, 1e-6, 0, None, 0, None) == -4
     assert lib.tlf_f32_gemm(a, 8, a, a, 2, 4, 16, None) == -2 and lib.tlf_f32_argmax(a, 4, a, 1, 8, None) == -2
 
 

@@ -207,7 +207,7 @@ CUTS = [[(0, 1500)], [(2048, 40)], [(0, 31), (0, 32), (0, 33), (96, 64), (95, 65
 
 @pytest.mark.parametrize("portions", CUTS, ids=str)
 @pytest.mark.parametrize("sizes", [(4, 2, 64, 64), (8, 8, 96, 40), (16, 8, 128, 128), (12, 12, 96, 80), (32, 8, 128, 128)], ids=str)
-def test_talking_heads_with_keys_cut(sizes, portions):
+def test_talking_heads_with_keys_cut(sizes, portions, monkeypatch):
     """Parts of a row tile's keys added up against whole tiles: sums of the same products in another order."""
     from tinyllmforge_amd import _lib, ops as P
     (H, G, D, V), g, bs = sizes, torch.Generator(device="cuda").manual_seed(3), 64
@@ -227,6 +227,7 @@ def test_talking_heads_with_keys_cut(sizes, portions):
     lib, ptr, most = _lib.load(), lambda t: t.data_ptr(), max(lens)
     stats = torch.empty(rows, H, device="cuda")
     assert lib.tlf_talk_attn_prefill_workspace_bytes(len(need), most, bt.stride(0) * bs, H, G, D, V) or bt.stride(0) * bs <= 96
+    monkeypatch.setattr(P, "talk_prefill_cuts", lambda *a: True)      # whether it pays or not
     P.talk_attention_prefill(q, kv, bt, cu, starts, 1, len(need), most, talk, got)
     assert lib.tlf_talk_attn_prefill(ptr(q), ptr(kv.k), ptr(kv.v), ptr(bt), bt.stride(0), ptr(cu), ptr(starts), 1, len(need), most, ptr(talk), ptr(stats),
                                      ptr(whole), whole.stride(0), H, G, D, V, bs, kv.k.shape[0], torch.cuda.current_stream().cuda_stream) == 0

@@ -409,6 +409,37 @@ def test_preparation_in_runs_of_every_length(singles, portions, sizes, run, laun
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("taps", [0, 2, 3, 4])
+@pytest.mark.parametrize("sizes,rot", [((6, 2, 56, 104), 48), ((3, 3, 64, 8), 0), ((16, 4, 96, 128), 32), ((2, 1, 128, 32), 128)], ids=str)
+def test_preparation_in_runs_of_other_sizes(sizes, rot, taps):
+    """Head sizes that are not whole, rotations of a part or none, weights that are not there: bit for bit what the kernel for few rows gives."""
+    from tinyllmforge_amd import ops as P
+    (H, G, D, V), g, BF, dev = sizes, torch.Generator(device="cuda").manual_seed(rot + taps), torch.bfloat16, "cuda"
+    lens, starts = [3000, 7, 1, 24, 2200, 5, 90], [0, 64, 3, 0, 2, 1, 700]
+    rows, channels, i32 = sum(lens), (H + G) * D + G * V, lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    randn = lambda *s: torch.randn(*s, generator=g, device=dev).to(BF)
+    proj, bias, conv, ring0 = randn(rows, channels + H * V), randn(channels), randn(max(taps, 1), channels), randn(len(lens), max(taps, 1), channels)
+    qn, table, temps = 1 + 0.1 * randn(D), torch.randn(3100, max(rot, 1), generator=g, device=dev), torch.rand(3100, generator=g, device=dev)
+    seq = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens))
+    cu = torch.tensor([0] + lens).cumsum(0)
+    pos, slots = (torch.arange(rows) - cu[seq] + torch.tensor(starts)[seq]).to(dev), torch.randperm(rows, generator=g, device=dev).to(torch.int32)
+    slots[[0, 3008, rows - 1]] = -1                                  # not stored
+
+    def prepared(parts, singles=0):
+        kv, ring, q = P.SinkKV(-(-rows // 64), 64, G, D, V, BF, dev), ring0.clone(), []
+        held = dict(bias=bias, conv=conv, ring=ring, state_slots=i32(list(range(len(lens)))), row_seq=seq.to(torch.int32).to(dev), cu_seqlens_q=i32(cu.tolist()),
+                    singles=singles) if taps else {}
+        for a, b in parts:
+            q.append(P.sink_prep(proj[a:b], kv, H, pos[a:b].contiguous(), slots[a:b].contiguous(), 1e-5, 0.3, 20.0, q_norm=qn, cos_sin=table if rot else None, rot_dims=rot,
+                                 q_mult=temps, **held)[0])
+        return torch.cat(q), kv.k, kv.v, ring
+
+    # with a convolution, all rows said to be sequences of their own; without one, few rows at a time
+    want = prepared([(0, rows)], rows) if taps else prepared([(a, min(a + 1000, rows)) for a in range(0, rows, 1000)])
+    for a, b in zip(prepared([(0, rows)]), want):
+        assert torch.equal(a, b)
+
+
 # ---------------------------------------------------------------------------------------------- experts
 @pytest.mark.parametrize("corr_dtype", DTYPES)
 @pytest.mark.parametrize("n,E,ident,top,splits", [(1, 5, 2, 2, 1), (64, 70, 7, 6, 3), (500, 16, 1, 1, 2), (1500, 33, 3, 4, 1), (9, 500, 12, 20, 1),

@@ -372,6 +372,9 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     assert room() > 0 and room(keys=96) == 0 and room(n=0) == 0 and room(n=600) == 0 and room(sizes=(33, 1, 20, 13)) == 0
     cut = lambda ws=None, nb=0, ldo=78, out=a, n=1: lib.tlf_talk_attn_prefill_cut(a, a, a, a, 4, a, a, 0, n, 8, a, a, out, ldo, *shape, 64, 10, ws, nb, None)
     assert cut() == WORK and cut(ws=a, nb=room() - 1) == WORK and cut(ldo=70) == SHAPE and cut(out=None) == NULL and cut(n=0) == 0
+    pays = lambda n=1, most=5000, rows=5000, keys=5056, sizes=(16, 8, 128, 128): lib.tlf_talk_attn_prefill_cuts(n, most, rows, keys, *sizes)
+    assert pays() == 1 and pays(n=0) == 0 and pays(most=0) == 0 and pays(sizes=(33, 1, 64, 64)) == 0 and pays(n=24, most=250, rows=6000, keys=256) == 0
+    assert lib.tlf_talk_attn_prefill_tile_rows(16, 8, 128, 128) == 32 and lib.tlf_talk_attn_prefill_tile_rows(33, 1, 64, 64) == 0
     ok = lib.tlf_talk_attn_prefill_supported
     assert ok(32, 8, 128, 128) == 1 and ok(33, 1, 64, 64) == 0 and ok(4, 2, 129, 64) == 0 and ok(4, 2, 64, 129) == 0 and ok(1, 1, 1, 1) == 1
 

@@ -351,6 +351,9 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     assert prep(bs=100) == -2 and prep(sizes=(3, 2, 20, 13)) == -2 and prep(sizes=(3, 1, 600, 13), ld=9999) == -2
     assert prep(conv=a, taps=3) == -1 and prep(conv=a, taps=99, ring=a) == -2 and prep(conv=a, taps=3, ring=a, seq=a) == -1
     assert prep(sp=3) == -1 and prep(sp=3, p=a) == -5 and prep(sp=3, p=a, gate=a) == -5 and prep(dt=7) == -5      # sizes not multiples of 8
+    step = lambda singles, seqs, n=2: lib.tlf_sink_prep_step(a, 136, None, 1, None, a, None, 0, None, a, 4, None, None, singles, seqs, a, a, a, a, None, 10, 12, a, a, a, a, None, n, *shape,
+                                                             64, 5, 1e-6, 0.1, 0.0, 0, None)
+    assert step(-1, 2) == -2 and step(3, 3) == -2 and step(0, -1) == -2 and step(0, 0, n=0) == 0
     tail = lambda taps=3, ld=136, ring=a, n=1: lib.tlf_conv_tail(a, ld, ring, a, 4, a, a, 0, n, taps, 93, 0, None)
     assert tail(ld=80) == -2 and tail(ring=None) == -1 and tail(n=0) == 0 and tail(taps=1) == 0 and tail(taps=0) == -2
     rows = lambda sizes=shape, cap=0.0, ldo=39, ldg=39, bt=4, most=200, out=a, ws=None, dt=0, n=2: lib.tlf_sink_attn_rows(
