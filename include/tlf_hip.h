@@ -812,9 +812,11 @@ int tlf_rows_rmsnorm(const void *x, int64_t x_stride, const void *w, void *out, 
  *   on kv_heads * vdim (tlf_talk_attn_prefill_supported).  stats: scratch, [rows of the step, heads].
  * tlf_talk_attn_prefill_cut: the same; with few portions the keys of long row tiles are cut into parts that run at once.  The workspace is
  *   sized for max_keys = bt_stride * block_size; 0 bytes: nothing will be cut, it may be NULL.
- * tlf_talk_attn_prefill_cuts: whether that is the faster one for portions of `rows` rows in all.  tlf_talk_attn_prefill_tile_rows: rows of a
- *   row tile, 0 for sizes that are not supported.  Every portion takes workgroups for the row tiles of the longest: portions of very
- *   different lengths are better left to calls of their own. */
+ * tlf_talk_attn_prefill_cuts: whether that is the faster one for portions of `rows` rows in all; reads: the keys that rows see, summed over the
+ *   rows (0: not known).  tlf_talk_attn_prefill_tile_rows: rows of a row tile, 0 for sizes that are not supported.
+ * tlf_talk_attn_prefill_route: how a step's short portions run fastest, beside its long ones and `singles` single tokens: 0 row by row
+ *   (tlf_talk_attn_rows), 1 in one call with the long ones, 2 in a call of their own.  Both arrays, on the host: portions, the most tokens of one,
+ *   rows in all, reads, the most keys of one. */
 int tlf_talk_prep(const void *proj, int64_t proj_stride, const float *partials, int32_t splits, const float *scale, const void
                   *q_norm, const void *k_norm, const void *temp, const int64_t *positions, const float *cos_sin, int32_t
                   max_pos, int32_t rot_dims, const int32_t *slot_mapping, void *q_out, void *k_cache, void *v_cache,
@@ -834,8 +836,10 @@ int tlf_talk_attn_prefill(const void *q, const void *k_cache, const void *v_cach
                           int32_t kv_heads, int32_t dim, int32_t vdim, int32_t block_size, int64_t num_pages, void
                           *stream);
 int tlf_talk_attn_prefill_tile_rows(int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim);
-int tlf_talk_attn_prefill_cuts(int32_t num_seqs, int32_t max_tokens, int32_t rows, int64_t max_keys, int32_t heads, int32_t kv_heads,
-                               int32_t dim, int32_t vdim);
+int tlf_talk_attn_prefill_cuts(int32_t num_seqs, int32_t max_tokens, int32_t rows, int64_t reads, int64_t max_keys, int32_t heads,
+                               int32_t kv_heads, int32_t dim, int32_t vdim);
+int tlf_talk_attn_prefill_route(int32_t singles, const int64_t *short_portions, const int64_t *long_portions, int32_t heads, int32_t kv_heads,
+                                int32_t dim, int32_t vdim);
 size_t tlf_talk_attn_prefill_workspace_bytes(int32_t num_seqs, int32_t max_tokens, int64_t max_keys, int32_t heads,
                                              int32_t kv_heads, int32_t dim, int32_t vdim);
 int tlf_talk_attn_prefill_cut(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables, int64_t

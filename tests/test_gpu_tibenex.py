@@ -276,7 +276,7 @@ def test_lists_of_more_items_than_workgroups(sizes, portions):
     torch.testing.assert_close(got.float(), whole.float(), rtol=2 ** -7, atol=2 ** -14)
 
 
-def layer_in_tiles_and_by_rows(lens, starts, monkeypatch):
+def layer_in_tiles_and_by_rows(lens, starts, monkeypatch, told=True):
     """What a layer of 8 heads gives for portions of ``lens`` tokens behind ``starts``, as it chooses and row by row, and the calls in row tiles:
     the first portion of each, their number."""
     from types import SimpleNamespace
@@ -292,7 +292,8 @@ def layer_in_tiles_and_by_rows(lens, starts, monkeypatch):
         at += need[i]
     d = {k: torch.from_numpy(v).cuda() if hasattr(v, "dtype") else v for k, v in portion_inputs(seqs, 64, 128).items()}
     positions = d.pop("positions")
-    d.pop("input_ids")
+    for name in ("input_ids",) + (() if told else ("max_short", "short_reads", "short_keys", "long_reads", "long_keys")):
+        d.pop(name)
     most = max(a + n for a, n in zip(starts, lens))
     with torch.device("cuda"):
         layer = TalkingHeadsAttention(H, G, D, D, D ** -0.5, 1e-6, BF, D).to(BF)
@@ -329,12 +330,20 @@ def test_short_portions_in_tiles(portions, tiles, monkeypatch):
 
 @pytest.mark.parametrize("short,long,held,calls", [([20] * 13, [2500], 70, [(1, 13), (14, 1)]), ([20] * 13, [300, 131], 70, [(1, 15)]), ([40] * 30, [500], 1000, [(1, 30), (31, 1)]), ([40] * 20, [700], 1000, [(1, 21)]),
                                                    ([20] * 7, [2500], 70, [(1, 8)]), ([2] * 3, [2500, 600], 70, [(4, 2)]),
-                                                   ([2] * 33, [200], 1000, [(34, 1)]), ([2] * 33, [], 400, []), ([3] * 33, [], 400, [(1, 33)])], ids=str)
+                                                   ([2] * 33, [], 1000, []), ([3] * 33, [], 400, []), ([3] * 100, [], 1000, [(1, 100)])], ids=str)
 def test_long_portions_among_short_ones(short, long, held, calls, monkeypatch):
     """Short portions share a call with the long ones only where these do not give them many row tiles that are empty."""
     lens, starts = [1] + short + long, [64] + [held] * len(short) + [0] * len(long)
     got, want, made = layer_in_tiles_and_by_rows(lens, starts, monkeypatch)
     assert made == calls
+    torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -10)      # as above
+
+
+@pytest.mark.parametrize("short,long", [([20] * 13, [2500]), ([20] * 13, [300]), ([60] * 30, [])], ids=str)
+def test_contexts_that_do_not_tell_what_portions_read(short, long, monkeypatch):
+    """The choice is a guess then, the results are not."""
+    got, want, calls = layer_in_tiles_and_by_rows([1] + short + long, [64] + [70] * len(short) + [0] * len(long), monkeypatch, told=False)
+    assert calls
     torch.testing.assert_close(got, want, rtol=2 ** -7, atol=2 ** -10)      # as above
 
 

@@ -13,7 +13,10 @@ SOURCE = """
 #include "talk_split.h"
 using namespace tlf;
 extern "C" int cuts(long portions, long tokens, long keys, int tq) { return talk_cuts(portions, tokens, keys, tq); }
-extern "C" int pays(long portions, long tokens, long rows, long keys, int tq) { return talk_cuts_pay(portions, tokens, rows, keys, tq); }
+extern "C" int pays(const long *l, int tq) { return talk_cuts_pay({l[0], l[1], l[2], l[3], l[4]}, tq); }
+extern "C" int route(int singles, const long *s, const long *l, int heads, int tq) {
+  return talk_route(singles, {s[0], s[1], s[2], s[3], s[4]}, {l[0], l[1], l[2], l[3], l[4]}, heads, tq);
+}
 extern "C" int steps(int start, int tokens, int tq, int x) { return talk_steps(start, tokens, tq, x); }
 extern "C" int tiles(int tokens, int tq) { return talk_tiles(tokens, tq); }
 extern "C" int extras(int n, int per) { return talk_extras(n, per); }
@@ -37,7 +40,6 @@ def lib(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-O2", "-I", CSRC, str(at / "split.cpp"), "-o", str(at / "split.so")], check=True)
     lib = ctypes.CDLL(str(at / "split.so"))
     lib.cuts.argtypes = [ctypes.c_long] * 3 + [ctypes.c_int]
-    lib.pays.argtypes = [ctypes.c_long] * 4 + [ctypes.c_int]
     return lib
 
 
@@ -67,14 +69,40 @@ def test_which_launches_are_cut(lib):
     assert not lib.cuts(1, 90, 96, 32) and not lib.cuts(16, 300, 4000, 16) and not lib.cuts(9, 2048, 2048, 32) and not lib.cuts(64, 128, 128, 32)
 
 
-# portions, their longest, rows of all, keys at most, rows of a tile
-@pytest.mark.parametrize("launch", [(1, 8000, 8000, 8000, 16), (4, 2048, 8192, 2048, 16), (3, 2600, 7800, 2624, 16), (24, 250, 6000, 256, 32), (48, 128, 6144, 1152, 32),
-                                    (24, 128, 3072, 1152, 16), (12, 250, 3000, 256, 16), (9, 2048, 18432, 2048, 32)], ids=str)
-def test_launches_that_whole_tiles_do_better(lib, launch):
-    assert not lib.pays(*launch)
+# portions as (tokens held before, tokens brought), rows of a tile; measured, us in parts and whole
+WHOLE = [([(0, 8000)], 16), ([(0, 2048)] * 4, 16), ([(0, 2600)] * 3, 16),                                     # 1530, 1421; 483, 449; 565, 535
+         ([(1024, 600)] * 8, 16), ([(0, 800)] * 7, 16), ([(1024, 600)] * 7, 16), ([(2048, 2000)] * 4, 16),    # 484, 448; 227, 199; 480, 432; 1279, 1205
+         ([(0, 250)] * 24, 32), ([(1024, 128)] * 48, 32), ([(1024, 128)] * 24, 16), ([(0, 250)] * 12, 16),    # 93, 89; 272, 251; 267, 230; 93, 88
+         ([(0, 2048)] * 9, 32)]                                                                               # more tiles than a plan holds
+PARTS = [([(0, 8000)], 32), ([(0, n) for n in range(1061, 2048, 141)], 32), ([(2048, 130)], 32), ([(0, 400)] * 12, 32),      # 795, 1280; 353, 399; 92, 355; 99, 106
+         ([(0, n) for n in (1024, 1365, 1706, 2048)], 16), ([(0, 4000)], 16), ([(0, 1500)] * 5, 16), ([(0, 1300)] * 6, 16),  # 347, 375; 453, 640; 419, 506; 388, 422
+         ([(0, 850)] * 9, 16), ([(0, 640)] * 12, 16), ([(4096, 300)] * 4, 16), ([(0, n) for n in range(300, 601, 15)], 32)]  # 288, 345; 235, 247; 357, 696; 153, 166
+load = lambda ps: (ctypes.c_long * 5)(len(ps), max([n for _, n in ps], default=0), sum(n for _, n in ps), sum(n * a + n * (n + 1) // 2 for a, n in ps),
+                                      max([a + n for a, n in ps], default=0))
 
 
-@pytest.mark.parametrize("launch", [(1, 8000, 8000, 8000, 32), (8, 2048, 12000, 2048, 32), (4, 2048, 6143, 2048, 16), (6, 1300, 7800, 1344, 16), (1, 130, 130, 2240, 32),
-                                    (12, 400, 4800, 448, 32), (1, 4000, 4000, 4032, 16), (20, 600, 9000, 640, 32)], ids=str)
-def test_launches_that_parts_do_better(lib, launch):
-    assert lib.pays(*launch) and lib.cuts(launch[0], launch[1], launch[3], launch[4])       # which is what the workspace is sized for
+@pytest.mark.parametrize("portions,tq,pays", [(*v, False) for v in WHOLE] + [(*v, True) for v in PARTS], ids=[f"whole {i}" for i in range(len(WHOLE))] + [f"parts {i}" for i in range(len(PARTS))])
+def test_launches_that_parts_do_better(lib, portions, tq, pays):
+    v = load(portions)
+    assert lib.pays(v, tq) == pays
+    if pays:                                                         # which is what the workspace is sized for
+        assert lib.cuts(v[0], v[1], v[4], tq)
+
+
+ROWS, TOGETHER, APART = range(3)
+
+
+# short and long portions as (tokens held before, tokens brought), single tokens, heads; measured, one by one in us: row by row, together, apart
+STEPS = [([(0, 9)] * 7, [], 0, 16, ROWS), ([(2048, 2)] * 33, [], 0, 16, ROWS),              # fewer than 64 rows; 128, 158
+         ([(0, 100)], [], 0, 16, ROWS), ([(4096, 100)], [], 0, 16, TOGETHER),               # 26, 43; 237, 146
+         ([(64, 4)] * 16, [], 0, 32, ROWS), ([(1024, 4)] * 64, [], 0, 32, TOGETHER),        # 22, 37; 194, 143
+         ([(2048, 3)] * 100, [], 0, 16, TOGETHER), ([(2048, 2)] * 200, [], 0, 32, TOGETHER),  # 445, 320; 683, 570
+         ([(64, 20)] * 30, [(0, 200)], 0, 16, TOGETHER), ([(1024, 20)] * 30, [(0, 200)], 0, 16, APART),         # 118, 66, 87; 399, 210, 140
+         ([(1024, 20)] * 40, [(0, 1000)], 0, 32, APART), ([(0, 100)] * 10, [(0, 300)] * 3, 0, 16, TOGETHER),    # 591, 376, 243; 158, 70, 100
+         ([(64, 10)] * 60, [(0, 4000)], 0, 32, APART), ([(2048, 2)] * 33, [(0, 4000)], 0, 32, ROWS),            # 533, 1419, 498; 585, 996, 649
+         ([(1024, 20)] * 4, [(0, 300)], 0, 32, TOGETHER), ([(0, 16)] * 4, [(64, 130)], 2, 16, TOGETHER)]        # 126, 79, 120; not measured
+
+
+@pytest.mark.parametrize("short,long,singles,heads,want", STEPS, ids=[str(i) for i in range(len(STEPS))])
+def test_how_short_portions_run(lib, short, long, singles, heads, want):
+    assert lib.route(singles, load(short), load(long), heads, 16 if heads > 16 else 32) == want

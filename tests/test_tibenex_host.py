@@ -372,7 +372,7 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     assert room() > 0 and room(keys=96) == 0 and room(n=0) == 0 and room(n=600) == 0 and room(sizes=(33, 1, 20, 13)) == 0
     cut = lambda ws=None, nb=0, ldo=78, out=a, n=1: lib.tlf_talk_attn_prefill_cut(a, a, a, a, 4, a, a, 0, n, 8, a, a, out, ldo, *shape, 64, 10, ws, nb, None)
     assert cut() == WORK and cut(ws=a, nb=room() - 1) == WORK and cut(ldo=70) == SHAPE and cut(out=None) == NULL and cut(n=0) == 0
-    pays = lambda n=1, most=5000, rows=5000, keys=5056, sizes=(16, 8, 128, 128): lib.tlf_talk_attn_prefill_cuts(n, most, rows, keys, *sizes)
+    pays = lambda n=1, most=5000, rows=5000, keys=5056, sizes=(16, 8, 128, 128): lib.tlf_talk_attn_prefill_cuts(n, most, rows, 0, keys, *sizes)
     assert pays() == 1 and pays(n=0) == 0 and pays(most=0) == 0 and pays(sizes=(33, 1, 64, 64)) == 0 and pays(n=24, most=250, rows=6000, keys=256) == 0
     assert lib.tlf_talk_attn_prefill_tile_rows(16, 8, 128, 128) == 32 and lib.tlf_talk_attn_prefill_tile_rows(33, 1, 64, 64) == 0
     ok = lib.tlf_talk_attn_prefill_supported
@@ -403,11 +403,3 @@ def test_few_state_space_groups_keep_a_head_per_workgroup(sizes, seqs, tokens, s
     parts = seqs * segments * H if segments > 1 else 0
     want = up(2 * rows * (H * P + 2 * G * N)) + 2 * up(4 * rows * H) + up(4 * parts) + up(4 * parts * N * P)
     assert _lib.load().tlf_ssd_portions_workspace_bytes(rows, seqs, tokens, *sizes, 0) == want
-
-
-def test_short_portions_of_few_rows_go_row_by_row():
-    from tinyllmforge_amd.layers.talking_attention import short_in_tiles
-    for portions, rows, keys in ((1, 64, 4160), (8, 64, 2112), (12, 72, 2112), (100, 200, 1088), (60, 900, 1088), (33, 66, 192), (4, 64, 192)):
-        assert short_in_tiles(portions, rows, keys)
-    for portions, rows, keys in ((0, 0, 64), (7, 63, 192), (33, 66, 512), (33, 66, 4160), (16, 64, 1088), (22, 66, 2112)):
-        assert not short_in_tiles(portions, rows, keys)

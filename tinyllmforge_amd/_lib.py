@@ -146,7 +146,8 @@ SIGNATURES = {
     "tlf_talk_attn_prefill": (c_int32, [_P, _P, _P, _P, _I64, _P, _P, _I32, _I32, _I32, _P, _P, _P, _I64, _I32, _I32,
                                         _I32, _I32, _I32, _I64, _P]),
     "tlf_talk_attn_prefill_tile_rows": (c_int32, [_I32, _I32, _I32, _I32]),
-    "tlf_talk_attn_prefill_cuts": (c_int32, [_I32, _I32, _I32, _I64, _I32, _I32, _I32, _I32]),
+    "tlf_talk_attn_prefill_cuts": (c_int32, [_I32, _I32, _I32, _I64, _I64, _I32, _I32, _I32, _I32]),
+    "tlf_talk_attn_prefill_route": (c_int32, [_I32, _P, _P, _I32, _I32, _I32, _I32]),
     "tlf_talk_attn_prefill_workspace_bytes": (_SZ, [_I32, _I32, _I64, _I32, _I32, _I32, _I32]),
     "tlf_talk_attn_prefill_cut": (c_int32, [_P, _P, _P, _P, _I64, _P, _P, _I32, _I32, _I32, _P, _P, _P, _I64, _I32,
                                             _I32, _I32, _I32, _I32, _I64, _P, _SZ, _P]),

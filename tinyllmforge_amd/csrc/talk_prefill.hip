@@ -807,10 +807,18 @@ extern "C" int tlf_talk_attn_prefill_tile_rows(int32_t heads, int32_t kv_heads, 
   return tlf_talk_attn_prefill_supported(heads, kv_heads, dim, vdim) ? talk_row_tiles(talk_quads(heads), kv_heads, (vdim + 31) / 32 * 32) * 16 : 0;
 }
 
-extern "C" int tlf_talk_attn_prefill_cuts(int32_t num_seqs, int32_t max_tokens, int32_t rows, int64_t max_keys, int32_t heads, int32_t kv_heads,
-                                          int32_t dim, int32_t vdim) {
+extern "C" int tlf_talk_attn_prefill_cuts(int32_t num_seqs, int32_t max_tokens, int32_t rows, int64_t reads, int64_t max_keys, int32_t heads,
+                                          int32_t kv_heads, int32_t dim, int32_t vdim) {
   const int tq = tlf_talk_attn_prefill_tile_rows(heads, kv_heads, dim, vdim);
-  return num_seqs > 0 && max_tokens > 0 && tq && tlf::talk_cuts_pay(num_seqs, max_tokens, rows, max_keys, tq);
+  return num_seqs > 0 && max_tokens > 0 && tq && tlf::talk_cuts_pay({num_seqs, max_tokens, rows, reads, max_keys}, tq);
+}
+
+extern "C" int tlf_talk_attn_prefill_route(int32_t singles, const int64_t *short_portions, const int64_t *long_portions, int32_t heads, int32_t kv_heads,
+                                           int32_t dim, int32_t vdim) {
+  using namespace tlf;
+  const int tq = tlf_talk_attn_prefill_tile_rows(heads, kv_heads, dim, vdim);
+  auto load = [](const int64_t *p) { return TalkLoad{p[0], p[1], p[2], p[3], p[4]}; };
+  return tq ? talk_route(singles > 0, load(short_portions), load(long_portions), heads, tq) : kTalkByRows;
 }
 
 extern "C" int tlf_talk_attn_prefill_cut(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables,

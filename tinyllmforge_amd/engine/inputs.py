@@ -106,6 +106,7 @@ def portion_inputs(seqs, block_size: int, long_portion: int | None = None, windo
     far = slice(single + short, None)
     keys = np.stack([np.minimum(start[far], w - 1) + n[far] for w in windows]) if windows else np.zeros((0, len(n[far])), np.int64)
     kv_offsets = np.concatenate([np.zeros((len(keys), 1), np.int64), np.cumsum(keys, axis=1)], axis=1)
+    reads, near = n * start + n * (n + 1) // 2, slice(single, single + short)
     chunks = -(-n[single:] // CHUNK)
     cu_chunks = np.concatenate([[0], np.cumsum(chunks)])
     chunk_seq = np.repeat(np.arange(len(chunks)), chunks)
@@ -118,6 +119,8 @@ def portion_inputs(seqs, block_size: int, long_portion: int | None = None, windo
         chunk_lens=np.minimum(CHUNK, n[single:][chunk_seq] - within).astype(np.int32),
         cu_chunks=cu_chunks.astype(np.int32), num_single=single, max_portion=int(n.max()),
         num_short=short, num_short_rows=int(cu[single + short]), max_short=int(n[single:single + short].max(initial=0)),
+        short_reads=int(reads[near].sum()), short_keys=int((start + n)[near].max(initial=0)),
+        long_reads=int(reads[far].sum()), long_keys=int((start + n)[far].max(initial=0)),
         kv_offsets=kv_offsets.astype(np.int32), kv_rows=tuple(kv_offsets[:, -1].tolist()),
         max_kv_rows=tuple(keys.max(axis=1, initial=0).tolist()),
     )

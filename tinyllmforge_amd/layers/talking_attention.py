@@ -9,15 +9,6 @@ from .. import ops
 from ..utils.context import get_context
 
 
-def short_in_tiles(portions: int, rows: int, keys: int) -> bool:
-    """Whether short portions, ``rows`` rows in all and contexts of up to ``keys``, go in row tiles: where they are few rows, row by row is faster.
-    A row tile starts with more latency, and its keys are read once for all its rows: a row costs what it reads, a tile about as much as one row and
-    all of them together as much as 40.  16 heads, the layer by rows and in tiles, us: portions behind 1024 keys, 8 of up to 8 tokens 57 and 67, 33 of 2
-    74 and 94, 16 of 4 63 and 75, one of 64 63 and 62, 8 of up to 16 93 and 67, 60 of up to 32 818 and 135; behind 2048, 33 of 2 121 and 149, 12 of 6
-    111 and 101, 100 of 2 326 and 310; behind 64, where either waits for the host, 33 of 2 41 and 37."""
-    return rows >= 64 and (keys <= 256 or rows >= 55 + 1.1 * portions)
-
-
 class TalkingHeadsAttention(nn.Module):
     def __init__(self, num_heads: int, num_kv_heads: int, dim: int, value_dim: int, scale: float, eps: float, dtype: torch.dtype,
                  rot_dims: int = 0, rope=None):
@@ -46,28 +37,31 @@ class TalkingHeadsAttention(nn.Module):
                           self.temp.data, self.cos_sin, self.rot_dims, self.eps, self.scale)
         out = torch.empty(n, self.num_heads * self.value_dim, dtype=self.dtype, device=q.device)
         tiles = self.dtype == torch.bfloat16 and ops.talk_prefill_supported(self.num_heads, self.num_kv_heads, self.dim, self.value_dim)
-        short = 0 if short_in_tiles(ctx.num_short, ctx.num_short_rows - ctx.num_single, ctx.block_tables.stride(0) * kv.k.shape[2]) else ctx.num_short
-        rows = (ctx.num_short_rows if short else ctx.num_single) if tiles else n
+        rows, calls = self._calls(n) if tiles else (n, ())
         if rows:
             ops.talk_attention_rows(q[:rows], kv, ctx.block_tables, positions[:rows], ctx.slot_mapping[:rows], self.talk.data, ctx.max_len,
                                     out[:rows], ctx.row_seq[:rows] if ctx.num_single < rows else None)
-        if rows < n:
-            first = ctx.num_single + short
-            portions = ctx.cu_seqlens_q.numel() - 1 - first
-            calls = [(first, portions, ctx.max_portion, n - rows)]
-            if 0 < ctx.num_short - short < portions and not self._together(portions, n - rows):
-                many, most = ctx.num_short, ctx.num_short_rows - rows
-                calls = [(first, many, ctx.max_short, most), (first + many, portions - many, ctx.max_portion, n - rows - most)]
-            for call in calls:
-                ops.talk_attention_prefill(q, kv, ctx.block_tables, ctx.cu_seqlens_q, ctx.seq_starts, *call[:3], self.talk.data, out, call[3])
+        for first, load in calls:
+            ops.talk_attention_prefill(q, kv, ctx.block_tables, ctx.cu_seqlens_q, ctx.seq_starts, first, *load[:2], self.talk.data, out, *load[2:])
         return out
 
-    def _together(self, portions: int, rows: int) -> bool:
-        """Whether short and long portions share a call, which has workgroups for the row tiles of the longest in every portion: while these
-        all fit the chip, or are cut, that is cheaper than two calls, the layer 65 us and 102 (16 heads, 3 of 300 tokens and 10 of 100).  Beyond
-        that the empty ones take their turn: one of 8000 tokens and 200 of 2 took 9690 us together, 863 apart, one of 200 and 30 of 20 behind 1024 keys 215
-        and 131, behind 64 63 and 89."""
+    def _calls(self, n: int):
+        """Rows of the step that run row by row, and the calls in row tiles: the first sequence of each, and its portions, their most tokens, rows,
+        reads and most keys.  The same for all layers of a step."""
         ctx = get_context()
-        most = -(-ctx.max_portion // ops.talk_tile_rows(self.num_heads, self.num_kv_heads, self.dim, self.value_dim)) * portions
-        keys = ctx.block_tables.stride(0) * self.kv.k.shape[2]
-        return most <= 192 or (most <= 512 and keys <= 512) or ops.talk_prefill_cuts(self.kv, ctx.block_tables, portions, ctx.max_portion, rows, self.num_heads)
+        single, near = ctx.num_single, ctx.num_short_rows if ctx.num_short else ctx.num_single
+        if single >= n or (near >= n and near - single < 64):
+            return n, ()                                             # few rows, where the host is waited for: not even asked
+        key = ("talk", self.num_heads, self.num_kv_heads, self.dim, self.value_dim, n)
+        if key not in ctx.plans:
+            first, seqs = single + ctx.num_short, ctx.cu_seqlens_q.numel() - 1
+            short = (ctx.num_short, ctx.max_short or ctx.max_portion, near - single, ctx.short_reads, ctx.short_keys)
+            long = (seqs - first, ctx.max_portion if seqs > first else 0, n - near, ctx.long_reads, ctx.long_keys)
+            if not ctx.short_reads + ctx.long_reads:                 # not told: as if contexts were half as long as the table
+                most = ctx.block_tables.stride(0) * self.kv.k.shape[2]
+                short, long = ((*v[:3], v[2] * most // 2, most) for v in (short, long))
+            route = ops.talk_prefill_route(self.kv, self.num_heads, single, short, long) if near - single >= 64 else 0
+            both = (short[0] + long[0], max(short[1], long[1]), short[2] + long[2], short[3] + long[3], max(short[4], long[4]))
+            calls = ([(first, long)], [(single, both)], [(single, short), (first, long)])[route]
+            ctx.plans[key] = near if route == 0 else single, [c for c in calls if c[1][0]]
+        return ctx.plans[key]

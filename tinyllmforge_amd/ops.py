@@ -7,6 +7,8 @@ enqueues the kernel on torch's current stream, so calls are capturable by
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -1237,18 +1239,23 @@ def talk_prefill_supported(heads, kv_heads, dim, vdim) -> bool:
     return bool(_lib.load().tlf_talk_attn_prefill_supported(heads, kv_heads, dim, vdim))
 
 
-def talk_tile_rows(heads, kv_heads, dim, vdim) -> int:
-    """Rows of a row tile of ``talk_attention_prefill``."""
-    return _lib.load().tlf_talk_attn_prefill_tile_rows(heads, kv_heads, dim, vdim)
+def talk_prefill_cuts(kv: SinkKV, block_tables, num_seqs, max_tokens, heads, rows=None, reads=0, keys=None) -> bool:
+    """Whether the keys of long row tiles are cut into parts.  Known or not: ``rows`` of all portions, ``reads``, the keys their rows see summed over
+    the rows, and the most ``keys`` of one."""
+    rows = num_seqs * max_tokens if rows is None else rows
+    keys = block_tables.stride(0) * kv.k.shape[2] if keys is None else keys
+    return bool(_lib.load().tlf_talk_attn_prefill_cuts(num_seqs, max_tokens, rows, reads, keys, heads, kv.k.shape[1], kv.dim, kv.vdim))
 
 
-def talk_prefill_cuts(kv: SinkKV, block_tables, num_seqs, max_tokens, rows, heads) -> bool:
-    """Whether the keys of long row tiles are cut into parts, for portions of up to ``max_tokens`` rows and ``rows`` in all."""
-    return bool(_lib.load().tlf_talk_attn_prefill_cuts(num_seqs, max_tokens, rows, block_tables.stride(0) * kv.k.shape[2], heads, kv.k.shape[1], kv.dim, kv.vdim))
+def talk_prefill_route(kv: SinkKV, heads, singles, short, long) -> int:
+    """``tlf_talk_attn_prefill_route`` for portions, most tokens, rows, reads and most keys of the short and the long ones."""
+    load = lambda v: (ctypes.c_int64 * 5)(*v)
+    return _lib.load().tlf_talk_attn_prefill_route(singles, load(short), load(long), heads, kv.k.shape[1], kv.dim, kv.vdim)
 
 
-def talk_attention_prefill(q, kv: SinkKV, block_tables, cu_seqlens_q, seq_starts, first_seq, num_seqs, max_tokens, talk, out, rows=None):
-    """Portions of sequences ``first_seq ..`` on the matrix cores (bf16), of ``rows`` rows in all where that is known; rows indexed as in the step."""
+def talk_attention_prefill(q, kv: SinkKV, block_tables, cu_seqlens_q, seq_starts, first_seq, num_seqs, max_tokens, talk, out, rows=None, reads=0, keys=None):
+    """Portions of sequences ``first_seq ..`` on the matrix cores (bf16), of ``rows`` rows with ``reads`` and ``keys`` as in ``talk_prefill_cuts``; rows
+    indexed as in the step."""
     _need(q, BF16, "q"); _need(talk, BF16, "talk"); _need(block_tables, torch.int32, "block_tables")
     n, heads, dp = q.shape
     pages, G, bs, _ = kv.k.shape
@@ -1259,7 +1266,7 @@ def talk_attention_prefill(q, kv: SinkKV, block_tables, cu_seqlens_q, seq_starts
     stats = torch.empty(n, heads, dtype=torch.float32, device=q.device)
     args = (q.data_ptr(), kv.k.data_ptr(), kv.v.data_ptr(), block_tables.data_ptr(), cols, cu_seqlens_q.data_ptr(), seq_starts.data_ptr(), first_seq, num_seqs,
             max_tokens, talk.data_ptr(), stats.data_ptr(), out.data_ptr(), out.stride(0), heads, G, kv.dim, kv.vdim, bs, pages)
-    if not talk_prefill_cuts(kv, block_tables, num_seqs, max_tokens, min(n, num_seqs * max_tokens) if rows is None else rows, heads):
+    if not talk_prefill_cuts(kv, block_tables, num_seqs, max_tokens, heads, min(n, num_seqs * max_tokens) if rows is None else rows, reads, keys):
         check(lib.tlf_talk_attn_prefill(*args, _stream()), "tlf_talk_attn_prefill")
         return out
     nbytes = lib.tlf_talk_attn_prefill_workspace_bytes(num_seqs, max_tokens, cols * bs, heads, G, kv.dim, kv.vdim)
