@@ -233,12 +233,12 @@ def test_short_and_long_portions():
     seqs = [seq_of(70, 69, 1, [4, 9]), seq_of(100, 60, 7, [7, 3]), seq_of(30, 0, 9, [5]), seq_of(200, 20, 40, [1, 2, 6, 8]), seq_of(64, 0, 64, [10])]
     d = I.portion_inputs(seqs, 64, long_portion=10, windows=(5, 30, 500))
     assert (d["num_single"], d["num_short"], d["num_short_rows"], d["max_short"], d["max_portion"]) == (1, 2, 17, 9, 64)
-    assert (d["short_reads"], d["short_keys"], d["long_reads"], d["long_keys"]) == (sum(range(61, 68)) + sum(range(10)), 67, sum(range(21, 61)) + sum(range(65)), 64)
+    assert d["portion_reads"] == (sum(range(61, 68)) + sum(range(10)), 67, sum(range(21, 61)) + sum(range(65)), 64)
     # keys from max(0, start - size + 1) to the portion's end
     assert d["kv_offsets"].tolist() == [[0, 44, 108], [0, 60, 124], [0, 60, 124]]
     assert d["kv_rows"] == (108, 124, 124) and d["max_kv_rows"] == (64, 64, 64)
     none = I.portion_inputs(seqs[:3], 64, long_portion=10, windows=(5,))
-    assert none["kv_rows"] == (0,) and none["max_kv_rows"] == (0,) and none["num_short"] == 2 and none["long_reads"] == none["long_keys"] == 0
+    assert none["kv_rows"] == (0,) and none["max_kv_rows"] == (0,) and none["num_short"] == 2 and none["portion_reads"][2:] == (0, 0)
     plain = I.portion_inputs(seqs, 64)
     assert plain["num_short"] == 0 and plain["num_short_rows"] == 1 and plain["kv_offsets"].shape == (0, 5)
     with pytest.raises(AssertionError):

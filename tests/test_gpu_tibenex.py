@@ -292,7 +292,7 @@ def layer_in_tiles_and_by_rows(lens, starts, monkeypatch, told=True):
         at += need[i]
     d = {k: torch.from_numpy(v).cuda() if hasattr(v, "dtype") else v for k, v in portion_inputs(seqs, 64, 128).items()}
     positions = d.pop("positions")
-    for name in ("input_ids",) + (() if told else ("max_short", "short_reads", "short_keys", "long_reads", "long_keys")):
+    for name in ("input_ids",) + (() if told else ("max_short", "portion_reads")):
         d.pop(name)
     most = max(a + n for a, n in zip(starts, lens))
     with torch.device("cuda"):

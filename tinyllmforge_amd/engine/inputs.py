@@ -119,8 +119,7 @@ def portion_inputs(seqs, block_size: int, long_portion: int | None = None, windo
         chunk_lens=np.minimum(CHUNK, n[single:][chunk_seq] - within).astype(np.int32),
         cu_chunks=cu_chunks.astype(np.int32), num_single=single, max_portion=int(n.max()),
         num_short=short, num_short_rows=int(cu[single + short]), max_short=int(n[single:single + short].max(initial=0)),
-        short_reads=int(reads[near].sum()), short_keys=int((start + n)[near].max(initial=0)),
-        long_reads=int(reads[far].sum()), long_keys=int((start + n)[far].max(initial=0)),
+        portion_reads=tuple(int(v) for at in (near, far) for v in (reads[at].sum(), (start + n)[at].max(initial=0))),
         kv_offsets=kv_offsets.astype(np.int32), kv_rows=tuple(kv_offsets[:, -1].tolist()),
         max_kv_rows=tuple(keys.max(axis=1, initial=0).tolist()),
     )

@@ -55,11 +55,12 @@ class TalkingHeadsAttention(nn.Module):
         key = ("talk", self.num_heads, self.num_kv_heads, self.dim, self.value_dim, n)
         if key not in ctx.plans:
             first, seqs = single + ctx.num_short, ctx.cu_seqlens_q.numel() - 1
-            short = (ctx.num_short, ctx.max_short or ctx.max_portion, near - single, ctx.short_reads, ctx.short_keys)
-            long = (seqs - first, ctx.max_portion if seqs > first else 0, n - near, ctx.long_reads, ctx.long_keys)
-            if not ctx.short_reads + ctx.long_reads:                 # not told: as if contexts were half as long as the table
-                most = ctx.block_tables.stride(0) * self.kv.k.shape[2]
-                short, long = ((*v[:3], v[2] * most // 2, most) for v in (short, long))
+            short = (ctx.num_short, ctx.max_short or ctx.max_portion, near - single)
+            long = (seqs - first, ctx.max_portion if seqs > first else 0, n - near)
+            reads, most = ctx.portion_reads, ctx.block_tables.stride(0) * self.kv.k.shape[2]
+            if reads is None:                                        # as if contexts were half as long as the table
+                reads = (short[2] * most // 2, most, long[2] * most // 2, most)
+            short, long = short + reads[:2], long + reads[2:]
             route = ops.talk_prefill_route(self.kv, self.num_heads, single, short, long) if near - single >= 64 else 0
             both = (short[0] + long[0], max(short[1], long[1]), short[2] + long[2], short[3] + long[3], max(short[4], long[4]))
             calls = ([(first, long)], [(single, both)], [(single, short), (first, long)])[route]
