@@ -1,5 +1,6 @@
 """Tibenex on the CPU: the plain implementation against closed forms, planted mistakes, configuration and checkpoint routing,
 tables, the host side of caches and state slots, and argument checks of the entry points."""
+import ctypes
 import copy
 import json
 import math
@@ -374,6 +375,9 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     assert cut() == WORK and cut(ws=a, nb=room() - 1) == WORK and cut(ldo=70) == SHAPE and cut(out=None) == NULL and cut(n=0) == 0
     pays = lambda n=1, most=5000, rows=5000, keys=5056, sizes=(16, 8, 128, 128): lib.tlf_talk_attn_prefill_cuts(n, most, rows, 0, keys, *sizes)
     assert pays() == 1 and pays(n=0) == 0 and pays(most=0) == 0 and pays(sizes=(33, 1, 64, 64)) == 0 and pays(n=24, most=250, rows=6000, keys=256) == 0
+    load = (ctypes.c_int64 * 10)(64, 4, 256, 256 * 1026, 1028)       # the second half: no long ones
+    route = lambda s=load, sizes=(16, 8, 128, 128): lib.tlf_talk_attn_prefill_route(0, s, ctypes.byref(load, 40), *sizes)
+    assert route() == 1 and route(s=None) == 0 and route(sizes=(33, 1, 64, 64)) == 0
     assert lib.tlf_talk_attn_prefill_tile_rows(16, 8, 128, 128) == 32 and lib.tlf_talk_attn_prefill_tile_rows(33, 1, 64, 64) == 0
     ok = lib.tlf_talk_attn_prefill_supported
     assert ok(32, 8, 128, 128) == 1 and ok(33, 1, 64, 64) == 0 and ok(4, 2, 129, 64) == 0 and ok(4, 2, 64, 129) == 0 and ok(1, 1, 1, 1) == 1

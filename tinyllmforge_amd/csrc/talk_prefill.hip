@@ -818,7 +818,7 @@ extern "C" int tlf_talk_attn_prefill_route(int32_t singles, const int64_t *short
   using namespace tlf;
   const int tq = tlf_talk_attn_prefill_tile_rows(heads, kv_heads, dim, vdim);
   auto load = [](const int64_t *p) { return TalkLoad{p[0], p[1], p[2], p[3], p[4]}; };
-  return tq ? talk_route(singles > 0, load(short_portions), load(long_portions), heads, tq) : kTalkByRows;
+  return tq && short_portions && long_portions ? talk_route(singles > 0, load(short_portions), load(long_portions), heads, tq) : kTalkByRows;
 }
 
 extern "C" int tlf_talk_attn_prefill_cut(const void *q, const void *k_cache, const void *v_cache, const int32_t *block_tables,
