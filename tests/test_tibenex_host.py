@@ -1,7 +1,7 @@
 """Tibenex on the CPU: the plain implementation against closed forms, planted mistakes, configuration and checkpoint routing,
 tables, the host side of caches and state slots, and argument checks of the entry points."""
-import ctypes
 import copy
+import ctypes
 import json
 import math
 
