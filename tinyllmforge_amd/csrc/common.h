@@ -75,35 +75,25 @@ __device__ __forceinline__ unsigned int pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(unsigned int, r);
 }
 
-// Two fp32 values as bf16 pairs, hi + lo: 16 significant bits.  For weights of attention: hi must be finite, since the other value's
-// hi enters each difference times zero.  v_dot2 takes the difference a - hi straight from the packed halves (exact: checked against
-// the subtraction over all exponents), four instructions where shifting and masking the halves takes six, and seven as the compiler
-// writes it.  The constant (-1, 0) has to come from a register: as the inline constant -1.0 the hardware reads (0, -1).
+// Two fp32 values as bf16 pairs, hi + lo: 16 significant bits.  For weights of attention: hi must be finite.  The differences a - hi are
+// exact.  v_dot2 would take them straight from the packed halves, two instructions fewer, but it waits for the matrix cores: a stream of
+// 16x16x32 products with one v_dot2 each takes 47 us where two shifts and subtractions in its place take 34 and nothing 33 (two waves
+// per SIMD, 1600 of each).  Without the empty asm the compiler rounds the two halves one by one.
 __device__ __forceinline__ void weight_pairs(float a, float b, unsigned int &hi, unsigned int &lo) {
-  typedef __bf16 pair __attribute__((ext_vector_type(2)));
-  unsigned int low;
-  asm("s_mov_b32 %0, 0xbf80" : "=s"(low));
   hi = pack_bf16x2(a, b);
-  const pair h = __builtin_bit_cast(pair, hi);
-  lo = pack_bf16x2(__builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, low), a, false),
-                   __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, 0xbf800000u), b, false));
+  asm("" : "+v"(hi));
+  lo = pack_bf16x2(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));
 }
 
 // Eight fp32 values as three bf16 pieces each: all 24 significant bits.
 __device__ __forceinline__ void bf16_pieces(const float (&v)[8], uint4 (&p)[3]) {
-  typedef __bf16 pair __attribute__((ext_vector_type(2)));
-  unsigned int low, w[3][4];
-  asm("s_mov_b32 %0, 0xbf80" : "=s"(low));       // (-1, 0), see weight_pairs
+  unsigned int w[3][4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    float a = v[2 * j], b = v[2 * j + 1];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      w[i][j] = pack_bf16x2(a, b);
-      const pair h = __builtin_bit_cast(pair, w[i][j]);
-      a = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, low), a, false);
-      b = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(pair, 0xbf800000u), b, false);
-    }
+    weight_pairs(v[2 * j], v[2 * j + 1], w[0][j], w[1][j]);
+    float a = v[2 * j] - __uint_as_float(w[0][j] << 16), b = v[2 * j + 1] - __uint_as_float(w[0][j] & 0xffff0000u);
+    asm("" : "+v"(w[1][j]));
+    w[2][j] = pack_bf16x2(a - __uint_as_float(w[1][j] << 16), b - __uint_as_float(w[1][j] & 0xffff0000u));
   }
 #pragma unroll
   for (int i = 0; i < 3; ++i) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
