@@ -84,6 +84,31 @@ def test_weights_follow_a_growing_maximum(dim, vdim, cap):
     torch.testing.assert_close(out.view(new, heads, vdim).double().cpu(), want, rtol=2 ** -8, atol=2 ** -10)
 
 
+@pytest.mark.parametrize("vdim,offset,gap", [(128, 0, 8), (128, 4, 8), (120, 0, 4), (72, 8, 0), (68, 4, 0), (33, 0, 0), (64, 1, 3)])
+def test_results_of_any_width_and_alignment(vdim, offset, gap):
+    """Results leave a unit's two lanes 16 bytes at a time, 8 or 2, whatever rows and their start allow; the bits are the same."""
+    torch.manual_seed(vdim)
+    dev, BF, n, heads, dim = "cuda", torch.bfloat16, 77, 6, 64
+    kv = ops.SinkKV(2, 64, 2, dim, vdim, BF, dev)
+    kv.k.normal_()
+    kv.v.normal_()
+    q, gate = torch.randn(n, heads, dim, device=dev).to(BF), torch.randn(n, heads * vdim, device=dev).to(BF)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=dev)
+    def run(offset, gap):
+        rows = torch.full((offset + n * (heads * vdim + gap),), 7.0, device=dev, dtype=BF)
+        out = rows[offset:].view(n, heads * vdim + gap)[:, :heads * vdim]
+        ops.sink_attention_prefill(q, kv, i32(1, 0).view(1, -1), i32(0, n), i32(0), 0, 1, n, None, gate, None, out)
+        kept = rows.clone()
+        kept[offset:].view(n, -1)[:, :heads * vdim] = 7.0
+        assert (kept == 7).all()
+        return out.clone()
+    got = run(offset, gap)
+    k, v = (t[[1, 0]].transpose(0, 1).flatten(1, 2)[:, :n].transpose(0, 1)[..., :w] for t, w in ((kv.k, dim), (kv.v, vdim)))
+    want = plain(q.float() * 0.6931471805599453, k, v) * torch.sigmoid(gate.float().cpu().view(n, heads, vdim))
+    torch.testing.assert_close(got.float().cpu().view(want.shape), want, rtol=2 ** -7, atol=2 ** -8)
+    assert torch.equal(got, run(1, 5))
+
+
 @pytest.mark.parametrize("lens", [(1,), (128,), (128, 5, 77), (100,) * 9, (129, 128, 3)], ids=str)
 @pytest.mark.parametrize("dim,rot,vdim", [(64, 32, 64), (128, 64, 128)])
 @pytest.mark.parametrize("heads", [3, 16])

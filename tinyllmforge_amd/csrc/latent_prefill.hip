@@ -2,14 +2,14 @@
 // latent_attn.h): row r of `expanded` holds the keys' own parts of all heads and then the values, the rotated key part
 // shared by the heads is read from the gathered cache rows.
 //
-// A workgroup owns one portion, one head and 64 CT query rows, 16 CT per wave, and walks the keys its window covers; the loop is
+// A workgroup owns one portion, one head and 128 query rows, 32 per wave, and walks the keys its window covers; the loop is
 // prompt_core.h's:
 //   P = 2^(S * scale - m)         fp32; m follows a row's maximum only when that has grown by more than 8 (a factor of 256,
 //                                 which the fp32 sums and the bf16 pair hold), so the accumulators are rarely rescaled.  Whether any
 //                                 has grown is asked lane by lane; maxima of rows are only formed when one has, and all rows of the wave
 //                                 follow theirs then: a largest weight of 1 is not rounded
 // 16 heads of 96 and 64 dimensions, eight prompts of 1061 to 2048 tokens: layer 189 us with the stages of a tile one after the other and
-// a window of 1024, 171 so; three prompts up to 3000, causal, 208 and 188.
+// a window of 1024, 171 with three stages side by side, 162 so; three waves per SIMD fit the registers (160 to 165 with two, 160 with three).
 #include "latent_attn.h"
 #include "prompt_core.h"
 #include "prompt_tiles.h"
@@ -74,42 +74,34 @@ __device__ __forceinline__ void latent_finish(const LatentPrefillArgs &p, const 
 
 // DC, VC: query / key and value dimensions in units of 32 (rounded up to what is instantiated)
 template <int DC, int VC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void latent_prefill_kernel(const LatentPrefillArgs p) {
-  constexpr int CT = 2;
-  using Core = PromptCore<DC, VC, CT>;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VC <= 5 ? 3 : 2))) void latent_prefill_kernel(const LatentPrefillArgs p) {
+  using Core = PromptCore<DC, VC>;
   __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
   int sq, h, xt;
   if (!latent_tile(p, sq, h, xt)) return;
   const LatentShape &s = p.s;
   const int seq = p.first_seq + sq;
   const int q0 = p.cu_q[seq], lq = p.cu_q[seq + 1] - q0, start = p.starts[seq];
-  const int row0 = xt * 64 * CT;
+  const int row0 = xt * 128;
   if (row0 >= lq) return;
   const int kv0 = p.kv_off[sq], kv_n = p.kv_off[sq + 1] - kv0;
   const int kbase = max(0, start - p.window + 1);            // position of the portion's first dense row
-  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
-  const int last_row = min(row0 + 64 * CT, lq) - 1;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+  const int last_row = min(row0 + 128, lq) - 1;
   const int i_first = start + row0, i_last = start + last_row;
   Core core;
   core.start(TLF_DL_LDSADDR(Ks), TLF_DL_LDSADDR(Vs), tid);
-  const int wave_first = i_first + core.wave * 16 * CT, wave_last = min(wave_first + 16 * CT - 1, i_last);
+  const int wave_first = i_first + core.wave * 32, wave_last = min(wave_first + 31, i_last);
 
-  int upos[CT];
-  bool uok[CT];
+  const int r = row0 + core.wave * 32 + n, row = min(r, last_row), upos = start + row;
+  const bool uok = r <= last_row;
+  const unsigned short *qp = p.q + (static_cast<int64_t>(q0 + row) * s.H + h) * s.Dq + g * 8;
 #pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    const int r = row0 + core.wave * 16 * CT + k * 16 + n;
-    uok[k] = r <= last_row;
-    const int row = uok[k] ? r : last_row;
-    upos[k] = start + row;
-    const unsigned short *qp = p.q + (static_cast<int64_t>(q0 + row) * s.H + h) * s.Dq + g * 8;
-#pragma unroll
-    for (int kc = 0; kc < DC; ++kc) {
-      Pack16 t;
-      t.u = kc * 32 < s.Dq ? *reinterpret_cast<const uint4 *>(qp + kc * 32) : make_uint4(0, 0, 0, 0);
-      t.u = make_uint4((t.u.x & p.q_keep) ^ p.q_flip, (t.u.y & p.q_keep) ^ p.q_flip, (t.u.z & p.q_keep) ^ p.q_flip, (t.u.w & p.q_keep) ^ p.q_flip);
-      core.qf[k][kc] = t.v;
-    }
+  for (int kc = 0; kc < 2 * DC; ++kc) {
+    Pack16 t;
+    t.u = kc * 16 < s.Dq ? *reinterpret_cast<const uint4 *>(qp + kc * 16) : make_uint4(0, 0, 0, 0);
+    t.u = make_uint4((t.u.x & p.q_keep) ^ p.q_flip, (t.u.y & p.q_keep) ^ p.q_flip, (t.u.z & p.q_keep) ^ p.q_flip, (t.u.w & p.q_keep) ^ p.q_flip);
+    core.qf[kc] = t.v;
   }
 
   // This lane's pieces of a tile's rows: their places in the row 0 of the portion's dense rows, their rows in the tile.  A piece of K
@@ -135,85 +127,60 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
   }
   const int w0 = max(0, i_first - p.window + 1);             // >= kbase
   const int tiles = (i_last - w0) / kPK + 1;
-  auto copy_k = [&](int t, auto) __attribute__((always_inline)) {
-    const int r0 = w0 - kbase + t * kPK;
+  auto copy = [&](int t, auto) __attribute__((always_inline)) {
+    const int r0 = w0 - kbase + t * kPK;                     // its own row is below kv_n
 #pragma unroll
     for (int i = 0; i < DC; ++i)
       prompt_copy_at(kat[i] + static_cast<uint64_t>(kstep[i]) * static_cast<unsigned int>(min(r0 + krow[i], kv_n - 1)), core.k_place(t, i));
-  };
-  auto copy_v = [&](int t, auto) __attribute__((always_inline)) {
-    const int r0 = w0 - kbase + t * kPK;                     // its own row is below kv_n
     const unsigned short *base = own + static_cast<int64_t>(r0) * p.lde + s.H * s.Da + h * s.Va;
 #pragma unroll
     for (int i = 0; i < VC; ++i)
       prompt_copy(ostep * static_cast<unsigned int>(min(vrow[i], kv_n - 1 - r0)) + vat[i], base, core.v_place(t, i));
   };
 
-  float m[CT], l[CT];
-  float x[CT];                                               // this lane's largest score of the half that comes next,
-  float over[CT];                                            // and what it must not exceed
-#pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    m[k] = over[k] = -INFINITY;                              // no key yet
-    l[k] = 0.f;
-  }
+  float m = -INFINITY, l = 0.f;                              // no key yet
   // tiles between the window's edge and the diagonal hide nothing from any of the wave's rows
   const int to = max(0, wave_last - w0) / kPK + 1;
   const int edge = wave_last - p.window >= w0 ? (wave_last - p.window - w0) / kPK + 1 : 0;
-  core.template walk<true, true, true>(
-      tiles, min(max(0, wave_first - p.window + 1 - w0) / kPK, to - 1), to, edge, min(tiles, max(0, (wave_first + 1 - w0) / kPK)), copy_k, copy_v,
-      [](float (&f)[CT]) __attribute__((always_inline)) {
+  core.template walk<true, true>(
+      tiles, min(max(0, wave_first - p.window + 1 - w0) / kPK, to - 1), to, edge, min(tiles, max(0, (wave_first + 1 - w0) / kPK)), copy,
+      []() __attribute__((always_inline)) { return Core::all(0.f); },
+      [&](int t, int hf, typename Core::Scores &sc, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
+        if (part.mask) {
+          const int seen = upos - (w0 + t * kPK + hf * 32 + g * 8), hidden = seen - p.window;
 #pragma unroll
-        for (int k = 0; k < CT; ++k) f[k] = 0.f;
-      },
-      [&](int hf, typename Core::Scores &sc, auto part) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < CT; ++k) {
-          if (part.mask) {
-            const int key = w0 + hf * 32 + g * 8;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              const bool seen = key + j <= upos[k] && (!part.lead || key + j > upos[k] - p.window);
-              sc[j >> 2][k][j & 3] = seen ? sc[j >> 2][k][j & 3] : -INFINITY;
-            }
+          for (int j = 0; j < 16; ++j) {
+            const int at = (j & 8) * 2 + (j & 7);
+            sc[j] = at <= seen && (!part.lead || at > hidden) ? sc[j] : -INFINITY;
           }
-          float y = sc[0][k][0];
-#pragma unroll
-          for (int j = 1; j < 8; ++j) y = fmaxf(y, sc[j >> 2][k][j & 3]);
-          y *= p.scale_log2;
-          x[k] = part.start && (hf & 1) ? fmaxf(x[k], y) : y;     // the first maximum is that of the whole first tile
         }
-      },
-      [&](int hf, typename Core::Scores &, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
-        bool grown = false;
-#pragma unroll
-        for (int k = 0; k < CT; ++k) grown = grown || x[k] > over[k];
-        if (!__any(grown)) return;
-        if (!part.start) core.add_values(hf - 1, w);
-#pragma unroll
-        for (int k = 0; k < CT; ++k) {                       // sums and accumulators to the new maximum
-          const float most = fmaxf(m[k], max_lanes_16_32_48(x[k]));
-          const float back = most == m[k] ? 1.f : __builtin_amdgcn_exp2f(m[k] - most);
-          m[k] = most;
-          over[k] = m[k] + 8.f;
-          l[k] *= back;
-#pragma unroll
-          for (int d = 0; d < 2 * VC; ++d) core.acc[k][d] *= back;
+        const float x = Core::largest(sc) * p.scale_log2;
+        if (__any(x > m + 8.f)) {                            // sums and accumulators to the new maximum
+          const float most = fmaxf(m, prompt_unit_max(x));
+          const float back = most == m ? 1.f : __builtin_amdgcn_exp2f(m - most);
+          m = most;
+          l *= back;
+          core.rescale(back);
         }
-      },
-      [&](int hf, const typename Core::Scores &sc, typename Core::Weights &w, auto) __attribute__((always_inline)) {
+        const float ms = m == -INFINITY ? 0.f : m;
+        float e[16];
 #pragma unroll
-        for (int k = 0; k < CT; ++k) {
-          const float ms = m[k] == -INFINITY ? 0.f : m[k];
-          float e[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) e[j] = __builtin_amdgcn_exp2f(sc[j >> 2][k][j & 3] * p.scale_log2 - ms);
-          l[k] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
-          Core::split(k, e, w);
-        }
+        for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(sc[j] * p.scale_log2 - ms);
+        l += Core::sum(e);
+        Core::split(e, w);
       });
 
-  latent_finish<VC, CT>(p, core.acc, l, uok, upos, q0, start, h, g);
+  const float den = prompt_unit_sum(l);
+  if (!uok) return;
+  float inv = 1.0f / den;                                    // a row sees itself: den > 0
+  if (p.gate) inv *= p.gate[static_cast<int64_t>(q0 + row) * s.H + h];
+  unsigned short *o = p.out + static_cast<int64_t>(q0 + row) * p.ldo + static_cast<int64_t>(h) * s.vdim;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(p.out);
+  core.store(o, s.vdim, (s.vdim & 3) == 0 && (p.ldo & 3) == 0 && (at & 7) == 0, (s.vdim & 7) == 0 && (p.ldo & 7) == 0 && (at & 15) == 0, g,
+             [&](int, float (&f)[4]) __attribute__((always_inline)) {
+#pragma unroll
+               for (int i = 0; i < 4; ++i) f[i] *= inv;
+             });
 }
 
 __device__ __forceinline__ int prefill_tile_row(int t) { return (t & 32) | ((t & 4) << 2) | ((t & 24) >> 1) | (t & 3); }

@@ -2,12 +2,12 @@
 // pooled_attn.h).
 //
 // A workgroup owns one sequence, one KV head and a tile of query rows; the (row, head) pairs of the KV head's query
-// heads are flattened into 64 CT units, 16 CT per wave.  It walks the pooled rows its last query sees and then the
+// heads are flattened into 128 units, 32 per wave (64 and 16 beyond 128 dimensions).  It walks the pooled rows its last query sees and then the
 // tokens from its first query's window on; the loop is prompt_core.h's:
 //   P = sigmoid(S * scale + bias)  fp32, masked on the pooled tiles and on those that a window's or the diagonal's edge cuts
 // The weights are not normalised: no maximum, no rescaling, no second pass.  Bound by the vector ALU: two quarter-rate operations
 // per score.  Eight prompts of 1061 to 2048 tokens, 32 heads of 128 on 8 KV heads, window 1024: layer 372 us with the stages of a tile
-// one after the other (and the staging registers, which the compiler had put in LDS), 299 so.
+// one after the other (and the staging registers, which the compiler had put in LDS), 296 with three stages side by side, 286 so.
 #include "pooled_attn.h"
 #include "prompt_core.h"
 #include "prompt_tiles.h"
@@ -65,8 +65,7 @@ __device__ __forceinline__ void pooled_finish(const PooledPrefillArgs &p, const 
 
 template <int DC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void pooled_prefill_kernel(const PooledPrefillArgs p) {
-  constexpr int CT = 2;
-  using Core = PromptCore<DC, DC, CT>;
+  using Core = PromptCore<DC, DC>;
   __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
   int sq, plane, xt;
   if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
@@ -76,7 +75,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   const int row0 = xt * p.bq;
   if (row0 >= lq) return;
   const int32_t *bt = c.bt + seq * c.bt_stride;
-  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
   const int nh = min(p.hpp, p.group - pass * p.hpp);         // heads of this pass
   const int last_row = min(row0 + p.bq, lq) - 1;
   const int i_first = start + row0, i_last = start + last_row;
@@ -84,29 +83,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   Core core;
   core.start(TLF_DL_LDSADDR(Ks), TLF_DL_LDSADDR(Vs), tid);
 
-  int upos[CT], unb[CT], uoff[CT];
-  bool uok[CT];
-  float pb[CT];
-  #pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    const int u = core.wave * CT * 16 + k * 16 + n;
-    const int r = row0 + u / p.hpp, hh = u % p.hpp;
-    uok[k] = u < p.bq * p.hpp && r <= last_row && hh < nh;
-    const int head = kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0);
-    const int row = uok[k] ? r : row0;
-    upos[k] = start + row;
-    unb[k] = pooled_visible(upos[k], c.size, c.pool);
-    uoff[k] = (q0 + row) * p.H + head;
-    pb[k] = -kLog2e * bf16_bits_to_float(p.bias[head]);
-    const unsigned short *qp = p.q + static_cast<int64_t>(uoff[k]) * Core::DP + g * 8;
+  const int u = core.wave * 32 + n, r = row0 + u / p.hpp, hh = u % p.hpp;
+  const bool uok = u < p.bq * p.hpp && r <= last_row && hh < nh;
+  const int head = kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0), row = uok ? r : row0;
+  const int upos = start + row, unb = pooled_visible(upos, c.size, c.pool);
+  const int64_t unit = static_cast<int64_t>(q0 + row) * p.H + head;
+  const float pb = -kLog2e * bf16_bits_to_float(p.bias[head]), nscale = -p.scale_log2;
+  const unsigned short *qp = p.q + unit * Core::DP + g * 8;
 #pragma unroll
-    for (int kc = 0; kc < DC; ++kc) {
-      Pack16 t;
-      t.u = *reinterpret_cast<const uint4 *>(qp + kc * 32);
-      core.qf[k][kc] = t.v;
-    }
+  for (int kc = 0; kc < 2 * DC; ++kc) {
+    Pack16 t;
+    t.u = *reinterpret_cast<const uint4 *>(qp + kc * 16);
+    core.qf[kc] = t.v;
   }
-  const float nscale = -p.scale_log2;
 
   const int nb = pooled_visible(i_last, c.size, c.pool);
   const int ptiles = (nb + kTK - 1) / kTK;
@@ -121,65 +110,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   unsigned int koff[DC], voff[DC];                           // this lane's pieces in a tile of tokens
 #pragma unroll
   for (int i = 0; i < DC; ++i) {
-    int row, piece;
-    core.k_piece(i, lane, row, piece);
-    koff[i] = static_cast<unsigned int>(row * static_cast<int>(rs) * 2 + piece * 16);
-    core.v_piece(i, lane, row, piece);
-    voff[i] = static_cast<unsigned int>(row * static_cast<int>(rs) * 2 + piece * 16);
+    int at, piece;
+    core.k_piece(i, lane, at, piece);
+    koff[i] = static_cast<unsigned int>(at * static_cast<int>(rs) * 2 + piece * 16);
+    core.v_piece(i, lane, at, piece);
+    voff[i] = static_cast<unsigned int>(at * static_cast<int>(rs) * 2 + piece * 16);
   }
-  auto copy_k = [&](int t, auto part) __attribute__((always_inline)) {
+  auto copy = [&](int t, auto part) __attribute__((always_inline)) {
     if (part.lead && t < ptiles) {                           // rows of one page's blocks, then the next page's
 #pragma unroll
       for (int i = 0; i < DC; ++i) {
-        int row, piece;
-        core.k_piece(i, lane, row, piece);
-        prompt_copy_at(pk_ + block_row(c, bt, min(t * kTK + row, nb - 1)) * rs + piece * 8, core.k_place(t, i));
+        int at, piece;
+        core.k_piece(i, lane, at, piece);
+        prompt_copy_at(pk_ + block_row(c, bt, min(t * kTK + at, nb - 1)) * rs + piece * 8, core.k_place(t, i));
+        core.v_piece(i, lane, at, piece);
+        prompt_copy_at(pv_ + block_row(c, bt, min(t * kTK + at, nb - 1)) * rs + piece * 8, core.v_place(t, i));
       }
       return;
     }
     // 64 tokens from a multiple of 64 on lie in one page; rows past the last query are masked
-    const unsigned short *base = kc_ + token_row(c, bt, w0 + (t - ptiles) * kTK) * rs;
+    const int64_t from = token_row(c, bt, w0 + (t - ptiles) * kTK) * rs;
 #pragma unroll
-    for (int i = 0; i < DC; ++i) prompt_copy(koff[i], base, core.k_place(t, i));
-  };
-  auto copy_v = [&](int t, auto part) __attribute__((always_inline)) {
-    if (part.lead && t < ptiles) {
+    for (int i = 0; i < DC; ++i) prompt_copy(koff[i], kc_ + from, core.k_place(t, i));
 #pragma unroll
-      for (int i = 0; i < DC; ++i) {
-        int row, piece;
-        core.v_piece(i, lane, row, piece);
-        prompt_copy_at(pv_ + block_row(c, bt, min(t * kTK + row, nb - 1)) * rs + piece * 8, core.v_place(t, i));
-      }
-      return;
-    }
-    const unsigned short *base = vc_ + token_row(c, bt, w0 + (t - ptiles) * kTK) * rs;
-#pragma unroll
-    for (int i = 0; i < DC; ++i) prompt_copy(voff[i], base, core.v_place(t, i));
+    for (int i = 0; i < DC; ++i) prompt_copy(voff[i], vc_ + from, core.v_place(t, i));
   };
   // tiles between the window's edge and the diagonal hide nothing from anyone
   const int edge = i_last - c.size >= w0 ? (i_last - c.size - w0) / kTK + 1 : 0;
-  core.template walk<true, false, false>(
-      tiles, 0, tiles, ptiles + edge, min(tiles, ptiles + max(0, (i_first + 1 - w0) / kTK)),
-      copy_k, copy_v,
-      [](float (&f)[CT]) __attribute__((always_inline)) { f[0] = f[1] = 0.f; }, [](int, typename Core::Scores &, auto) __attribute__((always_inline)) {},
-      [](int, typename Core::Scores &, typename Core::Weights &, auto) __attribute__((always_inline)) {},
-      [&](int h, const typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
+  core.template walk<true, false>(
+      tiles, 0, tiles, ptiles + edge, min(tiles, ptiles + max(0, (i_first + 1 - w0) / kTK)), copy, []() __attribute__((always_inline)) { return Core::all(0.f); },
+      [&](int t, int hf, const typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
+        float e[16];
 #pragma unroll
-        for (int k = 0; k < CT; ++k) {
-          float e[8];
+        for (int j = 0; j < 16; ++j) e[j] = sigmoid_neg_log2(fmaf(s[j], nscale, pb));
+        if (part.mask) {
+          const bool pooled = part.lead && t < ptiles;       // workgroup uniform
+          const int key = t * kTK + hf * 32 + (pooled ? 0 : w0 - ptiles * kTK) + g * 8;
+          const int lo = part.lead && !pooled ? upos - c.size + 1 : 0, hi = (pooled ? unb : upos + 1) - key;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) e[j] = sigmoid_neg_log2(fmaf(s[j >> 2][k][j & 3], nscale, pb[k]));
-          if (part.mask) {
-            const bool pooled = part.lead && h / 2 < ptiles;  // workgroup uniform
-            const int key = h * 32 + (pooled ? 0 : w0 - ptiles * kTK) + g * 8;
-            const int lo = pooled ? 0 : upos[k] - c.size + 1, hi = pooled ? unb[k] : upos[k] + 1;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) e[j] = key + j >= lo && key + j < hi ? e[j] : 0.f;
+          for (int j = 0; j < 16; ++j) {
+            const int at = (j & 8) * 2 + (j & 7);
+            e[j] = at < hi && (!part.lead || at >= lo - key) ? e[j] : 0.f;
           }
-          Core::split(k, e, w);
         }
+        Core::split(e, w);
       });
-  pooled_finish<DC, CT>(p, core.acc, uok, uoff, g);
+
+  if (!uok) return;
+  const float gt = p.gate[unit];
+  unsigned short *o = p.out + static_cast<int64_t>(q0 + row) * p.ldo + static_cast<int64_t>(head) * c.D;
+  const uintptr_t to = reinterpret_cast<uintptr_t>(p.out);
+  core.store(o, c.D, (c.D & 3) == 0 && (p.ldo & 3) == 0 && (to & 7) == 0, (c.D & 7) == 0 && (p.ldo & 7) == 0 && (to & 15) == 0, g,
+             [&](int, float (&f)[4]) __attribute__((always_inline)) {
+#pragma unroll
+               for (int x = 0; x < 4; ++x) f[x] *= gt;
+             });
 }
 
 // Heads beyond 128: the stages of a tile one after the other, staged through registers, one tile in LDS at a time.

@@ -1,7 +1,7 @@
 // Attention of sink_attn.h for prompt portions, bf16, on the matrix cores, from the paged cache.
 //
 // A workgroup owns one portion, one KV head and a tile of query rows; the (row, head) pairs of the KV head's query heads are
-// flattened into 64 CT units, 16 CT per wave.  The loop is prompt_core.h's; a tile of 64 keys is one contiguous piece of a page.
+// flattened into 128 units, 32 per wave (64 and 16 beyond 128 dimensions).  The loop is prompt_core.h's; a tile of 64 keys is one contiguous piece of a page.
 //   P = 2^(score - m)   fp32; m follows a unit's maximum only when that has grown by more than 8 (a factor of 256, which the fp32
 //                       sums and the bf16 pair hold), so the accumulators are rarely rescaled.  Without a cap the scores begin at -m,
 //                       and whether any has grown is asked lane by lane; maxima of units are only formed when one has
@@ -84,8 +84,7 @@ __device__ __forceinline__ void sink_finish(const SinkPrefillArgs &p, const floa
 // MODE 0: no cap, 1: a cap, 2: a cap small enough to take the largest score it allows as everyone's maximum
 template <int DC, int VC, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void sink_prefill_kernel(const SinkPrefillArgs p) {
-  constexpr int CT = 2;
-  using Core = PromptCore<DC, VC, CT>;
+  using Core = PromptCore<DC, VC>;
   __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
   int sq, plane, xt;
   if (!prompt_tile(p.tiles, prompt_block(blockIdx.x, blockIdx.y), sq, plane, xt)) return;
@@ -95,135 +94,119 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   const int row0 = xt * p.bq;
   if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
   const int32_t *bt = c.bt + seq * c.bt_stride;
-  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
   const int nh = min(p.hpp, p.group - pass * p.hpp);         // heads of this pass
   const int last_row = min(row0 + p.bq, lq) - 1;
   const int i_last = start + last_row;
   Core core;
   core.start(TLF_DL_LDSADDR(Ks), TLF_DL_LDSADDR(Vs), tid);
-  const int wave_first = start + row0 + core.wave * CT * 16 / p.hpp;
-  const int wave_last = min(start + row0 + ((core.wave + 1) * CT * 16 - 1) / p.hpp, i_last);
+  const int wave_first = start + row0 + core.wave * 32 / p.hpp;
+  const int wave_last = min(start + row0 + ((core.wave + 1) * 32 - 1) / p.hpp, i_last);
 
-  int upos[CT], urow[CT], uhead[CT];
-  bool uok[CT];
+  const int u = core.wave * 32 + n, r = row0 + u / p.hpp, hh = u % p.hpp;
+  const bool uok = u < p.bq * p.hpp && r <= last_row && hh < nh;
+  const int uhead = kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0), row = min(r, last_row), upos = start + row, urow = q0 + row;
+  const unsigned short *qp = p.q + (static_cast<int64_t>(urow) * p.H + uhead) * Core::DP + g * 8;
 #pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    const int u = core.wave * CT * 16 + k * 16 + n;
-    const int r = row0 + u / p.hpp, hh = u % p.hpp;
-    uok[k] = u < p.bq * p.hpp && r <= last_row && hh < nh;
-    uhead[k] = kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0);
-    const int row = min(r, last_row);
-    upos[k] = start + row;
-    urow[k] = q0 + row;
-    const unsigned short *qp = p.q + (static_cast<int64_t>(urow[k]) * p.H + uhead[k]) * Core::DP + g * 8;
-#pragma unroll
-    for (int kc = 0; kc < DC; ++kc) {
-      Pack16 t;
-      t.u = *reinterpret_cast<const uint4 *>(qp + kc * 32);
-      core.qf[k][kc] = t.v;
-    }
+  for (int kc = 0; kc < 2 * DC; ++kc) {
+    Pack16 t;
+    t.u = *reinterpret_cast<const uint4 *>(qp + kc * 16);
+    core.qf[kc] = t.v;
   }
 
   const int tiles = i_last / kSK + 1;
   unsigned int koff[DC], voff[VC];                           // this lane's pieces in a tile, which is one piece of a page
 #pragma unroll
   for (int i = 0; i < DC; ++i) {
-    int row, piece;
-    core.k_piece(i, lane, row, piece);
-    koff[i] = (row * Core::KCH + piece) * 16;
+    int at, piece;
+    core.k_piece(i, lane, at, piece);
+    koff[i] = (at * Core::KCH + piece) * 16;
   }
 #pragma unroll
   for (int i = 0; i < VC; ++i) {
-    int row, piece;
-    core.v_piece(i, lane, row, piece);
-    voff[i] = (row * (c.Vp / 8) + (piece < c.Vp / 8 ? piece : 0)) * 16;
+    int at, piece;
+    core.v_piece(i, lane, at, piece);
+    voff[i] = (at * (c.Vp / 8) + (piece < c.Vp / 8 ? piece : 0)) * 16;
   }
-  // K of a tile is asked for first, its V a tile later from the row carried over; the page is looked up another tile ahead
+  // the page is looked up a tile ahead
   auto page_of = [&](int t) __attribute__((always_inline)) { return bt[sink_page_of(c, min(t * kSK, i_last))]; };
-  int64_t row_k = 0;
   int page_next = page_of(0);
-  auto copy_k = [&](int t, auto) __attribute__((always_inline)) {  // rows past the last query are masked
-    row_k = sink_row(c, page_next, sink_page_of(c, t * kSK), kvh, t * kSK);
+  auto copy = [&](int t, auto) __attribute__((always_inline)) {    // rows past the last query are masked
+    const int64_t at = sink_row(c, page_next, sink_page_of(c, t * kSK), kvh, t * kSK);
     page_next = page_of(t + 1);
-    const unsigned char *kp = static_cast<const unsigned char *>(c.k) + row_k * (Core::DP * 2);
+    const unsigned char *kp = static_cast<const unsigned char *>(c.k) + at * (Core::DP * 2), *vp = static_cast<const unsigned char *>(c.v) + at * (c.Vp * 2);
 #pragma unroll
     for (int i = 0; i < DC; ++i) prompt_copy(koff[i], kp, core.k_place(t, i));
-  };
-  auto copy_v = [&](int t, auto) __attribute__((always_inline)) {  // before the next copy_k: of the tile that was asked for last
-    const unsigned char *vp = static_cast<const unsigned char *>(c.v) + row_k * (c.Vp * 2);
 #pragma unroll
     for (int i = 0; i < VC; ++i) prompt_copy(voff[i], vp, core.v_place(t, i));
   };
 
-  float m[CT], l[CT];
-  float x[CT];                                               // this lane's largest score of the half that comes next,
-  float over[CT];                                            // and what it must not exceed
+  float m = MODE == 2 ? p.cap_log2 : -INFINITY, l = 0.f;
+  float over = -INFINITY;                                    // what a score must not exceed; no key yet
+  typename Core::Scores from = Core::all(0.f);               // without a cap: the score less the maximum so far
+  core.template walk<false, true>(
+      tiles, 0, wave_last / kSK + 1, 0, min(tiles, (wave_first + 1) / kSK), copy,                      // the diagonal cuts the tiles behind
+      [&]() __attribute__((always_inline)) { return from; },
+      [&](int t, int hf, typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
 #pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    m[k] = MODE == 2 ? p.cap_log2 : -INFINITY;
-    l[k] = 0.f;
-    over[k] = -INFINITY;                                     // no key yet
-  }
-  core.template walk<false, true, false>(
-      tiles, 0, wave_last / kSK + 1, 0, min(tiles, (wave_first + 1) / kSK), copy_k, copy_v,            // the diagonal cuts the tiles behind
-      [&](float (&f)[CT]) __attribute__((always_inline)) {   // without a cap: the score less the maximum so far
-#pragma unroll
-        for (int k = 0; k < CT; ++k) f[k] = MODE == 0 && m[k] != -INFINITY ? -m[k] : 0.f;
-      },
-      [&](int h, typename Core::Scores &s, auto part) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < CT; ++k) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            float v = s[j >> 2][k][j & 3];
-            if (MODE == 2) v = -2.f * p.cap_log2 * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(v));
-            if (MODE == 1) v = sink_score_log2<true>(v, p.cap_log2);
-            if (part.mask) v = h * 32 + g * 8 + j <= upos[k] ? v : -INFINITY;
-            s[j >> 2][k][j & 3] = v;
-          }
-          if (MODE != 2) {
-            x[k] = s[0][k][0];
-#pragma unroll
-            for (int j = 1; j < 8; ++j) x[k] = fmaxf(x[k], s[j >> 2][k][j & 3]);
-          }
+        for (int j = 0; j < 16; ++j) {
+          if (MODE == 2) s[j] = -2.f * p.cap_log2 * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[j]));
+          if (MODE == 1) s[j] = sink_score_log2<true>(s[j], p.cap_log2);
         }
-      },
-      [&](int h, typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
+        if (part.mask) {
+          const int seen = upos - (t * kSK + hf * 32 + g * 8);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) s[j] = (j & 8) * 2 + (j & 7) <= seen ? s[j] : -INFINITY;
+        }
         if constexpr (MODE != 2) {
-          bool grown = false;
-#pragma unroll
-          for (int k = 0; k < CT; ++k) grown = grown || x[k] > over[k];
-          if (!__any(grown)) return;
-          if (!part.start) core.add_values(h - 1, w);
-#pragma unroll
-          for (int k = 0; k < CT; ++k) {                     // sums, accumulators and scores to the new maximum
-            const float most = max_lanes_16_32_48(x[k]), base = MODE == 0 && m[k] != -INFINITY ? m[k] : 0.f;
-            const bool up = most > over[k];
-            const float top = up ? base + most : m[k], back = up ? __builtin_amdgcn_exp2f(m[k] - top) : 1.f;
-            l[k] *= back;
-#pragma unroll
-            for (int d = 0; d < 2 * VC; ++d) core.acc[k][d] *= back;
-            if (MODE == 0 && up) {
-              s[0][k] -= floatx4{most, most, most, most};
-              s[1][k] -= floatx4{most, most, most, most};
-            }
-            m[k] = top;
-            over[k] = top == -INFINITY ? top : MODE == 0 ? 8.f : top + 8.f;
+          const float x = Core::largest(s);
+          if (__any(x > over)) {                             // sums, accumulators and scores to the new maximum
+            const float most = prompt_unit_max(x), base = MODE == 0 && m != -INFINITY ? m : 0.f;
+            const bool up = most > over;
+            const float top = up ? base + most : m, back = up ? __builtin_amdgcn_exp2f(m - top) : 1.f;
+            l *= back;
+            core.rescale(back);
+            if (MODE == 0) s -= up ? most : 0.f;
+            m = top;
+            if (MODE == 0) from = Core::all(top == -INFINITY ? 0.f : -top);
+            over = top == -INFINITY ? top : MODE == 0 ? 8.f : top + 8.f;
           }
         }
-      },
-      [&](int h, const typename Core::Scores &s, typename Core::Weights &w, auto) __attribute__((always_inline)) {
+        const float ms = MODE == 1 && m != -INFINITY ? m : 0.f;
+        float e[16];
 #pragma unroll
-        for (int k = 0; k < CT; ++k) {
-          const float ms = MODE == 1 && m[k] != -INFINITY ? m[k] : 0.f;
-          float e[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) e[j] = __builtin_amdgcn_exp2f(MODE == 1 ? s[j >> 2][k][j & 3] - ms : s[j >> 2][k][j & 3]);
-          l[k] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
-          Core::split(k, e, w);
-        }
+        for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(MODE == 1 ? s[j] - ms : s[j]);
+        l += Core::sum(e);
+        Core::split(e, w);
       });
-  sink_finish<VC, CT>(p, core.acc, m, l, uok, urow, uhead, g);
+
+  const float den = prompt_unit_sum(l);
+  if (!uok) return;
+  const float sk = p.sink ? bf16_bits_to_float(p.sink[uhead]) * kSinkLog2e : -INFINITY;
+  const float top = fmaxf(m, sk), f = __builtin_amdgcn_exp2f(m - top);
+  const float inv = f / (den * f + __builtin_amdgcn_exp2f(sk - top));
+  unsigned short *o = p.out + static_cast<int64_t>(urow) * p.ldo + static_cast<int64_t>(uhead) * c.Dv;
+  const unsigned short *gp = p.gate + static_cast<int64_t>(urow) * p.ldg + static_cast<int64_t>(uhead) * c.Dv;
+  const uintptr_t to = reinterpret_cast<uintptr_t>(p.out);
+  const bool vec = (c.Dv & 3) == 0 && (p.ldo & 3) == 0 && (p.ldg & 3) == 0 && (to & 7) == 0 && (reinterpret_cast<uintptr_t>(p.gate) & 7) == 0;
+  core.store(o, c.Dv, vec, vec && (c.Dv & 7) == 0 && (p.ldo & 7) == 0 && (to & 15) == 0, g, [&](int col, float (&x)[4]) __attribute__((always_inline)) {
+    float gt[4] = {1.f, 1.f, 1.f, 1.f};
+    if (p.gate) {
+      if (vec && col < c.Dv) {
+        const uint2 b = *reinterpret_cast<const uint2 *>(gp + col);
+        gt[0] = __uint_as_float(b.x << 16); gt[1] = __uint_as_float(b.x & 0xffff0000u);
+        gt[2] = __uint_as_float(b.y << 16); gt[3] = __uint_as_float(b.y & 0xffff0000u);
+      } else if (!vec) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col + r < c.Dv) gt[r] = bf16_bits_to_float(gp[col + r]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gt[r] = sigmoid_fast(gt[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = x[r] * inv * gt[r];
+  });
 }
 
 // Heads beyond 128: the stages of a tile one after the other, a tile staged through registers, one in LDS at a time (two of these
