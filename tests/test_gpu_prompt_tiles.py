@@ -206,6 +206,29 @@ def test_latent_maxima_follow_where_one_of_the_wave_grows():
     assert (out.view(n, heads, vdim).cpu() != want.to(BF)).double().mean().item() < 2 ** -14
 
 
+@pytest.mark.parametrize("heads,dim,rot,rank", [(16, 64, 32, 256), (32, 128, 64, 512), (3, 24, 8, 64), (5, 40, 24, 1000), (1, 32, 32, 8)])
+@pytest.mark.parametrize("n", [1025, 1030, 2051])
+def test_latent_rows_of_prompts_are_prepared_as_few_are(heads, dim, rot, rank, n):
+    """Beyond 1024 rows of the plain form two tokens go to a workgroup; up to there, and of other forms, latents and queries have workgroups
+    of their own.  Rows without a slot or a position among them, columns between queries and latents; the bits are the same."""
+    torch.manual_seed(n + rank)
+    dev, BF = "cuda", torch.bfloat16
+    s, col = ops.LatentShape(heads, dim, rot, rank, 16), heads * (dim + rot) + 16
+    proj, norm = torch.randn(n, col + rank + rot + 8, device=dev).to(BF), torch.randn(rank, device=dev).to(BF)
+    angles = torch.rand(512, rot // 2, device=dev) * 6.3
+    table = torch.cat([angles.cos(), angles.sin()], 1)
+    positions, slots = torch.randint(0, 512, (n,), device=dev), torch.randperm(64 * 40, device=dev)[:n].to(torch.int32)
+    positions[::97], positions[5::101], slots[3::53], slots[7::59] = -1, 512, -1, 64 * 40
+    def run(parts):
+        cache, q = torch.full((40, 64, s.lp), 7.0, device=dev, dtype=BF), []
+        for a in range(0, n, parts):
+            at = slice(a, min(n, a + parts))
+            q.append(ops.latent_prep(proj[at], col, norm, positions[at], table, slots[at], cache, s, 1e-6))
+        return torch.cat(q), cache
+    (q, cache), (q0, cache0) = run(n), run(1024)
+    assert torch.equal(q, q0) and torch.equal(cache, cache0)
+
+
 def test_more_workgroups_than_a_dimension_of_a_launch_holds():
     """The longest portion is the caller's bound: 2000 short ones under a bound of 300000 tokens are 12.5 million workgroups."""
     torch.manual_seed(0)

@@ -249,6 +249,125 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const LatentPrepArgs a
   }
 }
 
+// The same for rows of prompts of the plain form: bf16, parts in whole granules, queries without pads, pairs of neighbours, no query latents
+// and gates.  A workgroup has TOK tokens.  All it needs is on its way before the first of it is used: a granule of the queries is read where it is
+// written, four of them a thread (all at work whatever the row's size), then a wave reads a token's latent and rotated key; positions come by the
+// scalar path, and only granules that turn are unpacked.
+//
+// Bound by HBM: 12237 rows of 16 heads of 64 + 32 and latents of 256, 90 MB, took 35 us with latents and queries in workgroups of their own and
+// cosines asked for behind the row, 17 so; 28 with four tokens and 256 threads.  4000 rows 13.5 -> 7.5, of 32 heads of 128 + 64 and 512 34 -> 18.5;
+// 1000 rows 5.8 -> 6.2 and 10.2 -> 10.4, 24 rows 4.0 -> 4.5 and 4.0 -> 8.3, so few rows stay above.
+template <int TOK>
+__global__ __launch_bounds__(TOK * 64) void latent_prep_rows_kernel(const LatentPrepArgs a) {
+  typedef unsigned short T;
+  constexpr int kThreads = TOK * 64, kItems = 4, kKeep = 2;
+  const LatentShape &s = a.s;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nch = s.Dq / 8, own = s.dim / 8, half = s.rot / 2, per = s.H * nch;
+  const int tok0 = blockIdx.x * TOK, count = min(TOK, a.n - tok0);
+  const T *const proj = static_cast<const T *>(a.proj) + static_cast<int64_t>(tok0) * a.ld;
+  T *const q = static_cast<T *>(a.q_out) + static_cast<int64_t>(tok0) * s.H * s.Dq;
+  int at[TOK];                                               // row of cosines, negative: none
+#pragma unroll
+  for (int k = 0; k < TOK; ++k) {
+    const int64_t pos = a.positions[tok0 + min(k, count - 1)];
+    at[k] = pos >= 0 && pos < a.max_pos ? static_cast<int>(pos) : -1;
+  }
+  auto row_of = [&](int k) __attribute__((always_inline)) {
+    int r = at[0];
+#pragma unroll
+    for (int i = 1; i < TOK; ++i) r = k == i ? at[i] : r;
+    return r;
+  };
+  auto turn = [&](uint4 &u, const float4 &c, const float4 &sn) __attribute__((always_inline)) {
+    float f[8];
+    unpack8(u, f);
+    const float cs[4] = {c.x, c.y, c.z, c.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const float x = f[e], y = f[e + 1];
+      f[e] = __fmul_rn(x, cs[e / 2]) - __fmul_rn(y, ss[e / 2]);
+      f[e + 1] = __fmul_rn(y, cs[e / 2]) + __fmul_rn(x, ss[e / 2]);
+    }
+    u = pack8(f);
+  };
+
+  // a wave's token: granules `lane` and `lane + 64` of latent and rotated key
+  const int wt = min(wave, count - 1), lch = s.rank / 8, all = lch + s.rot / 8;
+  const int64_t slot = a.slots[tok0 + wt];
+  const int lat = row_of(wt);
+  uint4 l[kKeep], ln[kKeep];
+  float4 lc[kKeep], ls[kKeep];
+#pragma unroll
+  for (int k = 0; k < kKeep; ++k) {
+    const int d = lane + k * 64;
+    l[k] = ln[k] = make_uint4(0, 0, 0, 0);
+    if (d < all) l[k] = *reinterpret_cast<const uint4 *>(proj + wt * a.ld + a.off + d * 8);
+    if (d < lch) {
+      ln[k] = *reinterpret_cast<const uint4 *>(static_cast<const T *>(a.norm) + d * 8);
+    } else if (d < all && lat >= 0) {
+      const float *cs = a.cos_sin + static_cast<int64_t>(lat) * s.rot + (d - lch) * 4;
+      lc[k] = *reinterpret_cast<const float4 *>(cs);
+      ls[k] = *reinterpret_cast<const float4 *>(cs + half);
+    }
+  }
+  auto queries = [&](int first, auto between) __attribute__((always_inline)) {
+    uint4 u[kItems];
+    float4 c[kItems], sn[kItems];
+    bool turned[kItems];
+    int to[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const int item = first + i * kThreads + tid, k = item / per, ch = item - k * per, d = ch % nch - own;
+      to[i] = k < count ? item * 8 : -1;
+      const int row = row_of(k);
+      turned[i] = to[i] >= 0 && d >= 0 && row >= 0;
+      if (to[i] >= 0) u[i] = *reinterpret_cast<const uint4 *>(proj + k * a.ld + ch * 8);
+      if (turned[i]) {
+        const float *cs = a.cos_sin + static_cast<int64_t>(row) * s.rot + d * 4;
+        c[i] = *reinterpret_cast<const float4 *>(cs);
+        sn[i] = *reinterpret_cast<const float4 *>(cs + half);
+      }
+    }
+    between();
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      if (turned[i]) turn(u[i], c[i], sn[i]);
+      if (to[i] >= 0) *reinterpret_cast<uint4 *>(q + to[i]) = u[i];
+    }
+  };
+  queries(0, [&]() __attribute__((always_inline)) {
+    if (wave >= count || slot < 0 || slot >= a.num_slots) return;
+    T *row = static_cast<T *>(a.cache) + slot * s.Lp;
+    float f[kKeep][8], ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < kKeep; ++k) {
+      unpack8(l[k], f[k]);
+      if (lane + k * 64 < lch) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(f[k][e], f[k][e], ss);
+      }
+    }
+    ss = wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / static_cast<float>(s.rank) + a.eps);
+#pragma unroll
+    for (int k = 0; k < kKeep; ++k) {
+      const int d = lane + k * 64;
+      if (d < lch) {
+        float w[8];
+        unpack8(ln[k], w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[k][e] = f[k][e] * inv * w[e];
+        l[k] = pack8(f[k]);
+      } else if (d < all && lat >= 0) {
+        turn(l[k], lc[k], ls[k]);
+      }
+      if (d * 8 < s.Lp) *reinterpret_cast<uint4 *>(row + d * 8) = l[k];
+    }
+    for (int d = lane + kKeep * 64; d * 8 < s.Lp; d += 64) *reinterpret_cast<uint4 *>(row + d * 8) = make_uint4(0, 0, 0, 0);
+  });
+  for (int first = kItems * kThreads; first < count * per; first += kItems * kThreads) queries(first, []() __attribute__((always_inline)) {});
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // y[row, h, n] = sum_k W[h, n, k] x[row, h, k].  Rows n < n_main have weights in k < k_main only.
 struct HeadGemmArgs {
@@ -564,6 +683,11 @@ extern "C" int tlf_latent_prep(const void *proj, int64_t proj_stride, const floa
   a.norm8 = rank % 8 == 0 && aligned16(norm_weight);
   a.fours = rot_dim % 8 == 0 && aligned16(cos_sin);
   const int tok = splits <= 1 && n > 1024 ? 4 : 1;
+  if (tok == 4 && dtype == TLF_DT_BF16 && a.vec && a.norm8 && a.fours && q_out && cache && !halves && !cq_norm && !gate_out && a.s.Dq == dim + rot_dim &&
+      rank + rot_dim <= 1024) {
+    TLF_LAUNCH((latent_prep_rows_kernel<2>), dim3((n + 1) / 2), dim3(128), 0, static_cast<hipStream_t>(stream), a);
+    return launch_status();
+  }
   const dim3 grid((n + tok - 1) / tok, a.latents + (cq_norm ? 1 : 0) + (q_out ? (heads * (a.s.Dq / 8) + 255) / 256 : 0));
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define TLF_PREP(T, PART)                                                                        \
