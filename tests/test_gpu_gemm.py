@@ -106,6 +106,16 @@ def test_w8a16_full_size_exact_on_integer_data(M, N, K):
     assert (got.float().abs().max() > 0.05)               # not a vacuous comparison
 
 
+@pytest.mark.parametrize("M,N,K", [(8193, 2064, 64), (8320, 2048, 256), (4130, 4112, 320), (2190, 8208, 1024), (2190, 8208, 1088)])
+def test_bf16_many_rows_of_a_short_k_exact_on_integer_data(M, N, K):
+    """Products of up to 1024 columns, and the next ones, by many rows: whole and cut tiles on both sides, exact in any order."""
+    from tinyllmforge_amd import ops as P
+    x = torch.randint(-4, 5, (M, K), generator=g(M), dtype=torch.int32).to(BF).to(DEV)
+    w = torch.randint(-16, 17, (N, K), generator=g(N + K), dtype=torch.int32).to(BF).to(DEV)
+    got = P.bf16_linear(x, w)
+    assert torch.equal(got.view(torch.int16), (x.double() @ w.double().t()).to(BF).view(torch.int16))
+
+
 # BASELINE configs[2], every cell: M in {1, 16, 64, 256, 2048} x the four Qwen3-8B projection shapes.  The planner
 # is a threshold tree in M, N and K, so the cells the benchmark times are checked here one by one, not through
 # neighbours.
