@@ -403,6 +403,23 @@ int tlf_paged_decode_attn_planned(const void *q, int64_t q_stride,
                                   int64_t num_cache_blocks, float scale,
                                   void *workspace, size_t workspace_bytes, const void *plan, void *stream);
 
+/* a3 for few sequences (build-defined; up to 4 or 8 of them, heads of 128, 1, 2, 4 or 8 query heads per KV head, block_size % 16 == 0:
+ * tlf_decode_few_supported), spread over more workgroups than a sequence's bytes would need.  With q_norm_weight, x holds
+ * rows of the qkv projection [q heads | k heads | v heads]: the call does what tlf_qknorm_rope_store does for them too
+ * (models/qwen3.py:79-94, layers/attention.py:94-95) and the same bits go to the caches; no sequence of the call may read
+ * another one's new row.  Without it (NULL; the arguments up to slot_mapping are not read) x
+ * holds prepared queries and the caches every token.  Either way the results are the same bit for bit.  Empty sequences get zeros.
+ * The workspace (16-byte aligned) holds partial results. */
+int tlf_decode_few_supported(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size);
+size_t tlf_decode_few_workspace_bytes(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads);
+int tlf_decode_few(const void *x, int64_t x_stride, const void *q_norm_weight, const void *k_norm_weight, float eps,
+                   const int64_t *positions, const float *cos_sin, int32_t max_pos, const int32_t *slot_mapping,
+                   void *k_cache, void *v_cache, int32_t kv_dtype, const float *k_scale, const float *v_scale,
+                   const int32_t *block_tables, int64_t block_table_stride, const int32_t *context_lens, void *out,
+                   int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                   int32_t max_blocks, int64_t num_cache_blocks, float scale,
+                   void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---------------------------------------------------------------------------
  * a4  varlen causal prefill attention   replaces the prefill branch
  *     layers/attention.py:96-105 (flash_attn_varlen_func, causal=True)

@@ -1,0 +1,101 @@
+"""Decode attention of a few sequences: shares of all lengths against fp64, and the projection's rows against its separate kernels."""
+import pytest
+import torch
+
+from tinyllmforge_amd import ops
+
+pytestmark = pytest.mark.gpu
+BF, DEV = torch.bfloat16, "cuda"
+EPS, SCALE = 1e-6, 128 ** -0.5
+
+
+def step(ctxs, hq, hkv, bs, fp8, seed=0):
+    """Caches that hold all but the newest tokens, tables with scattered pages, the newest tokens' projection."""
+    g = torch.Generator().manual_seed(seed)
+    need = [max(1, -(-c // bs)) for c in ctxs]
+    pages = torch.randperm(sum(need) + 3, generator=g).tolist()
+    bt = torch.full((len(ctxs), max(need) + 1), -1, dtype=torch.int32)
+    for b, n in enumerate(need):
+        bt[b, :n] = torch.tensor([pages.pop() for _ in range(n)])
+    cache = lambda: torch.randn(sum(need) + 3, bs, hkv, 128, generator=g).to(BF)
+    k, v = cache(), cache()
+    scales = (None, None)
+    if fp8:
+        scales = torch.rand(hkv, generator=g) * 0.02 + 0.01, torch.rand(hkv, generator=g) * 0.02 + 0.01
+        k, v = ((t.float() / s[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn) for t, s in zip((k, v), scales))
+        scales = tuple(s.to(DEV) for s in scales)
+    slots = torch.tensor([bt[b, (c - 1) // bs] * bs + (c - 1) % bs if c else -1 for b, c in enumerate(ctxs)], dtype=torch.int32)
+    qkv = torch.randn(len(ctxs), (hq + 2 * hkv) * 128, generator=g).to(BF)
+    w = [(1 + 0.1 * torch.randn(128, generator=g)).to(BF).to(DEV) for _ in range(2)]
+    angles = torch.rand(9000, 64, generator=g) * 6.3
+    table = torch.cat([angles.cos(), angles.sin()], 1).to(DEV)
+    return (qkv.to(DEV), k.to(DEV), v.to(DEV), torch.tensor(ctxs, dtype=torch.int32, device=DEV), bt.to(DEV), scales, slots.to(DEV), w, table,
+            torch.tensor(ctxs, device=DEV))
+
+
+def exact(q, k, v, ctxs, bt, hq, hkv, scales):
+    q, k, v = q.double().view(len(ctxs), hq, 128), k.double(), v.double()
+    if scales[0] is not None:
+        k, v = k * scales[0].double()[:, None], v * scales[1].double()[:, None]
+    out = torch.zeros_like(q)
+    for b, c in enumerate(ctxs):
+        if c == 0:
+            continue
+        at = torch.arange(c, device=DEV)
+        page = bt[b].long()[at // k.shape[1]]
+        rows = [torch.where((page >= 0)[:, None, None], t[page.clamp(min=0), at % k.shape[1]], 0.0).repeat_interleave(hq // hkv, 1) for t in (k, v)]
+        w = torch.softmax(torch.einsum("hd,jhd->hj", q[b], rows[0]) * SCALE, -1)
+        out[b] = torch.einsum("hj,jhd->hd", w, rows[1])
+    return out.flatten(1)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hkv,bs,ctxs", [
+    (32, 8, 256, [700]), (32, 8, 16, [1, 64, 65, 0]), (32, 8, 256, [8000]), (16, 8, 256, [15, 16, 17, 63, 129, 1024, 1025, 2047]),
+    (8, 8, 64, [4096, 1, 1000]), (64, 8, 256, [64, 3000]), (16, 2, 48, [1, 2, 500, 66]), (2, 2, 32, [4097]), (16, 16, 256, [300, 4095, 64, 65])])
+def test_projection_rows_against_separate_kernels_and_fp64(hq, hkv, bs, ctxs, fp8):
+    n = len(ctxs)
+    assert ops.decode_few_supported(n, hq, hkv, 128, bs)
+    qkv, k, v, ctx, bt, scales, slots, w, table, positions = step(ctxs, hq, hkv, bs, fp8)
+    k2, v2 = k.clone(), v.clone()
+    got = ops.decode_few(qkv, hq, k, v, ctx, bt, SCALE, *scales, (*w, EPS, positions, table, slots))
+    q, _, _ = ops.qknorm_rope_store(qkv, *w, EPS, positions, table, hq, hkv, 128, k2, v2, slots, *scales)
+    bits = lambda t: t.view(torch.uint8)
+    assert torch.equal(bits(k), bits(k2)) and torch.equal(bits(v), bits(v2))
+    assert torch.equal(got, ops.decode_few(q, hq, k2, v2, ctx, bt, SCALE, *scales))
+    want = exact(q, k2, v2, ctxs, bt, hq, hkv, scales)
+    # fp32 scores of up to 2^3 (off by 2^-20), weights and sums: the result is off by 2^-17 of the values' size; then half a bf16 ulp
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2 ** -13)
+
+
+def test_rows_that_are_not_the_newest_token_come_from_the_cache():
+    """Without a slot position context_len - 1 is read from the cache, with an earlier row's slot that row is the new one; an
+    unmapped page reads as zeros; positions without cosines leave a head as normed."""
+    ctxs, hq, hkv, bs = [70, 300, 128, 65], 8, 4, 64
+    qkv, k, v, ctx, bt, scales, slots, w, table, positions = step(ctxs, hq, hkv, bs, False)
+    slots[0], slots[1] = -1, k.shape[0] * bs
+    slots[2] = bt[2, 0] * bs + 5
+    bt[3, 0] = -1
+    positions[3] = 9000
+    k2, v2 = k.clone(), v.clone()
+    got = ops.decode_few(qkv, hq, k, v, ctx, bt, SCALE, None, None, (*w, EPS, positions, table, slots))
+    q, _, _ = ops.qknorm_rope_store(qkv, *w, EPS, positions, table, hq, hkv, 128, k2, v2, slots)
+    assert torch.equal(k, k2) and torch.equal(v, v2)
+    assert torch.equal(got, ops.decode_few(q, hq, k2, v2, ctx, bt, SCALE))
+    torch.testing.assert_close(got.double(), exact(q, k2, v2, ctxs, bt, hq, hkv, (None, None)), rtol=2 ** -8, atol=2 ** -13)
+
+
+def test_replayed_with_other_lengths():
+    """A captured step follows the lengths and tables it finds."""
+    qkv, k, v, ctx, bt, _, slots, w, table, positions = step([4000, 90], 32, 8, 256, False)
+    args = lambda: (qkv, 32, k, v, ctx, bt, SCALE, None, None, (*w, EPS, positions, table, slots))
+    ops.decode_few(*args())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.decode_few(*args())
+    for lens in ([4000, 90], [65, 0], [1, 4000], [64, 700]):
+        ctx.copy_(torch.tensor(lens))
+        slots.copy_(torch.tensor([bt[b, (c - 1) // 256] * 256 + (c - 1) % 256 if c and bt[b, (c - 1) // 256] >= 0 else -1 for b, c in enumerate(lens)]))
+        graph.replay()
+        replayed = out.clone()
+        assert torch.equal(replayed, ops.decode_few(*args())), lens

@@ -34,6 +34,7 @@ FLAGS = [
 EXTRA_FLAGS = {
     "prefill_attn.hip": ["-fno-honor-nans"],
     "decode_attn.hip": ["-fno-honor-nans"],
+    "decode_few.hip": ["-fno-honor-nans"],
     "latent_prefill.hip": ["-fno-honor-nans"],
     "pooled_prefill.hip": ["-fno-honor-nans"],
     "sink_prefill.hip": ["-fno-honor-nans"],

@@ -71,8 +71,65 @@ __device__ __forceinline__ QkPieceTable qk_piece_table(const QkPieceMeta &m, int
   return t;
 }
 
-// raw = this lane's 8 bf16 values of token tok, head `head` (q heads first, then k, then v); all 16 lanes of
-// a head call together.
+// raw = this lane's 8 bf16 values of a head; all 16 lanes of it call together.  `normed`: a q or k head, which is normed with
+// weights `weight` and rotated; a v head stays as it is.
+__device__ __forceinline__ uint4 qk_piece_value(const uint4 raw, bool normed, const unsigned short *weight, int j, const QkPieceMeta &m,
+                                                const QkPieceTable &t, const QkRopeStoreArgs &a) {
+  constexpr int kDh = 128;
+  if (!normed) return raw;
+  float v[8];
+  unpack8(raw, v);
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
+  // sum over the head's 16 lanes: rotations by 8, 4, 2, 1 inside the row add the same pairs, in the same
+  // order, as a butterfly over lane ^ 8, 4, 2, 1 would (after each step the partial sums repeat with that
+  // period), so every lane of the head ends with the same bits
+  ss += row_ror<8>(ss);
+  ss += row_ror<4>(ss);
+  ss += row_ror<2>(ss);
+  ss += row_ror<1>(ss);
+  const float inv = 1.0f / sqrtf(ss / static_cast<float>(kDh) + a.eps);
+  float w[8];
+  unpack8(*reinterpret_cast<const uint4 *>(weight + j * 8), w);
+  float nrm[8], other[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float nn = bf16_bits_to_float(float_to_bf16_bits(__fmul_rn(v[i], inv)));
+    nrm[i] = bf16_bits_to_float(float_to_bf16_bits(__fmul_rn(nn, w[i])));
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) other[i] = row_ror<8>(nrm[i]);   // lane j ^ 8
+  const bool pos_ok = m.pos >= 0 && m.pos < a.max_pos;
+  const float cosv[8] = {t.c0.x, t.c0.y, t.c0.z, t.c0.w, t.c1.x, t.c1.y, t.c1.z, t.c1.w};
+  const float sinv[8] = {t.s0.x, t.s0.y, t.s0.z, t.s0.w, t.s1.x, t.s1.y, t.s1.z, t.s1.w};
+  float o[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    // lanes j < 8: cos*x1 - sin*x2 ; lanes j >= 8: cos*x2 + sin*x1
+    const float x = __fmul_rn(cosv[i], nrm[i]);
+    const float y = __fmul_rn(sinv[i], other[i]);
+    o[i] = (j < 8) ? __fsub_rn(x, y) : __fadd_rn(x, y);
+    if (!pos_ok) o[i] = nrm[i];
+  }
+  return pack8(o);
+}
+
+// Eight bf16 values as e4m3 values of scale s.
+__device__ __forceinline__ int2 qk_piece_e4m3(const uint4 v, float s) {
+  float f[8];
+  unpack8(v, f);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) f[i] = fminf(fmaxf(f[i] / s, -448.0f), 448.0f);
+  int lo = 0, hi = 0;
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], lo, false);
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
+  return make_int2(lo, hi);
+}
+
+// The piece of token tok, head `head` (q heads first, then k, then v).
 __device__ __forceinline__ void qk_piece_finish(const uint4 raw, int64_t tok, int head, int j, const QkPieceMeta &m,
                                                 const QkPieceTable &t, const QkRopeStoreArgs &a) {
   constexpr int kDh = 128;
@@ -81,45 +138,7 @@ __device__ __forceinline__ void qk_piece_finish(const uint4 raw, int64_t tok, in
   const bool is_k = !is_q && head < num_q_heads + num_kv_heads;
   const int kvh = is_q ? 0 : (is_k ? head - num_q_heads : head - num_q_heads - num_kv_heads);
   const int64_t slot = m.slot;
-  uint4 outp = raw;
-  if (is_q || is_k) {
-    float v[8];
-    unpack8(raw, v);
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
-    // sum over the head's 16 lanes: rotations by 8, 4, 2, 1 inside the row add the same pairs, in the same
-    // order, as a butterfly over lane ^ 8, 4, 2, 1 would (after each step the partial sums repeat with that
-    // period), so every lane of the head ends with the same bits
-    ss += row_ror<8>(ss);
-    ss += row_ror<4>(ss);
-    ss += row_ror<2>(ss);
-    ss += row_ror<1>(ss);
-    const float inv = 1.0f / sqrtf(ss / static_cast<float>(kDh) + a.eps);
-    float w[8];
-    unpack8(*reinterpret_cast<const uint4 *>((is_q ? a.qw : a.kw) + j * 8), w);
-    float nrm[8], other[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float nn = bf16_bits_to_float(float_to_bf16_bits(__fmul_rn(v[i], inv)));
-      nrm[i] = bf16_bits_to_float(float_to_bf16_bits(__fmul_rn(nn, w[i])));
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) other[i] = row_ror<8>(nrm[i]);   // lane j ^ 8
-    const bool pos_ok = m.pos >= 0 && m.pos < a.max_pos;
-    const float cosv[8] = {t.c0.x, t.c0.y, t.c0.z, t.c0.w, t.c1.x, t.c1.y, t.c1.z, t.c1.w};
-    const float sinv[8] = {t.s0.x, t.s0.y, t.s0.z, t.s0.w, t.s1.x, t.s1.y, t.s1.z, t.s1.w};
-    float o[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      // lanes j < 8: cos*x1 - sin*x2 ; lanes j >= 8: cos*x2 + sin*x1
-      const float x = __fmul_rn(cosv[i], nrm[i]);
-      const float y = __fmul_rn(sinv[i], other[i]);
-      o[i] = (j < 8) ? __fsub_rn(x, y) : __fadd_rn(x, y);
-      if (!pos_ok) o[i] = nrm[i];
-    }
-    outp = pack8(o);
-  }
+  const uint4 outp = qk_piece_value(raw, is_q || is_k, is_q ? a.qw : a.kw, j, m, t, a);
   if (is_q) {
     *reinterpret_cast<uint4 *>(a.q_out + tok * static_cast<int64_t>(num_q_heads) * kDh + head * kDh + j * 8) = outp;
     return;
@@ -129,21 +148,10 @@ __device__ __forceinline__ void qk_piece_finish(const uint4 raw, int64_t tok, in
   if (lin != nullptr) *reinterpret_cast<uint4 *>(lin + tok * row_elems + kvh * kDh + j * 8) = outp;
   if (slot < 0) return;
   unsigned char *cache = is_k ? a.k_cache : a.v_cache;
-  if (a.kv_dtype == TLF_KV_BF16) {
+  if (a.kv_dtype == TLF_KV_BF16)
     *reinterpret_cast<uint4 *>(cache + (slot * row_elems + kvh * kDh + j * 8) * 2) = outp;
-  } else {
-    float f[8];
-    unpack8(outp, f);
-    const float s = (is_k ? a.k_scale : a.v_scale)[kvh];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = fminf(fmaxf(f[i] / s, -448.0f), 448.0f);
-    int lo = 0, hi = 0;
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], lo, false);
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
-    *reinterpret_cast<int2 *>(cache + slot * row_elems + kvh * kDh + j * 8) = make_int2(lo, hi);
-  }
+  else
+    *reinterpret_cast<int2 *>(cache + slot * row_elems + kvh * kDh + j * 8) = qk_piece_e4m3(outp, (is_k ? a.k_scale : a.v_scale)[kvh]);
 }
 
 // The three steps on one piece.

@@ -24,6 +24,16 @@ class Attention(nn.Module):
     def has_cache(self) -> bool:
         return self.k_cache.numel() > 0 and self.v_cache.numel() > 0
 
+    def few(self, rows: int) -> bool:
+        """Whether a decode step over ``rows`` sequences takes ``ops.decode_few``."""
+        return self.has_cache() and ops.decode_few_supported(rows, self.num_heads, self.num_kv_heads, self.head_dim, self.k_cache.shape[1])
+
+    def forward_projected(self, qkv: torch.Tensor, q_norm, k_norm, positions: torch.Tensor, cos_sin: torch.Tensor):
+        """A decode step of a few sequences from the rows of the qkv projection: q / k norm, RoPE, cache write and attention."""
+        ctx = get_context()
+        return ops.decode_few(qkv, self.num_heads, self.k_cache, self.v_cache, ctx.context_lens, ctx.block_tables, self.scale, self.k_scale,
+                              self.v_scale, (q_norm.weight.data, k_norm.weight.data, q_norm.eps, positions, cos_sin, ctx.slot_mapping))
+
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv_stored: bool = False):
         """``q [N, Hq*Dh]``, ``k``/``v`` ``[N, Hkv*Dh]`` -> ``[N, Hq*Dh]``.
 
@@ -43,5 +53,8 @@ class Attention(nn.Module):
             return ops.varlen_prefill_attention(q, k.view(-1, self.num_kv_heads, self.head_dim),
                                                 v.view(-1, self.num_kv_heads, self.head_dim),
                                                 ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.max_seqlen_q, self.scale)
+        if self.few(q.shape[0]):
+            return ops.decode_few(q.flatten(1), self.num_heads, self.k_cache, self.v_cache, ctx.context_lens, ctx.block_tables, self.scale,
+                                  self.k_scale, self.v_scale)
         return ops.paged_decode_attention(q, self.k_cache, self.v_cache, ctx.context_lens, ctx.block_tables,
                                           self.scale, self.k_scale, self.v_scale, plan=ctx.decode_plan)

@@ -45,15 +45,19 @@ class QWen3Attention(nn.Module):
             ctx = get_context()
             attn = self.attn
             has_cache = attn.has_cache()
-            # prefill without a prefix hit attends over this step's own K/V rows
-            want_kv = ctx.is_prefill and ctx.block_tables is None
-            # projection, q/k norm, RoPE and cache store in one call (one kernel fewer when the projection's
-            # plan splits K across workgroups, which is the rule at decode sizes)
-            q, k, v = self.qkv_proj.forward_qknorm_rope_store(
-                hidden_states, self.q_norm, self.k_norm, positions, self.rotary_emb.cos_sin_cache,
-                attn.k_cache if has_cache else None, attn.v_cache if has_cache else None,
-                ctx.slot_mapping if has_cache else None, attn.k_scale, attn.v_scale, want_kv)
-            o = attn(q, k, v, kv_stored=True)
+            if not ctx.is_prefill and has_cache and attn.few(hidden_states.shape[0]):
+                # a few decoding sequences: what lies between the projection and the attention is part of the latter
+                o = attn.forward_projected(self.qkv_proj(hidden_states), self.q_norm, self.k_norm, positions, self.rotary_emb.cos_sin_cache)
+            else:
+                # prefill without a prefix hit attends over this step's own K/V rows
+                want_kv = ctx.is_prefill and ctx.block_tables is None
+                # projection, q/k norm, RoPE and cache store in one call (one kernel fewer when the projection's
+                # plan splits K across workgroups, which is the rule at decode sizes)
+                q, k, v = self.qkv_proj.forward_qknorm_rope_store(
+                    hidden_states, self.q_norm, self.k_norm, positions, self.rotary_emb.cos_sin_cache,
+                    attn.k_cache if has_cache else None, attn.v_cache if has_cache else None,
+                    ctx.slot_mapping if has_cache else None, attn.k_scale, attn.v_scale, want_kv)
+                o = attn(q, k, v, kv_stored=True)
         else:
             qkv = self.qkv_proj(hidden_states)
             q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
