@@ -22,9 +22,11 @@
 // segments 59 + 18 + 255 us, so 58 + 15 + 209; 12 of 450 to 900 48 + 24 + 216, and in one pass over whole ones 204.
 //
 // Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256, medians under the profiler: chunk 122 + scan 470 (both
-// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 149 + first pass 61 + chaining 15 + scan
-// 210 us (whole layer 614 and 390 us).  The blocks write 55 KB a record, 4 TB/s with what they read; the scan is held by its
-// barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's error against 64 bits is 5e-8 to 1.1e-7 on both, the
+// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 115 - 135 + first pass 61 + chaining 15 + scan
+// 210 us (whole layer 614 and 377 us).  The blocks write 55 KB a record, 3.7 TB/s with what they read: a workgroup waits for its rows, its decays and
+// its sums in turn, so what counts is how many a CU holds.  With keys towards the boundaries in LDS it held two and not three, and one workgroup in two
+// was launched for the second chunk of a block and left: 141 us where this takes 115, with strong decays, which make those keys anew for each
+// token, layer 450 and 425.  The scan is held by its barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's error against 64 bits is 5e-8 to 1.1e-7 on both, the
 // output's is its rounding to bf16.
 #include <algorithm>
 
@@ -51,26 +53,29 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   constexpr int TH = DK * 4, LD = DK + 4, LPT = DK / 8;      // lanes per token, eight channels each
   constexpr int NW = DK / 16;
   static_assert(NW * kGB * kGB <= 2 * kGB * LD, "the waves' parts of A take the place of keys and decays");
-  __shared__ __attribute__((aligned(16))) float kb2[2][kGB][LD], kh[48][LD], am[kGB][kGB + 4], rs[kGB][kGlaBlockMaxR + 4];
+  __shared__ __attribute__((aligned(16))) float kb2[2][kGB][LD], am[kGB][kGB + 4], rs[kGB][kGlaBlockMaxR + 4];
   float (&ks)[kGB][LD] = kb2[0], (&bs)[kGB][LD] = kb2[1];
   __shared__ float tots[4][DK];
-  __shared__ int where[2], harsh;
-  const int chunk = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-  if (tid == 0) where[1] = -1, harsh = 0;
-  __syncthreads();
-  for (int i = tid; i < a.seqs; i += TH)
-    if (a.cu_chunks[i] <= chunk && chunk < a.cu_chunks[i + 1]) {
-      where[0] = a.cu_chunks[i];
-      where[1] = i;
-    }
-  __syncthreads();
-  const int cbeg = where[0], seq = where[1];
-  if (seq < 0 || (chunk - cbeg) & 1) return;                 // the second chunk of a block
+  __shared__ int harsh;
+  const int block = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  if (tid == 0) harsh = 0;
+  int seq = -1, cbeg = 0, cend = 0;                          // each wave finds the block's sequence, 64 at a time
+  for (int i0 = 0; i0 < a.seqs && seq < 0; i0 += 64) {
+    const int i = min(i0 + (tid & 63), a.seqs - 1), lo = a.cu_chunks[i], hi = a.cu_chunks[i + 1], first = gla_first_block(lo, i);
+    const unsigned long long here = __ballot(block >= first && block < first + (hi - lo + 1) / 2);
+    if (here == 0) continue;
+    const int at = __builtin_ctzll(here);
+    seq = min(i0 + at, a.seqs - 1);
+    cbeg = __builtin_amdgcn_readlane(lo, at);
+    cend = __builtin_amdgcn_readlane(hi, at);
+  }
+  if (seq < 0) return;                                       // a slot that no sequence has
+  const int chunk = cbeg + (block - gla_first_block(cbeg, seq)) * 2;
   const int64_t tok0 = a.chunk_tok[chunk];
-  const int len = a.chunk_len[chunk] + (chunk + 1 < a.cu_chunks[seq + 1] ? a.chunk_len[chunk + 1] : 0);
+  const int len = a.chunk_len[chunk] + (chunk + 1 < cend ? a.chunk_len[chunk + 1] : 0);
   const int64_t hk = static_cast<int64_t>(a.H) * DK, hv = static_cast<int64_t>(a.H) * a.dv;
   const T *pr = static_cast<const T *>(a.proj) + tok0 * a.ld;
-  unsigned char *rec = reinterpret_cast<unsigned char *>(a.rec) + (static_cast<int64_t>(gla_first_block(cbeg, seq) + (chunk - cbeg) / 2) * a.H + h) * Rec::kSize;
+  unsigned char *rec = reinterpret_cast<unsigned char *>(a.rec) + (static_cast<int64_t>(block) * a.H + h) * Rec::kSize;
   for (int i = tid; i < kGB * a.R; i += TH) {
     const int t = i / a.R, r = i - t * a.R;
     rs[t][r] = t < len ? Elem<T>::ld(pr + t * a.ld + 2 * hk + 2 * hv + r) : 0.f;
@@ -159,11 +164,6 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   }
   __syncthreads();
   const bool apart = harsh != 0;
-  if (apart)                                                 // keys towards the boundaries at 8, 16 and 24 tokens, for A
-    for (int i = tid; i < 48 * DK; i += TH) {
-      const int row = i / DK, d = i % DK, sub = row < 8 ? 1 : row < 24 ? 2 : 3, s = row - (sub == 1 ? 0 : sub == 2 ? 8 : 24);
-      kh[row][d] = ks[s][d] * __builtin_amdgcn_exp2f(bs[sub * 8 - 1][d] - bs[s][d]);
-    }
   uint4 p3[3], k3[3];
   float bq[8];
 #pragma unroll
@@ -234,12 +234,12 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
       load_row(bs[my * 8 - 1], ref);
 #pragma unroll
       for (int i = 0; i < 8; ++i) qh[i] = q[i] * __builtin_amdgcn_exp2f(bt[i] - ref[i]);
-      const int base = my == 1 ? 0 : my == 2 ? 8 : 24;
-      for (int s = 0; s < my * 8; ++s) {
-        float kv[8], acc = 0.f;
-        load_row(kh[base + s], kv);
+      for (int s = 0; s < my * 8; ++s) {                     // keys towards the boundary
+        float kv[8], bv[8], acc = 0.f;
+        load_row(ks[s], kv);
+        load_row(bs[s], bv);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc = fmaf(qh[i], kv[i], acc);
+        for (int i = 0; i < 8; ++i) acc = fmaf(qh[i], kv[i] * __builtin_amdgcn_exp2f(ref[i] - bv[i]), acc);
         acc = group_sum<LPT>(acc);
         if (l == 0) am[t][s] = acc;
       }
@@ -650,7 +650,7 @@ int launch_gla_blocks_of(GlaArgs &a, int first_seq, hipStream_t stream) {
     return e;
   }();
   if (allowed != hipSuccess) return static_cast<int>(allowed);
-  TLF_LAUNCH((gla_block_kernel<DK>), dim3(a.chunks, a.H), dim3(DK * 4), 0, stream, a);
+  TLF_LAUNCH((gla_block_kernel<DK>), dim3((a.chunks + a.seqs + 1) / 2, a.H), dim3(DK * 4), 0, stream, a);
   if (!a.units) {
     TLF_LAUNCH((gla_block_scan_kernel<DK, 0>), dim3(a.H, 1, a.seqs), dim3(waves * 64), lds, stream, a, first_seq);
     return launch_status();
