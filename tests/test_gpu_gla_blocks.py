@@ -136,6 +136,14 @@ def test_stretches_over_sequences(H, dk, dv, lens, start):
     assert count() - before == 4                             # blocks, what stretches add, the states they start from, the scan
 
 
+@pytest.mark.parametrize("dk", [64, 128])
+@pytest.mark.parametrize("dv", [160, 192, 224, 256])           # five to eight waves: the fifth and later finish a block behind their products
+@pytest.mark.parametrize("lens,start", [([1], [3]), ([33, 95, 64], [0, 1, 1]), ([1500, 40], [5, 0])])
+def test_waves_that_share_a_simd(dk, dv, lens, start):
+    for n, out, state in run(2, dk, dv, 8, lens, start, 16.0, seed=dv + len(lens)):
+        assert out < OUT and state < STATE, (n, out, state)
+
+
 @pytest.mark.parametrize("seqs", [16, 17, 32, 33, 63, 64, 65])
 def test_stretches_over_many_sequences(seqs):
     """A lane for each sequence, up to all 64 of them; one more makes two groups."""

@@ -22,11 +22,13 @@
 // segments 59 + 18 + 255 us, so 58 + 15 + 209; 12 of 450 to 900 48 + 24 + 216, and in one pass over whole ones 204.
 //
 // Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256, medians under the profiler: chunk 122 + scan 470 (both
-// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 115 - 135 + first pass 61 + chaining 15 + scan
-// 210 us (whole layer 614 and 377 us).  The blocks write 55 KB a record, 3.7 TB/s with what they read: a workgroup waits for its rows, its decays and
+// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 115 - 135 + first pass 58 - 65 + chaining 15 + scan
+// 169 - 205 us (whole layer 614 and 352 us).  The blocks write 55 KB a record, 3.7 TB/s with what they read: a workgroup waits for its rows, its decays and
 // its sums in turn, so what counts is how many a CU holds.  With keys towards the boundaries in LDS it held two and not three, and one workgroup in two
 // was launched for the second chunk of a block and left: 141 us where this takes 115, with strong decays, which make those keys anew for each
-// token, layer 450 and 425.  The scan is held by its barriers, two waves on a SIMD (matrix cores busy a quarter of the time).  The state's error against 64 bits is 5e-8 to 1.1e-7 on both, the
+// token, layer 450 and 425.  The scan is held by its barriers, two waves on a SIMD: a block took 13900 cycles, 5000 of them products and some 7200
+// vector instructions on each SIMD, the second wave came to the barrier 4100 cycles behind the first.  10900 with the copies on four waves and
+// the block before finished in front of the products by these and behind them by the others: 198 -> 169 us.  The state's error against 64 bits is 5e-8 to 1.1e-7 on both, the
 // output's is its rounding to bf16.
 #include <algorithm>
 
@@ -361,10 +363,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const T *vbase = static_cast<const T *>(a.proj) + 2 * hk + static_cast<int64_t>(h) * a.dv + wave * 32;
   const T *gbase = vbase + static_cast<int64_t>(a.H) * a.dv + hi * 4;
   const unsigned char *rbase = reinterpret_cast<const unsigned char *>(a.rec) + (static_cast<int64_t>(gla_first_block(cbeg, a.seq0 + seq)) * a.H + h) * Rec::kSize;
+  // Two waves of a SIMD leave a barrier together and would go through products, and through what is vector instructions, at the same time.
+  // So the first four waves take the copies and finish the block before, then come to the products; the others begin with the products and
+  // finish the block before behind them.
+  const int early = min(waves, 4);
   auto copy = [&](int b, int buf) __attribute__((always_inline)) {
     const unsigned char *rec = rbase + static_cast<int64_t>(b) * a.H * Rec::kSize;
-    for (int i = (MODE == 1 ? Rec::kK / 1024 : 0) + wave; i < (MODE == 1 ? Rec::kA : Rec::kSize) / 1024; i += waves)
-      dl_copy(lane * 16, rec + i * 1024, recs + buf * Rec::kSize + i * 1024);
+    if (MODE == 1 || wave < early) {
+      const int step = MODE == 1 ? waves : early;
+      for (int i = (MODE == 1 ? Rec::kK / 1024 : 0) + wave; i < (MODE == 1 ? Rec::kA : Rec::kSize) / 1024; i += step)
+        dl_copy(lane * 16, rec + i * 1024, recs + buf * Rec::kSize + i * 1024);
+    }
     if (MODE == 1 && wave == waves - 1) dl_copy(lane * 16, rec + Rec::kDec, recs + buf * Rec::kSize + Rec::kDec);
     const T *vp = vbase + (row0 + static_cast<int64_t>(b) * kGB) * a.ld;
     const int last = min(kGB, tokens - b * kGB) - 1;
@@ -383,7 +392,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   uint2 gate[4];
   auto put = [&](int b, int buf) __attribute__((always_inline)) {
     float ss = 0.f;
-    for (int w = 0; w < waves; ++w) ss += rowsum[(buf * waves + w) * 32 + n];
+    float parts[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) parts[w] = w < waves ? rowsum[(buf * waves + w) * 32 + n] : 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) ss += parts[w];
     const float inv = 1.0f / sqrtf(ss / static_cast<float>(a.dv) + a.eps);
     if (n >= tokens - b * kGB) return;
     T *out = static_cast<T *>(a.out) + (row0 + static_cast<int64_t>(b) * kGB + n) * a.ldo + static_cast<int64_t>(h) * a.dv + wave * 32 + hi * 4;
@@ -413,7 +426,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     TLF_DL_BARRIER_KNOWN();                                  // the gate of the block before, too
     if (b + 1 < b1) copy(b + 1, buf ^ 1);
     if constexpr (MODE != 1) {
-      if (b > b0) put(b - 1, buf ^ 1);
+      if (wave < early && b > b0) put(b - 1, buf ^ 1);
     }
     const int len = min(kGB, tokens - b * kGB);
     const unsigned int rec = recs + buf * Rec::kSize, vt = vs + buf * VB;
@@ -435,8 +448,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     if constexpr (MODE != 1) {
       const T *gp = gbase + (row0 + static_cast<int64_t>(b) * kGB + min(n, len - 1)) * a.ld;
+      auto load_gate = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) gate[c] = *reinterpret_cast<const uint2 *>(gp + c * 8);
+        for (int c = 0; c < 4; ++c) gate[c] = *reinterpret_cast<const uint2 *>(gp + c * 8);
+      };
+      if (wave < early) load_gate();
       floatx16 o0, o1;
 #pragma unroll
       for (int r = 0; r < 16; ++r) o0[r] = o1[r] = 0.f;
@@ -487,6 +503,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < 3; ++i) o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0], af[i], o0, 0, 0, 0);
+      if (wave >= early) {
+        if (b > b0) put(b - 1, buf ^ 1);
+        load_gate();
+      }
       float ss = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
