@@ -21,6 +21,7 @@
 // least of twelve, where this took 209 + 68: twice the reads of B and C, twice the weights), and so were copies issued in a row (+2300 cycles
 // a chunk: a wave waits where several are queued) and step sizes masked as they are loaded (+2200: that waits for them).
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm_shared.h"
 #include "ssd.h"
@@ -100,14 +101,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
 
-  auto at_row = [&](int row, int granule) __attribute__((always_inline)) {      // of C and B: four rows of 64 bytes, and eight of 16, on different banks
+  // C and B: four rows of 64 bytes, and eight of 16, on different banks.  A granule's turn repeats every sixteen rows, so rows further down
+  // are a constant away and other granules an exclusive or.
+  auto at_row = [&](int row, int granule) __attribute__((always_inline)) {
     const int turn = GPR == 16 ? (row & 3) << 2 | (row >> 2 & 3) : GPR == 8 ? (row >> 1 & 1) << 2 | (row >> 2 & 3) : row >> 2 & 3;
     return static_cast<unsigned int>(row * ROW + ((granule ^ turn) << 4));
   };
-  // 32 columns of a wave's rows: sixteen of them
-  auto rows_of_own = [&](const T *p, int64_t ld, int last, unsigned int to, int i) __attribute__((always_inline)) {
-    const int row = i * 16 + (lane >> 2), granule = (lane & 3) ^ (row >> 2 & 3);
-    dl_copy(static_cast<unsigned int>(min(row, last)) * static_cast<unsigned int>(ld) * 2 + granule * 16, p, to + i * 1024);
+  // 32 columns of a wave's rows, sixteen of them at a time; behind the last row, that one
+  auto rows_of_own = [&](const T *p, int ld, int last, unsigned int to, int i) __attribute__((always_inline)) {
+    const int first = min(i * 16, last);
+    const unsigned int down = static_cast<unsigned int>(min(static_cast<int>(__umul24(lane >> 2, ld)), (last - first) * ld));
+    dl_copy(down * 2 + (((lane & 3) ^ (lane >> 4 & 3)) << 4), p + static_cast<int64_t>(first) * ld, to + i * 1024);
   };
   // a chunk's copies in six parts: B and C's first and second half, the wave's x
   constexpr int kParts = 6;
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     for (int i = part * (BB / 2048) + wave; i < (part + 1) * (BB / 2048); i += waves) {
       const int item = i * 64 + lane, row = item / GPR, granule = static_cast<int>(at_row(row, item % GPR) - row * ROW) >> 4;
-      const unsigned int offset = static_cast<unsigned int>(min(row, last)) * static_cast<unsigned int>(a.channels) * 2 + granule * 16;
+      const unsigned int offset = static_cast<unsigned int>(__umul24(min(row, last), a.channels)) * 2 + granule * 16;
       dl_copy(offset, bp, at + CB + i * 1024);
       if (MODE != 1) dl_copy(offset, cp, at + i * 1024);
     }
@@ -144,6 +148,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     h8 = __builtin_bit_cast(bf16x8, make_uint4(p[0], p[1], p[2], p[3]));
     l8 = __builtin_bit_cast(bf16x8, make_uint4(q[0], q[1], q[2], q[3]));
   };
+  if constexpr (MODE != 1) {                                 // the tiles above G's diagonal that are read with others
+    for (int i = tid; i < 512; i += blockDim.x) g_lds[((i >> 8) * 32 + (i >> 4 & 15)) * kSG + (i >> 8) * 32 + 16 + (i & 15)] = 0.f;
+  }
   const float D = MODE == 1 ? 0.f : Elem<T>::ld(static_cast<const T *>(a.D) + h);
   float total = 0.f;                                         // log2 decay of the whole segment
 
@@ -187,7 +194,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int kIssues = MODE == 1 ? kParts : kParts + 4;
     auto issue = [&](int i) __attribute__((always_inline)) {
       if (MODE != 1 && i < 4)
-        rows_of_own(static_cast<const T *>(a.proj) + (begin + static_cast<int64_t>(c) * kSC) * a.ld + h * a.P + p0, a.ld, min(kSC, tokens - c * kSC) - 1, xs, i);
+        rows_of_own(static_cast<const T *>(a.proj) + (begin + static_cast<int64_t>(c) * kSC) * a.ld + h * a.P + p0, static_cast<int>(a.ld), min(kSC, tokens - c * kSC) - 1, xs, i);
       else
         copy(next, ((c - c0) & 1) ^ 1, MODE == 1 ? i : i - 4);
     };
@@ -206,13 +213,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int tile = wave; tile < 10; tile += waves) {      // 16 x 16 tiles of G up to the diagonal
         const int tb = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3, sb = tile - tb * (tb + 1) / 2;
         floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+        const unsigned int at = at_row(m, g);
 #pragma unroll
         for (int k = 0; k < NN; ++k)
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(granule_of(bs + at_row(sb * 16 + m, k * 4 + g)), granule_of(buf + at_row(tb * 16 + m, k * 4 + g)), acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(granule_of(bs + sb * 16 * ROW + (at ^ k << 6)), granule_of(buf + tb * 16 * ROW + (at ^ k << 6)), acc, 0, 0, 0);
+        if (tb == sb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[e] = g * 4 + e <= m ? acc[e] : 0.f;
         *reinterpret_cast<floatx4 *>(g_lds + (tb * 16 + m) * kSG + sb * 16 + g * 4) = acc;
       }
     }
     if constexpr (MODE != 1) {
+      const unsigned int c_at = at_row(n, hi);
       floatx16 y[2];                                         // Y^T: columns t, rows p
 #pragma unroll
       for (int r = 0; r < 16; ++r) y[0][r] = y[1][r] = 0.f;
@@ -230,7 +242,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         pairs(s8, sh, sl);
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) {
-          const bf16x8 cf = granule_of(buf + at_row(tt * 32 + n, kb * 2 + hi));
+          const bf16x8 cf = granule_of(buf + tt * 32 * ROW + (c_at ^ kb << 5));
           y[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sh, cf, y[tt], 0, 0, 0);
           y[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sl, cf, y[tt], 0, 0, 0);
         }
@@ -239,7 +251,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       float scale[2];
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) scale[tt] = __builtin_amdgcn_exp2f(cum[tt * 32 + n]);
-      auto inside = [&](auto grow) __attribute__((always_inline)) {     // G's part, grow(tt, ks, m): the weights of eight values
+      // G's part, grow(tt, ks, m): the weights of eight values; what lies above the diagonal is zero, to be dropped anew where they may be infinite
+      auto inside = [&](auto drop, auto grow) __attribute__((always_inline)) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
@@ -247,7 +260,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             float m8[8];
             Elem<float>::ld8(g_lds + (tt * 32 + n) * kSG + ks * 16 + hi * 8, m8);
             grow(tt, ks, m8);
-            if (tt == ks >> 1) {                             // the diagonal; an exponent above 0 is dropped here
+            if (drop && tt == ks >> 1) {
               const int last = n - (ks & 1) * 16 - hi * 8;
 #pragma unroll
               for (int j = 0; j < 8; ++j) m8[j] = j <= last ? m8[j] : 0.f;
@@ -259,7 +272,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           }
       };
       if (mild) {
-        inside([&](int, int ks, float (&m)[8]) __attribute__((always_inline)) {
+        inside(std::false_type{}, [&](int, int ks, float (&m)[8]) __attribute__((always_inline)) {
           float w8[8];
           Elem<float>::ld8(weight + ks * 16 + hi * 8, w8);
 #pragma unroll
@@ -272,7 +285,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           for (int r = 0; r < 16; ++r) y[tt][r] *= scale[tt];
           scale[tt] = 1.f;
         }
-        inside([&](int tt, int ks, float (&m)[8]) __attribute__((always_inline)) {
+        inside(std::true_type{}, [&](int tt, int ks, float (&m)[8]) __attribute__((always_inline)) {
           const float ct = cum[tt * 32 + n];
 #pragma unroll
           for (int j = 0; j < 8; ++j) m[j] *= weight[ks * 16 + hi * 8 + j] * __builtin_amdgcn_exp2f(ct - cum[ks * 16 + hi * 8 + j]);
@@ -308,6 +321,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int r = 0; r < 16; ++r) S[i][r] *= keep;
     }
+    unsigned int b_at[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {                            // row m of the operand is state row m with bits 2 and 3 exchanged
+      const int chunk = (lane & 1) * 2 + (lane >> 1 & 1);
+      b_at[q] = at_row(hi * 8 + (lane >> 2 & 3) + q * 4, (lane >> 4 & 1) * 2 + (chunk >> 1)) + (chunk & 1) * 8;
+    }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       if constexpr (MODE == 1) {
@@ -323,12 +342,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       bf16_pieces(x8, x3);
 #pragma unroll
       for (int i = 0; i < NN; ++i) {
-        uint2 b[2];                                          // row m of the operand is state row m with bits 2 and 3 exchanged
+        uint2 b[2];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int row = ks * 16 + hi * 8 + (lane >> 2 & 3) + q * 4, chunk = (lane & 1) * 2 + (lane >> 1 & 1);
-          b[q] = turned(bs + at_row(row, i * 4 + (lane >> 4 & 1) * 2 + (chunk >> 1)) + (chunk & 1) * 8);
-        }
+        for (int q = 0; q < 2; ++q) b[q] = turned(bs + ks * 16 * ROW + (b_at[q] ^ i << 6));
         const bf16x8 bt = __builtin_bit_cast(bf16x8, make_uint4(b[0].x, b[0].y, b[1].x, b[1].y));
 #pragma unroll
         for (int e = 0; e < 3; ++e) S[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt, __builtin_bit_cast(bf16x8, x3[e]), S[i], 0, 0, 0);
