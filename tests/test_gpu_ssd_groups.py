@@ -44,6 +44,22 @@ def test_segments(sizes, lens):
             assert rel(got[s][-50:], want[s][-50:]) < 8e-3, (first, s)
 
 
+@pytest.mark.parametrize("sizes,lens,lost", [((64, 64, 64, 8, 4), [670] * 8, True), ((64, 64, 128, 8, 4), [1170, 1071, 970, 1170], False),
+                                             ((32, 64, 32, 8, 4), [770, 72, 700, 770], False)])
+def test_beginnings_that_are_gone_through_once(sizes, lens, lost):
+    """The first pass goes through a chunk or two of each long sequence for good, from nothing and from a state of its own; of a short one
+    through none, which hands its state on.  A sequence without a place for its state takes none along."""
+    proj, w, want = ssd_case(sizes, lens, BF, 9, decay=-5.0, step=-3.0)
+    slots = list(range(1, len(lens) + 1))
+    if lost:
+        slots[1] = -1
+    for steps in ([lens], [[70] * len(lens), [n - 70 for n in lens]]):
+        got = run_ssd(sizes, proj, w, steps, BF, slots)
+        for s in range(len(lens)):
+            if slots[s] > 0 or len(steps) == 1:
+                assert rel(got[s], want[s]) < TOL and rel(got[s][-50:], want[s][-50:]) < 8e-3, s
+
+
 @pytest.mark.parametrize("sizes", [(24, 64, 128, 8, 4), (32, 32, 64, 8, 3), (64, 96, 32, 16, 4)])
 def test_portions_behind_single_tokens(sizes):
     """A step's single tokens come first: portions begin at rows and sequences of their own, in the inputs and behind the convolution.

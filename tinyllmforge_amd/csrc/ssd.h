@@ -24,6 +24,7 @@ struct SsdArgs {
   int64_t ldo;
   int32_t rows, H, P, N, G, taps, inner, channels;
   int32_t first_seq, seqs, first_row, segs, slices;
+  int32_t begun;           // ssd_groups.hip: what the first pass goes through of a sequence, in 1/65536
   float *seg_state, *seg_decay;              // [seqs, segs, H, N, P], [seqs, segs, H]
 };
 
@@ -59,6 +60,6 @@ __device__ __forceinline__ float ssd_wave_scan(float v) {
 
 // ssd_groups.hip
 int ssd_groups_segments(int H, int P, int N, int G, int seqs, int max_tokens, int dtype);   // 0: not for these sizes
-int launch_ssd_groups(const SsdArgs &a, hipStream_t stream);
+int launch_ssd_groups(SsdArgs a, int max_tokens, hipStream_t stream);
 
 }  // namespace tlf

@@ -786,7 +786,7 @@ extern "C" int tlf_ssd_portions(const void *proj, int64_t proj_stride, const voi
                    (reinterpret_cast<uintptr_t>(proj) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
   if (vec && p.group_segs && a.ld % 8 == 0 && a.ld < (1 << 24) && out_stride % 8 == 0 && aligned16(proj) && aligned16(out)) {
     a.segs = p.group_segs;
-    return launch_ssd_groups(a, s);
+    return launch_ssd_groups(a, max_tokens, s);
   }
 #define TLF_SK(NN, PT)                                      \
   do {                                                      \

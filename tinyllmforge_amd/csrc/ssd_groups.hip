@@ -11,10 +11,11 @@
 //                      16 bytes swizzled by the row.  Where some w_s leaves 2^63 (or a head decays by more than 2^100 within a
 //                      chunk), the head takes 2^(c_t - c_s) dt_s pair by pair instead.
 //
-// A segment's contribution comes from a first pass over B and X (MODE 1); a segment adds up what lies before it as it starts.
+// A segment's contribution comes from a first pass over B and X (MODE 1); a segment adds up what lies before it as it starts.  The first pass
+// also goes through the beginning of each sequence for good (ssd_groups_begun).
 //
 // 128 heads of 64 in 8 groups, state 128, 4 sequences of up to 3000 tokens, medians under the profiler: 437 us with ssd_chunk_kernel, which
-// forms G for every head and passes S through LDS as pairs; here 254 + 95.  With the scaled X as pairs 249 + 81, but then 1 to 4 % more outputs
+// forms G for every head and passes S through LDS as pairs; here 254 + 95, or 104 + 178 at steady clocks where it was 82 + 220 without beginnings.  With the scaled X as pairs 249 + 81, but then 1 to 4 % more outputs
 // than with ssd_chunk_kernel missed their nearest bf16 value (1.3 in a thousand do; the state's error is 1.1e-6 to 2.6e-6 on both, and 2e-7
 // to 8e-7 with pieces).  With pairs a chunk of 4 heads took 18700 cycles, 5000 of them products and 9200 vector instructions on each SIMD, the
 // rest latency of two waves per SIMD (S alone takes 64 registers).  16 columns per wave and four waves per SIMD were slower (285 + 71, the
@@ -36,15 +37,13 @@ constexpr int ssd_group_lds(int np, int waves, bool contribution) {
   return 2 * ((contribution ? 1 : 2) * kSC * np * 2 + waves * kSC * 64) + (contribution ? 0 : kSC * kSG * 4) + waves * 3 * kSC * 4;
 }
 
-template <int NN, int MODE>   // N in units of 32; MODE as in ssd_chunk_kernel
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void ssd_group_kernel(const SsdArgs a) {
+// N in units of 32.  MODE 0: a whole sequence, 1: what segment `seg` adds to it, 2: segment `seg` from there, 3: a sequence's beginning.
+template <int NN, int MODE>
+__device__ __forceinline__ void ssd_group(const SsdArgs &a, const int sq, const int seg, unsigned char *smem) {
   typedef unsigned short T;
   constexpr int NP = NN * 32, GPR = NP / 8, ROW = NP * 2, CB = MODE == 1 ? 0 : kSC * ROW, BB = kSC * ROW;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
-  const int sq = MODE == 0 ? blockIdx.z : blockIdx.z / a.segs, seg = MODE == 0 ? 0 : blockIdx.z % a.segs;
-  const bool last_seg = MODE == 0 || seg == a.segs - 1;
   // workgroup w runs on XCD w % 8: those of one group on one where the groups are a multiple of 8
   const int grp = blockIdx.x % a.G, share = a.H / a.G, cols = a.P / 32, units = share * cols, unit = blockIdx.x / a.G * waves + wave;
   const bool active = unit < units;
@@ -52,11 +51,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int seq = a.first_seq + sq, slot = a.state_slots[seq];
   const bool slot_ok = slot >= 0 && slot < a.num_slots;
   const int begin = a.cu_q[seq], tokens = a.cu_q[seq + 1] - begin, chunks = (tokens + kSC - 1) / kSC;
-  int c0 = 0, c1 = chunks;
+  int c0 = 0, c1 = chunks, begun = 0;
   if (MODE != 0) {
-    const int per = (chunks + a.segs - 1) / a.segs;
-    c0 = min(seg * per, chunks);
-    c1 = min(c0 + per, chunks);
+    begun = static_cast<int>(static_cast<int64_t>(chunks) * a.begun >> 16);
+    const int per = (chunks - begun + a.segs - 1) / a.segs;
+    c0 = MODE == 3 ? 0 : min(begun + seg * per, chunks);
+    c1 = MODE == 3 ? begun : min(c0 + per, chunks);
   }
   const unsigned int bufs = TLF_DL_LDSADDR(smem), BUF = CB + BB + waves * kSC * 64;
   float *const g_lds = reinterpret_cast<float *>(smem + 2 * BUF);
@@ -71,24 +71,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (int i = 0; i < NN; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) S[i][r] = 0.f;
-  // The last segment writes the state back while others may yet have to start: the second pass reads it from the last segment's place,
-  // which holds no contribution and where the first pass has put it.
+  // The last segment writes the state back while others may yet have to start: the second pass reads the state behind a sequence's beginning
+  // from the last segment's place, which holds no contribution and where the first pass has put it.
   const bool held = slot_ok && a.starts[seq] != 0;
-  float *const at_start = MODE == 0 ? st : a.seg_state + ((static_cast<int64_t>(sq) * a.segs + a.segs - 1) * a.H + h) * plane + p0 + n;
-  if (MODE == 1 && last_seg) {
-    if (active && held) {
-#pragma unroll
-      for (int i = 0; i < NN; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) at_start[state_at(i, r)] = st[state_at(i, r)];
-    }
-    return;
-  }
-  if (MODE != 1 && active && held) {
+  float *const between = a.seg_state + ((static_cast<int64_t>(sq) * a.segs + a.segs - 1) * a.H + h) * plane + p0 + n;
+  if (MODE != 1 && active && (held || (MODE == 2 && begun))) {
+    const float *from = MODE == 2 ? between : st;
 #pragma unroll
     for (int i = 0; i < NN; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) S[i][r] = at_start[state_at(i, r)];
+      for (int r = 0; r < 16; ++r) S[i][r] = from[state_at(i, r)];
   }
   if (MODE == 2 && active) {
     for (int e = 0; e < seg; ++e) {
@@ -357,13 +349,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int64_t sg = (static_cast<int64_t>(sq) * a.segs + seg) * a.H + h;
     if (p0 == 0 && lane == 0) a.seg_decay[sg] = __builtin_amdgcn_exp2f(total);
     st = a.seg_state + sg * plane + p0 + n;
+  } else if constexpr (MODE == 3) {
+    if (!held && !begun) return;
+    st = between;
   } else {
-    if (!last_seg || !slot_ok || tokens == 0) return;
+    if ((MODE == 2 && seg != a.segs - 1) || !slot_ok || tokens == 0) return;
   }
 #pragma unroll
   for (int i = 0; i < NN; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[state_at(i, r)] = S[i][r];
+}
+
+template <int NN, int MODE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void ssd_group_kernel(const SsdArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int z = blockIdx.z;
+  if constexpr (MODE == 0) ssd_group<NN, 0>(a, z, 0, smem);
+  else if constexpr (MODE == 2) ssd_group<NN, 2>(a, z / a.segs, z % a.segs, smem);
+  else if (z < a.seqs) ssd_group<NN, 3>(a, z, 0, smem);
+  else ssd_group<NN, 1>(a, (z - a.seqs) / (a.segs - 1), (z - a.seqs) % (a.segs - 1), smem);
 }
 
 // A workgroup has the work of up to eight waves, so there are fewer of them than of ssd_chunk_kernel's, and short sequences have to be many:
@@ -381,6 +386,34 @@ int ssd_groups_segments(int H, int P, int N, int G, int seqs, int max_tokens, in
   return seqs * segs > 65535 ? 1 : static_cast<int>(segs);
 }
 
+// The part of each sequence, in 1/65536, that the first pass goes through for good: beside the workgroups that gather contributions half the
+// chip or more has nothing to do, and what is done there is not gone through twice.  The estimate is in tenths of a microsecond: 110 a chunk and
+// 39 where it only adds to the state, 40 to start; rounds of the average length, but none shorter than the longest sequence takes.  Four
+// sequences of 2035 to 3000 tokens, 128 heads in 8 groups: 82 + 220 us without, 104 + 178 with the first 7 of 47 chunks.  Over 1859 random sets of
+// sequences, of half to the whole of a length and of any, the estimate of both passes, but of every workgroup's own length, is 11 % less
+// for the 800 that begin so, more for 20 of them, 9 % at worst.
+int ssd_groups_begun(const SsdArgs &a, int max_tokens) {
+  const int64_t units = static_cast<int64_t>(a.H / a.G) * (a.P / 32), wgs = a.seqs * a.G * ((units + 7) / 8);
+  const int64_t chunks = (static_cast<int64_t>(max_tokens) + kSC - 1) / kSC, most = (chunks + a.segs - 1) / a.segs;
+  if (wgs > 128) return 0;
+  const double share = std::min(1.0, static_cast<double>(a.rows) / (static_cast<double>(a.seqs) * max_tokens));
+  auto pass = [&](int64_t jobs, int64_t cus, int64_t longest, int per_chunk) {
+    return std::max(per_chunk * longest + 40.0, static_cast<double>((jobs + cus - 1) / cus) * (per_chunk * longest * share + 40.0));
+  };
+  double least = 0.97 * (pass(wgs * (a.segs - 1), 256, most, 39) + pass(wgs * a.segs, 256, most, 110));
+  int64_t first = 0;
+  for (int64_t each = most - 1; each > 0 && chunks - a.segs * each <= chunks / 2; --each) {
+    const int64_t begun = chunks - a.segs * each;
+    if (begun <= 0) continue;
+    const double t = std::max(110.0 * begun + 40, pass(wgs * (a.segs - 1), 256 - wgs, each, 39)) + pass(wgs * a.segs, 256, each, 110);
+    if (t < least) {
+      least = 0.99 * t;
+      first = begun;
+    }
+  }
+  return static_cast<int>((first * 65536 + chunks - 1) / chunks);
+}
+
 template <int NN>
 int launch_ssd_groups_of(const SsdArgs &a, hipStream_t stream) {
   static const hipError_t allowed = [] {
@@ -396,12 +429,13 @@ int launch_ssd_groups_of(const SsdArgs &a, hipStream_t stream) {
   if (a.segs == 1) {
     TLF_LAUNCH((ssd_group_kernel<NN, 0>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
   } else {
-    TLF_LAUNCH((ssd_group_kernel<NN, 1>), grid, block, ssd_group_lds(NN * 32, waves, true), stream, a);
+    TLF_LAUNCH((ssd_group_kernel<NN, 1>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
     TLF_LAUNCH((ssd_group_kernel<NN, 2>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
   }
   return launch_status();
 }
-int launch_ssd_groups(const SsdArgs &a, hipStream_t stream) {
+int launch_ssd_groups(SsdArgs a, int max_tokens, hipStream_t stream) {
+  a.begun = a.segs > 1 ? ssd_groups_begun(a, max_tokens) : 0;
   return a.N == 32 ? launch_ssd_groups_of<1>(a, stream) : a.N == 64 ? launch_ssd_groups_of<2>(a, stream) : launch_ssd_groups_of<4>(a, stream);
 }
 
