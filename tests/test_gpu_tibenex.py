@@ -1,5 +1,6 @@
 """Tibenex on the GPU: every kernel against the plain implementation, then the mixers and the model under the engine's schedules."""
 import json
+import math
 import os
 import subprocess
 import sys
@@ -274,6 +275,40 @@ def test_lists_of_more_items_than_workgroups(sizes, portions):
     # up to 268 steps of two products, each rounding a partial sum below two in fp32: 2^9 * 2^-24 on either side; then a rounding to bf16 that may
     # fall to either side, an ulp apart
     torch.testing.assert_close(got.float(), whole.float(), rtol=2 ** -7, atol=2 ** -14)
+
+
+@pytest.mark.parametrize("H,G,D,V", [(4, 2, 32, 32), (8, 8, 96, 64), (16, 2, 128, 128), (24, 1, 64, 64)])
+@pytest.mark.parametrize("way", ["up", "down", "far below", "steps"])
+def test_sums_of_exponentials_follow_the_maximum(H, G, D, V, way):
+    """log2 of each row's and head's sum of exponentials, where scores rise and fall by hundreds along the keys."""
+    from tinyllmforge_amd import _lib
+    lib, bs, portions, g = _lib.load(), 64, [(0, 130), (70, 61), (0, 1), (33, 200)], torch.Generator().manual_seed(D)
+    need = [-(-(a + n) // bs) for a, n in portions]
+    k, v = (torch.randn(sum(need), G, bs, d, generator=g).bfloat16() for d in (D, V))
+    at = torch.arange(bs * max(need), dtype=torch.float32)
+    level = {"up": 1.5 * at, "down": 300 - 2 * at, "far below": at * 0 - 400, "steps": ((at * 7) % 41 - 20) * 12}[way]
+    bt = torch.full((len(need), max(need)), -1, dtype=torch.int32)
+    for s, n in enumerate(need):
+        bt[s, :n] = torch.arange(n) + sum(need[:s])
+        k[sum(need[:s]):sum(need[:s + 1]), :, :, 0] = level[:n * bs].view(n, 1, bs).bfloat16()
+    rows = sum(n for _, n in portions)
+    q = (D ** -0.5 * torch.randn(rows, H, D, generator=g)).bfloat16()
+    q[:, :, 0] = 1.0
+    want, row = torch.empty(rows, H, dtype=torch.float64), 0
+    for s, (a, n) in enumerate(portions):
+        keys = k[bt[s, :need[s]].long()].double().transpose(1, 2).reshape(-1, G, D).repeat_interleave(H // G, 1)
+        scores = torch.einsum("nhd,khd->nhk", q[row:row + n].double(), keys)
+        scores = scores.masked_fill(torch.arange(keys.shape[0]) > a + torch.arange(n)[:, None, None], -float("inf"))
+        want[row:row + n] = torch.logsumexp(scores * math.log(2), -1) / math.log(2)
+        row += n
+    cu, starts = i32(*([0] + torch.tensor([n for _, n in portions]).cumsum(0).tolist())), i32(*[a for a, _ in portions])
+    q, k, v, bt, talk = (t.cuda() for t in (q, k, v, bt, torch.eye(H).bfloat16()))
+    stats, out = torch.full((rows, H), 7.0, device="cuda"), torch.empty(rows, H * V, dtype=torch.bfloat16, device="cuda")
+    ptr = lambda t: t.data_ptr()
+    assert lib.tlf_talk_attn_prefill(ptr(q), ptr(k), ptr(v), ptr(bt), bt.stride(0), ptr(cu), ptr(starts), 0, len(need), 200, ptr(talk), ptr(stats), ptr(out), out.stride(0),
+                                     H, G, D, V, bs, sum(need), torch.cuda.current_stream().cuda_stream) == 0
+    # sums of D products in fp32, below 2^9: 2^9 * 2^-24 a step; the result is rounded like one of them, the sum of up to 233 exponentials to 2^-16
+    assert (stats.double().cpu() - want).abs().max() < (D + 1) * 2 ** -15 + 2 ** -16
 
 
 def layer_in_tiles_and_by_rows(lens, starts, monkeypatch, told=True):

@@ -1,4 +1,5 @@
-// The loop that the prompt kernels of sink_prefill.hip, pooled_prefill.hip and latent_prefill.hip share: bf16, on the matrix cores.
+// The loop that the prompt kernels of sink_prefill.hip, pooled_prefill.hip and latent_prefill.hip share, bf16, on the matrix cores; talk_prefill.hip
+// takes its scores.
 //
 // A workgroup of four waves has 128 units, a query row of one head each, 32 per wave, and walks its keys in tiles of 64:
 //   S^T[key, unit] = K . Q^T         v_mfma_f32_32x32x16_bf16

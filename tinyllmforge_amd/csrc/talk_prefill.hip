@@ -1,8 +1,8 @@
 // Attention of talk_attn.h for prompt portions, bf16, on the matrix cores, from the paged cache.  Mixing needs every head's
 // weights, and weights need their denominators, so there are two kernels:
 //
-//   talk_stats_kernel    log2 of every (row, head)'s sum of exponentials: m + log2 l.  A workgroup owns one KV head and 64 CT units
-//                        (row, head) of it and walks the keys 64 at a time through LDS; S^T[key, unit] = K . Q^T.
+//   talk_stats_kernel    log2 of every (row, head)'s sum of exponentials: m + log2 l.  A workgroup owns one KV head and 128 units
+//                        (row, head) of it and walks the keys 64 at a time through LDS; S^T[key, unit] = K . Q^T (prompt_core.h).
 //   talk_prefill_kernel  a workgroup owns 16 RT query rows with all their heads, a wave 16 rows of four heads, or 32 rows of two, or 64
 //                        of one (those that share a KV head), and walks the keys 32 at a time:
 //     S^T[key, row] = K . Q^T per head, K straight from the caches in operand order, half a tile ahead;
@@ -25,6 +25,7 @@
 #include <algorithm>
 
 #include "gemm_shared.h"
+#include "prompt_core.h"
 #include "prompt_tiles.h"
 #include "talk_attn.h"
 #include "talk_split.h"
@@ -154,15 +155,15 @@ __device__ __forceinline__ void talk_plan(const TalkPrefillArgs &p, int32_t *sha
   }
 }
 
-constexpr int kTS = 64;             // keys per tile of the first kernel
-__device__ __forceinline__ int talk_tile_row(int t) { return (t & 32) | ((t & 4) << 2) | ((t & 24) >> 1) | (t & 3); }
+constexpr int kTS = kPromptKeys;   // keys per tile of the first kernel
 
-// Bound by its exponentials and the vector ALU.  128 registers: with more, the compiler keeps the scores in accumulator registers and moves
-// each out and in (both kernels on 16 heads, eight prompts of up to 2048 tokens: 371 -> 344 us).
-template <int DC, int CT, bool PLAN>
+// A wave has 32 units, a unit's scores of 32 keys two lanes, each with a maximum and a sum of its own.  Bound by products and then
+// exponentials, 33 us of products at the rate of a large one: 16 heads, eight prompts of 1061 to 2048 tokens, 63 us, and 68 on 16x16x32 products
+// with K by way of registers, where a sixth of the time went to bank conflicts and a maximum was taken off every score.
+template <int DC, bool PLAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void talk_stats_kernel(const TalkPrefillArgs p) {
-  constexpr int DP = DC * 32, KCH = DC * 4;
-  __shared__ __attribute__((aligned(16))) unsigned short Ks[2][kTS][DP + 8];
+  typedef PromptCore<DC, 1> Core;
+  __shared__ __attribute__((aligned(16))) unsigned char Ks[2 * Core::KB];
   int sq, plane, xt, block = prompt_block(blockIdx.x, blockIdx.y);
   if constexpr (PLAN) {                                              // eight workgroups in front: the XCDs keep their tiles
     if (block == 0) talk_plan(p, reinterpret_cast<int32_t *>(Ks));
@@ -176,105 +177,77 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
   const int row0 = xt * p.bq;
   if (row0 >= lq || start + lq > static_cast<int64_t>(p.table_cols) * c.bs) return;
   const int32_t *bt = c.bt + seq * c.bt_stride;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
   const int nh = min(p.hpp, p.group - pass * p.hpp);
   const int last_row = min(row0 + p.bq, lq) - 1, i_last = start + last_row;
-  const int wave_first = start + min(row0 + wave * CT * 16 / p.hpp, last_row);
-  const int wave_last = min(start + row0 + ((wave + 1) * CT * 16 - 1) / p.hpp, i_last);
-
-  int upos[CT];
-  int64_t uat[CT];
-  bool uok[CT];
-  bf16x8 qf[CT][DC];
+  Core core;
+  core.start(TLF_DL_LDSADDR(Ks), TLF_DL_LDSADDR(Ks), tid);           // no values
+  const int wave_first = start + min(row0 + core.wave * 32 / p.hpp, last_row);
+  const int wave_last = min(start + row0 + ((core.wave + 1) * 32 - 1) / p.hpp, i_last);
+  const int u = core.wave * 32 + n, r = row0 + u / p.hpp, hh = u % p.hpp;
+  const bool uok = u < p.bq * p.hpp && r <= last_row && hh < nh;
+  const int row = min(r, last_row), upos = start + row;
+  const int64_t uat = static_cast<int64_t>(q0 + row) * p.H + kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0);
 #pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    const int u = wave * CT * 16 + k * 16 + n, r = row0 + u / p.hpp, hh = u % p.hpp;
-    uok[k] = u < p.bq * p.hpp && r <= last_row && hh < nh;
-    const int row = min(r, last_row), h = kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0);
-    upos[k] = start + row;
-    uat[k] = static_cast<int64_t>(q0 + row) * p.H + h;
-#pragma unroll
-    for (int kc = 0; kc < DC; ++kc) {
-      Pack16 t;
-      t.u = *reinterpret_cast<const uint4 *>(p.q + uat[k] * DP + g * 8 + kc * 32);
-      qf[k][kc] = t.v;
-    }
+  for (int kc = 0; kc < 2 * DC; ++kc) {
+    Pack16 t;
+    t.u = *reinterpret_cast<const uint4 *>(p.q + uat * Core::DP + g * 8 + kc * 16);
+    core.qf[kc] = t.v;
   }
-  uint4 kreg[DC];
+  unsigned int koff[DC];                                             // this lane's pieces in a tile, which is one piece of a page
 #pragma unroll
-  for (int i = 0; i < DC; ++i) kreg[i] = make_uint4(0, 0, 0, 0);
-  auto load_tile = [&](int j0) __attribute__((always_inline)) {
-    const int pg = sink_page_of(c, j0);
-    const unsigned short *kp = static_cast<const unsigned short *>(c.k) + sink_row(c, bt[pg], pg, kvh, j0) * DP;
+  for (int i = 0; i < DC; ++i) {
+    int at, piece;
+    core.k_piece(i, lane, at, piece);
+    koff[i] = (at * Core::KCH + piece) * 16;
+  }
+  auto page_of = [&](int t) __attribute__((always_inline)) { return bt[sink_page_of(c, min(t * kTS, i_last))]; };
+  int page_next = page_of(0);                                        // looked up a tile ahead
+  auto copy = [&](int t) __attribute__((always_inline)) {            // rows past the last query are masked
+    const int64_t at = sink_row(c, page_next, sink_page_of(c, t * kTS), kvh, t * kTS);
+    page_next = page_of(t + 1);
+    const unsigned char *kp = static_cast<const unsigned char *>(c.k) + at * (Core::DP * 2);
 #pragma unroll
-    for (int i = 0; i < DC; ++i) kreg[i] = *reinterpret_cast<const uint4 *>(kp + (tid + i * 256) * 8);
+    for (int i = 0; i < DC; ++i) prompt_copy(koff[i], kp, core.k_place(t, i));
   };
-  auto store_tile = [&](int stage) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < DC; ++i) {
-      const int item = tid + i * 256;
-      *reinterpret_cast<uint4 *>(&Ks[stage][talk_tile_row(item / KCH)][item % KCH * 8]) = kreg[i];
-    }
-  };
-  float m[CT], l[CT];
-#pragma unroll
-  for (int k = 0; k < CT; ++k) { m[k] = -INFINITY; l[k] = 0.f; }
+  float m = -INFINITY, l = 0.f, over = -INFINITY;                    // over: what a score must not exceed; no key yet
+  typename Core::Scores from = Core::all(0.f);                       // the score less what stands for the maximum
   const int tiles = i_last / kTS + 1;
-  load_tile(0);
-  store_tile(0);
-  lds_barrier();
+  copy(0);
   for (int t = 0; t < tiles; ++t) {
-    const int k0 = t * kTS, stage = t & 1;
-    if (t + 1 < tiles) load_tile(k0 + kTS);
-    if (k0 <= wave_last) {                                           // wave uniform: some unit sees some key
-      float w[CT][2][8];
+    TLF_DL_BARRIER(0);
+    if (t + 1 < tiles) copy(t + 1);
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        floatx4 s0[CT], s1[CT];
+    for (int hf = 0; hf < 2; ++hf) {
+      const int k0 = t * kTS + hf * 32;
+      if (k0 > wave_last) continue;                                  // wave uniform: some unit sees some key
+      typename Core::Scores s;
+      core.read_k(t, hf);
+      core.scores(from, s);
+      if (k0 + 31 > wave_first) {                                    // the diagonal cuts the half
+        const int seen = upos - (k0 + g * 8);
 #pragma unroll
-        for (int k = 0; k < CT; ++k) s0[k] = s1[k] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kc = 0; kc < DC; ++kc) {
-          Pack16 a0, a1;
-          a0.u = *reinterpret_cast<const uint4 *>(&Ks[stage][hf * 32 + n][kc * 32 + g * 8]);
-          a1.u = *reinterpret_cast<const uint4 *>(&Ks[stage][hf * 32 + n + 16][kc * 32 + g * 8]);
-#pragma unroll
-          for (int k = 0; k < CT; ++k) {
-            s0[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0.v, qf[k][kc], s0[k], 0, 0, 0);
-            s1[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1.v, qf[k][kc], s1[k], 0, 0, 0);
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < CT; ++k)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) w[k][hf][j] = j < 4 ? s0[k][j & 3] : s1[k][j & 3];
+        for (int j = 0; j < 16; ++j) s[j] = (j & 8) * 2 + (j & 7) <= seen ? s[j] : -INFINITY;
       }
-      if (k0 + kTS - 1 > wave_first)                                 // the diagonal cuts the tile
-#pragma unroll
-        for (int k = 0; k < CT; ++k)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) w[k][j >> 3][j & 7] = k0 + (j >> 3) * 32 + g * 8 + (j & 7) <= upos[k] ? w[k][j >> 3][j & 7] : -INFINITY;
-#pragma unroll
-      for (int k = 0; k < CT; ++k) {                                 // a lane's own maximum
-        float x = w[k][0][0];
-#pragma unroll
-        for (int j = 1; j < 16; ++j) x = fmaxf(x, w[k][j >> 3][j & 7]);
-        const float mn = fmaxf(m[k], x), ms = mn == -INFINITY ? 0.f : mn;
-        l[k] *= __builtin_amdgcn_exp2f(m[k] - ms);
-        m[k] = mn;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) l[k] += __builtin_amdgcn_exp2f(w[k][j >> 3][j & 7] - ms);
+      const float x = Core::largest(s);
+      if (__any(x > over)) {
+        const bool up = x > over;
+        const float top = up ? (m != -INFINITY ? m : 0.f) + x : m;
+        l *= up ? __builtin_amdgcn_exp2f(m - top) : 1.f;
+        s -= up ? x : 0.f;
+        m = top;
+        from = Core::all(top == -INFINITY ? 0.f : -top);
+        over = top == -INFINITY ? top : 8.f;
       }
+      float e[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(s[j]);
+      l += Core::sum(e);
     }
-    if (t + 1 < tiles) store_tile(stage ^ 1);
-    lds_barrier();
   }
-#pragma unroll
-  for (int k = 0; k < CT; ++k) {
-    const float top = max_lanes_16_32_48(m[k]);                      // a row sees itself: finite
-    const float sum = sum_lanes_16_32_48(l[k] * __builtin_amdgcn_exp2f(m[k] - top));
-    if (g == 0 && uok[k]) p.stats[uat[k]] = top + __builtin_amdgcn_logf(sum);
-  }
+  const float top = prompt_unit_max(m);                              // a row sees itself: finite
+  const float sum = prompt_unit_sum(l * __builtin_amdgcn_exp2f(m - top));
+  if (g == 0 && uok) p.stats[uat] = top + __builtin_amdgcn_logf(sum);
 }
 
 // Four values of a head's output.
@@ -679,14 +652,14 @@ TalkRoom talk_room(int64_t seqs, int64_t max_tokens, int64_t max_keys, int quads
 
 template <int DC>
 int launch_talk_stats(TalkPrefillArgs &a, int num_seqs, int max_tokens, hipStream_t s) {
-  constexpr int CT = 2, kUnits = 64 * CT;
+  constexpr int kUnits = 32 * kPromptWaves;
   a.hpp = a.group < kUnits ? a.group : kUnits;
   a.passes = (a.group + a.hpp - 1) / a.hpp;
   a.bq = kUnits / a.hpp;
   const int blocks = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, a.c.G * a.passes, num_seqs);
   if (!blocks) return TLF_E_SHAPE;
-  if (a.split.plan) TLF_LAUNCH((talk_stats_kernel<DC, CT, true>), prompt_grid<dim3>(blocks + 8), dim3(256), 0, s, a);
-  else TLF_LAUNCH((talk_stats_kernel<DC, CT, false>), prompt_grid<dim3>(blocks), dim3(256), 0, s, a);
+  if (a.split.plan) TLF_LAUNCH((talk_stats_kernel<DC, true>), prompt_grid<dim3>(blocks + 8), dim3(256), 0, s, a);
+  else TLF_LAUNCH((talk_stats_kernel<DC, false>), prompt_grid<dim3>(blocks), dim3(256), 0, s, a);
   return launch_status();
 }
 
