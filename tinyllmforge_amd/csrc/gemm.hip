@@ -798,6 +798,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_add_rmsnorm_kernel(const Ge
     splitk_reduce_add_rmsnorm_body<TPR, MAXC, W8, 7>(p, t);
 }
 
+// The add-norm in front of a skinny product of one row: rmsnorm_kernel's arithmetic, in its order.
+struct SkinnyNorm {
+  const unsigned short *residual, *weight;
+  unsigned short *residual_out;
+  float eps;
+};
+constexpr int kSkinnyNormK = 8192;
+
 // ---------------------------------------------------------------------------
 // Skinny GEMM for a handful of tokens (decode at small batch; up to 64 rows): weight-bandwidth bound.
 //
@@ -813,15 +821,72 @@ __global__ __launch_bounds__(256) void splitk_reduce_add_rmsnorm_kernel(const Ge
 // PIPE: two batches of weight and activation loads in flight (see below); measured faster up to 8 tokens, where
 // a wave's stream is bound by the latency of its own loads (down projection, 1 token: 15.4 -> 11.4 us), slower
 // from 9 tokens on, where the activation fragments are twice the weight bytes of a K-block.
-template <int MT, int TN, bool W8, bool PIPE>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(PIPE ? 4 : 2, PIPE ? 4 : 8)))
-void skinny_gemm_kernel(const GemmParams p) {
+//
+// NORM: x is the one row's sum with a residual, normalised, made by every workgroup while its first weights are on their way
+// (tlf_add_rmsnorm_gemm_silu_mul_supported).
+template <int TPR, int MAXC>
+__device__ __forceinline__ void skinny_norm_row(const GemmParams &p, const SkinnyNorm &t, unsigned short *xs) {
+  __shared__ float part[TPR / 64];
+  const int tid = threadIdx.x, nchunks = p.K / 8;
+  uint4 pw[MAXC], px[MAXC], pr[MAXC];
+  float v[MAXC][8], ss = 0.f;
+  if (tid < TPR) {
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {
+      const int at = min(tid + c * TPR, nchunks - 1);
+      pw[c] = reinterpret_cast<const uint4 *>(t.weight)[at];
+      px[c] = reinterpret_cast<const uint4 *>(p.x)[at];
+      pr[c] = reinterpret_cast<const uint4 *>(t.residual)[at];
+    }
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {
+      if (tid + c * TPR >= nchunks) break;
+      float r[8];
+      unpack8(px[c], v[c]);
+      unpack8(pr[c], r);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[c][i] = __fadd_rn(v[c][i], r[i]);
+      if (blockIdx.x == 0) reinterpret_cast<uint4 *>(t.residual_out)[tid + c * TPR] = pack8(v[c]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss = fmaf(v[c][i], v[c][i], ss);
+    }
+  }
+  // the order of rmsnorm_finish
+  if (TPR == 64) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+  } else {
+    ss = wave_sum(ss);
+    if (tid < TPR && (tid & 63) == 0) part[tid >> 6] = ss;
+    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < TPR / 64; ++w) ss += part[w];
+  }
+  if (tid < TPR) {
+    const float inv = 1.0f / sqrtf(ss / static_cast<float>(p.K) + t.eps);
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {
+      if (tid + c * TPR >= nchunks) break;
+      float w[8], o[8];
+      unpack8(pw[c], w);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = __fmul_rn(bf16_bits_to_float(float_to_bf16_bits(__fmul_rn(v[c][i], inv))), w[i]);
+      reinterpret_cast<uint4 *>(xs)[tid + c * TPR] = pack8(o);
+    }
+  }
+  __syncthreads();
+}
+
+template <int MT, int TN, bool W8, bool PIPE, bool NORM>
+__device__ __forceinline__ void skinny_gemm(const GemmParams &p, const SkinnyNorm &norm) {
   constexpr int kWaves = 8;
   // K-blocks of 64 per batch of loads: as many as two batches fit in about 64 registers per lane (the kernel
   // keeps to 128 registers, so that two workgroups share a CU)
   constexpr int kRegsPerBlock = TN * (W8 ? 4 : 8) + MT * 8;
   constexpr int kU = 2 * 4 * kRegsPerBlock <= 64 ? 4 : 2 * 2 * kRegsPerBlock <= 64 ? 2 : 1;
   __shared__ __attribute__((aligned(16))) float red[kWaves][TN * MT][64][4];
+  __shared__ __attribute__((aligned(16))) unsigned short xs[NORM ? kSkinnyNormK : 8];
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int r = lane & 15, g = lane >> 4;
@@ -865,7 +930,7 @@ void skinny_gemm_kernel(const GemmParams p) {
     constexpr int kWL = W8 ? 1 : 2;  // 128-bit weight loads per lane, tile and K-block
     struct Batch {
       uint4 w[kU][TN][kWL];
-      uint4 x[kU][MT][2];
+      uint4 x[NORM ? 1 : kU][MT][2];
     };
     auto issue = [&](int kb0, Batch &bt) {
   #pragma unroll
@@ -881,11 +946,13 @@ void skinny_gemm_kernel(const GemmParams p) {
             bt.w[u][t][kWL - 1] = load_nt_u4(src + 16);
           }
         }
+        if constexpr (!NORM) {
   #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          const unsigned char *src = xrow[m] + (static_cast<int64_t>(kb) * kBK + g * 16) * 2;
-          bt.x[u][m][0] = *reinterpret_cast<const uint4 *>(src);
-          bt.x[u][m][1] = *reinterpret_cast<const uint4 *>(src + 16);
+          for (int m = 0; m < MT; ++m) {
+            const unsigned char *src = xrow[m] + (static_cast<int64_t>(kb) * kBK + g * 16) * 2;
+            bt.x[u][m][0] = *reinterpret_cast<const uint4 *>(src);
+            bt.x[u][m][1] = *reinterpret_cast<const uint4 *>(src + 16);
+          }
         }
       }
     };
@@ -913,8 +980,14 @@ void skinny_gemm_kernel(const GemmParams p) {
   #pragma unroll
         for (int m = 0; m < MT; ++m) {
           Pack16 b0, b1;
-          b0.u = bt.x[u][m][0];
-          b1.u = bt.x[u][m][1];
+          if constexpr (NORM) {
+            const uint4 *at = reinterpret_cast<const uint4 *>(xs + (kb0 + u) * kBK + g * 16);
+            b0.u = at[0];
+            b1.u = at[1];
+          } else {
+            b0.u = bt.x[u][m][0];
+            b1.u = bt.x[u][m][1];
+          }
   #pragma unroll
           for (int t = 0; t < TN; ++t) {
             acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[t], b0.v, acc[t][m], 0, 0, 0);
@@ -923,9 +996,14 @@ void skinny_gemm_kernel(const GemmParams p) {
         }
       }
     };
+    Batch ba, bb;
+    if (kb_begin < kb_end) issue(kb_begin, ba);
+    if constexpr (NORM) {
+      if (p.K <= 2048) skinny_norm_row<64, 4>(p, norm, xs);
+      else if (p.K <= 4096) skinny_norm_row<256, 2>(p, norm, xs);
+      else skinny_norm_row<256, 4>(p, norm, xs);
+    }
     if (kb_begin < kb_end) {
-      Batch ba, bb;
-      issue(kb_begin, ba);
       for (int kb0 = kb_begin; kb0 < kb_end; kb0 += 2 * kU) {
         issue(kb0 + kU, bb);
         consume(kb0, ba);
@@ -1051,6 +1129,17 @@ void skinny_gemm_kernel(const GemmParams p) {
   }
 }
 
+template <int MT, int TN, bool W8, bool PIPE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(PIPE ? 4 : 2, PIPE ? 4 : 8)))
+void skinny_gemm_kernel(const GemmParams p) {
+  skinny_gemm<MT, TN, W8, PIPE, false>(p, SkinnyNorm{});
+}
+template <int TN, bool W8>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void skinny_norm_gemm_kernel(const GemmParams p, const SkinnyNorm norm) {
+  skinny_gemm<1, TN, W8, true, true>(p, norm);
+}
+
 // Tuning knobs for sweeps, read from the environment ONCE per process (the first GEMM call or
 // workspace query): what a query returned stays valid for every later call.
 //   TLF_GEMM_PLAN="bn,bm,splits,stages,occ[,kgroups,wn]"  forces one tiled plan
@@ -1117,16 +1206,18 @@ inline const GemmTuning &gemm_tuning() {
   return t;
 }
 
+// 16-channel tiles of a workgroup: more of them reuse the activation fragments, as long as the grid stays large
+int skinny_tiles(int tiles16) {
+  if (gemm_tuning().skinny_tn) return gemm_tuning().skinny_tn;
+  return tiles16 >= 4 * 512 ? 4 : tiles16 >= 2 * 512 ? 2 : 1;
+}
+
 template <bool W8>
 int launch_skinny(const GemmParams &p, hipStream_t stream) {
   if (p.M > 64) return TLF_E_UNSUPPORTED;  // four 16-token MFMA tiles at most
   const int mt = (p.M + 15) / 16;
   const int tiles16 = (p.N + 15) / 16;
-  // more channels per workgroup reuse the activation fragments, as long as the grid stays large
-  int tn = 1;
-  if (tiles16 >= 4 * 512) tn = 4;
-  else if (tiles16 >= 2 * 512) tn = 2;
-  if (gemm_tuning().skinny_tn) tn = gemm_tuning().skinny_tn;
+  const int tn = skinny_tiles(tiles16);
   const dim3 grid((tiles16 + tn - 1) / tn);
   // two batches in flight pay where a CU holds one workgroup or less (N <= 4096: o_proj 5.8 / 6.0 us at 6 / 8 tokens
   // against 6.4 / 6.7, down 12.3 / 12.7 against 14.5 / 15.5) and up to 4 tokens everywhere; a wide N at 5 ... 8 tokens
@@ -1915,6 +2006,48 @@ extern "C" int tlf_bf16_gemm_silu_mul(const void *x, int64_t x_stride, const voi
   if (rc != TLF_OK) return rc;
   return launch_gemm<false>(x, x_stride, w, nullptr, y, M, N, K, nullptr, 0, static_cast<hipStream_t>(stream),
                             nullptr, 1);
+}
+
+// One row, as long as the product would go to the pipelined skinny kernel and all its workgroups, two a CU, begin at once: each makes the norm
+// anew, behind its first weights, and those of a second round would wait for it.  A decoder layer on one token, us, with the norm in a
+// launch of its own and so: 6144 channels of 1024, 384 workgroups, int8 36.6 and 34.0, bf16 47.8 and 45.6; 24576 of 4096, 768 workgroups, 61.0 and
+// 60.8, 113.9 and 118.9.
+extern "C" int tlf_add_rmsnorm_gemm_silu_mul_supported(int32_t M, int32_t N, int32_t K, int32_t w8) {
+  GemmPlan g;
+  if (M != 1 || N <= 0 || N % 16 || K <= 0 || K % kBK || K > kSkinnyNormK) return 0;
+  const int pipe_m = gemm_tuning().skinny_pipe_m;
+  const int tn = skinny_tiles(N / 16);
+  return (N / 16 + tn - 1) / tn <= 512 && M <= skinny_max_m() && (pipe_m < 0 || pipe_m >= M) && !(w8 && plan_wstream(M, N, K, 1, g));
+}
+
+extern "C" int tlf_add_rmsnorm_gemm_silu_mul(const void *x, const void *residual, const void *norm_weight, const void *w, const float *scale, void *y,
+                                             void *residual_out, int32_t M, int32_t N, int32_t K, float eps, void *stream) {
+  const int rc = check_gemm_args(x, K, w, y, M, N, K);
+  if (rc != TLF_OK) return rc;
+  if (!tlf_add_rmsnorm_gemm_silu_mul_supported(M, N, K, scale != nullptr)) return TLF_E_UNSUPPORTED;
+  if (!residual || !norm_weight || !residual_out) return TLF_E_NULL;
+  if (!aligned16(residual) || !aligned16(norm_weight) || !aligned16(residual_out) || !aligned16(scale)) return TLF_E_ALIGN;
+  GemmParams p{};
+  p.x = static_cast<const unsigned char *>(x);
+  p.ldx_bytes = static_cast<int64_t>(K) * 2;
+  p.w = static_cast<const unsigned char *>(w);
+  p.scale = scale;
+  p.y = static_cast<unsigned short *>(y);
+  p.M = M; p.N = N; p.K = K;
+  p.k_per_split = K; p.splits = 1; p.m_tiles = 1; p.n_tiles = 1; p.group_n = 1; p.map_rem = 1;
+  p.act = 1;
+  const SkinnyNorm t{static_cast<const unsigned short *>(residual), static_cast<const unsigned short *>(norm_weight), static_cast<unsigned short *>(residual_out), eps};
+  const int tiles16 = N / 16, tn = skinny_tiles(tiles16);
+  const dim3 grid((tiles16 + tn - 1) / tn);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define TLF_SKN(TN_)                                                                                 \
+  if (scale) TLF_LAUNCH((skinny_norm_gemm_kernel<TN_, true>), grid, dim3(512), 0, s, p, t);          \
+  else TLF_LAUNCH((skinny_norm_gemm_kernel<TN_, false>), grid, dim3(512), 0, s, p, t)
+  if (tn == 4) { TLF_SKN(4); }
+  else if (tn == 2) { TLF_SKN(2); }
+  else { TLF_SKN(1); }
+#undef TLF_SKN
+  return launch_status();
 }
 
 extern "C" size_t tlf_gemm_add_rmsnorm_workspace_bytes(int32_t M, int32_t N, int32_t K) {

@@ -184,6 +184,18 @@ class MergedColumnParallelLinear(ColumnParallelLinear):
             return ops.bf16_linear_silu_mul(x, self.weight)
         return ops.silu_and_mul(super().forward(x))
 
+    def takes_add_norm(self, rows: int) -> bool:
+        """Whether ``forward_add_norm_silu_mul`` takes ``rows`` rows."""
+        return rows == 1 and getattr(self, "interleaved", False) and ops.add_rms_norm_linear_silu_mul_supported(
+            rows, sum(self.output_sizes) // self.tp_size, self.input_size, self.is_quantized)
+
+    def forward_add_norm_silu_mul(self, x: torch.Tensor, residual: torch.Tensor, norm):
+        """``self.forward_silu_mul(norm(x, residual))`` in one kernel; ``norm`` is the ``RMSNorm`` module before this projection.
+        Returns ``(activated, residual)``."""
+        if self.is_quantized:
+            return ops.add_rms_norm_linear_silu_mul(x, residual, norm.weight.data, norm.eps, self.pack_().qpacked, self.qscale)
+        return ops.add_rms_norm_linear_silu_mul(x, residual, norm.weight.data, norm.eps, self.weight.data, None)
+
     def weight_loader(self, param: nn.Parameter, loaded_weight: torch.Tensor, loaded_shard_id: int):
         if getattr(self, "interleaved", False):
             raise RuntimeError("this gate_up weight was re-ordered for the fused kernel: load weights before pack_linears_()")

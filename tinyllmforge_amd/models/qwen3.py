@@ -78,9 +78,11 @@ class Qwen3MLP(nn.Module):
         self.down_proj = RowParallelLinear(intermediate_size, hidden_size, bias=False)
         self.act_fn = SiluAndMul()
 
-    def forward(self, x: torch.Tensor, residual=None, norm=None):
-        # gate_up projection and activation in one kernel when the weights are int8 (qwen3.py:123-130)
-        act = self.gate_up_proj.forward_silu_mul(x)
+    def forward(self, x: torch.Tensor, residual=None, norm=None, before=None):
+        if before is not None:   # the add-norm in front of the layer is still to be done
+            act, residual = self.gate_up_proj.forward_add_norm_silu_mul(x, residual, before)
+        else:                    # gate_up projection and activation in one kernel when the weights are int8 (qwen3.py:123-130)
+            act = self.gate_up_proj.forward_silu_mul(x)
         if norm is not None:   # down_proj together with the add-norm that follows the layer
             return self.down_proj.forward_add_rmsnorm(act, residual, norm)
         return self.down_proj(act)
@@ -103,6 +105,9 @@ class Qwen3DecoderLayer(nn.Module):
         """The layer from after its input norm to after the NEXT norm (the following layer's
         ``input_layernorm`` or the model's final norm): each row-parallel projection runs together with
         the add-norm that consumes it.  Same ops and rounding points as ``forward`` chained with that norm."""
+        if self.self_attn.o_proj.tp_size == 1 and self.mlp.gate_up_proj.takes_add_norm(normed.shape[0]):
+            # one token: the norm in between is part of the projection behind it
+            return self.mlp(self.self_attn(positions, normed), residual, next_norm, self.post_attention_layernorm)
         hidden_states, residual = self.self_attn(positions, normed, residual, self.post_attention_layernorm)
         return self.mlp(hidden_states, residual, next_norm)
 

@@ -379,6 +379,35 @@ def bf16_linear_argmax(x, w):
     return out
 
 
+def add_rms_norm_linear_silu_mul_supported(rows, n, k, quantized):
+    """Whether ``add_rms_norm_linear_silu_mul`` takes ``rows`` rows of ``k`` values and a weight of ``n`` rows."""
+    return rows == 1 and bool(_lib.load().tlf_add_rmsnorm_gemm_silu_mul_supported(rows, n, k, quantized))
+
+
+def add_rms_norm_linear_silu_mul(x, residual, norm_weight, eps, w, scale):
+    """``silu_mul(linear(add_rms_norm(x, residual)))`` behind one call, for one row: ``w`` with interleaved gate and up rows, int8 with ``scale``
+    or bf16 with ``scale=None``.  Returns ``(activated, new_residual)``, the bits of the separate calls."""
+    lib = _lib.load()
+    if scale is not None:
+        w = _packed(w)
+        _need(scale, torch.float32, "scale")
+        N, wk = w.n, w.k
+    else:
+        _need(w, BF16, "w")
+        assert w.is_contiguous()
+        N, wk = w.shape
+    _need(x, BF16, "x"); _need(residual, BF16, "residual"); _need(norm_weight, BF16, "norm_weight")
+    x2 = x.reshape(-1, x.shape[-1]).contiguous()
+    M, K = x2.shape
+    assert residual.is_contiguous() and residual.numel() == M * K and norm_weight.numel() == K and wk == K
+    y = torch.empty(M, N // 2, dtype=BF16, device=x.device)
+    r = torch.empty(M, K, dtype=BF16, device=x.device)
+    check(lib.tlf_add_rmsnorm_gemm_silu_mul(x2.data_ptr(), residual.data_ptr(), norm_weight.data_ptr(), w.data_ptr(),
+                                            None if scale is None else scale.data_ptr(), y.data_ptr(), r.data_ptr(), M, N, K, float(eps), _stream()),
+          "tlf_add_rmsnorm_gemm_silu_mul")
+    return y.view(*x.shape[:-1], N // 2), r.view(x.shape)
+
+
 def linear_add_rms_norm(x, w, scale, residual, norm_weight, eps):
     """``add_rms_norm(linear(x), residual)`` behind one call: ``w`` int8 with ``scale`` (weight-only int8)
     or bf16 with ``scale=None``.  Returns ``(normed, new_residual)``, the bits of the two separate calls."""
