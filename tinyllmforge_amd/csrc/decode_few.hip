@@ -308,10 +308,14 @@ __global__ __launch_bounds__(256) void decode_few_merge_kernel(const FewArgs p) 
 
 // Shares there may be: about 512 workgroups, which is what a context of thousands wants (8 sequences of up to 4096 tokens, 32 heads on 8, layer:
 // 83 us with 16 shares, 95 with 32: what a workgroup ends with is a fifth of a share of 64).
-inline int few_splits(int batch, int kv_heads) {
+// The workspace stays within 1 MiB (63 shares and not 64): an allocator has such a piece at hand, and a graph that is captured takes no memory
+// of its own for it (a larger piece took 0.6 ms of a capture).
+inline int64_t few_share_bytes(int batch, int q_heads) { return static_cast<int64_t>(batch) * q_heads * (kFewDim + 2) * 4; }
+inline int few_splits(int batch, int q_heads, int kv_heads) {
   int splits = kFewMaxSplits;
   while (splits > 16 && splits * batch * kv_heads > 512) splits /= 2;
-  return splits;
+  const int64_t most = (1 << 20) / few_share_bytes(batch, q_heads);
+  return most < 1 ? 1 : most < splits ? static_cast<int>(most) : splits;
 }
 
 }  // namespace tlf
@@ -335,7 +339,7 @@ extern "C" int tlf_decode_few_supported(int32_t batch, int32_t num_q_heads, int3
 
 extern "C" size_t tlf_decode_few_workspace_bytes(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads) {
   if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0) return 0;
-  return static_cast<size_t>(batch) * tlf::few_splits(batch, num_kv_heads) * num_q_heads * (tlf::kFewDim + 2) * 4;
+  return static_cast<size_t>(tlf::few_splits(batch, num_q_heads, num_kv_heads) * tlf::few_share_bytes(batch, num_q_heads));
 }
 
 extern "C" int tlf_decode_few(const void *x, int64_t x_stride, const void *q_norm_weight, const void *k_norm_weight, float eps,
@@ -373,7 +377,7 @@ extern "C" int tlf_decode_few(const void *x, int64_t x_stride, const void *q_nor
   a.k_scale = k_scale; a.v_scale = v_scale; a.bt = block_tables; a.bt_stride = block_table_stride; a.ctx = context_lens;
   a.out = static_cast<unsigned short *>(out); a.blocks = num_cache_blocks; a.Hq = num_q_heads; a.Hkv = num_kv_heads; a.bs = block_size;
   a.max_blocks = max_blocks; a.scale_log2 = scale * kFewLog2e;
-  const int most = (max_blocks * block_size + kFewShare - 1) / kFewShare, splits = few_splits(batch, num_kv_heads);
+  const int most = (max_blocks * block_size + kFewShare - 1) / kFewShare, splits = few_splits(batch, num_q_heads, num_kv_heads);
   a.splits = splits < most ? splits : most;
   a.part = static_cast<float *>(workspace);
   a.ml = a.part + static_cast<int64_t>(batch) * num_q_heads * a.splits * kFewDim;
