@@ -1,6 +1,8 @@
 // In front of the attention of talk_attn.h: projection row [q | k | v] -> RMS norm over all of q and over all of k, rotation of
 // the first rot_dims dimensions of every head in pairs (2 i, 2 i + 1), the score's constants (with a temperature per head) into
 // q, keys and values into the paged caches.  One workgroup per token and part.  HBM bound: a row is read once and written once.
+#include <algorithm>
+
 #include "talk_attn.h"
 
 namespace tlf {
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(256) void talk_prep_kernel(const TalkPrepArgs a) {
 // of one of these.  A workgroup has eight rows of one part; WPR waves have a row, CH granules a lane, and NB rows each are on their way
 // at once: the kernel above waits for a row, for its sum and then for norm weights, cosines and sines.
 //
-// HBM bound: 12237 rows of 16 + 2 x 8 heads of 128, 200 MB, 65 us a row and part a workgroup, 53 so (a large copy 39); 32 heads 111 and 70.
+// HBM bound: 12237 rows of 16 + 2 x 8 heads of 128, 200 MB, 65 us a row and part a workgroup, 49 so (a large copy 39); 32 heads 111 and 70.
 constexpr int kPrepRows = 8;
 
 template <int WPR, int CH>
@@ -211,10 +213,12 @@ __device__ __forceinline__ void talk_prep_rows(const TalkPrepArgs &a, int kind, 
   }
 }
 
+// WIDE: some part has 512 granules.  Without, its two granules a lane cost the others no registers: 52 -> 49 us above.
+template <bool WIDE>
 __global__ __launch_bounds__(256) void talk_prep_rows_kernel(const TalkPrepArgs a) {
   __shared__ float part[kPrepRows][4];
   const int kind = blockIdx.y, granules = (kind == 0 ? a.H * a.c.D : a.c.G * (kind == 1 ? a.c.D : a.c.Dv)) / 8;
-  if (granules == 512) talk_prep_rows<4, 2>(a, kind, part);
+  if (WIDE && granules == 512) talk_prep_rows<4, 2>(a, kind, part);
   else if (granules == 256) talk_prep_rows<4, 1>(a, kind, part);
   else if (granules == 128) talk_prep_rows<2, 1>(a, kind, part);
   else talk_prep_rows<1, 1>(a, kind, part);
@@ -231,7 +235,10 @@ template <typename T, bool PART>
 int launch_talk_prep(const TalkPrepArgs &a, int pieces, hipStream_t s) {
   if constexpr (sizeof(T) == 2 && !PART)
     if (talk_prep_takes_rows(a)) {
-      TLF_LAUNCH(talk_prep_rows_kernel, dim3((a.n + kPrepRows - 1) / kPrepRows, 3), dim3(256), 0, s, a);
+      const dim3 grid((a.n + kPrepRows - 1) / kPrepRows, 3);
+      const int most = std::max(a.H * a.c.D, a.c.G * std::max(a.c.D, a.c.Dv));
+      if (most == 512 * 8) TLF_LAUNCH(talk_prep_rows_kernel<true>, grid, dim3(256), 0, s, a);
+      else TLF_LAUNCH(talk_prep_rows_kernel<false>, grid, dim3(256), 0, s, a);
       return launch_status();
     }
   const dim3 grid(a.n, 3);
