@@ -158,7 +158,7 @@ __device__ __forceinline__ void talk_plan(const TalkPrefillArgs &p, int32_t *sha
 constexpr int kTS = kPromptKeys;   // keys per tile of the first kernel
 
 // A wave has 32 units, a unit's scores of 32 keys two lanes, each with a maximum and a sum of its own.  Bound by products and then
-// exponentials, 33 us of products at the rate of a large one: 16 heads, eight prompts of 1061 to 2048 tokens, 63 us, and 68 on 16x16x32 products
+// exponentials, 33 us of products at the rate of a large one: 16 heads, eight prompts of 1061 to 2048 tokens, 56 us, and 68 on 16x16x32 products
 // with K by way of registers, where a sixth of the time went to bank conflicts and a maximum was taken off every score.
 template <int DC, bool PLAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void talk_stats_kernel(const TalkPrefillArgs p) {
@@ -201,7 +201,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
     core.k_piece(i, lane, at, piece);
     koff[i] = (at * Core::KCH + piece) * 16;
   }
-  auto page_of = [&](int t) __attribute__((always_inline)) { return bt[sink_page_of(c, min(t * kTS, i_last))]; };
+  // A scalar load: by way of the vector memory it would be waited for together with the copies that were issued before it
+  // (342 us a layer of the above and 63 with 87 tokens behind 768; so 334 and 59.5).
+  auto page_of = [&](int t) __attribute__((always_inline)) { return load_uniform(bt + sink_page_of(c, min(t * kTS, i_last))); };
   int page_next = page_of(0);                                        // looked up a tile ahead
   auto copy = [&](int t) __attribute__((always_inline)) {            // rows past the last query are masked
     const int64_t at = sink_row(c, page_next, sink_page_of(c, t * kTS), kvh, t * kTS);
