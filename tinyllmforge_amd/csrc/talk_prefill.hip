@@ -158,7 +158,7 @@ __device__ __forceinline__ void talk_plan(const TalkPrefillArgs &p, int32_t *sha
 constexpr int kTS = kPromptKeys;   // keys per tile of the first kernel
 
 // A wave has 32 units, a unit's scores of 32 keys two lanes, each with a maximum and a sum of its own.  Bound by products and then
-// exponentials, 33 us of products at the rate of a large one: 16 heads, eight prompts of 1061 to 2048 tokens, 56 us, and 68 on 16x16x32 products
+// exponentials, 33 us of products at the rate of a large one: 16 heads, eight prompts of 1061 to 2048 tokens, 59 us, and 68 on 16x16x32 products
 // with K by way of registers, where a sixth of the time went to bank conflicts and a maximum was taken off every score.
 template <int DC, bool PLAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void talk_stats_kernel(const TalkPrefillArgs p) {
