@@ -85,6 +85,26 @@ def test_rows_that_are_not_the_newest_token_come_from_the_cache():
     torch.testing.assert_close(got.double(), exact(q, k2, v2, ctxs, bt, hq, hkv, (None, None)), rtol=2 ** -8, atol=2 ** -13)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hkv,bs,held", [(32, 8, 16, 14), (32, 8, 256, 700), (16, 8, 64, 62), (8, 8, 16, 127), (64, 8, 256, 5000), (2, 2, 32, 8000)])
+def test_rows_of_one_sequence(hq, hkv, bs, held, fp8):
+    """Three tokens of one sequence between two others: a row's attention sees the rows that the same call writes, behind edges of pages and shares."""
+    n = 5 if hq // hkv <= 2 else 4
+    longest, ctxs = held + 3, [held + 2, 70, held + 1, held + 3, 300][:n]
+    mine = [0, 2, 3]
+    qkv, k, v, ctx, bt, scales, slots, w, table, _ = step([longest if i in mine else c for i, c in enumerate(ctxs)], hq, hkv, bs, fp8, seed=held)
+    bt[mine] = bt[0].clone()
+    ctx, positions = torch.tensor(ctxs, dtype=torch.int32, device=DEV), torch.tensor(ctxs, device=DEV) - 1
+    slots = (bt[torch.arange(n, device=DEV), positions // bs] * bs + positions % bs).to(torch.int32)
+    k2, v2 = k.clone(), v.clone()
+    got = ops.decode_few(qkv, hq, k, v, ctx, bt, SCALE, *scales, (*w, EPS, positions, table, slots))
+    q, _, _ = ops.qknorm_rope_store(qkv, *w, EPS, positions, table, hq, hkv, 128, k2, v2, slots, *scales)
+    bits = lambda t: t.view(torch.uint8)
+    assert torch.equal(bits(k), bits(k2)) and torch.equal(bits(v), bits(v2))
+    assert torch.equal(got, ops.decode_few(q, hq, k2, v2, ctx, bt, SCALE, *scales))
+    torch.testing.assert_close(got.double(), exact(q, k2, v2, ctxs, bt, hq, hkv, scales), rtol=2 ** -8, atol=2 ** -13)
+
+
 def test_replayed_with_other_lengths():
     """A captured step follows the lengths and tables it finds."""
     qkv, k, v, ctx, bt, _, slots, w, table, positions = step([4000, 90], 32, 8, 256, False)

@@ -70,13 +70,14 @@ __global__ __launch_bounds__(256) void decode_few_kernel(const FewArgs p) {
   __shared__ __attribute__((aligned(16))) uint4 rows[GROUP + 2][16];        // queries, new K and V, bf16
   __shared__ __attribute__((aligned(16))) float mixes[4][GROUP][kFewDim];
   __shared__ float stats[4][GROUP][2];
+  __shared__ int others[4];         // by wave: whether a page of the share gets another sequence's new row
   const int b = blockIdx.z, kvh = blockIdx.y, split = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, team = tid >> 4, j = tid & 15;
   const int ctx = min(p.ctx[b], p.max_blocks * p.bs), share = few_share(ctx, p.splits), t0 = split * share, t1 = min(ctx, t0 + share);
   const bool newest = RAW && (ctx > 0 ? t0 < ctx && ctx <= t0 + share : split == 0);
   if (t0 >= ctx && !newest) return;
   const int32_t *bt = p.bt + b * p.bt_stride;
   const int64_t row_bytes = static_cast<int64_t>(p.Hkv) * kFewDim * kBytes;
-  const int at = kvh * kFewDim + j * 8;
+  const int at = kvh * kFewDim + j * 8, batch = gridDim.z;
 
   struct Tokens {
     FewRow<FP8> k[kFewAhead], v[kFewAhead];
@@ -103,6 +104,12 @@ __global__ __launch_bounds__(256) void decode_few_kernel(const FewArgs p) {
     }
   };
 
+  auto store = [&](const uint4 v, bool is_k, int64_t slot) __attribute__((always_inline)) {
+    unsigned char *to = (is_k ? p.prep.k_cache : p.prep.v_cache) + slot * row_bytes;
+    if constexpr (FP8) *reinterpret_cast<int2 *>(to + at) = qk_piece_e4m3(v, (is_k ? p.k_scale : p.v_scale)[kvh]);
+    else *reinterpret_cast<uint4 *>(to + at * 2) = v;
+  };
+
   // what the preparation needs, then the first rows
   QkPieceMeta meta;
   QkPieceTable table;
@@ -120,6 +127,13 @@ __global__ __launch_bounds__(256) void decode_few_kernel(const FewArgs p) {
       table = qk_piece_table(meta, head, j, p.prep);
     }
   }
+  // another sequence's new row, and 32 pages of the share to look for it
+  const int seq = tid & 7, at_page = t0 / p.bs + (tid >> 3), last_page = t0 < t1 ? (t1 - 1) / p.bs : -1;
+  int to_slot = -1, page = -1;
+  if (RAW && batch > 1) {
+    if (seq < batch && seq != b && p.prep.slot_mapping) to_slot = p.prep.slot_mapping[seq];
+    if (at_page <= last_page) page = bt[at_page];
+  }
   Tokens cur;
   load(t0, cur);
   float q[GROUP][8];
@@ -128,14 +142,29 @@ __global__ __launch_bounds__(256) void decode_few_kernel(const FewArgs p) {
     if (mine) {
       const uint4 v = qk_piece_value(raw, team <= GROUP, team < GROUP ? p.prep.qw : p.prep.kw, j, meta, table, p.prep);
       rows[team][j] = v;
-      if (newest && team >= GROUP && meta.slot >= 0) {
-        unsigned char *to = (team == GROUP ? p.prep.k_cache : p.prep.v_cache) + meta.slot * row_bytes;
-        if constexpr (FP8) *reinterpret_cast<int2 *>(to + at) = qk_piece_e4m3(v, (team == GROUP ? p.k_scale : p.v_scale)[kvh]);
-        else *reinterpret_cast<uint4 *>(to + at * 2) = v;
-      }
+      if (newest && team >= GROUP && meta.slot >= 0) store(v, team == GROUP, meta.slot);
     }
+    const int to_page = to_slot >= 0 && to_slot < p.prep.num_slots ? to_slot / p.bs : -1;
+    bool other = to_page >= 0 && page == to_page;
+    for (int i = at_page + 32; to_page >= 0 && i <= last_page; i += 32) other = other || bt[i] == to_page;
+    const bool some = __any(other);
+    if (lane == 0) others[wave] = some;
     __syncthreads();
     if (ctx <= 0) return;
+    if (others[0] | others[1] | others[2] | others[3]) {
+      // rows of one sequence in a step: the workgroups that store the others' new rows may come later, so this one stores them, too, the same bits
+      const int from = team >> 1;
+      const bool is_k = team & 1;
+      const int64_t slot = from < batch && from != b ? p.prep.slot_mapping[from] : -1;
+      if (slot >= 0 && slot < p.prep.num_slots && slot != new_slot) {
+        const int row = p.Hq + (is_k ? 0 : p.Hkv) + kvh;
+        const QkPieceMeta m = qk_piece_meta(from, row, p.prep);
+        store(qk_piece_value(*reinterpret_cast<const uint4 *>(p.x + from * p.ldx + row * kFewDim + j * 8), is_k, p.prep.kw, j, m,
+                             qk_piece_table(m, row, j, p.prep), p.prep), is_k, slot);
+      }
+      __syncthreads();
+      load(t0, cur);
+    }
 #pragma unroll
     for (int h = 0; h < GROUP; ++h) unpack8(rows[h][j], q[h]);
     new_k.put(rows[GROUP][j], FP8 ? p.k_scale[kvh] : 1.f);
