@@ -259,9 +259,10 @@ int tlf_w8a16_gemm_silu_mul(const void *x, int64_t x_stride, const void *wq, con
 int tlf_bf16_gemm_silu_mul(const void *x, int64_t x_stride, const void *w, void *y,
                            int32_t M, int32_t N, int32_t K, void *stream);
 
-/* The add-norm in front of that product: tlf_add_rms_norm(x, residual) and then the product of its result, which is not stored; residual_out
+/* The add-norm in front of that product: tlf_add_rmsnorm(x, residual) and then the product of its result, which is not stored; residual_out
  * is.  The bits of the two separate calls.  x, residual, residual_out bf16 [M, K] contiguous, scale NULL with bf16 weights.  For one row (M = 1)
- * of K <= 8192 and not too many channels; _supported says whether these sizes are taken, others return TLF_E_UNSUPPORTED.  Needs no workspace. */
+ * of K <= 8192 and not too many channels; _supported says whether these sizes are taken, others return TLF_E_UNSUPPORTED.  So do outputs that
+ * overlap one another, x, residual or norm_weight: unlike the separate calls it cannot work in place.  Needs no workspace. */
 int tlf_add_rmsnorm_gemm_silu_mul_supported(int32_t M, int32_t N, int32_t K, int32_t w8);
 int tlf_add_rmsnorm_gemm_silu_mul(const void *x, const void *residual, const void *norm_weight,
                                   const void *w, const float *scale, void *y, void *residual_out,

@@ -87,6 +87,18 @@ def test_argument_rejection_happens_before_any_launch():
     assert lib.tlf_gemm_argmax_workspace_bytes(4, 151936, 4096) >= 4 * 151936 * 2 + lib.tlf_argmax_workspace_bytes(4, 151936)
 
 
+def test_a_norm_inside_a_product_does_not_work_in_place():
+    """Workgroups of one call read the row that others' results would overwrite: refused on the host, to the byte."""
+    from tinyllmforge_amd import _lib
+    call, n, k = _lib.load().tlf_add_rmsnorm_gemm_silu_mul, 6144, 1024
+    x, residual, norm, w, scale, y, out = (i << 24 for i in range(1, 8))
+    for a, b, in_out in ((x, y, residual), (x, y, x), (x, y, norm), (x, x, out), (x, residual, out), (x, norm, out), (x, y, y),
+                         (x, y, residual + 2 * k - 16), (x, y, residual - 2 * k + 16), (x, x - n + 16, out), (x, y, y + n - 16)):
+        assert call(a, residual, norm, w, scale, b, in_out, 1, n, k, 1e-6, None) == -5, (a, b, in_out)
+        assert call(a, residual, norm, w, None, b, in_out, 1, n, k, 1e-6, None) == -5, (a, b, in_out)
+    assert call(x, residual, norm, w, scale, y, None, 1, n, k, 1e-6, None) == -1
+
+
 def test_ops_refuse_cpu_tensors():
     import torch
     from tinyllmforge_amd import ops, _lib

@@ -1823,6 +1823,11 @@ int launch_gemm_qknorm_rope_store(const void *x, int64_t x_stride, const void *w
                                a.v_scale, M, a.num_q_heads, a.num_kv_heads, 128, stream);
 }
 
+inline bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+  return p < q + b_bytes && q < p + a_bytes;
+}
+
 inline int check_gemm_args(const void *x, int64_t x_stride, const void *w, const void *y, int32_t M,
                            int32_t N, int32_t K) {
   if (!x || !w || !y) return TLF_E_NULL;
@@ -2027,6 +2032,11 @@ extern "C" int tlf_add_rmsnorm_gemm_silu_mul(const void *x, const void *residual
   if (!tlf_add_rmsnorm_gemm_silu_mul_supported(M, N, K, scale != nullptr)) return TLF_E_UNSUPPORTED;
   if (!residual || !norm_weight || !residual_out) return TLF_E_NULL;
   if (!aligned16(residual) || !aligned16(norm_weight) || !aligned16(residual_out) || !aligned16(scale)) return TLF_E_ALIGN;
+  // every workgroup reads the row, and a first one may store before a last one does
+  const size_t row = static_cast<size_t>(K) * 2, act = static_cast<size_t>(N);
+  for (const void *in : {x, residual, norm_weight})
+    if (overlap(in, row, residual_out, row) || overlap(in, row, y, act)) return TLF_E_UNSUPPORTED;
+  if (overlap(y, act, residual_out, row)) return TLF_E_UNSUPPORTED;
   GemmParams p{};
   p.x = static_cast<const unsigned char *>(x);
   p.ldx_bytes = static_cast<int64_t>(K) * 2;
