@@ -119,3 +119,53 @@ def test_replayed_with_other_lengths():
         graph.replay()
         replayed = out.clone()
         assert torch.equal(replayed, ops.decode_few(*args())), lens
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("prefill,shape", [(False, (1, 1)), (False, (1, 3)), (False, (3, 1)), (True, (1, 5)), (True, (1, 1))])
+def test_a_layer_takes_rows_in_more_than_two_dimensions(prefill, shape, int8):
+    """A decoder layer flattens what comes in front of the hidden size, on one token and a few as on many."""
+    from tinyllmforge_amd.config import ModelConfig
+    from tinyllmforge_amd.layers.layernorm import RMSNorm
+    from tinyllmforge_amd.models.qwen3 import Qwen3DecoderLayer
+    from tinyllmforge_amd.utils.context import reset_context, set_context
+    g, n, width, bs = torch.Generator(device=DEV).manual_seed(3), shape[0] * shape[1], 1024, 16
+    cfg = ModelConfig(hidden_size=width, num_hidden_layers=1, num_attention_heads=16, num_key_value_heads=8, intermediate_size=512, vocab_size=16,
+                      head_dim=128, max_position_embeddings=256)
+    default = torch.get_default_dtype()
+    torch.set_default_dtype(BF)
+    try:
+        with torch.device(DEV):
+            layer, norm = Qwen3DecoderLayer(cfg).to(DEV), RMSNorm(width, EPS).to(DEV)
+    finally:
+        torch.set_default_dtype(default)
+    for lin in (layer.self_attn.qkv_proj, layer.self_attn.o_proj, layer.mlp.gate_up_proj, layer.mlp.down_proj):
+        rows, cols = lin.weight.shape
+        if int8:
+            lin.load_quantized(torch.randint(-127, 128, (rows, cols), dtype=torch.int8, device=DEV, generator=g), torch.full((rows,), cols ** -0.5 / 73, device=DEV))
+            lin.finish_quantized_load()
+            lin.pack_()
+        else:
+            lin.weight.data.normal_(0, cols ** -0.5, generator=g)
+            if lin is layer.mlp.gate_up_proj:
+                lin.interleave_()
+    for m in (layer.self_attn.q_norm, layer.self_attn.k_norm, layer.post_attention_layernorm, norm):
+        m.weight.data.fill_(1)
+    attn = layer.self_attn.attn
+    attn.k_cache, attn.v_cache = (torch.empty(2 * n, bs, 8, 128, dtype=BF, device=DEV).normal_(generator=g) for _ in range(2))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    if prefill:
+        fields = dict(is_prefill=True, cu_seqlens_q=i32([0, n]), cu_seqlens_k=i32([0, n]), max_seqlen_q=n, max_seqlen_k=n, slot_mapping=i32(list(range(n))))
+        positions = torch.arange(n, device=DEV)
+    else:
+        fields = dict(is_prefill=False, slot_mapping=i32([i * 32 + 20 for i in range(n)]), context_lens=i32([21] * n), block_tables=i32([[2 * i, 2 * i + 1] for i in range(n)]))
+        positions = torch.full((n,), 20, device=DEV)
+    x, residual = (torch.empty(n, width, dtype=BF, device=DEV).normal_(generator=g) for _ in range(2))
+    outs = []
+    for view in ((n, width), (*shape, width)):
+        set_context(**fields)
+        with torch.inference_mode():
+            outs.append(layer.forward_normed(positions, x.view(view), residual.view(view), norm))
+        reset_context()
+    for a, b in zip(*outs):
+        assert torch.equal(a, b.view(a.shape))

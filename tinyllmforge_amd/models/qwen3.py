@@ -45,9 +45,9 @@ class QWen3Attention(nn.Module):
             ctx = get_context()
             attn = self.attn
             has_cache = attn.has_cache()
-            if not ctx.is_prefill and has_cache and attn.few(hidden_states.shape[0]):
+            if not ctx.is_prefill and has_cache and attn.few(hidden_states.shape[:-1].numel()):
                 # a few decoding sequences: what lies between the projection and the attention is part of the latter
-                o = attn.forward_projected(self.qkv_proj(hidden_states), self.q_norm, self.k_norm, positions, self.rotary_emb.cos_sin_cache)
+                o = attn.forward_projected(self.qkv_proj(hidden_states.flatten(0, -2)), self.q_norm, self.k_norm, positions, self.rotary_emb.cos_sin_cache)
             else:
                 # prefill without a prefix hit attends over this step's own K/V rows
                 want_kv = ctx.is_prefill and ctx.block_tables is None
@@ -105,7 +105,7 @@ class Qwen3DecoderLayer(nn.Module):
         """The layer from after its input norm to after the NEXT norm (the following layer's
         ``input_layernorm`` or the model's final norm): each row-parallel projection runs together with
         the add-norm that consumes it.  Same ops and rounding points as ``forward`` chained with that norm."""
-        if self.self_attn.o_proj.tp_size == 1 and self.mlp.gate_up_proj.takes_add_norm(normed.shape[0]):
+        if self.self_attn.o_proj.tp_size == 1 and self.mlp.gate_up_proj.takes_add_norm(normed.shape[:-1].numel()):
             # one token: the norm in between is part of the projection behind it
             return self.mlp(self.self_attn(positions, normed), residual, next_norm, self.post_attention_layernorm)
         hidden_states, residual = self.self_attn(positions, normed, residual, self.post_attention_layernorm)
