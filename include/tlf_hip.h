@@ -416,7 +416,7 @@ int tlf_paged_decode_attn_planned(const void *q, int64_t q_stride,
  * tlf_decode_few_supported), spread over more workgroups than a sequence's bytes would need.  With q_norm_weight, x holds
  * rows of the qkv projection [q heads | k heads | v heads]: the call does what tlf_qknorm_rope_store does for them too
  * (models/qwen3.py:79-94, layers/attention.py:94-95) and the same bits go to the caches; rows may be tokens of one sequence, each with
- * its own context length.  Without it (NULL; the arguments up to slot_mapping are not read) x
+ * its own context length, and slot_mapping may be NULL (nothing is stored).  Without it (NULL; the arguments up to slot_mapping are not read) x
  * holds prepared queries and the caches every token.  Either way the results are the same bit for bit.  Empty sequences get zeros.
  * The workspace (16-byte aligned) holds partial results. */
 int tlf_decode_few_supported(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size);

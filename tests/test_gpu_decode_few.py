@@ -85,6 +85,20 @@ def test_rows_that_are_not_the_newest_token_come_from_the_cache():
     torch.testing.assert_close(got.double(), exact(q, k2, v2, ctxs, bt, hq, hkv, (None, None)), rtol=2 ** -8, atol=2 ** -13)
 
 
+def test_arrays_longer_than_the_rows_and_a_step_without_slots():
+    """Static arrays of a larger batch, and rows that nothing keeps, as the separate kernels take them."""
+    qkv, k, v, ctx, bt, _, slots, w, table, positions = step([70, 300, 5, 9], 16, 8, 64, False)
+    few = lambda n, to: ops.decode_few(qkv[:2], 16, k, v, ctx[:n], bt[:n], SCALE, None, None, (*w, EPS, positions[:n], table, to))
+    want = few(2, slots[:2])
+    assert torch.equal(few(4, slots), want)
+    k2, v2 = k.clone().normal_(), v.clone().normal_()
+    k.copy_(k2), v.copy_(v2)
+    got = few(2, None)
+    q, _, _ = ops.qknorm_rope_store(qkv[:2], *w, EPS, positions[:2], table, 16, 8, 128, k2, v2, None)
+    assert torch.equal(k, k2) and torch.equal(v, v2)
+    assert torch.equal(got, ops.decode_few(q, 16, k2, v2, ctx[:2], bt[:2], SCALE)) and not torch.equal(got, want)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("hq,hkv,bs,held", [(32, 8, 16, 14), (32, 8, 256, 700), (16, 8, 64, 62), (8, 8, 16, 127), (64, 8, 256, 5000), (2, 2, 32, 8000)])
 def test_rows_of_one_sequence(hq, hkv, bs, held, fp8):

@@ -383,7 +383,7 @@ extern "C" int tlf_decode_few(const void *x, int64_t x_stride, const void *q_nor
   if (!tlf_decode_few_supported(batch, num_q_heads, num_kv_heads, head_dim, block_size)) return TLF_E_UNSUPPORTED;
   if (kv_dtype != TLF_KV_BF16 && kv_dtype != TLF_KV_FP8_E4M3) return TLF_E_UNSUPPORTED;
   const bool raw = q_norm_weight != nullptr, f8 = kv_dtype == TLF_KV_FP8_E4M3;
-  if (raw && (!k_norm_weight || !positions || !cos_sin || !slot_mapping)) return TLF_E_NULL;
+  if (raw && (!k_norm_weight || !positions || !cos_sin)) return TLF_E_NULL;
   if (f8 && (!k_scale || !v_scale)) return TLF_E_NULL;
   const int64_t width = static_cast<int64_t>(num_q_heads + (raw ? 2 * num_kv_heads : 0)) * head_dim;
   if (x_stride < width || max_blocks <= 0 || num_cache_blocks <= 0 || block_table_stride < max_blocks || (raw && max_pos <= 0)) return TLF_E_SHAPE;

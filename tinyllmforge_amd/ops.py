@@ -539,23 +539,26 @@ def decode_few_supported(batch, num_q_heads, num_kv_heads, head_dim, block_size)
 def decode_few(x, num_q_heads, k_cache, v_cache, context_lens, block_tables, scale, k_scale=None, v_scale=None, prepare=None):
     """Decode attention of a few sequences (``decode_few_supported``) -> ``[B, Hq*Dh]``; caches ``[nblk, bs, Hkv, Dh]``.  ``x``: prepared
     queries ``[B, Hq*Dh]``, every token in the caches; or, with ``prepare = (q_weight, k_weight, eps, positions, cos_sin, slot_mapping)``,
-    rows of the qkv projection, whose q / k norm, RoPE and cache store the call does too (``qknorm_rope_store``, the same bits)."""
+    rows of the qkv projection, whose q / k norm, RoPE and cache store the call does too (``qknorm_rope_store``, the same bits; a row
+    without a slot is not stored, without ``slot_mapping`` none is).  The step's arrays may be longer than its rows."""
     lib = _lib.load()
     _need(x, BF16, "x"); _need(context_lens, torch.int32, "context_lens"); _need(block_tables, torch.int32, "block_tables")
     B = x.shape[0]
     nblk, bs, Hkv, Dh = k_cache.shape
     assert x.dim() == 2 and x.stride(1) == 1 and x.shape[1] == (num_q_heads + (2 * Hkv if prepare else 0)) * Dh
-    assert k_cache.is_contiguous() and v_cache.is_contiguous() and block_tables.stride(1) == 1 and context_lens.numel() == B
+    assert k_cache.is_contiguous() and v_cache.is_contiguous() and block_tables.stride(1) == 1 and min(context_lens.numel(), block_tables.shape[0]) >= B
     kvd = kv_dtype_code(k_cache)
     if kvd == KV_FP8_E4M3:
         _need(k_scale, torch.float32, "k_scale"); _need(v_scale, torch.float32, "v_scale")
     head = (None, None, 0.0, None, None, 0, None)
     if prepare:
         q_weight, k_weight, eps, positions, cos_sin, slot_mapping = prepare
-        _need(positions, torch.int64, "positions"); _need(slot_mapping, torch.int32, "slot_mapping")
-        assert positions.numel() == B and slot_mapping.numel() == B and cos_sin.shape[1] == Dh
+        _need(positions, torch.int64, "positions")
+        if slot_mapping is not None:
+            _need(slot_mapping, torch.int32, "slot_mapping")
+        assert positions.numel() >= B and (slot_mapping is None or slot_mapping.numel() >= B) and cos_sin.shape[1] == Dh
         head = (q_weight.data_ptr(), k_weight.data_ptr(), float(eps), positions.data_ptr(), cos_sin.data_ptr(), cos_sin.shape[0],
-                slot_mapping.data_ptr())
+                _opt(slot_mapping))
     out = torch.empty(B, num_q_heads * Dh, dtype=BF16, device=x.device)
     ws = torch.empty(lib.tlf_decode_few_workspace_bytes(B, num_q_heads, Hkv), dtype=torch.uint8, device=x.device)
     check(lib.tlf_decode_few(x.data_ptr(), x.stride(0), *head, k_cache.data_ptr(), v_cache.data_ptr(), kvd, _opt(k_scale), _opt(v_scale),
