@@ -336,15 +336,16 @@ __global__ __launch_bounds__(256) void decode_few_merge_kernel(const FewArgs p) 
 }
 
 // Shares there may be: about 512 workgroups, which is what a context of thousands wants (8 sequences of up to 4096 tokens, 32 heads on 8, layer:
-// 83 us with 16 shares, 95 with 32: what a workgroup ends with is a fifth of a share of 64).
+// 83 us with 16 shares, 95 with 32: what a workgroup ends with is a fifth of a share of 64).  With eight query heads per KV head a CU holds one workgroup
+// and not two or more: as many as there are CUs, or those without a share to work on take a round of their own (attention block, 64 heads on 8, one sequence of 60 tokens,
+// us: 33.0 with 31 shares, 36.3 with 64), but 16 at least (four of up to 4096 tokens: 67.6 with 7, 50.5 with 16).
 // Where one share fewer keeps the workspace within 1 MiB (63 and not 64 for 32 heads), it is left out: an allocator has such a piece at hand, and a graph that
-// is captured takes no memory of its own for it (a larger piece took 0.6 ms of a capture).  Giving up more for that costs more: 64 heads on 8, attention
-// block, us, with as many shares as fit and with all: 4 sequences of up to 8000 tokens 94.4 (7 shares) and 62.8 (16), 16384 157 and 104; 1 of 16384
-// 64.4 (31) and 55.4 (64).
+// is captured takes no memory of its own for it (a larger piece took 0.6 ms of a capture).
 inline int64_t few_share_bytes(int batch, int q_heads) { return static_cast<int64_t>(batch) * q_heads * (kFewDim + 2) * 4; }
 inline int few_splits(int batch, int q_heads, int kv_heads) {
+  const int workgroups = q_heads / kv_heads == 8 ? 256 : 512;
   int splits = kFewMaxSplits;
-  while (splits > 16 && splits * batch * kv_heads > 512) splits /= 2;
+  while (splits > 16 && splits * batch * kv_heads > workgroups) splits /= 2;
   return (1 << 20) / few_share_bytes(batch, q_heads) == splits - 1 ? splits - 1 : splits;
 }
 
