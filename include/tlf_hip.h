@@ -420,6 +420,8 @@ int tlf_paged_decode_attn_planned(const void *q, int64_t q_stride,
  * holds prepared queries and the caches every token.  Either way the results are the same bit for bit.  Empty sequences get zeros.
  * The workspace (16-byte aligned) holds partial results. */
 int tlf_decode_few_supported(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size);
+/* Whether it is the faster one, too, for contexts of any length that max_blocks table entries hold. */
+int tlf_decode_few_preferred(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_blocks);
 size_t tlf_decode_few_workspace_bytes(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads);
 int tlf_decode_few(const void *x, int64_t x_stride, const void *q_norm_weight, const void *k_norm_weight, float eps,
                    const int64_t *positions, const float *cos_sin, int32_t max_pos, const int32_t *slot_mapping,

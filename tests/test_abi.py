@@ -100,6 +100,20 @@ def test_decode_of_few_sequences_has_workgroups_for_the_chip(batch, hq, hkv):
     assert wanted - 1 <= shares <= wanted
 
 
+def test_decode_of_few_sequences_is_left_to_the_other_kernel_where_tables_are_wide():
+    """The choice follows the longest context that the block tables can hold, for any block size."""
+    from tinyllmforge_amd import _lib
+    few, takes = _lib.load().tlf_decode_few_preferred, _lib.load().tlf_decode_few_supported
+    for batch, hq, hkv, most in ((1, 32, 8, 65536), (1, 16, 16, 65536), (1, 64, 8, 32768), (2, 32, 8, 32768), (2, 16, 8, 32768), (2, 64, 8, 8192),
+                                 (3, 32, 8, 8192), (4, 32, 8, 8192), (8, 16, 8, 8192), (4, 16, 16, 8192), (3, 64, 8, 4096), (4, 32, 4, 4096)):
+        for bs in (16, 256, 4096):
+            assert takes(batch, hq, hkv, 128, bs)
+            assert few(batch, hq, hkv, 128, bs, 1) and few(batch, hq, hkv, 128, bs, most // bs) and not few(batch, hq, hkv, 128, bs, most // bs + 1)
+        assert not few(batch, hq, hkv, 128, 1 << 20, 1 << 20)
+    for sizes in ((5, 32, 8, 128, 256), (9, 16, 8, 128, 256), (0, 16, 8, 128, 256), (1, 32, 8, 64, 256), (1, 32, 8, 128, 24), (1, 24, 8, 128, 256)):
+        assert not takes(*sizes) and not few(*sizes, 4)
+
+
 def test_a_norm_inside_a_product_does_not_work_in_place():
     """Workgroups of one call read the row that others' results would overwrite: refused on the host, to the byte."""
     from tinyllmforge_amd import _lib

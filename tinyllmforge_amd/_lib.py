@@ -64,6 +64,7 @@ SIGNATURES = {
     "tlf_paged_decode_attn": (c_int32, [_P, _I64, _P, _P, _I32, _P, _P, _P, _I64, _P, _P,
                                         _I32, _I32, _I32, _I32, _I32, _I32, _I64, _F, _P, _SZ, _P]),
     "tlf_decode_few_supported": (c_int32, [_I32, _I32, _I32, _I32, _I32]),
+    "tlf_decode_few_preferred": (c_int32, [_I32, _I32, _I32, _I32, _I32, _I32]),
     "tlf_decode_few_workspace_bytes": (_SZ, [_I32, _I32, _I32]),
     "tlf_decode_few": (c_int32, [_P, _I64, _P, _P, _F, _P, _P, _I32, _P, _P, _P, _I32, _P, _P, _P, _I64, _P, _P, _I32, _I32,
                                  _I32, _I32, _I32, _I32, _I64, _F, _P, _SZ, _P]),

@@ -352,13 +352,7 @@ inline int few_splits(int batch, int q_heads, int kv_heads) {
 }  // namespace tlf
 
 // Up to 8 sequences of one or two query heads per KV head, up to 4 of more, whose queries and mixes fill the registers (a workgroup of four heads has
-// 130 to 160, three a CU): beyond, the kernel of decode_attn.hip is faster on long contexts.  Layer of a Qwen3-8B shape, int8, us, preparation,
-// paged_decode_kernel and merge / here, longest of contexts of up to a factor of eight:
-//   32 heads on 8     1 sequence of 100 64.8 / 59.4, 700 67.0 / 60.7, 4096 79.5 / 63.6, 8000 90.7 / 66.8;  4: 69.3 / 62.1, 70.6 / 64.0, 82.2 / 72.3,
-//                     94.4 / 84.0;  8: 73.8 / 65.9, 76.5 / 70.2, 87.7 / 83.2, 100.3 / 110.4
-//   16 heads on 8     1 of 700 43.2 / 36.1, of 8000 67.8 / 41.0;  8: 47.2 / 40.3, 71.3 / 69.8
-//   64 heads on 8     1 of 700 73.3 / 68.6;  4 of 700 78.2 / 73.7, of 8000 102.4 / 97.4;  8: 81.5 / 83.8, 108 / 133
-//   16 heads on 16    1 of 700 74.5 / 58.1;  4 of 8000 118 / 87
+// 130 to 160, three a CU).
 extern "C" int tlf_decode_few_supported(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size) {
   const int g = num_kv_heads;
   if (batch <= 0 || head_dim != tlf::kFewDim || block_size <= 0 || block_size % 16) return 0;
@@ -366,6 +360,22 @@ extern "C" int tlf_decode_few_supported(int32_t batch, int32_t num_q_heads, int3
   const int group = num_q_heads / g;
   if (group != 1 && group != 2 && group != 4 && group != 8) return 0;
   return group <= 2 ? batch <= 8 && batch * g <= 64 : batch <= 4 && batch * g <= 32;
+}
+
+// Whether it is the faster one for all lengths that the tables can hold (a captured step has the tables' width and no lengths): it has a share's rows on their way
+// when it has used those before, so where shares get long the kernel of decode_attn.hip overtakes it, and later with fewer sequences, which have more shares.
+// Attention block with int8 projections of a width of 4096, us, preparation, paged_decode_kernel and merge / here, longest of contexts of up to a factor of eight:
+//   32 heads on 8     1 sequence of 700 32.1 / 27.3, 4096 43.4 / 33.6, 16384 86.3 / 43.7, 65536 114 / 85, 131072 153 / 143;  2 of 700 32.7 / 27.6, 32768 87.6 / 78.1,
+//                     65536 115 / 123;  3 of 700 33.3 / 29.5, 8192 59.8 / 48.2, 16384 72.4 / 76.5;  4 of 700 34.8 / 30.1, 8192 59.0 / 54.0, 16384 71.1 / 78.4
+//   16 heads on 8     1 of 700 28.6 / 22.7, 65536 110 / 76;  2 of 32768 82.6 / 68.4;  4 of 8192 52.9 / 46.4, 16384 65.6 / 69.0;  8 of 700 32.1 / 27.3,
+//                     8192 54.6 / 49.1, 16384 87.2 / 90.4
+//   64 heads on 8     1 of 700 38.2 / 35.1, 32768 102 / 92;  2 of 700 39.1 / 35.8, 8192 67.2 / 64.5, 16384 80.9 / 93.8;  4 of 700 41.7 / 39.9, 4096 54.5 / 50.4, 8192 67.2 / 72.3
+//   16 heads on 16    1 of 700 40.1 / 25.0, 65536 171 / 132;  4 of 700 42.0 / 28.2, 8192 83.7 / 56.6, 32768 176 / 150 (8 on 8 91 / 109)
+extern "C" int tlf_decode_few_preferred(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_blocks) {
+  if (!tlf_decode_few_supported(batch, num_q_heads, num_kv_heads, head_dim, block_size)) return 0;
+  const bool eight = num_q_heads / num_kv_heads == 8;
+  const int64_t most = batch == 1 ? (eight ? 32768 : 65536) : batch == 2 ? (eight ? 8192 : 32768) : eight ? 4096 : 8192;
+  return static_cast<int64_t>(max_blocks) * block_size <= most;
 }
 
 extern "C" size_t tlf_decode_few_workspace_bytes(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads) {

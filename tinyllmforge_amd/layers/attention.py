@@ -26,7 +26,8 @@ class Attention(nn.Module):
 
     def few(self, rows: int) -> bool:
         """Whether a decode step over ``rows`` sequences takes ``ops.decode_few``."""
-        return self.has_cache() and ops.decode_few_supported(rows, self.num_heads, self.num_kv_heads, self.head_dim, self.k_cache.shape[1])
+        return self.has_cache() and ops.decode_few_preferred(rows, self.num_heads, self.num_kv_heads, self.head_dim, self.k_cache.shape[1],
+                                                             get_context().block_tables.shape[1])
 
     def forward_projected(self, qkv: torch.Tensor, q_norm, k_norm, positions: torch.Tensor, cos_sin: torch.Tensor):
         """A decode step of a few sequences from the rows of the qkv projection: q / k norm, RoPE, cache write and attention."""

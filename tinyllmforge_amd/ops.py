@@ -536,6 +536,11 @@ def decode_few_supported(batch, num_q_heads, num_kv_heads, head_dim, block_size)
     return bool(_lib.load().tlf_decode_few_supported(batch, num_q_heads, num_kv_heads, head_dim, block_size))
 
 
+def decode_few_preferred(batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks) -> bool:
+    """Whether ``decode_few`` takes these sizes and is the faster one for any contexts that ``max_blocks`` table entries hold."""
+    return bool(_lib.load().tlf_decode_few_preferred(batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks))
+
+
 def decode_few(x, num_q_heads, k_cache, v_cache, context_lens, block_tables, scale, k_scale=None, v_scale=None, prepare=None):
     """Decode attention of a few sequences (``decode_few_supported``) -> ``[B, Hq*Dh]``; caches ``[nblk, bs, Hkv, Dh]``.  ``x``: prepared
     queries ``[B, Hq*Dh]``, every token in the caches; or, with ``prepare = (q_weight, k_weight, eps, positions, cos_sin, slot_mapping)``,
