@@ -445,3 +445,29 @@ def test_decode_plan_made_once_per_step_gives_identical_tokens(eager):
             gc.collect()
             torch.cuda.empty_cache()
     assert runs[0] == runs[1] and all(len(t) == sp.max_tokens for t, sp in zip(runs[0], sps))
+
+
+@pytest.mark.parametrize("max_model_len,few", [(1024, (1, 2, 4, 8)), (16384, (1, 2))])
+def test_a_decode_plan_is_made_only_for_steps_that_read_it(max_model_len, few):
+    """Steps whose attention takes ``ops.decode_few`` have no kernel in front of their layers: as many as with the plan switched off."""
+    import gc
+    from tinyllmforge_amd import LLM, SamplingParams
+    from tinyllmforge_amd.config import QWEN3_SHAPES
+    kernels, shape = [], dict(QWEN3_SHAPES["qwen3-0.6b"], num_hidden_layers=2)
+    for plan in (False, True):
+        llm = LLM(shape, max_model_len=max_model_len, max_num_seqs=16, num_kvcache_blocks=80, enforce_eager=False, seed=4, decode_plan=plan)
+        try:
+            kernels.append(dict(llm.model_runner.graph_kernels))
+        finally:
+            llm.exit()
+            del llm
+            gc.collect()
+            torch.cuda.empty_cache()
+    assert {b: kernels[1][b] - kernels[0][b] for b in kernels[0]} == {b: int(b not in few) for b in (1, 2, 4, 8, 16)}
+    llm = LLM(shape, max_model_len=max_model_len, max_num_seqs=16, num_kvcache_blocks=80, enforce_eager=True, seed=4)
+    try:
+        for n in (2, 9):
+            llm.generate([[1, 2, 3 + i] for i in range(n)], SamplingParams(temperature=0.0, ignore_eos=True, max_tokens=3))
+            assert (getattr(llm.model_runner, "decode_plan_buf", None) is not None) == (n == 9)
+    finally:
+        llm.exit()

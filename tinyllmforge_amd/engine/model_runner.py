@@ -171,6 +171,7 @@ class ModelRunner:
             if hasattr(module, "k_cache") and hasattr(module, "v_cache"):
                 module.k_cache = self.kv_cache[0, layer_id]
                 module.v_cache = self.kv_cache[1, layer_id]
+                self.paged_attention = module        # of the last layer: all have the same sizes
                 if self.kv_dtype != torch.bfloat16:
                     # build-defined static per-head scales of the e4m3 cache (Config.kv_k_scale / kv_v_scale):
                     # |x| above 448 * scale saturates
@@ -351,8 +352,8 @@ class ModelRunner:
         lengths and the block tables) into one buffer that every step and every captured graph re-uses."""
         ctx = get_context()
         if (not self.config.decode_plan or ctx.context_lens is None or ctx.block_tables is None
-                or ctx.context_lens.numel() > 1024):
-            return      # switched off, or more sequences than a plan holds: every layer scans for itself
+                or ctx.context_lens.numel() > 1024 or self.paged_attention.few(ctx.context_lens.numel())):
+            return      # switched off, more sequences than a plan holds (every layer scans for itself), or so few that ops.decode_few, which has none, takes them
         ctx.decode_plan = self.decode_plan_buf = ops.paged_decode_plan(ctx.context_lens, ctx.block_tables, self.block_size,
                                                                        out=getattr(self, "decode_plan_buf", None))
 
