@@ -53,6 +53,8 @@ template <int DC, int VC>
 struct PromptCore {
   static constexpr int DP = DC * 32, VP = VC * 32, KCH = DC * 4, VCH = VC * 4;
   static constexpr int KB = kPromptKeys * DP * 2, VB = kPromptKeys * VP * 2;        // bytes of a tile
+  // Pieces of a row are found by an exclusive or on its address, so rows of an even number of units have to be a power of two, and buffers begin at a multiple of one
+  static_assert((DC % 2 == 1 || (DC & (DC - 1)) == 0) && (VC % 2 == 1 || (VC & (VC - 1)) == 0), "rows whose pieces an exclusive or finds");
   typedef floatx16 Scores;              // of a half; lane (n, g): keys 16 (r >> 3) + 8 g + (r & 7) of unit n
   struct Weights {
     uint4 hi[2], lo[2];
@@ -79,6 +81,7 @@ struct PromptCore {
   __device__ __forceinline__ unsigned int k_place(int t, int i) const { return klds + (t & 1) * KB + (i * kPromptWaves + wave) * 1024; }
   __device__ __forceinline__ unsigned int v_place(int t, int i) const { return vlds + (t & 1) * VB + (i * kPromptWaves + wave) * 1024; }
 
+  // k, v: LDS addresses of the buffers, aligned(1024)
   __device__ __forceinline__ void start(unsigned int k, unsigned int v, int tid) {
     const int lane = tid & 63, n = lane & 31, g = lane >> 5, vrow = g * 8 + (lane >> 2 & 3);
     wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -163,7 +163,7 @@ constexpr int kTS = kPromptKeys;   // keys per tile of the first kernel
 template <int DC, bool PLAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void talk_stats_kernel(const TalkPrefillArgs p) {
   typedef PromptCore<DC, 1> Core;
-  __shared__ __attribute__((aligned(16))) unsigned char Ks[2 * Core::KB];
+  __shared__ __attribute__((aligned(1024))) unsigned char Ks[2 * Core::KB];
   int sq, plane, xt, block = prompt_block(blockIdx.x, blockIdx.y);
   if constexpr (PLAN) {                                              // eight workgroups in front: the XCDs keep their tiles
     if (block == 0) talk_plan(p, reinterpret_cast<int32_t *>(Ks));
