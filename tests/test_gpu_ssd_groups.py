@@ -60,6 +60,20 @@ def test_beginnings_that_are_gone_through_once(sizes, lens, lost):
                 assert rel(got[s], want[s]) < TOL and rel(got[s][-50:], want[s][-50:]) < 8e-3, s
 
 
+@pytest.mark.parametrize("sizes", [(16, 64, 64, 8, 4), (24, 64, 128, 8, 4), (56, 32, 32, 8, 4)])
+def test_first_passes_without_beginnings(sizes):
+    """Sequences enough for half the chip: the first pass only gathers, in less LDS, and hands the states on that are there."""
+    lens, times = [1160, 300, 700], 9
+    proj, w, want = ssd_case(sizes, lens, BF, 11, decay=-5.0, step=-3.0)
+    slots = list(range(1, 3 * times + 1))
+    slots[4] = -1
+    for steps in ([lens], [[70, 2, 64], [1090, 298, 636]], [[8, 140, 1], [1152, 160, 699]]):
+        got = run_ssd(sizes, proj * times, w, [x * times for x in steps], BF, slots)
+        for s in range(3 * times):
+            if slots[s] > 0 or len(steps) == 1:
+                assert rel(got[s], want[s % 3]) < TOL and rel(got[s][-50:], want[s % 3][-50:]) < 8e-3, s
+
+
 @pytest.mark.parametrize("sizes", [(24, 64, 128, 8, 4), (32, 32, 64, 8, 3), (64, 96, 32, 16, 4)])
 def test_portions_behind_single_tokens(sizes):
     """A step's single tokens come first: portions begin at rows and sequences of their own, in the inputs and behind the convolution.

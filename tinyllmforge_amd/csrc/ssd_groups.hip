@@ -140,7 +140,7 @@ __device__ __forceinline__ void ssd_group(const SsdArgs &a, const int sq, const 
     h8 = __builtin_bit_cast(bf16x8, make_uint4(p[0], p[1], p[2], p[3]));
     l8 = __builtin_bit_cast(bf16x8, make_uint4(q[0], q[1], q[2], q[3]));
   };
-  if constexpr (MODE != 1) {                                 // the tiles above G's diagonal that are read with others
+  if (MODE != 1 && (MODE != 3 || begun)) {                   // the tiles above G's diagonal that are read with others
     for (int i = tid; i < 512; i += blockDim.x) g_lds[((i >> 8) * 32 + (i >> 4 & 15)) * kSG + (i >> 8) * 32 + 16 + (i & 15)] = 0.f;
   }
   const float D = MODE == 1 ? 0.f : Elem<T>::ld(static_cast<const T *>(a.D) + h);
@@ -429,7 +429,9 @@ int launch_ssd_groups_of(const SsdArgs &a, hipStream_t stream) {
   if (a.segs == 1) {
     TLF_LAUNCH((ssd_group_kernel<NN, 0>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
   } else {
-    TLF_LAUNCH((ssd_group_kernel<NN, 1>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
+    // Without beginnings it needs no C and no G, so that workgroups of four waves, of which registers allow two a CU, find the LDS for it.  20 sequences of up to
+    // 2000 tokens, 16 heads of 64 in 8 groups, layer 331 us with all of it and 328 so, state 64 258 and 251; 18 of up to 4000 540 and 534, 409 and 398.
+    TLF_LAUNCH((ssd_group_kernel<NN, 1>), grid, block, ssd_group_lds(NN * 32, waves, a.begun == 0), stream, a);
     TLF_LAUNCH((ssd_group_kernel<NN, 2>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
   }
   return launch_status();
