@@ -162,3 +162,15 @@ def test_gemm_plan_has_a_kernel_for_every_shape_the_models_use():
                         assert lib.tlf_w8a16_gemm_workspace_bytes(m, n, k) >= splits * m * n * 4
     assert len(seen) >= 6, seen          # the sweep reaches the skinny kernel and several tile shapes
     assert lib.tlf_gemm_plan(4, 1024, 100, 1, plan) == -2   # K not a multiple of 64
+
+
+def test_gemm_plan_of_a_short_k_follows_what_stays_in_the_caches():
+    """bf16 products of up to 1024 columns: 128 x 128 tiles, but the wider ones where the longer operand has more than 64 MB."""
+    import ctypes
+    from tinyllmforge_amd import _lib
+    plan = (ctypes.c_int32 * 8)()
+    for m, n, k, small in ((12240, 2048, 256, True), (4200, 6144, 1024, True), (12240, 2048, 1088, False), (512, 32768, 1024, True), (512, 32784, 1024, False),
+                           (256, 151936, 1024, False), (700, 151936, 768, False), (512, 151936, 512, True), (513, 151936, 512, False), (512, 151936, 576, False),
+                           (32768, 512, 1024, True), (32769, 512, 1024, False), (49152, 512, 768, False), (1500, 8192, 512, True)):
+        assert _lib.load().tlf_gemm_plan(m, n, k, 0, plan) == 0
+        assert list(plan)[:3] == ([128, 128, 2] if small else [256, 128, 3]), (m, n, k, list(plan))

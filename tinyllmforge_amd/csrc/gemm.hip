@@ -28,6 +28,7 @@
 // (each with a private L2), so workgroup b belongs to XCD b % 8.  Each XCD is
 // given whole columns of N-tiles, so the workgroups that share an L2 share W
 // and x panels and step through K together.
+#include <algorithm>
 #include <stdio.h>
 #include <type_traits>
 #include <stdlib.h>
@@ -1459,11 +1460,14 @@ inline GemmPlan plan_gemm(int M, int N, int K, bool w8) {
     // 16384 tokens: 6144 x 4096 1125 / 1207 against 944 / 1102, 4096 x 4096 1272 / 1252 against 1117 / 1157,
     // 24576 x 4096 1196 / 1189 against 1109 / 1122; 4096 x 12288 (192 K-tiles) ties or loses 1-3 %, hence the bound on K.
     g.bn = 256; g.bm = 256; g.stages = 2; g.occ = 2; g.wn = 8;
-  } else if (ktiles <= 16) {
+  } else if (ktiles <= 16 && (static_cast<int64_t>(std::max(M, N)) * K <= 1 << 25 || (ktiles <= 8 && std::min(M, N) <= 512))) {
     // K up to 1024: a workgroup is mostly its first copies and its stores, which a second one on the CU hides.  128 x 128 with two stages
     // (64 KB) against one 256 x 128 workgroup per CU, us: 2048 channels at 12240 tokens K = 128 18.6 / 22.1, 256 23.7 / 27.1,
     // 512 33.5 / 36.8, 1024 55.3 / 64.5, 1536 93 / 88 - 95, 2048 104 / 100, 4096 191 / 182; at 4200 tokens 256 12.5 / 16.6, 1024 30.3 /
     // 33.6; 6144 x 1024 at 4000 54.4 / 59.2; 8192 x 512 at 1500 19.2 / 21.2.
+    // Smaller tiles read their operands more often, so not where the longer one leaves the caches (64 MB): 151936 x 1024 at 256 tokens 118.8 / 112.5, at 700
+    // 286 / 270, 65536 x 1024 at 512 89 / 84, 768 columns at 49152 tokens 66 / 62 (512 channels), 32000 x 1024 at 512 tokens 38.1 / 40.4; with up to 512
+    // columns and 512 tokens it is no matter (151936 x 512 at 512 127 / 132, at 768 186 / 181).
     g.bn = 128; g.bm = 128; g.stages = 2; g.occ = 2; g.wn = 2;
   } else {  // bf16, one 256 x 128 tile per CU or more (measured 7-10 % faster than 128 x 128 from there on)
     g.bn = 256; g.bm = 128; g.stages = 3; g.occ = 1;
