@@ -388,10 +388,12 @@ int ssd_groups_segments(int H, int P, int N, int G, int seqs, int max_tokens, in
 
 // The part of each sequence, in 1/65536, that the first pass goes through for good: beside the workgroups that gather contributions half the
 // chip or more has nothing to do, and what is done there is not gone through twice.  The estimate is in tenths of a microsecond: 110 a chunk and
-// 39 where it only adds to the state, 40 to start; rounds of the average length, but none shorter than the longest sequence takes.  Four
-// sequences of 2035 to 3000 tokens, 128 heads in 8 groups: 82 + 220 us without, 104 + 178 with the first 7 of 47 chunks.  Over 1859 random sets of
-// sequences, of half to the whole of a length and of any, the estimate of both passes, but of every workgroup's own length, is 11 % less
-// for the 800 that begin so, more for 20 of them, 9 % at worst.
+// 39 where it only adds to the state, 40 to start (128 rows of state; fewer take less in all passes alike); rounds of the average length, but none shorter
+// than the longest sequence takes.  Four sequences of 2035 to 3000 tokens, 128 heads in 8 groups: 82 + 220 us without, 104 + 178 with the first 7 of 47 chunks.
+//
+// Layer, us, without and with, states of 32, 64 and 128 rows: 12 sequences of up to 900 tokens, 32 heads of 64, 110 / 108, 24 heads in 4 groups 114 / 108,
+// 32 heads 140 / 136; 3 of up to 1000, 64 heads, 73 / 68, 78 / 73.5, 93 / 87; 4 of up to 3000 184 / 181, 195 / 191, 225 / 223; of 33 such sets none was slower but 12 of up
+// to 450, 70.4 / 72.2, 74.0 / 75.9, 86.9 / 88.2, where the estimate promises 4.6 us: so less than 8 does not count.
 int ssd_groups_begun(const SsdArgs &a, int max_tokens) {
   const int64_t units = static_cast<int64_t>(a.H / a.G) * (a.P / 32), wgs = a.seqs * a.G * ((units + 7) / 8);
   const int64_t chunks = (static_cast<int64_t>(max_tokens) + kSC - 1) / kSC, most = (chunks + a.segs - 1) / a.segs;
@@ -400,7 +402,8 @@ int ssd_groups_begun(const SsdArgs &a, int max_tokens) {
   auto pass = [&](int64_t jobs, int64_t cus, int64_t longest, int per_chunk) {
     return std::max(per_chunk * longest + 40.0, static_cast<double>((jobs + cus - 1) / cus) * (per_chunk * longest * share + 40.0));
   };
-  double least = 0.97 * (pass(wgs * (a.segs - 1), 256, most, 39) + pass(wgs * a.segs, 256, most, 110));
+  const double without = pass(wgs * (a.segs - 1), 256, most, 39) + pass(wgs * a.segs, 256, most, 110);
+  double least = std::min(0.97 * without, without - 80);
   int64_t first = 0;
   for (int64_t each = most - 1; each > 0 && chunks - a.segs * each <= chunks / 2; --each) {
     const int64_t begun = chunks - a.segs * each;
