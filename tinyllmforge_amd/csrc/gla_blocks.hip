@@ -392,11 +392,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   uint2 gate[4];
   auto put = [&](int b, int buf) __attribute__((always_inline)) {
     float ss = 0.f;
-    float parts[8];
-#pragma unroll
-    for (int w = 0; w < 8; ++w) parts[w] = w < waves ? rowsum[(buf * waves + w) * 32 + n] : 0.f;
-#pragma unroll
-    for (int w = 0; w < 8; ++w) ss += parts[w];
+    for (int w = 0; w < waves; ++w) ss += rowsum[(buf * waves + w) * 32 + n];
     const float inv = 1.0f / sqrtf(ss / static_cast<float>(a.dv) + a.eps);
     if (n >= tokens - b * kGB) return;
     T *out = static_cast<T *>(a.out) + (row0 + static_cast<int64_t>(b) * kGB + n) * a.ldo + static_cast<int64_t>(h) * a.dv + wave * 32 + hi * 4;
