@@ -144,14 +144,16 @@ __global__ __launch_bounds__(256) void decode_few_kernel(const FewArgs p) {
       rows[team][j] = v;
       if (newest && team >= GROUP && meta.slot >= 0) store(v, team == GROUP, meta.slot);
     }
-    const int to_page = to_slot >= 0 && to_slot < p.prep.num_slots ? to_slot / p.bs : -1;
-    bool other = to_page >= 0 && page == to_page;
-    for (int i = at_page + 32; to_page >= 0 && i <= last_page; i += 32) other = other || bt[i] == to_page;
-    const bool some = __any(other);
-    if (lane == 0) others[wave] = some;
+    if (batch > 1) {
+      const int to_page = to_slot >= 0 && to_slot < p.prep.num_slots ? to_slot / p.bs : -1;
+      bool other = to_page >= 0 && page == to_page;
+      for (int i = at_page + 32; to_page >= 0 && i <= last_page; i += 32) other = other || bt[i] == to_page;
+      const bool some = __any(other);
+      if (lane == 0) others[wave] = some;
+    }
     __syncthreads();
     if (ctx <= 0) return;
-    if (others[0] | others[1] | others[2] | others[3]) {
+    if (batch > 1 && (others[0] | others[1] | others[2] | others[3])) {
       // rows of one sequence in a step: the workgroups that store the others' new rows may come later, so this one stores them, too, the same bits
       const int from = team >> 1;
       const bool is_k = team & 1;
