@@ -37,7 +37,8 @@ constexpr int ssd_group_lds(int np, int waves, bool contribution) {
   return 2 * ((contribution ? 1 : 2) * kSC * np * 2 + waves * kSC * 64) + (contribution ? 0 : kSC * kSG * 4) + waves * 3 * kSC * 4;
 }
 
-// N in units of 32.  MODE 0: a whole sequence, 1: what segment `seg` adds to it, 2: segment `seg` from there, 3: a sequence's beginning.
+// N in units of 32.  MODE 0: a whole sequence, 1: what segment `seg` adds to it, 2: segment `seg` from there, 3: a sequence's beginning, 4: none, the state
+// is only handed on.
 template <int NN, int MODE>
 __device__ __forceinline__ void ssd_group(const SsdArgs &a, const int sq, const int seg, unsigned char *smem) {
   typedef unsigned short T;
@@ -81,6 +82,15 @@ __device__ __forceinline__ void ssd_group(const SsdArgs &a, const int sq, const 
     for (int i = 0; i < NN; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) S[i][r] = from[state_at(i, r)];
+  }
+  if constexpr (MODE == 4) {
+    if (active && held) {
+#pragma unroll
+      for (int i = 0; i < NN; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) between[state_at(i, r)] = S[i][r];
+    }
+    return;
   }
   if (MODE == 2 && active) {
     for (int e = 0; e < seg; ++e) {
@@ -140,7 +150,7 @@ __device__ __forceinline__ void ssd_group(const SsdArgs &a, const int sq, const 
     h8 = __builtin_bit_cast(bf16x8, make_uint4(p[0], p[1], p[2], p[3]));
     l8 = __builtin_bit_cast(bf16x8, make_uint4(q[0], q[1], q[2], q[3]));
   };
-  if (MODE != 1 && (MODE != 3 || begun)) {                   // the tiles above G's diagonal that are read with others
+  if constexpr (MODE != 1) {                                 // the tiles above G's diagonal that are read with others
     for (int i = tid; i < 512; i += blockDim.x) g_lds[((i >> 8) * 32 + (i >> 4 & 15)) * kSG + (i >> 8) * 32 + 16 + (i & 15)] = 0.f;
   }
   const float D = MODE == 1 ? 0.f : Elem<T>::ld(static_cast<const T *>(a.D) + h);
@@ -367,7 +377,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int z = blockIdx.z;
   if constexpr (MODE == 0) ssd_group<NN, 0>(a, z, 0, smem);
   else if constexpr (MODE == 2) ssd_group<NN, 2>(a, z / a.segs, z % a.segs, smem);
-  else if (z < a.seqs) ssd_group<NN, 3>(a, z, 0, smem);
+  else if (z < a.seqs) ssd_group<NN, MODE == 1 ? 3 : 4>(a, z, 0, smem);
   else ssd_group<NN, 1>(a, (z - a.seqs) / (a.segs - 1), (z - a.seqs) % (a.segs - 1), smem);
 }
 
@@ -422,7 +432,7 @@ int launch_ssd_groups_of(const SsdArgs &a, hipStream_t stream) {
   static const hipError_t allowed = [] {
     hipError_t e = hipSuccess;
     for (const void *k : {reinterpret_cast<const void *>(&ssd_group_kernel<NN, 0>), reinterpret_cast<const void *>(&ssd_group_kernel<NN, 1>),
-                          reinterpret_cast<const void *>(&ssd_group_kernel<NN, 2>)})
+                          reinterpret_cast<const void *>(&ssd_group_kernel<NN, 2>), reinterpret_cast<const void *>(&ssd_group_kernel<NN, 3>)})
       if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, ssd_group_lds(NN * 32, 8, false));
     return e;
   }();
@@ -432,9 +442,10 @@ int launch_ssd_groups_of(const SsdArgs &a, hipStream_t stream) {
   if (a.segs == 1) {
     TLF_LAUNCH((ssd_group_kernel<NN, 0>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
   } else {
-    // Without beginnings it needs no C and no G, so that workgroups of four waves, of which registers allow two a CU, find the LDS for it.  20 sequences of up to
+    // Without beginnings the first pass needs no C and no G, so that workgroups of four waves, of which registers allow two a CU, find the LDS for it.  20 sequences of up to
     // 2000 tokens, 16 heads of 64 in 8 groups, layer 331 us with all of it and 328 so, state 64 258 and 251; 18 of up to 4000 540 and 534, 409 and 398.
-    TLF_LAUNCH((ssd_group_kernel<NN, 1>), grid, block, ssd_group_lds(NN * 32, waves, a.begun == 0), stream, a);
+    if (a.begun) TLF_LAUNCH((ssd_group_kernel<NN, 1>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
+    else TLF_LAUNCH((ssd_group_kernel<NN, 3>), grid, block, ssd_group_lds(NN * 32, waves, true), stream, a);
     TLF_LAUNCH((ssd_group_kernel<NN, 2>), grid, block, ssd_group_lds(NN * 32, waves, false), stream, a);
   }
   return launch_status();
