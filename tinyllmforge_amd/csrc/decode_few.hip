@@ -6,7 +6,8 @@
 //   one workgroup per (share of a sequence, KV head, sequence), 16 teams of 16 lanes; a team takes every 16th token of the share, 8 dimensions a
 //   lane, and asks for four tokens' rows of K and V at once, which is a whole share up to 64 tokens.  While they are on their way every
 //   workgroup norms and rotates the queries of its KV head and the new token's K and V, and takes these where a token's row is the one they go to;
-//   the share with the newest token stores them.  Scores and sums in fp32 on the vector ALU; partial results (maximum, sum, mix) per share, merged by a second kernel.
+//   the share with the newest token stores them, and so does one with a page that another row's new token goes to (rows of one sequence).  Scores and sums in
+//   fp32 on the vector ALU; partial results (maximum, sum, mix) per share, merged by a second kernel.
 //
 // Qwen3-8B shape (32 heads on 8), one sequence of 700 tokens, us: preparation 4.6, attention 9.5 on 12 workgroups, merge 3.9 before; layer 67.0 -> 60.7.
 #include "qknorm_rope.h"
