@@ -68,6 +68,18 @@ def test_projection_rows_against_separate_kernels_and_fp64(hq, hkv, bs, ctxs, fp
     torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2 ** -13)
 
 
+@pytest.mark.parametrize("hq,hkv,ctxs", [(32, 8, [700]), (32, 8, [8000, 1000, 2000, 5000]), (16, 8, [3000, 700, 64, 1500, 900, 2048, 333, 2999]), (64, 8, [4096]), (16, 16, [3000, 400])])
+def test_results_are_no_further_from_64_bits_than_the_other_kernels(hq, hkv, ctxs):
+    """The share of results that are not the nearest bfloat16 value: a layer's outputs may change by roundings where it takes the other kernel, and not more."""
+    qkv, k, v, ctx, bt, _, _, _, _, _ = step(ctxs, hq, hkv, 256, False, seed=1)
+    q = qkv[:, :hq * 128].contiguous()
+    nearest = exact(q, k, v, ctxs, bt, hq, hkv, (None, None)).to(BF)
+    off = lambda t: (t != nearest).double().mean().item()
+    few, other = ops.decode_few(q, hq, k, v, ctx, bt, SCALE), ops.paged_decode_attention(q.view(len(ctxs), hq, 128), k, v, ctx, bt, SCALE)
+    # fp32 weights against pairs of 16 bits: a result within 2^-17 of its values' size of a border may go either way, 2^-8 of them in bfloat16
+    assert off(few) <= max(off(other), 2 ** -9) and off(few) < 2 ** -9
+
+
 def test_rows_that_are_not_the_newest_token_come_from_the_cache():
     """Without a slot position context_len - 1 is read from the cache, with an earlier row's slot that row is the new one; an
     unmapped page reads as zeros; positions without cosines leave a head as normed."""
