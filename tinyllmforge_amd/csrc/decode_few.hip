@@ -372,7 +372,8 @@ extern "C" int tlf_decode_few_supported(int32_t batch, int32_t num_q_heads, int3
 //                     65536 115 / 123;  3 of 700 33.3 / 29.5, 8192 59.8 / 48.2, 16384 72.4 / 76.5;  4 of 700 34.8 / 30.1, 8192 59.0 / 54.0, 16384 71.1 / 78.4
 //   16 heads on 8     1 of 700 28.6 / 22.7, 65536 110 / 76;  2 of 32768 82.6 / 68.4;  4 of 8192 52.9 / 46.4, 16384 65.6 / 69.0;  8 of 700 32.1 / 27.3,
 //                     8192 54.6 / 49.1, 16384 87.2 / 90.4
-//   64 heads on 8     1 of 700 38.2 / 35.1, 32768 102 / 92;  2 of 700 39.1 / 35.8, 8192 67.2 / 64.5, 16384 80.9 / 93.8;  4 of 700 41.7 / 39.9, 4096 54.5 / 50.4, 8192 67.2 / 72.3
+//   64 heads on 8     1 of 700 38.2 / 35.1, 32768 102 / 92;  2 of 700 39.1 / 35.8, 8192 67.2 / 64.5, 16384 80.9 / 93.8;  3 of 700 39.9 / 39.5, 4096 54.0 / 54.8;
+//                     4 of 700 41.7 / 39.9, 4096 54.5 / 50.4, 8192 67.2 / 72.3 (32 on 4 34.4 / 33.9 of 1000, 43.6 / 45.4 of 4096: up to there it is as good either way)
 //   16 heads on 16    1 of 700 40.1 / 25.0, 65536 171 / 132;  4 of 700 42.0 / 28.2, 8192 83.7 / 56.6, 32768 176 / 150 (8 on 8 91 / 109)
 extern "C" int tlf_decode_few_preferred(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_blocks) {
   if (!tlf_decode_few_supported(batch, num_q_heads, num_kv_heads, head_dim, block_size)) return 0;
