@@ -557,7 +557,11 @@ int tlf_f32_argmax(const float *logits, int64_t row_stride, int64_t *out, int32_
  *   out = 0.  pool_new: also write the pooled row of a block that a row's own token completes (decode).
  *   max_len bounds the positions.  out rows: Hq * head_dim values.
  * tlf_pooled_attn_prefill: bf16 matrix-core kernel for the portions of sequences first_seq .. + num_seqs - 1 (all other
- *   arguments as above; q, gate and out are indexed by the step's rows). */
+ *   arguments as above; q, gate and out are indexed by the step's rows).
+ * tlf_pooled_attn_portions: the portions of sequences first_seq .. + num_seqs - 1 from the projection, bf16: keys, values and pooled
+ *   rows are stored, queries and gates made where they are read; what tlf_attn_prep, tlf_pool_blocks and tlf_pooled_attn_prefill
+ *   give together.  head_dim <= 128; head_dim, rot_dims and proj_stride multiples of 8, proj, biases and cos_sin aligned to
+ *   16 bytes (TLF_E_UNSUPPORTED otherwise). */
 int tlf_attn_prep(const void *proj, int64_t proj_stride, const float *partials, int32_t splits, const float *scale,
                   const void *q_bias, const void *k_bias,
                   const int64_t *positions, const float *cos_sin, int32_t max_pos, int32_t rot_dims,
@@ -585,6 +589,13 @@ int tlf_pooled_attn_prefill(const void *q, const void *score_bias, const float *
                             void *out, int64_t out_stride, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                             int32_t block_size, int32_t pool, int32_t window, int64_t num_pages, float scale,
                             void *stream);
+
+int tlf_pooled_attn_portions(const void *proj, int64_t proj_stride, const void *q_bias, const void *k_bias, const int64_t *positions,
+                             const float *cos_sin, int32_t max_pos, int32_t rot_dims, const int32_t *slot_mapping, const void *score_bias,
+                             void *k_cache, void *v_cache, void *pk_cache, void *pv_cache, const int32_t *block_tables, int64_t bt_stride,
+                             const int32_t *cu_seqlens_q, const int32_t *seq_starts, int32_t first_seq, int32_t num_seqs, int32_t max_tokens,
+                             void *out, int64_t out_stride, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                             int32_t pool, int32_t window, int64_t num_pages, float scale, float eps, void *stream);
 
 /* Gated linear attention with a decay per key channel.  Projection rows are [q | k | v | g | r] (heads * key_dim twice,
  * heads * value_dim twice, rank values).  Per head, state S [key_dim, value_dim] fp32 at state[slot, head]:

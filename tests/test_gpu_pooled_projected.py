@@ -1,0 +1,108 @@
+"""Portions of pooled-window attention whose queries are made where they are read, against the separate preparation."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+import torch
+
+from tinyllmforge_amd import ops
+from tinyllmforge_amd.engine.inputs import portion_inputs
+from tinyllmforge_amd.layers.pooled_attention import PooledWindowAttention
+from tinyllmforge_amd.layers.rotary_embedding import rotation_table
+from tinyllmforge_amd.utils.context import reset_context, set_portions_context
+
+BF16 = torch.bfloat16
+
+
+class Sized(SimpleNamespace):
+    def __len__(self):
+        return self.size
+
+
+def layer_of(H, G, D, rot, size, pool, pages, seed, scale):
+    g = torch.Generator().manual_seed(seed)
+    layer = PooledWindowAttention(H, G, D, scale, size, pool, rot, rotation_table(rot, 2048, 1e4).cuda(), 1e-6, BF16)
+    layer.score_bias.data = torch.randn(H, generator=g).to(BF16).cuda() - 2
+    layer.bind_pages(pages, 64, "cuda")
+    for t in (layer.kv.k, layer.kv.v, layer.kv.pk, layer.kv.pv):
+        t.fill_(3.0)
+        t[..., D:] = 0
+    return layer
+
+
+def steps_of(lens, schedule):
+    """Context fields of each step: ``schedule``: lists of (sequence, tokens), single tokens first."""
+    rng = np.random.RandomState(len(lens))
+    free = list(rng.permutation(sum(-(-n // 64) for n in lens) + 2))
+    tables = [[int(free.pop()) for _ in range(-(-n // 64))] for n in lens]
+    done = [0] * len(lens)
+    for parts in schedule:
+        seqs = [Sized(num_scheduled=n, num_computed=done[s], num_cached_tokens=done[s], num_cached_blocks=done[s] // 64, token_ids=range(done[s] + n),
+                      last_token=0, block_table=tables[s][:-(-(done[s] + n) // 64)], state_slot=s, size=done[s] + n) for s, n in parts]
+        fields = {k: torch.from_numpy(v).cuda() if isinstance(v, np.ndarray) else v for k, v in portion_inputs(seqs, 64, None, ()).items()}
+        fields.pop("input_ids")
+        for s, n in parts:
+            done[s] += n
+        yield fields
+
+
+# heads, KV heads, dimensions, rotated ones, window, pool, biases
+FORMS = [(4, 2, 40, 24, 37, 5, True), (8, 8, 128, 128, 64, 16, True), (6, 2, 64, 0, 100, 8, False), (20, 1, 96, 32, 130, 100, True),
+         (2, 2, 8, 8, 1, 1, False), (32, 8, 128, 64, 80, 17, True), (9, 3, 32, 32, 20, 33, False)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,rot,size,pool,biased", FORMS)
+def test_projected_portions_are_the_prepared_ones(monkeypatch, H, G, D, rot, size, pool, biased):
+    lens = [150, 67, 210]
+    schedules = [[[(0, 150), (1, 67), (2, 210)]],
+                 [[(0, 2), (1, 3)], [(0, 62), (2, 130)], [(0, 1), (1, 2), (2, 2)], [(0, 85), (1, 62), (2, 78)]],
+                 [[(0, 100), (2, 64)], [(0, 1), (2, 1), (1, 20)], [(0, 1), (1, 1), (2, 145)], [(0, 48), (1, 46)]]]
+    pages = sum(-(-n // 64) for n in lens) + 2
+    width = -(-((H + G) * D + H) // 8) * 8 + 8                # rows of a wider array
+    for i, schedule in enumerate(schedules):
+        g = torch.Generator().manual_seed(i)
+        r = lambda *s: torch.randn(*s, generator=g).to(BF16).cuda()
+        qb, kb = (r(H * D), r(G * D)) if biased else (None, None)
+        new, old = (layer_of(H, G, D, rot, size, pool, pages, i, 1.5 / D ** 0.5) for _ in range(2))
+        for fields in steps_of(lens, schedule):
+            positions = fields.pop("positions")
+            proj = r(positions.numel(), width)[:, :(H + G) * D + H]
+            outs, taken = [], []
+            real = ops.pooled_attention_projected
+            for layer, form in ((new, lambda *a: taken.append(real(*a)) or taken[-1]), (old, lambda *a: False)):
+                monkeypatch.setattr(ops, "pooled_attention_projected", form)
+                set_portions_context(**fields, max_len=256)
+                outs.append(layer(proj, qb, kb, positions))
+                reset_context()
+            monkeypatch.undo()
+            assert taken == [True]
+            assert torch.equal(new.kv.v, old.kv.v) and torch.equal(new.kv.pv, old.kv.pv)
+            for a, b in ((new.kv.k, old.kv.k), (new.kv.pk, old.kv.pk)):
+                # the rotation's products are rounded at other places: values on the border of two bf16 numbers become either
+                assert ((a.float() - b.float()).abs() <= 2 ** -7 * b.float().abs() + 1e-6).all() and (a != b).float().mean() < 2e-3
+            # fewer than one key or query in a few hundred differs, and by half a unit in the last place of 2^-8: below the results' own rounding
+            assert (outs[0].float() - outs[1].float()).norm() <= 2e-3 * outs[1].float().norm()
+
+
+@pytest.mark.gpu
+def test_rows_that_are_not_read_eight_at_a_time_are_prepared():
+    """Refused, before anything is launched, and the layer prepares such rows apart."""
+    fields = next(steps_of([70], [[(0, 70)]]))
+    positions = fields.pop("positions")
+    t = lambda *s: torch.randn(*s).to(BF16).cuda()
+    for D, rot, width, first, biases, dtype, takes in ((32, 32, 80, 0, (64, 0), BF16, True), (32, 32, 84, 0, (64, 0), BF16, False),
+                                                       (32, 32, 80, 4, (64, 0), BF16, False), (32, 32, 80, 0, (64, 4), BF16, False),
+                                                       (32, 20, 80, 0, (64, 0), BF16, False), (36, 32, 120, 0, (72, 0), BF16, False),
+                                                       (160, 32, 328, 0, (320, 0), BF16, False)):
+        layer = layer_of(1, 1, D, rot, 20, 8, 5, 0, 0.2)
+        proj, qb = t(71, width)[:, first:first + 2 * D + 1][:70], t(D + 8)[biases[1]:biases[1] + D]
+        out = torch.full((70, D), 5.0, dtype=BF16, device="cuda")
+        before = layer.kv.k.clone()
+        args = (positions, layer.cos_sin, rot, fields["slot_mapping"], layer.score_bias.data, layer.kv, fields["block_tables"], fields["cu_seqlens_q"],
+                fields["seq_starts"], 0, 1, 70, 0.2, 1e-6, out)
+        assert ops.pooled_attention_projected(proj, qb, None, *args) == takes
+        assert takes or ((out == 5).all() and torch.equal(layer.kv.k, before))
+        set_portions_context(**fields, max_len=128)
+        assert layer(proj, qb, None, positions).isfinite().all()
+        reset_context()

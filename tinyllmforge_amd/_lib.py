@@ -18,6 +18,7 @@ KV_BF16 = 0
 KV_FP8_E4M3 = 1
 DT_BF16 = 0
 DT_F32 = 1
+E_UNSUPPORTED = -5
 
 _P, _I32, _I64, _F, _SZ = c_void_p, c_int32, c_int64, c_float, c_size_t
 
@@ -90,6 +91,8 @@ SIGNATURES = {
                                        _I32, _I32, _I32, _I32, _I64, _F, _I32, _I32, _P, _SZ, _P]),
     "tlf_pooled_attn_prefill": (c_int32, [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _I32, _I32, _I32, _P, _I64,
                                           _I32, _I32, _I32, _I32, _I32, _I32, _I64, _F, _P]),
+    "tlf_pooled_attn_portions": (c_int32, [_P, _I64, _P, _P, _P, _P, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _I32, _I32, _I32, _P, _I64,
+                                           _I32, _I32, _I32, _I32, _I32, _I32, _I64, _F, _F, _P]),
     "tlf_gla_decode": (c_int32, [_P, _I64, _P, _I32, _P, _P, _P, _P, _P, _P, _I32, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _F, _F,
                                  _F, _I32, _P]),
     "tlf_gla_portions_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32, _I32, _I32]),

@@ -142,6 +142,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VC <= 
   // tiles between the window's edge and the diagonal hide nothing from any of the wave's rows
   const int to = max(0, wave_last - w0) / kPK + 1;
   const int edge = wave_last - p.window >= w0 ? (wave_last - p.window - w0) / kPK + 1 : 0;
+  copy(0, PromptPart<true, true>{});
   core.template walk<true, true>(
       tiles, min(max(0, wave_first - p.window + 1 - w0) / kPK, to - 1), to, edge, min(tiles, max(0, (wave_first + 1 - w0) / kPK)), copy,
       []() __attribute__((always_inline)) { return Core::all(0.f); },

@@ -75,4 +75,42 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 int pooled_cache_check(const PooledCache &c, int32_t dtype);
 
+// What turns rows of a bf16 projection [q heads | k heads | a gate value per q head] into queries, keys and values.
+struct PooledProj {
+  const unsigned short *rows;   // [n, ld]
+  int64_t ld;
+  const unsigned short *q_bias, *k_bias;     // NULL: none
+  const int64_t *positions;
+  const float *cos_sin;         // [max_pos, rot_dims]: cos of the pairs, then sin
+  int32_t max_pos, rot_dims;
+  float eps;
+};
+// Whether rows are read eight values at a time.
+inline bool pooled_proj_takes(const PooledProj &p, int32_t head_dim) {
+  return head_dim % 8 == 0 && head_dim <= 128 && p.rot_dims % 8 == 0 && p.ld % 8 == 0 && aligned16(p.rows) && aligned16(p.q_bias) && aligned16(p.k_bias) &&
+         aligned16(p.cos_sin);
+}
+// Keys, values and pooled rows of portions (pooled_attn.hip); of p, what keys are made from.
+int launch_pooled_kv(const PooledCache &c, const PooledProj &p, const int32_t *slots, const int32_t *cu_q, const int32_t *starts, int first_seq, int num_seqs,
+                     int max_tokens, int H, hipStream_t stream);
+// The pairs of dimensions 8 ch .. 8 ch + 7 turned.
+__device__ __forceinline__ void pooled_rotate(float (&x)[8], const float4 &co, const float4 &si) {
+  const float cv[4] = {co.x, co.y, co.z, co.w}, sv[4] = {si.x, si.y, si.z, si.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float u = x[2 * e], v = x[2 * e + 1];
+    x[2 * e] = fmaf(u, cv[e], -(v * sv[e]));
+    x[2 * e + 1] = fmaf(v, cv[e], u * sv[e]);
+  }
+}
+__device__ __forceinline__ void pooled_angles(const PooledProj &p, int64_t pos, int ch, float4 &co, float4 &si) {
+  co = make_float4(1.f, 1.f, 1.f, 1.f);
+  si = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (pos >= 0 && pos < p.max_pos && ch * 8 < p.rot_dims) {
+    const float *cs = p.cos_sin + pos * p.rot_dims + ch * 4;
+    co = *reinterpret_cast<const float4 *>(cs);
+    si = *reinterpret_cast<const float4 *>(cs + p.rot_dims / 2);
+  }
+}
+
 }  // namespace tlf

@@ -5,6 +5,7 @@
 //   attn_prep_kernel    projection row [q | k | gate] -> biases, V store (the projected key), interleaved RoPE on the
 //                       first rot_dims dimensions, unit RMS per head, K store, q, sigmoid of the per-head gate
 //   pool_blocks_kernel  means of the blocks that a step's prompt portions complete
+//   pooled_kv_kernel    for portions, both for keys and values alone
 //   rows_kernel         one workgroup per (query row, KV head, split of the keys): decode, and every row in 32-bit mode
 //   rows_merge_kernel   sum of the splits (the weights are not normalised, so partial outputs just add) and the gate
 #include <algorithm>
@@ -245,6 +246,99 @@ __global__ __launch_bounds__(256) void pool_blocks_kernel(const PooledCache c, c
   if (b < last) pool_block_chunk<T>(c, bt, b, t / per, t % per);
 }
 
+// Keys and values of prompt portions from the projection, and the means of the blocks that they complete: a wave takes a KV head's tokens of one
+// block, 16 lanes a quarter of them, eight dimensions a lane.  Queries are made where they are read (pooled_prefill.hip).
+//
+// Eight prompts of 1061 to 2048 tokens, 8 KV heads of 128, blocks of 16: 25 MB read and 53 written in some 10 us.  With 16 lanes for a whole block, one or
+// two waves on a SIMD, a layer took 272 us where it takes 262 so (285 with all 16 tokens' loads under way at once), and one prompt of 203 tokens behind
+// 320 took 36 and takes 27: the tokens of a lane come one after the other.
+struct PooledKvArgs {
+  PooledCache c;
+  PooledProj p;
+  const int32_t *slots, *cu_q, *starts;
+  int64_t num_slots;
+  int32_t first_seq, H;
+};
+
+__global__ __launch_bounds__(256) void pooled_kv_kernel(const PooledKvArgs a) {
+  constexpr int kBatch = 4;                                  // tokens whose loads are under way at once
+  const PooledCache &c = a.c;
+  const int seq = a.first_seq + blockIdx.y, q0 = a.cu_q[seq], n = a.cu_q[seq + 1] - q0, start = a.starts[seq];
+  const int lane = threadIdx.x & 63, wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = lane % 16, quarter = lane / 16, b = start / c.pool + wave / c.G, head = wave % c.G;
+  if (n <= 0 || b > (start + n - 1) / c.pool) return;        // whole waves leave together
+  const int32_t *bt = c.bt + seq * c.bt_stride;
+  const int col = min(j * 8, c.D - 8), per = (c.pool + 3) / 4, first = b * c.pool + quarter * per, end = min((b + 1) * c.pool, first + per);
+  const bool mine = j * 8 < c.Dp, real = j * 8 < c.D;
+  const bool whole = (b + 1) * c.pool <= start + n;          // its mean is due
+  const unsigned short *rows = a.p.rows + static_cast<int64_t>(a.H + head) * c.D + col;
+  unsigned short *kc = static_cast<unsigned short *>(const_cast<void *>(c.k)), *vc = static_cast<unsigned short *>(const_cast<void *>(c.v));
+  float bias[8], ks[8], vs[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) bias[e] = ks[e] = vs[e] = 0.f;
+  if (a.p.k_bias) Elem<unsigned short>::ld8(a.p.k_bias + head * c.D + col, bias);
+  const int64_t rs = static_cast<int64_t>(c.G) * c.Dp;
+  for (int r0 = 0; r0 < per; r0 += kBatch) {
+    uint4 raw[kBatch];
+    int64_t slot[kBatch];
+    float4 co[kBatch], si[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const int64_t tok = q0 + min(max(first + r0 + k - start, 0), n - 1);
+      raw[k] = *reinterpret_cast<const uint4 *>(rows + tok * a.p.ld);
+      slot[k] = a.slots[tok];
+      pooled_angles(a.p, a.p.positions[tok], j, co[k], si[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const int at = first + r0 + k;
+      float x[8], ss = 0.f;
+      unpack8(raw[k], x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = real ? x[e] + bias[e] : 0.f;
+      uint4 vr = pack8(x);
+      pooled_rotate(x, co[k], si[k]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
+      ss = group_sum<16>(ss);
+      const float inv = 1.0f / sqrtf(ss / static_cast<float>(c.D) + a.p.eps);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] *= inv;
+      uint4 kr = pack8(x);
+      if (at >= end || at >= start + n) continue;
+      if (at >= start && slot[k] >= 0 && slot[k] < a.num_slots) {
+        const int64_t to = (slot[k] * c.G + head) * c.Dp + j * 8;
+        if (mine) {
+          *reinterpret_cast<uint4 *>(vc + to) = vr;
+          *reinterpret_cast<uint4 *>(kc + to) = kr;
+        }
+      } else if (whole) {                                    // of an earlier portion
+        const int64_t from = token_row(c, bt, at) * rs + head * c.Dp + (mine ? j * 8 : 0);
+        kr = *reinterpret_cast<const uint4 *>(kc + from);
+        vr = *reinterpret_cast<const uint4 *>(vc + from);
+      }
+      float kf[8], vf[8];
+      unpack8(kr, kf);
+      unpack8(vr, vf);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        ks[e] += kf[e];
+        vs[e] += vf[e];
+      }
+    }
+  }
+  if (!whole) return;
+  const float inv = 1.0f / static_cast<float>(c.pool);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    ks[e] = sum_lanes_16_32_48(ks[e]) * inv;
+    vs[e] = sum_lanes_16_32_48(vs[e]) * inv;
+  }
+  if (!mine || quarter > 1) return;
+  const int64_t to = block_row(c, bt, b) * rs + head * c.Dp + j * 8;
+  Elem<unsigned short>::st8(static_cast<unsigned short *>(const_cast<void *>(quarter ? c.pv : c.pk)) + to, quarter ? vs : ks);
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 struct RowsArgs {
   PooledCache c;
@@ -451,6 +545,17 @@ extern "C" int tlf_pool_blocks(const void *k_cache, const void *v_cache, void *p
   else TLF_LAUNCH((pool_blocks_kernel<float>), grid, dim3(256), 0, s, c, cu_seqlens_q, seq_starts, first_seq);
   return launch_status();
 }
+
+namespace tlf {
+int launch_pooled_kv(const PooledCache &c, const PooledProj &p, const int32_t *slots, const int32_t *cu_q, const int32_t *starts, int first_seq, int num_seqs,
+                     int max_tokens, int H, hipStream_t stream) {
+  const int64_t waves = (static_cast<int64_t>(max_tokens - 1) / c.pool + 2) * c.G;           // a portion may begin inside a block
+  const dim3 grid(static_cast<unsigned>((waves + 3) / 4), num_seqs);
+  const PooledKvArgs a{c, p, slots, cu_q, starts, c.pages * c.bs, first_seq, H};
+  TLF_LAUNCH(pooled_kv_kernel, grid, dim3(256), 0, stream, a);
+  return launch_status();
+}
+}  // namespace tlf
 
 extern "C" size_t tlf_pooled_attn_rows_workspace_bytes(int32_t rows, int32_t num_q_heads, int32_t num_kv_heads,
                                                        int32_t head_dim, int32_t pool, int32_t window, int32_t max_len) {

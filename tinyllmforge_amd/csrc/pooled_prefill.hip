@@ -7,7 +7,13 @@
 //   P = sigmoid(S * scale + bias)  fp32, masked on the pooled tiles and on those that a window's or the diagonal's edge cuts
 // The weights are not normalised: no maximum, no rescaling, no second pass.  Bound by the vector ALU: two quarter-rate operations
 // per score.  Eight prompts of 1061 to 2048 tokens, 32 heads of 128 on 8 KV heads, window 1024: layer 372 us with the stages of a tile
-// one after the other (and the staging registers, which the compiler had put in LDS), 296 with three stages side by side, 286 so.
+// one after the other (and the staging registers, which the compiler had put in LDS), 296 with three stages side by side, 286 - 293 in
+// prompt_core.h's.
+//
+// Where rows of the projection can be read eight values at a time, queries and gates are made from them here, by the one workgroup that reads them
+// (PROJ): 12240 tokens write and read 200 MB less, and a layer has two launches in place of three.  Eight prompts as above 285 -> 262 us: preparing
+// and pooling took 55 + 13, keys and values alone take some 10 (pooled_attn.hip: pooled_kv_kernel); making queries adds 27 to the launch, 17 of them
+// waiting for rows that come from memory instead of the caches and the norm, 10 biases and rotation.  One prompt of up to 320 tokens 30 -> 21.
 #include "pooled_attn.h"
 #include "prompt_core.h"
 #include "prompt_tiles.h"
@@ -21,6 +27,7 @@ struct PooledPrefillArgs {
   const unsigned short *q;     // [rows, H, Dp]
   const unsigned short *bias;  // [H]
   const float *gate;           // [rows, H]
+  PooledProj proj;             // or what both are made from
   const int32_t *cu_q, *starts;
   unsigned short *out;
   int64_t ldo;
@@ -63,7 +70,7 @@ __device__ __forceinline__ void pooled_finish(const PooledPrefillArgs &p, const 
   }
 }
 
-template <int DC>
+template <int DC, bool PROJ>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void pooled_prefill_kernel(const PooledPrefillArgs p) {
   using Core = PromptCore<DC, DC>;
   __shared__ __attribute__((aligned(1024))) unsigned char Ks[2][Core::KB], Vs[2][Core::VB];
@@ -89,13 +96,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   const int upos = start + row, unb = pooled_visible(upos, c.size, c.pool);
   const int64_t unit = static_cast<int64_t>(q0 + row) * p.H + head;
   const float pb = -kLog2e * bf16_bits_to_float(p.bias[head]), nscale = -p.scale_log2;
-  const unsigned short *qp = p.q + unit * Core::DP + g * 8;
+  const unsigned short *qp = PROJ ? p.proj.rows + static_cast<int64_t>(q0 + row) * p.proj.ld + head * c.D : p.q + unit * Core::DP;
+  const int64_t pos = PROJ ? p.proj.positions[q0 + row] : 0;
+  uint4 raw[2 * DC];                                         // of this lane's pieces of 8, every other one of the row
 #pragma unroll
-  for (int kc = 0; kc < 2 * DC; ++kc) {
-    Pack16 t;
-    t.u = *reinterpret_cast<const uint4 *>(qp + kc * 16);
-    core.qf[kc] = t.v;
-  }
+  for (int kc = 0; kc < 2 * DC; ++kc) raw[kc] = *reinterpret_cast<const uint4 *>(qp + (PROJ ? min(kc * 16 + g * 8, c.D - 8) : kc * 16 + g * 8));
 
   const int nb = pooled_visible(i_last, c.size, c.pool);
   const int ptiles = (nb + kTK - 1) / kTK;
@@ -135,6 +140,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
     for (int i = 0; i < DC; ++i) prompt_copy(voff[i], vc_ + from, core.v_place(t, i));
   };
+  if constexpr (PROJ) {
+    float4 co[2 * DC], si[2 * DC];
+#pragma unroll
+    for (int kc = 0; kc < 2 * DC; ++kc) pooled_angles(p.proj, pos, kc * 2 + g, co[kc], si[kc]);
+    copy(0, PromptPart<true, true>{});
+    float x[2 * DC][8], ss = 0.f;
+#pragma unroll
+    for (int kc = 0; kc < 2 * DC; ++kc) {
+      const int col = kc * 16 + g * 8;
+      unpack8(raw[kc], x[kc]);
+      if (p.proj.q_bias) {
+        float b[8];
+        unpack8(*reinterpret_cast<const uint4 *>(p.proj.q_bias + head * c.D + min(col, c.D - 8)), b);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[kc][e] += b[e];
+      }
+      pooled_rotate(x[kc], co[kc], si[kc]);
+      if (col >= c.D) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[kc][e] = 0.f;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = fmaf(x[kc][e], x[kc][e], ss);
+    }
+    const float inv = 1.0f / sqrtf(prompt_unit_sum(ss) / static_cast<float>(c.D) + p.proj.eps);
+#pragma unroll
+    for (int kc = 0; kc < 2 * DC; ++kc) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[kc][e] *= inv;
+      raw[kc] = pack8(x[kc]);
+    }
+  } else {
+    copy(0, PromptPart<true, true>{});
+  }
+#pragma unroll
+  for (int kc = 0; kc < 2 * DC; ++kc) core.qf[kc] = __builtin_bit_cast(bf16x8, raw[kc]);
   // tiles between the window's edge and the diagonal hide nothing from anyone
   const int edge = i_last - c.size >= w0 ? (i_last - c.size - w0) / kTK + 1 : 0;
   core.template walk<true, false>(
@@ -157,7 +198,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
       });
 
   if (!uok) return;
-  const float gt = p.gate[unit];
+  const float gt = PROJ ? sigmoid_f32(bf16_bits_to_float(p.proj.rows[static_cast<int64_t>(q0 + row) * p.proj.ld + static_cast<int64_t>(p.H + c.G) * c.D + head])) : p.gate[unit];
   unsigned short *o = p.out + static_cast<int64_t>(q0 + row) * p.ldo + static_cast<int64_t>(head) * c.D;
   const uintptr_t to = reinterpret_cast<uintptr_t>(p.out);
   core.store(o, c.D, (c.D & 3) == 0 && (p.ldo & 3) == 0 && (to & 7) == 0, (c.D & 7) == 0 && (p.ldo & 7) == 0 && (to & 15) == 0, g,
@@ -328,6 +369,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   pooled_finish<DC, CT>(p, acc, uok, uoff, g);
 }
 
+namespace {
+int launch_pooled_prefill(PooledPrefillArgs &a, int num_seqs, int max_tokens, hipStream_t s) {
+  const PooledCache &c = a.c;
+  const int dc = c.Dp / 32, ct = dc <= 4 ? 2 : 1, units = 64 * ct;
+  a.group = a.H / c.G;
+  a.hpp = a.group < units ? a.group : units;
+  a.passes = (a.group + a.hpp - 1) / a.hpp;
+  a.bq = units / a.hpp;
+  const int blocks = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, c.G * a.passes, num_seqs);
+  const dim3 grid = prompt_grid<dim3>(blocks);
+  if (!blocks) return TLF_E_SHAPE;
+#define TLF_POOLED(DC)                                                                             \
+  do {                                                                                             \
+    if (a.proj.rows) TLF_LAUNCH((pooled_prefill_kernel<DC, true>), grid, dim3(256), 0, s, a);      \
+    else TLF_LAUNCH((pooled_prefill_kernel<DC, false>), grid, dim3(256), 0, s, a);                 \
+  } while (0)
+  switch (dc) {
+    case 1: TLF_POOLED(1); break;
+    case 2: TLF_POOLED(2); break;
+    case 3: TLF_POOLED(3); break;
+    case 4: TLF_POOLED(4); break;
+    case 5: TLF_LAUNCH((pooled_prefill_wide_kernel<5, 1>), grid, dim3(256), 0, s, a); break;
+    case 6: TLF_LAUNCH((pooled_prefill_wide_kernel<6, 1>), grid, dim3(256), 0, s, a); break;
+    case 7: TLF_LAUNCH((pooled_prefill_wide_kernel<7, 1>), grid, dim3(256), 0, s, a); break;
+    default: TLF_LAUNCH((pooled_prefill_wide_kernel<8, 1>), grid, dim3(256), 0, s, a); break;
+  }
+#undef TLF_POOLED
+  return launch_status();
+}
+}  // namespace
+
 }  // namespace tlf
 
 extern "C" int tlf_pooled_attn_prefill(const void *q, const void *score_bias, const float *gate, const void *k_cache,
@@ -348,26 +420,37 @@ extern "C" int tlf_pooled_attn_prefill(const void *q, const void *score_bias, co
   if (!q || !score_bias || !gate || !cu_seqlens_q || !seq_starts || !out) return TLF_E_NULL;
   if (!aligned16(q)) return TLF_E_ALIGN;
   pooled_cache_finish(c);
-  const int dc = c.Dp / 32, ct = dc <= 4 ? 2 : 1, units = 64 * ct;
-  PooledPrefillArgs a{c, static_cast<const unsigned short *>(q), static_cast<const unsigned short *>(score_bias), gate,
+  PooledPrefillArgs a{c, static_cast<const unsigned short *>(q), static_cast<const unsigned short *>(score_bias), gate, {},
                       cu_seqlens_q, seq_starts, static_cast<unsigned short *>(out), out_stride, num_q_heads,
-                      num_q_heads / num_kv_heads, 0, 0, 0, first_seq, {}, scale * kLog2e};
-  a.hpp = a.group < units ? a.group : units;
-  a.passes = (a.group + a.hpp - 1) / a.hpp;
-  a.bq = units / a.hpp;
-  const int blocks = prompt_tiles_make(a.tiles, (max_tokens + a.bq - 1) / a.bq, num_kv_heads * a.passes, num_seqs);
-  const dim3 grid = prompt_grid<dim3>(blocks);
-  if (!blocks) return TLF_E_SHAPE;
+                      0, 0, 0, 0, first_seq, {}, scale * kLog2e};
+  return launch_pooled_prefill(a, num_seqs, max_tokens, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tlf_pooled_attn_portions(const void *proj, int64_t proj_stride, const void *q_bias, const void *k_bias, const int64_t *positions,
+                                        const float *cos_sin, int32_t max_pos, int32_t rot_dims, const int32_t *slot_mapping, const void *score_bias,
+                                        void *k_cache, void *v_cache, void *pk_cache, void *pv_cache, const int32_t *block_tables, int64_t bt_stride,
+                                        const int32_t *cu_seqlens_q, const int32_t *seq_starts, int32_t first_seq, int32_t num_seqs, int32_t max_tokens,
+                                        void *out, int64_t out_stride, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                        int32_t pool, int32_t window, int64_t num_pages, float scale, float eps, void *stream) {
+  using namespace tlf;
+  if (num_seqs < 0 || num_seqs > 65535 || max_tokens < 0 || first_seq < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads)
+    return TLF_E_SHAPE;
+  if (out_stride < static_cast<int64_t>(num_q_heads) * head_dim) return TLF_E_SHAPE;
+  if (num_seqs == 0 || max_tokens == 0) return TLF_OK;
+  PooledCache c{k_cache, v_cache, pk_cache, pv_cache, block_tables, bt_stride, block_size, pool, 0, window,
+                num_kv_heads, head_dim, (head_dim + 31) / 32 * 32, num_pages, -1};
+  if (int rc = pooled_cache_check(c, TLF_DT_BF16)) return rc;
+  if (rot_dims < 0 || rot_dims % 2 || rot_dims > head_dim) return TLF_E_SHAPE;
+  if (proj_stride < static_cast<int64_t>(num_q_heads + num_kv_heads) * head_dim + num_q_heads) return TLF_E_SHAPE;
+  if (!proj || !positions || (rot_dims && !cos_sin) || !slot_mapping || !score_bias || !cu_seqlens_q || !seq_starts || !out) return TLF_E_NULL;
+  pooled_cache_finish(c);
+  const PooledProj p{static_cast<const unsigned short *>(proj), proj_stride, static_cast<const unsigned short *>(q_bias),
+                     static_cast<const unsigned short *>(k_bias), positions, cos_sin, max_pos, rot_dims, eps};
+  if (!pooled_proj_takes(p, head_dim)) return TLF_E_UNSUPPORTED;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (dc) {
-    case 1: TLF_LAUNCH((pooled_prefill_kernel<1>), grid, dim3(256), 0, s, a); break;
-    case 2: TLF_LAUNCH((pooled_prefill_kernel<2>), grid, dim3(256), 0, s, a); break;
-    case 3: TLF_LAUNCH((pooled_prefill_kernel<3>), grid, dim3(256), 0, s, a); break;
-    case 4: TLF_LAUNCH((pooled_prefill_kernel<4>), grid, dim3(256), 0, s, a); break;
-    case 5: TLF_LAUNCH((pooled_prefill_wide_kernel<5, 1>), grid, dim3(256), 0, s, a); break;
-    case 6: TLF_LAUNCH((pooled_prefill_wide_kernel<6, 1>), grid, dim3(256), 0, s, a); break;
-    case 7: TLF_LAUNCH((pooled_prefill_wide_kernel<7, 1>), grid, dim3(256), 0, s, a); break;
-    default: TLF_LAUNCH((pooled_prefill_wide_kernel<8, 1>), grid, dim3(256), 0, s, a); break;
-  }
-  return launch_status();
+  if (int rc = launch_pooled_kv(c, p, slot_mapping, cu_seqlens_q, seq_starts, first_seq, num_seqs, max_tokens, num_q_heads, s)) return rc;
+  PooledPrefillArgs a{c, nullptr, static_cast<const unsigned short *>(score_bias), nullptr, p,
+                      cu_seqlens_q, seq_starts, static_cast<unsigned short *>(out), out_stride, num_q_heads,
+                      0, 0, 0, 0, first_seq, {}, scale * kLog2e};
+  return launch_pooled_prefill(a, num_seqs, max_tokens, s);
 }

@@ -158,7 +158,7 @@ struct PromptCore {
 
   // The workgroup's walk over `tiles` tiles, of which the wave computes first_tile <= t < end: those that some of its units see.  A value
   // behind or before them, infinite or no number as it may be, does not reach its rows.  The kernel's parts:
-  //   copy(t, part)               the tile's copies; called for t = 0, 1, .. in turn
+  //   copy(t, part)               the tile's copies; called for t = 1, 2, .. in turn, the first one's are under way
   //   from()                      where the unit's scores begin (registers that are kept: set anew for each half they are a ninth of a wave's vector work)
   //   weights(t, hf, s, w, part)  of half hf of tile t, when all values of the halves before are in acc
   // part.mask is not set where all keys of the tile are seen by all units: tiles clear_from <= t < clear_to of them (wave uniform),
@@ -188,7 +188,6 @@ struct PromptCore {
         weights(t, hf, s, w, part);
       }
     };
-    copy(0, first);
     int t = 0;
     if constexpr (LEAD && SOME)
       for (; t < first_tile; ++t) arrive(t, first);

@@ -145,6 +145,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   float m = MODE == 2 ? p.cap_log2 : -INFINITY, l = 0.f;
   float over = -INFINITY;                                    // what a score must not exceed; no key yet
   typename Core::Scores from = Core::all(0.f);               // without a cap: the score less the maximum so far
+  copy(0, PromptPart<false, true>{});
   core.template walk<false, true>(
       tiles, 0, wave_last / kSK + 1, 0, min(tiles, (wave_first + 1) / kSK), copy,                      // the diagonal cuts the tiles behind
       [&]() __attribute__((always_inline)) { return from; },

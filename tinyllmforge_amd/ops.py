@@ -691,8 +691,8 @@ def embed_group_rms_norm(ids, table, w_next, groups, eps, w_offset=0.0):
     return x, h
 
 
-def attn_prep(proj, q_bias, k_bias, positions, cos_sin, rot_dims, slot_mapping, k_cache, v_cache, num_q_heads, head_dim, eps):
-    """Biases, V store, interleaved RoPE, unit RMS, K store.  Returns ``(q [N, Hq, Dp], gate fp32 [N, Hq])``."""
+def attn_prep(proj, q_bias, k_bias, positions, cos_sin, rot_dims, slot_mapping, k_cache, v_cache, num_q_heads, head_dim, eps, rows=None):
+    """Biases, V store, interleaved RoPE, unit RMS, K store, of the first ``rows`` rows or all.  Returns ``(q [N, Hq, Dp], gate fp32 [N, Hq])``."""
     lib = _lib.load()
     assert proj.dtype == k_cache.dtype
     _need(positions, torch.int64, "positions"); _need(slot_mapping, torch.int32, "slot_mapping")
@@ -700,6 +700,9 @@ def attn_prep(proj, q_bias, k_bias, positions, cos_sin, rot_dims, slot_mapping, 
     pages, bs, hkv, dp = k_cache.shape
     assert positions.numel() == n and slot_mapping.numel() == n
     assert k_cache.is_contiguous() and v_cache.is_contiguous() and (rot_dims == 0 or cos_sin.shape[1] == rot_dims)
+    if rows is not None:
+        assert rows <= n and isinstance(proj, torch.Tensor)       # partial sums lie a whole projection apart
+        n = rows
     q = torch.empty(n, num_q_heads, dp, dtype=proj.dtype, device=proj.device)
     gate = torch.empty(n, num_q_heads, dtype=torch.float32, device=proj.device)
     check(lib.tlf_attn_prep(*_source(proj), _opt(q_bias), _opt(k_bias), positions.data_ptr(),
@@ -771,6 +774,30 @@ def pooled_attention_prefill(q, score_bias, gate, kv: PooledKV, block_tables, cu
         first_seq, num_seqs, max_tokens, out.data_ptr(), out.stride(0), hq, hkv, kv.head_dim, bs, kv.pool, kv.window,
         pages, float(scale), _stream()), "tlf_pooled_attn_prefill")
     return out
+
+
+def pooled_attention_projected(proj, q_bias, k_bias, positions, cos_sin, rot_dims, slot_mapping, score_bias, kv: PooledKV, block_tables, cu_seqlens_q,
+                               seq_starts, first_seq, num_seqs, max_tokens, scale, eps, out) -> bool:
+    """Portions of sequences ``first_seq ..`` from their projection ``[q | k | gate]``, bf16: keys, values and pooled rows into the caches, then the rows
+    of ``out``; what ``attn_prep``, ``pool_blocks`` and ``pooled_attention_prefill`` give together.  False, and nothing done, for sizes or addresses that
+    ``tlf_pooled_attn_portions`` does not take."""
+    lib = _lib.load()
+    _need(proj, BF16, "proj"); _need(kv.k, BF16, "k_cache"); _need(score_bias, BF16, "score_bias")
+    _need(positions, torch.int64, "positions"); _need(slot_mapping, torch.int32, "slot_mapping"); _need(block_tables, torch.int32, "block_tables")
+    n, hq = proj.shape[0], score_bias.numel()
+    pages, bs, hkv, _ = kv.k.shape
+    assert positions.numel() == n and slot_mapping.numel() == n and proj.stride(1) == 1 and out.stride(1) == 1 and out.shape[0] == n
+    assert rot_dims == 0 or cos_sin.shape[1] == rot_dims
+    assert block_tables.shape[0] >= first_seq + num_seqs and block_tables.stride(1) == 1
+    rc = lib.tlf_pooled_attn_portions(
+        proj.data_ptr(), proj.stride(0), _opt(q_bias), _opt(k_bias), positions.data_ptr(), _opt(cos_sin), cos_sin.shape[0] if cos_sin is not None else 0,
+        rot_dims, slot_mapping.data_ptr(), score_bias.data_ptr(), kv.k.data_ptr(), kv.v.data_ptr(), kv.pk.data_ptr(), kv.pv.data_ptr(),
+        block_tables.data_ptr(), block_tables.stride(0), cu_seqlens_q.data_ptr(), seq_starts.data_ptr(), first_seq, num_seqs, max_tokens, out.data_ptr(),
+        out.stride(0), hq, hkv, kv.head_dim, bs, kv.pool, kv.window, pages, float(scale), float(eps), _stream())
+    if rc == _lib.E_UNSUPPORTED:
+        return False
+    check(rc, "tlf_pooled_attn_portions")
+    return True
 
 
 def gla_decode(proj, a2, a2_bias, norm_weight, state, state_slots, positions, tau, eps, out):
