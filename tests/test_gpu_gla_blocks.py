@@ -168,3 +168,25 @@ def test_one_long_sequence_among_short_ones(H, lens, known, kernels):
     for n, out, state in run(H, 32, 64, 16, lens, [i % 3 for i in range(len(lens))], 16.0, H, known=known):
         assert out < OUT and state < STATE, (n, out, state)
     assert count() - before == kernels
+
+
+@pytest.mark.parametrize("rank", [1, 5, 8, 17, 24, 40, 63])
+@pytest.mark.parametrize("dk,dv", [(32, 64), (128, 96)])
+def test_ranks_of_the_decays_projection(dk, dv, rank):
+    """As with a rank of 64 whose other columns are zeros; what lies behind a row's own columns is not read."""
+    from tinyllmforge_amd import ops as P
+    H, lens = 2, [33, 100, 520]
+    g, dt, n = torch.Generator().manual_seed(rank), torch.bfloat16, sum(lens)
+    head = torch.randn(n, 2 * H * (dk + dv), generator=g).to(dt)
+    r, a2 = torch.randn(n, rank, generator=g).to(dt), torch.randn(H * dk, rank, generator=g).to(dt)
+    a2b, nw = 1 + torch.randn(H * dk, generator=g).to(dt), torch.randn(dv, generator=g).to(dt)
+    t = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    zeros = torch.nn.functional.pad
+    res = []
+    for rows, weights, behind in ((r, a2, float("nan")), (zeros(r, (0, 64 - rank)), zeros(a2, (0, 64 - rank)), 0.0)):
+        proj = torch.full((n, -(-(head.shape[1] + rows.shape[1]) // 8) * 8 + 8), behind, dtype=dt)
+        proj[:, :head.shape[1]], proj[:, head.shape[1]:head.shape[1] + rows.shape[1]] = head, rows
+        state, out = torch.zeros(3, H, dk, dv, device="cuda"), torch.zeros(n, H * dv, dtype=dt, device="cuda")
+        P.gla_portions(proj.cuda(), weights.cuda(), a2b.cuda(), nw.cuda(), state, t([0, 1, 2]), t([0, 0, 0]), *portions(lens), 0, 3, 8.0, 1e-5, out, 520)
+        res.append((out, state))
+    assert all(x.isfinite().all() and torch.equal(x, y) for x, y in zip(*res))

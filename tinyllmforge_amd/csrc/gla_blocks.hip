@@ -22,11 +22,11 @@
 // segments 59 + 18 + 255 us, so 58 + 15 + 209; 12 of 450 to 900 48 + 24 + 216, and in one pass over whole ones 204.
 //
 // Eight prompts of 1061 to 2048 tokens, 16 heads, key dim 128, value dim 256, medians under the profiler: chunk 122 + scan 470 (both
-// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 115 - 135 + first pass 58 - 65 + chaining 15 + scan
-// 169 - 205 us (whole layer 614 and 352 us).  The blocks write 55 KB a record, 3.7 TB/s with what they read: a workgroup waits for its rows, its decays and
+// passes) + segments 18 + norm and gate 92 us over 16-token chunks with fp32 products; here blocks 103 - 120 + first pass 58 - 65 + chaining 15 + scan
+// 169 - 205 us (whole layer 614 and 343 us).  The blocks write 55 KB a record, 3.7 TB/s with what they read: a workgroup waits for its rows, its decays and
 // its sums in turn, so what counts is how many a CU holds.  With keys towards the boundaries in LDS it held two and not three, and one workgroup in two
-// was launched for the second chunk of a block and left: 141 us where this takes 115, with strong decays, which make those keys anew for each
-// token, layer 450 and 425.  The scan is held by its barriers, two waves on a SIMD: a block took 13900 cycles, 5000 of them products and some 7200
+// was launched for the second chunk of a block and left: 141 us where this took 115, with strong decays, which make those keys anew for each
+// token, layer 450 and 425.  The decays' projection by the vector ALU took 13 more (layer 355 -> 343 us as a product).  The scan is held by its barriers, two waves on a SIMD: a block took 13900 cycles, 5000 of them products and some 7200
 // vector instructions on each SIMD, the second wave came to the barrier 4100 cycles behind the first.  10900 with the copies on four waves and
 // the block before finished in front of the products by these and behind them by the others: 198 -> 169 us.  The state's error against 64 bits is 5e-8 to 1.1e-7 on both, the
 // output's is its rounding to bf16.
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   constexpr int TH = DK * 4, LD = DK + 4, LPT = DK / 8;      // lanes per token, eight channels each
   constexpr int NW = DK / 16;
   static_assert(NW * kGB * kGB <= 2 * kGB * LD, "the waves' parts of A take the place of keys and decays");
-  __shared__ __attribute__((aligned(16))) float kb2[2][kGB][LD], am[kGB][kGB + 4], rs[kGB][kGlaBlockMaxR + 4];
+  __shared__ __attribute__((aligned(16))) float kb2[2][kGB][LD], am[kGB][kGB + 4];
   float (&ks)[kGB][LD] = kb2[0], (&bs)[kGB][LD] = kb2[1];
   __shared__ float tots[4][DK];
   __shared__ int harsh;
@@ -78,10 +78,6 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   const int64_t hk = static_cast<int64_t>(a.H) * DK, hv = static_cast<int64_t>(a.H) * a.dv;
   const T *pr = static_cast<const T *>(a.proj) + tok0 * a.ld;
   unsigned char *rec = reinterpret_cast<unsigned char *>(a.rec) + (static_cast<int64_t>(block) * a.H + h) * Rec::kSize;
-  for (int i = tid; i < kGB * a.R; i += TH) {
-    const int t = i / a.R, r = i - t * a.R;
-    rs[t][r] = t < len ? Elem<T>::ld(pr + t * a.ld + 2 * hk + 2 * hv + r) : 0.f;
-  }
   for (int i = tid; i < kGB * (kGB + 4); i += TH) (&am[0][0])[i] = 0.f;
   // token t, channels l * 4 .. and DK / 2 + l * 4 .. of it
   const int t = tid / LPT, l = tid % LPT;
@@ -111,35 +107,42 @@ __global__ __launch_bounds__(DK * 4) void gla_block_kernel(const GlaArgs a) {
   load_bf16(pr + min(qt, len - 1) * a.ld + h * DK + qc, q, 8);
 #pragma unroll
   for (int j = 0; j < 8; ++j) q[j] = qt < len ? q[j] * a.q_scale : 0.f;
-  __syncthreads();
   {
-    // decays: a thread has one channel and eight tokens, summed up here; the sums of the eights around them through LDS.  Sums towards the
-    // end are made on their own: as differences they would lose what the tokens before have decayed by
-    const int d = (tid >> 7) * 32 + qt, t0 = (tid >> 6 & 1) * 16 + hi * 8;
-    const T *w = static_cast<const T *>(a.a2) + (static_cast<int64_t>(h) * DK + d) * a.R;
+    // Decays: a thread has one channel and eight tokens, summed up here; the sums of the eights around them through LDS.  Sums towards the
+    // end are made on their own: as differences they would lose what the tokens before have decayed by.  Their projection is a product of the matrix
+    // cores, 32 channels a wave by its 16 tokens (twice), rows labelled so that a lane's first eight results are its tokens in turn
+    const int d = (tid >> 7) * 32 + qt, t16 = (tid >> 6 & 1) * 16, t0 = t16 + hi * 8;
+    const T *const rp = pr + min(t16 + ((lane & 3) | (lane & 4) << 1 | (lane & 8) >> 1), len - 1) * a.ld + 2 * hk + 2 * hv;
+    const T *const w = static_cast<const T *>(a.a2) + (static_cast<int64_t>(h) * DK + d) * a.R;
+    floatx16 zs;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) zs[r] = 0.f;
+    const bool whole = a.R % 8 == 0 && (reinterpret_cast<uintptr_t>(a.a2) & 15) == 0;
+    for (int r0 = 0; r0 < a.R; r0 += 16) {
+      const int at = r0 + hi * 8;
+      uint4 x = make_uint4(0, 0, 0, 0), y = x;
+      if (whole) {
+        if (at < a.R) {
+          x = *reinterpret_cast<const uint4 *>(rp + at);
+          y = *reinterpret_cast<const uint4 *>(w + at);
+        }
+      } else {
+        unsigned int xs[4] = {0, 0, 0, 0}, ys[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (at + e < a.R) {
+            xs[e / 2] |= static_cast<unsigned int>(rp[at + e]) << (e & 1) * 16;
+            ys[e / 2] |= static_cast<unsigned int>(w[at + e]) << (e & 1) * 16;
+          }
+        x = make_uint4(xs[0], xs[1], xs[2], xs[3]);
+        y = make_uint4(ys[0], ys[1], ys[2], ys[3]);
+      }
+      zs = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, y), zs, 0, 0, 0);
+    }
     const float bias = Elem<T>::ld(static_cast<const T *>(a.a2_bias) + h * DK + d);
     float z[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) z[j] = bias;
-    int r = 0;
-    for (; r + 4 <= a.R; r += 4) {
-      float wr[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) wr[e] = Elem<T>::ld(w + r + e);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float4 x = *reinterpret_cast<const float4 *>(&rs[t0 + j][r]);
-        z[j] = fmaf(wr[0], x.x, z[j]);
-        z[j] = fmaf(wr[1], x.y, z[j]);
-        z[j] = fmaf(wr[2], x.z, z[j]);
-        z[j] = fmaf(wr[3], x.w, z[j]);
-      }
-    }
-    for (; r < a.R; ++r) {
-      const float wr = Elem<T>::ld(w + r);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) z[j] = fmaf(wr, rs[t0 + j][r], z[j]);
-    }
+    for (int j = 0; j < 8; ++j) z[j] = zs[j] + bias;
     float sum = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
