@@ -65,6 +65,8 @@ __global__ __launch_bounds__(256) void talk_scores_kernel(const TalkRowsArgs a) 
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int kc = 0; kc < DC; ++kc) kreg[s][kc] = make_uint4(0, 0, 0, 0);
+    // An instruction has half a line of each row, the next one the other half, so K is not marked as read once (84 sequences of up to 2639 tokens,
+    // 16 heads on 8, layer 140 -> 121 us)
     const int krow = (n >> 2) * 8 + (n & 3);
     auto load_k = [&](int j, int page) __attribute__((always_inline)) {
       const int64_t r0 = sink_row(c, page, sink_page_of(c, j), kvh, j);
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(256) void talk_scores_kernel(const TalkRowsArgs a) 
       for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int kc = 0; kc < DC; ++kc)
-          if (kc * 32 < c.Dp) kreg[s][kc] = load_nt_u4(kp + s * 4 * c.Dp + kc * 32);
+          if (kc * 32 < c.Dp) kreg[s][kc] = *reinterpret_cast<const uint4 *>(kp + s * 4 * c.Dp + kc * 32);
     };
     float *sp = a.scores + (row * a.H + h0 + min(n, nh - 1)) * a.keys + g * 8;
     load_k(j0, bt[sink_page_of(c, j0)]);
