@@ -221,7 +221,8 @@ int tlf_sample(const void *logits, int64_t row_stride, const float *temperatures
  * below takes the weight in this order.
  * workspace: fp32 partial sums when the kernel plan for (M, N, K) splits K across workgroups
  * (few output tiles, long K); tlf_w8a16_gemm_workspace_bytes gives the size for this and for
- * tlf_bf16_gemm (0 when neither plan splits), 16-byte aligned.
+ * tlf_bf16_gemm (0 when neither plan splits), 16-byte aligned.  A product of many rows may end in a
+ * part with a plan of its own that splits K: without that scratch it runs in one part (other bits, same precision).
  */
 size_t tlf_w8a16_packed_bytes(int32_t N, int32_t K);   /* = round_up(N, 32) * K */
 int tlf_w8a16_pack_weight(const void *wq_rowmajor, void *packed, int32_t N, int32_t K, void *stream);
@@ -251,7 +252,8 @@ int tlf_bf16_gemm(const void *x, int64_t x_stride, const void *w, void *y,
  * wq / scale rows are INTERLEAVED (before tlf_w8a16_pack_weight): rows 16 j .. 16 j + 7 are gate channels 8 j .. 8 j + 7 and rows
  * 16 j + 8 .. 16 j + 15 the matching up channels (N = 2 x intermediate size, N % 16 == 0), so that
  * both halves of a product sit in one lane's accumulators.  Bit-identical to tlf_w8a16_gemm on
- * the same interleaved weight followed by tlf_silu_and_mul on the de-interleaved result.
+ * the same interleaved weight followed by tlf_silu_and_mul on the de-interleaved result, wherever
+ * that splits no K (else to rounding).
  * Needs no workspace (K is never split across workgroups).  Other constraints as tlf_w8a16_gemm. */
 int tlf_w8a16_gemm_silu_mul(const void *x, int64_t x_stride, const void *wq, const float *scale,
                             void *y, int32_t M, int32_t N, int32_t K, void *stream);

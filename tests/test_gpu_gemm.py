@@ -116,6 +116,43 @@ def test_bf16_many_rows_of_a_short_k_exact_on_integer_data(M, N, K):
     assert torch.equal(got.view(torch.int16), (x.double() @ w.double().t()).to(BF).view(torch.int16))
 
 
+@pytest.mark.parametrize("M,N,K,w8,rest", [
+    (4097, 4096, 256, True, 1), (4113, 4096, 64, True, 17), (5888, 4096, 192, True, 1792), (5889, 4096, 192, True, 0),
+    (4300, 4080, 2048, True, 204), (4200, 4096, 8192, True, 104), (12301, 2064, 128, True, 0),
+    (8193, 4096, 320, False, 1), (8449, 4080, 2048, False, 257), (2050, 4096, 4160, False, 2), (2560, 4080, 4160, False, 512),
+    (2561, 4096, 4160, False, 0)])
+def test_product_in_two_parts_exact_on_integer_data(M, N, K, w8, rest):
+    """Whole rounds of large tiles and ``rest`` rows behind them (one row, the skinny kernel's last and the next one, whole and cut tiles, the most
+    there are, splits of K) and their neighbours in one part: exact in any order, so the same with rows that are not contiguous, without the scratch
+    that the second part asks for, and from the entry point that leaves partial sums."""
+    import ctypes
+    from tinyllmforge_amd import _lib, ops as P
+    lib = _lib.load()
+    plans = [(ctypes.c_int32 * 8)() for _ in range(2)]
+    assert all(lib.tlf_gemm_plan(m, N, K, int(w8), plan) == 0 for m, plan in zip((M, M - rest), plans)) and list(plans[0]) == list(plans[1])
+    x = torch.randint(-2, 3, (M, K + 8), generator=g(M), dtype=torch.int32).to(BF).to(DEV)[:, :K]
+    wi = torch.randint(-127, 128, (N, K), generator=g(N + K), dtype=torch.int32)
+    ref = torch.cat([x[m:m + 2048].double() @ wi.to(DEV).double().t() * 2.0 ** -12 for m in range(0, M, 2048)]).to(BF)
+    scale = torch.full((N,), 2.0 ** -12, device=DEV) if w8 else None
+    w = P.pack_w8(wi.to(torch.int8).to(DEV)) if w8 else (wi * 2.0 ** -12).to(BF).to(DEV)
+    got = P.w8a16_linear(x, w, scale) if w8 else P.bf16_linear(x, w)
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    tight = P.w8a16_linear(x.contiguous(), w, scale) if w8 else P.bf16_linear(x.contiguous(), w)
+    assert torch.equal(tight.view(torch.int16), ref.view(torch.int16))
+    bare = torch.zeros(M + 1, N, dtype=BF, device=DEV)
+    at = (x.data_ptr(), x.stride(0), w.data_ptr())
+    stream = torch.cuda.current_stream().cuda_stream
+    rc = lib.tlf_w8a16_gemm(*at, scale.data_ptr(), bare.data_ptr(), M, N, K, None, 0, stream) if w8 else \
+        lib.tlf_bf16_gemm(*at, bare.data_ptr(), M, N, K, None, 0, stream)
+    assert rc == 0 and torch.equal(bare[:M].view(torch.int16), ref.view(torch.int16)) and not bare[M].any()
+    later = P.linear_deferred(x, w, scale)
+    assert later.splits == 1 and torch.equal(later.y.view(torch.int16), ref.view(torch.int16))
+    if N % 32 == 0:                                         # the activation behind it: both sides are the same sums
+        gate, up = (ref.view(M, -1, 2, 8)[:, :, i].reshape(M, -1) for i in range(2))
+        act = P.w8a16_linear_silu_mul(x, w, scale) if w8 else P.bf16_linear_silu_mul(x, w)
+        assert torch.equal(act.view(torch.int16), P.silu_and_mul(torch.cat([gate, up], dim=1)).view(torch.int16))
+
+
 # BASELINE configs[2], every cell: M in {1, 16, 64, 256, 2048} x the four Qwen3-8B projection shapes.  The planner
 # is a threshold tree in M, N and K, so the cells the benchmark times are checked here one by one, not through
 # neighbours.

@@ -1505,10 +1505,10 @@ inline int skinny_max_m() { return gemm_tuning().skinny_max_m; }
 // plan_out != nullptr: nothing is launched; the eight plan fields are written there instead and the
 // return code says whether a kernel instance exists for the plan.
 template <bool W8>
-int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *scale, void *y,
-                int32_t M, int32_t N, int32_t K, void *workspace, size_t workspace_bytes,
-                hipStream_t stream, int32_t *plan_out = nullptr, int32_t act = 0,
-                const NormTail *tail = nullptr, const QkRopeStoreArgs *qk = nullptr, int32_t *deferred = nullptr) {
+int launch_gemm_rows(const void *x, int64_t x_stride, const void *w, const float *scale, void *y,
+                     int32_t M, int32_t N, int32_t K, void *workspace, size_t workspace_bytes,
+                     hipStream_t stream, int32_t *plan_out = nullptr, int32_t act = 0,
+                     const NormTail *tail = nullptr, const QkRopeStoreArgs *qk = nullptr, int32_t *deferred = nullptr) {
   if (deferred) *deferred = 1;
   const bool dry = plan_out != nullptr;
   GemmParams p;
@@ -1689,6 +1689,61 @@ int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *sca
   return rc;
 }
 
+// Rows of a product that run as tiles of one workgroup per CU, the rest behind them with a plan of its own; 0: all in one.
+//
+// Such tiles take rounds of 256, and a round of a few takes as long as one tile does on its own.  Where the last round has few tiles its
+// rows go to the plan for so many tokens instead, which has the whole chip.  us in one part / in two:
+//   4096 x 12288, int8   at 12288 + 64 tokens (three rounds 954) 1122 / 971, + 157 1122 / 973, + 400 1128 / 1010, + 1200 1143 / 1100, + 1600 (112 tiles) 1154 / 1112,
+//                        + 2200 (144 tiles) 1165 / 1203
+//   4096 x 4096, int8    at 12288 + 157 389 / 341, + 1600 401 / 384, + 2200 403 / 413; bf16 at 8192 + 157 278 / 232, + 1600 292 / 275, + 2200 299 / 314
+//   24576 x 4096         at 12288 + 157 (96 tiles) int8 1991 / 1961, bf16 2151 / 2126, + 400 (192 tiles) 2010 / 2019, 2185 / 2183
+//   256 x 128 tiles, bf16, half as long a round: 4096 x 12288 at 8192 + 400 (64 tiles) 800 / 756, + 800 (112 tiles) 810 / 831
+// They are worth no more than a second pass over a wide weight: 10240 x 5120 in bf16 at 6537, nine rows in the second part, 630 / 642.
+inline int32_t gemm_main_rows(int32_t M, int32_t N, int32_t K, bool w8) {
+  constexpr int kCUs = 256;
+  const int n = (N + 255) / 256;
+  if (gemm_tuning().has_plan || static_cast<int64_t>(n) * ((M + 127) / 128) <= kCUs) return 0;
+  for (const int bm : {256, 128}) {
+    if (bm == 128 && N > (w8 ? 16384 : 8192)) continue;
+    const int m = (M + bm - 1) / bm, over = static_cast<int>((static_cast<int64_t>(n) * m - 1) % kCUs + 1);   // tiles of the last round
+    const int rows = (over + n - 1) / n;                     // of tiles that have to go to end a round earlier
+    if (rows >= m || rows * n > (bm == 256 ? 120 : 64)) continue;
+    const int32_t first = (m - rows) * bm;
+    const GemmPlan g = plan_gemm(first, N, K, w8);
+    if (g.bn == 256 && g.bm == bm && (bm == 256 || g.stages == 3) && g.splits == 1 && g.kgroups == 1) return first;
+  }
+  return 0;
+}
+
+// Scratch of a product whose plan splits K, for M tokens in one part.
+template <bool W8>
+size_t gemm_split_bytes(int32_t M, int32_t N, int32_t K) {
+  int32_t plan[8];
+  if (launch_gemm_rows<W8>(nullptr, K, nullptr, nullptr, nullptr, M, N, K, nullptr, 0, nullptr, plan) != TLF_OK) return ~size_t{0};
+  return plan[5] > 1 ? static_cast<size_t>(plan[5]) * M * N * sizeof(float) : 0;
+}
+
+// The whole product, in one or two parts.  The second one's split of K needs scratch that the first one would not: without it there is one part.
+template <bool W8>
+int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *scale, void *y,
+                int32_t M, int32_t N, int32_t K, void *workspace, size_t workspace_bytes,
+                hipStream_t stream, int32_t *plan_out = nullptr, int32_t act = 0,
+                const NormTail *tail = nullptr, const QkRopeStoreArgs *qk = nullptr, int32_t *deferred = nullptr) {
+  const int32_t first = act == 2 || tail || qk ? 0 : gemm_main_rows(M, N, K, W8);
+  if (first) {
+    if (plan_out) return launch_gemm_rows<W8>(nullptr, K, nullptr, nullptr, nullptr, first, N, K, nullptr, 0, nullptr, plan_out, act);
+    if (act || gemm_split_bytes<W8>(M - first, N, K) <= (reinterpret_cast<uintptr_t>(workspace) & 15u ? 0 : workspace_bytes)) {
+      if (deferred) *deferred = 1;
+      const int rc = launch_gemm_rows<W8>(x, x_stride, w, scale, y, first, N, K, nullptr, 0, stream, nullptr, act);
+      if (rc != TLF_OK) return rc;
+      return launch_gemm_rows<W8>(static_cast<const unsigned short *>(x) + first * x_stride, x_stride, w, scale,
+                                  static_cast<unsigned short *>(y) + static_cast<int64_t>(first) * (act ? N / 2 : N), M - first, N, K,
+                                  workspace, workspace_bytes, stream, nullptr, act);
+    }
+  }
+  return launch_gemm_rows<W8>(x, x_stride, w, scale, y, M, N, K, workspace, workspace_bytes, stream, plan_out, act, tail, qk, deferred);
+}
+
 // Grouped product (bf16): rows in expert order, tiles of `bm` rows of one expert each.  The host picks bm by the average rows
 // per expert (ClippedGLUExperts.tile_rows): few, and the weights stream from HBM once, the column tiles of an expert side by
 // side on an XCD; many, and the largest tile saves copies.  From a sweep of the tile instances over two mixtures, us for
@@ -1866,15 +1921,11 @@ extern "C" size_t tlf_w8a16_gemm_workspace_bytes(int32_t M, int32_t N, int32_t K
   if (M <= 0 || N <= 0 || K <= 0 || K % kBK) return 0;
   // fp32 partial sums of the plan's split of K (the larger of the int8 and the bf16 plan: both
   // entry points share this query); a tuning override may pick any split up to 16
-  int splits = 16;
-  if (!gemm_tuning().has_plan) {
-    int32_t p8[8], p16[8];
-    if (launch_gemm<true>(nullptr, K, nullptr, nullptr, nullptr, M, N, K, nullptr, 0, nullptr, p8) == TLF_OK &&
-        launch_gemm<false>(nullptr, K, nullptr, nullptr, nullptr, M, N, K, nullptr, 0, nullptr, p16) == TLF_OK)
-      splits = p8[5] > p16[5] ? p8[5] : p16[5];
-  }
-  if (splits <= 1) return 0;
-  return static_cast<size_t>(splits) * M * N * sizeof(float);
+  if (gemm_tuning().has_plan) return static_cast<size_t>(16) * M * N * sizeof(float);
+  const int32_t first8 = gemm_main_rows(M, N, K, true), first16 = gemm_main_rows(M, N, K, false);
+  const size_t b8 = gemm_split_bytes<true>(M - first8, N, K), b16 = gemm_split_bytes<false>(M - first16, N, K);
+  if (b8 == ~size_t{0} || b16 == ~size_t{0}) return static_cast<size_t>(16) * M * N * sizeof(float);
+  return b8 > b16 ? b8 : b16;
 }
 
 extern "C" int tlf_w8a16_gemm(const void *x, int64_t x_stride, const void *wq, const float *scale,
