@@ -153,6 +153,19 @@ def test_product_in_two_parts_exact_on_integer_data(M, N, K, w8, rest):
         assert torch.equal(act.view(torch.int16), P.silu_and_mul(torch.cat([gate, up], dim=1)).view(torch.int16))
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448])
+@pytest.mark.parametrize("M,N,w8", [(1300, 6160, True), (2000, 8208, True), (600, 2064, True), (2100, 8208, False), (1200, 2064, False)])
+def test_pipelines_of_few_steps_exact_on_integer_data(M, N, K, w8):
+    """Copies ahead of the products, and the steps behind the last copy: one to seven K-tiles with three and two stages, exact in any order."""
+    from tinyllmforge_amd import ops as P
+    x = torch.randint(-2, 3, (M, K), generator=g(M), dtype=torch.int32).to(BF).to(DEV)
+    wi = torch.randint(-127, 128, (N, K), generator=g(N + K), dtype=torch.int32)
+    scale = torch.full((N,), 2.0 ** -12, device=DEV)
+    ref = (x.double() @ wi.to(DEV).double().t() * 2.0 ** -12).to(BF)
+    got = P.w8a16_linear(x, wi.to(torch.int8).to(DEV), scale) if w8 else P.bf16_linear(x, (wi * 2.0 ** -12).to(BF).to(DEV))
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
 # BASELINE configs[2], every cell: M in {1, 16, 64, 256, 2048} x the four Qwen3-8B projection shapes.  The planner
 # is a threshold tree in M, N and K, so the cells the benchmark times are checked here one by one, not through
 # neighbours.
