@@ -1721,19 +1721,24 @@ int launch_gemm_rows(const void *x, int64_t x_stride, const void *w, const float
 //   4096 x 4096, int8    at 12288 + 157 389 / 341, + 1600 401 / 384, + 2200 403 / 413; bf16 at 8192 + 157 278 / 232, + 1600 292 / 275, + 2200 299 / 314
 //   24576 x 4096         at 12288 + 157 (96 tiles) int8 1991 / 1961, bf16 2151 / 2126, + 400 (192 tiles) 2010 / 2019, 2185 / 2183
 //   256 x 128 tiles, bf16, half as long a round: 4096 x 12288 at 8192 + 400 (64 tiles) 800 / 756, + 800 (112 tiles) 810 / 831
-// They are worth no more than a second pass over a wide weight: 10240 x 5120 in bf16 at 6537, nine rows in the second part, 630 / 642.
+//   128 x 128 tiles of three stages, bf16 (of int8 two are on a CU): 2560 x 9728 at 3403 226 / 175,
+//                        1024 x 3072 at 4142 45 / 39, 4096 x 4096 at 1208 59 / 53, 2048 x 2048 at 2065 33.1 / 30.7
+// Tiles of 256 x 128 are worth no more than a second pass over a wide weight: 10240 x 5120 in bf16 at 6537, nine rows in the second part, 630 / 642.
 inline int32_t gemm_main_rows(int32_t M, int32_t N, int32_t K, bool w8) {
   constexpr int kCUs = 256;
-  const int n = (N + 255) / 256;
-  if (gemm_tuning().has_plan || static_cast<int64_t>(n) * ((M + 127) / 128) <= kCUs) return 0;
-  for (const int bm : {256, 128}) {
-    if (bm == 128 && N > (w8 ? 16384 : 8192)) continue;
-    const int m = (M + bm - 1) / bm, over = static_cast<int>((static_cast<int64_t>(n) * m - 1) % kCUs + 1);   // tiles of the last round
+  if (gemm_tuning().has_plan || static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128) <= kCUs) return 0;
+  struct { int bn, bm, most; } const tiles[] = {{256, 256, 120}, {256, 128, 64}, {128, 128, 64}};
+  for (const auto &c : tiles) {
+    if (c.bn == 256 && c.bm == 128 && N > (w8 ? 16384 : 8192)) continue;
+    if (c.bn == 128 && w8) continue;
+    const int n = (N + c.bn - 1) / c.bn, m = (M + c.bm - 1) / c.bm;
+    if (static_cast<int64_t>(n) * m <= kCUs) continue;
+    const int over = static_cast<int>((static_cast<int64_t>(n) * m - 1) % kCUs + 1);   // tiles of the last round
     const int rows = (over + n - 1) / n;                     // of tiles that have to go to end a round earlier
-    if (rows >= m || rows * n > (bm == 256 ? 120 : 64)) continue;
-    const int32_t first = (m - rows) * bm;
+    if (rows >= m || rows * n > c.most) continue;
+    const int32_t first = (m - rows) * c.bm;
     const GemmPlan g = plan_gemm(first, N, K, w8);
-    if (g.bn == 256 && g.bm == bm && (bm == 256 || g.stages == 3) && g.splits == 1 && g.kgroups == 1) return first;
+    if (g.bn == c.bn && g.bm == c.bm && (c.bm == 256 || g.stages == 3) && g.splits == 1 && g.kgroups == 1) return first;
   }
   return 0;
 }
