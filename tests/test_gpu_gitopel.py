@@ -207,6 +207,12 @@ def test_one_key_stands_out_at_every_edge(dtype, size, pool, n):
     # a difference of one key is at least 1 (values are whole numbers), of one block's mean at least the mean itself
 
 
+@pytest.mark.parametrize("size,pool,n", [(31, 3, 190), (32, 5, 200), (33, 1, 230), (96, 4, 260), (65, 2, 131)])
+def test_one_key_stands_out_at_the_halves_of_tiles(size, pool, n):
+    """Windows and means that end on either side of 32 keys of a tile of 64."""
+    test_one_key_stands_out_at_every_edge("bf16", size, pool, n)
+
+
 GLA = [(3, 24, 20, 5), (2, 64, 64, 16), (1, 16, 16, 1), (2, 128, 256, 16), (1, 256, 512, 33), (2, 100, 50, 7), (1, 5, 3, 2)]
 
 

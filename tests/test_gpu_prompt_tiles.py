@@ -54,6 +54,12 @@ def test_every_row_of_uneven_batches(lens, heads, kv_heads):
     close(out)
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(1, 1), (8, 2), (12, 6)])
+def test_halves_of_tiles_that_no_row_sees(heads, kv_heads):
+    """Portions that end on either side of the halves of a tile, 32 keys, and row tiles of 128, 32 and 64 rows that do."""
+    test_every_row_of_uneven_batches((31, 32, 33, 63, 64, 65, 95, 96, 97, 128, 160, 161, 226), heads, kv_heads)
+
+
 @pytest.mark.parametrize("dim,vdim", [(32, 32), (56, 100), (96, 64), (128, 128), (136, 128), (128, 136)])
 @pytest.mark.parametrize("cap", [None, 20.0, 50.0])
 def test_weights_follow_a_growing_maximum(dim, vdim, cap):

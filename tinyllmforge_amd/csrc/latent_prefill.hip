@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VC <= 
   copy(0, PromptPart<true, true>{});
   core.template walk<true, true>(
       tiles, min(max(0, wave_first - p.window + 1 - w0) / kPK, to - 1), to, edge, min(tiles, max(0, (wave_first + 1 - w0) / kPK)), copy,
-      []() __attribute__((always_inline)) { return Core::all(0.f); },
+      [&](int t, int hf, auto) __attribute__((always_inline)) { return t * kPK + hf * 32 <= wave_last - w0; }, []() __attribute__((always_inline)) { return Core::all(0.f); },
       [&](int t, int hf, typename Core::Scores &sc, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
         if (part.mask) {
           const int seen = upos - (w0 + t * kPK + hf * 32 + g * 8), hidden = seen - p.window;

@@ -184,9 +184,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
   for (int kc = 0; kc < 2 * DC; ++kc) core.qf[kc] = __builtin_bit_cast(bf16x8, raw[kc]);
   // tiles between the window's edge and the diagonal hide nothing from anyone
+  const int last = i_last - w0 + ptiles * kTK, edge0 = i_first - c.size + 1 - w0 + ptiles * kTK;      // of the keys in the window, counted as tiles are
   const int edge = i_last - c.size >= w0 ? (i_last - c.size - w0) / kTK + 1 : 0;
   core.template walk<true, false>(
-      tiles, 0, tiles, ptiles + edge, min(tiles, ptiles + max(0, (i_first + 1 - w0) / kTK)), copy, []() __attribute__((always_inline)) { return Core::all(0.f); },
+      tiles, 0, tiles, ptiles + edge, min(tiles, ptiles + max(0, (i_first + 1 - w0) / kTK)), copy,
+      [&](int t, int hf, auto part) __attribute__((always_inline)) {
+        const int at = t * kTK + hf * 32;
+        if (part.lead && t < ptiles) return at < nb;
+        return at <= last && (!part.lead || at + 31 >= edge0);
+      },
+      []() __attribute__((always_inline)) { return Core::all(0.f); },
       [&](int t, int hf, const typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
         float e[16];
 #pragma unroll

@@ -18,6 +18,8 @@
 // faster card 161 -> 152; 250, 198 and 168 registers a lane (251, 236 and 192 before).  In a stream of nothing but these products and weights from
 // registers two waves take 2150 cycles where the products alone take 1540: beside another wave's vector instructions a product takes a
 // fifth longer.  Without copies sinks take 331, without LDS reads of V pooled heads 287.
+// Halves of masked tiles that none of the wave's units sees are left out (half of the row tiles end in the first half of a tile): layers
+// 265.6 -> 262.5 us (pooled, whose window begins in a second half as often, and whose means may end in a first one) and 350.5 -> 347.6 (sinks).
 // Measured and not taken: scores in front of the values (no difference), reads kept behind the products (3 % slower), wave priorities around the
 // products (3 % slower), workgroups that take their row tiles from a list (1 - 2 % slower, though a new one starts 3.5 us after the one before
 // it ends: while one is away the other runs faster).
@@ -159,13 +161,14 @@ struct PromptCore {
   // The workgroup's walk over `tiles` tiles, of which the wave computes first_tile <= t < end: those that some of its units see.  A value
   // behind or before them, infinite or no number as it may be, does not reach its rows.  The kernel's parts:
   //   copy(t, part)               the tile's copies; called for t = 1, 2, .. in turn, the first one's are under way
+  //   seen(t, hf, part)           whether any of the wave's units sees a key of half hf of tile t, which is masked
   //   from()                      where the unit's scores begin (registers that are kept: set anew for each half they are a ninth of a wave's vector work)
   //   weights(t, hf, s, w, part)  of half hf of tile t, when all values of the halves before are in acc
   // part.mask is not set where all keys of the tile are seen by all units: tiles clear_from <= t < clear_to of them (wave uniform),
   // clear_from 0 without LEAD.  part.lead is set where t may be below clear_from.
   // SOME: the wave's tiles may be some only; otherwise first_tile is 0 and `end` is `tiles`.
-  template <bool LEAD, bool SOME, class Copy, class From, class Weigh>
-  __device__ __forceinline__ void walk(int tiles, int first_tile, int end, int clear_from, int clear_to, Copy copy, From from, Weigh weights) {
+  template <bool LEAD, bool SOME, class Copy, class Seen, class From, class Weigh>
+  __device__ __forceinline__ void walk(int tiles, int first_tile, int end, int clear_from, int clear_to, Copy copy, Seen seen, From from, Weigh weights) {
     constexpr PromptPart<true, true> lead{};
     constexpr PromptPart<false, false> plain{};
     constexpr PromptPart<false, true> tail{};
@@ -180,6 +183,7 @@ struct PromptCore {
       arrive(t, part);
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
+        if (part.mask && !seen(t, hf, part)) continue;       // wave uniform
         Scores s;
         read_k(t, hf);
         values(w);

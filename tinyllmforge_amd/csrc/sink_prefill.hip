@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   copy(0, PromptPart<false, true>{});
   core.template walk<false, true>(
       tiles, 0, wave_last / kSK + 1, 0, min(tiles, (wave_first + 1) / kSK), copy,                      // the diagonal cuts the tiles behind
-      [&]() __attribute__((always_inline)) { return from; },
+      [&](int t, int hf, auto) __attribute__((always_inline)) { return t * kSK + hf * 32 <= wave_last; }, [&]() __attribute__((always_inline)) { return from; },
       [&](int t, int hf, typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
