@@ -1526,12 +1526,12 @@ inline bool plan_override(GemmPlan &g, int K) {
 inline int skinny_max_m() { return gemm_tuning().skinny_max_m; }
 
 // plan_out != nullptr: nothing is launched; the eight plan fields are written there instead and the
-// return code says whether a kernel instance exists for the plan.
+// return code says whether a kernel instance exists for the plan.  tiled: no skinny kernel, however few the rows.
 template <bool W8>
 int launch_gemm_rows(const void *x, int64_t x_stride, const void *w, const float *scale, void *y,
                      int32_t M, int32_t N, int32_t K, void *workspace, size_t workspace_bytes,
-                     hipStream_t stream, int32_t *plan_out = nullptr, int32_t act = 0,
-                     const NormTail *tail = nullptr, const QkRopeStoreArgs *qk = nullptr, int32_t *deferred = nullptr) {
+                     hipStream_t stream, int32_t *plan_out = nullptr, int32_t act = 0, const NormTail *tail = nullptr,
+                     const QkRopeStoreArgs *qk = nullptr, int32_t *deferred = nullptr, bool tiled = false) {
   if (deferred) *deferred = 1;
   const bool dry = plan_out != nullptr;
   GemmParams p;
@@ -1549,7 +1549,7 @@ int launch_gemm_rows(const void *x, int64_t x_stride, const void *w, const float
   p.map_main = 0; p.map_full = 0; p.map_rem = 1;
   GemmPlan g;
   const bool wstream = W8 && plan_wstream(M, N, K, act, g);
-  if (M <= skinny_max_m() && !wstream) {
+  if (M <= skinny_max_m() && !wstream && !tiled) {
     p.k_per_split = K; p.splits = 1; p.m_tiles = 1; p.n_tiles = 1; p.group_n = 1; p.xcd_rows = 0;
     p.map_main = 0; p.map_full = 0; p.map_rem = 1;
     if (dry) {
@@ -1723,35 +1723,46 @@ int launch_gemm_rows(const void *x, int64_t x_stride, const void *w, const float
 //   256 x 128 tiles, bf16, half as long a round: 4096 x 12288 at 8192 + 400 (64 tiles) 800 / 756, + 800 (112 tiles) 810 / 831
 //   128 x 128 tiles of three stages, bf16 (of int8 two are on a CU): 2560 x 9728 at 3403 226 / 175,
 //                        1024 x 3072 at 4142 45 / 39, 4096 x 4096 at 1208 59 / 53, 2048 x 2048 at 2065 33.1 / 30.7
-// Tiles of 256 x 128 are worth no more than a second pass over a wide weight: 10240 x 5120 in bf16 at 6537, nine rows in the second part, 630 / 642.
+// Tiles of 256 x 128 are worth no more than a second pass over a wide weight: 10240 x 5120 in bf16 at 6537, nine rows in the second part, 630 / 642; and
+// those of 128 rows no second launch below K = 1024: int8 6144 x 256 at 1409 15.1 / 18.6, 8192 x 512 at 1224 19.6 / 25.5, bf16 4096 x 512 at 1224 15.6 / 16.5,
+// nor where the whole product has another plan (int8 2048 x 1024 at 12328 61.8 / 66.5).  Below K = 1536 more than 64 tiles of 256 x 256 are as well off in
+// the round (int8 4096 x 320 at 5496, 96 tiles, 23.8 / 25.9, 6144 x 768 at 3716, 120 tiles, 39.6 / 42.0);
+// below 256 a tile of 256 x 256 is little more than a launch (4096 x 128 at 8292 in bf16 34 / 39; x 512 at 12588 72 / 66; 6144 x 256 in int8 at 8492 49 / 46).
 inline int32_t gemm_main_rows(int32_t M, int32_t N, int32_t K, bool w8) {
   constexpr int kCUs = 256;
-  if (gemm_tuning().has_plan || static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128) <= kCUs) return 0;
+  if (gemm_tuning().has_plan || K < 256 || static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128) <= kCUs) return 0;
   struct { int bn, bm, most; } const tiles[] = {{256, 256, 120}, {256, 128, 64}, {128, 128, 64}};
   for (const auto &c : tiles) {
-    if (c.bn == 256 && c.bm == 128 && N > (w8 ? 16384 : 8192)) continue;
+    if (c.bm == 128 && (K < 1024 || (c.bn == 256 && N > (w8 ? 16384 : 8192)))) continue;
     if (c.bn == 128 && w8) continue;
     const int n = (N + c.bn - 1) / c.bn, m = (M + c.bm - 1) / c.bm;
     if (static_cast<int64_t>(n) * m <= kCUs) continue;
     const int over = static_cast<int>((static_cast<int64_t>(n) * m - 1) % kCUs + 1);   // tiles of the last round
     const int rows = (over + n - 1) / n;                     // of tiles that have to go to end a round earlier
-    if (rows >= m || rows * n > c.most) continue;
+    if (rows >= m || rows * n > (K < 1536 ? 64 : c.most)) continue;
     const int32_t first = (m - rows) * c.bm;
     const GemmPlan g = plan_gemm(first, N, K, w8);
-    if (g.bn == c.bn && g.bm == c.bm && (c.bm == 256 || g.stages == 3) && g.splits == 1 && g.kgroups == 1) return first;
+    if (g.bn != c.bn || g.bm != c.bm || (c.bm == 128 && g.stages != 3) || g.splits != 1 || g.kgroups != 1) continue;
+    if (c.bm == 128) {                                       // not where the whole product would take two smaller or shallower workgroups a CU
+      const GemmPlan whole = plan_gemm(M, N, K, w8);
+      if (whole.bn != g.bn || whole.bm != g.bm || whole.stages != g.stages) continue;
+    }
+    return first;
   }
   return 0;
 }
 
 // Scratch of a product whose plan splits K, for M tokens in one part.
 template <bool W8>
-size_t gemm_split_bytes(int32_t M, int32_t N, int32_t K) {
+size_t gemm_split_bytes(int32_t M, int32_t N, int32_t K, bool tiled) {
   int32_t plan[8];
-  if (launch_gemm_rows<W8>(nullptr, K, nullptr, nullptr, nullptr, M, N, K, nullptr, 0, nullptr, plan) != TLF_OK) return ~size_t{0};
+  if (launch_gemm_rows<W8>(nullptr, K, nullptr, nullptr, nullptr, M, N, K, nullptr, 0, nullptr, plan, 0, nullptr, nullptr, nullptr, tiled) != TLF_OK) return ~size_t{0};
   return plan[5] > 1 ? static_cast<size_t>(plan[5]) * M * N * sizeof(float) : 0;
 }
 
-// The whole product, in one or two parts.  The second one's split of K needs scratch that the first one would not: without it there is one part.
+// The whole product, in one or two parts.  The second one's split of K needs scratch that the first one would not: without it there is one part.  bf16
+// weights, which the skinny kernel reads past the caches, go to the tiled one there for up to 16 rows too, since the first part has just read them (6144
+// x 1024 at 8193 rows: 119 us with the skinny kernel, 100 so, 116 in one part; int8 ones are as fast either way).
 template <bool W8>
 int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *scale, void *y,
                 int32_t M, int32_t N, int32_t K, void *workspace, size_t workspace_bytes,
@@ -1760,13 +1771,13 @@ int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *sca
   const int32_t first = act == 2 || tail || qk ? 0 : gemm_main_rows(M, N, K, W8);
   if (first) {
     if (plan_out) return launch_gemm_rows<W8>(nullptr, K, nullptr, nullptr, nullptr, first, N, K, nullptr, 0, nullptr, plan_out, act);
-    if (act || gemm_split_bytes<W8>(M - first, N, K) <= (reinterpret_cast<uintptr_t>(workspace) & 15u ? 0 : workspace_bytes)) {
+    if (act || gemm_split_bytes<W8>(M - first, N, K, !W8) <= (reinterpret_cast<uintptr_t>(workspace) & 15u ? 0 : workspace_bytes)) {
       if (deferred) *deferred = 1;
       const int rc = launch_gemm_rows<W8>(x, x_stride, w, scale, y, first, N, K, nullptr, 0, stream, nullptr, act);
       if (rc != TLF_OK) return rc;
       return launch_gemm_rows<W8>(static_cast<const unsigned short *>(x) + first * x_stride, x_stride, w, scale,
                                   static_cast<unsigned short *>(y) + static_cast<int64_t>(first) * (act ? N / 2 : N), M - first, N, K,
-                                  workspace, workspace_bytes, stream, nullptr, act);
+                                  workspace, workspace_bytes, stream, nullptr, act, nullptr, nullptr, nullptr, !W8);
     }
   }
   return launch_gemm_rows<W8>(x, x_stride, w, scale, y, M, N, K, workspace, workspace_bytes, stream, plan_out, act, tail, qk, deferred);
@@ -1962,7 +1973,7 @@ extern "C" size_t tlf_w8a16_gemm_workspace_bytes(int32_t M, int32_t N, int32_t K
   // entry points share this query); a tuning override may pick any split up to 16
   if (gemm_tuning().has_plan) return static_cast<size_t>(16) * M * N * sizeof(float);
   const int32_t first8 = gemm_main_rows(M, N, K, true), first16 = gemm_main_rows(M, N, K, false);
-  const size_t b8 = gemm_split_bytes<true>(M - first8, N, K), b16 = gemm_split_bytes<false>(M - first16, N, K);
+  const size_t b8 = gemm_split_bytes<true>(M - first8, N, K, false), b16 = gemm_split_bytes<false>(M - first16, N, K, first16 > 0);
   if (b8 == ~size_t{0} || b16 == ~size_t{0}) return static_cast<size_t>(16) * M * N * sizeof(float);
   return b8 > b16 ? b8 : b16;
 }
