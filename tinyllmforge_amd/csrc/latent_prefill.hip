@@ -7,8 +7,7 @@
 //   P = 2^(S * scale - m)         fp32; m follows a row's maximum only when that has grown by more than 8 (a factor of 256,
 //                                 which the fp32 sums and the bf16 pair hold), so the accumulators are rarely rescaled.  Whether any
 //                                 has grown is asked lane by lane; maxima of rows are only formed when one has, and all rows of the wave
-//                                 follow theirs then: a largest weight is 1 but for the product's own rounding
-//                                 The scale and the maximum in one fma, its rounding less than the product's (layer 139 -> 136.5 us)
+//                                 follow theirs then: a largest weight of 1 is not rounded
 // 16 heads of 96 and 64 dimensions, eight prompts of 1061 to 2048 tokens: layer 189 us with the stages of a tile one after the other and
 // a window of 1024, 171 with three stages side by side, 162 so; three waves per SIMD fit the registers (160 to 165 with two, 160 with three).
 #include "latent_attn.h"
@@ -167,7 +166,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VC <= 
         const float ms = m == -INFINITY ? 0.f : m;
         float e[16];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], p.scale_log2, -ms));
+        for (int j = 0; j < 16; ++j) e[j] = __builtin_amdgcn_exp2f(sc[j] * p.scale_log2 - ms);
         l += Core::sum(e);
         Core::split(e, w);
       });
