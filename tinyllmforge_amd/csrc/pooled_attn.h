@@ -93,14 +93,15 @@ inline bool pooled_proj_takes(const PooledProj &p, int32_t head_dim) {
 // Keys, values and pooled rows of portions (pooled_attn.hip); of p, what keys are made from.
 int launch_pooled_kv(const PooledCache &c, const PooledProj &p, const int32_t *slots, const int32_t *cu_q, const int32_t *starts, int first_seq, int num_seqs,
                      int max_tokens, int H, hipStream_t stream);
-// The pairs of dimensions 8 ch .. 8 ch + 7 turned.
+// The pairs of dimensions 8 ch .. 8 ch + 7 turned, each product rounded as in rows that are prepared on their own: a token's key has the same bits
+// whichever way its step was cut.
 __device__ __forceinline__ void pooled_rotate(float (&x)[8], const float4 &co, const float4 &si) {
   const float cv[4] = {co.x, co.y, co.z, co.w}, sv[4] = {si.x, si.y, si.z, si.w};
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float u = x[2 * e], v = x[2 * e + 1];
-    x[2 * e] = fmaf(u, cv[e], -(v * sv[e]));
-    x[2 * e + 1] = fmaf(v, cv[e], u * sv[e]);
+    x[2 * e] = __fmul_rn(u, cv[e]) - __fmul_rn(v, sv[e]);
+    x[2 * e + 1] = __fmul_rn(v, cv[e]) + __fmul_rn(u, sv[e]);
   }
 }
 __device__ __forceinline__ void pooled_angles(const PooledProj &p, int64_t pos, int ch, float4 &co, float4 &si) {
