@@ -247,11 +247,14 @@ __global__ __launch_bounds__(256) void pool_blocks_kernel(const PooledCache c, c
 }
 
 // Keys and values of prompt portions from the projection, and the means of the blocks that they complete: a wave takes a KV head's tokens of one
-// block, 16 lanes a quarter of them, eight dimensions a lane.  Queries are made where they are read (pooled_prefill.hip).
+// block, 16 at a time, 16 lanes four of them, eight dimensions a lane.  Queries are made where they are read (pooled_prefill.hip).  Means are sums of
+// the tokens in turn, as pool_block_chunk makes them, so rows go through LDS, from which a lane adds up four dimensions of all of them.
 //
-// Eight prompts of 1061 to 2048 tokens, 8 KV heads of 128, blocks of 16: 25 MB read and 53 written in some 10 us.  With 16 lanes for a whole block, one or
-// two waves on a SIMD, a layer took 272 us where it takes 262 so (285 with all 16 tokens' loads under way at once), and one prompt of 203 tokens behind
-// 320 took 36 and takes 27: the tokens of a lane come one after the other.
+// Eight prompts of 1061 to 2048 tokens, 8 KV heads of 128, blocks of 16: 25 MB read and 53 written in 22 - 26 us under the profiler, where a copy of as
+// much takes 15; a wave lives for one round of loads, a sum over 16 lanes and its stores.  With 16 lanes for a whole block, one or
+// two waves on a SIMD, a layer took 272 us where it took 262 so (285 with all 16 tokens' loads under way at once), and one prompt of 203 tokens behind
+// 320 took 36 and takes 26: the tokens of a lane come one after the other.  Means from quarters added up by lane exchanges, in another order, took
+// the same time (layer 263.0 and 262.4).
 struct PooledKvArgs {
   PooledCache c;
   PooledProj p;
@@ -261,37 +264,40 @@ struct PooledKvArgs {
 };
 
 __global__ __launch_bounds__(256) void pooled_kv_kernel(const PooledKvArgs a) {
-  constexpr int kBatch = 4;                                  // tokens whose loads are under way at once
+  constexpr int kEach = 4, kRows = 4 * kEach;                // tokens of a lane, whose loads are under way at once, and of the wave
+  __shared__ __attribute__((aligned(16))) unsigned short rows_lds[4][kRows][2][128];       // K, V
   const PooledCache &c = a.c;
   const int seq = a.first_seq + blockIdx.y, q0 = a.cu_q[seq], n = a.cu_q[seq + 1] - q0, start = a.starts[seq];
-  const int lane = threadIdx.x & 63, wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = blockIdx.x * 4 + w;
   const int j = lane % 16, quarter = lane / 16, b = start / c.pool + wave / c.G, head = wave % c.G;
   if (n <= 0 || b > (start + n - 1) / c.pool) return;        // whole waves leave together
   const int32_t *bt = c.bt + seq * c.bt_stride;
-  const int col = min(j * 8, c.D - 8), per = (c.pool + 3) / 4, first = b * c.pool + quarter * per, end = min((b + 1) * c.pool, first + per);
+  const int col = min(j * 8, c.D - 8), end = (b + 1) * c.pool;
   const bool mine = j * 8 < c.Dp, real = j * 8 < c.D;
-  const bool whole = (b + 1) * c.pool <= start + n;          // its mean is due
+  const bool whole = end <= start + n;                       // its mean is due
   const unsigned short *rows = a.p.rows + static_cast<int64_t>(a.H + head) * c.D + col;
   unsigned short *kc = static_cast<unsigned short *>(const_cast<void *>(c.k)), *vc = static_cast<unsigned short *>(const_cast<void *>(c.v));
-  float bias[8], ks[8], vs[8];
+  float bias[8], sum[4];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) bias[e] = ks[e] = vs[e] = 0.f;
+  for (int e = 0; e < 8; ++e) bias[e] = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) sum[e] = 0.f;
   if (a.p.k_bias) Elem<unsigned short>::ld8(a.p.k_bias + head * c.D + col, bias);
   const int64_t rs = static_cast<int64_t>(c.G) * c.Dp;
-  for (int r0 = 0; r0 < per; r0 += kBatch) {
-    uint4 raw[kBatch];
-    int64_t slot[kBatch];
-    float4 co[kBatch], si[kBatch];
+  for (int r0 = b * c.pool; r0 < end; r0 += kRows) {
+    uint4 raw[kEach];
+    int64_t slot[kEach];
+    float4 co[kEach], si[kEach];
 #pragma unroll
-    for (int k = 0; k < kBatch; ++k) {
-      const int64_t tok = q0 + min(max(first + r0 + k - start, 0), n - 1);
+    for (int k = 0; k < kEach; ++k) {
+      const int64_t tok = q0 + min(max(r0 + quarter * kEach + k - start, 0), n - 1);
       raw[k] = *reinterpret_cast<const uint4 *>(rows + tok * a.p.ld);
       slot[k] = a.slots[tok];
       pooled_angles(a.p, a.p.positions[tok], j, co[k], si[k]);
     }
 #pragma unroll
-    for (int k = 0; k < kBatch; ++k) {
-      const int at = first + r0 + k;
+    for (int k = 0; k < kEach; ++k) {
+      const int at = r0 + quarter * kEach + k;
       float x[8], ss = 0.f;
       unpack8(raw[k], x);
 #pragma unroll
@@ -317,26 +323,28 @@ __global__ __launch_bounds__(256) void pooled_kv_kernel(const PooledKvArgs a) {
         kr = *reinterpret_cast<const uint4 *>(kc + from);
         vr = *reinterpret_cast<const uint4 *>(vc + from);
       }
-      float kf[8], vf[8];
-      unpack8(kr, kf);
-      unpack8(vr, vf);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        ks[e] += kf[e];
-        vs[e] += vf[e];
+      if (whole) {
+        *reinterpret_cast<uint4 *>(&rows_lds[w][quarter * kEach + k][0][j * 8]) = kr;
+        *reinterpret_cast<uint4 *>(&rows_lds[w][quarter * kEach + k][1][j * 8]) = vr;
       }
     }
+    if (!whole) continue;
+    wave_lds_fence();
+#pragma unroll 4
+    for (int r = 0; r < min(kRows, end - r0); ++r) {
+      const uint2 u = *reinterpret_cast<const uint2 *>(&rows_lds[w][r][lane / 32][lane % 32 * 4]);
+      sum[0] += __uint_as_float(u.x << 16);
+      sum[1] += __uint_as_float(u.x & 0xffff0000u);
+      sum[2] += __uint_as_float(u.y << 16);
+      sum[3] += __uint_as_float(u.y & 0xffff0000u);
+    }
+    wave_lds_fence();
   }
-  if (!whole) return;
+  if (!whole || lane % 32 * 4 >= c.Dp) return;
   const float inv = 1.0f / static_cast<float>(c.pool);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    ks[e] = sum_lanes_16_32_48(ks[e]) * inv;
-    vs[e] = sum_lanes_16_32_48(vs[e]) * inv;
-  }
-  if (!mine || quarter > 1) return;
-  const int64_t to = block_row(c, bt, b) * rs + head * c.Dp + j * 8;
-  Elem<unsigned short>::st8(static_cast<unsigned short *>(const_cast<void *>(quarter ? c.pv : c.pk)) + to, quarter ? vs : ks);
+  const int64_t to = block_row(c, bt, b) * rs + head * c.Dp + lane % 32 * 4;
+  *reinterpret_cast<uint2 *>(static_cast<unsigned short *>(const_cast<void *>(lane < 32 ? c.pk : c.pv)) + to) =
+      make_uint2(pack_bf16x2(sum[0] * inv, sum[1] * inv), pack_bf16x2(sum[2] * inv, sum[3] * inv));
 }
 
 // ---------------------------------------------------------------------------------------------------------------
