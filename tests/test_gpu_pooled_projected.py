@@ -79,10 +79,7 @@ def test_projected_portions_are_the_prepared_ones(monkeypatch, H, G, D, rot, siz
             assert taken == [True]
             for name in ("k", "v", "pk", "pv"):
                 assert torch.equal(getattr(new.kv, name), getattr(old.kv, name)), name
-            # Queries are rounded to bf16 with the scale in one form and without it in the other: a score of unit heads, scale * D ** 0.5 = 1.5, is off
-            # by 1.5 * 2 ** -9 * (2 / 3) ** 0.5 between them (root mean square), a weight by no larger a share; the two results' own rounding adds
-            # (2 / 3) ** 0.5 * 2 ** -9.  Together 2.9e-3
-            assert (outs[0].float() - outs[1].float()).norm() <= 2 * 2.9e-3 * outs[1].float().norm()
+            assert torch.equal(outs[0], outs[1])
 
 
 @pytest.mark.gpu
@@ -115,6 +112,30 @@ def test_means_add_up_tokens_in_turn(pool):
 
 
 @pytest.mark.gpu
+def test_weights_of_a_strongly_negative_bias():
+    """2^-bias leaves the range of fp32 where 2^-(score + bias) does not: weights of 2^-90 and the like, not zeros."""
+    H, G, D = 4, 2, 128
+    fields = next(steps_of([150], [[(0, 150)]]))
+    positions, g, outs = fields.pop("positions"), torch.Generator().manual_seed(5), []
+    proj = torch.randn(150, (H + G) * D + 8, generator=g).to(BF16).cuda()
+    proj[:, :G * D] = proj[:, H * D:(H + G) * D]               # heads 0 and 1 ask for their own token: scores of scale * D
+    for projected in (True, False):
+        layer = layer_of(H, G, D, 0, 40, 8, 8, 0, 0.25)
+        layer.score_bias.data.copy_(torch.tensor([-89.0, -100.0, -60.0, 89.0]))
+        out = torch.empty(150, H * D, dtype=BF16, device="cuda")
+        args = (layer.kv, fields["block_tables"], fields["cu_seqlens_q"], fields["seq_starts"], 0, 1, 150)
+        rows, slots, bias = proj[:, :(H + G) * D + H], fields["slot_mapping"], layer.score_bias.data
+        if projected:
+            assert ops.pooled_attention_projected(rows, None, None, positions, layer.cos_sin, 0, slots, bias, *args, 0.25, 1e-6, out)
+        else:
+            q, gate = ops.attn_prep(rows, None, None, positions, layer.cos_sin, 0, slots, layer.kv.k, layer.kv.v, H, D, 1e-6)
+            ops.pool_blocks(*args)
+            ops.pooled_attention_prefill(q, bias, gate, *args, 0.25, out)
+        outs.append(out)
+    assert torch.equal(*outs) and outs[0].view(150, H, D)[:, 0].any()
+
+
+@pytest.mark.gpu
 def test_rows_that_are_not_read_eight_at_a_time_are_prepared():
     """Refused, before anything is launched, and the layer prepares such rows apart."""
     fields = next(steps_of([70], [[(0, 70)]]))
@@ -122,7 +143,7 @@ def test_rows_that_are_not_read_eight_at_a_time_are_prepared():
     t = lambda *s: torch.randn(*s).to(BF16).cuda()
     for D, rot, width, first, bias, scale, takes in ((32, 32, 80, 0, 0, 0.2, True), (32, 32, 84, 0, 0, 0.2, False), (32, 32, 80, 4, 0, 0.2, False),
                                                      (32, 32, 80, 0, 4, 0.2, False), (32, 20, 80, 0, 0, 0.2, False), (36, 32, 120, 0, 0, 0.2, False),
-                                                     (160, 32, 328, 0, 0, 0.2, False), (32, 32, 80, 0, 0, 2.1, True), (32, 32, 80, 0, 0, 2.2, False)):
+                                                     (160, 32, 328, 0, 0, 0.2, False), (32, 32, 80, 0, 0, 2.1, True), (32, 32, 80, 0, 0, 2.2, True)):
         layer = layer_of(1, 1, D, rot, 20, 8, 5, 0, scale)
         proj, qb = t(71, width)[:, first:first + 2 * D + 1][:70], t(D + 8)[bias:bias + D]
         out = torch.full((70, D), 5.0, dtype=BF16, device="cuda")

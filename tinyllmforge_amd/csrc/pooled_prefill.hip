@@ -11,12 +11,12 @@
 // prompt_core.h's.
 //
 // Where rows of the projection can be read eight values at a time, queries and gates are made from them here, by the one workgroup that reads them
-// (PROJ): 12240 tokens write and read 200 MB less, and a layer has two launches in place of three.  Eight prompts as above 285 -> 262 us: preparing
-// and pooling took 55 + 13, keys and values alone take some 10 (pooled_attn.hip: pooled_kv_kernel); making queries adds 27 to the launch, 17 of them
-// waiting for rows that come from memory instead of the caches and the norm, 10 biases and rotation.  One prompt of up to 320 tokens 30 -> 21.  With the
-// scale in the queries, which are fp32 until they are rounded, a score takes an instruction less: 263 -> 259, and 256 with pages by scalar loads.
-#include <math.h>
-
+// (PROJ): 12240 tokens write and read 200 MB less, and a layer has two launches in place of three.  All bits are those of rows prepared on their own.
+// Eight prompts as above 296 -> 266 us: under the profiler, least times, preparing took 54, pooling 13 and this 238; now keys, values and means
+// take 22 (pooled_attn.hip: pooled_kv_kernel) and this 258: rows that come from memory instead of the caches, the norm, biases and rotation.  Three
+// of the 30 are pages by scalar loads.  One prompt of up to 320 tokens 30 -> 22.  With the scale in the queries before they are rounded, and 2^-bias
+// as a factor, a score takes an instruction less, 262 for 266; but results then are not those of prepared rows, and such a factor leaves the range of
+// fp32 at a bias of -89.
 #include "pooled_attn.h"
 #include "prompt_core.h"
 #include "prompt_tiles.h"
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   const int head = kvh * p.group + pass * p.hpp + (hh < nh ? hh : 0), row = uok ? r : row0;
   const int upos = start + row, unb = pooled_visible(upos, c.size, c.pool);
   const int64_t unit = static_cast<int64_t>(q0 + row) * p.H + head;
-  const float nscale = -p.scale_log2, pb = -kLog2e * bf16_bits_to_float(p.bias[head]), tb = PROJ ? __builtin_amdgcn_exp2f(pb) : 0.f;
+  const float pb = -kLog2e * bf16_bits_to_float(p.bias[head]), nscale = -p.scale_log2;
   const unsigned short *qp = PROJ ? p.proj.rows + static_cast<int64_t>(q0 + row) * p.proj.ld + head * c.D : p.q + unit * Core::DP;
   const int64_t pos = PROJ ? p.proj.positions[q0 + row] : 0;
   uint4 raw[2 * DC];                                         // of this lane's pieces of 8, every other one of the row
@@ -152,7 +152,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
 #pragma unroll
     for (int kc = 0; kc < 2 * DC; ++kc) pooled_angles(p.proj, pos, kc * 2 + g, co[kc], si[kc]);
     copy(0, PromptPart<true, true>{});
-    float x[2 * DC][8], ss = 0.f;
+    float x[2 * DC][8], ss[8];                               // sums of squares added up as 16 lanes with a piece each add them
+#pragma unroll
+    for (int kc = 0; kc < 8; ++kc) ss[kc] = 0.f;
 #pragma unroll
     for (int kc = 0; kc < 2 * DC; ++kc) {
       const int col = kc * 16 + g * 8;
@@ -169,9 +171,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         for (int e = 0; e < 8; ++e) x[kc][e] = 0.f;
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ss = fmaf(x[kc][e], x[kc][e], ss);
+      for (int e = 0; e < 8; ++e) ss[kc] = fmaf(x[kc][e], x[kc][e], ss[kc]);
+      ss[kc] = prompt_unit_sum(ss[kc]);
     }
-    const float inv = nscale / sqrtf(prompt_unit_sum(ss) / static_cast<float>(c.D) + p.proj.eps);
+    const float sum = ((ss[0] + ss[1]) + (ss[2] + ss[3])) + ((ss[4] + ss[5]) + (ss[6] + ss[7]));
+    const float inv = 1.0f / sqrtf(sum / static_cast<float>(c.D) + p.proj.eps);
 #pragma unroll
     for (int kc = 0; kc < 2 * DC; ++kc) {
 #pragma unroll
@@ -197,7 +201,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
       [&](int t, int hf, const typename Core::Scores &s, typename Core::Weights &w, auto part) __attribute__((always_inline)) {
         float e[16];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) e[j] = PROJ ? __builtin_amdgcn_rcpf(fmaf(__builtin_amdgcn_exp2f(s[j]), tb, 1.0f)) : sigmoid_neg_log2(fmaf(s[j], nscale, pb));
+        for (int j = 0; j < 16; ++j) e[j] = sigmoid_neg_log2(fmaf(s[j], nscale, pb));
         if (part.mask) {
           const bool pooled = part.lead && t < ptiles;       // workgroup uniform
           const int key = t * kTK + hf * 32 + (pooled ? 0 : w0 - ptiles * kTK) + g * 8;
@@ -460,9 +464,7 @@ extern "C" int tlf_pooled_attn_portions(const void *proj, int64_t proj_stride, c
   pooled_cache_finish(c);
   const PooledProj p{static_cast<const unsigned short *>(proj), proj_stride, static_cast<const unsigned short *>(q_bias),
                      static_cast<const unsigned short *>(k_bias), positions, cos_sin, max_pos, rot_dims, eps};
-  // Queries come with the scale, so that a weight is 1 / (1 + 2^s 2^b), one instruction less: no 2^s may leave the range of fp32, and none of unit
-  // heads does at less than this
-  if (!pooled_proj_takes(p, head_dim) || !(fabsf(scale) * static_cast<float>(c.Dp) * kLog2e <= 100.f)) return TLF_E_UNSUPPORTED;
+  if (!pooled_proj_takes(p, head_dim)) return TLF_E_UNSUPPORTED;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (int rc = launch_pooled_kv(c, p, slot_mapping, cu_seqlens_q, seq_starts, first_seq, num_seqs, max_tokens, num_q_heads, s)) return rc;
   PooledPrefillArgs a{c, nullptr, static_cast<const unsigned short *>(score_bias), nullptr, p,
