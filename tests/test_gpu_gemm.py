@@ -153,6 +153,28 @@ def test_product_in_two_parts_exact_on_integer_data(M, N, K, w8, rest):
         assert torch.equal(act.view(torch.int16), P.silu_and_mul(torch.cat([gate, up], dim=1)).view(torch.int16))
 
 
+@pytest.mark.parametrize("M,N,K,w8", [(4200, 4096, 8192, True), (8293, 4096, 4096, False)])
+def test_second_part_without_its_scratch(M, N, K, w8):
+    """No scratch, whatever its size is said to be, or one that is not aligned: one part, and the same sums of whole numbers."""
+    from tinyllmforge_amd import _lib, ops as P
+    lib = _lib.load()
+    need = lib.tlf_w8a16_gemm_workspace_bytes(M, N, K)
+    x = torch.randint(-2, 3, (M, K), generator=g(M), dtype=torch.int32).to(BF).to(DEV)
+    wi = torch.randint(-127, 128, (N, K), generator=g(N + K), dtype=torch.int32)
+    scale = torch.full((N,), 2.0 ** -12, device=DEV)
+    w = P.pack_w8(wi.to(torch.int8).to(DEV)) if w8 else (wi * 2.0 ** -12).to(BF).to(DEV)
+    want = P.w8a16_linear(x, w, scale) if w8 else P.bf16_linear(x, w)
+    room = torch.zeros(need + 16, dtype=torch.uint8, device=DEV)
+    assert need and room.data_ptr() % 16 == 0
+    stream = torch.cuda.current_stream().cuda_stream
+    for ws, size in ((None, need), (None, 0), (room.data_ptr() + 4, need), (room.data_ptr(), need - 1)):
+        y = torch.zeros_like(want)
+        rc = lib.tlf_w8a16_gemm(x.data_ptr(), K, w.data_ptr(), scale.data_ptr(), y.data_ptr(), M, N, K, ws, size, stream) if w8 else \
+            lib.tlf_bf16_gemm(x.data_ptr(), K, w.data_ptr(), y.data_ptr(), M, N, K, ws, size, stream)
+        assert rc == 0 and torch.equal(y, want), (ws is None, size)
+    assert not room.any()
+
+
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448])
 @pytest.mark.parametrize("M,N,w8", [(1300, 6160, True), (2000, 8208, True), (600, 2064, True), (2100, 8208, False), (1200, 2064, False)])
 def test_pipelines_of_few_steps_exact_on_integer_data(M, N, K, w8):

@@ -1771,7 +1771,7 @@ int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *sca
   const int32_t first = act == 2 || tail || qk ? 0 : gemm_main_rows(M, N, K, W8);
   if (first) {
     if (plan_out) return launch_gemm_rows<W8>(nullptr, K, nullptr, nullptr, nullptr, first, N, K, nullptr, 0, nullptr, plan_out, act);
-    if (act || gemm_split_bytes<W8>(M - first, N, K, !W8) <= (reinterpret_cast<uintptr_t>(workspace) & 15u ? 0 : workspace_bytes)) {
+    if (act || gemm_split_bytes<W8>(M - first, N, K, !W8) <= (workspace && aligned16(workspace) ? workspace_bytes : 0)) {
       if (deferred) *deferred = 1;
       const int rc = launch_gemm_rows<W8>(x, x_stride, w, scale, y, first, N, K, nullptr, 0, stream, nullptr, act);
       if (rc != TLF_OK) return rc;
