@@ -308,3 +308,17 @@ def test_entry_points_reject_bad_arguments_on_the_host():
     assert fused(col=44) == -2 and fused(cols=60) == -2 and fused(ld=56) == -2 and fused(pq=None) == -1
     assert lib.tlf_xielu(a, 10, None, 1, None, 4, a, a, 8, 2, 8, 8, 0, None) == -2
     assert lib.tlf_xielu(a, 16, None, 1, None, 4, None, a, 8, 2, 8, 8, 0, None) == -1
+
+
+@pytest.mark.parametrize("experts,identity,top,inter,columns,edges", [
+    (32, 2, 4, 768, 1024, (8, 32, 511)), (32, 2, 4, 768, 2048, (8, 32, 511)), (64, 0, 4, 960, 2048, (8, 32, 511)), (32, 0, 2, 1024, 4096, (16, 32, 511)),
+    (16, 0, 4, 1536, 4096, (16, 32, 511)), (64, 0, 1, 1024, 1024, (22, 32, 511)), (64, 4, 8, 1536, 4096, (22, 32, 511)), (16, 1, 8, 4096, 3072, (22, 32, 511))])
+def test_tile_rows_on_both_sides_of_each_bound(experts, identity, top, inter, columns, edges):
+    """The most rows an expert that a tile of 32, 64 and 128 rows is taken for; identity experts move no bound."""
+    from types import SimpleNamespace
+    from tinyllmforge_amd.layers.moe import GroupedExperts
+    layer = SimpleNamespace(router=torch.zeros(1, dtype=torch.bfloat16), experts=experts, identity=identity, top=top, inter=inter, columns=columns)
+    per = experts // top                                      # tokens for one row an expert
+    for rows, below, above in zip(edges, (32, 64, 128), (64, 128, 256)):
+        assert GroupedExperts.tile_rows(layer, rows * per) == below and GroupedExperts.tile_rows(layer, (rows + 1) * per) == above
+    assert GroupedExperts.tile_rows(SimpleNamespace(router=torch.zeros(1)), 100) == 64

@@ -1801,22 +1801,28 @@ int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *sca
 //   62 rows, 64 of 1536 (500 tokens)                        K 1536 127, 130, 138; 2048 195, 175, 185; 3072 231, 229, 240; 4096 363, 307, 319
 //   250 rows, 64 of 1536 (2000 tokens)                      K 1536 235, 235, 245; 2048 299, 295, 310; 3072 431, 421, 435; 4096 565, 546, 571
 //   2048 rows (16,384 tokens, 4096)                         256 x 256: 3066 / 1704   256 x 128: 3187 / 1879 128 x 128: 3865 / 2298
-// Both products, us, in 32 / 64 / 128 rows, for even loads and, behind them, for a router whose corrections spread them (up to 5 times the mean):
-//   32 of 768 at 1024   9 rows 28.9, 30.3, 33.1; 29.3, 30.0, 31.4    17 rows 29.2, 30.8, 32.8; 29.4, 30.5, 32.0    28 rows 35.4, 31.7, 33.1; 35.0, 31.9, 32.7
-//   64 of 1024 at 2048                         153, 189, 177                              156, 192, 178             26 rows 171, 192, 180; 30 171, 191, 183
-//   64 of 1536 at 4096         403, 451, 430; 418, 454, 438                   413, 458, 435; 436, 493, 448          28 rows 461, 466, 443; 496, 496, 483
-// and in 128 / 192 / 256 rows, where second tiles of 128 rows begin a second round of two workgroups a CU (192 rows by 128 channels, two of them a CU as well):
-//   32 of 768 at 1024   117 rows 42.6, 47.6, 53.6   122 53.5, 48.3, 54.3   132 57.0, 49.6, 54.5; 54.3, 49.1, 53.5   154 62.6, 49.5, 55.9
-//                       162 70.7, 51.7, 55.4; 58.1, 64.9, 55.1   188 68.5, 68.6, 57.3   226 80.1, 82.7, 60.3; 71.5, 72.3, 61.9   254 80.2, 87.1, 91.2; 73.0, 77.0, 89.0
-//   at 1536             150 81.1, 61.3, 67.3; 80.4, 65.1, 68.1   190 87.5, 70.7, 70.1; 85.9, 90.0, 71.8   240 95.0, 108, 75.9; 95.5, 99.3, 81.0
-// Elsewhere 128 rows stay the better choice or the safer one: 64 of 512 at 1024, 150 rows 70.3, 57.1, 59.2 but spread 66.0, 70.1, 92.6; 64 of 1536 at 4096, 132
-// rows 633, 592, 638 but spread 607, 666, 724; 16 of 1024 at 512, 150 rows 29.0, 29.3, 43.6.
+// Which rows a tile has is GroupedExperts.tile_rows's choice, from sizes alone; how a router spreads its tokens is not known to it.  Both products, of 64
+// rows = 100, for a random router and for corrections that spread the loads (deviation about half the mean, and the mean itself; experts of ff at width):
+//   in 32 rows, by rows an expert   8           12          16          18          22          27
+//   32 of 768 at 1024               96 98 104   96 97 106   95 96 113   96 97 114   96 112 113  109 112 126
+//   32 of 768 at 2048               97 96 96    98 96 100   98 97 102   97 97 100   97 101 114  105 119 120
+//   64 of 768 at 1024               97 94 106   95 95 109   95 95 108   95 95 89    97 108 89   109 111 97
+//   32 of 1024 at 4096              77 78 79    78 77 86    79 77 86    79 87 87    79 86 87    88 98 102
+//   16 of 1536 at 4096              83 83 83    83 84 92    84 84 101   84 85 99    84 109 102  84 107 102
+//   128 of 512 at 1024              88 88 89    87 89 92    87 88 91    88 94 91    95 93 92    93 94 99
+//   32 of 2048 at 2048              79 79 83    79 79 84    79 80 84    79 80 84    79 84 83    83 81 88
+//   64 of 1536 at 3072              97 98 99    98 98 100   98 98 91    98 104 90   103 101 96  106 112 102
+//   64 of 1536 at 4096              90 90 90    90 88 94    90 90 90    91 95 90    90 95 94    98 101 102
+// In 128 rows at 27: 32 of 768 at 2048 103 105 116, 32 of 2048 at 2048 96 96 113, 32 of 1024 at 4096 100 100 126, 64 of 1536 at 4096 94 95 92.
+// Measured and not taken: 192 x 128 tiles, two of them on a CU, and 256 x 256 ones where second tiles of 128 rows begin a second round.  Of 128
+// rows = 100 at 145 rows an expert: 32 of 768 at 1024 82 90 113 and 90 90 97, 24 of 768 72 112 104 and 89 139 123, 16 of 1280 79 116 90 and 105 143 111,
+// 32 of 640 69 77 88 and 84 88 94; at 205: 102 - 114 88 - 114 84 - 114, and 83 - 107 83 - 109 88 - 123.
 int launch_grouped(GemmParams p, int bm, hipStream_t stream) {
   if (p.N % 16 || p.K % kBK || p.m_tiles <= 0) return TLF_E_SHAPE;
   const int ktiles = p.K / kBK;
   const bool deep = bm == 32 && ktiles >= 64 && ktiles % 4 == 0;
   const bool pairs = bm == 128 && p.act && ktiles < 32;
-  const int bn = deep ? 64 : bm <= 64 || bm == 192 || pairs ? 128 : 256;
+  const int bn = deep ? 64 : bm <= 64 || pairs ? 128 : 256;
   p.splits = 1;
   p.k_per_split = p.K;
   p.n_tiles = (p.N + bn - 1) / bn;
@@ -1836,7 +1842,6 @@ int launch_grouped(GemmParams p, int bm, hipStream_t stream) {
   if (deep) TLF_GROUPED(64, 32, 2, 1, 3, 4, 4);
   else if (bm == 32) TLF_GROUPED(128, 32, 4, 1, 4, 4, 1);
   else if (bm == 64) TLF_GROUPED(128, 64, 4, 1, 2, 3, 1);
-  else if (bm == 192) TLF_GROUPED(128, 192, 4, 2, 2, 2, 1);
   else if (pairs) TLF_GROUPED(128, 128, 4, 2, 2, 2, 1);
   else if (bm == 128) TLF_GROUPED(256, 128, 4, 2, 3, 2, 1);
   else if (bm == 256) TLF_GROUPED(256, 256, 4, 2, 2, 2, 1);

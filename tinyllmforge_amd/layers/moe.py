@@ -57,13 +57,10 @@ class GroupedExperts(nn.Module):
         """Rows of a tile of the grouped products: rows per expert decide between streaming the weights and reusing them."""
         if self.router.dtype == torch.float32:
             return 64
-        rows = tokens * self.top / (self.experts + self.identity)
-        if rows <= 32:
-            return 32 if rows <= (18 if self.columns < 2048 else 22) else 64 if self.columns < 2048 else 128
-        # a round of 512 workgroups takes a tile of each expert and some more, and not two of each
-        if 125 < rows <= 243 and 256 < self.experts * -(-self.inter // 64) <= 384 and self.columns <= 2048:
-            return 192 if rows <= 164 else 256
-        return 128 if rows < 480 else 256
+        rows = tokens * self.top / self.experts
+        # Tiles of 32 rows beyond 8 where that pays for uneven loads too: many workgroups, or K long enough to be split inside one
+        few = 22 if self.experts * (self.inter // 64) >= 1024 else 16 if self.columns >= 4096 else 8
+        return 32 if rows <= few else 64 if rows <= 32 else 128 if rows < 512 else 256
 
     def routes(self) -> dict:
         """Checkpoint names -> (parameter, part of it)."""
