@@ -471,3 +471,26 @@ def test_a_decode_plan_is_made_only_for_steps_that_read_it(max_model_len, few):
             assert (getattr(llm.model_runner, "decode_plan_buf", None) is not None) == (n == 9)
     finally:
         llm.exit()
+
+
+@pytest.mark.parametrize("quantization", [None, "w8a16"])
+def test_steps_of_any_size_find_the_products_scratch_there(monkeypatch, quantization):
+    """The largest step does not ask for the most: after the engine's set-up no prompt step allocates scratch for a product."""
+    from tinyllmforge_amd import LLM, SamplingParams, _lib, ops
+    from tinyllmforge_amd.config import QWEN3_SHAPES
+    monkeypatch.setattr(ops, "_workspaces", {})
+    monkeypatch.setattr(ops, "_retired", [])
+    lib, most = _lib.load(), 4000
+    need = lambda m: max(lib.tlf_gemm_add_rmsnorm_workspace_bytes(m, n, k) for n, k in ((4096, 1024), (1024, 2048), (1024, 3072)))
+    worst = max(range(1, most + 1), key=need)
+    assert need(worst) > need(most)
+    llm = LLM(dict(QWEN3_SHAPES["qwen3-0.6b"], num_hidden_layers=1, vocab_size=1024), max_model_len=most, max_num_batched_tokens=most, max_num_seqs=4,
+              num_kvcache_blocks=40, quantization=quantization, enforce_eager=True, seed=1)
+    try:
+        key = (llm.model_runner.device, "gemm")
+        held = ops._workspaces[key]
+        for n in (worst, 7, 900):
+            llm.generate([[i % 1000 for i in range(n)]], SamplingParams(temperature=0.0, max_tokens=2, ignore_eos=True))
+        assert ops._workspaces[key] is held and not any(t is held for t in ops._retired)
+    finally:
+        llm.exit()

@@ -13,6 +13,7 @@ import torch
 
 from .. import _lib, ops
 from ..config import Config
+from ..layers.linear import LinearBase
 from ..layers.sampler import Sampler
 from ..models.registry import model_class
 from ..utils.context import get_context, reset_context, set_context, set_portions_context
@@ -100,7 +101,13 @@ class ModelRunner:
         num_seqs = max(1, min(cfg.max_num_batched_tokens // cfg.max_model_len, cfg.max_num_seqs))
         seqs = [Sequence([0] * cfg.max_model_len) for _ in range(num_seqs)]
         self.run(seqs, True)
+        self.reserve_products()
         torch.cuda.empty_cache()
+
+    def reserve_products(self):
+        """The products' scratch for steps of any size, before the cache takes what is left."""
+        linears = [m for m in self.model.modules() if isinstance(m, LinearBase) and (m.is_quantized or m.weight.dtype == torch.bfloat16)]
+        ops.reserve_products({m.product() for m in linears}, self.config.max_num_batched_tokens, self.device)
 
     def bind_caches(self, pages: int, slots: int):
         """Every layer's paged cache (``pages`` blocks) and recurrent state (``slots`` sequences); 0 frees them.  The
@@ -133,6 +140,7 @@ class ModelRunner:
             seqs.append(seq)
         self.bind_caches(at, cfg.num_state_slots)
         self.run_portions(seqs)
+        self.reserve_products()
         torch.cuda.synchronize()
         stats = torch.cuda.memory_stats()
         held = at * page + slot * cfg.num_state_slots

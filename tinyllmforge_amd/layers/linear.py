@@ -23,6 +23,8 @@ def quantize_per_channel(weight: torch.Tensor):
 
 
 class LinearBase(nn.Module):
+    norm_behind = False            # its rows may be staged in the products' scratch, for a norm
+
     def __init__(self, input_size: int, output_size: int, tp_dim: int | None = None):
         super().__init__()
         self.input_size = input_size
@@ -66,6 +68,11 @@ class LinearBase(nn.Module):
     def load_quantized(self, qweight: torch.Tensor, qscale: torch.Tensor):
         self.qweight, self.qscale = qweight.contiguous(), qscale.contiguous()
         self.weight.data = torch.empty(0, dtype=self.weight.dtype, device=qweight.device)
+
+    def product(self):
+        """Its sizes as ``ops.reserve_products`` takes them."""
+        held = [w for w in (self.qpacked, self.qweight, self.weight) if w is not None]
+        return *held[0].shape, self.norm_behind and self.bias is None
 
     def shard_rows(self, shard_id=None):
         """(first output row, row count) of a checkpoint tensor inside this layer's weight."""
@@ -344,6 +351,7 @@ class GatedUpLinear(MergedColumnParallelLinear):
 
 class QKVParallelLinear(ColumnParallelLinear):
     """q, k and v projections stacked as [q | k | v] along the output dim."""
+    norm_behind = True
 
     def __init__(self, hidden_size: int, head_size: int, total_num_heads: int,
                  total_num_kv_heads: int | None = None, bias: bool = False):
@@ -378,6 +386,8 @@ class QKVParallelLinear(ColumnParallelLinear):
 
 
 class RowParallelLinear(LinearBase):
+    norm_behind = True
+
     def __init__(self, input_size: int, output_size: int, bias: bool = False):
         super().__init__(input_size, output_size, 1)
         self.input_size_per_partition = input_size // self.tp_size

@@ -47,6 +47,14 @@ def _workspace(nbytes: int, device, tag: str) -> torch.Tensor:
     return ws
 
 
+def reserve_products(sizes, rows: int, device):
+    """Allocates the scratch of products, ``sizes`` of ``(channels, K, whether a norm is made behind it)``, for any number of rows up to ``rows``.
+    It does not only grow with them: a product of few rows, or the last rows of many, may split K where the largest does not."""
+    lib = _lib.load()
+    need = (lib.tlf_w8a16_gemm_workspace_bytes, lib.tlf_gemm_add_rmsnorm_workspace_bytes)
+    _workspace(max((need[norm](m, n, k) for n, k, norm in sizes for m in range(1, rows + 1)), default=0), device, "gemm")
+
+
 def kv_dtype_code(cache: torch.Tensor) -> int:
     if cache.dtype == BF16:
         return KV_BF16
