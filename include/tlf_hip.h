@@ -347,12 +347,14 @@ int tlf_bf16_gemm_argmax(const void *x, int64_t x_stride, const void *w, int64_t
                          int32_t M, int32_t N, int32_t K,
                          void *workspace, size_t workspace_bytes, void *stream);
 
-/* Diagnostic, no counterpart in the reference, touches no GPU: the kernel plan the two GEMM entry
- * points would use for a shape.  plan8 = {tile channels, tile tokens, LDS stages, waves/SIMD budget,
- * K-groups per workgroup, split-K factor, K per split, N-tile columns per XCD patch}; tile 0 x 0
+/* Diagnostics, no counterpart in the reference, touch no GPU.  tlf_gemm_plan: the kernel plan that the two GEMM entry
+ * points would use for a shape, of a product in two parts the first one's.  plan8 = {tile channels, tile tokens, LDS stages,
+ * waves/SIMD budget, K-groups per workgroup, split-K factor, K per split, N-tile columns per XCD patch}; tile 0 x 0
  * means the skinny kernel.  Returns TLF_OK when a kernel instance exists for the plan,
- * TLF_E_UNSUPPORTED otherwise (the GEMM call would return the same). */
+ * TLF_E_UNSUPPORTED otherwise (the GEMM call would return the same).
+ * tlf_gemm_parts: the rows of the first part, 0 for a product in one, and the plan of the rows behind it (of all). */
 int tlf_gemm_plan(int32_t M, int32_t N, int32_t K, int32_t w8, int32_t *plan8);
+int tlf_gemm_parts(int32_t M, int32_t N, int32_t K, int32_t w8, int32_t *first_rows, int32_t *plan8);
 
 /* ---------------------------------------------------------------------------
  * a3  paged decode attention   replaces the decode branch layers/attention.py:106-109

@@ -162,6 +162,7 @@ def test_gemm_plan_has_a_kernel_for_every_shape_the_models_use():
                         assert lib.tlf_w8a16_gemm_workspace_bytes(m, n, k) >= splits * m * n * 4
     assert len(seen) >= 6, seen          # the sweep reaches the skinny kernel and several tile shapes
     assert lib.tlf_gemm_plan(4, 1024, 100, 1, plan) == -2   # K not a multiple of 64
+    assert lib.tlf_gemm_parts(4, 1024, 100, 1, plan, plan) == -2 and lib.tlf_gemm_parts(4, 1024, 128, 1, None, plan) == -1
 
 
 def test_gemm_plan_of_a_short_k_follows_what_stays_in_the_caches():

@@ -51,6 +51,7 @@ SIGNATURES = {
     "tlf_add_rmsnorm_gemm_silu_mul_supported": (c_int32, [_I32, _I32, _I32, _I32]),
     "tlf_add_rmsnorm_gemm_silu_mul": (c_int32, [_P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _F, _P]),
     "tlf_gemm_plan": (c_int32, [_I32, _I32, _I32, _I32, _P]),
+    "tlf_gemm_parts": (c_int32, [_I32, _I32, _I32, _I32, _P, _P]),
     "tlf_gemm_add_rmsnorm_workspace_bytes": (_SZ, [_I32, _I32, _I32]),
     "tlf_gemm_argmax_workspace_bytes": (_SZ, [_I32, _I32, _I32]),
     "tlf_gemm_qknorm_rope_store_workspace_bytes": (_SZ, [_I32, _I32, _I32]),

@@ -2102,6 +2102,14 @@ extern "C" int tlf_gemm_plan(int32_t M, int32_t N, int32_t K, int32_t w8, int32_
             : launch_gemm<false>(nullptr, K, nullptr, nullptr, nullptr, M, N, K, nullptr, 0, nullptr, plan8);
 }
 
+extern "C" int tlf_gemm_parts(int32_t M, int32_t N, int32_t K, int32_t w8, int32_t *first_rows, int32_t *plan8) {
+  if (!first_rows || !plan8) return TLF_E_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || K % kBK || N % 16) return TLF_E_SHAPE;
+  const int32_t first = *first_rows = gemm_main_rows(M, N, K, w8 != 0);
+  return w8 ? launch_gemm_rows<true>(nullptr, K, nullptr, nullptr, nullptr, M - first, N, K, nullptr, 0, nullptr, plan8)
+            : launch_gemm_rows<false>(nullptr, K, nullptr, nullptr, nullptr, M - first, N, K, nullptr, 0, nullptr, plan8, 0, nullptr, nullptr, nullptr, first > 0);
+}
+
 extern "C" int tlf_w8a16_gemm_silu_mul(const void *x, int64_t x_stride, const void *wq,
                                        const float *scale, void *y, int32_t M, int32_t N, int32_t K,
                                        void *stream) {
