@@ -117,14 +117,15 @@ def test_bf16_many_rows_of_a_short_k_exact_on_integer_data(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,w8,rest", [
-    (4097, 4096, 256, True, 1), (4113, 4096, 320, True, 17), (5120, 4096, 256, True, 1024), (5121, 4096, 256, True, 0), (5888, 4096, 1536, True, 1792), (5889, 4096, 1536, True, 0),
-    (4300, 4080, 2048, True, 204), (4200, 4096, 8192, True, 104), (12301, 2064, 256, True, 0), (4113, 4096, 192, True, 0), (8208, 4096, 4096, False, 16),
-    (8193, 4096, 320, False, 1), (8449, 4080, 2048, False, 257), (2050, 4096, 4160, False, 2), (2560, 4080, 4160, False, 512),
-    (2561, 4096, 4160, False, 0), (2100, 2048, 2048, False, 52), (2300, 2032, 1024, False, 252), (2300, 2048, 960, False, 0), (2689, 2048, 1024, False, 0), (1025, 4096, 4096, False, 1)])
+    (4097, 4096, 512, True, 1), (4113, 4096, 576, True, 17), (5120, 4096, 512, True, 1024), (5121, 4096, 512, True, 0), (9984, 4096, 1536, True, 1792), (9985, 4096, 1536, True, 0),
+    (4300, 4080, 2048, True, 204), (4200, 4096, 8192, True, 104), (12301, 2064, 512, True, 0), (4113, 4096, 448, True, 0), (5888, 4096, 1536, True, 0), (8208, 4096, 4096, False, 16),
+    (8193, 4096, 576, False, 1), (8449, 4080, 2048, False, 257), (2050, 4096, 4160, False, 2), (2560, 4080, 4160, False, 512),
+    (2561, 4096, 4160, False, 0), (2100, 2048, 2048, False, 52), (2300, 2032, 2048, False, 252), (2300, 2048, 1984, False, 0), (2689, 2048, 2048, False, 0), (1025, 4096, 4096, False, 1),
+    (6095, 6912, 4160, False, 0)])
 def test_product_in_two_parts_exact_on_integer_data(M, N, K, w8, rest):
     """Whole rounds of large tiles and ``rest`` rows behind them (one row, the skinny kernel's last and the next one, whole and cut tiles, the most
-    there are, splits of K) and their neighbours in one part: exact in any order, so the same with rows that are not contiguous, without the scratch
-    that the second part asks for, and from the entry point that leaves partial sums."""
+    there are, splits of K) and their neighbours in one part (more rows behind, a short K, a whole with another plan, a first part of 47 tile rows): exact in
+    any order, so the same with rows that are not contiguous, without the scratch that the second part asks for, and from the entry point that leaves partial sums."""
     import ctypes
     from tinyllmforge_amd import _lib, ops as P
     lib = _lib.load()

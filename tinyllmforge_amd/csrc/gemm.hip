@@ -329,7 +329,7 @@ void gemm_dlds_kernel(const GemmParams params) {
   TLF_DL_ISSUE(Xs0, Ws0, 0)
   if constexpr (NS == 3) {
     // The last two steps copy nothing: a copy that only keeps the count even would be waited for before LDS is released.  With that and the
-    // scales above, us: 4096 x 4096 in int8 at 12288 tokens 338 -> 327, x 12288 961 -> 946; gated experts of 1021 rows 89.8 -> 88.7 a layer.
+    // scales above, us: 4096 x 4096 in int8 at 12288 tokens 338 -> 327, x 12288 961 -> 946.
     if (nkt > 1) TLF_DL_ISSUE(Xs1, Ws1, 1)
     const int rest = (nkt - 2) % 3;                          // (-1 for one tile)
     for (int t = 0; t < nkt - 2 - rest; t += 3) {
@@ -1525,6 +1525,13 @@ inline bool plan_override(GemmPlan &g, int K) {
 
 inline int skinny_max_m() { return gemm_tuning().skinny_max_m; }
 
+// Tile rows (columns) that an XCD walks side by side, as many as divide its share; an XCD owns rows from 16 of them on.
+inline bool gemm_xcd_rows(int m_tiles) { return m_tiles >= 16; }
+inline int gemm_xcd_patch(int owned, int walked) {
+  const int each = owned / 8;
+  return walked < 8 || each == 0 ? 1 : each % 4 == 0 ? 4 : each % 3 == 0 ? 3 : each % 2 == 0 ? 2 : 1;
+}
+
 // plan_out != nullptr: nothing is launched; the eight plan fields are written there instead and the
 // return code says whether a kernel instance exists for the plan.  tiled: no skinny kernel, however few the rows.
 template <bool W8>
@@ -1602,13 +1609,12 @@ int launch_gemm_rows(const void *x, int64_t x_stride, const void *w, const float
   // Qwen3-8B shapes 0 ... +4 %; at 4096 tokens (16 tile rows) -4 ... +6 %.  (With whole rows or columns per XCD 50 tile
   // rows cost 7 rounds on two XCDs against 6.25 on average: 5120 x 8192 at 12800 tokens 1104 -> 1281 TFLOP/s.)
   // TLF_GEMM_XCD_ROWS = 0 / 1 forces the choice for tuning.
-  p.xcd_rows = p.m_tiles >= 16;
+  p.xcd_rows = gemm_xcd_rows(p.m_tiles);
   if (gemm_tuning().xcd_rows >= 0) p.xcd_rows = gemm_tuning().xcd_rows && p.m_tiles >= 8;
   const int owned_total = p.xcd_rows ? p.m_tiles : p.n_tiles, walked = p.xcd_rows ? p.n_tiles : p.m_tiles;
   const int owned_each = owned_total / 8;     // rows (columns) every XCD owns; the other owned_total % 8 are dealt out tile by tile
   {
-    g.group_n = 1;
-    if (walked >= 8 && owned_each > 0) g.group_n = owned_each % 4 == 0 ? 4 : owned_each % 3 == 0 ? 3 : owned_each % 2 == 0 ? 2 : 1;
+    g.group_n = gemm_xcd_patch(owned_total, walked);
     if (gemm_tuning().group_n && owned_each > 0 && owned_each % gemm_tuning().group_n == 0) g.group_n = gemm_tuning().group_n;
   }
   p.group_n = g.group_n;
@@ -1723,18 +1729,23 @@ int launch_gemm_rows(const void *x, int64_t x_stride, const void *w, const float
 //   256 x 128 tiles, bf16, half as long a round: 4096 x 12288 at 8192 + 400 (64 tiles) 800 / 756, + 800 (112 tiles) 810 / 831
 //   128 x 128 tiles of three stages, bf16 (of int8 two are on a CU): 2560 x 9728 at 3403 226 / 175,
 //                        1024 x 3072 at 4142 45 / 39, 4096 x 4096 at 1208 59 / 53, 2048 x 2048 at 2065 33.1 / 30.7
-// Tiles of 256 x 128 are worth no more than a second pass over a wide weight: 10240 x 5120 in bf16 at 6537, nine rows in the second part, 630 / 642; and
-// those of 128 rows no second launch below K = 1024: int8 6144 x 256 at 1409 15.1 / 18.6, 8192 x 512 at 1224 19.6 / 25.5, bf16 4096 x 512 at 1224 15.6 / 16.5,
-// nor where the whole product has another plan (int8 2048 x 1024 at 12328 61.8 / 66.5).  Below K = 1536 more than 64 tiles of 256 x 256 are as well off in
-// the round (int8 4096 x 320 at 5496, 96 tiles, 23.8 / 25.9, 6144 x 768 at 3716, 120 tiles, 39.6 / 42.0);
-// below 256 a tile of 256 x 256 is little more than a launch (4096 x 128 at 8292 in bf16 34 / 39; x 512 at 12588 72 / 66; 6144 x 256 in int8 at 8492 49 / 46).
-inline int32_t gemm_main_rows(int32_t M, int32_t N, int32_t K, bool w8) {
+// In one part stay, by random shapes timed both ways (1024 to 16384 channels, K 256 to 12288, 500 to 16384 tokens; two parts as a share of one, mean and most):
+// - K below 512, where a tile is little more than a launch: 618 shapes 0.95, 1.29 (13920 x 256 at 3380 in bf16 46.1 / 50.6); at 512 0.94, 1.07.  Tiles of
+//   128 x 128 below 2048 (0.99, 1.06), and below 1536 more than 64 tiles of 256 x 256 (int8 6144 x 768 at 3716, 120 tiles, 39.6 / 42.0).
+// - a whole product with another plan, which fills its rounds in its own way: 803 shapes 1.02, 1.29 (int8 11392 x 4096 at 1353 118 / 137).  Not so the 256 x 128
+//   tiles with two stages, two on a CU: 2116 shapes 0.83.
+// - an activation behind 128 x 128 tiles, for which the rows behind must not split K: 79 shapes 0.98, 1.15.
+// - a first part whose tile rows the XCDs walk one by one, where they walk the whole's three or four at a time (47 rows and 48): 6912 x 5120 in bf16 at 6095 404 / 532.
+// What is cut then: 12972 shapes 0.89, 1.07; 32 of them more than 1.02.  bf16 weights of more than 8192 channels stay whole in 256 x 128 tiles: 10240 x 5120 at
+// 6537 (nine rows behind eight rounds) 630 / 642; with up to five rounds two parts would take 0.91 in the mean of 154 shapes (8448 channels up to 1.09).
+inline int32_t gemm_main_rows(int32_t M, int32_t N, int32_t K, bool w8, bool act = false) {
   constexpr int kCUs = 256;
-  if (gemm_tuning().has_plan || K < 256 || static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128) <= kCUs) return 0;
+  if (gemm_tuning().has_plan || K < 512 || static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128) <= kCUs) return 0;
   struct { int bn, bm, most; } const tiles[] = {{256, 256, 120}, {256, 128, 64}, {128, 128, 64}};
+  const GemmPlan whole = plan_gemm(M, N, K, w8);
   for (const auto &c : tiles) {
-    if (c.bm == 128 && (K < 1024 || (c.bn == 256 && N > (w8 ? 16384 : 8192)))) continue;
-    if (c.bn == 128 && w8) continue;
+    if (c.bm == 128 && K < (c.bn == 128 ? 2048 : 1024)) continue;
+    if (c.bn == 128 ? w8 || act : c.bm == 128 && !w8 && N > 8192) continue;
     const int n = (N + c.bn - 1) / c.bn, m = (M + c.bm - 1) / c.bm;
     if (static_cast<int64_t>(n) * m <= kCUs) continue;
     const int over = static_cast<int>((static_cast<int64_t>(n) * m - 1) % kCUs + 1);   // tiles of the last round
@@ -1743,10 +1754,10 @@ inline int32_t gemm_main_rows(int32_t M, int32_t N, int32_t K, bool w8) {
     const int32_t first = (m - rows) * c.bm;
     const GemmPlan g = plan_gemm(first, N, K, w8);
     if (g.bn != c.bn || g.bm != c.bm || (c.bm == 128 && g.stages != 3) || g.splits != 1 || g.kgroups != 1) continue;
-    if (c.bm == 128) {                                       // not where the whole product would take two smaller or shallower workgroups a CU
-      const GemmPlan whole = plan_gemm(M, N, K, w8);
-      if (whole.bn != g.bn || whole.bm != g.bm || whole.stages != g.stages) continue;
-    }
+    const bool same = whole.bn == g.bn && whole.bm == g.bm && whole.stages == g.stages, pairs = c.bm == 256 && whole.bn == 256 && whole.bm == 128 && whole.stages == 2;
+    if (!same && !pairs) continue;
+    const int left = m - rows;
+    if (same && gemm_xcd_rows(left) && gemm_xcd_patch(left, n) == 1 && gemm_xcd_patch(m, n) >= 3) continue;
     return first;
   }
   return 0;
@@ -1768,7 +1779,7 @@ int launch_gemm(const void *x, int64_t x_stride, const void *w, const float *sca
                 int32_t M, int32_t N, int32_t K, void *workspace, size_t workspace_bytes,
                 hipStream_t stream, int32_t *plan_out = nullptr, int32_t act = 0,
                 const NormTail *tail = nullptr, const QkRopeStoreArgs *qk = nullptr, int32_t *deferred = nullptr) {
-  const int32_t first = act == 2 || tail || qk ? 0 : gemm_main_rows(M, N, K, W8);
+  const int32_t first = act == 2 || tail || qk ? 0 : gemm_main_rows(M, N, K, W8, act != 0);
   if (first) {
     if (plan_out) return launch_gemm_rows<W8>(nullptr, K, nullptr, nullptr, nullptr, first, N, K, nullptr, 0, nullptr, plan_out, act);
     if (act || gemm_split_bytes<W8>(M - first, N, K, !W8) <= (workspace && aligned16(workspace) ? workspace_bytes : 0)) {
