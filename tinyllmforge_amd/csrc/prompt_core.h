@@ -18,8 +18,8 @@
 // faster card 161 -> 152; 250, 198 and 168 registers a lane (251, 236 and 192 before).  In a stream of nothing but these products and weights from
 // registers two waves take 2150 cycles where the products alone take 1540: beside another wave's vector instructions a product takes a
 // fifth longer.  Without copies sinks take 331, without LDS reads of V pooled heads 287.
-// Halves of masked tiles that none of the wave's units sees are left out (half of the row tiles end in the first half of a tile): layers
-// 265.6 -> 262.5 us (pooled, whose window begins in a second half as often, and whose means may end in a first one) and 350.5 -> 347.6 (sinks).
+// Halves of masked tiles that none of the wave's units sees are left out (half of the row tiles end in the first half of a tile, a pooled window begins in a
+// second one as often): layers 261.2 -> 258.9 us (pooled), 347.2 -> 344.7 (sinks) and 141.2 -> 141.1 (latents), where runs of one side differ by 1.5 %.
 // Measured and not taken: scores in front of the values (no difference), reads kept behind the products (3 % slower), wave priorities around the
 // products (3 % slower), workgroups that take their row tiles from a list (1 - 2 % slower, though a new one starts 3.5 us after the one before
 // it ends: while one is away the other runs faster).

@@ -31,7 +31,10 @@ class PooledWindowAttention(nn.Module):
                                self.dtype, device) if pages else None
 
     def forward(self, proj: torch.Tensor, q_bias, k_bias, positions: torch.Tensor) -> torch.Tensor:
-        """``proj``: rows ``[q | k | gate]`` -> ``[N, heads * head_dim]``, gated."""
+        """``proj``: rows ``[q | k | gate]`` -> ``[N, heads * head_dim]``, gated.  Partial sums of a projection (``ops.Deferred``) are added up by the
+        separate preparation, so portions of 17 to 64 and 385 to 768 rows of width 4096 come that way.  (Projection and attention, us, with partial sums and with rows
+        that are finished and read by the attention: 400 rows 63.9 and 59.6, 700 90.1 and 86.4, 64 behind 512 45.3 and 43.2; int8 65.1 and 62.5, 89.3 and 84.2,
+        41.1 and 41.1.)"""
         ctx, kv = get_context(), self.kv
         n, single, bias = proj.shape[0], ctx.num_single, self.score_bias.data
         out = torch.empty(n, self.num_heads * self.head_dim, dtype=proj.dtype, device=proj.device)
@@ -62,8 +65,10 @@ class PooledWindowAttention(nn.Module):
 
     def _from_projection(self, rows: int, portions: int, dtype) -> bool:
         """Whether portions make their queries where the attention reads them.  A workgroup makes those of a tile of rows, there or not, so many short
-        portions are faster with rows prepared: 256 of up to 35 tokens, 26 on average in tiles of 64, 62 us and 68 from the projection, 172 of up
-        to 63 62 and 56; while they do not fill the chip the launches count (24 of up to 141 38 and 29)."""
+        portions are faster with rows prepared, the more so without a context.  us prepared and from the projection, 16 heads on 8, tiles of 64: 256 of up to 12 tokens
+        22.1 and 29.2, of up to 35 34.4 and 37.3, 172 of up to 63 36.5 and 32.8; while they do not fill the chip the launches count: 64 of up to 20
+        20.0 and 12.6, 128 of up to 35 23.8 and 22.4.  On the wrong side of it: 256 of up to 35 in tiles of 32, some in two of them, 44.3 and 45.9; 100 of up to 12 behind 256 held
+        tokens 26.8 and 29.0; prepared, 256 of up to 26 in tiles of 64 behind 256 71.6 and 64.0."""
         if dtype != torch.bfloat16:
             return False
         tile = max(1, 128 * self.num_kv_heads // self.num_heads)
